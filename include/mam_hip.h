@@ -48,7 +48,7 @@ extern "C" {
                                  likewise for min (the retired convolution modules' literal rule)        */
 
 /* Run-time switches for mam_set_option().  Their initial values come from the environment variables of
- * the same names, read once when the library is loaded: MAM_FORWARD_TILING = auto | wide | 0 | 1 | 2 | 3,
+ * the same names, read once when the library is loaded: MAM_FORWARD_TILING = auto | wide | 0 .. 5,
  * MAM_BACKWARD_FORK = auto | -1 | 0 | 1, MAM_BACKWARD_ONE_LAUNCH = auto | 0 (off) | 1 (auto) | 2 (on),
  * MAM_BACKWARD_EXACT = 0 | 1.  A value outside an
  * option's range is refused by mam_set_option() and ignored (with the default kept) in the environment. */
@@ -57,11 +57,15 @@ extern "C" {
 #define MAM_OPT_BACKWARD_ONE_LAUNCH 2 /* both gradients in one launch where the shape allows it    */
 #define MAM_OPT_BACKWARD_EXACT 3 /* w_grad accumulated in 64-bit fixed-point cells (exact sums)    */
 #define MAM_OPT_COUNT_ 4
-#define MAM_FORWARD_TILING_AUTO 0 /* wave-uniform-rows tiling where the layout allows it           */
+#define MAM_FORWARD_TILING_AUTO 0 /* large calls by magnitude-ordered lists; otherwise, and where the data
+                                     does not suit them, the wave-uniform-rows tiling where the layout allows */
 #define MAM_FORWARD_TILING_WIDE 1 /* every call on the general 64 x 128 tiling                     */
 #define MAM_FORWARD_TILING_GROUPS16 2 /* as AUTO, but indices recorded per 16 products at every K   */
 #define MAM_FORWARD_TILING_FUSED_MERGE 3 /* as AUTO, but a K-split call merges inside the forward launch: the
                                             last of a tile's workgroups to finish combines and resolves   */
+#define MAM_FORWARD_TILING_LISTS 4 /* as AUTO, but lists at every size (a dense tiling still serves data that
+                                      does not suit them, and K too large for the LDS)                   */
+#define MAM_FORWARD_TILING_DENSE 5 /* as AUTO, but never by lists                                         */
 #define MAM_BACKWARD_FORK_AUTO (-1) /* where it pays: from 2^23 outputs on with at least 1024 neurons (dense),
                                        2^22 outputs (CSR); under stream capture from 2^16 outputs       */
 #define MAM_BACKWARD_FORK_OFF 0

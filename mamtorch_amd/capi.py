@@ -22,6 +22,8 @@ OPT_BACKWARD_EXACT = 3
 FORWARD_TILING_AUTO = 0
 FORWARD_TILING_WIDE = 1
 FORWARD_TILING_GROUPS16 = 2
+FORWARD_TILING_LISTS = 4
+FORWARD_TILING_DENSE = 5
 BACKWARD_FORK_AUTO = -1
 COUNT_REFERENCE = 0
 COUNT_HITS = 1

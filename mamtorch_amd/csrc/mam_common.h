@@ -37,8 +37,11 @@ int option(int which);
 // Compute units of the current device (read from the device at its set-up).
 int num_cus();
 
-// dst (cols, rows) contiguous = transpose of src (rows, cols), row stride ld.
-int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, hipStream_t stream);
+// dst (cols, rows) contiguous = transpose of src (rows, cols), row stride ld.  `guard` (mam_ordered.h): the
+// kernel exits at once where the guard says that nobody reads the copy.
+namespace ordered { struct Guard; }
+int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, hipStream_t stream,
+              const ordered::Guard *guard = nullptr);
 
 // Two independent kernels of one call side by side: the first runs on a second stream of the library
 // (default priority, one per device) between a fork and a join event on the caller's stream.

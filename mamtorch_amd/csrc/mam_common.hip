@@ -1,5 +1,5 @@
 // Error reporting and version of libmam_hip.so.
-#include "mam_common.h"
+#include "mam_ordered.h"
 
 #include <stdarg.h>
 #include <stdlib.h>
@@ -48,8 +48,10 @@ int fill_zero(void *ptr, int64_t count, hipStream_t stream)
 // dst (cols, rows) contiguous = transpose of src (rows, cols) with row stride ld: 64 x 64 tiles through LDS,
 // 16-byte accesses on both sides when the shapes allow it.
 __global__ __launch_bounds__(256) void transpose_kernel(const float *__restrict__ src, int64_t ld,
-                                                        float *__restrict__ dst, int rows, int cols, int vec)
+                                                        float *__restrict__ dst, int rows, int cols, int vec,
+                                                        const ordered::Guard guard)
 {
+    if (ordered::guarded_off(guard)) return;
     __shared__ float tile[64][65];
     const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
     const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
@@ -90,14 +92,15 @@ __global__ __launch_bounds__(256) void transpose_kernel(const float *__restrict_
     }
 }
 
-int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, hipStream_t stream)
+int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, hipStream_t stream,
+              const ordered::Guard *guard)
 {
     if (rows <= 0 || cols <= 0) return MAM_OK;
     const int64_t gx = ceil_div(cols, 64), gy = ceil_div(rows, 64);
     if (gy > 65535 || gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "matrix too large for the transpose grid");
     const int vec = (ld % 4 == 0) && ((uintptr_t)src % 16 == 0) && ((uintptr_t)dst % 16 == 0);
     hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream, src, ld, dst,
-                       (int)rows, (int)cols, vec);
+                       (int)rows, (int)cols, vec, guard ? *guard : ordered::Guard{nullptr, 0});
     return check_launch("transpose_kernel");
 }
 
@@ -120,7 +123,7 @@ int g_num_hooks = 0;
 // The values each option accepts.
 struct OptionRange { const char *env; int lo, hi, fallback; bool wide_word; };
 constexpr OptionRange kOptionRanges[MAM_OPT_COUNT_] = {
-    {"MAM_FORWARD_TILING", MAM_FORWARD_TILING_AUTO, MAM_FORWARD_TILING_FUSED_MERGE, MAM_FORWARD_TILING_AUTO, true},
+    {"MAM_FORWARD_TILING", MAM_FORWARD_TILING_AUTO, MAM_FORWARD_TILING_DENSE, MAM_FORWARD_TILING_AUTO, true},
     {"MAM_BACKWARD_FORK", MAM_BACKWARD_FORK_AUTO, MAM_BACKWARD_FORK_ON, MAM_BACKWARD_FORK_AUTO, false},
     {"MAM_BACKWARD_ONE_LAUNCH", MAM_BACKWARD_ONE_LAUNCH_OFF, MAM_BACKWARD_ONE_LAUNCH_ON, MAM_BACKWARD_ONE_LAUNCH_AUTO,
      false},

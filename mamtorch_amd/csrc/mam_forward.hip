@@ -32,7 +32,7 @@
 // Small N*M (the 256 x 4096 headline shape has only 256 tiles for 256 CUs x 2) is split
 // along K; each split writes (value, group) partials and a merge kernel combines them in
 // ascending k order with the same strict comparisons before resolving indices.
-#include "mam_common.h"
+#include "mam_ordered.h"
 #include "mam_offsets.h"
 
 #include <stdlib.h>
@@ -71,6 +71,7 @@ struct Params {
     int fast;          // the k-invariant 32-bit-offset staging path is legal
     int coop;          // the cooperative resolve is legal: (M,K) w, 16-byte rows, K % G == 0
     int group_n;       // row tiles swept under one W panel (tile order of the launch)
+    ordered::Guard guard;   // the kernels exit at once where the lists serve the call (mam_ordered.hip)
     int gt;            // products per recorded group: G, or 2 G on the wave-uniform-rows tiling at large K
 };
 
@@ -472,6 +473,7 @@ __device__ __forceinline__ void compute_tile(const float *tile, int tx, int ty, 
 template <int LAYOUT, bool ARGS>
 __global__ __launch_bounds__(NT, 2) void mam_fwd_kernel(const Params p)
 {
+    if (ordered::guarded_off(p.guard)) return;
     // Two tile buffers as two separate arrays: the compiler can then see that loads in flight
     // into one never alias reads of the other, and lets them overlap.
     __shared__ __attribute__((aligned(16))) float tile_a[TILE_FLOATS];
@@ -684,6 +686,7 @@ __global__ __launch_bounds__(NT, 2) void mam_fwd_kernel(const Params p)
 template <int LAYOUT, bool ARGS, bool COOP, int GT = G>
 __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
 {
+    if (ordered::guarded_off(p.guard)) return;
     // A workgroup owns a PR x PC patch of c (16 x 16; with the cooperative resolve 4 x 64: a wave takes one batch
     // row, and its piece of every partial plane and of every output array is two whole 128-byte lines; measured at
     // 256 x 4096 x 4096: 28.4 us with 16 x 16, 27.0 with 8 x 32, 26.6 with 4 x 64).  Resolving re-reads GT
@@ -871,6 +874,7 @@ typedef const __attribute__((address_space(4))) float const_f32;
 template <int TJ, bool ARGS, bool SPLIT, bool TAIL, int GT = G, bool FUSE = false>
 __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
 {
+    if (ordered::guarded_off(p.guard)) return;
     using C = sx::Cfg<TJ>;
     __shared__ __attribute__((aligned(16))) float tile_a[C::TILE_FLOATS];
     __shared__ __attribute__((aligned(16))) float tile_b[C::TILE_FLOATS];
@@ -1300,6 +1304,7 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     }
     p.splits = (int)ceil_div(K, p.k_per_split);
     p.part = nullptr;
+    p.guard = ordered::Guard{nullptr, 0};
     plan.need = p.splits > 1 ? (size_t)p.splits * (args ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float) : 0;
     // the fused merge keeps one ticket per tile behind the partials
     plan.tickets_at = plan.need;
@@ -1350,6 +1355,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     // workspace has room, b is transposed ONCE into it and the wave-uniform-rows tiling runs on the copy
     // (0.22 ms + the transpose): every output is the same, bit for bit.
     size_t wt_bytes = 0;
+    const int operand_layout = w_layout;
     if (w_layout == MAM_W_KM && transposed_operand_pays(N, K, M)) {
         Plan tplan;
         float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
@@ -1397,9 +1403,19 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
         rc = fill_zero(p.tickets, (int64_t)p.tiles_n * p.tiles_m, st);
         if (rc != MAM_OK) return rc;
     }
+    // Large calls by magnitude-ordered lists, where the workspace has room for them; the kernels below then run
+    // only if the data turns out not to suit the lists.
+    if (range_len == 0 && !static_scratch && ordered::applies(N, K, M)) {
+        const size_t at = (wt_bytes + need + 255) / 256 * 256;
+        if (avail >= at + ordered::workspace_bytes(N, K, M) && (uintptr_t)workspace % 16 == 0) {
+            const ordered::Call call = {x, ldx, w, ldw, operand_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M};
+            rc = ordered::launch(call, scratch_base + at, p.guard, st);
+            if (rc != MAM_OK) return rc;
+        }
+    }
     if (wt_bytes > 0) {
         float *wt = reinterpret_cast<float *>(scratch_base);
-        rc = transpose(w, ldw, wt, K, M, st);
+        rc = transpose(w, ldw, wt, K, M, st, &p.guard);
         if (rc != MAM_OK) return rc;
         p.w = wt;
     }
@@ -1469,6 +1485,7 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     // room for the transposed copy of a (K, M) operand (see launch); without it the call still works
     if (w_layout == MAM_W_KM && K % mam::fwd::G == 0 && mam::fwd::transposed_operand_pays(N, K, M))
         bytes += ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256;
+    if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M);
     return bytes;
 }
 

@@ -1,0 +1,120 @@
+"""The forward over magnitude-ordered lists (csrc/mam_ordered.hip) against the C oracle, bit for bit: sizes on both
+sides of every tile width, list operands on either side, and data that the lists do not finish (ties, zeros,
+NaN / infinities, one sign, sparse rows, denormal and overflowing products)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from helpers import assert_bits_equal, assert_index_equal
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _data(kind, rows, k, g):
+    t = torch.randn(rows, k, generator=g)
+    r = torch.rand(rows, k, generator=g)
+    if kind == "uniform":
+        t = r * 2 - 1
+    elif kind == "ties":
+        t = (t * 4).round() / 4
+    elif kind == "positive":
+        t = r + 0.1
+    elif kind == "zero rows":
+        t[torch.rand(rows, generator=g) < 0.3] = 0
+        t[0] = -0.0
+    elif kind == "nan and inf":
+        t[r < 1e-3] = float("nan")
+        t[(r > 0.5) & (r < 0.501)] = float("inf")
+        t[(r > 0.6) & (r < 0.601)] = -float("inf")
+        t[(r > 0.7) & (r < 0.8)] = -0.0
+    elif kind == "sparse":
+        t[r < 0.97] = 0
+    elif kind == "denormal":
+        t = t * 1e-24
+    elif kind == "overflow":
+        t = t * 1e25
+    return t
+
+
+def _check(N, K, M, kind_x, kind_w, layout_mk=True, pad=0, seed=0):
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(seed)
+    x = _data(kind_x, N, K + pad, g)[:, :K]
+    w = _data(kind_w, M, K, g)
+    bias = torch.randn(M, generator=g)
+    want = oracle.forward(x.contiguous().numpy(), w.numpy(), oracle.W_MK, bias.numpy())
+    xd = _strided(x, pad)
+    wd = (w if layout_mk else w.T.contiguous()).to(DEV)
+    layout = capi.W_MK if layout_mk else capi.W_KM
+    w_sel, x_sel = torch.zeros(2, N, M, device=DEV), torch.zeros(2, N, M, device=DEV)
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
+    try:
+        c, amax, amin = capi.fc_forward(xd, wd, layout, bias.to(DEV), w_sel=w_sel, x_sel=x_sel)
+        values = capi.fc_forward_values(xd, wd, layout, bias.to(DEV))
+        torch.cuda.synchronize()
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    tag = "%s x %s, N %d K %d M %d" % (kind_x, kind_w, N, K, M)
+    assert_bits_equal(c.cpu().numpy(), want[0], tag + " c")
+    assert_bits_equal(values.cpu().numpy(), want[0], tag + " values-only c")
+    assert_index_equal(amax.cpu().numpy(), want[1], tag + " argmax")
+    assert_index_equal(amin.cpu().numpy(), want[2], tag + " argmin")
+    rows, cols = np.arange(N)[:, None], np.arange(M)[None, :]
+    for plane, index in enumerate(want[1:3]):
+        assert_bits_equal(x_sel[plane].cpu().numpy(), x.numpy()[rows, index], tag + " x_sel")
+        assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
+
+
+def _strided(x, pad):
+    N, K = x.shape
+    out = torch.zeros(N, K + pad, device=DEV)[:, :K]
+    out.copy_(x.to(DEV))
+    return out
+
+
+@pytest.mark.parametrize("N,K,M", [
+    (64, 1216, 70), (65, 1217, 33), (64, 2432, 34), (33, 2433, 64), (130, 4864, 40), (40, 4865, 36), (34, 9728, 33),
+    (33, 9729, 32), (5, 200, 7), (1, 130, 300), (300, 131, 1), (257, 96, 129), (520, 768, 96)])
+@pytest.mark.parametrize("kinds", [("normal", "uniform"), ("uniform", "normal"), ("normal", "normal")])
+@pytest.mark.parametrize("layout_mk", [True, False])
+def test_sizes_on_both_sides_of_every_tile_width(N, K, M, kinds, layout_mk):
+    _check(N, K, M, *kinds, layout_mk=layout_mk, pad=3 if layout_mk else 0)
+
+
+@pytest.mark.parametrize("kind", ["ties", "positive", "zero rows", "nan and inf", "sparse", "denormal", "overflow"])
+@pytest.mark.parametrize("other", ["uniform", "normal", "same"])
+def test_data_the_lists_do_not_finish(kind, other):
+    for K in (300, 2500):
+        _check(70, K, 68, kind, kind if other == "same" else other, seed=1)
+        _check(70, K, 68, kind if other == "same" else other, kind, seed=2)
+
+
+def test_a_few_bad_rows_among_good_ones():
+    """Rows of zeros, of NaN and of constants inside an otherwise ordinary batch: most of the call goes by lists."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(5)
+    N, K, M = 640, 768, 96
+    x, w = torch.randn(N, K, generator=g), torch.rand(M, K, generator=g) * 2 - 1
+    x[7] = 0.0
+    x[100, 3] = float("nan")
+    x[200] = 1.5
+    x[300, 5] = float("inf")
+    x[400].abs_()
+    w[11] = 0.0
+    w[12] = -0.25
+    w[13, 700] = float("nan")
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK)
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
+    try:
+        c, amax, amin = capi.fc_forward(x.to(DEV), w.to(DEV), capi.W_MK)
+        values = capi.fc_forward_values(x.to(DEV), w.to(DEV), capi.W_MK)
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    assert_bits_equal(c.cpu().numpy(), want[0], "c")
+    assert_bits_equal(values.cpu().numpy(), want[0], "values-only c")
+    assert_index_equal(amax.cpu().numpy(), want[1], "argmax")
+    assert_index_equal(amin.cpu().numpy(), want[2], "argmin")
