@@ -17,8 +17,8 @@
 //   forward_kernel the search itself (below).
 //   dense kernels  exit at once unless the decision was "neither".
 //
-// Measured against the dense tilings (forward call, hand-over arrays written): 207 -> 72 us at 256 x 4096 x 4096,
-// 1.70 -> 0.69 ms and 1.47 -> 0.35 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.81 ms (values only) and 3.13 -> 0.60 ms
+// Measured against the dense tilings (forward call, hand-over arrays written): 207 -> 66 us at 256 x 4096 x 4096,
+// 1.70 -> 0.61 ms and 1.47 -> 0.24 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.82 ms (values only) and 3.13 -> 0.40 ms
 // at 16384 x 4096 -> 4096 / 1024.  A wave's search ends with the slowest of its 256 outputs: 92 entries at K = 4096
 // where the mean output needs 28.
 #include "mam_ordered.h"
@@ -41,13 +41,19 @@ constexpr uint32_t INF_BITS = 0x7f800000u;
 struct Params {
     Call call;
     const Sample *samples;
-    uint4 *lists;          // [entry pair][listed row]: (value, ~k, value, ~k)
+    uint4 *lists;          // [entry pair][listed row]: (value, key, value, key)
     float *bound;          // [chunk][listed row]: bound on the magnitudes from this chunk on
     int limit;             // longest list a sample may ask for
     int cap;               // entries a list can hold (a multiple of CHUNK)
     int rows_pad;          // listed rows, padded, of the longer operand
     int splits_x, splits_w;   // row ranges per tile when x (w) is listed
 };
+
+// A list entry's key: (65535 - k) in the upper half, so that the lower k is the larger key, and its place in the
+// list + 1 in the lower half (0: not from a list), from which the listed value is found again.
+__host__ __device__ __forceinline__ uint32_t key(uint32_t k, uint32_t place) { return ((65535u - k) << 16) | place; }
+__device__ __forceinline__ int index_in(uint32_t key) { return (int)(65535u - (key >> 16)); }
+__device__ __forceinline__ int place_in(uint32_t key) { return (int)(key & 65535u) - 1; }
 
 // rows of one operand: element (row, k)
 struct Rows {
@@ -129,7 +135,7 @@ template <int R>
 __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
 {
     constexpr int WAVES = BUILD_NT / 64;
-    extern __shared__ uint4 lds[];          // [cap] (value, ~k) pairs
+    extern __shared__ uint4 lds[];          // [cap] (value, key) pairs
     __shared__ uint32_t hist[BUCKETS];
     __shared__ uint32_t part[WAVES], part2[WAVES];
     __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
@@ -153,7 +159,7 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     }
 #pragma unroll
     for (int j = 0; j < BUCKETS / BUILD_NT; ++j) hist[j * BUILD_NT + tid] = 0;
-    for (int j = tid; j < len; j += BUILD_NT) items[j] = make_uint2(0u, ~0u);
+    for (int j = tid; j < len; j += BUILD_NT) items[j] = make_uint2(0u, key(0, 0));
     uint32_t top = 0;
 #pragma unroll
     for (int t = 0; t < R; ++t) {
@@ -215,7 +221,7 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
         if (b < (uint32_t)open && k < K) {
             const uint32_t at = atomicAdd(&hist[b], 1u);
             if (at < (uint32_t)len) {
-                items[at] = make_uint2(__float_as_uint(v[t]), ~(uint32_t)k);
+                items[at] = make_uint2(__float_as_uint(v[t]), key((uint32_t)k, at + 1));
                 listed = true;
             }
         }
@@ -266,20 +272,20 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
 
 // ---- search ------------------------------------------------------------------------------------------------
 // The two running extremes of an output are kept as doubles whose high word is the fp32 product and whose low
-// word is ~k: for products of one sign, doubles order by (product, lower k first), so v_max_f64 / v_min_f64 keep
-// value AND first index in one instruction, in any order of k.  (A product of the wrong sign never decides: an
+// word is the entry's key: for products of one sign, doubles order by (product, lower k first), so v_max_f64 /
+// v_min_f64 keep value AND first index in one instruction, in any order of k.  (A product of the wrong sign never decides: an
 // output is finished by its bound only with a positive maximum and a negative minimum.  fp32 infinities read as
 // finite doubles; NaN products cannot occur in a listed row with finite tile values.)
-__device__ __forceinline__ double keyed(float product, uint32_t not_k)
+__device__ __forceinline__ double keyed(float product, uint32_t key)
 {
     typedef uint32_t pair_t __attribute__((ext_vector_type(2)));
     pair_t v;
-    v.x = not_k;
+    v.x = key;
     v.y = __float_as_uint(product);
     return __builtin_bit_cast(double, v);
 }
 __device__ __forceinline__ float product_of(double d) { return __uint_as_float((uint32_t)(__builtin_bit_cast(uint64_t, d) >> 32)); }
-__device__ __forceinline__ int index_of(double d) { return (int)~(uint32_t)__builtin_bit_cast(uint64_t, d); }
+__device__ __forceinline__ uint32_t key_of(double d) { return (uint32_t)__builtin_bit_cast(uint64_t, d); }
 // (the builtins would canonicalise their operands first: one more instruction each)
 __device__ __forceinline__ void max64(double &a, double b) { asm("v_max_f64 %0, %0, %1" : "+v"(a) : "v"(b)); }
 __device__ __forceinline__ void min64(double &a, double b) { asm("v_min_f64 %0, %0, %1" : "+v"(a) : "v"(b)); }
@@ -308,13 +314,13 @@ template <>
 struct Extremes<true> {
     typedef double value;
     double mx[4], mn[4];
-    static __device__ __forceinline__ value low() { return keyed(-__builtin_inff(), ~0u); }
-    static __device__ __forceinline__ value high() { return keyed(__builtin_inff(), ~0u); }
-    static __device__ __forceinline__ value make(float product, int k) { return keyed(product, ~(uint32_t)k); }
+    static __device__ __forceinline__ value low() { return keyed(-__builtin_inff(), key(0, 0)); }
+    static __device__ __forceinline__ value high() { return keyed(__builtin_inff(), key(0, 0)); }
+    static __device__ __forceinline__ value make(float product, int k) { return keyed(product, key((uint32_t)k, 0)); }
     static __device__ __forceinline__ float product(value v) { return product_of(v); }
-    static __device__ __forceinline__ void both(value &a, value &b, float product, uint32_t not_k)
+    static __device__ __forceinline__ void both(value &a, value &b, float product, uint32_t key)
     {
-        const double d = keyed(product, not_k);
+        const double d = keyed(product, key);
         max64(a, d);
         min64(b, d);
     }
@@ -323,9 +329,9 @@ struct Extremes<true> {
         max64(a, shfl_xor64(a, s));
         min64(b, shfl_xor64(b, s));
     }
-    // one pair of list entries against 4 tile values each.  Written out because the compiler copies ~k into the low
+    // one pair of list entries against 4 tile values each.  Written out because the compiler copies the key into the low
     // word of every key: here two register pairs hold it for the four products of an entry.
-    __device__ __forceinline__ void entry(float x, uint32_t nk, const float4 &w)
+    __device__ __forceinline__ void entry(float x, uint32_t key, const float4 &w)
     {
         asm("v_mov_b32 v120, %9\n\tv_mov_b32 v122, %9\n\t"
             "v_mul_f32 v121, %8, %10\n\tv_mul_f32 v123, %8, %11\n\t"
@@ -336,7 +342,7 @@ struct Extremes<true> {
             "v_max_f64 %2, %2, v[120:121]\n\tv_min_f64 %6, %6, v[120:121]\n\t"
             "v_max_f64 %3, %3, v[122:123]\n\tv_min_f64 %7, %7, v[122:123]"
             : "+&v"(mx[0]), "+&v"(mx[1]), "+&v"(mx[2]), "+&v"(mx[3]), "+&v"(mn[0]), "+&v"(mn[1]), "+&v"(mn[2]), "+&v"(mn[3])
-            : "v"(x), "v"(nk), "v"(w.x), "v"(w.y), "v"(w.z), "v"(w.w)
+            : "v"(x), "v"(key), "v"(w.x), "v"(w.y), "v"(w.z), "v"(w.w)
             : "v120", "v121", "v122", "v123");
     }
     __device__ __forceinline__ void entries(const uint4 &it, const float4 &w0, const float4 &w1)
@@ -380,7 +386,7 @@ struct Extremes<false> {
 // One output by the whole wave: first the rest of its list, 64 entries at a time, then (the list is not enough,
 // or the row or the tile column holds what no bound covers: NaN, infinity, a zero extreme) every k, in the exact
 // terms of the ascending scan with ordered strict compares.
-//   column: the output's column of the tile; at: chunks already searched; bmax: bound on the tile column
+//   column: the output's column of the tile, by 65535 - k; at: chunks already searched; bmax: bound on the tile column
 template <int TB, class E>
 __device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int row, const float *column, int at, int chunks,
                                            float bmax, int lane, typename E::value &mx, typename E::value &mn)
@@ -391,7 +397,7 @@ __device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int r
         const float u = p.bound[(int64_t)next * p.rows_pad + row] * bmax;
         if (e < chunks * CHUNK) {
             const uint2 it = reinterpret_cast<const uint2 *>(p.lists + (int64_t)(e >> 1) * p.rows_pad + row)[e & 1];
-            E::both(mx, mn, __uint_as_float(it.x) * column[~it.y * TB], it.y);
+            E::both(mx, mn, __uint_as_float(it.x) * column[(int)(it.y >> 16) * TB], it.y);
         }
 #pragma unroll
         for (int s = 32; s > 0; s >>= 1) E::merge(mx, mn, s);
@@ -411,7 +417,7 @@ __device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int r
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int past = k0 + i * 64 + lane, k = past < K ? past : K - 1;     // past the end the last k again
-            const float q = v[i] * column[k * TB];
+            const float q = v[i] * column[(65535 - k) * TB];
             if (q > hi) { hi = q; ih = k; }
             if (q < lo) { lo = q; il = k; }
         }
@@ -428,13 +434,14 @@ __device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int r
     mn = E::make(lo, il == INT32_MAX ? 0 : il);
 }
 
-// A workgroup holds a tile of TB rows of the other operand in LDS, whole rows, as [k][TB]; a lane owns one
+// A workgroup holds a tile of TB rows of the other operand in LDS, whole rows, as [K - 1 - k][TB] (a key's upper half
+// is then the address but for a constant); a lane owns one
 // listed row x 4 consecutive tile rows, and TB / 4 neighbouring lanes share a listed row, so that an entry costs
 // each lane one 16-byte LDS read for 4 products and the lanes of a row read TB * 4 contiguous bytes.  Waves take
 // blocks of 64 * 4 / TB listed rows in turn and need no barrier after the tile is loaded.  A wave looks at its
 // lists chunk by chunk until all but FEW of its 256 outputs are finished by their bound, and then finishes those
 // one by one with all its lanes (FEW = 0, 1, 2, 4: 75 / 72 / 72 / 73 us at 256 x 4096 x 4096, 608 / 593 / 593 / 602 us at
-// 16384 x 4096 -> 1024).  Bound: v_max_f64 / v_min_f64, ~13 of the ~17 cycles per product and SIMD; the random 16-byte
+// 16384 x 4096 -> 1024, while the selected operands still came from the row).  Bound: v_max_f64 / v_min_f64, ~13 of the ~17 cycles per product and SIMD; the random 16-byte
 // LDS reads take half of that.  (9.9 T products/s in a loop of its own against 14.3 T with fp32 extremes and no
 // indices.)
 constexpr int FEW = 2;
@@ -445,7 +452,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
     typedef Extremes<ARGS> E;
     constexpr int Q = TB / 4;               // lanes per listed row
     constexpr int RW = 64 / Q;              // listed rows per wave
-    extern __shared__ float tile[];         // [K][TB]
+    extern __shared__ float tile[];         // [K][TB], k descending
     __shared__ float tops[TB];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -485,7 +492,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         for (int k = wave / Q * 64 + lane; k < K; k += STEP) {
             float4 v;
             v.x = src[0][(uint32_t)k]; v.y = src[1][(uint32_t)k]; v.z = src[2][(uint32_t)k]; v.w = src[3][(uint32_t)k];
-            *reinterpret_cast<float4 *>(&tile[k * TB + my_quad * 4]) = v;
+            *reinterpret_cast<float4 *>(&tile[(K - 1 - k) * TB + my_quad * 4]) = v;
             see(0, v.x); see(1, v.y); see(2, v.z); see(3, v.w);
         }
 #pragma unroll
@@ -502,7 +509,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             const float *src = b.p + k * b.k_stride;
             float4 v;
             v.x = src[r[0]]; v.y = src[r[1]]; v.z = src[r[2]]; v.w = src[r[3]];
-            *reinterpret_cast<float4 *>(&tile[k * TB + my_quad * 4]) = v;
+            *reinterpret_cast<float4 *>(&tile[(K - 1 - k) * TB + my_quad * 4]) = v;
             see(0, v.x); see(1, v.y); see(2, v.z); see(3, v.w);
         }
 #pragma unroll
@@ -529,8 +536,12 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         const float t = tops[q * 4 + j];
         bmax[j] = t == 0.0f ? -1.0f : t < __builtin_inff() ? t : __builtin_nanf("");
     }
-    const char *mine = reinterpret_cast<const char *>(tile) + q * 16;
+    const float *by_key = tile + (K - 65536) * TB;      // element (65535 - k) * TB + row
+    const char *mine = reinterpret_cast<const char *>(by_key) + q * 16;
     const int64_t pair_bytes = (int64_t)p.rows_pad * 16, bound_bytes = (int64_t)p.rows_pad * 4;
+
+    const bool whole = b0 + q * 4 + 3 < b.rows && (c.M & 3) == 0;
+    const uint32_t lane_off = lists_x ? (uint32_t)(lane / Q) * (uint32_t)c.M + q * 4 : q * 4 * (uint32_t)c.M + lane / Q;
 
     const int blocks = (a.rows + RW - 1) / RW;
     const int per_split = (blocks + splits - 1) / splits;
@@ -560,8 +571,8 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             asm volatile("" ::: "memory");      // the loads stay ahead of the arithmetic
 #pragma unroll
             for (int i = 0; i < CHUNK / 2; ++i) {
-                const float4 w0 = *reinterpret_cast<const float4 *>(mine + ~cur[i].y * (TB * 4));
-                const float4 w1 = *reinterpret_cast<const float4 *>(mine + ~cur[i].w * (TB * 4));
+                const float4 w0 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].y >> 16) * (TB * 4));
+                const float4 w1 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].w >> 16) * (TB * 4));
                 e.entries(cur[i], w0, w1);
             }
             ++ch;
@@ -589,7 +600,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             typename E::value fx = lane_value(j == 0 ? e.mx[0] : j == 1 ? e.mx[1] : j == 2 ? e.mx[2] : e.mx[3], l);
             typename E::value fn = lane_value(j == 0 ? e.mn[0] : j == 1 ? e.mn[1] : j == 2 ? e.mn[2] : e.mn[3], l);
             const float bm = lane_value(j == 0 ? bmax[0] : j == 1 ? bmax[1] : j == 2 ? bmax[2] : bmax[3], l);
-            finish_one<TB, E>(p, a, __builtin_amdgcn_readlane(row, l), tile + (l % Q) * 4 + j, ch, chunks, bm, lane, fx, fn);
+            finish_one<TB, E>(p, a, __builtin_amdgcn_readlane(row, l), by_key + (l % Q) * 4 + j, ch, chunks, bm, lane, fx, fn);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (i == j) {
@@ -605,47 +616,55 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if ((u0 == -1.0f) != (bmax[j] == -1.0f) && u0 == u0 && bmax[j] == bmax[j]) {
-                    const float z = *a.at(row, 0) * tile[q * 4 + j];
+                    const float z = *a.at(row, 0) * tile[(K - 1) * TB + q * 4 + j];
                     e.mx[j] = e.mn[j] = E::make(z, 0);
                 }
                 sum[j] = E::product(e.mx[j]) + E::product(e.mn[j]);
                 const int m = lists_x ? b0 + q * 4 + j : arow;
                 if (c.bias && m < (int)c.M) sum[j] = sum[j] + c.bias[m];
             }
+            // uniform base of the block + 32-bit offset of the lane
+            const int64_t base = lists_x ? (int64_t)blk * RW * c.M + b0 : (int64_t)b0 * c.M + blk * RW;
             auto put = [&](float *dst, const float (&v)[4]) {
+                float *to = dst + base;
                 if (lists_x) {
-                    const int64_t o = (int64_t)arow * c.M + b0 + q * 4;
-                    if (b0 + q * 4 + 3 < b.rows && (c.M & 3) == 0 && ((uintptr_t)dst & 15) == 0) {
-                        *reinterpret_cast<float4 *>(dst + o) = make_float4(v[0], v[1], v[2], v[3]);
+                    if (whole && ((uintptr_t)dst & 15) == 0) {
+                        *reinterpret_cast<float4 *>(to + lane_off) = make_float4(v[0], v[1], v[2], v[3]);
                     } else {
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
-                            if (b0 + q * 4 + j < b.rows) dst[o + j] = v[j];
+                            if (b0 + q * 4 + j < b.rows) to[lane_off + j] = v[j];
                     }
                 } else {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        if (b0 + q * 4 + j < b.rows) dst[(int64_t)(b0 + q * 4 + j) * c.M + arow] = v[j];
+                        if (b0 + q * 4 + j < b.rows) to[lane_off + j * (uint32_t)c.M] = v[j];
                 }
             };
             if constexpr (ARGS) {
 #pragma unroll
                 for (int side2 = 0; side2 < 2; ++side2) {
-                    int k[4];
+                    uint32_t kk[4];
                     float f[4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
-                        k[j] = index_of(side2 ? e.mn[j] : e.mx[j]);
-                        f[j] = __int_as_float(k[j]);
+                        kk[j] = key_of(side2 ? e.mn[j] : e.mx[j]);
+                        f[j] = __int_as_float(index_in(kk[j]));
                     }
                     put(reinterpret_cast<float *>(side2 ? c.argmin : c.argmax), f);
                     if (c.wsel) {
-                        // the selected operands, of the listed row and of the tile
+                        // the selected operands, of the tile and of the listed row: from the list, which this
+                        // XCD's L2 still holds, rather than from anywhere in the row (16384 x 4096 -> 1024: 593 ->
+                        // 405 us, 12608 x 3072 -> 768: 345 -> 235 us)
                         float sa[4], sb[4];
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
-                            sa[j] = *a.at(row, k[j]);
-                            sb[j] = tile[k[j] * TB + q * 4 + j];
+                            const int place = place_in(kk[j]);
+                            const char *at = reinterpret_cast<const char *>(p.lists) + (int64_t)(place >> 1) * pair_bytes;
+                            const float *from = reinterpret_cast<const float *>(at + list_off + (place & 1) * 8);
+                            if (place < 0) from = a.at(row, index_in(kk[j]));
+                            sa[j] = *from;
+                            sb[j] = by_key[(int)(kk[j] >> 16) * TB + q * 4 + j];
                         }
                         put(c.wsel + side2 * plane, lists_x ? sb : sa);
                         put(c.xsel + side2 * plane, lists_x ? sa : sb);
@@ -676,7 +695,7 @@ static int list_cap(int64_t K)
 
 bool applies(int64_t N, int64_t K, int64_t M)
 {
-    if (tile_rows(K) == 0 || N * M * K <= 0) return false;
+    if (tile_rows(K) == 0 || N * M * K <= 0 || M > (1 << 24)) return false;
     const int choice = option(MAM_OPT_FORWARD_TILING);
     if (choice == MAM_FORWARD_TILING_LISTS) return true;
     return choice == MAM_FORWARD_TILING_AUTO && K >= 128 && N >= 32 && M >= 32 && N * M >= MIN_PRODUCTS / K;
