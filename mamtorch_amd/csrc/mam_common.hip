@@ -100,7 +100,7 @@ int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t co
     if (gy > 65535 || gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "matrix too large for the transpose grid");
     const int vec = (ld % 4 == 0) && ((uintptr_t)src % 16 == 0) && ((uintptr_t)dst % 16 == 0);
     hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream, src, ld, dst,
-                       (int)rows, (int)cols, vec, guard ? *guard : ordered::Guard{nullptr, 0});
+                       (int)rows, (int)cols, vec, guard ? *guard : ordered::Guard{nullptr});
     return check_launch("transpose_kernel");
 }
 

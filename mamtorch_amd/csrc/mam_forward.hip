@@ -1304,7 +1304,7 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     }
     p.splits = (int)ceil_div(K, p.k_per_split);
     p.part = nullptr;
-    p.guard = ordered::Guard{nullptr, 0};
+    p.guard = ordered::Guard{nullptr};
     plan.need = p.splits > 1 ? (size_t)p.splits * (args ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float) : 0;
     // the fused merge keeps one ticket per tile behind the partials
     plan.tickets_at = plan.need;
@@ -1405,7 +1405,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     }
     // Large calls by magnitude-ordered lists, where the workspace has room for them; the kernels below then run
     // only if the data turns out not to suit the lists.
-    if (range_len == 0 && !static_scratch && ordered::applies(N, K, M)) {
+    if (range_len == 0 && !static_scratch && ordered::applies(N, K, M) && (operand_layout == MAM_W_MK || ldw < (1 << 22))) {
         const size_t at = (wt_bytes + need + 255) / 256 * 256;
         if (avail >= at + ordered::workspace_bytes(N, K, M) && (uintptr_t)workspace % 16 == 0) {
             const ordered::Call call = {x, ldx, w, ldw, operand_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M};

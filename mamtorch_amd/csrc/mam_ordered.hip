@@ -7,20 +7,28 @@
 // output on average and 2.1 % decide 99 % of them; with normal weights 10 %.  The roles may be swapped: lists of
 // the rows of w, bounded by max|x|.  Results are those of the scan over every k, bit for bit.
 //
-// Four launches, all decisions on the device:
-//   sample_kernel  64 outputs computed in full: how long would their lists have to be, on either side?  Every
-//                  later kernel of the call reads these 64 pairs and takes the same decision from them: lists of
-//                  x, lists of w, or (when products of a call do not fall off that way: constant magnitudes,
-//                  all-positive products) neither, and then the dense kernels run instead.
-//   build_kernel   a workgroup per listed row: counting sort of the leading entries by magnitude (512 buckets over 4
-//                  octaves), written chunk by chunk with the bound U of what follows each chunk.
-//   forward_kernel the search itself (below).
-//   dense kernels  exit at once unless the decision was "neither".
+// With normal weights as well the largest |w| is far out and one list gets long (10 % on average at K = 4096).  Then
+// the leading few percent of the OTHER operand's entries are taken first, for every output; what is left of that
+// operand is bounded by its next entry instead of by its largest, and the two short lists together replace the long
+// one (an entry in both is met twice, which changes nothing).  K = 768, both normal: 36 % -> 13 % of the products for
+// a wave's slowest output, K = 4096: 23 % -> 5.5 %.
 //
-// Measured against the dense tilings (forward call, hand-over arrays written): 207 -> 66 us at 256 x 4096 x 4096,
-// 1.70 -> 0.61 ms and 1.47 -> 0.24 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.82 ms (values only) and 3.13 -> 0.40 ms
-// at 16384 x 4096 -> 4096 / 1024.  A wave's search ends with the slowest of its 256 outputs: 92 entries at K = 4096
-// where the mean output needs 28.
+// Four launches, all decisions on the device:
+//   sample_kernel  64 outputs computed in full: how long would their lists have to be, on either side and with any
+//                  of LEADS leading shares of the other side?
+//   build_kernel   first the decision (large calls: decide_kernel): the cheapest of these, or (when products do not
+//                  fall off that way: constant magnitudes, all-positive products) none, and then the dense kernels run
+//                  instead.  A workgroup per listed row: counting sort of the leading entries by magnitude (512 buckets over 4 octaves),
+//                  written chunk by chunk with the bound U of what follows each chunk; and, for a leading share, the
+//                  searched operand transposed.
+//   forward_kernel the search itself (below).
+//   dense kernels  exit at once unless the decision was "none".
+//
+// Measured against the dense tilings (forward call, hand-over arrays written).  Uniform weights or inputs, one-sided:
+// 207 -> 67 us at 256 x 4096 x 4096, 1.70 -> 0.63 ms and 1.48 -> 0.25 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.84 ms
+// (values only) and 3.13 -> 0.42 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.17 ms
+// at 12608 x 768 -> 3072, 3.13 -> 1.09 ms at 16384 x 4096 -> 1024, 0.84 -> 0.40 ms at 4096 x 2048 x 2048.  A wave's search
+// ends with the slowest of its 256 outputs: 92 entries at K = 4096 where the mean output needs 28.
 #include "mam_ordered.h"
 
 namespace mam {
@@ -30,24 +38,42 @@ constexpr int BUCKETS = 512;          // 128 per octave below the row's largest 
 constexpr int BUCKET_SHIFT = 16;
 constexpr int BUILD_NT = 256;         // threads of the build, per listed row
 constexpr int BUILD_MAX_K = 40 * BUILD_NT;
-constexpr int BUILD_MAX_CHUNKS = BUILD_MAX_K * 3 / 8 / CHUNK + 16;
 constexpr int NT = 1024;              // threads of the forward
 constexpr int MAX_TILE_BYTES = 152 * 1024;
+// ... and from which two-sided searches are considered (a launch more, 4.5 us when it is not taken)
+constexpr int64_t MIN_TWO_SIDED = 1ll << 33;
+constexpr int LEAD_CAP = 96;          // leading entries kept per tile row (LDS)
 // N * K * M from which a call takes the lists: sampling, lists and the idle dense launches cost ~35 us, which a
 // call that then goes to the dense tilings (200 us for 2^32 products) pays as well
 constexpr int64_t MIN_PRODUCTS = 1ll << 32;
 constexpr uint32_t INF_BITS = 0x7f800000u;
 
+constexpr int CHUNK = 8;         // list entries between two tests of the bound
+constexpr int BUILD_MAX_CHUNKS = (BUILD_MAX_K / 4 + 64) / CHUNK + 1;
+constexpr int SAMPLES = 64;      // sampled outputs of a call, one per lane of a deciding wave
+constexpr int LEADS = 9;         // leading shares tried
+constexpr int OPTIONS = 2 * LEADS;
+
 struct Params {
     Call call;
-    const Sample *samples;
-    uint4 *lists;          // [entry pair][listed row]: (value, key, value, key)
-    float *bound;          // [chunk][listed row]: bound on the magnitudes from this chunk on
-    int limit;             // longest list a sample may ask for
-    int cap;               // entries a list can hold (a multiple of CHUNK)
-    int rows_pad;          // listed rows, padded, of the longer operand
-    int splits_x, splits_w;   // row ranges per tile when x (w) is listed
+    int *samples;             // [OPTIONS][SAMPLES]: entries of the searched list a sampled output needs
+    Decision *decision;
+    uint4 *lists_x, *lists_w; // [entry pair][row]: (value, key, value, key)
+    float *bound_x, *bound_w; // [chunk][row]: bound on the magnitudes from this chunk on
+    float *turned;            // [K][turned_ld]: the searched operand transposed (two-sided searches)
+    int turned_ld;            // 0: no room for it, one-sided searches only
+    int cap;                  // entries a list can hold (a multiple of CHUNK)
+    int pad_x, pad_w;         // rows of the list arrays
+    int cus;                  // compute units
 };
+
+// Leading shares in 1/1024 of K.
+__device__ const int kLeadShare[LEADS] = {0, 8, 16, 24, 32, 48, 64, 92, 128};
+__device__ __forceinline__ int lead_entries(int option, int K)
+{
+    const int lead = (int)((int64_t)kLeadShare[option % LEADS] * K / 1024 / CHUNK) * CHUNK;
+    return lead < LEAD_CAP ? lead : LEAD_CAP;
+}
 
 // A list entry's key: (65535 - k) in the upper half, so that the lower k is the larger key, and its place in the
 // list + 1 in the lower half (0: not from a list), from which the listed value is found again.
@@ -68,21 +94,70 @@ __device__ __forceinline__ Rows w_rows(const Call &c)
     return {c.w, c.w_layout == MAM_W_MK ? c.ldw : 1, c.w_layout == MAM_W_MK ? 1 : c.ldw, (int)c.M};
 }
 
-// entries written per list, from the longest sampled need: twice that and 64 more, so that hardly any of the
-// outputs that are finished one by one need more than their list (the full scan of an output costs ~20 us, 64
-// entries more of its list 1 us)
-__device__ __forceinline__ int list_length(const Params &p, int longest)
+__device__ __forceinline__ int wave_sum(int v)
 {
-    const int want = (longest * 2 + 64 + CHUNK - 1) / CHUNK * CHUNK;
-    return want < p.cap ? want : p.cap;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) v += __shfl_xor(v, s);
+    return v;
+}
+__device__ __forceinline__ int wave_max(int v)
+{
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) {
+        const int o = __shfl_xor(v, s);
+        v = o > v ? o : v;
+    }
+    return v;
+}
+
+// Exclusive prefix over hist[BUCKETS] in LDS, in place, by BUILD_NT threads; the number of buckets that start below
+// `len` is returned.  part: one word per wave.
+__device__ __forceinline__ uint32_t prefix_buckets(uint32_t *hist, uint32_t *part, uint32_t len)
+{
+    constexpr int BPT = BUCKETS / BUILD_NT;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    uint32_t own[BPT], sum = 0;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+        own[j] = hist[tid * BPT + j];
+        sum += own[j];
+    }
+    uint32_t incl = sum;
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1) {
+        const uint32_t o = __shfl_up(incl, s);
+        if (lane >= s) incl += o;
+    }
+    if (lane == 63) part[wave] = incl;
+    __syncthreads();
+    uint32_t run = incl - sum;
+#pragma unroll
+    for (int i = 0; i < BUILD_NT / 64; ++i) run += i < wave ? part[i] : 0u;
+    int open = 0;
+#pragma unroll
+    for (int j = 0; j < BPT; ++j) {
+        hist[tid * BPT + j] = run;
+        open += run < len;
+        run += own[j];
+    }
+    open = wave_sum(open);
+    __syncthreads();
+    if (lane == 0) part[wave] = (uint32_t)open;
+    __syncthreads();
+    open = 0;
+#pragma unroll
+    for (int i = 0; i < BUILD_NT / 64; ++i) open += (int)part[i];
+    return (uint32_t)open;
 }
 
 // ---- sampling ----------------------------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void sample_kernel(const Params p, Sample *out)
+__global__ __launch_bounds__(BUILD_NT) void sample_kernel(const Params p)
 {
-    __shared__ float red[4][4];
-    __shared__ int cnt[4][2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int WAVES = BUILD_NT / 64;
+    __shared__ uint32_t hist[2][BUCKETS];
+    __shared__ uint32_t part[WAVES];
+    __shared__ float red[WAVES][4];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const Call &c = p.call;
     const int K = (int)c.K;
     const uint32_t i = blockIdx.x;
@@ -91,7 +166,7 @@ __global__ __launch_bounds__(256) void sample_kernel(const Params p, Sample *out
     const Rows xr = x_rows(c), wr = w_rows(c);
     float hi = -__builtin_inff(), lo = __builtin_inff(), ax = 0.0f, aw = 0.0f;
 #pragma unroll 4
-    for (int k = threadIdx.x; k < K; k += 256) {
+    for (int k = tid; k < K; k += BUILD_NT) {
         const float a = *xr.at(n, k), b = *wr.at(m, k), q = a * b;
         hi = __builtin_fmaxf(hi, q);
         lo = __builtin_fminf(lo, q);
@@ -106,56 +181,166 @@ __global__ __launch_bounds__(256) void sample_kernel(const Params p, Sample *out
         aw = __builtin_fmaxf(aw, __shfl_xor(aw, s));
     }
     if (lane == 0) { red[wave][0] = hi; red[wave][1] = lo; red[wave][2] = ax; red[wave][3] = aw; }
+    for (int j = tid; j < 2 * BUCKETS; j += BUILD_NT) (&hist[0][0])[j] = 0;
     __syncthreads();
-    hi = __builtin_fmaxf(__builtin_fmaxf(red[0][0], red[1][0]), __builtin_fmaxf(red[2][0], red[3][0]));
-    lo = __builtin_fminf(__builtin_fminf(red[0][1], red[1][1]), __builtin_fminf(red[2][1], red[3][1]));
-    ax = __builtin_fmaxf(__builtin_fmaxf(red[0][2], red[1][2]), __builtin_fmaxf(red[2][2], red[3][2]));
-    aw = __builtin_fmaxf(__builtin_fmaxf(red[0][3], red[1][3]), __builtin_fmaxf(red[2][3], red[3][3]));
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) {
+        hi = __builtin_fmaxf(hi, red[v][0]);
+        lo = __builtin_fminf(lo, red[v][1]);
+        ax = __builtin_fmaxf(ax, red[v][2]);
+        aw = __builtin_fmaxf(aw, red[v][3]);
+    }
     const float reach = __builtin_fminf(hi, -lo);      // a bound below this ends both searches
-    int nx = 0, nw = 0;
+    if (p.turned_ld == 0) {
+        // one-sided searches only: options 0 and LEADS
+        __shared__ int counts[WAVES][2];
+        int nx = 0, nw = 0;
 #pragma unroll 4
-    for (int k = threadIdx.x; k < K; k += 256) {
-        nx += !(__builtin_fabsf(*xr.at(n, k)) * aw < reach);
-        nw += !(__builtin_fabsf(*wr.at(m, k)) * ax < reach);
+        for (int k = tid; k < K; k += BUILD_NT) {
+            nx += !(__builtin_fabsf(*xr.at(n, k)) * aw < reach);
+            nw += !(__builtin_fabsf(*wr.at(m, k)) * ax < reach);
+        }
+        nx = wave_sum(nx);
+        nw = wave_sum(nw);
+        if (lane == 0) { counts[wave][0] = nx; counts[wave][1] = nw; }
+        __syncthreads();
+        if (tid < 2) {
+            int sum = 0;
+            for (int v = 0; v < WAVES; ++v) sum += counts[v][tid];
+            p.samples[tid * LEADS * SAMPLES + blockIdx.x] = sum;
+        }
+        return;
     }
-    nx = wave_sum(nx);
-    nw = wave_sum(nw);
-    if (lane == 0) { cnt[wave][0] = nx; cnt[wave][1] = nw; }
+    const uint32_t top_x = __float_as_uint(ax), top_w = __float_as_uint(aw);
+#pragma unroll 4
+    for (int k = tid; k < K; k += BUILD_NT) {
+        const uint32_t bx = (top_x - (__float_as_uint(*xr.at(n, k)) & 0x7fffffffu)) >> BUCKET_SHIFT;
+        const uint32_t bw = (top_w - (__float_as_uint(*wr.at(m, k)) & 0x7fffffffu)) >> BUCKET_SHIFT;
+        if (bx < (uint32_t)BUCKETS) atomicAdd(&hist[0][bx], 1u);
+        if (bw < (uint32_t)BUCKETS) atomicAdd(&hist[1][bw], 1u);
+    }
     __syncthreads();
-    if (threadIdx.x == 0) {
-        out[i].need_x = cnt[0][0] + cnt[1][0] + cnt[2][0] + cnt[3][0];
-        out[i].need_w = cnt[0][1] + cnt[1][1] + cnt[2][1] + cnt[3][1];
+    prefix_buckets(hist[0], part, 0);
+    __syncthreads();
+    prefix_buckets(hist[1], part, 0);
+    if (tid >= OPTIONS) return;
+    // an option: LEADS shares of w ahead of a search of x, then LEADS shares of x ahead of a search of w
+    const bool search_x = tid < LEADS;
+    const uint32_t *led = hist[search_x ? 1 : 0], *searched = hist[search_x ? 0 : 1];
+    const uint32_t top_led = search_x ? top_w : top_x, top_searched = search_x ? top_x : top_w;
+    // what is left of the led operand: at most the upper edge of the last bucket that starts inside the share
+    const uint32_t lead = (uint32_t)lead_entries(tid, K);
+    int b = 0;
+    for (int step = BUCKETS / 2; step > 0; step >>= 1)
+        if (led[b + step] <= lead) b += step;
+    const float left = __uint_as_float(top_led - ((uint32_t)b << BUCKET_SHIFT));
+    int need = K;
+    if (reach > 0.0f && left > 0.0f) {
+        const uint32_t from = __float_as_uint(reach / left);
+        if (from > top_searched) {
+            need = 0;
+        } else {
+            const uint32_t d = ((top_searched - from) >> BUCKET_SHIFT) + 1;      // everything down to this bucket
+            if (d < (uint32_t)BUCKETS) need = (int)searched[d];
+        }
     }
+    p.samples[tid * SAMPLES + blockIdx.x] = need;
+}
+
+// The largest t that at least `rank` of the 64 lanes' values reach.
+__device__ __forceinline__ int nth_largest(int v, int rank)
+{
+    int t = 0;
+    for (int bit = 1 << 15; bit > 0; bit >>= 1)
+        if (__popcll(__ballot(v >= (t | bit))) >= rank) t |= bit;
+    return t;
+}
+
+// The cheapest option, by all waves of a workgroup.  In units of one product of a dense kernel per output (12608 x 768 x
+// 3072: 2.25 us): a searched product costs 3.5, a leading one 6, a wave's slowest output needs ~1.3 times what 95 % of
+// the samples need; the launches, outputs and lists cost 0.15 K, a leading share passes over both operands.  The dense
+// kernels cost K.
+template <int WAVES>
+__device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTIONS], int (&long_s)[OPTIONS])
+{
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const float K = (float)p.call.K;
+    const int step = p.turned_ld > 0 ? 1 : LEADS;         // one-sided searches only: options 0 and LEADS
+    for (int o = wave * step; o < OPTIONS; o += WAVES * step) {
+        const bool search_x = o < LEADS, two_sided = o % LEADS != 0;
+        const int lead = lead_entries(o, (int)p.call.K);
+        // the rows of a (K, M) weight are columns in memory: they are not listed
+        const bool possible = (!two_sided || lead > 0) && (p.call.w_layout == MAM_W_MK || (search_x && !two_sided));
+        const int v = p.samples[o * SAMPLES + lane];
+        const float tiled = (float)(search_x ? p.call.M : p.call.N), listed = (float)(search_x ? p.call.N : p.call.M);
+        float cost = 0.15f * K + 3.5f * 1.3f * (float)nth_largest(v, 4);
+        if (two_sided) cost += 6.0f * (float)lead + K * (36.0f / tiled + 18.0f / listed);
+        const int longest = nth_largest(v, 2);
+        if (lane == 0) {
+            cost_s[o] = possible ? cost : 1e30f;
+            long_s[o] = longest;
+        }
+    }
+    __syncthreads();
+    int best = 0;
+    for (int o = step; o < OPTIONS; o += step)
+        if (cost_s[o] < cost_s[best]) best = o;
+    Decision d;
+    d.side = cost_s[best] < 0.95f * K ? (best < LEADS ? SIDE_X : SIDE_W) : SIDE_NONE;
+    d.lead = lead_entries(best, (int)p.call.K);
+    // entries written per list: twice the longest sampled need and 64 more, so that hardly any of the outputs that
+    // are finished one by one need more than their list (64 entries more of it: 1 us; the full scan: ~20 us)
+    const int want = (long_s[best] * 2 + 64 + CHUNK - 1) / CHUNK * CHUNK;
+    d.length = want < p.cap ? want : p.cap;
+    d.pad = 0;
+    return d;
+}
+
+// Two-sided searches have 18 options: decided once, in a launch of its own (4 us; the two one-sided ones are decided by
+// every workgroup of build_kernel).
+__global__ __launch_bounds__(64 * LEADS) void decide_kernel(const Params p)
+{
+    __shared__ float cost_s[OPTIONS];
+    __shared__ int long_s[OPTIONS];
+    const Decision d = decide<LEADS>(p, cost_s, long_s);
+    if (threadIdx.x == 0) *p.decision = d;
 }
 
 // ---- lists -------------------------------------------------------------------------------------------------
-// A workgroup per listed row, R elements per thread in registers.  Rows of one 64-byte piece of the list array
-// are built on one XCD.
+// 64 x 64 of `rows` transposed into dst[k][ld] through LDS.
+__device__ __forceinline__ void turn_tile(const Rows &rows, int K, float *dst, int ld, int r0, int k0, float (*t)[65])
+{
+    const int lo = threadIdx.x & 63, hi = threadIdx.x >> 6;
+#pragma unroll 8
+    for (int i = 0; i < 64; i += BUILD_NT / 64) {
+        const int r = r0 + i + hi, k = k0 + lo;
+        t[i + hi][lo] = r < rows.rows && k < K ? *rows.at(r, k) : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int i = 0; i < 64; i += BUILD_NT / 64) {
+        const int k = k0 + i + hi, r = r0 + lo;
+        if (k < K && r < rows.rows) dst[(int64_t)k * ld + r] = t[lo][i + hi];
+    }
+}
+
+// The list of one row by a workgroup, R elements per thread in registers.  `place`: entries carry their place.
 template <int R>
-__global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
+__device__ __forceinline__ void build_row(const Rows &rows, int row, int K, int len, bool place, uint4 *lists, float *bound, int pad,
+                                          uint4 *lds, uint32_t *hist, uint32_t *part, uint32_t *part2, uint32_t *chunk_top)
 {
     constexpr int WAVES = BUILD_NT / 64;
-    extern __shared__ uint4 lds[];          // [cap] (value, key) pairs
-    __shared__ uint32_t hist[BUCKETS];
-    __shared__ uint32_t part[WAVES], part2[WAVES];
-    __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
     uint2 *items = reinterpret_cast<uint2 *>(lds);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int longest;
-    const int side = decide(p.samples, p.limit, lane, longest);
-    if (side == SIDE_NONE) return;
-    const Rows rows = side == SIDE_X ? x_rows(p.call) : w_rows(p.call);
-    if ((int)blockIdx.x >= rows.rows) return;
-    const int row = xcd_remap(blockIdx.x, rows.rows);
-    const int len = list_length(p, longest), chunks = len / CHUNK;
-    const int K = (int)p.call.K;
+    const int chunks = len / CHUNK;
     const float *src = rows.at(row, 0);
-
+    const uint32_t mine = (uint32_t)tid * (uint32_t)rows.k_stride;
     float v[R];
 #pragma unroll
     for (int t = 0; t < R; ++t) {
-        const int k = t * BUILD_NT + tid;
-        v[t] = k < K ? src[k * rows.k_stride] : 0.0f;
+        const float *from = src + (int64_t)(t * BUILD_NT) * rows.k_stride;
+        v[t] = t * BUILD_NT + tid < K ? from[mine] : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < BUCKETS / BUILD_NT; ++j) hist[j * BUILD_NT + tid] = 0;
@@ -179,38 +364,7 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
         if (b < (uint32_t)BUCKETS && t * BUILD_NT + tid < K) atomicAdd(&hist[b], 1u);
     }
     __syncthreads();
-    // exclusive prefix over the buckets, BUCKETS / BUILD_NT consecutive ones per thread
-    constexpr int BPT = BUCKETS / BUILD_NT;
-    uint32_t own[BPT], sum = 0;
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-        own[j] = hist[tid * BPT + j];
-        sum += own[j];
-    }
-    uint32_t incl = sum;
-#pragma unroll
-    for (int s = 1; s < 64; s <<= 1) {
-        const uint32_t o = __shfl_up(incl, s);
-        if (lane >= s) incl += o;
-    }
-    if (lane == 63) part2[wave] = incl;
-    __syncthreads();
-    uint32_t run = incl - sum;
-#pragma unroll
-    for (int i = 0; i < WAVES - 1; ++i) run += i < wave ? part2[i] : 0u;
-    int open = 0;                 // buckets that start inside the list
-#pragma unroll
-    for (int j = 0; j < BPT; ++j) {
-        hist[tid * BPT + j] = run;
-        open += run < (uint32_t)len;
-        run += own[j];
-    }
-    open = wave_sum(open);
-    if (lane == 0) part[wave] = (uint32_t)open;
-    __syncthreads();
-    open = 0;
-#pragma unroll
-    for (int i = 0; i < WAVES; ++i) open += (int)part[i];
+    const uint32_t open = prefix_buckets(hist, part2, (uint32_t)len);     // buckets that start inside the list
     uint32_t rest = 0;            // largest magnitude that is not listed
 #pragma unroll
     for (int t = 0; t < R; ++t) {
@@ -218,17 +372,17 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
         const uint32_t b = (top - bits) >> BUCKET_SHIFT;
         const int k = t * BUILD_NT + tid;
         bool listed = false;
-        if (b < (uint32_t)open && k < K) {
+        if (b < open && k < K) {
             const uint32_t at = atomicAdd(&hist[b], 1u);
             if (at < (uint32_t)len) {
-                items[at] = make_uint2(__float_as_uint(v[t]), key((uint32_t)k, at + 1));
+                items[at] = make_uint2(__float_as_uint(v[t]), key((uint32_t)k, place ? at + 1 : 0));
                 listed = true;
             }
         }
         if (!listed) rest = bits > rest ? bits : rest;
     }
     rest = (uint32_t)wave_max((int)rest);
-    if (lane == 0) part2[wave] = rest;
+    if (lane == 0) part[wave] = rest;
     __syncthreads();
     for (int c = tid; c < chunks; c += BUILD_NT) {
         uint32_t t = 0;
@@ -239,13 +393,13 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
         }
         chunk_top[c] = t;
     }
-    for (int j = tid; j < len / 2; j += BUILD_NT) p.lists[(int64_t)j * p.rows_pad + row] = lds[j];
+    for (int j = tid; j < len / 2; j += BUILD_NT) lists[(int64_t)j * pad + row] = lds[j];
     __syncthreads();
     if (wave != 0) return;
     // bound[c] = largest magnitude from chunk c on.  A row with a NaN or an infinity gets NaN (never finished by a
     // bound), a row of zeros -1 (finished at once: see the forward).
 #pragma unroll
-    for (int i = 0; i < WAVES; ++i) rest = part2[i] > rest ? part2[i] : rest;
+    for (int i = 0; i < WAVES; ++i) rest = part[i] > rest ? part[i] : rest;
     const int per = (chunks + 1 + 63) / 64;
     uint32_t suffix = 0;
     for (int j = per - 1; j >= 0; --j) {
@@ -266,7 +420,50 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     for (int j = per - 1; j >= 0; --j) {
         const int c = lane * per + j;
         if (c < chunks) tail = chunk_top[c] > tail ? chunk_top[c] : tail;
-        if (c <= chunks) p.bound[(int64_t)c * p.rows_pad + row] = special ? instead : __uint_as_float(tail);
+        if (c <= chunks) bound[(int64_t)c * pad + row] = special ? instead : __uint_as_float(tail);
+    }
+}
+
+// One work item per workgroup: the rows of the searched operand; with a leading share also the rows of the other one
+// and the 64 x 64 tiles of the transpose.
+template <int R>
+__global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
+{
+    extern __shared__ uint4 lds[];          // [cap] (value, key) pairs
+    __shared__ uint32_t hist[BUCKETS];
+    __shared__ uint32_t part[BUILD_NT / 64], part2[BUILD_NT / 64];
+    __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
+    __shared__ float turn[64][65];
+    __shared__ float cost_s[OPTIONS];
+    __shared__ int long_s[OPTIONS];
+    Decision d;
+    if (p.turned_ld > 0) {
+        d = *p.decision;
+    } else {
+        d = decide<BUILD_NT / 64>(p, cost_s, long_s);
+        d.side = __builtin_amdgcn_readfirstlane(d.side);
+        d.length = __builtin_amdgcn_readfirstlane(d.length);
+        d.lead = 0;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *p.decision = d;       // for the kernels that follow
+    }
+    if (d.side == SIDE_NONE) return;
+    const bool sx = d.side == SIDE_X;
+    const Rows a = sx ? x_rows(p.call) : w_rows(p.call), b = sx ? w_rows(p.call) : x_rows(p.call);
+    const int K = (int)p.call.K;
+    const int row_tiles = (a.rows + 63) / 64;
+    // (an operand stored (K, rows) is its own transpose)
+    const int turns = d.lead > 0 && a.k_stride == 1 ? row_tiles * ((K + 63) / 64) : 0;
+    const int total = a.rows + (d.lead > 0 ? b.rows : 0) + turns;
+    if ((int)blockIdx.x >= total) return;
+    const int item = xcd_remap(blockIdx.x, total);
+    if (item < total - turns) {
+        const bool searched = item < a.rows, is_x = searched == sx;
+        build_row<R>(is_x ? x_rows(p.call) : w_rows(p.call), searched ? item : item - a.rows, K, searched ? d.length : d.lead, searched,
+                     is_x ? p.lists_x : p.lists_w, is_x ? p.bound_x : p.bound_w, is_x ? p.pad_x : p.pad_w, lds, hist, part, part2,
+                     chunk_top);
+    } else {
+        const int t = item - (total - turns);
+        turn_tile(a, K, p.turned, p.turned_ld, t % row_tiles * 64, t / row_tiles * 64, turn);
     }
 }
 
@@ -387,17 +584,20 @@ struct Extremes<false> {
 // or the row or the tile column holds what no bound covers: NaN, infinity, a zero extreme) every k, in the exact
 // terms of the ascending scan with ordered strict compares.
 //   column: the output's column of the tile, by 65535 - k; at: chunks already searched; bmax: bound on the tile column
-template <int TB, class E>
-__device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int row, const float *column, int at, int chunks,
+template <int STRIDE, class E>
+__device__ __forceinline__ void finish_one(const Params &p, bool sx, const Rows &a, int row, const float *column, int at, int chunks,
                                            float bmax, int lane, typename E::value &mx, typename E::value &mn)
 {
+    const uint4 *lists = sx ? p.lists_x : p.lists_w;
+    const float *bound = sx ? p.bound_x : p.bound_w;
+    const int pad = sx ? p.pad_x : p.pad_w;
     for (int ch = at; ch < chunks; ch += 64 / CHUNK) {
         const int e = ch * CHUNK + lane;
         const int next = (ch + 64 / CHUNK) < chunks ? ch + 64 / CHUNK : chunks;
-        const float u = p.bound[(int64_t)next * p.rows_pad + row] * bmax;
+        const float u = bound[(int64_t)next * pad + row] * bmax;
         if (e < chunks * CHUNK) {
-            const uint2 it = reinterpret_cast<const uint2 *>(p.lists + (int64_t)(e >> 1) * p.rows_pad + row)[e & 1];
-            E::both(mx, mn, __uint_as_float(it.x) * column[(int)(it.y >> 16) * TB], it.y);
+            const uint2 it = reinterpret_cast<const uint2 *>(lists + (int64_t)(e >> 1) * pad + row)[e & 1];
+            E::both(mx, mn, __uint_as_float(it.x) * column[(int)(it.y >> 16) * STRIDE], it.y);
         }
 #pragma unroll
         for (int s = 32; s > 0; s >>= 1) E::merge(mx, mn, s);
@@ -417,7 +617,7 @@ __device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int r
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int past = k0 + i * 64 + lane, k = past < K ? past : K - 1;     // past the end the last k again
-            const float q = v[i] * column[(65535 - k) * TB];
+            const float q = v[i] * column[(65535 - k) * STRIDE];
             if (q > hi) { hi = q; ih = k; }
             if (q < lo) { lo = q; il = k; }
         }
@@ -446,28 +646,54 @@ __device__ __forceinline__ void finish_one(const Params &p, const Rows &a, int r
 // indices.)
 constexpr int FEW = 2;
 
-template <int TB, bool ARGS>
+// Where a lane sits and how the tile lies in LDS.  One-sided: neighbouring lanes share a searched row, the tile is
+// [k][TB], so that the lanes of a row read TB * 4 contiguous bytes and write as many.  Two-sided: neighbouring lanes are
+// neighbouring searched rows, which is how the transposed operand is read contiguously; the tile is [TB / 4][k][4],
+// so that the lanes of one quad still spread over all banks.  (k descending: a key's upper half is then the address
+// but for a constant.)
+template <int TB, bool TWO>
+struct Lanes {
+    static constexpr int Q = TB / 4;               // quads of tile rows
+    static constexpr int RW = 64 / Q;              // searched rows per wave
+    static constexpr int STRIDE = TWO ? 4 : TB;    // floats from one k to the next
+    static __device__ __forceinline__ int quad(int lane) { return TWO ? lane / RW : lane % Q; }
+    static __device__ __forceinline__ int row(int lane) { return TWO ? lane % RW : lane / Q; }
+    static __device__ __forceinline__ int base(int quad, int K) { return TWO ? quad * K * 4 : quad * 4; }
+};
+
+// Row ranges per tile: three rounds of workgroups over the chip, but at least one block of rows per wave.
+template <int TB>
+__host__ __device__ __forceinline__ int splits_of(int searched, int tiles, int cus)
+{
+    const int blocks = (searched + 256 / TB - 1) / (256 / TB);
+    const int s = (3 * cus + tiles - 1) / tiles, most = (blocks + NT / 64 - 1) / (NT / 64);
+    return s < most ? s : most;
+}
+
+template <int TB, bool ARGS, bool TWO>
 __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 {
     typedef Extremes<ARGS> E;
-    constexpr int Q = TB / 4;               // lanes per listed row
-    constexpr int RW = 64 / Q;              // listed rows per wave
-    extern __shared__ float tile[];         // [K][TB], k descending
+    typedef Lanes<TB, TWO> L;
+    constexpr int Q = L::Q, RW = L::RW;
+    extern __shared__ float tile[];         // the tile; two-sided: then [TB][lead] (value, key)
     __shared__ float tops[TB];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int longest;
-    const int side = decide(p.samples, p.limit, lane, longest);
-    if (side == SIDE_NONE) return;
+    const Decision d = *p.decision;
+    if (d.side == SIDE_NONE || (d.lead > 0) != TWO) return;
     const Call &c = p.call;
-    const bool lists_x = side == SIDE_X;
+    const bool lists_x = d.side == SIDE_X;
+    const uint4 *const lists = lists_x ? p.lists_x : p.lists_w, *const lists_b = lists_x ? p.lists_w : p.lists_x;
+    const float *const bound = lists_x ? p.bound_x : p.bound_w, *const bound_b = lists_x ? p.bound_w : p.bound_x;
+    const int pad = lists_x ? p.pad_x : p.pad_w, pad_b = lists_x ? p.pad_w : p.pad_x;
     const Rows a = lists_x ? x_rows(c) : w_rows(c), b = lists_x ? w_rows(c) : x_rows(c);
     const int K = (int)c.K;
-    const int tiles = (b.rows + TB - 1) / TB, splits = lists_x ? p.splits_x : p.splits_w;
+    const int tiles = (b.rows + TB - 1) / TB, splits = splits_of<TB>(a.rows, tiles, p.cus);
     if ((int)blockIdx.x >= tiles * splits) return;
     const int logical = xcd_remap(blockIdx.x, tiles * splits);
     const int split = logical / tiles, b0 = (logical - split * tiles) * TB;
-    const int chunks = list_length(p, longest) / CHUNK;
+    const int chunks = d.length / CHUNK;
 
     // ---- tile: rows b0 .. b0 + TB - 1 (past the end: the last one again), and the largest magnitude of each ----
     // (bit patterns of magnitudes order as integers; infinities and NaN stay on top)
@@ -476,6 +702,11 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         const uint32_t bits = __float_as_uint(v) & 0x7fffffffu;
         top[i] = bits > top[i] ? bits : top[i];
     };
+    uint2 *const lead_s = reinterpret_cast<uint2 *>(tile + TB * K);
+    for (int i = threadIdx.x; TWO && i < TB * (d.lead / 2); i += NT) {
+        const int r = i % TB, pair = i / TB, row = b0 + r < b.rows ? b0 + r : b.rows - 1;
+        *reinterpret_cast<uint4 *>(&lead_s[r * d.lead + pair * 2]) = lists_b[(int64_t)pair * pad_b + row];
+    }
     if (threadIdx.x < TB) tops[threadIdx.x] = 0.0f;
     int my_quad;
     if (b.k_stride == 1) {
@@ -492,7 +723,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         for (int k = wave / Q * 64 + lane; k < K; k += STEP) {
             float4 v;
             v.x = src[0][(uint32_t)k]; v.y = src[1][(uint32_t)k]; v.z = src[2][(uint32_t)k]; v.w = src[3][(uint32_t)k];
-            *reinterpret_cast<float4 *>(&tile[(K - 1 - k) * TB + my_quad * 4]) = v;
+            *reinterpret_cast<float4 *>(&tile[L::base(my_quad, K) + (K - 1 - k) * L::STRIDE]) = v;
             see(0, v.x); see(1, v.y); see(2, v.z); see(3, v.w);
         }
 #pragma unroll
@@ -509,7 +740,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             const float *src = b.p + k * b.k_stride;
             float4 v;
             v.x = src[r[0]]; v.y = src[r[1]]; v.z = src[r[2]]; v.w = src[r[3]];
-            *reinterpret_cast<float4 *>(&tile[(K - 1 - k) * TB + my_quad * 4]) = v;
+            *reinterpret_cast<float4 *>(&tile[L::base(my_quad, K) + (K - 1 - k) * L::STRIDE]) = v;
             see(0, v.x); see(1, v.y); see(2, v.z); see(3, v.w);
         }
 #pragma unroll
@@ -529,25 +760,34 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
     // An output is finished when bound * bmax is below both extremes.  A tile row with an infinity or a NaN gets a
     // NaN for bmax (never finished that way); a zero row on one side gets -1 (finished at once: every product is a
     // zero and the first one decides), zero rows on both sides make +1 and are finished by the full scan.
-    const int q = lane % Q;
+    const int q = L::quad(lane);
     float bmax[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
+        if (TWO) {              // what the leading share leaves of the tile row (the same special values)
+            const int r = b0 + q * 4 + j < b.rows ? b0 + q * 4 + j : b.rows - 1;
+            bmax[j] = bound_b[(int64_t)(d.lead / CHUNK) * pad_b + r];
+            continue;
+        }
         const float t = tops[q * 4 + j];
         bmax[j] = t == 0.0f ? -1.0f : t < __builtin_inff() ? t : __builtin_nanf("");
     }
-    const float *by_key = tile + (K - 65536) * TB;      // element (65535 - k) * TB + row
-    const char *mine = reinterpret_cast<const char *>(by_key) + q * 16;
-    const int64_t pair_bytes = (int64_t)p.rows_pad * 16, bound_bytes = (int64_t)p.rows_pad * 4;
+    const float *by_key = tile + L::base(q, K) + (K - 65536) * L::STRIDE;      // element (65535 - k) * STRIDE + row of the quad
+    const char *mine = reinterpret_cast<const char *>(by_key);
+    const int64_t pair_bytes = (int64_t)pad * 16, bound_bytes = (int64_t)pad * 4;
 
-    const bool whole = b0 + q * 4 + 3 < b.rows && (c.M & 3) == 0;
-    const uint32_t lane_off = lists_x ? (uint32_t)(lane / Q) * (uint32_t)c.M + q * 4 : q * 4 * (uint32_t)c.M + lane / Q;
+    // Stores with x searched: a row's outputs lie along the tile rows.  Two-sided, the lanes that hold them change places
+    // first (lane r * Q + q takes over from lane q * RW + r).
+    const int sq = lane % Q, sr = lane / Q;
+    const int swap_from = (sq * RW + sr) * 4;
+    const bool whole = b0 + sq * 4 + 3 < b.rows && (c.M & 3) == 0;
+    const uint32_t lane_off = lists_x ? (uint32_t)sr * (uint32_t)c.M + sq * 4 : q * 4 * (uint32_t)c.M + L::row(lane);
 
     const int blocks = (a.rows + RW - 1) / RW;
     const int per_split = (blocks + splits - 1) / splits;
     const int last = (split + 1) * per_split < blocks ? (split + 1) * per_split : blocks;
     for (int blk = split * per_split + wave; blk < last; blk += NT / 64) {
-        const int arow = blk * RW + lane / Q;
+        const int arow = blk * RW + L::row(lane);
         const int row = arow < a.rows ? arow : a.rows - 1;
         const uint32_t list_off = (uint32_t)row * 16u, bound_off = (uint32_t)row * 4u;
         E e;
@@ -556,10 +796,50 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             e.mx[j] = E::low();
             e.mn[j] = E::high();
         }
+        // ---- the leading entries of the tile rows: (value, key) from their lists, the other factor of four
+        // consecutive tile rows x neighbouring listed rows from the transposed operand ----
+        if constexpr (TWO) {
+            const char *turned = reinterpret_cast<const char *>(a.k_stride == 1 ? p.turned : a.p);
+            const uint32_t ld4 = (uint32_t)(a.k_stride == 1 ? p.turned_ld : (int)a.k_stride) * 4u;
+            const uint32_t turned_off = (uint32_t)row * 4u + 65535u * ld4;
+            const uint2 *mine_led = lead_s + q * 4 * d.lead;
+            auto lead_rows = [&](float (&to)[8], int pair) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint4 l = *reinterpret_cast<const uint4 *>(&mine_led[j * d.lead + pair * 2]);
+                    to[2 * j] = *reinterpret_cast<const float *>(turned + (turned_off - __umul24(l.y >> 16, ld4)));
+                    to[2 * j + 1] = *reinterpret_cast<const float *>(turned + (turned_off - __umul24(l.w >> 16, ld4)));
+                }
+                asm volatile("" ::: "memory");
+            };
+            auto lead_products = [&](const float (&v)[8], int pair) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const uint4 l = *reinterpret_cast<const uint4 *>(&mine_led[j * d.lead + pair * 2]);
+                    E::both(e.mx[j], e.mn[j], v[2 * j] * __uint_as_float(l.x), l.y);
+                    E::both(e.mx[j], e.mn[j], v[2 * j + 1] * __uint_as_float(l.z), l.w);
+                }
+            };
+            // rows two pairs ahead of the products; a multiple of 4 pairs (past the end: the last pair again)
+            const int pairs = d.lead / 2;
+            float v0[8], v1[8], v2[8], v3[8];
+            lead_rows(v0, 0);
+            lead_rows(v1, 1);
+            for (int i = 0; i < pairs; i += 4) {
+                lead_rows(v2, i + 2);
+                lead_products(v0, i);
+                lead_rows(v3, i + 3);
+                lead_products(v1, i + 1);
+                lead_rows(v0, i + 4 < pairs ? i + 4 : pairs - 1);
+                lead_products(v2, i + 2);
+                lead_rows(v1, i + 5 < pairs ? i + 5 : pairs - 1);
+                lead_products(v3, i + 3);
+            }
+        }
         int ch = 0;
         uint64_t open[4];
         auto fetch = [&](uint4 (&to)[CHUNK / 2], int chunk) {
-            const char *base = reinterpret_cast<const char *>(p.lists) + (int64_t)chunk * (CHUNK / 2) * pair_bytes;
+            const char *base = reinterpret_cast<const char *>(lists) + (int64_t)chunk * (CHUNK / 2) * pair_bytes;
             asm volatile("" : "+s"(base));      // scalar base + 32-bit lane offset
 #pragma unroll
             for (int i = 0; i < CHUNK / 2; ++i) to[i] = *reinterpret_cast<const uint4 *>(base + i * pair_bytes + list_off);
@@ -567,12 +847,12 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         // true when the search is over
         auto step = [&](const uint4 (&cur)[CHUNK / 2], uint4 (&nxt)[CHUNK / 2]) {
             fetch(nxt, ch + 1 < chunks ? ch + 1 : ch);
-            const float u = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(p.bound) + (ch + 1) * bound_bytes + bound_off);
+            const float u = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(bound) + (ch + 1) * bound_bytes + bound_off);
             asm volatile("" ::: "memory");      // the loads stay ahead of the arithmetic
 #pragma unroll
             for (int i = 0; i < CHUNK / 2; ++i) {
-                const float4 w0 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].y >> 16) * (TB * 4));
-                const float4 w1 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].w >> 16) * (TB * 4));
+                const float4 w0 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].y >> 16) * (L::STRIDE * 4));
+                const float4 w1 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].w >> 16) * (L::STRIDE * 4));
                 e.entries(cur[i], w0, w1);
             }
             ++ch;
@@ -600,7 +880,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             typename E::value fx = lane_value(j == 0 ? e.mx[0] : j == 1 ? e.mx[1] : j == 2 ? e.mx[2] : e.mx[3], l);
             typename E::value fn = lane_value(j == 0 ? e.mn[0] : j == 1 ? e.mn[1] : j == 2 ? e.mn[2] : e.mn[3], l);
             const float bm = lane_value(j == 0 ? bmax[0] : j == 1 ? bmax[1] : j == 2 ? bmax[2] : bmax[3], l);
-            finish_one<TB, E>(p, a, __builtin_amdgcn_readlane(row, l), by_key + (l % Q) * 4 + j, ch, chunks, bm, lane, fx, fn);
+            finish_one<L::STRIDE, E>(p, lists_x, a, __builtin_amdgcn_readlane(row, l), tile + L::base(L::quad(l), K) + (K - 65536) * L::STRIDE + j, ch, chunks, bm, lane, fx, fn);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
                 if (i == j) {
@@ -609,14 +889,14 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                 }
         }
         // ---- outputs ----
-        if (arow < a.rows) {
-            const float u0 = p.bound[row];
+        {
+            const float u0 = bound[row];
             const int64_t plane = c.N * c.M;
             float sum[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 if ((u0 == -1.0f) != (bmax[j] == -1.0f) && u0 == u0 && bmax[j] == bmax[j]) {
-                    const float z = *a.at(row, 0) * tile[(K - 1) * TB + q * 4 + j];
+                    const float z = *a.at(row, 0) * tile[L::base(q, K) + (K - 1) * L::STRIDE + j];
                     e.mx[j] = e.mn[j] = E::make(z, 0);
                 }
                 sum[j] = E::product(e.mx[j]) + E::product(e.mn[j]);
@@ -628,14 +908,18 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             auto put = [&](float *dst, const float (&v)[4]) {
                 float *to = dst + base;
                 if (lists_x) {
-                    if (whole && ((uintptr_t)dst & 15) == 0) {
-                        *reinterpret_cast<float4 *>(to + lane_off) = make_float4(v[0], v[1], v[2], v[3]);
+                    float t[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) t[j] = TWO ? __int_as_float(__builtin_amdgcn_ds_bpermute(swap_from, __float_as_int(v[j]))) : v[j];
+                    if (blk * RW + sr >= a.rows) {
+                    } else if (whole && ((uintptr_t)dst & 15) == 0) {
+                        *reinterpret_cast<float4 *>(to + lane_off) = make_float4(t[0], t[1], t[2], t[3]);
                     } else {
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
-                            if (b0 + q * 4 + j < b.rows) to[lane_off + j] = v[j];
+                            if (b0 + sq * 4 + j < b.rows) to[lane_off + j] = t[j];
                     }
-                } else {
+                } else if (arow < a.rows) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         if (b0 + q * 4 + j < b.rows) to[lane_off + j * (uint32_t)c.M] = v[j];
@@ -660,11 +944,11 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 #pragma unroll
                         for (int j = 0; j < 4; ++j) {
                             const int place = place_in(kk[j]);
-                            const char *at = reinterpret_cast<const char *>(p.lists) + (int64_t)(place >> 1) * pair_bytes;
+                            const char *at = reinterpret_cast<const char *>(lists) + (int64_t)(place >> 1) * pair_bytes;
                             const float *from = reinterpret_cast<const float *>(at + list_off + (place & 1) * 8);
                             if (place < 0) from = a.at(row, index_in(kk[j]));
                             sa[j] = *from;
-                            sb[j] = by_key[(int)(kk[j] >> 16) * TB + q * 4 + j];
+                            sb[j] = by_key[(int)(kk[j] >> 16) * L::STRIDE + j];
                         }
                         put(c.wsel + side2 * plane, lists_x ? sb : sa);
                         put(c.xsel + side2 * plane, lists_x ? sa : sb);
@@ -687,8 +971,7 @@ static int tile_rows(int64_t K)
 
 static int list_cap(int64_t K)
 {
-    int64_t cap = K * 3 / 8;
-    if (cap < 128) cap = 128;
+    int64_t cap = K / 4 + 64;
     if (cap > K) cap = K;
     return (int)(ceil_div(cap, CHUNK) * CHUNK);
 }
@@ -701,34 +984,62 @@ bool applies(int64_t N, int64_t K, int64_t M)
     return choice == MAM_FORWARD_TILING_AUTO && K >= 128 && N >= 32 && M >= 32 && N * M >= MIN_PRODUCTS / K;
 }
 
-static int64_t rows_padded(int64_t N, int64_t M) { return ceil_div(N > M ? N : M, 64) * 64; }
-
-size_t workspace_bytes(int64_t N, int64_t K, int64_t M)
+// Offsets in the workspace.
+struct Layout { size_t lists_x, lists_w, bound_x, bound_w, turned, total; int cap, pad_x, pad_w, turned_ld; };
+static Layout layout(int64_t N, int64_t K, int64_t M)
 {
-    const size_t cap = (size_t)list_cap(K), rows = (size_t)rows_padded(N, M);
-    return 1024 + cap * 8 * rows + ceil_div((cap / CHUNK + 1) * rows * 4, 256) * 256;
+    Layout l;
+    l.cap = list_cap(K);
+    l.pad_x = (int)(ceil_div(N, 64) * 64);
+    l.pad_w = (int)(ceil_div(M, 64) * 64);
+    const size_t chunks = (size_t)l.cap / CHUNK + 1;
+    size_t at = 8192;             // decision, samples
+    auto take = [&](size_t bytes) {
+        const size_t here = at;
+        at += (bytes + 255) / 256 * 256;
+        return here;
+    };
+    l.lists_x = take((size_t)l.cap * 8 * l.pad_x);
+    l.lists_w = take((size_t)l.cap * 8 * l.pad_w);
+    l.bound_x = take(chunks * 4 * l.pad_x);
+    l.bound_w = take(chunks * 4 * l.pad_w);
+    // the transposed operand is addressed with 32-bit byte offsets, its row length in 24 bits
+    l.turned_ld = l.pad_x > l.pad_w ? l.pad_x : l.pad_w;
+    if (tile_rows(K) < 8 || (N * K * M < MIN_TWO_SIDED && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_LISTS) ||
+        (size_t)l.turned_ld * 4 >= (1u << 24) || (size_t)l.turned_ld * 4 * K >= ((size_t)1 << 32)) l.turned_ld = 0;
+    if (l.turned_ld == 0) l.turned = at;
+    else l.turned = take((size_t)l.turned_ld * 4 * K);
+    l.total = at;
+    return l;
 }
 
-template <int TB>
-static int launch_forward(const Params &p, unsigned blocks, hipStream_t st)
+size_t workspace_bytes(int64_t N, int64_t K, int64_t M) { return layout(N, K, M).total; }
+
+template <int TB, bool TWO>
+static int launch_forward(const Params &p, hipStream_t st)
 {
-    const size_t lds = (size_t)p.call.K * TB * 4;
+    const size_t lds = (size_t)p.call.K * TB * 4 + (TWO ? LEAD_CAP * TB * 8 : 0);
+    const int N = (int)p.call.N, M = (int)p.call.M;
+    const int tx = (int)ceil_div(M, TB), tw = (int)ceil_div(N, TB);
+    const int64_t bx = (int64_t)tx * splits_of<TB>(N, tx, p.cus), bw = (int64_t)tw * splits_of<TB>(M, tw, p.cus);
+    const unsigned blocks = (unsigned)(bx > bw ? bx : bw);
     if (p.call.argmax)
-        hipLaunchKernelGGL((forward_kernel<TB, true>), dim3(blocks), dim3(NT), lds, st, p);
+        hipLaunchKernelGGL((forward_kernel<TB, true, TWO>), dim3(blocks), dim3(NT), lds, st, p);
     else
-        hipLaunchKernelGGL((forward_kernel<TB, false>), dim3(blocks), dim3(NT), lds, st, p);
+        hipLaunchKernelGGL((forward_kernel<TB, false, TWO>), dim3(blocks), dim3(NT), lds, st, p);
     return check_launch("ordered::forward_kernel");
 }
 
 static int setup_device(int)
 {
     const void *kernels[] = {
-        (const void *)forward_kernel<4, true>, (const void *)forward_kernel<8, true>, (const void *)forward_kernel<16, true>,
-        (const void *)forward_kernel<32, true>, (const void *)forward_kernel<4, false>, (const void *)forward_kernel<8, false>,
-        (const void *)forward_kernel<16, false>, (const void *)forward_kernel<32, false>,
-        (const void *)build_kernel<4>, (const void *)build_kernel<8>, (const void *)build_kernel<16>, (const void *)build_kernel<40>};
+        (const void *)forward_kernel<4, true, false>,   (const void *)forward_kernel<8, true, false>,
+        (const void *)forward_kernel<16, true, false>,  (const void *)forward_kernel<32, true, false>,
+        (const void *)forward_kernel<4, false, false>,  (const void *)forward_kernel<8, false, false>,
+        (const void *)forward_kernel<16, false, false>, (const void *)forward_kernel<32, false, false>,
+        (const void *)forward_kernel<8, true, true>,    (const void *)forward_kernel<8, false, true>};
     for (const void *k : kernels)
-        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_TILE_BYTES) != hipSuccess) {
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) != hipSuccess) {
             (void)hipGetLastError();
             return fail(MAM_ERR_LAUNCH, "could not raise the LDS limit of the list kernels");
         }
@@ -741,36 +1052,35 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     Params p;
     p.call = call;
     const int64_t N = call.N, K = call.K, M = call.M;
+    const Layout l = layout(N, K, M);
     char *base = static_cast<char *>(workspace);
-    Sample *samples = reinterpret_cast<Sample *>(base);
-    p.samples = samples;
-    p.cap = list_cap(K);
-    p.rows_pad = (int)rows_padded(N, M);
-    p.lists = reinterpret_cast<uint4 *>(base + 1024);
-    p.bound = reinterpret_cast<float *>(base + 1024 + (size_t)p.cap * 8 * p.rows_pad);
-    // a product found through the lists costs two to three dense ones, and the longest search of a wave's 256
-    // outputs is what the wave does: the dense kernels are as fast where the sampled searches reach K / 6
-    p.limit = (int)(K / 6);
-    guard.samples = samples;
-    guard.limit = p.limit;
+    p.decision = reinterpret_cast<Decision *>(base);
+    p.samples = reinterpret_cast<int *>(base + 256);
+    p.lists_x = reinterpret_cast<uint4 *>(base + l.lists_x);
+    p.lists_w = reinterpret_cast<uint4 *>(base + l.lists_w);
+    p.bound_x = reinterpret_cast<float *>(base + l.bound_x);
+    p.bound_w = reinterpret_cast<float *>(base + l.bound_w);
+    p.turned = reinterpret_cast<float *>(base + l.turned);
+    p.turned_ld = l.turned_ld;
+    // a (K, M) weight takes the place of its transpose, with its own row length
+    if (call.w_layout == MAM_W_KM && (call.ldw * 4 >= (1 << 24) || call.ldw * 4 * K >= ((int64_t)1 << 32))) p.turned_ld = 0;
+    p.cap = l.cap;
+    p.pad_x = l.pad_x;
+    p.pad_w = l.pad_w;
+    guard.decision = p.decision;
 
-    const int tb = tile_rows(K);
-    const int rw = 256 / tb;                      // listed rows per wave
-    auto splits = [&](int64_t listed, int64_t tiled) {
-        // three rounds of workgroups over the chip, but at least one block of listed rows per wave
-        const int64_t tiles = ceil_div(tiled, tb), blocks = ceil_div(listed, rw);
-        int64_t s = ceil_div(3 * num_cus(), tiles);
-        const int64_t most = ceil_div(blocks, NT / 64);
-        return (int)(s < most ? s : most);
-    };
-    p.splits_x = splits(N, M);
-    p.splits_w = splits(M, N);
-    const int64_t bx = ceil_div(M, tb) * p.splits_x, bw = ceil_div(N, tb) * p.splits_w;
-
-    hipLaunchKernelGGL(sample_kernel, dim3(SAMPLES), dim3(256), 0, st, p, samples);
+    p.cus = num_cus();
+    hipLaunchKernelGGL(sample_kernel, dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
     int rc = check_launch("ordered::sample_kernel");
     if (rc != MAM_OK) return rc;
-    const dim3 build_grid((unsigned)(N > M ? N : M)), build_block(BUILD_NT);
+    const int64_t longer = N > M ? N : M;
+    if (p.turned_ld > 0) {
+        hipLaunchKernelGGL(decide_kernel, dim3(1), dim3(64 * LEADS), 0, st, p);
+        rc = check_launch("ordered::decide_kernel");
+        if (rc != MAM_OK) return rc;
+    }
+    const int64_t items = p.turned_ld > 0 ? N + M + ceil_div(longer, 64) * ceil_div(K, 64) : longer;
+    const dim3 build_grid((unsigned)items), build_block(BUILD_NT);
     const size_t lds = (size_t)p.cap * 8;
     if (K <= 4 * BUILD_NT) hipLaunchKernelGGL((build_kernel<4>), build_grid, build_block, lds, st, p);
     else if (K <= 8 * BUILD_NT) hipLaunchKernelGGL((build_kernel<8>), build_grid, build_block, lds, st, p);
@@ -778,13 +1088,15 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     else hipLaunchKernelGGL((build_kernel<40>), build_grid, build_block, lds, st, p);
     rc = check_launch("ordered::build_kernel");
     if (rc != MAM_OK) return rc;
-    const unsigned blocks = (unsigned)(bx > bw ? bx : bw);
-    switch (tb) {
-        case 32: return launch_forward<32>(p, blocks, st);
-        case 16: return launch_forward<16>(p, blocks, st);
-        case 8: return launch_forward<8>(p, blocks, st);
-        default: return launch_forward<4>(p, blocks, st);
+    switch (tile_rows(K)) {
+        case 32: rc = launch_forward<32, false>(p, st); break;
+        case 16: rc = launch_forward<16, false>(p, st); break;
+        case 8: rc = launch_forward<8, false>(p, st); break;
+        default: return launch_forward<4, false>(p, st);
     }
+    // Narrow tiles for the leading entries: 32 searched rows per wave, 128 contiguous bytes (12608 x 768 -> 3072, normal
+    // weights: 1740 / 1515 / 1206 us with 32 / 16 / 8 tile rows, 1730 us dense).
+    return rc != MAM_OK || p.turned_ld == 0 ? rc : launch_forward<8, true>(p, st);
 }
 
 }  // namespace ordered

@@ -118,3 +118,11 @@ def test_a_few_bad_rows_among_good_ones():
     assert_bits_equal(values.cpu().numpy(), want[0], "values-only c")
     assert_index_equal(amax.cpu().numpy(), want[1], "argmax")
     assert_index_equal(amin.cpu().numpy(), want[2], "argmin")
+
+
+@pytest.mark.parametrize("N,K,M", [(66, 520, 70), (97, 2432, 33), (64, 4864, 65), (40, 4095, 64)])
+@pytest.mark.parametrize("kind_x", ["normal", "sparse"])
+def test_two_sided_searches(N, K, M, kind_x):
+    """Normal weights: the leading entries of one operand first, then a search bounded by what they leave."""
+    _check(N, K, M, kind_x, "normal", seed=3)
+    _check(N, K, M, "normal", kind_x, layout_mk=False, seed=4)
