@@ -66,7 +66,7 @@ def build_torch_ops(verbose=False):
     cmd = (["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unknown-pragmas",
             "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
             "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)]
-           + inc + [os.path.join(CSRC, "torch_binding.cpp"), "-o", OPS_LIB,
+           + inc + [os.path.join(CSRC, "torch_binding.cpp"), os.path.join(CSRC, "torch_autograd.cpp"), "-o", OPS_LIB,
                     "-L" + LIB_DIR, "-lmam_hip", "-L" + torch_lib, "-ltorch", "-ltorch_cpu", "-lc10",
                     "-ltorch_hip", "-lc10_hip", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + torch_lib,
                     "-Wl,--no-as-needed"])

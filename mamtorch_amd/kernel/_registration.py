@@ -1,8 +1,5 @@
-"""Fake (meta) kernels and autograd formulas shared by the operator namespaces.
-
-Follows mamtorch/kernel/v4/fullyconnected.py:12-64 and mamtorch/kernel/v1/fullyconnected.py:12-64:
-the forward saves (a, b) only when a gradient is needed and always saves both index tensors; the
-backward calls the namespace's own ``fullyconnected_backward`` with the gradient of C only.
+"""Fake (meta) kernels shared by the operator namespaces (mamtorch/kernel/v4/fullyconnected.py:12-28,
+mamtorch/kernel/v1/fullyconnected.py:12-28).  The autograd formulas are registered in csrc/torch_autograd.cpp.
 """
 import torch
 
@@ -17,8 +14,6 @@ def _check_forward(a, b):
 
 def register_exact_forward(ns):
     """ns::fullyconnected(a, b) -> [C, argmax, argmin] and ns::fullyconnected_backward."""
-    ops = getattr(torch.ops, ns)
-
     @torch.library.register_fake(f"{ns}::fullyconnected")
     def _(a, b):
         _check_forward(a, b)
@@ -26,24 +21,6 @@ def register_exact_forward(ns):
         return [torch.empty(shape, dtype=torch.float, device=a.device),
                 torch.empty(shape, dtype=torch.int, device=a.device),
                 torch.empty(shape, dtype=torch.int, device=a.device)]
-
-    def _setup_context(ctx, inputs, output):
-        a, b = inputs
-        _, argmax, argmin = output
-        need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        ctx.save_for_backward(a if need else None, b if need else None, argmax, argmin)
-        # the index outputs never receive a gradient: without this autograd fills two (N, out) tensors with
-        # zeros for them before every backward
-        ctx.set_materialize_grads(False)
-
-    def _backward(ctx, grad):
-        a, b, argmax, argmin = ctx.saved_tensors
-        a_grad, b_grad = None, None
-        if grad[0] is not None and (ctx.needs_input_grad[0] or ctx.needs_input_grad[1]):
-            a_grad, b_grad = ops.fullyconnected_backward.default(a, b, grad[0].contiguous(), argmax, argmin)
-        return a_grad, b_grad
-
-    torch.library.register_autograd(f"{ns}::fullyconnected", _backward, setup_context=_setup_context)
 
     @torch.library.register_fake(f"{ns}::fullyconnected_backward")
     def _(a, b, grad, argmax, argmin):

@@ -32,25 +32,6 @@ def _(a, b):
     return torch.empty((a.size(0), b.size(1)), dtype=torch.float, device=a.device)
 
 
-def _setup_context(ctx, inputs, output):
-    a, b = inputs
-    need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-    ctx.save_for_backward(a if need else None, b if need else None)
-
-
-def _backward(ctx, grad):
-    a, b = ctx.saved_tensors
-    a_grad, b_grad = None, None
-    if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-        a_grad = grad @ b.T
-        b_grad = a.T @ grad
-    return a_grad, b_grad
-
-
-torch.library.register_autograd(
-    f"{library_name}::fullyconnected_fast", _backward, setup_context=_setup_context)
-
-
 @torch.library.register_fake(f"{library_name}::fullyconnected_fast_wt")
 def _(a, weight, bias):
     torch._check(a.dim() == 2 and weight.dim() == 2)
@@ -58,24 +39,3 @@ def _(a, weight, bias):
     torch._check(a.dtype == torch.float)
     torch._check(weight.dtype == torch.float)
     return torch.empty((a.size(0), weight.size(0)), dtype=torch.float, device=a.device)
-
-
-def _wt_setup_context(ctx, inputs, output):
-    a, weight, bias = inputs
-    need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-    ctx.save_for_backward(a if need else None, weight if need else None)
-
-
-def _wt_backward(ctx, grad):
-    a, weight = ctx.saved_tensors
-    a_grad, w_grad, bias_grad = None, None, None
-    if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-        a_grad = grad @ weight
-        w_grad = grad.T @ a
-    if ctx.needs_input_grad[2]:
-        bias_grad = grad.sum(dim=0)
-    return a_grad, w_grad, bias_grad
-
-
-torch.library.register_autograd(
-    f"{library_name}::fullyconnected_fast_wt", _wt_backward, setup_context=_wt_setup_context)

@@ -37,35 +37,6 @@ def _(a, weight, grad, argmax, argmin, range_len):
             torch.empty(weight.shape, dtype=torch.float, device=a.device)]
 
 
-def _ranges_setup(ctx, inputs, output):
-    a, weight, _, range_len, with_indices = inputs
-    _, argmax, argmin = output
-    need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-    ctx.range_len, ctx.with_indices = range_len, with_indices
-    ctx.save_for_backward(a if need else None, weight if need else None, argmax, argmin)
-    ctx.set_materialize_grads(False)      # no zero-filled gradients for the index outputs
-
-
-def _ranges_backward(ctx, grad):
-    a, weight, argmax, argmin = ctx.saved_tensors
-    a_grad = w_grad = bias_grad = None
-    g = grad[0]
-    if g is None:
-        return None, None, None, None, None
-    if ctx.needs_input_grad[0] or ctx.needs_input_grad[1]:
-        if not ctx.with_indices:
-            raise RuntimeError("fullyconnected_ranges was run without indices; its gradient needs them")
-        a_grad, w_grad = K.fullyconnected_ranges_backward.default(a, weight, g.contiguous(), argmax, argmin,
-                                                                  ctx.range_len)
-    if ctx.needs_input_grad[2]:
-        bias_grad = K.bias_grad.default(g)
-    return a_grad, w_grad, bias_grad, None, None
-
-
-torch.library.register_autograd("mamtorch_kernel_v4::fullyconnected_ranges", _ranges_backward,
-                                setup_context=_ranges_setup)
-
-
 def blend(mam: Tensor, mac: Tensor, bias, alpha: float, beta: float) -> Tensor:
     """(alpha * mam + beta * mac) + bias in the reference's rounding order; (N, out) operands."""
     return K.blend.default(mam, mac, bias, float(alpha), float(beta))
@@ -102,37 +73,10 @@ def _(mam, mac, bias, alpha, beta):
     return torch.empty(mam.shape, dtype=torch.float, device=mam.device)
 
 
-def _blend_setup(ctx, inputs, output):
-    _, _, _, alpha, beta = inputs
-    ctx.alpha, ctx.beta = alpha, beta
-
-
-def _blend_backward(ctx, grad):
-    g_mam = grad * ctx.alpha if ctx.needs_input_grad[0] else None
-    g_mac = grad * ctx.beta if ctx.needs_input_grad[1] else None
-    g_bias = grad.sum(dim=0) if ctx.needs_input_grad[2] else None
-    return g_mam, g_mac, g_bias, None, None
-
-
-torch.library.register_autograd("mamtorch_kernel_v4::blend", _blend_backward, setup_context=_blend_setup)
-
-
 @torch.library.register_fake("mamtorch_kernel_v4::apply_keep")
 def _(weight, keep):
     torch._check(weight.dim() == 2 and weight.dtype == torch.float and keep.shape == weight.shape)
     return torch.empty(weight.shape, dtype=torch.float, device=weight.device)
-
-
-def _keep_setup(ctx, inputs, output):
-    ctx.save_for_backward(inputs[1])
-
-
-def _keep_backward(ctx, grad):
-    (keep,) = ctx.saved_tensors
-    return K.apply_keep.default(grad, keep), None
-
-
-torch.library.register_autograd("mamtorch_kernel_v4::apply_keep", _keep_backward, setup_context=_keep_setup)
 
 
 def _out_positions(H, W, k1, k2, s1, s2):
@@ -151,28 +95,3 @@ def _(x, k1, k2, s1, s2):
 def _(cols, B, C, H, W, k1, k2, s1, s2):
     torch._check(cols.dim() == 2 and cols.dtype == torch.float)
     return torch.empty((B, C, H, W), dtype=torch.float, device=cols.device)
-
-
-def _im2col_setup(ctx, inputs, output):
-    x, k1, k2, s1, s2 = inputs
-    ctx.geom = (tuple(x.shape), k1, k2, s1, s2)
-
-
-def _im2col_backward(ctx, grad):
-    shape, k1, k2, s1, s2 = ctx.geom
-    return K.col2im.default(grad.contiguous(), *shape, k1, k2, s1, s2), None, None, None, None
-
-
-torch.library.register_autograd("mamtorch_kernel_v4::im2col", _im2col_backward, setup_context=_im2col_setup)
-
-
-def _col2im_setup(ctx, inputs, output):
-    ctx.geom = inputs[5:]
-
-
-def _col2im_backward(ctx, grad):
-    k1, k2, s1, s2 = ctx.geom
-    return (K.im2col.default(grad.contiguous(), k1, k2, s1, s2),) + (None,) * 8
-
-
-torch.library.register_autograd("mamtorch_kernel_v4::col2im", _col2im_backward, setup_context=_col2im_setup)

@@ -169,7 +169,7 @@ class FullyConnected(Module):
         if self.relu_in:
             input = F.relu(input)
 
-        input_flat = input.reshape(-1, input.size()[-1])
+        input_flat = input if input.dim() == 2 else input.reshape(-1, input.size()[-1])
         w = self._dropped_weight()
         # without a MAC blend the bias rides along in the MAM kernel, after the sum of max and min (and
         # after the sum over the splits): the reference's rounding order; with a blend the blend adds it
@@ -197,7 +197,7 @@ class FullyConnected(Module):
             mac_weight = self.weight.detach() if self.train_mam_only else self.weight
             C_flat = K.v4.blend(C_flat, F.linear(input_flat, mac_weight), self.bias, self.alpha, self.beta)
 
-        C = C_flat.view(input.shape[:-1] + (self.weight.size(0),))
+        C = C_flat if input.dim() == 2 else C_flat.view(input.shape[:-1] + (self.weight.size(0),))
 
         if self.drop_rate > 0:
             C = F.dropout(C, self.drop_rate, self.training)

@@ -36,10 +36,13 @@ class SparseFullyConnectedFunction(torch.autograd.Function):
         ctx.save_for_backward(a, values, crow_indices, col_indices, argmax, argmin, w_sel, pos_sel)
         ctx.out_features = out_features
         ctx.mark_non_differentiable(argmax, argmin)
+        ctx.set_materialize_grads(False)      # no zero-filled gradients for the index outputs
         return c, argmax, argmin
 
     @staticmethod
     def backward(ctx, grad, _gmax, _gmin):
+        if grad is None:
+            return None, None, None, None, None
         a, values, crow_indices, col_indices, argmax, argmin, w_sel, pos_sel = ctx.saved_tensors
         w_csr = torch.sparse_csr_tensor(crow_indices, col_indices, values.detach(),
                                         size=(ctx.out_features, a.size(1)))
