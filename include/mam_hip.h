@@ -117,10 +117,10 @@ int mam_set_option(int option, int value);
  * `x_sel` (optional, may be NULL): the same for the inputs, x[n, argmax[n,m]] and x[n, argmin[n,m]]; it
  * spares mam_fc_backward the 2*N*M random reads of x behind w_grad.
  * mam_fc_forward_workspace_for() is the same query for a given operand layout and output set
- * (with_indices: mam_fc_forward, else mam_fc_forward_values): for MAM_W_KM it adds room for one transposed
- * copy of w, with which the call runs the faster (M, K) tiling (from 16 batch rows on, K a multiple of 64;
- * 1.5 times as fast at the 256 x 4096 x 4096 shape, 1.7 times at batch 16384).  A (K, M) call whose workspace only has
- * mam_fc_forward_workspace() bytes still works, on the general tiling.
+ * (with_indices: mam_fc_forward, else mam_fc_forward_values) with room for what makes the call faster: copies of the
+ * operands for MAM_W_KM weights and for K that is no multiple of 16 (1.5 to 3 times as fast), and the lists of large
+ * calls (2^32 products and more; 2 to 12 times as fast).  A call whose workspace only has
+ * mam_fc_forward_workspace() bytes still works, without them.
  */
 size_t mam_fc_forward_workspace(int64_t N, int64_t K, int64_t M);
 size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, int w_layout, int with_indices);

@@ -37,11 +37,17 @@ int option(int which);
 // Compute units of the current device (read from the device at its set-up).
 int num_cus();
 
-// dst (cols, rows) contiguous = transpose of src (rows, cols), row stride ld.  `guard` (mam_ordered.h): the
-// kernel exits at once where the guard says that nobody reads the copy.
+// dst (cols, ld_dst) = transpose of src (rows, cols), row stride ld; columns rows .. ld_dst - 1 repeat the last one.
+// `guard` (mam_ordered.h): the kernel exits at once where the guard says that nobody reads the copy.
 namespace ordered { struct Guard; }
-int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, hipStream_t stream,
+int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, int64_t ld_dst, hipStream_t stream,
               const ordered::Guard *guard = nullptr);
+
+// dst (rows, ld_dst) = src (rows, cols) with row stride ld, the last element of a row repeated up to ld_dst; two matrices
+// in one launch (rows == 0: none).  ld_dst is a multiple of 4, dst 16-byte aligned, at most 65535 rows together.
+struct LengthenRows { const float *src; int64_t ld; float *dst; int rows; };
+int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, hipStream_t stream,
+                  const ordered::Guard *guard = nullptr);
 
 // Two independent kernels of one call side by side: the first runs on a second stream of the library
 // (default priority, one per device) between a fork and a join event on the caller's stream.

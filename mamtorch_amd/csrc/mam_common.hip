@@ -45,11 +45,11 @@ int fill_zero(void *ptr, int64_t count, hipStream_t stream)
     return check_launch("fill_zero_kernel");
 }
 
-// dst (cols, rows) contiguous = transpose of src (rows, cols) with row stride ld: 64 x 64 tiles through LDS,
-// 16-byte accesses on both sides when the shapes allow it.
+// dst (cols, ld_dst) = transpose of src (rows, cols) with row stride ld; columns rows .. ld_dst - 1 of dst repeat the
+// last one.  64 x 64 tiles through LDS, 16-byte accesses on both sides when the shapes allow it.
 __global__ __launch_bounds__(256) void transpose_kernel(const float *__restrict__ src, int64_t ld,
-                                                        float *__restrict__ dst, int rows, int cols, int vec,
-                                                        const ordered::Guard guard)
+                                                        float *__restrict__ dst, int rows, int cols, int ld_dst,
+                                                        int vec_src, int vec_dst, const ordered::Guard guard)
 {
     if (ordered::guarded_off(guard)) return;
     __shared__ float tile[64][65];
@@ -57,18 +57,16 @@ __global__ __launch_bounds__(256) void transpose_kernel(const float *__restrict_
     const int c0 = blockIdx.x * 64, r0 = blockIdx.y * 64;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        const int r = r0 + ty + 16 * i, c = c0 + tx * 4;
+        const int r = (r0 + ty + 16 * i) < rows ? r0 + ty + 16 * i : rows - 1, c = c0 + tx * 4;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (r < rows) {
-            const float *row = src + (int64_t)r * ld;
-            if (vec && c + 3 < cols) {
-                v = *reinterpret_cast<const float4 *>(row + c);
-            } else {
-                if (c < cols) v.x = row[c];
-                if (c + 1 < cols) v.y = row[c + 1];
-                if (c + 2 < cols) v.z = row[c + 2];
-                if (c + 3 < cols) v.w = row[c + 3];
-            }
+        const float *row = src + (int64_t)r * ld;
+        if (vec_src && c + 3 < cols) {
+            v = *reinterpret_cast<const float4 *>(row + c);
+        } else {
+            if (c < cols) v.x = row[c];
+            if (c + 1 < cols) v.y = row[c + 1];
+            if (c + 2 < cols) v.z = row[c + 2];
+            if (c + 3 < cols) v.w = row[c + 3];
         }
         float *t = &tile[ty + 16 * i][tx * 4];
         t[0] = v.x; t[1] = v.y; t[2] = v.z; t[3] = v.w;
@@ -78,30 +76,60 @@ __global__ __launch_bounds__(256) void transpose_kernel(const float *__restrict_
     for (int i = 0; i < 4; ++i) {
         const int c = c0 + ty + 16 * i, r = r0 + tx * 4;       // dst row c, dst columns r .. r + 3
         if (c >= cols) continue;
-        float *out = dst + (int64_t)c * rows;
+        float *out = dst + (int64_t)c * ld_dst;
         const float4 v = make_float4(tile[tx * 4][ty + 16 * i], tile[tx * 4 + 1][ty + 16 * i],
                                      tile[tx * 4 + 2][ty + 16 * i], tile[tx * 4 + 3][ty + 16 * i]);
-        if (vec && r + 3 < rows && (rows & 3) == 0) {
+        if (vec_dst && r + 3 < ld_dst) {
             *reinterpret_cast<float4 *>(out + r) = v;
         } else {
-            if (r < rows) out[r] = v.x;
-            if (r + 1 < rows) out[r + 1] = v.y;
-            if (r + 2 < rows) out[r + 2] = v.z;
-            if (r + 3 < rows) out[r + 3] = v.w;
+            if (r < ld_dst) out[r] = v.x;
+            if (r + 1 < ld_dst) out[r + 1] = v.y;
+            if (r + 2 < ld_dst) out[r + 2] = v.z;
+            if (r + 3 < ld_dst) out[r + 3] = v.w;
         }
     }
 }
 
-int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, hipStream_t stream,
+int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t cols, int64_t ld_dst, hipStream_t stream,
               const ordered::Guard *guard)
 {
     if (rows <= 0 || cols <= 0) return MAM_OK;
-    const int64_t gx = ceil_div(cols, 64), gy = ceil_div(rows, 64);
+    const int64_t gx = ceil_div(cols, 64), gy = ceil_div(ld_dst, 64);
     if (gy > 65535 || gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "matrix too large for the transpose grid");
-    const int vec = (ld % 4 == 0) && ((uintptr_t)src % 16 == 0) && ((uintptr_t)dst % 16 == 0);
+    const int vec_src = (ld % 4 == 0) && ((uintptr_t)src % 16 == 0), vec_dst = (ld_dst % 4 == 0) && ((uintptr_t)dst % 16 == 0);
     hipLaunchKernelGGL(transpose_kernel, dim3((unsigned)gx, (unsigned)gy), dim3(256), 0, stream, src, ld, dst,
-                       (int)rows, (int)cols, vec, guard ? *guard : ordered::Guard{nullptr});
+                       (int)rows, (int)cols, (int)ld_dst, vec_src, vec_dst, guard ? *guard : ordered::Guard{nullptr});
     return check_launch("transpose_kernel");
+}
+
+// Two matrices copied with their rows lengthened: row r of dst is row r of src, then its last element up to ld_dst.
+// Bound by memory; a workgroup takes 1024 consecutive floats of a row.
+__global__ __launch_bounds__(256) void lengthen_rows_kernel(const LengthenRows a, const LengthenRows b, int cols, int ld_dst,
+                                                            const ordered::Guard guard)
+{
+    if (ordered::guarded_off(guard)) return;
+    const bool first = (int)blockIdx.y < a.rows;
+    const LengthenRows &m = first ? a : b;
+    const int64_t row = first ? blockIdx.y : blockIdx.y - a.rows;
+    const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
+    if (c >= ld_dst) return;
+    const float *src = m.src + row * m.ld;
+    const int last = cols - 1;
+    float4 v;
+    v.x = src[c < last ? c : last];
+    v.y = src[c + 1 < last ? c + 1 : last];
+    v.z = src[c + 2 < last ? c + 2 : last];
+    v.w = src[c + 3 < last ? c + 3 : last];
+    *reinterpret_cast<float4 *>(m.dst + row * ld_dst + c) = v;
+}
+
+int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, hipStream_t stream,
+                  const ordered::Guard *guard)
+{
+    if (a.rows + b.rows == 0) return MAM_OK;
+    hipLaunchKernelGGL(lengthen_rows_kernel, dim3((unsigned)ceil_div(ld_dst, 1024), (unsigned)(a.rows + b.rows)), dim3(256), 0,
+                       stream, a, b, (int)cols, (int)ld_dst, guard ? *guard : ordered::Guard{nullptr});
+    return check_launch("lengthen_rows_kernel");
 }
 
 namespace {

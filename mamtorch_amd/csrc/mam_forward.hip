@@ -26,8 +26,9 @@
 // a wave's W reads cover all banks and its X reads broadcast.  Ragged edges are handled by
 // replicating the last row / column / k on load: a replicated k duplicates an earlier product
 // and can never win a strict comparison.  The second one (mam_fwd_sx_kernel, further down)
-// serves the module's case -- (out, in) weight, aligned rows, K a multiple of 64 -- with
-// wave-uniform batch rows whose x operands come through the scalar cache.
+// serves the module's case -- (out, in) weight, aligned rows, K a multiple of 16 -- with
+// wave-uniform batch rows whose x operands come through the scalar cache; calls with other operands are
+// copied into that form once where the workspace has room (Staging).
 //
 // Small N*M (the 256 x 4096 headline shape has only 256 tiles for 256 CUs x 2) is split
 // along K; each split writes (value, group) partials and a merge kernel combines them in
@@ -686,6 +687,8 @@ __global__ __launch_bounds__(NT, 2) void mam_fwd_kernel(const Params p)
 template <int LAYOUT, bool ARGS, bool COOP, int GT = G>
 __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
 {
+    // (the arguments of the prologue in one fetch with the guard's, not in a second one behind its branch)
+    asm volatile("" ::"s"(p.part), "s"(p.N), "s"(p.splits), "s"(p.x), "s"(p.w), "s"(p.bias), "s"(p.c));
     if (ordered::guarded_off(p.guard)) return;
     // A workgroup owns a PR x PC patch of c (16 x 16; with the cooperative resolve 4 x 64: a wave takes one batch
     // row, and its piece of every partial plane and of every output array is two whole 128-byte lines; measured at
@@ -874,6 +877,8 @@ typedef const __attribute__((address_space(4))) float const_f32;
 template <int TJ, bool ARGS, bool SPLIT, bool TAIL, int GT = G, bool FUSE = false>
 __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
 {
+    // (the arguments of the prologue in one fetch with the guard's, not in a second one behind its branch)
+    asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.ldx), "s"(p.ldw), "s"(p.tiles_n), "s"(p.k_per_split), "s"(p.group_n));
     if (ordered::guarded_off(p.guard)) return;
     using C = sx::Cfg<TJ>;
     __shared__ __attribute__((aligned(16))) float tile_a[C::TILE_FLOATS];
@@ -1216,7 +1221,9 @@ static int choose_splits(int64_t N, int64_t K, int64_t M, int bn = BN, int bm = 
 static size_t workspace_bytes(int64_t N, int64_t K, int64_t M, bool args)
 {
     // whichever tiling the launch picks (it depends on alignment, unknown here): the larger need
-    const int s1 = choose_splits(N, K, M), s2 = choose_splits(N, K, M, sx::BN, sx::BM_MAX);
+    // (and whether it runs on lengthened rows or not)
+    const int64_t longer = K % G == 0 ? K : ceil_div(K, sx::KT) * sx::KT;
+    const int s1 = choose_splits(N, K, M), s2 = choose_splits(N, longer, M, sx::BN, sx::BM_MAX);
     const int s = s1 > s2 ? s1 : s2;
     if (s == 1) return 0;
     size_t tickets = 0;     // of the fused merge, one per tile of the finer tiling
@@ -1326,6 +1333,28 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     return MAM_OK;
 }
 
+// Operands that the wave-uniform-rows tiling does not take as they are -- a (K, M) weight, rows that are not 16-byte
+// aligned, K not a multiple of 16 -- are copied into the workspace once per call in the form that it does take.  Rows of
+// a ragged K are lengthened to whole 64-k tiles by their own last element: a repeated product never wins a strict
+// comparison, so every result stays what it was.
+struct Staging {
+    bool x, w;             // copied
+    int64_t K;             // row length of the copies (and of the call)
+    size_t x_bytes, w_bytes;
+    size_t bytes() const { return x_bytes + w_bytes; }
+};
+static Staging staging_of(bool x_fits, bool w_fits, int64_t N, int64_t K, int64_t M)
+{
+    Staging s;
+    s.K = K % G == 0 ? K : ceil_div(K, sx::KT) * sx::KT;
+    s.x = !x_fits || s.K != K;
+    s.w = !w_fits || s.K != K;
+    auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    s.x_bytes = s.x ? padded((size_t)N * (size_t)s.K * sizeof(float)) : 0;
+    s.w_bytes = s.w ? padded((size_t)M * (size_t)s.K * sizeof(float)) : 0;
+    return s;
+}
+
 // Whether to transpose a (K, M) operand once and run the (M, K) tilings on the copy: two more passes
 // over the weight against a kernel that is 1.7 times as fast per triple.  Measured, (K, M) operand as it
 // is / transposed first / the same weight given as (M, K): 0.371 / 0.240 / 0.221 ms at 256 x 4096 x 4096,
@@ -1335,6 +1364,32 @@ static bool transposed_operand_pays(int64_t N, int64_t K, int64_t M)
     (void)K;
     (void)M;
     return N >= 16 && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
+}
+
+// Whether to lengthen ragged rows: one launch that reads and writes both operands once, against the general tiling, at
+// every size measured ((N, K, M): 1 x 4001 x 4096 100 / 61 us, 16 x 1001 x 512 47 / 22, 250 x 1001 x 517 69 / 32, 1000 x 777 x
+// 1000 187 / 74, 4000 x 531 x 3712 1597 / 571; values only 69 / 55, 35 / 18, 39 / 24, 75 / 50, 466 / 361).
+static bool lengthened_rows_pay(int64_t N, int64_t M)
+{
+    return N + M <= 65535 && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
+}
+
+// The plan of a call on staged operands, for a call that the wave-uniform-rows tiling does not take as it is; false:
+// there is none, or it does not pay.
+static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, const float *x, int64_t ldx, const float *w,
+                        int64_t ldw, int w_layout, const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel,
+                        float *x_sel, int64_t N, int64_t K, int64_t M, int64_t range_len)
+{
+    if (plan.use_sx) return false;
+    const bool turn = w_layout == MAM_W_KM;
+    st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M);
+    const bool lengthen = st.x || (st.w && !turn);
+    if (turn && !transposed_operand_pays(N, K, M)) return false;
+    if (lengthen && (!lengthened_rows_pay(N, M) || range_len > 0)) return false;
+    float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
+    const int rc = make_plan(staged, args, st.x ? aligned : x, st.x ? st.K : ldx, st.w ? aligned : w, st.w ? st.K : ldw, MAM_W_MK, bias,
+                             c, argmax, argmin, w_sel, x_sel, N, st.K, M, range_len);
+    return rc == MAM_OK && staged.use_sx;
 }
 
 template <bool ARGS>
@@ -1350,24 +1405,21 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     if (!x || !w || !c || (ARGS && (!argmax || !argmin)))
         return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     const size_t avail = static_scratch ? static_scratch_bytes() : (workspace ? workspace_size : (size_t)0);
-    // The operand b of the reference operators is (K, M).  The general tiling takes it as it is and
-    // transposes every tile through registers (0.37 ms at the 256 x 4096 x 4096 shape).  When the
-    // workspace has room, b is transposed ONCE into it and the wave-uniform-rows tiling runs on the copy
-    // (0.22 ms + the transpose): every output is the same, bit for bit.
-    size_t wt_bytes = 0;
+    // Where the workspace has room, operands that the wave-uniform-rows tiling does not take are staged in it (see
+    // Staging): every output is the same, bit for bit.
     const int operand_layout = w_layout;
-    if (w_layout == MAM_W_KM && transposed_operand_pays(N, K, M)) {
-        Plan tplan;
-        float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
-        const int trc = make_plan(tplan, ARGS, x, ldx, aligned, K, MAM_W_MK, bias, c, argmax, argmin, w_sel, x_sel,
-                                  N, K, M, range_len);
-        const size_t bytes = ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256;
-        if (trc == MAM_OK && tplan.use_sx && bytes + tplan.need <= avail &&
-            (static_scratch || (uintptr_t)workspace % 16 == 0)) {
-            plan = tplan;
-            wt_bytes = bytes;
-            w_layout = MAM_W_MK;
-        }
+    const int64_t operand_K = K;
+    size_t wt_bytes = 0;
+    Staging stage = {false, false, K, 0, 0};
+    Plan tplan;
+    Staging st_plan;
+    if (staged_plan(tplan, st_plan, plan, ARGS, x, ldx, w, ldw, w_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M, range_len) &&
+        st_plan.bytes() + tplan.need <= avail && (static_scratch || (uintptr_t)workspace % 16 == 0)) {
+        plan = tplan;
+        stage = st_plan;
+        wt_bytes = stage.bytes();
+        w_layout = MAM_W_MK;
+        K = stage.K;
     }
     Params &p = plan.p;
     const bool use_sx = plan.use_sx;
@@ -1405,19 +1457,23 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     }
     // Large calls by magnitude-ordered lists, where the workspace has room for them; the kernels below then run
     // only if the data turns out not to suit the lists.
-    if (range_len == 0 && !static_scratch && ordered::applies(N, K, M) && (operand_layout == MAM_W_MK || ldw < (1 << 22))) {
+    if (range_len == 0 && !static_scratch && ordered::applies(N, operand_K, M) && (operand_layout == MAM_W_MK || ldw < (1 << 22))) {
         const size_t at = (wt_bytes + need + 255) / 256 * 256;
-        if (avail >= at + ordered::workspace_bytes(N, K, M) && (uintptr_t)workspace % 16 == 0) {
-            const ordered::Call call = {x, ldx, w, ldw, operand_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M};
+        if (avail >= at + ordered::workspace_bytes(N, operand_K, M) && (uintptr_t)workspace % 16 == 0) {
+            const ordered::Call call = {x, ldx, w, ldw, operand_layout, bias, c, argmax, argmin, w_sel, x_sel, N, operand_K, M};
             rc = ordered::launch(call, scratch_base + at, p.guard, st);
             if (rc != MAM_OK) return rc;
         }
     }
     if (wt_bytes > 0) {
-        float *wt = reinterpret_cast<float *>(scratch_base);
-        rc = transpose(w, ldw, wt, K, M, st, &p.guard);
+        float *const ws = reinterpret_cast<float *>(scratch_base), *const xs = reinterpret_cast<float *>(scratch_base + stage.w_bytes);
+        const bool turn = operand_layout == MAM_W_KM;
+        const LengthenRows rx = {x, ldx, xs, stage.x ? (int)N : 0}, rw = {w, ldw, ws, stage.w && !turn ? (int)M : 0};
+        rc = lengthen_rows(rx, rw, operand_K, K, st, &p.guard);
+        if (rc == MAM_OK && turn) rc = transpose(w, ldw, ws, operand_K, M, K, st, &p.guard);
         if (rc != MAM_OK) return rc;
-        p.w = wt;
+        if (stage.x) p.x = xs;
+        if (stage.w) p.w = ws;
     }
     const bool tail = K % sx::KT != 0;
     if (fuse)
@@ -1482,9 +1538,10 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
 {
     if (N <= 0 || K <= 0 || M <= 0) return 0;
     size_t bytes = mam::fwd::workspace_bytes(N, K, M, with_indices != 0);
-    // room for the transposed copy of a (K, M) operand (see launch); without it the call still works
-    if (w_layout == MAM_W_KM && K % mam::fwd::G == 0 && mam::fwd::transposed_operand_pays(N, K, M))
-        bytes += ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256;
+    // room for staged operands (see launch); without it the call still works
+    const bool turn = w_layout == MAM_W_KM, ragged = K % mam::fwd::G != 0;
+    if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || mam::fwd::lengthened_rows_pay(N, M)))
+        bytes += mam::fwd::staging_of(true, !turn, N, K, M).bytes();
     if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M);
     return bytes;
 }
@@ -1547,25 +1604,23 @@ extern "C" int mam_fc_forward_describe(const float *x, int64_t ldx, const float 
         snprintf(text, text_bytes, "nothing to launch");
         return MAM_OK;
     }
-    // A (K, M) operand is transposed once into the workspace when that has room (what
-    // mam_fc_forward_workspace_for() asks for) and the wave-uniform-rows tiling then runs on the copy: both
-    // routes are named, the one a call takes depends on the workspace it brings.
-    if (w_layout == MAM_W_KM && fwd::transposed_operand_pays(N, K, M)) {
-        fwd::Plan tplan;
-        float *const aligned = reinterpret_cast<float *>((uintptr_t)256);
-        const int trc = fwd::make_plan(tplan, with_indices != 0, x, ldx, aligned, K, MAM_W_MK, nullptr, nullptr,
-                                       nullptr, nullptr, nullptr, nullptr, N, K, M);
-        if (trc == MAM_OK && tplan.use_sx) {
-            const size_t copy = ((size_t)M * (size_t)K * sizeof(float) + 255) / 256 * 256;
-            int used = snprintf(text, text_bytes, "with %zu workspace bytes: transpose_kernel + ", copy + tplan.need);
-            if (used < 0 || (size_t)used >= text_bytes) return MAM_OK;
-            describe_plan(tplan, MAM_W_MK, K, with_indices != 0, text + used, text_bytes - used);
-            used = (int)strlen(text);
-            const int more = snprintf(text + used, text_bytes - used, "; with less: ");
-            if (more < 0 || (size_t)(used + more) >= text_bytes) return MAM_OK;
-            describe_plan(plan, w_layout, K, with_indices != 0, text + used + more, text_bytes - used - more);
-            return MAM_OK;
-        }
+    // Operands are staged in the workspace when that has room (what mam_fc_forward_workspace_for() asks for) and the
+    // wave-uniform-rows tiling then runs on the copies: both routes are named, the one a call takes depends on the
+    // workspace it brings.
+    fwd::Plan tplan;
+    fwd::Staging st;
+    if (fwd::staged_plan(tplan, st, plan, with_indices != 0, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr,
+                         nullptr, N, K, M, 0)) {
+        const bool turn = w_layout == MAM_W_KM;
+        int used = snprintf(text, text_bytes, "with %zu workspace bytes: %s%s", st.bytes() + tplan.need,
+                            st.x || !turn ? "lengthen_rows_kernel + " : "", turn ? "transpose_kernel + " : "");
+        if (used < 0 || (size_t)used >= text_bytes) return MAM_OK;
+        describe_plan(tplan, MAM_W_MK, st.K, with_indices != 0, text + used, text_bytes - used);
+        used = (int)strlen(text);
+        const int more = snprintf(text + used, text_bytes - used, "; with less: ");
+        if (more < 0 || (size_t)(used + more) >= text_bytes) return MAM_OK;
+        describe_plan(plan, w_layout, K, with_indices != 0, text + used + more, text_bytes - used - more);
+        return MAM_OK;
     }
     describe_plan(plan, w_layout, K, with_indices != 0, text, text_bytes);
     return MAM_OK;
