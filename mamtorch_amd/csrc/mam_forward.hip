@@ -843,7 +843,8 @@ constexpr int TI = 4;     // batch rows per wave
 constexpr int KT = 64;    // k extent of one W tile
 constexpr int CHUNKS = KT / 4;    // 16-byte chunks per neuron and tile
 constexpr int RPB = 64 / KT < 1 ? 1 : 64 / KT;   // neurons per 256 bytes of LDS (all 64 banks)
-// TJ = neurons per lane.  2 (128 neurons per workgroup) is what the launch uses.  Measured at the
+// TJ = neurons per lane.  2 (128 neurons per workgroup) is what the launch uses unless half of the last tile would be
+// empty (Plan::narrow).  Measured at the
 // 256 x 4096 x 4096 shape: 1 (64 neurons per workgroup, 512 tiles, no split of K and no merge) 0.226 ms
 // against 0.217 ms for 2 with K split in two plus the merge -- the k loop with one neuron per lane is 7 %
 // slower (twice the scalar loads per product), which costs more than the merge; 4 with 32-k tiles: the
@@ -1223,6 +1224,7 @@ static size_t workspace_bytes(int64_t N, int64_t K, int64_t M, bool args)
     // whichever tiling the launch picks (it depends on alignment, unknown here): the larger need
     // (and whether it runs on lengthened rows or not)
     const int64_t longer = K % G == 0 ? K : ceil_div(K, sx::KT) * sx::KT;
+    // (64-neuron tiles are as many or more, and split no further)
     const int s1 = choose_splits(N, K, M), s2 = choose_splits(N, longer, M, sx::BN, sx::BM_MAX);
     const int s = s1 > s2 ? s1 : s2;
     if (s == 1) return 0;
@@ -1260,6 +1262,7 @@ static void *static_scratch_of(int dev) { return g_scratch[dev]; }
 struct Plan {
     Params p;
     bool use_sx;
+    bool narrow;          // of the wave-uniform-rows tiling: 64 neurons per workgroup instead of 128
     size_t need;          // workspace bytes: the partials, then the tickets of the fused merge
     size_t tickets_at;    // offset of the tickets
 };
@@ -1293,7 +1296,12 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
                         (range_len % sx::KT == 0) && (ldw * sx::BM_MAX < (1ll << 30)) &&
                         option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
     plan.use_sx = use_sx;
-    const int bn = use_sx ? sx::BN : BN, bm = use_sx ? sx::BM_MAX : BM;
+    // Half of the last 128-neuron tile is work for neurons that are not there when M is an odd multiple of 64 (or
+    // little less): with 1, 3 or 5 of them that is 50, 25 or 17 % of the call, against 7 % that a product costs more
+    // in a 64-neuron tile (21632 x 288 -> 64: 92 us with 128 neurons per tile, 54 us with 64).
+    const int64_t m64 = ceil_div(M, 64);
+    plan.narrow = use_sx && m64 % 2 == 1 && m64 <= 5 && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_FUSED_MERGE;
+    const int bn = use_sx ? sx::BN : BN, bm = use_sx ? (plan.narrow ? sx::Cfg<1>::BM : sx::BM_MAX) : BM;
     p.tiles_n = (int)ceil_div(N, bn);
     p.tiles_m = (int)ceil_div(M, bm);
     // Tile order: GROUP_N row tiles are swept under one W panel, panel after panel.  An XCD has 64 tiles in
@@ -1392,6 +1400,24 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
     return rc == MAM_OK && staged.use_sx;
 }
 
+// The wave-uniform-rows tiling with 64 * TJ neurons per workgroup; tail: a partial last k tile.
+template <int TJ, bool ARGS>
+static void launch_sx(const Params &p, bool tail, unsigned blocks, hipStream_t st)
+{
+    constexpr int GT = ARGS ? 2 * G : G;
+    const dim3 grid(blocks), block(sx::NT);
+    const bool spans = ARGS && p.gt == 2 * G;
+    if (p.splits > 1) {
+        if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, true, true>), grid, block, 0, st, p);
+        else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, true, false, GT>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, true, false>), grid, block, 0, st, p);
+    } else {
+        if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, false, true>), grid, block, 0, st, p);
+        else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, false, false, GT>), grid, block, 0, st, p);
+        else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, false, false>), grid, block, 0, st, p);
+    }
+}
+
 template <bool ARGS>
 static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                   const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel, float *x_sel,
@@ -1478,18 +1504,10 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     const bool tail = K % sx::KT != 0;
     if (fuse)
         hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, false, ARGS ? 2 * G : G, ARGS>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && p.splits > 1 && tail)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, true>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && p.splits > 1 && ARGS && p.gt == 2 * G)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, false, ARGS ? 2 * G : G>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && p.splits > 1)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, false>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && tail)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, false, true>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && ARGS && p.gt == 2 * G)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, false, false, ARGS ? 2 * G : G>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
+    else if (use_sx && plan.narrow)
+        launch_sx<1, ARGS>(p, tail, (unsigned)nblk, st);
     else if (use_sx)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, false, false>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
+        launch_sx<2, ARGS>(p, tail, (unsigned)nblk, st);
     else if (w_layout == MAM_W_MK)
         hipLaunchKernelGGL((mam_fwd_kernel<MAM_W_MK, ARGS>), dim3((unsigned)nblk), dim3(NT), 0, st, p);
     else
@@ -1577,9 +1595,9 @@ static void describe_plan(const mam::fwd::Plan &plan, int w_layout, int64_t K, b
     const fwd::Params &p = plan.p;
     const char *what = with_indices ? "args" : "values";
     if (plan.use_sx)
-        snprintf(text, text_bytes, "mam_fwd_sx_kernel<%s%s%s%s> %d x %d tiles of 32 x 128", what, p.splits > 1 ? ", split" : "",
+        snprintf(text, text_bytes, "mam_fwd_sx_kernel<%s%s%s%s> %d x %d tiles of 32 x %d", what, p.splits > 1 ? ", split" : "",
                  K % fwd::sx::KT != 0 ? ", partial last k tile" : "", p.gt > fwd::G ? ", indices per 32 k" : "", p.tiles_n,
-                 p.tiles_m);
+                 p.tiles_m, plan.narrow ? 64 : 128);
     else
         snprintf(text, text_bytes, "mam_fwd_kernel<%s, %s> %d x %d tiles of 64 x 128", w_layout == MAM_W_MK ? "(M,K)" : "(K,M)",
                  what, p.tiles_n, p.tiles_m);

@@ -205,3 +205,27 @@ def test_window_gather_operators():
     bias = torch.randn(5, generator=g).to(DEV).requires_grad_(True)
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.blend, (a, b, bias, 0.75, 0.25))
     assert torch.equal(mt.kernel.v4.blend(a, b, bias, 0.75, 0.25), (0.75 * a + 0.25 * b) + bias)
+
+
+@pytest.mark.parametrize("B,C,H,W,k1,k2,s1,s2", [
+    (2, 4, 5, 33, 3, 3, 1, 1), (1, 5, 7, 32, 2, 3, 2, 1), (2, 36, 6, 70, 3, 2, 1, 2), (1, 32, 9, 9, 9, 9, 1, 1),
+    (3, 1, 4, 40, 1, 1, 3, 3), (1, 8, 12, 300, 5, 40, 1, 3), (2, 65, 5, 34, 4, 3, 1, 1)])
+def test_windows_and_their_adjoint(B, C, H, W, k1, k2, s1, s2):
+    """Window gather and adjoint at the edges of their 32-channel, 32-column tiles, with and without 16-byte rows and
+    with input rows that do not fit the staged kernel: the gather exactly, the adjoint in ascending window order."""
+    g = torch.Generator().manual_seed(C * W)
+    x = torch.randn(B, C, H, W, generator=g)
+    L1, L2 = (H - k1) // s1 + 1, (W - k2) // s2 + 1
+    want = torch.stack([x[:, :, j1:j1 + (L1 - 1) * s1 + 1:s1, j2:j2 + (L2 - 1) * s2 + 1:s2]
+                        for j2 in range(k2) for j1 in range(k1)], 1)            # (B, window, C, L1, L2)
+    want = want.permute(0, 3, 4, 1, 2).reshape(B * L1 * L2, k1 * k2 * C)
+    got = mt.kernel.v4.im2col(x.to(DEV), k1, k2, s1, s2)
+    assert_bits_equal(got.cpu().numpy(), want.numpy(), "im2col")
+    cols = torch.randn(B * L1 * L2, k1 * k2 * C, generator=g)
+    parts = cols.view(B, L1, L2, k2, k1, C).permute(0, 5, 4, 3, 1, 2)            # (B, C, k1, k2, L1, L2)
+    acc = torch.zeros(B, C, H, W)
+    for j1 in range(k1):
+        for j2 in range(k2):
+            acc[:, :, j1:j1 + (L1 - 1) * s1 + 1:s1, j2:j2 + (L2 - 1) * s2 + 1:s2] += parts[:, :, j1, j2]
+    back = mt.kernel.v4.col2im(cols.to(DEV), (B, C, H, W), k1, k2, s1, s2)
+    assert_bits_equal(back.cpu().numpy(), acc.numpy(), "col2im")

@@ -41,3 +41,27 @@ def test_ragged_rows(N, K, M, layout_mk, pad):
         assert_index_equal(got.cpu().numpy(), index, tag + " index")
         assert_bits_equal(x_sel[plane].cpu().numpy(), x.numpy()[rows, index], tag + " x_sel")
         assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
+
+
+@pytest.mark.parametrize("N,K,M", [(33, 64, 1), (5, 80, 63), (64, 288, 64), (31, 272, 65), (70, 2048, 129), (40, 4096, 192),
+                                   (65, 528, 257), (33, 64, 320), (200, 2064, 64)])
+def test_tiles_of_64_neurons(N, K, M):
+    """Aligned (M, K) weights around odd multiples of 64 neurons: one, two and four k tiles, a partial last one, split and
+    unsplit K."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(N + K + M)
+    x, w, bias = torch.randn(N, K, generator=g), torch.randn(M, K, generator=g), torch.randn(M, generator=g)
+    xd, wd = x.to(DEV), w.to(DEV)
+    w_sel, x_sel = torch.zeros(2, N, M, device=DEV), torch.zeros(2, N, M, device=DEV)
+    c, amax, amin = capi.fc_forward(xd, wd, capi.W_MK, bias.to(DEV), w_sel=w_sel, x_sel=x_sel)
+    values = capi.fc_forward_values(xd, wd, capi.W_MK, bias.to(DEV))
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, bias.numpy())
+    tag = "N %d K %d M %d" % (N, K, M)
+    assert_bits_equal(c.cpu().numpy(), want[0], tag + " c")
+    assert_bits_equal(values.cpu().numpy(), want[0], tag + " values-only c")
+    rows, cols = np.arange(N)[:, None], np.arange(M)[None, :]
+    for plane, (got, index) in enumerate(zip((amax, amin), want[1:3])):
+        assert_index_equal(got.cpu().numpy(), index, tag + " index")
+        assert_bits_equal(x_sel[plane].cpu().numpy(), x.numpy()[rows, index], tag + " x_sel")
+        assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
