@@ -216,3 +216,29 @@ def test_thresholds_of_product_and_count_scores_and_corner_cases():
     assert prune.layer_threshold(torch.tensor([[-3.5]], device=DEV), 0.7) == 3.5
     same = torch.full((64, 64), -0.25, device=DEV)
     assert prune.layer_threshold(same, 0.33) == 0.25 and prune.global_threshold([same, same], 0.99) == 0.25
+
+
+@pytest.mark.parametrize("M,K,pad", [(3, 5, 0), (6, 2730, 0), (64, 1027, 0), (1025, 1028, 0), (1025, 1028, 4), (66, 1001, 3),
+                                     (4100, 1024, 0)])
+@pytest.mark.parametrize("kind", ["normal", "equal", "two values", "counts"])
+def test_selection_over_gapless_and_strided_matrices(M, K, pad, kind):
+    """Matrices that are read as one row and such that are not, ends that leave part of a thread's loads, and scores that
+    all share a digit; ranks whose neighbours lie in one bin and in two."""
+    from mamtorch_amd.sparse import prune
+
+    g = torch.Generator().manual_seed(M + K)
+    w = torch.randn(M, K + pad, generator=g).to(DEV)
+    counts = None
+    if kind == "equal":
+        w.fill_(-0.375)
+    elif kind == "two values":
+        w = torch.where(w > 0, 3.0, -1e-3)
+    elif kind == "counts":
+        counts = torch.randint(0, 3000, (M, K + pad), generator=g, dtype=torch.int32).to(DEV)
+        counts[w > -0.5] = 0
+        counts = counts[:, :K]
+    w = w[:, :K]
+    ordered = _sorted_abs(w) if counts is None else torch.sort(counts.flatten().float())[0]
+    for p in (0.0, 0.31, 0.5, 0.9, 1.0):
+        got = prune.layer_threshold(w, p, counts=counts)
+        assert np.float32(got).view(np.int32) == np.float32(_quantile_by_sort(ordered, p)).view(np.int32), p
