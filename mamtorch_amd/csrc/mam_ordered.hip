@@ -976,9 +976,18 @@ static int list_cap(int64_t K)
     return (int)(ceil_div(cap, CHUNK) * CHUNK);
 }
 
+// Workgroups of build_kernel: a listed row each, and with a leading share the other rows and the tiles of the transpose.
+static int64_t build_items(int64_t N, int64_t K, int64_t M, bool two_sided)
+{
+    const int64_t longer = N > M ? N : M;
+    return two_sided ? N + M + ceil_div(longer, 64) * ceil_div(K, 64) : longer;
+}
+
 bool applies(int64_t N, int64_t K, int64_t M)
 {
-    if (tile_rows(K) == 0 || N * M * K <= 0 || M > (1 << 24)) return false;
+    if (tile_rows(K) == 0 || N * M * K <= 0) return false;
+    // A launch holds less than 2^32 threads: calls of more rows stay on the dense tilings.
+    if (build_items(N, K, M, true) > UINT32_MAX / BUILD_NT) return false;
     const int choice = option(MAM_OPT_FORWARD_TILING);
     if (choice == MAM_FORWARD_TILING_LISTS) return true;
     return choice == MAM_FORWARD_TILING_AUTO && K >= 128 && N >= 32 && M >= 32 && N * M >= MIN_PRODUCTS / K;
@@ -1073,14 +1082,12 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     hipLaunchKernelGGL(sample_kernel, dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
     int rc = check_launch("ordered::sample_kernel");
     if (rc != MAM_OK) return rc;
-    const int64_t longer = N > M ? N : M;
     if (p.turned_ld > 0) {
         hipLaunchKernelGGL(decide_kernel, dim3(1), dim3(64 * LEADS), 0, st, p);
         rc = check_launch("ordered::decide_kernel");
         if (rc != MAM_OK) return rc;
     }
-    const int64_t items = p.turned_ld > 0 ? N + M + ceil_div(longer, 64) * ceil_div(K, 64) : longer;
-    const dim3 build_grid((unsigned)items), build_block(BUILD_NT);
+    const dim3 build_grid((unsigned)build_items(N, K, M, p.turned_ld > 0)), build_block(BUILD_NT);
     const size_t lds = (size_t)p.cap * 8;
     if (K <= 4 * BUILD_NT) hipLaunchKernelGGL((build_kernel<4>), build_grid, build_block, lds, st, p);
     else if (K <= 8 * BUILD_NT) hipLaunchKernelGGL((build_kernel<8>), build_grid, build_block, lds, st, p);

@@ -34,6 +34,15 @@ def test_c_abi_exports_every_declared_symbol():
     assert capi.lib().mam_error_string(-3).decode() == "workspace missing or too small"
 
 
+@pytest.mark.parametrize("N, K, M", [(2 ** 24, 128, 64), (2 ** 24 - 64, 128, 64), (128 * 224 * 224 * 4, 160, 32)])
+def test_calls_of_more_rows_than_a_list_launch_holds_stay_on_the_dense_tilings(N, K, M):
+    # the lists are built by a workgroup of 256 threads per row, and a launch holds less than 2^32 threads
+    l = capi.lib()
+    assert l.mam_fc_forward_workspace_for(N, K, M, capi.W_MK, 1) == l.mam_fc_forward_workspace(N, K, M)
+    below = 2 ** 22
+    assert l.mam_fc_forward_workspace_for(below, K, M, capi.W_MK, 1) > l.mam_fc_forward_workspace(below, K, M)
+
+
 def test_workspace_queries_are_pure_host_calls():
     l = capi.lib()
     assert l.mam_fc_forward_workspace(12608, 768, 3072) == 0          # enough tiles: no split-K
