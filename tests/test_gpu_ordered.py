@@ -126,3 +126,31 @@ def test_two_sided_searches(N, K, M, kind_x):
     """Normal weights: the leading entries of one operand first, then a search bounded by what they leave."""
     _check(N, K, M, kind_x, "normal", seed=3)
     _check(N, K, M, "normal", kind_x, layout_mk=False, seed=4)
+
+
+def test_every_replay_of_a_graph_decides_anew():
+    """A captured call on data that suits the lists, then data that does not (dense kernels), then lists again."""
+    from mamtorch_amd import capi
+
+    N, K, M = 66, 520, 70
+    g = torch.Generator().manual_seed(6)
+    x, w = torch.zeros(N, K, device=DEV), torch.zeros(M, K, device=DEV)
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
+    try:
+        capi.fc_forward(x, w, capi.W_MK)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = capi.fc_forward(x, w, capi.W_MK)
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    for kinds in [("uniform", "uniform"), ("positive", "positive"), ("normal", "normal"), ("ties", "positive")]:
+        xs, ws = _data(kinds[0], N, K, g), _data(kinds[1], M, K, g)
+        x.copy_(xs)
+        w.copy_(ws)
+        graph.replay()
+        torch.cuda.synchronize()
+        want = oracle.forward(xs.numpy(), ws.numpy(), oracle.W_MK)
+        assert_bits_equal(out[0].cpu().numpy(), want[0], "%s x %s c" % kinds)
+        assert_index_equal(out[1].cpu().numpy(), want[1], "%s x %s argmax" % kinds)
+        assert_index_equal(out[2].cpu().numpy(), want[2], "%s x %s argmin" % kinds)
