@@ -936,7 +936,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                         f[j] = __int_as_float(index_in(kk[j]));
                     }
                     put(reinterpret_cast<float *>(side2 ? c.argmin : c.argmax), f);
-                    if (c.wsel) {
+                    if (c.wsel || c.xsel) {
                         // the selected operands, of the tile and of the listed row: from the list, which this
                         // XCD's L2 still holds, rather than from anywhere in the row (16384 x 4096 -> 1024: 593 ->
                         // 405 us, 12608 x 3072 -> 768: 345 -> 235 us)
@@ -950,8 +950,8 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                             sa[j] = *from;
                             sb[j] = by_key[(int)(kk[j] >> 16) * L::STRIDE + j];
                         }
-                        put(c.wsel + side2 * plane, lists_x ? sb : sa);
-                        put(c.xsel + side2 * plane, lists_x ? sa : sb);
+                        if (c.wsel) put(c.wsel + side2 * plane, lists_x ? sb : sa);
+                        if (c.xsel) put(c.xsel + side2 * plane, lists_x ? sa : sb);
                     }
                 }
             }

@@ -154,3 +154,27 @@ def test_every_replay_of_a_graph_decides_anew():
         assert_bits_equal(out[0].cpu().numpy(), want[0], "%s x %s c" % kinds)
         assert_index_equal(out[1].cpu().numpy(), want[1], "%s x %s argmax" % kinds)
         assert_index_equal(out[2].cpu().numpy(), want[2], "%s x %s argmin" % kinds)
+
+
+@pytest.mark.parametrize("side", ["normal", "uniform"])      # of x: its rows are searched, the rows of w are searched
+@pytest.mark.parametrize("keep", ["w_sel", "x_sel"])
+def test_either_hand_over_array_alone(side, keep):
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(7)
+    N, K, M = 640, 768, 616
+    x, w = _data(side, N, K, g), _data("uniform" if side == "normal" else "normal", M, K, g)
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK)
+    sel = torch.full((2, N, M), float("nan"), device=DEV)
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
+    try:
+        c, amax, amin = capi.fc_forward(x.to(DEV), w.to(DEV), capi.W_MK, **{keep: sel})
+        torch.cuda.synchronize()
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    assert_bits_equal(c.cpu().numpy(), want[0], "c")
+    assert_index_equal(amax.cpu().numpy(), want[1], "argmax")
+    assert_index_equal(amin.cpu().numpy(), want[2], "argmin")
+    for plane, index in enumerate(want[1:3]):
+        operand, rows = (x, np.arange(N)[:, None]) if keep == "x_sel" else (w, np.arange(M)[None, :])
+        assert_bits_equal(sel[plane].cpu().numpy(), operand.numpy()[rows, index], keep)
