@@ -209,10 +209,12 @@ def test_window_gather_operators():
 
 @pytest.mark.parametrize("B,C,H,W,k1,k2,s1,s2", [
     (2, 4, 5, 33, 3, 3, 1, 1), (1, 5, 7, 32, 2, 3, 2, 1), (2, 36, 6, 70, 3, 2, 1, 2), (1, 32, 9, 9, 9, 9, 1, 1),
-    (3, 1, 4, 40, 1, 1, 3, 3), (1, 8, 12, 300, 5, 40, 1, 3), (2, 65, 5, 34, 4, 3, 1, 1)])
+    (3, 1, 4, 40, 1, 1, 3, 3), (1, 8, 12, 300, 5, 40, 1, 3), (2, 65, 5, 34, 4, 3, 1, 1),
+    (2, 3, 35, 70, 16, 16, 16, 16), (1, 8, 20, 37, 7, 7, 2, 2), (2, 4, 23, 47, 3, 11, 5, 4), (1, 12, 11, 66, 2, 2, 3, 4), (2, 8, 8, 8, 8, 8, 1, 1)])
 def test_windows_and_their_adjoint(B, C, H, W, k1, k2, s1, s2):
     """Window gather and adjoint at the edges of their 32-channel, 32-column tiles, with and without 16-byte rows and
-    with input rows that do not fit the staged kernel: the gather exactly, the adjoint in ascending window order."""
+    with input rows that do not fit the staged kernel, strides below, at and above the window size: the gather exactly, the
+    adjoint in ascending window order."""
     g = torch.Generator().manual_seed(C * W)
     x = torch.randn(B, C, H, W, generator=g)
     L1, L2 = (H - k1) // s1 + 1, (W - k2) // s2 + 1
