@@ -844,7 +844,7 @@ constexpr int KT = 64;    // k extent of one W tile
 constexpr int CHUNKS = KT / 4;    // 16-byte chunks per neuron and tile
 constexpr int RPB = 64 / KT < 1 ? 1 : 64 / KT;   // neurons per 256 bytes of LDS (all 64 banks)
 // TJ = neurons per lane.  2 (128 neurons per workgroup) is what the launch uses unless half of the last tile would be
-// empty (Plan::narrow).  Measured at the
+// empty (narrow_tiles_pay).  Measured at the
 // 256 x 4096 x 4096 shape: 1 (64 neurons per workgroup, 512 tiles, no split of K and no merge) 0.226 ms
 // against 0.217 ms for 2 with K split in two plus the merge -- the k loop with one neuron per lane is 7 %
 // slower (twice the scalar loads per product), which costs more than the merge; 4 with 32-k tiles: the
@@ -1267,6 +1267,26 @@ struct Plan {
     size_t tickets_at;    // offset of the tickets
 };
 
+// Whether the wave-uniform-rows tiling takes 64 neurons per workgroup.  Half of the last 128-neuron tile is work for
+// neurons that are not there when M is an odd multiple of 64 (or little less): with 1, 3 or 5 of them that is 50, 25 or
+// 17 % of the call, against 7 % that a product costs more in a 64-neuron tile.  More tiles also split K less and can
+// end in a round that is nearly empty, so what decides is the rounds of workgroups (two per CU) times the k of each
+// ((N, K, M), with indices, 128 / 64 neurons per tile: 21632 x 288 -> 64 82 / 51 us, 12608 x 768 -> 192 188 / 137,
+// 12608 x 768 -> 320 238 / 208; 2048 x 2048 -> 192, 576 workgroups of 704 k instead of 512 of 512 k, 67 / 85; 256 x 4096
+// -> 320 42 / 45).
+static bool narrow_tiles_pay(int64_t N, int64_t K, int64_t M, int64_t range_len)
+{
+    const int64_t m64 = ceil_div(M, 64);
+    if (m64 % 2 == 0 || m64 > 5) return false;
+    auto length = [&](int bm, float per_k) {
+        int64_t k = range_len < K ? range_len : K;
+        if (range_len <= 0) k = ceil_div(ceil_div(K, choose_splits(N, K, M, sx::BN, bm)), sx::KT) * sx::KT;
+        const int64_t blocks = ceil_div(N, sx::BN) * ceil_div(M, bm) * ceil_div(K, k);
+        return (float)ceil_div(blocks, 2 * num_cus()) * (float)k * per_k;
+    };
+    return length(sx::Cfg<1>::BM, 1.07f) < length(sx::BM_MAX, 2.0f);
+}
+
 static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                      const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel, float *x_sel,
                      int64_t N, int64_t K, int64_t M, int64_t range_len = 0)
@@ -1296,11 +1316,7 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
                         (range_len % sx::KT == 0) && (ldw * sx::BM_MAX < (1ll << 30)) &&
                         option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
     plan.use_sx = use_sx;
-    // Half of the last 128-neuron tile is work for neurons that are not there when M is an odd multiple of 64 (or
-    // little less): with 1, 3 or 5 of them that is 50, 25 or 17 % of the call, against 7 % that a product costs more
-    // in a 64-neuron tile (21632 x 288 -> 64: 92 us with 128 neurons per tile, 54 us with 64).
-    const int64_t m64 = ceil_div(M, 64);
-    plan.narrow = use_sx && m64 % 2 == 1 && m64 <= 5 && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_FUSED_MERGE;
+    plan.narrow = use_sx && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_FUSED_MERGE && narrow_tiles_pay(N, K, M, range_len);
     const int bn = use_sx ? sx::BN : BN, bm = use_sx ? (plan.narrow ? sx::Cfg<1>::BM : sx::BM_MAX) : BM;
     p.tiles_n = (int)ceil_div(N, bn);
     p.tiles_m = (int)ceil_div(M, bm);

@@ -43,6 +43,17 @@ def test_calls_of_more_rows_than_a_list_launch_holds_stay_on_the_dense_tilings(N
     assert l.mam_fc_forward_workspace_for(below, K, M, capi.W_MK, 1) > l.mam_fc_forward_workspace(below, K, M)
 
 
+@pytest.mark.parametrize("N, K, M, neurons", [
+    (21632, 288, 64, 64), (12608, 768, 192, 64), (2048, 2048, 320, 64), (256, 4096, 192, 64), (1024, 512, 320, 64),
+    (2048, 2048, 192, 128), (2048, 2048, 180, 128), (256, 4096, 320, 128), (12608, 768, 256, 128), (12608, 768, 448, 128)])
+def test_neurons_per_tile_follow_the_rounds_of_workgroups(N, K, M, neurons):
+    # 64 neurons per tile only where they end sooner than 128 (on 256 compute units)
+    text = ctypes.create_string_buffer(400)
+    one = ctypes.c_void_p(256)
+    assert capi.lib().mam_fc_forward_describe(one, K, one, K, capi.W_MK, N, K, M, 1, text, 400) == 0
+    assert b"tiles of 32 x %d" % neurons in text.value, text.value
+
+
 def test_workspace_queries_are_pure_host_calls():
     l = capi.lib()
     assert l.mam_fc_forward_workspace(12608, 768, 3072) == 0          # enough tiles: no split-K
