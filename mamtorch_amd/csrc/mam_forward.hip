@@ -1390,12 +1390,22 @@ static bool transposed_operand_pays(int64_t N, int64_t K, int64_t M)
     return N >= 16 && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
 }
 
-// Whether to lengthen ragged rows: one launch that reads and writes both operands once, against the general tiling, at
-// every size measured ((N, K, M): 1 x 4001 x 4096 100 / 61 us, 16 x 1001 x 512 47 / 22, 250 x 1001 x 517 69 / 32, 1000 x 777 x
-// 1000 187 / 74, 4000 x 531 x 3712 1597 / 571; values only 69 / 55, 35 / 18, 39 / 24, 75 / 50, 466 / 361).
-static bool lengthened_rows_pay(int64_t N, int64_t M)
+// Whether to lengthen ragged rows: one launch more, which reads and writes both operands once, against the general tiling.
+// With indices nearly everywhere ((N, K, M): 1 x 4001 x 4096 100 / 61 us, 16 x 1001 x 512 47 / 22, 250 x 1001 x 517 69 / 32,
+// 4000 x 531 x 3712 1597 / 571, 500 x 17 x 500 100 / 24; not for 4 x 63 x 10, 18.8 / 21.7, and 16 x 24 x 64 by (K, M),
+// 20.3 / 23.6).  Values only, the general tiling pads K to 32 where the copies pad it to 64 and has no copy to make:
+// from K = 256 on (4000 x 531 x 3712 466 / 361, 250 x 1001 x 517 39 / 24), from 128 on where both pad it alike (30000 x 250
+// x 60 58 / 49, but 4000 x 200 x 1000 52 / 57), below that for calls that leave it most of the chip idle (64 x 100 x 100
+// 25 / 16; 4000 x 130 x 1000 42 / 45, 30000 x 31 x 60 14 / 32).
+static bool lengthened_rows_pay(int64_t N, int64_t K, int64_t M, bool turn, bool args)
 {
-    return N + M <= 65535 && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
+    if (N + M > 65535 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
+    if (K >= 256) return true;
+    const int64_t outputs = N * M;
+    if (args) return K >= 64 || (outputs >= 16384 ? K > 4 || N >= 64 : outputs >= 1000 && K > (turn ? 32 : 16));
+    if (K >= 128 && (K - 1) % sx::KT >= KT) return true;
+    if (K >= 64) return outputs <= (1 << 20) && (K >= 96 || turn || N + M < 8192);
+    return K > 32 && !turn && N >= 64 && outputs >= 16384 && outputs <= (1 << 18);
 }
 
 // The plan of a call on staged operands, for a call that the wave-uniform-rows tiling does not take as it is; false:
@@ -1409,7 +1419,7 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
     st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M);
     const bool lengthen = st.x || (st.w && !turn);
     if (turn && !transposed_operand_pays(N, K, M)) return false;
-    if (lengthen && (!lengthened_rows_pay(N, M) || range_len > 0)) return false;
+    if (lengthen && (!lengthened_rows_pay(N, K, M, turn, args) || range_len > 0)) return false;
     float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
     const int rc = make_plan(staged, args, st.x ? aligned : x, st.x ? st.K : ldx, st.w ? aligned : w, st.w ? st.K : ldw, MAM_W_MK, bias,
                              c, argmax, argmin, w_sel, x_sel, N, st.K, M, range_len);
@@ -1574,7 +1584,7 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     size_t bytes = mam::fwd::workspace_bytes(N, K, M, with_indices != 0);
     // room for staged operands (see launch); without it the call still works
     const bool turn = w_layout == MAM_W_KM, ragged = K % mam::fwd::G != 0;
-    if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || mam::fwd::lengthened_rows_pay(N, M)))
+    if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0)))
         bytes += mam::fwd::staging_of(true, !turn, N, K, M).bytes();
     if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M);
     return bytes;

@@ -54,6 +54,23 @@ def test_neurons_per_tile_follow_the_rounds_of_workgroups(N, K, M, neurons):
     assert b"tiles of 32 x %d" % neurons in text.value, text.value
 
 
+@pytest.mark.parametrize("N, K, M, with_indices, mk, copied", [
+    (250, 1001, 517, 1, 1, True), (250, 1001, 517, 0, 1, True), (250, 1001, 517, 0, 0, True), (500, 17, 500, 1, 1, True),
+    (4, 63, 10, 1, 1, False), (16, 24, 64, 1, 0, False), (16, 33, 64, 1, 0, True), (30000, 31, 60, 0, 1, False),
+    (30000, 31, 60, 1, 1, True), (4000, 130, 1000, 0, 1, False), (4000, 130, 1000, 0, 0, False), (64, 100, 100, 0, 1, True)])
+def test_ragged_rows_are_lengthened_where_the_copy_pays(N, K, M, with_indices, mk, copied):
+    l = capi.lib()
+    text = ctypes.create_string_buffer(400)
+    one = ctypes.c_void_p(256)
+    layout = capi.W_MK if mk else capi.W_KM
+    assert l.mam_fc_forward_describe(one, K, one, K if mk else M, layout, N, K, M, with_indices, text, 400) == 0
+    assert (b"lengthen_rows_kernel" in text.value) == copied, text.value
+    # the workspace query asks for the copies of the operands exactly where they are made
+    need = (l.mam_fc_forward_workspace if with_indices else l.mam_fc_forward_values_workspace)(N, K, M)
+    copies = l.mam_fc_forward_workspace_for(N, K, M, layout, with_indices) - need
+    assert (copies >= 4 * (N + M) * K) if copied else copies == 0
+
+
 def test_workspace_queries_are_pure_host_calls():
     l = capi.lib()
     assert l.mam_fc_forward_workspace(12608, 768, 3072) == 0          # enough tiles: no split-K
