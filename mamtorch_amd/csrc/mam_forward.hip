@@ -1457,16 +1457,25 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     if (!x || !w || !c || (ARGS && (!argmax || !argmin)))
         return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     const size_t avail = static_scratch ? static_scratch_bytes() : (workspace ? workspace_size : (size_t)0);
-    // Where the workspace has room, operands that the wave-uniform-rows tiling does not take are staged in it (see
-    // Staging): every output is the same, bit for bit.
+    // Large calls go by magnitude-ordered lists where the workspace has room for them (the kernels below then run only if
+    // the data turns out not to suit the lists), and operands that the wave-uniform-rows tiling does not take are staged
+    // in it (see Staging): every output is the same, bit for bit.  The lists come first: they lie at the start of the workspace and
+    // take the operands as they are, so the copies get what is left.
     const int operand_layout = w_layout;
     const int64_t operand_K = K;
-    size_t wt_bytes = 0;
-    Staging stage = {false, false, K, 0, 0};
+    const bool on_16 = static_scratch || (uintptr_t)workspace % 16 == 0;
     Plan tplan;
-    Staging st_plan;
-    if (staged_plan(tplan, st_plan, plan, ARGS, x, ldx, w, ldw, w_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M, range_len) &&
-        st_plan.bytes() + tplan.need <= avail && (static_scratch || (uintptr_t)workspace % 16 == 0)) {
+    Staging stage = {false, false, K, 0, 0}, st_plan;
+    const bool can_stage = on_16 && staged_plan(tplan, st_plan, plan, ARGS, x, ldx, w, ldw, w_layout, bias, c, argmax, argmin, w_sel,
+                                                x_sel, N, K, M, range_len);
+    const size_t staged_need = can_stage ? st_plan.bytes() + tplan.need : 0;
+    size_t list_bytes = 0;
+    if (range_len == 0 && !static_scratch && on_16 && ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22))) {
+        list_bytes = ordered::workspace_bytes(N, K, M);
+        if (list_bytes + (can_stage && staged_need < plan.need ? staged_need : plan.need) > avail) list_bytes = 0;
+    }
+    size_t wt_bytes = 0;
+    if (can_stage && list_bytes + staged_need <= avail) {
         plan = tplan;
         stage = st_plan;
         wt_bytes = stage.bytes();
@@ -1491,7 +1500,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     if (nblk > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "too many tiles");
     const int dev = ensure_device(static_cast<hipStream_t>(stream));
     if (dev < 0) return dev;
-    char *scratch_base = static_cast<char *>(workspace);
+    char *scratch_base = static_cast<char *>(workspace) + list_bytes;
     if (static_scratch && wt_bytes + need > 0) {
         scratch_base = static_cast<char *>(static_scratch_of(dev));
         if (!scratch_base) return fail(MAM_ERR_LAUNCH, "the built-in scratch array has no device address");
@@ -1507,15 +1516,10 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
         rc = fill_zero(p.tickets, (int64_t)p.tiles_n * p.tiles_m, st);
         if (rc != MAM_OK) return rc;
     }
-    // Large calls by magnitude-ordered lists, where the workspace has room for them; the kernels below then run
-    // only if the data turns out not to suit the lists.
-    if (range_len == 0 && !static_scratch && ordered::applies(N, operand_K, M) && (operand_layout == MAM_W_MK || ldw < (1 << 22))) {
-        const size_t at = (wt_bytes + need + 255) / 256 * 256;
-        if (avail >= at + ordered::workspace_bytes(N, operand_K, M) && (uintptr_t)workspace % 16 == 0) {
-            const ordered::Call call = {x, ldx, w, ldw, operand_layout, bias, c, argmax, argmin, w_sel, x_sel, N, operand_K, M};
-            rc = ordered::launch(call, scratch_base + at, p.guard, st);
-            if (rc != MAM_OK) return rc;
-        }
+    if (list_bytes > 0) {
+        const ordered::Call call = {x, ldx, w, ldw, operand_layout, bias, c, argmax, argmin, w_sel, x_sel, N, operand_K, M};
+        rc = ordered::launch(call, workspace, p.guard, st);
+        if (rc != MAM_OK) return rc;
     }
     if (wt_bytes > 0) {
         float *const ws = reinterpret_cast<float *>(scratch_base), *const xs = reinterpret_cast<float *>(scratch_base + stage.w_bytes);

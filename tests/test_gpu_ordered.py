@@ -68,6 +68,27 @@ def _check(N, K, M, kind_x, kind_w, layout_mk=True, pad=0, seed=0):
         assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
 
 
+def _by_lists(xd, wd, layout, bias=None, indices=True, w_sel=None, x_sel=None):
+    """A call with the lists allowed at every size: its outputs, and what the device decided -- (side, leading entries, entries
+    per list), side 0: the dense kernels, 1: rows of x are searched, 2: rows of w -- which lies at the start of the workspace."""
+    from mamtorch_amd import capi
+
+    N, K = xd.shape
+    M = wd.shape[0] if layout == capi.W_MK else wd.shape[1]
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
+    try:
+        need = capi.lib().mam_fc_forward_workspace_for(N, K, M, layout, int(indices))
+        ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
+        if indices:
+            out = capi.fc_forward(xd, wd, layout, bias, workspace=ws, w_sel=w_sel, x_sel=x_sel)
+        else:
+            out = (capi.fc_forward_values(xd, wd, layout, bias, workspace=ws),)
+        torch.cuda.synchronize()
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    return out, ws[:12].view(torch.int32).tolist()
+
+
 def _strided(x, pad):
     N, K = x.shape
     out = torch.zeros(N, K + pad, device=DEV)[:, :K]
@@ -178,3 +199,20 @@ def test_either_hand_over_array_alone(side, keep):
     for plane, index in enumerate(want[1:3]):
         operand, rows = (x, np.arange(N)[:, None]) if keep == "x_sel" else (w, np.arange(M)[None, :])
         assert_bits_equal(sel[plane].cpu().numpy(), operand.numpy()[rows, index], keep)
+
+
+@pytest.mark.parametrize("indices", [True, False])
+@pytest.mark.parametrize("pad, offset", [(3, 0), (4, 1)])
+def test_rows_that_are_not_aligned_go_by_lists(indices, pad, offset):
+    """The copies that the dense tiling would make of such operands do not take the lists' room."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(8)
+    N, K, M = 640, 768, 616
+    x, w = torch.randn(N, K + pad, generator=g), torch.rand(M, K, generator=g) * 2 - 1
+    want = oracle.forward(x[:, offset:offset + K].contiguous().numpy(), w.numpy(), oracle.W_MK)
+    out, (side, lead, _) = _by_lists(x.to(DEV)[:, offset:offset + K], w.to(DEV), capi.W_MK, indices=indices)
+    assert (side, lead) == (1, 0)
+    assert_bits_equal(out[0].cpu().numpy(), want[0], "c")
+    for got, expected in zip(out[1:], want[1:]):
+        assert_index_equal(got.cpu().numpy(), expected, "index")
