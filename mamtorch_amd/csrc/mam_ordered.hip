@@ -258,10 +258,12 @@ __device__ __forceinline__ int nth_largest(int v, int rank)
 
 // The cheapest option, by all waves of a workgroup.  In units of one product of a dense kernel per output (12608 x 768 x
 // 3072: 2.25 us): a searched product costs 3.5, a leading one 6, a wave's slowest output needs ~1.3 times what 95 % of
-// the samples need; the launches, outputs and lists cost 0.15 K, a leading share passes over both operands.  The dense
-// kernels cost K.
+// the samples need; the launches, outputs and lists cost 0.15 K, a leading share passes over both operands.  Outputs that no list
+// finishes (a sampled need beyond the longest list) cost SCAN a product over the whole row, and their waves a whole list first; four
+// such samples of 64 need too much by the rule above.  The dense kernels cost K.
+constexpr float SCAN = 5.0f;
 template <int WAVES>
-__device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTIONS], int (&long_s)[OPTIONS])
+__device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTIONS], int (&length_s)[OPTIONS])
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -274,12 +276,18 @@ __device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTI
         const bool possible = (!two_sided || lead > 0) && (p.call.w_layout == MAM_W_MK || (search_x && !two_sided));
         const int v = p.samples[o * SAMPLES + lane];
         const float tiled = (float)(search_x ? p.call.M : p.call.N), listed = (float)(search_x ? p.call.N : p.call.M);
-        float cost = 0.15f * K + 3.5f * 1.3f * (float)nth_largest(v, 4);
+        // entries written per list: twice the longest sampled need and 64 more, so that hardly any of the outputs that
+        // are finished one by one need more than their list; needs that no list meets do not count
+        const int want = (nth_largest(v <= p.cap ? v : 0, 2) * 2 + 64 + CHUNK - 1) / CHUNK * CHUNK;
+        const int length = want < p.cap ? want : p.cap;
+        const int beyond = __popcll(__ballot(v > p.cap));
+        float searched = 1.3f * (float)nth_largest(v, 4);
+        if (beyond > 0 && searched < (float)length) searched = (float)length;
+        float cost = 0.15f * K + 3.5f * searched + SCAN * K * (float)beyond / SAMPLES;
         if (two_sided) cost += 6.0f * (float)lead + K * (36.0f / tiled + 18.0f / listed);
-        const int longest = nth_largest(v, 2);
         if (lane == 0) {
             cost_s[o] = possible ? cost : 1e30f;
-            long_s[o] = longest;
+            length_s[o] = length;
         }
     }
     __syncthreads();
@@ -289,10 +297,7 @@ __device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTI
     Decision d;
     d.side = cost_s[best] < 0.95f * K ? (best < LEADS ? SIDE_X : SIDE_W) : SIDE_NONE;
     d.lead = lead_entries(best, (int)p.call.K);
-    // entries written per list: twice the longest sampled need and 64 more, so that hardly any of the outputs that
-    // are finished one by one need more than their list (64 entries more of it: 1 us; the full scan: ~20 us)
-    const int want = (long_s[best] * 2 + 64 + CHUNK - 1) / CHUNK * CHUNK;
-    d.length = want < p.cap ? want : p.cap;
+    d.length = length_s[best];
     d.pad = 0;
     return d;
 }
@@ -302,8 +307,8 @@ __device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTI
 __global__ __launch_bounds__(64 * LEADS) void decide_kernel(const Params p)
 {
     __shared__ float cost_s[OPTIONS];
-    __shared__ int long_s[OPTIONS];
-    const Decision d = decide<LEADS>(p, cost_s, long_s);
+    __shared__ int length_s[OPTIONS];
+    const Decision d = decide<LEADS>(p, cost_s, length_s);
     if (threadIdx.x == 0) *p.decision = d;
 }
 
@@ -435,12 +440,12 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
     __shared__ float turn[64][65];
     __shared__ float cost_s[OPTIONS];
-    __shared__ int long_s[OPTIONS];
+    __shared__ int length_s[OPTIONS];
     Decision d;
     if (p.turned_ld > 0) {
         d = *p.decision;
     } else {
-        d = decide<BUILD_NT / 64>(p, cost_s, long_s);
+        d = decide<BUILD_NT / 64>(p, cost_s, length_s);
         d.side = __builtin_amdgcn_readfirstlane(d.side);
         d.length = __builtin_amdgcn_readfirstlane(d.length);
         d.lead = 0;
@@ -486,11 +491,15 @@ __device__ __forceinline__ uint32_t key_of(double d) { return (uint32_t)__builti
 // (the builtins would canonicalise their operands first: one more instruction each)
 __device__ __forceinline__ void max64(double &a, double b) { asm("v_max_f64 %0, %0, %1" : "+v"(a) : "v"(b)); }
 __device__ __forceinline__ void min64(double &a, double b) { asm("v_min_f64 %0, %0, %1" : "+v"(a) : "v"(b)); }
-__device__ __forceinline__ double shfl_xor64(double d, int s)
+__device__ __forceinline__ double lane_value_at(double d, int from)      // from: lane * 4, of each lane its own
 {
     const uint64_t b = __builtin_bit_cast(uint64_t, d);
-    const uint32_t lo = __shfl_xor((uint32_t)b, s), hi = __shfl_xor((uint32_t)(b >> 32), s);
+    const uint32_t lo = __builtin_amdgcn_ds_bpermute(from, (uint32_t)b), hi = __builtin_amdgcn_ds_bpermute(from, (uint32_t)(b >> 32));
     return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ float lane_value_at(float v, int from)
+{
+    return __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(v)));
 }
 __device__ __forceinline__ double lane_value(double d, int l)
 {
@@ -521,10 +530,10 @@ struct Extremes<true> {
         max64(a, d);
         min64(b, d);
     }
-    static __device__ __forceinline__ void merge(value &a, value &b, int s)
+    static __device__ __forceinline__ void merge(value &a, value &b, int from)
     {
-        max64(a, shfl_xor64(a, s));
-        min64(b, shfl_xor64(b, s));
+        max64(a, lane_value_at(a, from));
+        min64(b, lane_value_at(b, from));
     }
     // one pair of list entries against 4 tile values each.  Written out because the compiler copies the key into the low
     // word of every key: here two register pairs hold it for the four products of an entry.
@@ -562,10 +571,10 @@ struct Extremes<false> {
         a = __builtin_fmaxf(a, product);
         b = __builtin_fminf(b, product);
     }
-    static __device__ __forceinline__ void merge(value &a, value &b, int s)
+    static __device__ __forceinline__ void merge(value &a, value &b, int from)
     {
-        a = __builtin_fmaxf(a, __shfl_xor(a, s));
-        b = __builtin_fminf(b, __shfl_xor(b, s));
+        a = __builtin_fmaxf(a, lane_value_at(a, from));
+        b = __builtin_fminf(b, lane_value_at(b, from));
     }
     __device__ __forceinline__ void entries(const uint4 &it, const float4 &w0, const float4 &w1)
     {
@@ -580,13 +589,11 @@ struct Extremes<false> {
     }
 };
 
-// One output by the whole wave: first the rest of its list, 64 entries at a time, then (the list is not enough,
-// or the row or the tile column holds what no bound covers: NaN, infinity, a zero extreme) every k, in the exact
-// terms of the ascending scan with ordered strict compares.
+// One output by the whole wave over the rest of its list, 64 entries at a time; whether its bound finished it.
 //   column: the output's column of the tile, by 65535 - k; at: chunks already searched; bmax: bound on the tile column
 template <int STRIDE, class E>
-__device__ __forceinline__ void finish_one(const Params &p, bool sx, const Rows &a, int row, const float *column, int at, int chunks,
-                                           float bmax, int lane, typename E::value &mx, typename E::value &mn)
+__device__ __forceinline__ bool finish_by_list(const Params &p, bool sx, int row, const float *column, int at, int chunks, float bmax,
+                                               int lane, typename E::value &mx, typename E::value &mn)
 {
     const uint4 *lists = sx ? p.lists_x : p.lists_w;
     const float *bound = sx ? p.bound_x : p.bound_w;
@@ -600,38 +607,122 @@ __device__ __forceinline__ void finish_one(const Params &p, bool sx, const Rows 
             E::both(mx, mn, __uint_as_float(it.x) * column[(int)(it.y >> 16) * STRIDE], it.y);
         }
 #pragma unroll
-        for (int s = 32; s > 0; s >>= 1) E::merge(mx, mn, s);
-        if (E::product(mx) > u && E::product(mn) < -u) return;
+        for (int s = 32; s > 0; s >>= 1) E::merge(mx, mn, (lane ^ s) << 2);
+        if (E::product(mx) > u && E::product(mn) < -u) return true;
     }
-    float hi = -__builtin_inff(), lo = __builtin_inff();
-    int ih = INT32_MAX, il = INT32_MAX;
-    const int K = (int)p.call.K;
-    const float *src = a.at(row, 0);
-    for (int k0 = 0; k0 < K; k0 += 64 * 8) {
-        float v[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int k = k0 + i * 64 + lane;
-            v[i] = src[(k < K ? k : K - 1) * a.k_stride];
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int past = k0 + i * 64 + lane, k = past < K ? past : K - 1;     // past the end the last k again
-            const float q = v[i] * column[(65535 - k) * STRIDE];
-            if (q > hi) { hi = q; ih = k; }
-            if (q < lo) { lo = q; il = k; }
-        }
+    return false;
+}
+
+// What a list does not finish (it is too short, or the row or a tile column holds what no bound covers: NaN, infinity, a zero
+// extreme) is scanned over every k, in the exact terms of the ascending scan with ordered strict compares.
+struct Scan {
+    float hi, lo;
+    int ih, il;
+    __device__ __forceinline__ void clear()
+    {
+        hi = -__builtin_inff();
+        lo = __builtin_inff();
+        ih = il = INT32_MAX;
     }
-#pragma unroll
-    for (int s = 32; s > 0; s >>= 1) {
-        const float oh = __shfl_xor(hi, s), ol = __shfl_xor(lo, s);
-        const int jh = __shfl_xor(ih, s), jl = __shfl_xor(il, s);
+    __device__ __forceinline__ void take(float q, int k)
+    {
+        if (q > hi) { hi = q; ih = k; }
+        if (q < lo) { lo = q; il = k; }
+    }
+    __device__ __forceinline__ void merge(int from)         // with another lane's
+    {
+        const float oh = lane_value_at(hi, from), ol = lane_value_at(lo, from);
+        const int jh = __builtin_amdgcn_ds_bpermute(from, ih), jl = __builtin_amdgcn_ds_bpermute(from, il);
         if (oh > hi || (oh == hi && jh < ih)) { hi = oh; ih = jh; }
         if (ol < lo || (ol == lo && jl < il)) { lo = ol; il = jl; }
     }
     // an extreme that was never improved keeps the first k
-    mx = E::make(hi, ih == INT32_MAX ? 0 : ih);
-    mn = E::make(lo, il == INT32_MAX ? 0 : il);
+    template <class E>
+    __device__ __forceinline__ void give(typename E::value &mx, typename E::value &mn) const
+    {
+        mx = E::make(hi, ih == INT32_MAX ? 0 : ih);
+        mn = E::make(lo, il == INT32_MAX ? 0 : il);
+    }
+};
+
+// One output by the whole wave, a lane every 64th k; column as in finish_by_list.
+template <int STRIDE, class E>
+__device__ __forceinline__ void scan_one(const float *src, int K, const float *column, int lane, typename E::value &mx,
+                                         typename E::value &mn)
+{
+    constexpr int AHEAD = 8;
+    Scan r;
+    r.clear();
+    for (int k0 = 0; k0 < K; k0 += 64 * AHEAD) {
+        float v[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int k = k0 + i * 64 + lane;
+            v[i] = src[(uint32_t)(k < K ? k : K - 1)];
+        }
+#pragma unroll
+        for (int i = 0; i < AHEAD; ++i) {
+            const int past = k0 + i * 64 + lane, k = past < K ? past : K - 1;     // past the end the last k again
+            r.take(v[i] * column[(65535 - k) * STRIDE], k);
+        }
+    }
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) r.merge((lane ^ s) << 2);
+    r.give<E>(mx, mn);
+}
+
+// The outputs of one searched row, all columns of the tile, by the whole wave.  A lane takes every RWth k of two columns of its
+// own quad (four would cost the search registers); bound by instruction issue, ~35 per k and two columns.  On return each lane
+// holds the outputs of its columns.  As many instructions per output as scan_one, but the tile is read contiguously where that one
+// reads 4 bytes of every row of it (forward call with 4 % of the rows all +-1, anywhere / next to each other, scan_one and scan_row and dense: 3707 /
+// 1595 and 1620 / 1542 and 1680 us at 12608 x 768 -> 3072, 3466 / 11189 and 1716 / 1560 and 3110 us at 16384 x 4096 -> 1024).
+//   src: the row, contiguous; by_key: the lane's columns of the tile, by 65535 - k
+template <int STRIDE, int RW, int LANE_STEP, class E>
+__device__ __forceinline__ void scan_row(const float *src, int K, const float *by_key, int lane, int slice, typename E::value (&mx)[2],
+                                         typename E::value (&mn)[2])
+{
+    constexpr int AHEAD = 4, STEP = AHEAD * RW;
+    Scan r[2];
+    r[0].clear();
+    r[1].clear();
+    const char *const end = reinterpret_cast<const char *>(by_key + 65535 * STRIDE);      // k = 0
+    auto k_of = [&](int k0, int u) {            // (past the end of the row the last k again)
+        const int k = k0 + u * RW + slice;
+        return k < K ? k : K - 1;
+    };
+    auto fetch = [&](float (&v)[AHEAD], int k0) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) v[u] = src[(uint32_t)k_of(k0, u)];
+        asm volatile("" ::: "memory");          // the loads stay ahead of the arithmetic
+    };
+    auto products = [&](const float (&v)[AHEAD], int k0) {
+        float2 w[AHEAD];
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) w[u] = *reinterpret_cast<const float2 *>(end - __mul24(k_of(k0, u), STRIDE * 4));
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const float f[2] = {w[u].x, w[u].y};
+            const int k = k_of(k0, u);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) r[j].take(v[u] * f[j], k);
+        }
+    };
+    float first[AHEAD], second[AHEAD];
+    fetch(first, 0);
+#pragma unroll 1
+    for (int k0 = 0; k0 < K; k0 += 2 * STEP) {
+        fetch(second, k0 + STEP);
+        products(first, k0);
+        if (k0 + STEP >= K) break;
+        fetch(first, k0 + 2 * STEP);
+        products(second, k0 + STEP);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int s = LANE_STEP; s < LANE_STEP * RW; s <<= 1) r[j].merge((lane ^ s) << 2);
+        r[j].give<E>(mx[j], mn[j]);
+    }
 }
 
 // A workgroup holds a tile of TB rows of the other operand in LDS, whole rows, as [K - 1 - k][TB] (a key's upper half
@@ -873,20 +964,65 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                 if (step(second, first)) break;
             }
         }
+        // the rows past the end are copies of the last one
+#pragma unroll
+        for (int j = 0; j < 4; ++j) open[j] &= __ballot(arow < a.rows);
+        int own = lane;
+        asm volatile("" : "+v"(own));           // what is derived from it below is not kept in registers during the search
+        // (one copy of the code each: the output's state is picked by selects)
+        if (ch < chunks) {
+            uint64_t todo[4] = {open[0], open[1], open[2], open[3]};
+            while (todo[0] | todo[1] | todo[2] | todo[3]) {
+                const int j = todo[0] ? 0 : todo[1] ? 1 : todo[2] ? 2 : 3;
+                const int l = __builtin_ctzll(todo[0] ? todo[0] : todo[1] ? todo[1] : todo[2] ? todo[2] : todo[3]);
+                typename E::value fx = lane_value(j == 0 ? e.mx[0] : j == 1 ? e.mx[1] : j == 2 ? e.mx[2] : e.mx[3], l);
+                typename E::value fn = lane_value(j == 0 ? e.mn[0] : j == 1 ? e.mn[1] : j == 2 ? e.mn[2] : e.mn[3], l);
+                const float bm = lane_value(j == 0 ? bmax[0] : j == 1 ? bmax[1] : j == 2 ? bmax[2] : bmax[3], l);
+                const bool done = finish_by_list<L::STRIDE, E>(p, lists_x, __builtin_amdgcn_readlane(row, l),
+                                                               tile + L::base(L::quad(l), K) + (K - 65536) * L::STRIDE + j, ch, chunks, bm,
+                                                               own, fx, fn);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i == j) {
+                        todo[i] &= todo[i] - 1;
+                        if (done) open[i] &= ~(1ull << l);
+                        if (own == l) { e.mx[i] = fx; e.mn[i] = fn; }
+                    }
+            }
+        }
         while (open[0] | open[1] | open[2] | open[3]) {
-            // (one copy of the code: the output's state is picked by selects)
             const int j = open[0] ? 0 : open[1] ? 1 : open[2] ? 2 : 3;
             const int l = __builtin_ctzll(open[0] ? open[0] : open[1] ? open[1] : open[2] ? open[2] : open[3]);
-            typename E::value fx = lane_value(j == 0 ? e.mx[0] : j == 1 ? e.mx[1] : j == 2 ? e.mx[2] : e.mx[3], l);
-            typename E::value fn = lane_value(j == 0 ? e.mn[0] : j == 1 ? e.mn[1] : j == 2 ? e.mn[2] : e.mn[3], l);
-            const float bm = lane_value(j == 0 ? bmax[0] : j == 1 ? bmax[1] : j == 2 ? bmax[2] : bmax[3], l);
-            finish_one<L::STRIDE, E>(p, lists_x, a, __builtin_amdgcn_readlane(row, l), tile + L::base(L::quad(l), K) + (K - 65536) * L::STRIDE + j, ch, chunks, bm, lane, fx, fn);
+            const float *src = a.at(__builtin_amdgcn_readlane(row, l), 0);
+            const bool mine = L::row(own) == L::row(l);
+            const uint64_t lanes = __ballot(mine);
+            if (__popcll(open[0] & lanes) + __popcll(open[1] & lanes) + __popcll(open[2] & lanes) + __popcll(open[3] & lanes) > FEW) {
+                // one word of each 128-byte line of the row, so that the scan waits for the memory behind the L2 once
+                float touched = 0.0f;
+                for (int k = own * 32; k < K; k += 64 * 32) touched += src[(uint32_t)k];
+                asm volatile("" ::"v"(touched));
+                // (what the row's finished outputs hold already is what the scan gives them)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (i == j) {
-                    open[i] &= open[i] - 1;
-                    if (lane == l) { e.mx[i] = fx; e.mn[i] = fn; }
+                for (int i = 0; i < 4; i += 2) {
+                    typename E::value fx[2], fn[2];
+                    scan_row<L::STRIDE, RW, TWO ? 1 : Q, E>(src, K, by_key + i, own, L::row(own), fx, fn);
+                    if (mine) {
+                        e.mx[i] = fx[0]; e.mx[i + 1] = fx[1];
+                        e.mn[i] = fn[0]; e.mn[i + 1] = fn[1];
+                    }
                 }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) open[i] &= ~lanes;
+            } else {
+                typename E::value fx, fn;
+                scan_one<L::STRIDE, E>(src, K, tile + L::base(L::quad(l), K) + (K - 65536) * L::STRIDE + j, own, fx, fn);
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (i == j) {
+                        open[i] &= open[i] - 1;
+                        if (own == l) { e.mx[i] = fx; e.mn[i] = fn; }
+                    }
+            }
         }
         // ---- outputs ----
         {

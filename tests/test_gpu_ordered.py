@@ -216,3 +216,78 @@ def test_rows_that_are_not_aligned_go_by_lists(indices, pad, offset):
     assert_bits_equal(out[0].cpu().numpy(), want[0], "c")
     for got, expected in zip(out[1:], want[1:]):
         assert_index_equal(got.cpu().numpy(), expected, "index")
+
+
+def _unsampled(N, M):
+    """Rows of x and of w that no sampled output of the device's decision belongs to."""
+    x_rows = {(2 * i + 1) * N // 128 for i in range(64)}
+    w_rows = {((i * 2654435769 & 0xffffffff) * M) >> 32 for i in range(64)}
+    return [r for r in range(N) if r not in x_rows], [r for r in range(M) if r not in w_rows]
+
+
+@pytest.mark.parametrize("N, K, M", [(640, 768, 300), (330, 1300, 202), (330, 2500, 202), (323, 4900, 101)])     # 32, 16, 8, 4 tile rows
+@pytest.mark.parametrize("searched", ["x", "w"])
+@pytest.mark.parametrize("indices", [True, False])
+def test_rows_that_no_list_finishes(N, K, M, searched, indices):
+    """Rows of one magnitude, of one sign, of few entries, NaN and infinities on the searched side and on the other one, next to each
+    other and alone, at the ends too, inside a call that goes by lists."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(K)
+    if searched == "w":
+        N, M = M, N
+    x, w = torch.randn(N, K, generator=g), torch.rand(M, K, generator=g) * 2 - 1
+    if searched == "w":
+        x, w = torch.rand(N, K, generator=g) * 2 - 1, torch.randn(M, K, generator=g)
+    a, b = (x, w) if searched == "x" else (w, x)
+    free_a, free_b = _unsampled(N, M) if searched == "x" else _unsampled(N, M)[::-1]
+    ones = torch.randint(0, 2, (4, K), generator=g).float() * 2 - 1
+    near = next(r for r in free_a[10:] if r + 1 in free_a and r + 2 in free_a)
+    a[free_a[0]] = ones[0]
+    a[near:near + 3] = ones[1:]
+    a[free_a[40], 5:] = 0.0
+    a[free_a[41]].abs_()
+    a[free_a[-1]] = -0.5
+    b[free_b[0]] = 0.25 * ones[0]
+    b[free_b[20]].abs_()
+    b[free_b[21], 1:] = 0.0
+    b[free_b[22], K - 1] = float("nan")
+    b[free_b[-1], 2] = -float("inf")
+    bias = torch.randn(M, generator=g)
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, bias.numpy())
+    out, (side, lead, _) = _by_lists(x.to(DEV), w.to(DEV), capi.W_MK, bias.to(DEV), indices)
+    assert (side, lead) == (1 if searched == "x" else 2, 0)
+    assert_bits_equal(out[0].cpu().numpy(), want[0], "c")
+    for got, expected in zip(out[1:], want[1:]):
+        assert_index_equal(got.cpu().numpy(), expected, "index")
+
+
+@pytest.mark.parametrize("scattered", [True, False])
+def test_rows_that_no_list_finishes_do_not_hold_up_the_call(scattered):
+    """4 % of the rows of x all +-1, which the lists take (0.55 and 0.50 of the dense tilings' time): within 0.9 of it.  One output
+    of such a row at a time took 1.1 and 3.6 times the dense tilings' time."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(9)
+    N, K, M = 16384, 4096, 1024
+    x, w = torch.randn(N, K, generator=g, device=DEV), torch.rand(M, K, generator=g, device=DEV) * 2 - 1
+    rows = torch.randperm(N, generator=g, device=DEV)[:N // 25] if scattered else torch.arange(N // 25, device=DEV)
+    x[rows] = torch.randint(0, 2, (N // 25, K), generator=g, device=DEV).float() * 2 - 1
+    times = {}
+    for tiling in ("DENSE", "AUTO"):
+        capi.set_option(capi.OPT_FORWARD_TILING, getattr(capi, "FORWARD_TILING_" + tiling))
+        try:
+            for _ in range(3):
+                out = capi.fc_forward(x, w, capi.W_MK)
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(5):
+                out = capi.fc_forward(x, w, capi.W_MK)
+            end.record()
+            end.synchronize()
+        finally:
+            capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+        times[tiling] = (start.elapsed_time(end), out)
+    assert times["AUTO"][0] < 0.9 * times["DENSE"][0], (times["AUTO"][0], times["DENSE"][0])
+    for got, dense in zip(times["AUTO"][1], times["DENSE"][1]):
+        assert torch.equal(got, dense)
