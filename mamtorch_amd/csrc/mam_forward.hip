@@ -1471,7 +1471,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     const size_t staged_need = can_stage ? st_plan.bytes() + tplan.need : 0;
     size_t list_bytes = 0;
     if (range_len == 0 && !static_scratch && on_16 && ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22))) {
-        list_bytes = ordered::workspace_bytes(N, K, M);
+        list_bytes = ordered::workspace_bytes(N, K, M, w_layout);
         if (list_bytes + (can_stage && staged_need < plan.need ? staged_need : plan.need) > avail) list_bytes = 0;
     }
     size_t wt_bytes = 0;
@@ -1590,7 +1590,7 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     const bool turn = w_layout == MAM_W_KM, ragged = K % mam::fwd::G != 0;
     if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0)))
         bytes += mam::fwd::staging_of(true, !turn, N, K, M).bytes();
-    if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M);
+    if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M, w_layout);
     return bytes;
 }
 

@@ -30,7 +30,7 @@ struct Call {
 
 // Whether the path takes a call of this size at all, and the workspace it needs (a multiple of 256).
 bool applies(int64_t N, int64_t K, int64_t M);
-size_t workspace_bytes(int64_t N, int64_t K, int64_t M);
+size_t workspace_bytes(int64_t N, int64_t K, int64_t M, int w_layout);
 // Samples, builds the lists and runs the forward where they pay; `guard` is what the caller's dense kernels
 // take so that they run only where they do not.
 int launch(const Call &call, void *workspace, Guard &guard, hipStream_t stream);

@@ -272,8 +272,8 @@ __device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTI
     for (int o = wave * step; o < OPTIONS; o += WAVES * step) {
         const bool search_x = o < LEADS, two_sided = o % LEADS != 0;
         const int lead = lead_entries(o, (int)p.call.K);
-        // the rows of a (K, M) weight are columns in memory: they are not listed
-        const bool possible = (!two_sided || lead > 0) && (p.call.w_layout == MAM_W_MK || (search_x && !two_sided));
+        // the rows of a (K, M) weight are columns in memory: they are not listed, and there is no two-sided search
+        const bool possible = (!two_sided || lead > 0) && (p.call.w_layout == MAM_W_MK || search_x);
         const int v = p.samples[o * SAMPLES + lane];
         const float tiled = (float)(search_x ? p.call.M : p.call.N), listed = (float)(search_x ? p.call.N : p.call.M);
         // entries written per list: twice the longest sampled need and 64 more, so that hardly any of the outputs that
@@ -340,13 +340,9 @@ __device__ __forceinline__ void build_row(const Rows &rows, int row, int K, int 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int chunks = len / CHUNK;
     const float *src = rows.at(row, 0);
-    const uint32_t mine = (uint32_t)tid * (uint32_t)rows.k_stride;
     float v[R];
 #pragma unroll
-    for (int t = 0; t < R; ++t) {
-        const float *from = src + (int64_t)(t * BUILD_NT) * rows.k_stride;
-        v[t] = t * BUILD_NT + tid < K ? from[mine] : 0.0f;
-    }
+    for (int t = 0; t < R; ++t) v[t] = t * BUILD_NT + tid < K ? src[t * BUILD_NT + tid] : 0.0f;
 #pragma unroll
     for (int j = 0; j < BUCKETS / BUILD_NT; ++j) hist[j * BUILD_NT + tid] = 0;
     for (int j = tid; j < len; j += BUILD_NT) items[j] = make_uint2(0u, key(0, 0));
@@ -456,8 +452,7 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     const Rows a = sx ? x_rows(p.call) : w_rows(p.call), b = sx ? w_rows(p.call) : x_rows(p.call);
     const int K = (int)p.call.K;
     const int row_tiles = (a.rows + 63) / 64;
-    // (an operand stored (K, rows) is its own transpose)
-    const int turns = d.lead > 0 && a.k_stride == 1 ? row_tiles * ((K + 63) / 64) : 0;
+    const int turns = d.lead > 0 ? row_tiles * ((K + 63) / 64) : 0;
     const int total = a.rows + (d.lead > 0 ? b.rows : 0) + turns;
     if ((int)blockIdx.x >= total) return;
     const int item = xcd_remap(blockIdx.x, total);
@@ -890,8 +885,8 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         // ---- the leading entries of the tile rows: (value, key) from their lists, the other factor of four
         // consecutive tile rows x neighbouring listed rows from the transposed operand ----
         if constexpr (TWO) {
-            const char *turned = reinterpret_cast<const char *>(a.k_stride == 1 ? p.turned : a.p);
-            const uint32_t ld4 = (uint32_t)(a.k_stride == 1 ? p.turned_ld : (int)a.k_stride) * 4u;
+            const char *turned = reinterpret_cast<const char *>(p.turned);
+            const uint32_t ld4 = (uint32_t)p.turned_ld * 4u;
             const uint32_t turned_off = (uint32_t)row * 4u + 65535u * ld4;
             const uint2 *mine_led = lead_s + q * 4 * d.lead;
             auto lead_rows = [&](float (&to)[8], int pair) {
@@ -1131,12 +1126,12 @@ bool applies(int64_t N, int64_t K, int64_t M)
 
 // Offsets in the workspace.
 struct Layout { size_t lists_x, lists_w, bound_x, bound_w, turned, total; int cap, pad_x, pad_w, turned_ld; };
-static Layout layout(int64_t N, int64_t K, int64_t M)
+static Layout layout(int64_t N, int64_t K, int64_t M, int w_layout)
 {
     Layout l;
     l.cap = list_cap(K);
     l.pad_x = (int)(ceil_div(N, 64) * 64);
-    l.pad_w = (int)(ceil_div(M, 64) * 64);
+    l.pad_w = w_layout == MAM_W_MK ? (int)(ceil_div(M, 64) * 64) : 0;       // (K, M) weights are not listed
     const size_t chunks = (size_t)l.cap / CHUNK + 1;
     size_t at = 8192;             // decision, samples
     auto take = [&](size_t bytes) {
@@ -1150,7 +1145,7 @@ static Layout layout(int64_t N, int64_t K, int64_t M)
     l.bound_w = take(chunks * 4 * l.pad_w);
     // the transposed operand is addressed with 32-bit byte offsets, its row length in 24 bits
     l.turned_ld = l.pad_x > l.pad_w ? l.pad_x : l.pad_w;
-    if (tile_rows(K) < 8 || (N * K * M < MIN_TWO_SIDED && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_LISTS) ||
+    if (w_layout != MAM_W_MK || tile_rows(K) < 8 || (N * K * M < MIN_TWO_SIDED && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_LISTS) ||
         (size_t)l.turned_ld * 4 >= (1u << 24) || (size_t)l.turned_ld * 4 * K >= ((size_t)1 << 32)) l.turned_ld = 0;
     if (l.turned_ld == 0) l.turned = at;
     else l.turned = take((size_t)l.turned_ld * 4 * K);
@@ -1158,7 +1153,7 @@ static Layout layout(int64_t N, int64_t K, int64_t M)
     return l;
 }
 
-size_t workspace_bytes(int64_t N, int64_t K, int64_t M) { return layout(N, K, M).total; }
+size_t workspace_bytes(int64_t N, int64_t K, int64_t M, int w_layout) { return layout(N, K, M, w_layout).total; }
 
 template <int TB, bool TWO>
 static int launch_forward(const Params &p, hipStream_t st)
@@ -1167,7 +1162,7 @@ static int launch_forward(const Params &p, hipStream_t st)
     const int N = (int)p.call.N, M = (int)p.call.M;
     const int tx = (int)ceil_div(M, TB), tw = (int)ceil_div(N, TB);
     const int64_t bx = (int64_t)tx * splits_of<TB>(N, tx, p.cus), bw = (int64_t)tw * splits_of<TB>(M, tw, p.cus);
-    const unsigned blocks = (unsigned)(bx > bw ? bx : bw);
+    const unsigned blocks = (unsigned)(bx > bw || p.call.w_layout != MAM_W_MK ? bx : bw);
     if (p.call.argmax)
         hipLaunchKernelGGL((forward_kernel<TB, true, TWO>), dim3(blocks), dim3(NT), lds, st, p);
     else
@@ -1197,7 +1192,7 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     Params p;
     p.call = call;
     const int64_t N = call.N, K = call.K, M = call.M;
-    const Layout l = layout(N, K, M);
+    const Layout l = layout(N, K, M, call.w_layout);
     char *base = static_cast<char *>(workspace);
     p.decision = reinterpret_cast<Decision *>(base);
     p.samples = reinterpret_cast<int *>(base + 256);
@@ -1207,8 +1202,6 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     p.bound_w = reinterpret_cast<float *>(base + l.bound_w);
     p.turned = reinterpret_cast<float *>(base + l.turned);
     p.turned_ld = l.turned_ld;
-    // a (K, M) weight takes the place of its transpose, with its own row length
-    if (call.w_layout == MAM_W_KM && (call.ldw * 4 >= (1 << 24) || call.ldw * 4 * K >= ((int64_t)1 << 32))) p.turned_ld = 0;
     p.cap = l.cap;
     p.pad_x = l.pad_x;
     p.pad_w = l.pad_w;
@@ -1223,7 +1216,7 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
         rc = check_launch("ordered::decide_kernel");
         if (rc != MAM_OK) return rc;
     }
-    const dim3 build_grid((unsigned)build_items(N, K, M, p.turned_ld > 0)), build_block(BUILD_NT);
+    const dim3 build_grid((unsigned)(call.w_layout == MAM_W_MK ? build_items(N, K, M, p.turned_ld > 0) : N)), build_block(BUILD_NT);
     const size_t lds = (size_t)p.cap * 8;
     if (K <= 4 * BUILD_NT) hipLaunchKernelGGL((build_kernel<4>), build_grid, build_block, lds, st, p);
     else if (K <= 8 * BUILD_NT) hipLaunchKernelGGL((build_kernel<8>), build_grid, build_block, lds, st, p);

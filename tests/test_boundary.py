@@ -43,6 +43,16 @@ def test_calls_of_more_rows_than_a_list_launch_holds_stay_on_the_dense_tilings(N
     assert l.mam_fc_forward_workspace_for(below, K, M, capi.W_MK, 1) > l.mam_fc_forward_workspace(below, K, M)
 
 
+def test_a_km_call_asks_for_the_lists_of_its_inputs_alone():
+    l, (N, K, M) = capi.lib(), (16384, 4096, 4096)
+    dense = l.mam_fc_forward_workspace(N, K, M)
+    km, mk = (l.mam_fc_forward_workspace_for(N, K, M, layout, 1) - dense for layout in (capi.W_KM, capi.W_MK))
+    entries = K // 4 + 64
+    lists = lambda rows: rows * (8 * entries + 4 * (entries // 8 + 1))
+    assert 4 * K * M + lists(N) <= km < 4 * K * M + lists(N) + 16384      # a copy of the weight, lists, samples
+    assert 4 * N * K + lists(N + M) <= mk < 4 * N * K + lists(N + M) + 16384      # the searched operand transposed, lists of both
+
+
 @pytest.mark.parametrize("N, K, M, neurons", [
     (21632, 288, 64, 64), (12608, 768, 192, 64), (2048, 2048, 320, 64), (256, 4096, 192, 64), (1024, 512, 320, 64),
     (2048, 2048, 192, 128), (2048, 2048, 180, 128), (256, 4096, 320, 128), (12608, 768, 256, 128), (12608, 768, 448, 128)])
