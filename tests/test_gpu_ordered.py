@@ -291,3 +291,30 @@ def test_rows_that_no_list_finishes_do_not_hold_up_the_call(scattered):
     assert times["AUTO"][0] < 0.9 * times["DENSE"][0], (times["AUTO"][0], times["DENSE"][0])
     for got, dense in zip(times["AUTO"][1], times["DENSE"][1]):
         assert torch.equal(got, dense)
+
+
+@pytest.mark.parametrize("indices", [True, False])
+def test_a_call_without_room_for_its_lists_still_runs(indices):
+    """A device with too little memory left for the lists: the operator asks for what the dense tilings need instead."""
+    import mamtorch_amd as mt
+
+    g = torch.Generator(device=DEV).manual_seed(10)
+    N, K, M = 8192, 4096, 1024
+    x, w = torch.randn(N, K, generator=g, device=DEV), torch.rand(M, K, generator=g, device=DEV) * 2 - 1
+    forward = (lambda: mt.kernel.v4.fullyconnected_wt(x, w)) if indices else (
+        lambda: [mt.kernel.v4.fullyconnected_fast_wt(x, w)])
+    want = forward()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    from mamtorch_amd import capi
+    least = 3 * N * M * 4
+    assert capi.lib().mam_fc_forward_workspace_for(N, K, M, capi.W_MK, int(indices)) > least + (64 << 20)
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(DEV) + least + (48 << 20)) / total, DEV)
+    try:
+        got = forward()
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, DEV)
+    for one, other in zip(got, want):
+        assert torch.equal(one, other)
