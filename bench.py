@@ -142,19 +142,15 @@ class Layer:
 
     def describe(self):
         """Which kernels the library takes for this layer's forward (asked of the library itself)."""
-        buf = ctypes.create_string_buffer(256)
+        buf = ctypes.create_string_buffer(640)
         fn = self.lib.mam_fc_forward_describe
         fn(self._p(self.x), self.K, self._p(self.w), self.K, self.capi.W_MK, self.N, self.K, self.M,
-           0 if self.values_only else 1, buf, 256)
-        text = buf.value.decode()
-        if self.lists():
-            text = "forward by magnitude-ordered lists where the data suits them (decided on the device), else " + text
-        return text
+           0 if self.values_only else 1, buf, 640)
+        return buf.value.decode()
 
     def lists(self):
-        """Whether the workspace asked for has room for the lists, which leave most products out."""
-        need = self.lib.mam_fc_forward_values_workspace if self.values_only else self.lib.mam_fc_forward_workspace
-        return self.K % 16 == 0 and self.ws_bytes > need(self.N, self.K, self.M)
+        """Whether the forward may go by lists, which leave most products out (its workspace has room for them)."""
+        return "magnitude-ordered lists" in self.describe()
 
     def backward_bytes(self):
         N, K, M = self.N, self.K, self.M

@@ -133,7 +133,8 @@ int mam_fc_forward(const float *x, int64_t ldx, const float *w, int64_t ldw, int
  * Writes into `text` (a host buffer of `text_bytes` bytes, NUL-terminated) which kernels mam_fc_forward
  * (with_indices != 0) or mam_fc_forward_values (with_indices == 0) would launch for these operands: the
  * tiling, the tile grid, the number of K ranges and the bytes of partials.  The choice depends on the
- * alignment of x and w, so the pointers are looked at but never dereferenced.  Pure host call; for bench
+ * alignment of x and w, so the pointers are looked at but never dereferenced.  Where it depends on the workspace (copies
+ * of the operands, lists) or on the data (lists), each route is named, with the bytes that it needs.  Pure host call; for bench
  * labels and logs.  No counterpart in the reference, which has one kernel per operator.
  */
 int mam_fc_forward_describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,

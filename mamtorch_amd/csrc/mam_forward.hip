@@ -1653,12 +1653,22 @@ extern "C" int mam_fc_forward_describe(const float *x, int64_t ldx, const float 
         return MAM_OK;
     }
     // Operands are staged in the workspace when that has room (what mam_fc_forward_workspace_for() asks for) and the
-    // wave-uniform-rows tiling then runs on the copies: both routes are named, the one a call takes depends on the
-    // workspace it brings.
+    // wave-uniform-rows tiling then runs on the copies, and large calls go by lists: every route is named, the one a call
+    // takes depends on the workspace it brings and, with lists, on the data.
     fwd::Plan tplan;
     fwd::Staging st;
-    if (fwd::staged_plan(tplan, st, plan, with_indices != 0, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr,
-                         nullptr, N, K, M, 0)) {
+    const bool staged = fwd::staged_plan(tplan, st, plan, with_indices != 0, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr,
+                                         nullptr, nullptr, N, K, M, 0);
+    if (ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22))) {
+        const size_t dense = staged && st.bytes() + tplan.need < plan.need ? st.bytes() + tplan.need : plan.need;
+        const int used = snprintf(text, text_bytes, "with %zu workspace bytes: magnitude-ordered lists (ordered::sample_kernel, build_kernel, "
+                                  "forward_kernel) where the device finds that the data suits them; otherwise ",
+                                  ordered::workspace_bytes(N, K, M, w_layout) + dense);
+        if (used < 0 || (size_t)used >= text_bytes) return MAM_OK;
+        text += used;
+        text_bytes -= used;
+    }
+    if (staged) {
         const bool turn = w_layout == MAM_W_KM;
         int used = snprintf(text, text_bytes, "with %zu workspace bytes: %s%s", st.bytes() + tplan.need,
                             st.x || !turn ? "lengthen_rows_kernel + " : "", turn ? "transpose_kernel + " : "");

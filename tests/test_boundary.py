@@ -53,6 +53,33 @@ def test_a_km_call_asks_for_the_lists_of_its_inputs_alone():
     assert 4 * N * K + lists(N + M) <= mk < 4 * N * K + lists(N + M) + 16384      # the searched operand transposed, lists of both
 
 
+@pytest.mark.parametrize("N, K, M, mk, lists", [
+    (256, 4096, 4096, 1, True), (128, 4096, 4096, 1, False), (16384, 4096, 1024, 0, True), (16384, 4001, 1024, 1, True),
+    (16384, 16384, 1024, 1, False), (24, 65536, 65536, 1, False)])
+def test_describe_names_every_route_that_a_call_can_take(N, K, M, mk, lists):
+    l = capi.lib()
+    text = ctypes.create_string_buffer(640)
+    one = ctypes.c_void_p(256)
+    layout = capi.W_MK if mk else capi.W_KM
+    describe = lambda: l.mam_fc_forward_describe(one, K, one, K if mk else M, layout, N, K, M, 1, text, 640)
+    assert describe() == 0
+    with_lists = text.value
+    assert (b"magnitude-ordered lists" in with_lists) == lists, with_lists
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_DENSE)
+    try:
+        assert describe() == 0
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    dense = text.value
+    assert b"lists" not in dense and with_lists.endswith(dense) and (with_lists == dense) == (not lists)
+    if lists:
+        # what it says the lists need is no more than what the workspace query asks for
+        need = int(with_lists.split(b"with ")[1].split()[0])
+        assert need <= l.mam_fc_forward_workspace_for(N, K, M, layout, 1)
+    assert l.mam_fc_forward_describe(one, K, one, K if mk else M, layout, N, K, M, 1, text, 40) == 0      # cut off, not overrun
+    assert len(text.value) < 40
+
+
 @pytest.mark.parametrize("N, K, M, neurons", [
     (21632, 288, 64, 64), (12608, 768, 192, 64), (2048, 2048, 320, 64), (256, 4096, 192, 64), (1024, 512, 320, 64),
     (2048, 2048, 192, 128), (2048, 2048, 180, 128), (256, 4096, 320, 128), (12608, 768, 256, 128), (12608, 768, 448, 128)])
