@@ -31,6 +31,8 @@
 // ends with the slowest of its 256 outputs: 92 entries at K = 4096 where the mean output needs 28.
 #include "mam_ordered.h"
 
+#include <math.h>
+
 namespace mam {
 namespace ordered {
 
@@ -48,14 +50,33 @@ constexpr int LEAD_CAP = 96;          // leading entries kept per tile row (LDS)
 constexpr int64_t MIN_PRODUCTS = 1ll << 32;
 constexpr uint32_t INF_BITS = 0x7f800000u;
 
+constexpr int MAX_UNDECIDED = 4096;
 constexpr int CHUNK = 8;         // list entries between two tests of the bound
 constexpr int BUILD_MAX_CHUNKS = (BUILD_MAX_K / 4 + 64) / CHUNK + 1;
 constexpr int SAMPLES = 64;      // sampled outputs of a call, one per lane of a deciding wave
 constexpr int LEADS = 9;         // leading shares tried
 constexpr int OPTIONS = 2 * LEADS;
 
+// Microseconds of the dense kernels and of the lists of a call, from its sizes alone; launches that come either way are
+// left out.  What a search costs per product is not all: its workgroups load their tiles (14.5 us for 128 KiB), a round of 16 blocks
+// of rows costs 4 to 6 us beside its products, a round of fewer waves hardly less, and the lists themselves 2 to 10 ns a row.
+// Calls of few rows on either side lose there what the search saves (normal x normal, lists / dense: 64 x 4096 -> 16384 416 / 241 us,
+// 65536 x 1024 -> 64 896 / 317, 40 x 8000 -> 16384 2014 / 444; 256 x 4096 -> 4096 148 / 217).  Constants fitted to 180 timed
+// calls (K 256 .. 8000, N and M 40 .. 65536), most of which they give within 20 %.
+struct Times {
+    struct Side { float fixed, per_entry, rounds, round; };      // of a search of this operand's rows
+    float dense, product, led;
+    Side one_sided[2], two_sided[2];                             // rows of x are searched, rows of w
+    __device__ __forceinline__ float lists_us(int side, int lead, int length, float searched) const
+    {
+        const Side &s = side == SIDE_X ? (lead > 0 ? two_sided[0] : one_sided[0]) : lead > 0 ? two_sided[1] : one_sided[1];
+        return s.fixed + s.per_entry * (float)length + s.rounds * (s.round + product * searched + led * (float)lead);
+    }
+};
+
 struct Params {
     Call call;
+    Times times;
     int *samples;             // [OPTIONS][SAMPLES]: entries of the searched list a sampled output needs
     Decision *decision;
     uint4 *lists_x, *lists_w; // [entry pair][row]: (value, key, value, key)
@@ -65,6 +86,8 @@ struct Params {
     int cap;                  // entries a list can hold (a multiple of CHUNK)
     int pad_x, pad_w;         // rows of the list arrays
     int cus;                  // compute units
+    int decided;              // by decide_kernel; otherwise by every workgroup of build_kernel
+    int any_size;             // lists wherever they save products, whatever the rest of them costs (option LISTS)
 };
 
 // Leading shares in 1/1024 of K.
@@ -247,13 +270,42 @@ __global__ __launch_bounds__(BUILD_NT) void sample_kernel(const Params p)
     p.samples[tid * SAMPLES + blockIdx.x] = need;
 }
 
-// The largest t that at least `rank` of the 64 lanes' values reach.
-__device__ __forceinline__ int nth_largest(int v, int rank)
+// The COUNT largest of the 64 lanes' values (not negative), in falling order.  Every workgroup of build_kernel waits for this:
+// lane shifts instead of trips through the LDS.
+template <int COUNT>
+__device__ __forceinline__ void largest(int v, int (&top)[COUNT])
 {
-    int t = 0;
-    for (int bit = 1 << 15; bit > 0; bit >>= 1)
-        if (__popcll(__ballot(v >= (t | bit))) >= rank) t |= bit;
-    return t;
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) {
+        int m = v;
+        auto fold = [&](int other) { m = other > m ? other : m; };
+        fold(__builtin_amdgcn_update_dpp(m, m, 0x111, 0xf, 0xf, false));        // row_shr 1, 2, 4, 8
+        fold(__builtin_amdgcn_update_dpp(m, m, 0x112, 0xf, 0xf, false));
+        fold(__builtin_amdgcn_update_dpp(m, m, 0x114, 0xf, 0xf, false));
+        fold(__builtin_amdgcn_update_dpp(m, m, 0x118, 0xf, 0xf, false));
+        fold(__builtin_amdgcn_update_dpp(m, m, 0x142, 0xa, 0xf, false));        // last lane of a row of 16 to the next row
+        fold(__builtin_amdgcn_update_dpp(m, m, 0x143, 0xc, 0xf, false));        // of the lower half to the upper half
+        top[i] = __builtin_amdgcn_readlane(m, 63);
+        if (lane == (int)__builtin_ctzll(__ballot(v == top[i]))) v = -1;
+    }
+}
+
+// rows of the tile operand per workgroup: as many as fit the LDS as whole rows (0: not even 4)
+__host__ __device__ __forceinline__ int tile_rows(int64_t K)
+{
+    for (int tb = 32; tb >= 4; tb /= 2)
+        if (K * tb * 4 <= MAX_TILE_BYTES) return tb;
+    return 0;
+}
+constexpr int TWO_SIDED_ROWS = 8;     // of a two-sided search
+
+// Row ranges per tile: three rounds of workgroups over the chip, but at least one block of rows per wave.
+__host__ __device__ __forceinline__ int splits_of(int tb, int searched, int tiles, int cus)
+{
+    const int blocks = (searched + 256 / tb - 1) / (256 / tb);
+    const int s = (3 * cus + tiles - 1) / tiles, most = (blocks + NT / 64 - 1) / (NT / 64);
+    return s < most ? s : most;
 }
 
 // The cheapest option, by all waves of a workgroup.  In units of one product of a dense kernel per output (12608 x 768 x
@@ -262,8 +314,9 @@ __device__ __forceinline__ int nth_largest(int v, int rank)
 // finishes (a sampled need beyond the longest list) cost SCAN a product over the whole row, and their waves a whole list first; four
 // such samples of 64 need too much by the rule above.  The dense kernels cost K.
 constexpr float SCAN = 5.0f;
+struct Weighed { float cost, searched, scans; int length; };     // of an option; searched: entries; scans: share of outputs no list finishes
 template <int WAVES>
-__device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTIONS], int (&length_s)[OPTIONS])
+__device__ __forceinline__ Decision decide(const Params &p, Weighed (&weighed)[OPTIONS])
 {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -278,37 +331,40 @@ __device__ __forceinline__ Decision decide(const Params &p, float (&cost_s)[OPTI
         const float tiled = (float)(search_x ? p.call.M : p.call.N), listed = (float)(search_x ? p.call.N : p.call.M);
         // entries written per list: twice the longest sampled need and 64 more, so that hardly any of the outputs that
         // are finished one by one need more than their list; needs that no list meets do not count
-        const int want = (nth_largest(v <= p.cap ? v : 0, 2) * 2 + 64 + CHUNK - 1) / CHUNK * CHUNK;
-        const int length = want < p.cap ? want : p.cap;
         const int beyond = __popcll(__ballot(v > p.cap));
-        float searched = 1.3f * (float)nth_largest(v, 4);
+        int top[5];
+        largest<5>(v, top);
+        const int second = beyond == 0 ? top[1] : beyond == 1 ? top[2] : beyond == 2 ? top[3] : top[4];
+        const int want = (second * 2 + 64 + CHUNK - 1) / CHUNK * CHUNK;
+        const int length = want < p.cap ? want : p.cap;
+        float searched = 1.3f * (float)top[3];
         if (beyond > 0 && searched < (float)length) searched = (float)length;
-        float cost = 0.15f * K + 3.5f * searched + SCAN * K * (float)beyond / SAMPLES;
+        const float scans = (float)beyond / SAMPLES;
+        float cost = 0.15f * K + 3.5f * searched + SCAN * K * scans;
         if (two_sided) cost += 6.0f * (float)lead + K * (36.0f / tiled + 18.0f / listed);
-        if (lane == 0) {
-            cost_s[o] = possible ? cost : 1e30f;
-            length_s[o] = length;
-        }
+        if (lane == 0) weighed[o] = {possible ? cost : 1e30f, searched, scans, length};
     }
     __syncthreads();
     int best = 0;
     for (int o = step; o < OPTIONS; o += step)
-        if (cost_s[o] < cost_s[best]) best = o;
+        if (weighed[o].cost < weighed[best].cost) best = o;
     Decision d;
-    d.side = cost_s[best] < 0.95f * K ? (best < LEADS ? SIDE_X : SIDE_W) : SIDE_NONE;
+    d.side = best < LEADS ? SIDE_X : SIDE_W;
     d.lead = lead_entries(best, (int)p.call.K);
-    d.length = length_s[best];
+    d.length = weighed[best].length;
+    const float us = p.times.lists_us(d.side, d.lead, d.length, weighed[best].searched) + SCAN * weighed[best].scans * p.times.dense;
+    if (!(weighed[best].cost < 0.95f * K) || !(p.any_size || us < p.times.dense)) d.side = SIDE_NONE;
     d.pad = 0;
     return d;
 }
 
-// Two-sided searches have 18 options: decided once, in a launch of its own (4 us; the two one-sided ones are decided by
-// every workgroup of build_kernel).
+// Two-sided searches have 18 options: decided once, in a launch of its own (6 us).  The two one-sided ones are decided by
+// every workgroup of build_kernel, up to MAX_UNDECIDED of them (build_kernel alone, where none is chosen: 3 us more with 4096, 51 us
+// with 16384, 87 us with 65536).
 __global__ __launch_bounds__(64 * LEADS) void decide_kernel(const Params p)
 {
-    __shared__ float cost_s[OPTIONS];
-    __shared__ int length_s[OPTIONS];
-    const Decision d = decide<LEADS>(p, cost_s, length_s);
+    __shared__ Weighed weighed[OPTIONS];
+    const Decision d = decide<LEADS>(p, weighed);
     if (threadIdx.x == 0) *p.decision = d;
 }
 
@@ -435,13 +491,12 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     __shared__ uint32_t part[BUILD_NT / 64], part2[BUILD_NT / 64];
     __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
     __shared__ float turn[64][65];
-    __shared__ float cost_s[OPTIONS];
-    __shared__ int length_s[OPTIONS];
+    __shared__ Weighed weighed[OPTIONS];
     Decision d;
-    if (p.turned_ld > 0) {
+    if (p.decided) {
         d = *p.decision;
     } else {
-        d = decide<BUILD_NT / 64>(p, cost_s, length_s);
+        d = decide<BUILD_NT / 64>(p, weighed);
         d.side = __builtin_amdgcn_readfirstlane(d.side);
         d.length = __builtin_amdgcn_readfirstlane(d.length);
         d.lead = 0;
@@ -747,15 +802,6 @@ struct Lanes {
     static __device__ __forceinline__ int base(int quad, int K) { return TWO ? quad * K * 4 : quad * 4; }
 };
 
-// Row ranges per tile: three rounds of workgroups over the chip, but at least one block of rows per wave.
-template <int TB>
-__host__ __device__ __forceinline__ int splits_of(int searched, int tiles, int cus)
-{
-    const int blocks = (searched + 256 / TB - 1) / (256 / TB);
-    const int s = (3 * cus + tiles - 1) / tiles, most = (blocks + NT / 64 - 1) / (NT / 64);
-    return s < most ? s : most;
-}
-
 template <int TB, bool ARGS, bool TWO>
 __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 {
@@ -775,7 +821,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
     const int pad = lists_x ? p.pad_x : p.pad_w, pad_b = lists_x ? p.pad_w : p.pad_x;
     const Rows a = lists_x ? x_rows(c) : w_rows(c), b = lists_x ? w_rows(c) : x_rows(c);
     const int K = (int)c.K;
-    const int tiles = (b.rows + TB - 1) / TB, splits = splits_of<TB>(a.rows, tiles, p.cus);
+    const int tiles = (b.rows + TB - 1) / TB, splits = splits_of(TB, a.rows, tiles, p.cus);
     if ((int)blockIdx.x >= tiles * splits) return;
     const int logical = xcd_remap(blockIdx.x, tiles * splits);
     const int split = logical / tiles, b0 = (logical - split * tiles) * TB;
@@ -1092,14 +1138,6 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 }
 
 // ---- host ----------------------------------------------------------------------------------------------------
-// rows of the tile operand per workgroup: as many as fit the LDS as whole rows (0: not even 4)
-static int tile_rows(int64_t K)
-{
-    for (int tb = 32; tb >= 4; tb /= 2)
-        if (K * tb * 4 <= MAX_TILE_BYTES) return tb;
-    return 0;
-}
-
 static int list_cap(int64_t K)
 {
     int64_t cap = K / 4 + 64;
@@ -1161,7 +1199,7 @@ static int launch_forward(const Params &p, hipStream_t st)
     const size_t lds = (size_t)p.call.K * TB * 4 + (TWO ? LEAD_CAP * TB * 8 : 0);
     const int N = (int)p.call.N, M = (int)p.call.M;
     const int tx = (int)ceil_div(M, TB), tw = (int)ceil_div(N, TB);
-    const int64_t bx = (int64_t)tx * splits_of<TB>(N, tx, p.cus), bw = (int64_t)tw * splits_of<TB>(M, tw, p.cus);
+    const int64_t bx = (int64_t)tx * splits_of(TB, N, tx, p.cus), bw = (int64_t)tw * splits_of(TB, M, tw, p.cus);
     const unsigned blocks = (unsigned)(bx > bw || p.call.w_layout != MAM_W_MK ? bx : bw);
     if (p.call.argmax)
         hipLaunchKernelGGL((forward_kernel<TB, true, TWO>), dim3(blocks), dim3(NT), lds, st, p);
@@ -1187,6 +1225,43 @@ static int setup_device(int)
 }
 static DeviceHookRegistration g_registration(setup_device);
 
+static Times::Side side_times(int64_t listed, int64_t tiled, int64_t K, bool args, bool search_x, bool two_sided, int cus)
+{
+    const int tb = two_sided ? TWO_SIDED_ROWS : tile_rows(K);
+    const int tiles = (int)ceil_div(tiled, tb), splits = splits_of(tb, (int)listed, tiles, cus);
+    const int per_split = (int)ceil_div(ceil_div(listed, 256 / tb), splits), waves = NT / 64, last = per_split % waves;
+    const float alone = two_sided ? 0.45f : 0.3f;                // of a full round's time, by a single wave
+    const float rounds = (float)(per_split / waves) + (last ? alone + (1.0f - alone) * (float)last / (float)waves : 0.0f);
+    const float lds = (float)K * (float)tb * 4.0f + (two_sided ? (float)(LEAD_CAP * TWO_SIDED_ROWS * 8) : 0.0f);
+    const float load = 4.4e-4f * (float)K * (float)tb * (lds <= 80.0f * 1024.0f ? 0.5f : 1.0f);     // two workgroups share a CU where their tiles fit
+    float workgroups = (float)tiles * (float)splits / (float)cus;
+    workgroups = workgroups < 4.0f ? ceilf(workgroups) : workgroups + 0.3f;
+    const float row = 1e-3f + (K > 16 * BUILD_NT ? 1.4e-6f : 0.95e-6f) * (float)K;
+    Times::Side s;
+    s.fixed = 4.0f + row * (float)listed + workgroups * load;
+    if (two_sided) s.fixed += 0.9f * row * (float)tiled + 4.4e-6f * (float)K * (float)listed;       // lists of the leading entries, transpose
+    s.per_entry = 5.3e-6f * (float)listed;
+    s.rounds = workgroups * rounds;
+    s.round = args ? 6.0f + (search_x ? 0.0f : 0.1f * (float)tb) : 4.0f;                            // (with w searched the stores are columns)
+    return s;
+}
+static Times times_of(const Call &c, int cus)
+{
+    const bool args = c.argmax != nullptr;
+    const int64_t m64 = ceil_div(c.M, 64);
+    const bool narrow = m64 % 2 == 1 && m64 <= 5;                // 64 neurons per tile
+    const float K = (float)c.K, per = (args ? 0.043f + 11.0f / K : 0.036f + 1.5f / K) * (narrow ? (args ? 1.3f : 1.1f) : 1.0f);
+    Times t;
+    t.dense = (float)(ceil_div(c.N, 32) * 32) * (float)(narrow ? m64 * 64 : ceil_div(m64, 2) * 128) * K * per * 1e-6f;
+    t.product = args ? 0.135f : 0.095f;
+    t.led = args ? 0.35f : 0.25f;
+    t.one_sided[0] = side_times(c.N, c.M, c.K, args, true, false, cus);
+    t.one_sided[1] = side_times(c.M, c.N, c.K, args, false, false, cus);
+    t.two_sided[0] = side_times(c.N, c.M, c.K, args, true, true, cus);
+    t.two_sided[1] = side_times(c.M, c.N, c.K, args, false, true, cus);
+    return t;
+}
+
 int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
 {
     Params p;
@@ -1208,15 +1283,19 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     guard.decision = p.decision;
 
     p.cus = num_cus();
+    p.times = times_of(call, p.cus);
+    const int64_t items = call.w_layout == MAM_W_MK ? build_items(N, K, M, p.turned_ld > 0) : N;
+    p.decided = p.turned_ld > 0 || items > MAX_UNDECIDED;
+    p.any_size = option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_LISTS;
     hipLaunchKernelGGL(sample_kernel, dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
     int rc = check_launch("ordered::sample_kernel");
     if (rc != MAM_OK) return rc;
-    if (p.turned_ld > 0) {
+    if (p.decided) {
         hipLaunchKernelGGL(decide_kernel, dim3(1), dim3(64 * LEADS), 0, st, p);
         rc = check_launch("ordered::decide_kernel");
         if (rc != MAM_OK) return rc;
     }
-    const dim3 build_grid((unsigned)(call.w_layout == MAM_W_MK ? build_items(N, K, M, p.turned_ld > 0) : N)), build_block(BUILD_NT);
+    const dim3 build_grid((unsigned)items), build_block(BUILD_NT);
     const size_t lds = (size_t)p.cap * 8;
     if (K <= 4 * BUILD_NT) hipLaunchKernelGGL((build_kernel<4>), build_grid, build_block, lds, st, p);
     else if (K <= 8 * BUILD_NT) hipLaunchKernelGGL((build_kernel<8>), build_grid, build_block, lds, st, p);
@@ -1232,7 +1311,7 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     }
     // Narrow tiles for the leading entries: 32 searched rows per wave, 128 contiguous bytes (12608 x 768 -> 3072, normal
     // weights: 1740 / 1515 / 1206 us with 32 / 16 / 8 tile rows, 1730 us dense).
-    return rc != MAM_OK || p.turned_ld == 0 ? rc : launch_forward<8, true>(p, st);
+    return rc != MAM_OK || p.turned_ld == 0 ? rc : launch_forward<TWO_SIDED_ROWS, true>(p, st);
 }
 
 }  // namespace ordered

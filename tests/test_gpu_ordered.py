@@ -68,14 +68,14 @@ def _check(N, K, M, kind_x, kind_w, layout_mk=True, pad=0, seed=0):
         assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
 
 
-def _by_lists(xd, wd, layout, bias=None, indices=True, w_sel=None, x_sel=None):
-    """A call with the lists allowed at every size: its outputs, and what the device decided -- (side, leading entries, entries
+def _by_lists(xd, wd, layout, bias=None, indices=True, w_sel=None, x_sel=None, tiling="LISTS"):
+    """A call with the lists allowed at every size (or as ``tiling`` says): its outputs, and what the device decided -- (side, leading entries, entries
     per list), side 0: the dense kernels, 1: rows of x are searched, 2: rows of w -- which lies at the start of the workspace."""
     from mamtorch_amd import capi
 
     N, K = xd.shape
     M = wd.shape[0] if layout == capi.W_MK else wd.shape[1]
-    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
+    capi.set_option(capi.OPT_FORWARD_TILING, getattr(capi, "FORWARD_TILING_" + tiling))
     try:
         need = capi.lib().mam_fc_forward_workspace_for(N, K, M, layout, int(indices))
         ws = torch.full((need,), 255, dtype=torch.uint8, device=DEV)
@@ -318,3 +318,25 @@ def test_a_call_without_room_for_its_lists_still_runs(indices):
         torch.cuda.set_per_process_memory_fraction(1.0, DEV)
     for one, other in zip(got, want):
         assert torch.equal(one, other)
+
+
+@pytest.mark.parametrize("N, K, M", [(64, 4096, 16384), (16384, 4096, 64), (40, 8000, 16384), (64, 4096, 32768)])
+@pytest.mark.parametrize("indices", [True, False])
+def test_calls_of_few_rows_go_by_lists_only_where_the_search_is_short(N, K, M, indices):
+    """Too few rows for the waves of a workgroup: the dense tilings, unless one side is uniform; the results are the same."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(11)
+    x, w = torch.randn(N, K, generator=g, device=DEV), torch.randn(M, K, generator=g, device=DEV)
+    for uniform in (False, True):
+        if uniform:
+            x = torch.rand(N, K, generator=g, device=DEV) * 2 - 1
+        out, (side, _, _) = _by_lists(x, w, capi.W_MK, indices=indices, tiling="AUTO")
+        assert (side != 0) == uniform, side
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_DENSE)
+        try:
+            dense = capi.fc_forward(x, w, capi.W_MK) if indices else (capi.fc_forward_values(x, w, capi.W_MK),)
+        finally:
+            capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+        for one, other in zip(out, dense):
+            assert torch.equal(one, other)
