@@ -17,6 +17,8 @@ def _data(kind, rows, k, g):
     r = torch.rand(rows, k, generator=g)
     if kind == "uniform":
         t = r * 2 - 1
+    elif kind == "relu":
+        t = t.relu()
     elif kind == "ties":
         t = (t * 4).round() / 4
     elif kind == "positive":
@@ -50,13 +52,8 @@ def _check(N, K, M, kind_x, kind_w, layout_mk=True, pad=0, seed=0):
     wd = (w if layout_mk else w.T.contiguous()).to(DEV)
     layout = capi.W_MK if layout_mk else capi.W_KM
     w_sel, x_sel = torch.zeros(2, N, M, device=DEV), torch.zeros(2, N, M, device=DEV)
-    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_LISTS)
-    try:
-        c, amax, amin = capi.fc_forward(xd, wd, layout, bias.to(DEV), w_sel=w_sel, x_sel=x_sel)
-        values = capi.fc_forward_values(xd, wd, layout, bias.to(DEV))
-        torch.cuda.synchronize()
-    finally:
-        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    (c, amax, amin), decision = _by_lists(xd, wd, layout, bias.to(DEV), w_sel=w_sel, x_sel=x_sel)
+    (values,), _ = _by_lists(xd, wd, layout, bias.to(DEV), indices=False)
     tag = "%s x %s, N %d K %d M %d" % (kind_x, kind_w, N, K, M)
     assert_bits_equal(c.cpu().numpy(), want[0], tag + " c")
     assert_bits_equal(values.cpu().numpy(), want[0], tag + " values-only c")
@@ -66,6 +63,7 @@ def _check(N, K, M, kind_x, kind_w, layout_mk=True, pad=0, seed=0):
     for plane, index in enumerate(want[1:3]):
         assert_bits_equal(x_sel[plane].cpu().numpy(), x.numpy()[rows, index], tag + " x_sel")
         assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
+    return decision
 
 
 def _by_lists(xd, wd, layout, bias=None, indices=True, w_sel=None, x_sel=None, tiling="LISTS"):
@@ -102,12 +100,16 @@ def _strided(x, pad):
 @pytest.mark.parametrize("kinds", [("normal", "uniform"), ("uniform", "normal"), ("normal", "normal")])
 @pytest.mark.parametrize("layout_mk", [True, False])
 def test_sizes_on_both_sides_of_every_tile_width(N, K, M, kinds, layout_mk):
-    _check(N, K, M, *kinds, layout_mk=layout_mk, pad=3 if layout_mk else 0)
+    side, lead, _ = _check(N, K, M, *kinds, layout_mk=layout_mk, pad=3 if layout_mk else 0)
+    if 768 <= K <= 9728 and "uniform" in kinds:
+        # the rows of the normal operand are searched; a (K, M) weight's are not listed
+        assert (side, lead) == ((1 if kinds[0] == "normal" else 2 if layout_mk else 0), 0)
 
 
 @pytest.mark.parametrize("kind", ["ties", "positive", "zero rows", "nan and inf", "sparse", "denormal", "overflow"])
 @pytest.mark.parametrize("other", ["uniform", "normal", "same"])
 def test_data_the_lists_do_not_finish(kind, other):
+    """With the lists allowed: most of these the device hands to the dense kernels, which are behind the same guard."""
     for K in (300, 2500):
         _check(70, K, 68, kind, kind if other == "same" else other, seed=1)
         _check(70, K, 68, kind if other == "same" else other, kind, seed=2)
@@ -141,12 +143,72 @@ def test_a_few_bad_rows_among_good_ones():
     assert_index_equal(amin.cpu().numpy(), want[2], "argmin")
 
 
-@pytest.mark.parametrize("N,K,M", [(66, 520, 70), (97, 2432, 33), (64, 4864, 65), (40, 4095, 64)])
-@pytest.mark.parametrize("kind_x", ["normal", "sparse"])
-def test_two_sided_searches(N, K, M, kind_x):
+@pytest.mark.parametrize("N, K, M", [(640, 768, 640), (700, 1024, 701), (1000, 2432, 300), (300, 2432, 1000), (512, 4864, 513),
+                                     (400, 4095, 402), (1200, 520, 333), (333, 520, 1201)])
+@pytest.mark.parametrize("kinds", [("normal", "normal"), ("relu", "normal")])
+def test_two_sided_searches(N, K, M, kinds):
     """Normal weights: the leading entries of one operand first, then a search bounded by what they leave."""
-    _check(N, K, M, kind_x, "normal", seed=3)
-    _check(N, K, M, "normal", kind_x, layout_mk=False, seed=4)
+    side, lead, _ = _check(N, K, M, *kinds, seed=3)
+    assert lead > 0 and side == (2 if N > 2 * M and (kinds[0] == "normal" or K > 1000) else 1)
+
+
+@pytest.mark.parametrize("N, K, M", [(640, 768, 640), (300, 2432, 1000), (1000, 2432, 300), (400, 4095, 402)])
+def test_two_sided_searches_over_special_rows(N, K, M):
+    """Rows of zeros, of one magnitude, of few entries, ties, NaN and infinities on either operand of a two-sided search."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(K + N)
+    x, w = torch.randn(N, K, generator=g), torch.randn(M, K, generator=g)
+    for t, free in zip((x, w), _unsampled(N, M)):
+        t[free[0]] = 0.0
+        t[free[5]] = -0.75
+        t[free[6]] = torch.randint(0, 2, (K,), generator=g).float() * 2 - 1
+        t[free[10], 4:] = 0.0
+        t[free[20]] = (t[free[20]] * 2).round() / 2
+        t[free[30], K // 2] = float("nan")
+        t[free[31], K - 1] = float("inf")
+        t[free[32], 0] = -float("inf")
+        t[free[-1]].abs_()
+    bias = torch.randn(M, generator=g)
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, bias.numpy())
+    sel = torch.zeros(4, N, M, device=DEV)
+    out, d = _by_lists(x.to(DEV), w.to(DEV), capi.W_MK, bias.to(DEV), w_sel=sel[:2], x_sel=sel[2:])
+    values, dv = _by_lists(x.to(DEV), w.to(DEV), capi.W_MK, bias.to(DEV), indices=False)
+    assert d == dv and d[0] != 0 and d[1] > 0
+    assert_bits_equal(out[0].cpu().numpy(), want[0], "c")
+    assert_bits_equal(values[0].cpu().numpy(), want[0], "values-only c")
+    for plane in range(2):
+        assert_index_equal(out[1 + plane].cpu().numpy(), want[1 + plane], "index")
+        index = want[1 + plane]
+        assert_bits_equal(sel[plane].cpu().numpy(), w.numpy()[np.arange(M)[None, :], index], "w_sel")
+        assert_bits_equal(sel[2 + plane].cpu().numpy(), x.numpy()[np.arange(N)[:, None], index], "x_sel")
+
+
+@pytest.mark.parametrize("N, K, M", [(256, 4096, 4096), (12608, 768, 3072), (12608, 3072, 768), (16384, 4096, 1024)])
+@pytest.mark.parametrize("kinds", [("normal", "uniform"), ("uniform", "normal"), ("normal", "normal")])
+def test_lists_and_dense_tilings_agree_on_full_size_calls(N, K, M, kinds):
+    """The layers that training and inference run: every output of both routes, bit for bit."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(12)
+    make = {"normal": lambda r: torch.randn(r, K, generator=g, device=DEV),
+            "uniform": lambda r: torch.rand(r, K, generator=g, device=DEV) * 2 - 1}
+    x, w, bias = make[kinds[0]](N), make[kinds[1]](M) * 0.02, torch.randn(M, generator=g, device=DEV)
+    got = {}
+    for tiling in ("LISTS", "DENSE"):
+        sel = torch.zeros(4, N, M, device=DEV)
+        out, d = _by_lists(x, w, capi.W_MK, bias, w_sel=sel[:2], x_sel=sel[2:], tiling=tiling)
+        values, _ = _by_lists(x, w, capi.W_MK, bias, indices=False, tiling=tiling)
+        got[tiling] = (*out, sel, *values)
+        if tiling == "LISTS":
+            assert d[0] != 0 and (d[1] > 0) == (kinds == ("normal", "normal"))
+    for one, other in zip(got["LISTS"], got["DENSE"]):
+        assert torch.equal(one.view(torch.int32), other.view(torch.int32))
+    if N == 256:
+        want = oracle.forward(x.cpu().numpy(), w.cpu().numpy(), oracle.W_MK, bias.cpu().numpy())
+        assert_bits_equal(got["DENSE"][0].cpu().numpy(), want[0], "c")
+        assert_index_equal(got["DENSE"][1].cpu().numpy(), want[1], "argmax")
+        assert_index_equal(got["DENSE"][2].cpu().numpy(), want[2], "argmin")
 
 
 def test_every_replay_of_a_graph_decides_anew():
