@@ -75,13 +75,13 @@ struct FwdShape { int64_t N, K, M; };
 // 4096 -> 4096), or, where the device has not that much left, what the call cannot do without.
 at::Tensor forward_workspace(const FwdShape &s, int layout, bool with_indices, const at::Tensor &like)
 {
-    const size_t least = with_indices ? mam_fc_forward_workspace(s.N, s.K, s.M) : mam_fc_forward_values_workspace(s.N, s.K, s.M);
     const size_t most = mam_fc_forward_workspace_for(s.N, s.K, s.M, layout, with_indices ? 1 : 0);
-    if (most > least) {
-        try {
-            return workspace_for(most, like);
-        } catch (const c10::OutOfMemoryError &) {
-        }
+    size_t least = 0;
+    try {
+        return workspace_for(most, like);
+    } catch (const c10::OutOfMemoryError &) {
+        least = with_indices ? mam_fc_forward_workspace(s.N, s.K, s.M) : mam_fc_forward_values_workspace(s.N, s.K, s.M);
+        if (least >= most) throw;
     }
     return workspace_for(least, like);
 }
