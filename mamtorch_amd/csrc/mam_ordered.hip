@@ -16,18 +16,19 @@
 // Four launches, all decisions on the device:
 //   sample_kernel  64 outputs computed in full: how long would their lists have to be, on either side and with any
 //                  of LEADS leading shares of the other side?
-//   build_kernel   first the decision (large calls: decide_kernel): the cheapest of these, or (when products do not
-//                  fall off that way: constant magnitudes, all-positive products) none, and then the dense kernels run
-//                  instead.  A workgroup per listed row: counting sort of the leading entries by magnitude (512 buckets over 4 octaves),
+//   build_kernel   first the decision (two-sided searches and many rows: decide_kernel): the cheapest of these, or none, and then
+//                  the dense kernels run instead: where products do not fall off that way (constant magnitudes, products of one
+//                  sign), or where the search of so few rows takes longer all the same.
+//                  A workgroup per listed row: counting sort of the leading entries by magnitude (512 buckets over 4 octaves),
 //                  written chunk by chunk with the bound U of what follows each chunk; and, for a leading share, the
 //                  searched operand transposed.
 //   forward_kernel the search itself (below).
 //   dense kernels  exit at once unless the decision was "none".
 //
 // Measured against the dense tilings (forward call, hand-over arrays written).  Uniform weights or inputs, one-sided:
-// 207 -> 67 us at 256 x 4096 x 4096, 1.70 -> 0.63 ms and 1.48 -> 0.25 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.84 ms
-// (values only) and 3.13 -> 0.42 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.17 ms
-// at 12608 x 768 -> 3072, 3.13 -> 1.09 ms at 16384 x 4096 -> 1024, 0.84 -> 0.40 ms at 4096 x 2048 x 2048.  A wave's search
+// 207 -> 67 to 75 us at 256 x 4096 x 4096, 1.70 -> 0.63 ms and 1.48 -> 0.25 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.84 ms
+// (values only) and 3.13 -> 0.42 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.43 ms
+// at 12608 x 768 -> 3072, 3.12 -> 1.07 ms at 16384 x 4096 -> 1024, 0.84 -> 0.44 ms at 4096 x 2048 x 2048.  A wave's search
 // ends with the slowest of its 256 outputs: 92 entries at K = 4096 where the mean output needs 28.
 #include "mam_ordered.h"
 
@@ -42,11 +43,15 @@ constexpr int BUILD_NT = 256;         // threads of the build, per listed row
 constexpr int BUILD_MAX_K = 40 * BUILD_NT;
 constexpr int NT = 1024;              // threads of the forward
 constexpr int MAX_TILE_BYTES = 152 * 1024;
-// ... and from which two-sided searches are considered (a launch more, 4.5 us when it is not taken)
+// N * K * M from which two-sided searches are considered.  They cost two launches and a longer sampling, 9 us, where they are not
+// taken (256 x 4096 -> 4096, uniform weights, 2^32 products: 67 us without, 76 us with them; normal weights 224 and 147 us, dense
+// 207 us): up to 2^33 products 2 to 13 % of the call.
 constexpr int64_t MIN_TWO_SIDED = 1ll << 33;
 constexpr int LEAD_CAP = 96;          // leading entries kept per tile row (LDS)
-// N * K * M from which a call takes the lists: sampling, lists and the idle dense launches cost ~35 us, which a
-// call that then goes to the dense tilings (200 us for 2^32 products) pays as well
+// N * K * M from which a call takes the lists.  Uniform on one side, they win from 2^30 products on (lists / dense, with indices:
+// 128 x 2048 -> 4096 50 / 65 us, 128 x 4096 -> 4096 68 / 109), but only the device finds out what the data is, and a call that it
+// hands to the dense tilings has paid for sampling and idle launches: 13 to 20 us, 6 to 9 % of the 165 to 210 us that 2^32
+// products take there, twice that share at 2^31.
 constexpr int64_t MIN_PRODUCTS = 1ll << 32;
 constexpr uint32_t INF_BITS = 0x7f800000u;
 
@@ -398,7 +403,7 @@ __device__ __forceinline__ void build_row(const Rows &rows, int row, int K, int 
     const float *src = rows.at(row, 0);
     float v[R];
 #pragma unroll
-    for (int t = 0; t < R; ++t) v[t] = t * BUILD_NT + tid < K ? src[t * BUILD_NT + tid] : 0.0f;
+    for (int t = 0; t < R; ++t) v[t] = t * BUILD_NT + tid < K ? (src + t * BUILD_NT)[(uint32_t)tid] : 0.0f;
 #pragma unroll
     for (int j = 0; j < BUCKETS / BUILD_NT; ++j) hist[j * BUILD_NT + tid] = 0;
     for (int j = tid; j < len; j += BUILD_NT) items[j] = make_uint2(0u, key(0, 0));
@@ -491,7 +496,9 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     __shared__ uint32_t part[BUILD_NT / 64], part2[BUILD_NT / 64];
     __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
     __shared__ float turn[64][65];
-    __shared__ Weighed weighed[OPTIONS];
+    // (with turns the decision has been made before; the LDS of one more array would cost a workgroup per CU at K = 3072)
+    Weighed (&weighed)[OPTIONS] = reinterpret_cast<Weighed (&)[OPTIONS]>(turn);
+    static_assert(sizeof(weighed) <= sizeof(turn), "decision and transpose share LDS");
     Decision d;
     if (p.decided) {
         d = *p.decision;
@@ -782,10 +789,14 @@ __device__ __forceinline__ void scan_row(const float *src, int K, const float *b
 // blocks of 64 * 4 / TB listed rows in turn and need no barrier after the tile is loaded.  A wave looks at its
 // lists chunk by chunk until all but FEW of its 256 outputs are finished by their bound, and then finishes those
 // one by one with all its lanes (FEW = 0, 1, 2, 4: 75 / 72 / 72 / 73 us at 256 x 4096 x 4096, 608 / 593 / 593 / 602 us at
-// 16384 x 4096 -> 1024, while the selected operands still came from the row).  Bound: v_max_f64 / v_min_f64, ~13 of the ~17 cycles per product and SIMD; the random 16-byte
-// LDS reads take half of that.  (9.9 T products/s in a loop of its own against 14.3 T with fp32 extremes and no
+// 16384 x 4096 -> 1024, while the selected operands still came from the row).  Bound: v_max_f64 / v_min_f64 where rows
+// are many (at 4 cycles each, VALU instructions take 0.76 of the busy cycles at 12608 x 768 -> 3072, and those two hold the unit longer);
+// the random 16-byte LDS reads take half of the cycles beside them, two to three fifths of it bank conflicts.  256 x 4096 -> 4096: 0.44,
+// for each workgroup waits 14 us for its tile and half of its waves have no rows.  (9.9 T products/s in a loop of its own against 14.3 T with fp32 extremes and no
 // indices.)
 constexpr int FEW = 2;
+// Outputs of a row that are scanned one by one, 8 to 17 us each beside the other waves' work; the whole row takes 30 to 60 us.
+constexpr int FEW_OF_ROW = 4;
 
 // Where a lane sits and how the tile lies in LDS.  One-sided: neighbouring lanes share a searched row, the tile is
 // [k][TB], so that the lanes of a row read TB * 4 contiguous bytes and write as many.  Two-sided: neighbouring lanes are
@@ -1037,7 +1048,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
             const float *src = a.at(__builtin_amdgcn_readlane(row, l), 0);
             const bool mine = L::row(own) == L::row(l);
             const uint64_t lanes = __ballot(mine);
-            if (__popcll(open[0] & lanes) + __popcll(open[1] & lanes) + __popcll(open[2] & lanes) + __popcll(open[3] & lanes) > FEW) {
+            if (__popcll(open[0] & lanes) + __popcll(open[1] & lanes) + __popcll(open[2] & lanes) + __popcll(open[3] & lanes) > FEW_OF_ROW) {
                 // one word of each 128-byte line of the row, so that the scan waits for the memory behind the L2 once
                 float touched = 0.0f;
                 for (int k = own * 32; k < K; k += 64 * 32) touched += src[(uint32_t)k];
