@@ -119,7 +119,8 @@ int mam_set_option(int option, int value);
  * mam_fc_forward_workspace_for() is the same query for a given operand layout and output set
  * (with_indices: mam_fc_forward, else mam_fc_forward_values) with room for what makes the call faster: copies of the
  * operands for MAM_W_KM weights and for K that is no multiple of 16 (1.5 to 3 times as fast), and the lists of large
- * calls (2^32 products and more; 2 to 12 times as fast).  A call whose workspace only has
+ * calls (2^32 products and more; 1.2 to 12 times as fast where the data suits
+ * them, 2 to 10 % slower where the device finds that it does not).  A call whose workspace only has
  * mam_fc_forward_workspace() bytes still works, without them.
  */
 size_t mam_fc_forward_workspace(int64_t N, int64_t K, int64_t M);
