@@ -7,15 +7,23 @@
 //
 // Lanes are output columns: a stored entry (r, k, v) adds v * b[k, :] to c[r, :], and b[k, c0..c0+255]
 // is one coalesced 1 KiB load for a wave (4 columns per lane).
-//   CSR: a wave owns one row for one tile of 256 columns; column indices and values are wave-uniform
+//   CSR: a wave owns one row for one panel of 256 columns; column indices and values are wave-uniform
 //        scalar loads; the loads of the next 8 entries are in flight while 8 are consumed; the row of c
-//        is written once, no atomics, no zero fill.
+//        is written once, no atomics, no zero fill.  Workgroups are numbered panel by panel and dealt out so that
+//        an XCD works on panels of its own: its L2 then holds the panel of b (1 KiB per row of b) instead of all
+//        eight fetching the same one, and c goes past it (non-temporal stores).  4096 x 4096 at 1 % x 4096 columns: 128 ->
+//        102 us, 27 TB/s of b rows (0.2 %: 58 -> 29 us; 10 %: 880 -> 870 us, 31.6 TB/s); 90 us where K = 2048 leaves
+//        room beside the panel.  Bound by the 64 bytes per clock and CU of the vector memory path (39 TB/s).
+//        Entries handed out by v_readlane from lane-held blocks that run on over the wave's rows: 116 us (97 registers, 4
+//        waves per SIMD); 2 columns per lane (panels of half the size): 150 us; 4 entries in flight: 108 us.
+//        Narrow c: two or four entries per load instead of idle lanes (4096 x 4096 at 5 %, 128 / 64 columns: 26 -> 17, 26 -> 11 us;
+//        256 columns 34 and 33 us, 4096 columns at 1 % 102 and 123 us).
 //   COO: entries may come in any order and may repeat, so c is cleared first; a wave takes 64
 //        consecutive entries, keeps a run of equal row indices in registers and flushes it with
 //        atomic adds when the row changes.  On row-sorted input (what Tensor.to_sparse() and
 //        coalesce() produce) that is about one flush per row and wave.
-// Products are fused multiply-adds in ascending entry order within a wave; sums that span waves
-// (COO only) are combined in no fixed order.
+// Products are fused multiply-adds in ascending entry order within a wave (narrow c: within each of the two or four
+// parts of a row); sums that span waves (COO only) are combined in no fixed order.
 #include "mam_common.h"
 
 namespace mam {
@@ -27,6 +35,8 @@ constexpr int COO_CHUNK = 64;  // entries per wave and pass
 
 typedef const __attribute__((address_space(4))) int64_t const_i64;
 typedef const __attribute__((address_space(4))) float const_f32;
+
+template <int N> struct Count { static constexpr int value = N; };
 
 template <int TI> struct Vec;
 template <> struct Vec<1> { typedef float type; };
@@ -41,41 +51,85 @@ __device__ __forceinline__ void axpy(float (&acc)[4], float v, const float4 &b)
     acc[3] = __builtin_fmaf(v, b.w, acc[3]);
 }
 
-// TI = 4: b rows and c rows are 16-byte aligned and C is a multiple of 4; TI = 1 otherwise.
-template <int TI>
+// four consecutive words, 4-byte aligned
+typedef float words4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void store4(float *dst, const float (&a)[4])
+{
+    const words4 v = {a[0], a[1], a[2], a[3]};
+    __builtin_nontemporal_store(v, reinterpret_cast<words4 *>(dst));
+}
+__device__ __forceinline__ void store4(float *, const float (&)[1]) {}
+
+// PER: entries per load, each by 64 / PER lanes (NEAR only).
+// NEAR: b spans less than 4 GiB; a b row is then a buffer load with the row's byte offset in a scalar register, of any
+// alignment (a load of 4 words needs 4 bytes), and lanes past the last column read on into the next row or, past the end
+// of b, zeros.  Otherwise TI = 4 needs C a multiple of 4 and 16-byte aligned rows.
+template <int TI, bool NEAR, int PER>
 __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict__ crow,
                                                       const int64_t *__restrict__ col,
                                                       const float *__restrict__ val,
-                                                      const float *__restrict__ b, int64_t ldb,
-                                                      float *__restrict__ c, int R, int C)
+                                                      const float *__restrict__ b, int64_t ldb, uint32_t b_bytes,
+                                                      float *__restrict__ c, int R, int C, int row_blocks)
 {
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = blockIdx.x * (NT / 64) + wave;
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int panel = logical / row_blocks;
+    const int r = (logical - panel * row_blocks) * (NT / 64) + wave;
     if (r >= R) return;
-    const int c0 = blockIdx.y * 64 * TI + lane * TI;
-    const bool live = c0 < C;
-    const int cl = live ? c0 : 0;  // lanes past the last column read column 0 and store nothing
+    constexpr int LANES = 64 / PER;      // of one entry; the parts are added at the end
+    const int c0 = panel * LANES * TI + lane % LANES * TI;
+    const int cl = c0 < C ? c0 : 0;  // lanes past the last column read column 0 and store nothing
+    const int part = lane / LANES;
 
     const_i64 *ccol = (const_i64 *)col;
     const_f32 *cval = (const_f32 *)val;
     const int64_t beg = ((const_i64 *)crow)[r], end = ((const_i64 *)crow)[r + 1];
     const int nnz = (int)(end - beg);
     const float *bl = b + cl;
+    const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
+    const uint32_t row_bytes = (uint32_t)ldb * 4u;
+    auto near_row = [&](uint32_t lane_bytes, uint32_t bytes) {
+        return __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(near, lane_bytes, bytes, 0));
+    };
+    auto b_row = [&](int64_t e) -> vec {
+        if constexpr (PER > 1) {
+            uint32_t at = (uint32_t)ccol[e] * row_bytes;
+#pragma unroll
+            for (int p = 1; p < PER; ++p) {
+                const uint32_t other = (uint32_t)ccol[e + p] * row_bytes;
+                at = part == p ? other : at;
+            }
+            return near_row(at + cl * 4, 0);
+        } else if constexpr (NEAR) {
+            return near_row(cl * 4, (uint32_t)ccol[e] * row_bytes);
+        } else {
+            return *reinterpret_cast<const vec *>(bl + ccol[e] * ldb);
+        }
+    };
+    auto value = [&](int64_t e) {
+        float v = cval[e];
+#pragma unroll
+        for (int p = 1; p < PER; ++p) {
+            const float other = cval[e + p];
+            v = part == p ? other : v;
+        }
+        return v;
+    };
 
     float acc[TI];
 #pragma unroll
     for (int t = 0; t < TI; ++t) acc[t] = 0.0f;
 
-    const int ng = nnz / EG;
+    const int ng = nnz / (EG * PER);
     vec xa[EG], xb[EG];
     float wa[EG], wb[EG];
     auto issue = [&](int g, vec (&xv)[EG], float (&wv)[EG]) {
 #pragma unroll
         for (int u = 0; u < EG; ++u) {
-            xv[u] = *reinterpret_cast<const vec *>(bl + ccol[beg + g * EG + u] * ldb);
-            wv[u] = cval[beg + g * EG + u];
+            xv[u] = b_row(beg + (g * EG + u) * PER);
+            wv[u] = value(beg + (g * EG + u) * PER);
         }
     };
     auto consume = [&](const vec (&xv)[EG], const float (&wv)[EG]) {
@@ -94,17 +148,42 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
         consume(xb, wb);
         __builtin_amdgcn_sched_barrier(0);
     }
-    for (int i = ng * EG; i < nnz; ++i) {
-        const vec xv = *reinterpret_cast<const vec *>(bl + ccol[beg + i] * ldb);
-        axpy(acc, cval[beg + i], xv);
-    }
-    if (live) {
-        float *dst = c + (int64_t)r * C + c0;
-        if (TI == 4) {
-            *reinterpret_cast<float4 *>(dst) = make_float4(acc[0], acc[TI > 1 ? 1 : 0], acc[TI > 2 ? 2 : 0], acc[TI > 3 ? 3 : 0]);
-        } else {
-            dst[0] = acc[0];
+    int i = ng * EG * PER;
+    auto few = [&](auto count) {
+        constexpr int n = decltype(count)::value;
+        if (nnz - i < n * PER) return;
+        vec x[n];
+        float w[n];
+#pragma unroll
+        for (int u = 0; u < n; ++u) {
+            x[u] = b_row(beg + i + u * PER);
+            w[u] = value(beg + i + u * PER);
         }
+#pragma unroll
+        for (int u = 0; u < n; ++u) axpy(acc, w[u], x[u]);
+        i += n * PER;
+    };
+    few(Count<4>());
+    few(Count<2>());
+    few(Count<1>());
+    if constexpr (PER > 1) {
+        if (i + part < nnz) {            // fewer entries than parts
+            const int64_t e = beg + i + part;
+            axpy(acc, val[e], near_row((uint32_t)col[e] * row_bytes + cl * 4, 0));
+        }
+    }
+#pragma unroll
+    for (int s = LANES; s < 64; s <<= 1)
+#pragma unroll
+        for (int t = 0; t < TI; ++t) acc[t] += __shfl_xor(acc[t], s);
+    if (part != 0) return;
+    float *dst = c + (int64_t)r * C + c0;
+    if (TI == 4 && c0 + 3 < C) {
+        store4(dst, acc);
+    } else {
+#pragma unroll
+        for (int t = 0; t < TI; ++t)
+            if (c0 + t < C) dst[t] = acc[t];
     }
 }
 
@@ -116,28 +195,38 @@ __device__ __forceinline__ void flush_row(float *__restrict__ c, int64_t row, in
         float *dst = c + row * C + c0;
 #pragma unroll
         for (int t = 0; t < TI; ++t) {
-            unsafeAtomicAdd(dst + t, acc[t]);
+            if (c0 + t < C) unsafeAtomicAdd(dst + t, acc[t]);
             acc[t] = 0.0f;
         }
     }
 }
 
-template <int TI>
+// Panels go to the XCDs as in csr_spmm_kernel, and b rows are read as there.
+template <int TI, bool NEAR>
 __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict__ row,
                                                       const int64_t *__restrict__ col,
                                                       const float *__restrict__ val, int64_t nnz,
-                                                      const float *__restrict__ b, int64_t ldb,
-                                                      float *__restrict__ c, int C)
+                                                      const float *__restrict__ b, int64_t ldb, uint32_t b_bytes,
+                                                      float *__restrict__ c, int C, int chunk_blocks)
 {
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int64_t e0 = ((int64_t)blockIdx.x * (NT / 64) + wave) * COO_CHUNK;
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    const int panel = logical / chunk_blocks;
+    const int64_t e0 = ((int64_t)(logical - panel * chunk_blocks) * (NT / 64) + wave) * COO_CHUNK;
     if (e0 >= nnz) return;
     const int n = (int)((nnz - e0) < COO_CHUNK ? (nnz - e0) : COO_CHUNK);
-    const int c0 = blockIdx.y * 64 * TI + lane * TI;
+    const int c0 = panel * 64 * TI + lane * TI;
     const bool live = c0 < C;
-    const float *bl = b + (live ? c0 : 0);
+    const int cl = live ? c0 : 0;
+    const float *bl = b + cl;
+    const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
+    const uint32_t row_bytes = (uint32_t)ldb * 4u;
+    auto b_row = [&](int64_t k) -> vec {
+        if constexpr (NEAR) return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(near, cl * 4, (uint32_t)k * row_bytes, 0));
+        else return *reinterpret_cast<const vec *>(bl + k * ldb);
+    };
 
     const_i64 *crow = (const_i64 *)row;
     const_i64 *ccol = (const_i64 *)col;
@@ -147,7 +236,7 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
     for (int t = 0; t < TI; ++t) acc[t] = 0.0f;
     int64_t cur = crow[e0];
     for (int i = 0; i < n; i += EG) {
-        // loads of up to EG entries first; entries past the end repeat the last one with weight 0
+        // loads of up to EG entries first; entries past the end repeat the last one and are not added
         vec xv[EG];
         float wv[EG];
         int64_t rv[EG];
@@ -155,8 +244,8 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
         for (int u = 0; u < EG; ++u) {
             const bool ok = i + u < n;
             const int64_t e = e0 + (ok ? i + u : n - 1);
-            xv[u] = *reinterpret_cast<const vec *>(bl + ccol[e] * ldb);
-            wv[u] = ok ? cval[e] : 0.0f;
+            xv[u] = b_row(ccol[e]);
+            wv[u] = cval[e];
             rv[u] = crow[e];
         }
 #pragma unroll
@@ -165,7 +254,7 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
                 flush_row<TI>(c, cur, C, c0, live, acc);
                 cur = rv[u];
             }
-            axpy(acc, wv[u], xv[u]);
+            if (i + u < n) axpy(acc, wv[u], xv[u]);
         }
     }
     flush_row<TI>(c, cur, C, c0, live, acc);
@@ -250,18 +339,21 @@ extern "C" int mam_csr_spmm(const int64_t *crow, const int64_t *col, const float
     if (rc != MAM_OK || R == 0 || C == 0) return rc;
     if (!crow) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const unsigned gx = (unsigned)ceil_div(R, spmm::NT / 64);
-    if (spmm::wide(b, ldb, c, C)) {
-        const int64_t gy = ceil_div(C, 256);
-        if (gy > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-        hipLaunchKernelGGL((spmm::csr_spmm_kernel<4>), dim3(gx, (unsigned)gy), dim3(spmm::NT), 0, st, crow, col,
-                           val, b, ldb, c, (int)R, (int)C);
-    } else {
-        const int64_t gy = ceil_div(C, 64);
-        if (gy > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-        hipLaunchKernelGGL((spmm::csr_spmm_kernel<1>), dim3(gx, (unsigned)gy), dim3(spmm::NT), 0, st, crow, col,
-                           val, b, ldb, c, (int)R, (int)C);
-    }
+    const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
+    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
+    const int per = !near ? 1 : C <= 64 ? 4 : C <= 128 ? 2 : 1;          // entries per load
+    const int64_t panels = ceil_div(C, near || wide ? 256 / per : 64);
+    const int64_t row_blocks = ceil_div(R, spmm::NT / 64);
+    if (panels * row_blocks > INT32_MAX / 4) return fail(MAM_ERR_UNSUPPORTED, "too many rows and columns for the SpMM grid");
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(panels * row_blocks)), dim3(spmm::NT), 0, st, crow, col, val, b, ldb,
+                           (uint32_t)b_bytes, c, (int)R, (int)C, (int)row_blocks);
+    };
+    if (per == 4) launch(spmm::csr_spmm_kernel<4, true, 4>);
+    else if (per == 2) launch(spmm::csr_spmm_kernel<4, true, 2>);
+    else if (near) launch(spmm::csr_spmm_kernel<4, true, 1>);
+    else if (wide) launch(spmm::csr_spmm_kernel<4, false, 1>);
+    else launch(spmm::csr_spmm_kernel<1, false, 1>);
     return check_launch("csr_spmm_kernel");
 }
 
@@ -279,17 +371,17 @@ extern "C" int mam_coo_spmm(const int64_t *row, const int64_t *col, const float 
     if (!row || !col || !val) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     const int64_t gx = ceil_div(nnz, (int64_t)spmm::COO_CHUNK * (spmm::NT / 64));
     if (gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "too many entries for the SpMM grid");
-    if (spmm::wide(b, ldb, c, C)) {
-        const int64_t gy = ceil_div(C, 256);
-        if (gy > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-        hipLaunchKernelGGL((spmm::coo_spmm_kernel<4>), dim3((unsigned)gx, (unsigned)gy), dim3(spmm::NT), 0, st,
-                           row, col, val, nnz, b, ldb, c, (int)C);
-    } else {
-        const int64_t gy = ceil_div(C, 64);
-        if (gy > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-        hipLaunchKernelGGL((spmm::coo_spmm_kernel<1>), dim3((unsigned)gx, (unsigned)gy), dim3(spmm::NT), 0, st,
-                           row, col, val, nnz, b, ldb, c, (int)C);
-    }
+    const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
+    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
+    const int64_t panels = ceil_div(C, near || wide ? 256 : 64);
+    if (panels * gx > INT32_MAX / 4) return fail(MAM_ERR_UNSUPPORTED, "too many entries and columns for the SpMM grid");
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(panels * gx)), dim3(spmm::NT), 0, st, row, col, val, nnz, b, ldb,
+                           (uint32_t)b_bytes, c, (int)C, (int)gx);
+    };
+    if (near) launch(spmm::coo_spmm_kernel<4, true>);
+    else if (wide) launch(spmm::coo_spmm_kernel<4, false>);
+    else launch(spmm::coo_spmm_kernel<1, false>);
     return check_launch("coo_spmm_kernel");
 }
 

@@ -50,6 +50,31 @@ def test_csr_and_coo_against_oracle(rows, k, cols, rate):
     _check(c2, want, floor, "coo")
 
 
+@pytest.mark.parametrize("cols", [2, 3, 63, 64, 65, 126, 128, 131, 255, 257, 516])
+def test_column_counts_around_the_panels(cols):
+    """One, two or four entries per load, ragged last panels, b rows of any alignment; rows of 0 to 70 entries end in
+    every remainder of a group, and the last row of b ends the allocation."""
+    from mamtorch_amd import capi
+
+    rows, k = 71, 150
+    g = torch.Generator().manual_seed(cols)
+    a = torch.zeros(rows, k)
+    for r in range(rows):
+        a[r, torch.randperm(k, generator=g)[:r]] = torch.randn(r, generator=g)
+    a[:, k - 1] = 1.0
+    csr = a.to_sparse_csr()
+    crow, col, val = (t.to(DEV) for t in (csr.crow_indices(), csr.col_indices(), csr.values()))
+    coo = a.to_sparse_coo().coalesce()
+    idx, values = coo.indices().to(DEV), coo.values().to(DEV)
+    for offset in (0, 1):                       # words past a 16-byte boundary
+        store = torch.randn(offset + k * cols, generator=g)
+        b = store[offset:].view(k, cols)
+        want, floor = oracle.csr_spmm(crow.cpu().numpy(), col.cpu().numpy(), val.cpu().numpy(), b.numpy())
+        bd = store.to(DEV)[offset:].view(k, cols)
+        _check(capi.csr_spmm(crow, col, val, bd, rows), want, floor, "csr, offset %d" % offset)
+        _check(capi.coo_spmm(idx[0].contiguous(), idx[1].contiguous(), values, bd, rows), want, floor, "coo, offset %d" % offset)
+
+
 def test_coo_unsorted_with_duplicates_and_strided_b():
     from mamtorch_amd import capi
 
