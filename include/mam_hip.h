@@ -300,6 +300,11 @@ int mam_csr_spmm(const int64_t *crow, const int64_t *col, const float *val, cons
                  float *c, int64_t R, int64_t K, int64_t C, void *stream);
 int mam_coo_spmm(const int64_t *row, const int64_t *col, const float *val, int64_t nnz, const float *b,
                  int64_t ldb, float *c, int64_t R, int64_t K, int64_t C, void *stream);
+/*
+ * crow (R+1) of a COO operand whose rows ascend (a coalesced torch COO tensor): with its col / val it is then the CSR
+ * operand of the same matrix.  Offsets lie in 0 .. nnz whatever the rows are.
+ */
+int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, void *stream);
 
 /*
  * The sparse operand written out as a dense (R, K) fp32 matrix with row stride ld (cleared first; repeated

@@ -37,7 +37,7 @@ EXPORTS = (
     "mam_fc_backward", "mam_fc_backward_count", "mam_selection_count",
     "mam_fc_forward_ranges_workspace", "mam_fc_forward_ranges", "mam_fc_backward_ranges",
     "mam_csr_fc_forward_workspace", "mam_csr_fc_forward", "mam_csr_fc_backward", "mam_csr_validate",
-    "mam_csr_spmm", "mam_coo_spmm", "mam_csr_to_dense", "mam_coo_to_dense",
+    "mam_csr_spmm", "mam_coo_spmm", "mam_coo_row_offsets", "mam_csr_to_dense", "mam_coo_to_dense",
     "mam_blend", "mam_bias_grad_workspace", "mam_bias_grad", "mam_apply_keep", "mam_im2col", "mam_col2im",
     "mam_prune_row_offsets", "mam_prune_fill_csr", "mam_prune_apply",
     "mam_select_workspace", "mam_select_begin", "mam_select_accumulate", "mam_select_advance", "mam_select_result",
@@ -97,6 +97,7 @@ def lib():
         l.mam_csr_validate.argtypes = [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr]
         l.mam_csr_spmm.argtypes = [_ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr]
         l.mam_coo_spmm.argtypes = [_ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr]
+        l.mam_coo_row_offsets.argtypes = [_ptr, _i64, _ptr, _i64, _ptr]
         l.mam_csr_to_dense.argtypes = [_ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr]
         l.mam_coo_to_dense.argtypes = [_ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr]
         _f = ctypes.c_float
@@ -305,6 +306,15 @@ def csr_spmm(crow, col, val, b, R):
     with torch.cuda.device(b.device):
         _check(l.mam_csr_spmm(_p(crow), _p(col), _p(val), _p(b), _ld(b), _p(c), R, K, C, _stream(b)))
     return c
+
+
+def coo_row_offsets(row, R):
+    """crow (R+1) of ascending row indices."""
+    l = lib()
+    crow = torch.empty(R + 1, dtype=torch.int64, device=row.device)
+    with torch.cuda.device(row.device):
+        _check(l.mam_coo_row_offsets(_p(row), row.numel(), _p(crow), R, _stream(row)))
+    return crow
 
 
 def coo_spmm(row, col, val, b, R):

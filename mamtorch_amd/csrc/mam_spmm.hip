@@ -260,6 +260,26 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
     flush_row<TI>(c, cur, C, c0, live, acc);
 }
 
+// crow[r] = entries whose row is below r, for rows in ascending order.  A wave per r narrows the place down to one entry
+// 64-fold a step (four steps for 2^24 entries); for rows in any other order it ends all the same, inside 0 .. nnz.
+__global__ __launch_bounds__(NT) void row_offsets_kernel(const int64_t *__restrict__ row, int64_t nnz,
+                                                         int64_t *__restrict__ crow, int64_t R)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t r = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
+    if (r > R) return;
+    int64_t lo = 0, count = nnz;          // the place is one of lo .. lo + count
+    while (count > 0) {
+        const int64_t step = (count + 63) >> 6, at = lo + (lane + 1) * step - 1;
+        const int below = __popcll(__ballot(at < lo + count && row[at < nnz ? at : nnz - 1] < r));
+        const int64_t end = lo + count;
+        lo += below * step;
+        // the next probe was not below r (or lay past the end): what is left lies before it
+        count = (end - lo) < step - 1 ? end - lo : step - 1;
+    }
+    if (lane == 0) crow[r] = lo;
+}
+
 static int check_common(const float *b, int64_t ldb, float *c, int64_t R, int64_t K, int64_t C)
 {
     if (R < 0 || K < 0 || C < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
@@ -383,6 +403,17 @@ extern "C" int mam_coo_spmm(const int64_t *row, const int64_t *col, const float 
     else if (wide) launch(spmm::coo_spmm_kernel<4, false>);
     else launch(spmm::coo_spmm_kernel<1, false>);
     return check_launch("coo_spmm_kernel");
+}
+
+extern "C" int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, void *stream)
+{
+    using namespace mam;
+    if (nnz < 0 || R < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
+    if (R > INT32_MAX / 2) return fail(MAM_ERR_UNSUPPORTED, "a dimension exceeds 2^30");
+    if (!crow || (nnz > 0 && !row)) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
+    hipLaunchKernelGGL(spmm::row_offsets_kernel, dim3((unsigned)ceil_div(R + 1, spmm::NT / 64)), dim3(spmm::NT), 0,
+                       static_cast<hipStream_t>(stream), row, nnz, crow, R);
+    return check_launch("row_offsets_kernel");
 }
 
 extern "C" int mam_csr_to_dense(const int64_t *crow, const int64_t *col, const float *val, float *dense, int64_t ld,

@@ -503,9 +503,9 @@ void check_spmm_operands(const at::Tensor &a, const at::Tensor &b)
 // dense fp32 GEMM over the zero-filled operand: the operand is written out dense (one pass) and the
 // product is the platform's library GEMM.  4096 x 4096 x 4096: 3.06 -> ~1.05 ms at 30 % density; the two
 // routes cross at ~10 %.
-// `one_in`: the density from which the route is taken, one stored entry in `one_in`: 8 for CSR; 16 for COO,
-// whose kernel (any order, duplicates, atomics) takes about twice the CSR kernel's time per entry (4096^3 at
-// 10 % density: 1.89 against 1.05 ms, the GEMM 0.99 ms).
+// `one_in`: the density from which the route is taken, one stored entry in `one_in`: 8 for the CSR kernel; 16 for the
+// COO kernel (any order, duplicates, atomics), which takes about twice as long per entry (4096^3 at
+// 10 % density: 1.89 against 0.87 ms, the GEMM 0.99 ms).
 bool dense_route_pays(int64_t nnz, int64_t R, int64_t K, int64_t C, int64_t one_in)
 {
     return R > 0 && K > 0 && C >= 64 && nnz >= (R * K + one_in - 1) / one_in && R * K <= (int64_t(1) << 29);
@@ -546,7 +546,11 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     const at::Tensor idx = a._indices().to(at::kLong).contiguous();   // (2, nnz); need not be coalesced
     const at::Tensor val = a._values().contiguous();
     const int64_t nnz = val.numel();
-    if (dense_route_pays(nnz, R, K, C, 16)) {
+    // A coalesced operand's rows ascend: with row offsets it is a CSR operand, whose kernel adds a row up in registers instead of
+    // clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns: 364 -> 107 us).  A row is one wave's there, at most K / 8 rounds of
+    // loads, 0.4 us each: not for K so large that one crowded row would outlast the COO kernel.
+    const bool by_rows = a.is_coalesced() && K <= 32768;
+    if (dense_route_pays(nnz, R, K, C, by_rows ? 8 : 16)) {
         auto dense = at::empty({R, K}, b.options());
         check_rc(mam_coo_to_dense(idx.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(), nnz,
                                   dense.data_ptr<float>(), K, R, K, current_stream(b)),
@@ -555,6 +559,15 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     }
     auto c = at::empty({R, C}, b.options());
     if (R == 0 || C == 0) return c;
+    if (by_rows) {
+        const at::Tensor crow = at::empty({R + 1}, idx.options());
+        check_rc(mam_coo_row_offsets(idx.data_ptr<int64_t>(), nnz, crow.data_ptr<int64_t>(), R, current_stream(b)),
+                 "mam_coo_row_offsets");
+        check_rc(mam_csr_spmm(crow.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(),
+                              b.data_ptr<float>(), row_stride(b, "b"), c.data_ptr<float>(), R, K, C, current_stream(b)),
+                 "mam_csr_spmm");
+        return c;
+    }
     check_rc(mam_coo_spmm(idx.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(), nnz,
                           b.data_ptr<float>(), row_stride(b, "b"), c.data_ptr<float>(), R, K, C,
                           current_stream(b)),

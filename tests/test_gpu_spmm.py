@@ -75,6 +75,17 @@ def test_column_counts_around_the_panels(cols):
         _check(capi.coo_spmm(idx[0].contiguous(), idx[1].contiguous(), values, bd, rows), want, floor, "coo, offset %d" % offset)
 
 
+@pytest.mark.parametrize("nnz,rows", [(0, 5), (1, 1), (63, 9), (64, 300), (65, 3), (4096, 70), (4097, 1), (300000, 4001)])
+def test_row_offsets(nnz, rows):
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(nnz)
+    row = torch.randint(0, rows, (nnz,), generator=g) ** 2 // max(rows - 1, 1)      # crowded first rows, empty ones
+    row = row.clamp(max=rows - 1).sort()[0]
+    got = capi.coo_row_offsets(row.to(DEV), rows).cpu()
+    assert torch.equal(got, torch.searchsorted(row, torch.arange(rows + 1)))
+
+
 def test_coo_unsorted_with_duplicates_and_strided_b():
     from mamtorch_amd import capi
 
