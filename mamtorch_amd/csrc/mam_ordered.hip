@@ -26,10 +26,9 @@
 //   dense kernels  exit at once unless the decision was "none".
 //
 // Measured against the dense tilings (forward call, hand-over arrays written).  Uniform weights or inputs, one-sided:
-// 207 -> 67 to 75 us at 256 x 4096 x 4096, 1.70 -> 0.63 ms and 1.48 -> 0.25 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.84 ms
-// (values only) and 3.13 -> 0.42 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.43 ms
-// at 12608 x 768 -> 3072, 3.12 -> 1.07 ms at 16384 x 4096 -> 1024, 0.84 -> 0.44 ms at 4096 x 2048 x 2048.  A wave's search
-// ends with the slowest of its 256 outputs: 92 entries at K = 4096 where the mean output needs 28.
+// 207 -> 60 to 67 us at 256 x 4096 x 4096, 1.70 -> 0.49 ms and 1.48 -> 0.24 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.74 ms
+// (values only) and 3.13 -> 0.36 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.36 ms
+// at 12608 x 768 -> 3072, 3.12 -> 0.92 ms at 16384 x 4096 -> 1024, 0.84 -> 0.43 ms at 4096 x 2048 x 2048.
 #include "mam_ordered.h"
 
 #include <math.h>
@@ -530,6 +529,25 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
 }
 
 // ---- search ------------------------------------------------------------------------------------------------
+typedef uint32_t words4 __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(1))) words4 global_words4;
+typedef const __attribute__((address_space(1))) float global_float;
+typedef const __attribute__((address_space(1))) char global_bytes;
+// Address in the LDS of a key's place in a column: upper half times the bytes from one k to the next, on top of the
+// column's. One instruction (the compiler takes two).
+template <int BYTES>
+__device__ __forceinline__ uint32_t lds_place(uint32_t key, uint32_t column)
+{
+    uint32_t at;
+    asm("v_mad_u32_u16 %0, %1, %2, %3 op_sel:[1,0,0,0]" : "=v"(at) : "v"(key), "s"(BYTES), "v"(column));
+    return at;
+}
+typedef const __attribute__((address_space(3))) char lds_bytes;
+template <class T>
+__device__ __forceinline__ T lds_read(uint32_t at) { return *(const __attribute__((address_space(3))) T *)(uintptr_t)at; }
+__device__ __forceinline__ uint32_t lds_address(const float *p) { return (uint32_t)(uintptr_t)(lds_bytes *)p; }
+typedef float floats4 __attribute__((ext_vector_type(4)));
+
 // The two running extremes of an output are kept as doubles whose high word is the fp32 product and whose low
 // word is the entry's key: for products of one sign, doubles order by (product, lower k first), so v_max_f64 /
 // v_min_f64 keep value AND first index in one instruction, in any order of k.  (A product of the wrong sign never decides: an
@@ -587,14 +605,22 @@ struct Extremes<true> {
         max64(a, d);
         min64(b, d);
     }
-    static __device__ __forceinline__ void merge(value &a, value &b, int from)
+    static __device__ __forceinline__ void both(value &a, value &b, const uint4 &it, float w0, float w1)
     {
-        max64(a, lane_value_at(a, from));
-        min64(b, lane_value_at(b, from));
+        both(a, b, __uint_as_float(it.x) * w0, it.y);
+        both(a, b, __uint_as_float(it.z) * w1, it.w);
     }
+    // a running extreme whose entry is another lane's to know: below every listed entry of the same product
+    static __device__ __forceinline__ value start(float product) { return keyed(product, 0); }
+    static __device__ __forceinline__ void merge(value &a, value &b, value theirs_a, value theirs_b, int from)
+    {
+        max64(a, lane_value_at(theirs_a, from));
+        min64(b, lane_value_at(theirs_b, from));
+    }
+    static __device__ __forceinline__ void merge(value &a, value &b, int from) { merge(a, b, a, b, from); }
     // one pair of list entries against 4 tile values each.  Written out because the compiler copies the key into the low
     // word of every key: here two register pairs hold it for the four products of an entry.
-    __device__ __forceinline__ void entry(float x, uint32_t key, const float4 &w)
+    __device__ __forceinline__ void entry(float x, uint32_t key, const floats4 &w)
     {
         asm("v_mov_b32 v120, %9\n\tv_mov_b32 v122, %9\n\t"
             "v_mul_f32 v121, %8, %10\n\tv_mul_f32 v123, %8, %11\n\t"
@@ -608,7 +634,7 @@ struct Extremes<true> {
             : "v"(x), "v"(key), "v"(w.x), "v"(w.y), "v"(w.z), "v"(w.w)
             : "v120", "v121", "v122", "v123");
     }
-    __device__ __forceinline__ void entries(const uint4 &it, const float4 &w0, const float4 &w1)
+    __device__ __forceinline__ void entries(const uint4 &it, const floats4 &w0, const floats4 &w1)
     {
         entry(__uint_as_float(it.x), it.y, w0);
         entry(__uint_as_float(it.z), it.w, w1);
@@ -628,12 +654,20 @@ struct Extremes<false> {
         a = __builtin_fmaxf(a, product);
         b = __builtin_fminf(b, product);
     }
-    static __device__ __forceinline__ void merge(value &a, value &b, int from)
+    static __device__ __forceinline__ void both(value &a, value &b, const uint4 &it, float w0, float w1)
     {
-        a = __builtin_fmaxf(a, lane_value_at(a, from));
-        b = __builtin_fminf(b, lane_value_at(b, from));
+        const float p0 = __uint_as_float(it.x) * w0, p1 = __uint_as_float(it.z) * w1;
+        a = __builtin_fmaxf(__builtin_fmaxf(a, p0), p1);
+        b = __builtin_fminf(__builtin_fminf(b, p0), p1);
     }
-    __device__ __forceinline__ void entries(const uint4 &it, const float4 &w0, const float4 &w1)
+    static __device__ __forceinline__ value start(float product) { return product; }
+    static __device__ __forceinline__ void merge(value &a, value &b, value theirs_a, value theirs_b, int from)
+    {
+        a = __builtin_fmaxf(a, lane_value_at(theirs_a, from));
+        b = __builtin_fminf(b, lane_value_at(theirs_b, from));
+    }
+    static __device__ __forceinline__ void merge(value &a, value &b, int from) { merge(a, b, a, b, from); }
+    __device__ __forceinline__ void entries(const uint4 &it, const floats4 &w0, const floats4 &w1)
     {
         const float x0 = __uint_as_float(it.x), x1 = __uint_as_float(it.z);
         const float f0[4] = {w0.x, w0.y, w0.z, w0.w}, f1[4] = {w1.x, w1.y, w1.z, w1.w};
@@ -787,14 +821,19 @@ __device__ __forceinline__ void scan_row(const float *src, int K, const float *b
 // listed row x 4 consecutive tile rows, and TB / 4 neighbouring lanes share a listed row, so that an entry costs
 // each lane one 16-byte LDS read for 4 products and the lanes of a row read TB * 4 contiguous bytes.  Waves take
 // blocks of 64 * 4 / TB listed rows in turn and need no barrier after the tile is loaded.  A wave looks at its
-// lists chunk by chunk until all but FEW of its 256 outputs are finished by their bound, and then finishes those
-// one by one with all its lanes (FEW = 0, 1, 2, 4: 75 / 72 / 72 / 73 us at 256 x 4096 x 4096, 608 / 593 / 593 / 602 us at
-// 16384 x 4096 -> 1024, while the selected operands still came from the row).  Bound: v_max_f64 / v_min_f64 where rows
-// are many (at 4 cycles each, VALU instructions take 0.76 of the busy cycles at 12608 x 768 -> 3072, and those two hold the unit longer);
-// the random 16-byte LDS reads take half of the cycles beside them, two to three fifths of it bank conflicts.  256 x 4096 -> 4096: 0.44,
-// for each workgroup waits 14 us for its tile and half of its waves have no rows.  (9.9 T products/s in a loop of its own against 14.3 T with fp32 extremes and no
-// indices.)
-constexpr int FEW = 2;
+// lists chunk by chunk until TOGETHER of its 256 outputs are not yet finished by their bound (53 entries at K = 4096, where all but
+// FEW take 90 and the mean output needs 28), then goes on with a lane for each of those -- one product per entry instead of four of
+// which most are decided -- and finishes the last FEW one by one with all its lanes.  (Us; TOGETHER, FEW = none, 2 / 32, 2 / 64, 2 / 64, 1 /
+// 48, 1 / 64, 0: 256 x 4096 x 4096 65.8 / 63.3 / 62.3 / 61.0 / 60.5 / 61.7, 12608 x 768 -> 3072 587 / 581 / 577 / 566 / 560 / 560, 16384 x 4096 ->
+// 4096 values only 752 / 756 / 758 / 751 / 745 / 779, 16384 x 4096 -> 1024 405 / 394 / 386 / 385 / 383 / 396.  Handing lanes out anew at every
+// quarter, 1 to 64 an output, costs more in exchanges than it saves: 64.0 / 625 / 898 / 422.)
+// What bounds it (counters, values only at K = 4096): VALU instructions at 4 cycles take 0.63 of the busy cycles, the random
+// 16-byte LDS reads 0.67 (three fifths of it bank conflicts), list entries on their way from the caches to the registers 0.95
+// -- but with the lanes of a row loading a quarter or half of its entries each and passing them round the quad the calls take the
+// same: 562 / 735 / 384 us for 560 / 745 / 383.  16384 x 4096 -> 4096: 61 us before the search, 59 us of tile loads, 320 us until
+// TOGETHER, 260 us for those, 42 us for the last one.
+constexpr int FEW = 1;
+constexpr int TOGETHER = 48;         // at most a wave's lanes
 // Outputs of a row that are scanned one by one, 8 to 17 us each beside the other waves' work; the whole row takes 30 to 60 us.
 constexpr int FEW_OF_ROW = 4;
 
@@ -821,6 +860,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
     constexpr int Q = L::Q, RW = L::RW;
     extern __shared__ float tile[];         // the tile; two-sided: then [TB][lead] (value, key)
     __shared__ float tops[TB];
+    __shared__ uint8_t places[NT / 64][64];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Decision d = *p.decision;
@@ -916,7 +956,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         bmax[j] = t == 0.0f ? -1.0f : t < __builtin_inff() ? t : __builtin_nanf("");
     }
     const float *by_key = tile + L::base(q, K) + (K - 65536) * L::STRIDE;      // element (65535 - k) * STRIDE + row of the quad
-    const char *mine = reinterpret_cast<const char *>(by_key);
+    const uint32_t mine = lds_address(by_key);
     const int64_t pair_bytes = (int64_t)pad * 16, bound_bytes = (int64_t)pad * 4;
 
     // Stores with x searched: a row's outputs lie along the tile rows.  Two-sided, the lanes that hold them change places
@@ -981,22 +1021,35 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         }
         int ch = 0;
         uint64_t open[4];
-        auto fetch = [&](uint4 (&to)[CHUNK / 2], int chunk) {
-            const char *base = reinterpret_cast<const char *>(lists) + (int64_t)chunk * (CHUNK / 2) * pair_bytes;
-            asm volatile("" : "+s"(base));      // scalar base + 32-bit lane offset
+        // a chunk and the bound on what follows it, as global loads: flat ones would count as LDS accesses too, and every read of
+        // the tile would wait for them
+        auto fetch = [&](uint4 (&to)[CHUNK / 2], float &u, int chunk, uint32_t off) {
+            asm volatile("" : "+v"(off));       // scalar base + 32-bit lane offset: the offset is not widened outside the loop
+            u = *(global_float *)((global_bytes *)bound + (chunk + 1) * bound_bytes + (off >> 2));
+            global_bytes *base = (global_bytes *)lists + (int64_t)chunk * (CHUNK / 2) * pair_bytes;
 #pragma unroll
-            for (int i = 0; i < CHUNK / 2; ++i) to[i] = *reinterpret_cast<const uint4 *>(base + i * pair_bytes + list_off);
+            for (int i = 0; i < CHUNK / 2; ++i, base += pair_bytes) {
+                asm volatile("" : "+s"(base));
+                const words4 v = *(global_words4 *)(base + off);
+                to[i] = make_uint4(v.x, v.y, v.z, v.w);
+            }
         };
+        constexpr int AHEAD = 1;
         // true when the search is over
-        auto step = [&](const uint4 (&cur)[CHUNK / 2], uint4 (&nxt)[CHUNK / 2]) {
-            fetch(nxt, ch + 1 < chunks ? ch + 1 : ch);
-            const float u = *reinterpret_cast<const float *>(reinterpret_cast<const char *>(bound) + (ch + 1) * bound_bytes + bound_off);
+        auto step = [&](const uint4 (&cur)[CHUNK / 2], float u, uint4 (&nxt)[CHUNK / 2], float &unxt) {
+            fetch(nxt, unxt, ch + 1 < chunks ? ch + 1 : ch, list_off);
             asm volatile("" ::: "memory");      // the loads stay ahead of the arithmetic
 #pragma unroll
-            for (int i = 0; i < CHUNK / 2; ++i) {
-                const float4 w0 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].y >> 16) * (L::STRIDE * 4));
-                const float4 w1 = *reinterpret_cast<const float4 *>(mine + (int)(cur[i].w >> 16) * (L::STRIDE * 4));
-                e.entries(cur[i], w0, w1);
+            for (int i0 = 0; i0 < CHUNK / 2; i0 += AHEAD) {
+                floats4 w[2 * AHEAD];
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i) {
+                    w[2 * i] = lds_read<floats4>(lds_place<L::STRIDE * 4>(cur[i0 + i].y, mine));
+                    w[2 * i + 1] = lds_read<floats4>(lds_place<L::STRIDE * 4>(cur[i0 + i].w, mine));
+                }
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int i = 0; i < AHEAD; ++i) e.entries(cur[i0 + i], w[2 * i], w[2 * i + 1]);
             }
             ++ch;
             int left = 0;
@@ -1006,14 +1059,15 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                 open[j] = ~(__ballot(E::product(e.mx[j]) > ub) & __ballot(E::product(e.mn[j]) < -ub));
                 left += __popcll(open[j]);
             }
-            return left <= FEW || ch == chunks;
+            return left <= TOGETHER || ch == chunks;
         };
         {
             uint4 first[CHUNK / 2], second[CHUNK / 2];
-            fetch(first, 0);
+            float u1, u2;
+            fetch(first, u1, 0, list_off);
             while (true) {
-                if (step(first, second)) break;
-                if (step(second, first)) break;
+                if (step(first, u1, second, u2)) break;
+                if (step(second, u2, first, u1)) break;
             }
         }
         // the rows past the end are copies of the last one
@@ -1021,6 +1075,60 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         for (int j = 0; j < 4; ++j) open[j] &= __ballot(arow < a.rows);
         int own = lane;
         asm volatile("" : "+v"(own));           // what is derived from it below is not kept in registers during the search
+        // ---- the last TOGETHER outputs: a lane each instead of four on a lane of which most are finished ----
+        const int unfinished = __popcll(open[0]) + __popcll(open[1]) + __popcll(open[2]) + __popcll(open[3]);
+        if (unfinished > FEW && ch < chunks) {
+            int rank[4], before = 0;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                rank[j] = before + __builtin_amdgcn_mbcnt_hi((uint32_t)(open[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)open[j], 0));
+                if (open[j] >> own & 1) places[wave][rank[j]] = (uint8_t)(own * 4 + j);
+                before += __popcll(open[j]);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const int task = own < unfinished ? places[wave][own] : 0, from = task & ~3, tj = task & 3, tl = task >> 2;
+            const int trow = blk * RW + L::row(tl) < a.rows ? blk * RW + L::row(tl) : a.rows - 1;
+            uint4 first[CHUNK / 2], second[CHUNK / 2];
+            float u1, u2;
+            fetch(first, u1, ch, (uint32_t)trow * 16u);
+            typename E::value tmx = E::start(lane_value_at(E::product(e.mx[0]), from)), tmn = E::start(lane_value_at(E::product(e.mn[0]), from));
+            float tb = lane_value_at(bmax[0], from);
+#pragma unroll
+            for (int j = 1; j < 4; ++j) {
+                const float hi = lane_value_at(E::product(e.mx[j]), from), lo = lane_value_at(E::product(e.mn[j]), from);
+                const float bj = lane_value_at(bmax[j], from);
+                if (tj == j) { tmx = E::start(hi); tmn = E::start(lo); tb = bj; }
+            }
+            const uint32_t column = lds_address(tile + L::base(L::quad(tl), K) + (K - 65536) * L::STRIDE + tj);
+            const uint64_t used = (2ull << (unfinished - 1)) - 1;
+            uint64_t still;
+            auto tail = [&](const uint4 (&cur)[CHUNK / 2], float u, uint4 (&nxt)[CHUNK / 2], float &unxt) {
+                fetch(nxt, unxt, ch + 1 < chunks ? ch + 1 : ch, (uint32_t)trow * 16u);
+                asm volatile("" ::: "memory");
+#pragma unroll
+                for (int i = 0; i < CHUNK / 2; ++i) {
+                    const float w0 = lds_read<float>(lds_place<L::STRIDE * 4>(cur[i].y, column));
+                    const float w1 = lds_read<float>(lds_place<L::STRIDE * 4>(cur[i].w, column));
+                    E::both(tmx, tmn, cur[i], w0, w1);
+                }
+                ++ch;
+                const float ub = u * tb;
+                still = ~(__ballot(E::product(tmx) > ub) & __ballot(E::product(tmn) < -ub)) & used;
+                return __popcll(still) <= FEW || ch == chunks;
+            };
+            while (true) {
+                if (tail(first, u1, second, u2)) break;
+                if (tail(second, u2, first, u1)) break;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const bool mine = open[j] >> own & 1;
+                typename E::value hi = e.mx[j], lo = e.mn[j];
+                E::merge(hi, lo, tmx, tmn, rank[j] << 2);
+                if (mine) { e.mx[j] = hi; e.mn[j] = lo; }
+                open[j] = __ballot(mine && (still >> (rank[j] & 63) & 1));
+            }
+        }
         // (one copy of the code each: the output's state is picked by selects)
         if (ch < chunks) {
             uint64_t todo[4] = {open[0], open[1], open[2], open[3]};
@@ -1091,7 +1199,9 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                 const int m = lists_x ? b0 + q * 4 + j : arow;
                 if (c.bias && m < (int)c.M) sum[j] = sum[j] + c.bias[m];
             }
-            // uniform base of the block + 32-bit offset of the lane
+            // Stores that cover whole 128-byte lines go past the L2 (12608 x 768 -> 3072, seven planes: 560 -> 495 us,
+            // 16384 x 4096 -> 1024: 383 -> 363); narrower ones meet their neighbours' there (12608 x 3072 -> 768 past it: 238 ->
+            // 473 us).  Uniform base of the block + 32-bit offset of the lane.
             const int64_t base = lists_x ? (int64_t)blk * RW * c.M + b0 : (int64_t)b0 * c.M + blk * RW;
             auto put = [&](float *dst, const float (&v)[4]) {
                 float *to = dst + base;
@@ -1101,7 +1211,9 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                     for (int j = 0; j < 4; ++j) t[j] = TWO ? __int_as_float(__builtin_amdgcn_ds_bpermute(swap_from, __float_as_int(v[j]))) : v[j];
                     if (blk * RW + sr >= a.rows) {
                     } else if (whole && ((uintptr_t)dst & 15) == 0) {
-                        *reinterpret_cast<float4 *>(to + lane_off) = make_float4(t[0], t[1], t[2], t[3]);
+                        const floats4 all = {t[0], t[1], t[2], t[3]};
+                        if constexpr (TB == 32) __builtin_nontemporal_store(all, reinterpret_cast<floats4 *>(to + lane_off));
+                        else *reinterpret_cast<floats4 *>(to + lane_off) = all;
                     } else {
 #pragma unroll
                         for (int j = 0; j < 4; ++j)
@@ -1110,7 +1222,10 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                 } else if (arow < a.rows) {
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
-                        if (b0 + q * 4 + j < b.rows) to[lane_off + j * (uint32_t)c.M] = v[j];
+                        if (b0 + q * 4 + j < b.rows) {
+                            if constexpr (RW >= 32) __builtin_nontemporal_store(v[j], to + lane_off + j * (uint32_t)c.M);
+                            else to[lane_off + j * (uint32_t)c.M] = v[j];
+                        }
                 }
             };
             if constexpr (ARGS) {
@@ -1228,7 +1343,7 @@ static int setup_device(int)
         (const void *)forward_kernel<16, false, false>, (const void *)forward_kernel<32, false, false>,
         (const void *)forward_kernel<8, true, true>,    (const void *)forward_kernel<8, false, true>};
     for (const void *k : kernels)
-        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024) != hipSuccess) {
+        if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024) != hipSuccess) {
             (void)hipGetLastError();
             return fail(MAM_ERR_LAUNCH, "could not raise the LDS limit of the list kernels");
         }

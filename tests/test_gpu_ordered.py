@@ -21,6 +21,10 @@ def _data(kind, rows, k, g):
         t = t.relu()
     elif kind == "ties":
         t = (t * 4).round() / 4
+    elif kind == "levels":                  # as the lists like it, and many equal products
+        t = (t * 8).round() / 8
+    elif kind == "bounded levels":
+        t = ((r * 2 - 1) * 8).round() / 8
     elif kind == "positive":
         t = r + 0.1
     elif kind == "zero rows":
@@ -104,6 +108,14 @@ def test_sizes_on_both_sides_of_every_tile_width(N, K, M, kinds, layout_mk):
     if 768 <= K <= 9728 and "uniform" in kinds:
         # the rows of the normal operand are searched; a (K, M) weight's are not listed
         assert (side, lead) == ((1 if kinds[0] == "normal" else 2 if layout_mk else 0), 0)
+
+
+@pytest.mark.parametrize("N, K, M", [(8, 800, 32), (9, 800, 33), (65, 900, 97), (33, 2000, 41), (32, 3000, 9), (129, 3000, 66),
+                                     (64, 5000, 6)])       # 32, 16, 8, 4 tile rows; blocks of one row to all
+@pytest.mark.parametrize("kinds", [("levels", "bounded levels"), ("bounded levels", "levels"), ("levels", "levels")])
+def test_equal_products_met_by_different_lanes(N, K, M, kinds):
+    """A wave's last outputs are finished by lanes of their own: the first index wins wherever an equal product was met."""
+    _check(N, K, M, *kinds, seed=N)
 
 
 @pytest.mark.parametrize("kind", ["ties", "positive", "zero rows", "nan and inf", "sparse", "denormal", "overflow"])
