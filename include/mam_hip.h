@@ -197,6 +197,17 @@ int mam_fc_backward(const float *x, int64_t ldx, const float *w, int64_t ldw, in
                     const float *x_sel, float *x_grad, float *w_grad, int64_t N, int64_t K, int64_t M, void *stream);
 
 /*
+ * mam_fc_backward (range_len 0) or mam_fc_backward_ranges (w_sel and x_sel NULL or [plane][2][N*M]) and the bias gradient,
+ * bias_grad[m] = sum over the batch rows of grad[n, m], as ONE call: the launch that forms w_grad reads grad anyway and adds it up,
+ * in fp32 and in a fixed order.  `workspace`: mam_fc_backward_bias_workspace(N, K, M) bytes, NULL where that is 0.
+ */
+size_t mam_fc_backward_bias_workspace(int64_t N, int64_t K, int64_t M);
+int mam_fc_backward_bias(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
+                         const float *grad, const int32_t *argmax, const int32_t *argmin, const float *w_sel,
+                         const float *x_sel, float *x_grad, float *w_grad, float *bias_grad, int64_t N, int64_t K,
+                         int64_t M, int64_t range_len, void *workspace, size_t workspace_bytes, void *stream);
+
+/*
  * mam_fc_backward followed by mam_selection_count(argmax, argmin, max_count, min_count, ..., count_mode) as
  * ONE call: what a training step does after FullyConnected.forward when the layer keeps selection counts
  * (mamtorch/kernel/v4/csrc/cuda/fullyconnected_backward.cu:80-135 and then

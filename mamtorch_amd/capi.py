@@ -38,6 +38,7 @@ EXPORTS = (
     "mam_fc_forward_ranges_workspace", "mam_fc_forward_ranges", "mam_fc_backward_ranges",
     "mam_csr_fc_forward_workspace", "mam_csr_fc_forward", "mam_csr_fc_backward", "mam_csr_validate",
     "mam_csr_spmm", "mam_coo_spmm", "mam_coo_row_offsets", "mam_csr_to_dense", "mam_coo_to_dense",
+    "mam_fc_backward_bias_workspace", "mam_fc_backward_bias",
     "mam_blend", "mam_bias_grad_workspace", "mam_bias_grad", "mam_apply_keep", "mam_im2col", "mam_col2im",
     "mam_prune_row_offsets", "mam_prune_fill_csr", "mam_prune_apply",
     "mam_select_workspace", "mam_select_begin", "mam_select_accumulate", "mam_select_advance", "mam_select_result",
@@ -75,6 +76,9 @@ def lib():
                                               _size]
         l.mam_fc_forward_values.argtypes = [_ptr, _i64, _ptr, _i64, _int, _ptr, _ptr, _i64, _i64, _i64,
                                             _ptr, _size, _ptr]
+        l.mam_fc_backward_bias_workspace.argtypes = [_i64, _i64, _i64]
+        l.mam_fc_backward_bias_workspace.restype = ctypes.c_size_t
+        l.mam_fc_backward_bias.argtypes = [_ptr, _i64, _ptr, _i64, _int] + [_ptr] * 8 + [_i64] * 4 + [_ptr, ctypes.c_size_t, _ptr]
         l.mam_fc_backward.argtypes = [_ptr, _i64, _ptr, _i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
                                       _i64, _i64, _i64, _ptr]
         l.mam_fc_forward_ranges_workspace.restype = _size

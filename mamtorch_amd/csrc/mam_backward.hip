@@ -34,6 +34,7 @@ using namespace fixedpoint;
 
 constexpr int NT_X = 1024;
 constexpr int NT_W = 512;
+constexpr int MAX_NEURONS = 32;      // of a w_grad slab
 
 // ds_add_f32 costs ~3 cycles per active lane on this chip, ~190 per full 64-lane instruction,
 // whatever the addresses (an integer LDS atomic: ~5 per instruction, ~8 for 64 bits).  Only the fp32
@@ -422,6 +423,9 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
 // COUNT: the workgroup also owns the slab's selection counters (hits mode, mam_selcount.hip): the picks it
 // scatters are counted in a second LDS plane behind the histogram and added to max_count / min_count when the
 // slab is streamed out -- the index arrays are read once for both, and one launch serves both.
+// bias_out ([share][M], workgroups of the first k chunk): the sum of grad over the share's rows, from the items that are read
+// anyway; a thread's items lie in one quad of neurons, so it adds in registers and the threads of a quad are added in a
+// fixed order.
 template <int LAYOUT, int NT, bool COUNT = false>
 __device__ __forceinline__ void bwd_w_vec_body(
     float *hist, int bx, int nbx, int by, int bz, int nbz,
@@ -429,8 +433,11 @@ __device__ __forceinline__ void bwd_w_vec_body(
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
     const float *__restrict__ x_sel, int64_t nm, float *__restrict__ w_grad, int N, int K, int M, int log2r,
     int kc, int vec_out, int mtiles, int tiles_per_wg, int rows_per_split, int planes, int range_len,
-    int32_t *__restrict__ max_count = nullptr, int32_t *__restrict__ min_count = nullptr)
+    int32_t *__restrict__ max_count = nullptr, int32_t *__restrict__ min_count = nullptr,
+    float *__restrict__ bias_out = nullptr)
 {
+    __shared__ float bias_part[COUNT ? 1 : NT / 64][MAX_NEURONS];
+    const bool sum_bias = !COUNT && bias_out != nullptr && by == 0;
     uint32_t *cnt = reinterpret_cast<uint32_t *>(hist) + ((size_t)kc << log2r);
     const int tid = threadIdx.x;
     const int R = 1 << log2r;
@@ -486,6 +493,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
             *reinterpret_cast<float4 *>(&hist[i]) = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
         if (have) scatter_quad<LAYOUT, COUNT>(hist, g, i1, i2, x1, x2, r_first, k0, kn, kc, log2r, cnt);
+        float4 bias_sum = have && pf == 0 ? g : make_float4(0.f, 0.f, 0.f, 0.f);
         for (int64_t it = tid + NT; it < items; it += NT) {
             const int pl = npl > 1 ? (int)(it / per_plane) : 0;
             const int64_t rem = npl > 1 ? it - pl * per_plane : it;
@@ -506,8 +514,29 @@ __device__ __forceinline__ void bwd_w_vec_body(
                 gather_quad(x + (int64_t)n * ldx + k0, j1, j2, k0, kn, y1, y2);
             }
             scatter_quad<LAYOUT, COUNT>(hist, gg, j1, j2, y1, y2, r0, k0, kn, kc, log2r, cnt);
+            if (sum_bias && pl == 0) {
+                bias_sum.x += gg.x;
+                bias_sum.y += gg.y;
+                bias_sum.z += gg.z;
+                bias_sum.w += gg.w;
+            }
+        }
+        if (sum_bias) {
+            for (int s = qpr; s < 64; s <<= 1) {
+                bias_sum.x += __shfl_xor(bias_sum.x, s);
+                bias_sum.y += __shfl_xor(bias_sum.y, s);
+                bias_sum.z += __shfl_xor(bias_sum.z, s);
+                bias_sum.w += __shfl_xor(bias_sum.w, s);
+            }
+            if ((tid & 63) < qpr) *reinterpret_cast<float4 *>(&bias_part[tid >> 6][(tid & 63) * 4]) = bias_sum;
         }
         __syncthreads();
+        if (sum_bias && tid < rn) {
+            float sum = bias_part[0][tid];
+#pragma unroll
+            for (int v = 1; v < (COUNT ? 1 : NT / 64); ++v) sum += bias_part[v][tid];
+            bias_out[(int64_t)bz * M + m0 + tid] = sum;
+        }
         if (t + 1 < tiles_per_wg && mt + 1 < mtiles) load_first(m0 + R);
         // the counters first: their read-modify-write is the longer chain, the plain stores of w_grad follow it
         // (measured at 256 x 4096 x 4096, x_grad + this kernel: 58.7 us this way round, 61.2 the other)
@@ -523,12 +552,13 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_vec_kernel(
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
     const float *__restrict__ x_sel, int64_t nm, float *__restrict__ w_grad, int N, int K, int M, int log2r,
-    int kc, int vec_out, int mtiles, int tiles_per_wg, int rows_per_split, int planes, int range_len)
+    int kc, int vec_out, int mtiles, int tiles_per_wg, int rows_per_split, int planes, int range_len,
+    float *__restrict__ bias_out)
 {
     extern __shared__ float hist[];
     bwd_w_vec_body<LAYOUT, NT_W>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
                                  argmin, x_sel, nm, w_grad, N, K, M, log2r, kc, vec_out, mtiles, tiles_per_wg,
-                                 rows_per_split, planes, range_len);
+                                 rows_per_split, planes, range_len, nullptr, nullptr, bias_out);
 }
 
 // w_grad and the selection counts (hits) of the same slabs in one launch.
@@ -680,7 +710,7 @@ __global__ __launch_bounds__(NT_E) void mam_bwd_w_exact_kernel(
 struct BothParams {
     const float *x, *w, *grad, *w_sel, *x_sel;
     const int32_t *argmax, *argmin;
-    float *x_grad, *w_grad;
+    float *x_grad, *w_grad, *bias_grad;
     int64_t ldx, ldw, nm;
     int N, K, M, planes, range_len, span, kc_x;
     int log2r, kc_w, vec_out, mtiles, tiles_per_wg, x_wgs;
@@ -696,7 +726,7 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
         bwd_w_vec_body<LAYOUT, NT_X>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
                                      0, 1, p.x, p.ldx, p.grad, p.argmax, p.argmin, p.x_sel, p.nm, p.w_grad, p.N, p.K,
                                      p.M, p.log2r, p.kc_w, p.vec_out, p.mtiles, p.tiles_per_wg, p.N, p.planes,
-                                     p.range_len);
+                                     p.range_len, nullptr, nullptr, p.bias_grad);
     }
 }
 
@@ -706,9 +736,12 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
     const float *__restrict__ x_sel, int64_t nm, float *__restrict__ w_grad, int N, int K, int M, int log2r,
-    int kc, int vec_out, int planes, int range_len)
+    int kc, int vec_out, int planes, int range_len, float *__restrict__ bias_out)
 {
     extern __shared__ float hist[];
+    __shared__ float bias_part[NT_W / 64][MAX_NEURONS];
+    const bool sum_bias = bias_out != nullptr && blockIdx.y == 0;       // as in bwd_w_vec_body, a neuron per thread
+    float bias_sum = 0.0f;
     const int tid = threadIdx.x;
     const int R = 1 << log2r;
     const int mt = xcd_remap(blockIdx.x, gridDim.x);
@@ -733,6 +766,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
             if (r >= rn) continue;
             const int64_t o = (int64_t)n * M + m0 + r;
             const float g = grad[o];
+            if (sum_bias && pl == 0) bias_sum += g;
             const int a1 = amax_pl[o] - k0, a2 = amin_pl[o] - k0;
             const float *xr = x + (int64_t)n * ldx + k0;
             if ((unsigned)a1 < (unsigned)kn)
@@ -743,7 +777,17 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
                                (x_sel_pl ? x_sel_pl[nm + o] : xr[a2]) * g);
         }
     }
+    if (sum_bias) {
+        for (int s = R; s < 64; s <<= 1) bias_sum += __shfl_xor(bias_sum, s);
+        if ((tid & 63) < R) bias_part[tid >> 6][tid & 63] = bias_sum;
+    }
     __syncthreads();
+    if (sum_bias && tid < rn) {
+        float sum = bias_part[0][tid];
+#pragma unroll
+        for (int v = 1; v < NT_W / 64; ++v) sum += bias_part[v][tid];
+        bias_out[m0 + tid] = sum;
+    }
     store_slab<LAYOUT, NT_W>(hist, w_grad, tid, m0, k0, rn, kn, kc, log2r, K, M, vec_out, false);
 }
 
@@ -777,11 +821,20 @@ static int setup_device(int dev)
 }
 static DeviceHookRegistration g_registration(setup_device);
 
+// Where a bias gradient goes and room for its partial sums; `done` by the launch that writes w_grad, or left to mam_bias_grad.
+struct BiasGrad {
+    float *out, *partial;
+    int64_t partials;        // rows of M that `partial` holds
+    bool done;
+};
+// shares of the batch that a w_grad launch may use and the partial sums of a bias gradient they need
+static int64_t most_shares(int64_t N, int64_t K) { return N / (K > 512 ? K : 512) < 1 ? 1 : N / (K > 512 ? K : 512); }
+
 template <int LAYOUT>
 static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *grad,
                          const int32_t *argmax, const int32_t *argmin, const float *w_sel, const float *x_sel,
                          float *x_grad, float *w_grad, int64_t N, int64_t K, int64_t M, hipStream_t st,
-                         int planes = 1, int range_len = 0)
+                         int planes, int range_len, BiasGrad *bias)
 {
     int rc = MAM_OK;
     if (planes <= 1) range_len = (int)K;
@@ -861,7 +914,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
                 if (per_cu < 1) per_cu = 1;
                 shares = (2 * per_cu * cus + mtiles * ktiles / 2) / (mtiles * ktiles);
                 // a share adds a whole slab to w_grad with atomics: worth it only against >= K rows of work
-                if (shares > N / (K > 512 ? K : 512)) shares = N / (K > 512 ? K : 512);
+                if (shares > most_shares(N, K)) shares = most_shares(N, K);
                 if (shares > 65535) shares = 65535;
                 if (shares < 1) shares = 1;
             }
@@ -871,16 +924,25 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
                 rc = fill_zero(w_grad, M * K, st);
                 if (rc != MAM_OK) return rc;
             }
+            float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
             hipLaunchKernelGGL((mam_bwd_w_vec_kernel<LAYOUT>),
                                dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT_W),
                                (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
                                w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
-                               (int)rows_per_share, planes, range_len);
+                               (int)rows_per_share, planes, range_len, bias_out);
+            if (bias_out) {
+                bias->done = true;
+                if (shares > 1) {
+                    rc = check_launch("mam_bwd_w_kernel");
+                    return rc != MAM_OK ? rc : sum_slabs(bias_out, bias->out, M, shares, st);
+                }
+            }
         } else {
             hipLaunchKernelGGL((mam_bwd_w_kernel<LAYOUT>), dim3((unsigned)mtiles, (unsigned)ktiles),
                                dim3(NT_W), (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax,
                                argmin, x_sel, N * M, w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, planes,
-                               range_len);
+                               range_len, bias ? bias->out : nullptr);
+            if (bias) bias->done = true;
         }
         rc = check_launch("mam_bwd_w_kernel");
     }
@@ -894,7 +956,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
 static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *grad,
                        const int32_t *argmax, const int32_t *argmin, const float *w_sel, const float *x_sel,
                        float *x_grad, float *w_grad, int64_t N, int64_t K, int64_t M, hipStream_t st, int planes,
-                       int range_len, bool auto_mode)
+                       int range_len, bool auto_mode, BiasGrad *bias)
 {
     if (planes <= 1) range_len = (int)K;
     const int dev = ensure_device(st);
@@ -922,6 +984,8 @@ static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw,
     BothParams p;
     p.x = x; p.w = w; p.grad = grad; p.w_sel = w_sel; p.x_sel = x_sel;
     p.argmax = argmax; p.argmin = argmin; p.x_grad = x_grad; p.w_grad = w_grad;
+    p.bias_grad = bias ? bias->out : nullptr;
+    if (bias) bias->done = true;
     p.ldx = ldx; p.ldw = ldw; p.nm = N * M;
     p.N = (int)N; p.K = (int)K; p.M = (int)M; p.planes = planes; p.range_len = range_len;
     p.span = window_span(2 * M * planes); p.kc_x = (int)K;
@@ -990,7 +1054,8 @@ int x_grad_from_selected(const float *grad, const int32_t *argmax, const int32_t
 static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                          const float *grad, const int32_t *argmax, const int32_t *argmin,
                          const float *w_sel, const float *x_sel, float *x_grad, float *w_grad,
-                         int64_t N, int64_t K, int64_t M, int planes, int range_len, void *stream)
+                         int64_t N, int64_t K, int64_t M, int planes, int range_len, void *stream,
+                         mam::bwd::BiasGrad *bias = nullptr)
 {
     using namespace mam;
     if (N < 0 || K < 0 || M < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
@@ -1012,9 +1077,9 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
     auto launch = [&](float *xg, float *wg, hipStream_t on) {
         if (w_layout == MAM_W_MK)
             return bwd::launch_layout<MAM_W_MK>(x, ldx, w, ldw, grad, argmax, argmin, w_sel, x_sel, xg, wg, N, K, M, on,
-                                                planes, range_len);
+                                                planes, range_len, bias);
         return bwd::launch_layout<MAM_W_KM>(x, ldx, w, ldw, grad, argmax, argmin, w_sel, x_sel, xg, wg, N, K, M, on,
-                                            planes, range_len);
+                                            planes, range_len, bias);
     };
     // x_grad is bound by LDS atomics and w_grad by memory traffic, and neither depends on the other: one
     // launch that holds both where the shape allows it, else two streams where that pays
@@ -1023,7 +1088,7 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
         option(MAM_OPT_BACKWARD_EXACT) != MAM_BACKWARD_EXACT_ON) {
         const int rc = bwd::launch_both(x, ldx, w, ldw, grad, argmax, argmin, w_sel, x_sel, x_grad, w_grad, N, K, M, st,
                                         planes, range_len,
-                                        option(MAM_OPT_BACKWARD_ONE_LAUNCH) == MAM_BACKWARD_ONE_LAUNCH_AUTO);
+                                        option(MAM_OPT_BACKWARD_ONE_LAUNCH) == MAM_BACKWARD_ONE_LAUNCH_AUTO, bias);
         if (rc != 1) return rc;
     }
     if (x_grad && w_grad) {
@@ -1051,6 +1116,36 @@ extern "C" int mam_fc_backward(const float *x, int64_t ldx, const float *w, int6
 {
     return backward_impl(x, ldx, w, ldw, w_layout, grad, argmax, argmin, w_sel, x_sel, x_grad, w_grad, N, K, M, 1, 0,
                          stream);
+}
+
+extern "C" size_t mam_fc_backward_bias_workspace(int64_t N, int64_t K, int64_t M)
+{
+    if (N <= 0 || K <= 0 || M <= 0) return 0;
+    const size_t shares = N >= 2048 ? (size_t)mam::bwd::most_shares(N, K) * (size_t)M * sizeof(float) : 0;
+    const size_t slabs = mam_bias_grad_workspace(N, M);
+    return shares > slabs ? shares : slabs;
+}
+
+extern "C" int mam_fc_backward_bias(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
+                                    const float *grad, const int32_t *argmax, const int32_t *argmin,
+                                    const float *w_sel, const float *x_sel, float *x_grad, float *w_grad,
+                                    float *bias_grad, int64_t N, int64_t K, int64_t M, int64_t range_len,
+                                    void *workspace, size_t workspace_bytes, void *stream)
+{
+    using namespace mam;
+    if (range_len < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative range_len");
+    if (N > 0 && K > 0 && M > 0 && workspace_bytes < mam_fc_backward_bias_workspace(N, K, M))
+        return fail(MAM_ERR_WORKSPACE, "the bias gradient needs %zu workspace bytes, got %zu",
+                    mam_fc_backward_bias_workspace(N, K, M), workspace_bytes);
+    if (M > 0 && !bias_grad) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
+    const int64_t planes = range_len > 0 && K > 0 ? (K + range_len - 1) / range_len : 1;
+    if (planes > 65535) return fail(MAM_ERR_UNSUPPORTED, "more than 65535 ranges");
+    bwd::BiasGrad bias = {bias_grad, static_cast<float *>(workspace), 0, false};
+    if (workspace && N > 0 && M > 0) bias.partials = (int64_t)(workspace_bytes / ((size_t)M * sizeof(float)));
+    const int rc = backward_impl(x, ldx, w, ldw, w_layout, grad, argmax, argmin, w_sel, x_sel, x_grad, w_grad, N, K, M,
+                                 (int)planes, (int)(range_len > 0 && range_len < K ? range_len : K), stream, &bias);
+    if (rc != MAM_OK || bias.done) return rc;
+    return mam_bias_grad(grad, M, bias_grad, N, M, workspace, workspace_bytes, stream);
 }
 
 extern "C" int mam_fc_backward_count(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,

@@ -94,6 +94,9 @@ __device__ __forceinline__ float load_w(const float *__restrict__ w, int64_t ldw
     return LAYOUT == MAM_W_MK ? w[m * ldw + k] : w[k * ldw + m];
 }
 
+// out[m] = sum over s of partial[s][m], in slab order (mam_module.hip).
+int sum_slabs(const float *partial, float *out, int64_t M, int64_t slabs, hipStream_t stream);
+
 namespace bwd {
 // x_grad (N,K) from the selected weights (2,N,M) written by a forward (mam_backward.hip).
 int x_grad_from_selected(const float *grad, const int32_t *argmax, const int32_t *argmin, const float *w_sel,

@@ -328,6 +328,12 @@ __global__ __launch_bounds__(64) void slab_sum_kernel(const float *__restrict__ 
     out[m] = acc;
 }
 
+int sum_slabs(const float *partial, float *out, int64_t M, int64_t slabs, hipStream_t st)
+{
+    hipLaunchKernelGGL(slab_sum_kernel, dim3((unsigned)ceil_div(M, 64)), dim3(64), 0, st, partial, out, (int)M, (int)slabs);
+    return check_launch("slab_sum_kernel");
+}
+
 // slabs of the batch: one up to 512 rows, else slabs of at least 128 rows, at most 64 of them
 static int64_t bias_grad_slabs(int64_t N)
 {
@@ -368,9 +374,7 @@ extern "C" int mam_bias_grad(const float *grad, int64_t ld, float *bias_grad, in
                        (int)N, (int)M, (int)rows_per_slab);
     int rc = check_launch("col_sum_kernel");
     if (rc != MAM_OK || slabs == 1) return rc;
-    hipLaunchKernelGGL(slab_sum_kernel, dim3((unsigned)ceil_div(M, 64)), dim3(64), 0, st, first, bias_grad, (int)M,
-                       (int)slabs);
-    return check_launch("slab_sum_kernel");
+    return sum_slabs(first, bias_grad, M, slabs, st);
 }
 
 extern "C" int mam_blend(const float *mam_out, const float *mac_out, const float *bias, float alpha, float beta,

@@ -111,18 +111,20 @@ struct Wt : public Function<Wt> {
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        static const auto op = find<Tensors(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &,
-                                            const MaybeTensor &)>("mamtorch_kernel_v4::fullyconnected_wt_backward");
+        typedef Tensors Backward(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &, const MaybeTensor &);
+        static const auto op = find<Backward>("mamtorch_kernel_v4::fullyconnected_wt_backward");
+        static const auto op_bias = find<Backward>("mamtorch_kernel_v4::fullyconnected_wt_backward_bias");
         variable_list out(4);
         const Tensor &g = grads[0];
         if (!g.defined()) return out;
+        const bool bias = ctx->saved_data["bias"].toBool();
         if (ctx->saved_data["operands"].toBool()) {
             const variable_list s = ctx->get_saved_variables();
-            const Tensors both = op.call(s[0], s[1], g.contiguous(), s[2], s[3], s[4]);
-            out[0] = both[0];
-            out[1] = both[1];
+            const Tensors all = (bias ? op_bias : op).call(s[0], s[1], g.contiguous(), s[2], s[3], s[4]);
+            for (size_t i = 0; i < all.size(); ++i) out[i] = all[i];
+        } else if (bias) {
+            out[2] = bias_grad(g);
         }
-        if (ctx->saved_data["bias"].toBool()) out[2] = bias_grad(g);
         return out;
     }
 };
@@ -157,20 +159,23 @@ struct Ranges : public Function<Ranges> {
     }
     static variable_list backward(AutogradContext *ctx, variable_list grads)
     {
-        static const auto op = find<Tensors(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t)>(
-            "mamtorch_kernel_v4::fullyconnected_ranges_backward");
+        typedef Tensors Backward(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &, int64_t);
+        static const auto op = find<Backward>("mamtorch_kernel_v4::fullyconnected_ranges_backward");
+        static const auto op_bias = find<Backward>("mamtorch_kernel_v4::fullyconnected_ranges_backward_bias");
         variable_list out(5);
         const Tensor &g = grads[0];
         if (!g.defined()) return out;
+        const bool bias = ctx->saved_data["bias"].toBool();
         if (ctx->saved_data["operands"].toBool()) {
             TORCH_CHECK(ctx->saved_data["with_indices"].toBool(),
                         "fullyconnected_ranges was run without indices; its gradient needs them");
             const variable_list s = ctx->get_saved_variables();
-            const Tensors both = op.call(s[0], s[1], g.contiguous(), s[2], s[3], ctx->saved_data["range_len"].toInt());
-            out[0] = both[0];
-            out[1] = both[1];
+            const Tensors all =
+                (bias ? op_bias : op).call(s[0], s[1], g.contiguous(), s[2], s[3], ctx->saved_data["range_len"].toInt());
+            for (size_t i = 0; i < all.size(); ++i) out[i] = all[i];
+        } else if (bias) {
+            out[2] = bias_grad(g);
         }
-        if (ctx->saved_data["bias"].toBool()) out[2] = bias_grad(g);
         return out;
     }
 };

@@ -158,7 +158,8 @@ at::Tensor forward_values_impl(const at::Tensor &a, const at::Tensor &w, int lay
 
 std::vector<at::Tensor> backward_impl(const at::Tensor &a, const at::Tensor &w, int layout,
                                       const at::Tensor &grad, const at::Tensor &argmax,
-                                      const at::Tensor &argmin, const c10::optional<at::Tensor> &sel)
+                                      const at::Tensor &argmin, const c10::optional<at::Tensor> &sel,
+                                      bool with_bias = false)
 {
     const FwdShape s = check_forward(a, w, layout, c10::nullopt);
     check_f32_2d(grad, "grad");
@@ -179,6 +180,18 @@ std::vector<at::Tensor> backward_impl(const at::Tensor &a, const at::Tensor &w, 
     const at::Tensor g = grad.contiguous();
     auto a_grad = at::empty({s.N, s.K}, a.options());
     auto w_grad = at::empty(w.sizes(), w.options());
+    if (with_bias) {
+        auto b_grad = at::empty({s.M}, a.options());
+        const size_t ws_bytes = mam_fc_backward_bias_workspace(s.N, s.K, s.M);
+        auto ws = workspace_for(ws_bytes, a);
+        check_rc(mam_fc_backward_bias(a.data_ptr<float>(), row_stride(a, "a"), w.data_ptr<float>(),
+                                      row_stride(w, "the weight operand"), layout, g.data_ptr<float>(),
+                                      argmax.data_ptr<int32_t>(), argmin.data_ptr<int32_t>(), w_sel_ptr, x_sel_ptr,
+                                      a_grad.data_ptr<float>(), w_grad.data_ptr<float>(), b_grad.data_ptr<float>(), s.N,
+                                      s.K, s.M, 0, ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
+                 "mam_fc_backward_bias");
+        return {a_grad, w_grad, b_grad};
+    }
     check_rc(mam_fc_backward(a.data_ptr<float>(), row_stride(a, "a"), w.data_ptr<float>(),
                              row_stride(w, "the weight operand"), layout, g.data_ptr<float>(),
                              argmax.data_ptr<int32_t>(), argmin.data_ptr<int32_t>(), w_sel_ptr, x_sel_ptr,
@@ -228,6 +241,14 @@ std::vector<at::Tensor> fullyconnected_wt_backward(const at::Tensor &a, const at
     return backward_impl(a, weight, MAM_W_MK, grad, argmax, argmin, sel);
 }
 
+std::vector<at::Tensor> fullyconnected_wt_backward_bias(const at::Tensor &a, const at::Tensor &weight,
+                                                        const at::Tensor &grad, const at::Tensor &argmax,
+                                                        const at::Tensor &argmin,
+                                                        const c10::optional<at::Tensor> &sel)
+{
+    return backward_impl(a, weight, MAM_W_MK, grad, argmax, argmin, sel, true);
+}
+
 // ---- the module's `splits`: consecutive K ranges, each a MAM neuron of its own, summed ----
 std::vector<at::Tensor> fullyconnected_ranges(const at::Tensor &a, const at::Tensor &weight,
                                               const c10::optional<at::Tensor> &bias, int64_t range_len,
@@ -252,9 +273,9 @@ std::vector<at::Tensor> fullyconnected_ranges(const at::Tensor &a, const at::Ten
     return {c, argmax, argmin};
 }
 
-std::vector<at::Tensor> fullyconnected_ranges_backward(const at::Tensor &a, const at::Tensor &weight,
-                                                       const at::Tensor &grad, const at::Tensor &argmax,
-                                                       const at::Tensor &argmin, int64_t range_len)
+std::vector<at::Tensor> ranges_backward_impl(const at::Tensor &a, const at::Tensor &weight, const at::Tensor &grad,
+                                             const at::Tensor &argmax, const at::Tensor &argmin, int64_t range_len,
+                                             bool with_bias)
 {
     const FwdShape s = check_forward(a, weight, MAM_W_MK, c10::nullopt);
     check_f32_2d(grad, "grad");
@@ -269,12 +290,38 @@ std::vector<at::Tensor> fullyconnected_ranges_backward(const at::Tensor &a, cons
     const at::Tensor g = grad.contiguous();
     auto a_grad = at::empty({s.N, s.K}, a.options());
     auto w_grad = at::empty(weight.sizes(), weight.options());
+    if (with_bias) {
+        auto b_grad = at::empty({s.M}, a.options());
+        const size_t ws_bytes = mam_fc_backward_bias_workspace(s.N, s.K, s.M);
+        auto ws = workspace_for(ws_bytes, a);
+        check_rc(mam_fc_backward_bias(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
+                                      row_stride(weight, "weight"), MAM_W_MK, g.data_ptr<float>(), argmax.data_ptr<int32_t>(),
+                                      argmin.data_ptr<int32_t>(), nullptr, nullptr, a_grad.data_ptr<float>(),
+                                      w_grad.data_ptr<float>(), b_grad.data_ptr<float>(), s.N, s.K, s.M, range_len,
+                                      ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
+                 "mam_fc_backward_bias");
+        return {a_grad, w_grad, b_grad};
+    }
     check_rc(mam_fc_backward_ranges(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
                                     row_stride(weight, "weight"), MAM_W_MK, g.data_ptr<float>(),
                                     argmax.data_ptr<int32_t>(), argmin.data_ptr<int32_t>(), a_grad.data_ptr<float>(),
                                     w_grad.data_ptr<float>(), s.N, s.K, s.M, range_len, current_stream(a)),
              "mam_fc_backward_ranges");
     return {a_grad, w_grad};
+}
+
+std::vector<at::Tensor> fullyconnected_ranges_backward(const at::Tensor &a, const at::Tensor &weight,
+                                                       const at::Tensor &grad, const at::Tensor &argmax,
+                                                       const at::Tensor &argmin, int64_t range_len)
+{
+    return ranges_backward_impl(a, weight, grad, argmax, argmin, range_len, false);
+}
+
+std::vector<at::Tensor> fullyconnected_ranges_backward_bias(const at::Tensor &a, const at::Tensor &weight,
+                                                            const at::Tensor &grad, const at::Tensor &argmax,
+                                                            const at::Tensor &argmin, int64_t range_len)
+{
+    return ranges_backward_impl(a, weight, grad, argmax, argmin, range_len, true);
 }
 
 void selection_count(const at::Tensor &argmax, const at::Tensor &argmin, at::Tensor max_count,
@@ -591,9 +638,11 @@ TORCH_LIBRARY(mamtorch_kernel_v4, m)
     m.def("fullyconnected_wt(Tensor a, Tensor weight, Tensor? bias, bool hand_over) -> Tensor[]");
     m.def("fullyconnected_fast_wt(Tensor a, Tensor weight, Tensor? bias) -> Tensor");
     m.def("fullyconnected_wt_backward(Tensor a, Tensor weight, Tensor grad, Tensor argmax, Tensor argmin, Tensor? sel) -> Tensor[]");
+    m.def("fullyconnected_wt_backward_bias(Tensor a, Tensor weight, Tensor grad, Tensor argmax, Tensor argmin, Tensor? sel) -> Tensor[]");
     m.def("selection_count(Tensor argmax, Tensor argmin, Tensor(a!) max_count, Tensor(b!) min_count, int mode) -> ()");
     m.def("fullyconnected_ranges(Tensor a, Tensor weight, Tensor? bias, int range_len, bool with_indices) -> Tensor[]");
     m.def("fullyconnected_ranges_backward(Tensor a, Tensor weight, Tensor grad, Tensor argmax, Tensor argmin, int range_len) -> Tensor[]");
+    m.def("fullyconnected_ranges_backward_bias(Tensor a, Tensor weight, Tensor grad, Tensor argmax, Tensor argmin, int range_len) -> Tensor[]");
     m.def("blend(Tensor mam, Tensor mac, Tensor? bias, float alpha, float beta) -> Tensor");
     m.def("bias_grad(Tensor grad) -> Tensor");
     m.def("apply_keep(Tensor weight, Tensor keep) -> Tensor");
@@ -625,9 +674,11 @@ TORCH_LIBRARY_IMPL(mamtorch_kernel_v4, CUDA, m)
     m.impl("fullyconnected_wt", &fullyconnected_wt);
     m.impl("fullyconnected_fast_wt", &fullyconnected_fast_wt);
     m.impl("fullyconnected_wt_backward", &fullyconnected_wt_backward);
+    m.impl("fullyconnected_wt_backward_bias", &fullyconnected_wt_backward_bias);
     m.impl("selection_count", &selection_count);
     m.impl("fullyconnected_ranges", &fullyconnected_ranges);
     m.impl("fullyconnected_ranges_backward", &fullyconnected_ranges_backward);
+    m.impl("fullyconnected_ranges_backward_bias", &fullyconnected_ranges_backward_bias);
     m.impl("blend", &blend);
     m.impl("bias_grad", &bias_grad);
     m.impl("apply_keep", &apply_keep);

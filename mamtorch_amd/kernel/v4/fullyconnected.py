@@ -61,3 +61,17 @@ def _(a, weight, grad, argmax, argmin, sel):
     torch._check(argmin.dtype == torch.int)
     return [torch.empty((a.size(0), a.size(1)), dtype=torch.float, device=a.device),
             torch.empty((weight.size(0), weight.size(1)), dtype=torch.float, device=a.device)]
+
+
+@torch.library.register_fake(f"{library_name}::fullyconnected_wt_backward_bias")
+def _(a, weight, grad, argmax, argmin, sel):
+    torch._check(a.size(1) == weight.size(1))
+    torch._check(grad.size(0) == a.size(0))
+    torch._check(grad.size(1) == weight.size(0))
+    torch._check(grad.shape == argmax.shape)
+    torch._check(grad.shape == argmin.shape)
+    torch._check(argmax.dtype == torch.int)
+    torch._check(argmin.dtype == torch.int)
+    return [torch.empty((a.size(0), a.size(1)), dtype=torch.float, device=a.device),
+            torch.empty((weight.size(0), weight.size(1)), dtype=torch.float, device=a.device),
+            torch.empty((weight.size(0),), dtype=torch.float, device=a.device)]

@@ -37,6 +37,14 @@ def _(a, weight, grad, argmax, argmin, range_len):
             torch.empty(weight.shape, dtype=torch.float, device=a.device)]
 
 
+@torch.library.register_fake("mamtorch_kernel_v4::fullyconnected_ranges_backward_bias")
+def _(a, weight, grad, argmax, argmin, range_len):
+    torch._check(a.size(1) == weight.size(1) and grad.size(0) == a.size(0) and grad.size(1) == weight.size(0))
+    return [torch.empty(a.shape, dtype=torch.float, device=a.device),
+            torch.empty(weight.shape, dtype=torch.float, device=a.device),
+            torch.empty((weight.size(0),), dtype=torch.float, device=a.device)]
+
+
 def blend(mam: Tensor, mac: Tensor, bias, alpha: float, beta: float) -> Tensor:
     """(alpha * mam + beta * mac) + bias in the reference's rounding order; (N, out) operands."""
     return K.blend.default(mam, mac, bias, float(alpha), float(beta))

@@ -371,3 +371,23 @@ def test_bias_gradient_through_the_module():
     g = torch.randn(50, 40, generator=torch.Generator().manual_seed(4)).to(DEV)
     layer(x).backward(g)
     torch.testing.assert_close(layer.bias.grad, g.sum(dim=0), rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("N,K,M", [(1, 40, 4), (64, 784, 256), (65, 784, 260), (50, 33, 7), (250, 1001, 517), (300, 5000, 68),
+                                   (2048, 768, 96), (2600, 3072, 40), (5000, 96, 132), (2100, 64, 33), (3000, 9000, 12)])
+@pytest.mark.parametrize("splits", [1, 3])
+def test_bias_gradient_from_the_launch_that_forms_the_weight_gradient(N, K, M, splits):
+    """Every route of the weight gradient (one launch for both gradients, quads, single neurons, several k chunks, shares of a
+    large batch): the column sums within the rounding of an fp32 sum, the same bits on every call."""
+    layer = mt.nn.FullyConnected(K, M, bias=True, splits=splits).to(DEV).train()
+    gen = torch.Generator().manual_seed(N + M)
+    x = torch.randn(N, K, generator=gen).to(DEV).requires_grad_(True)
+    g = torch.randn(N, M, generator=gen).to(DEV)
+    seen = []
+    for _ in range(2):
+        layer.bias.grad = None
+        layer(x).backward(g)
+        seen.append(layer.bias.grad)
+    want, floor = g.double().sum(dim=0), g.abs().double().sum(dim=0)
+    assert torch.equal(*seen)
+    assert bool(((seen[0].double() - want).abs() <= 1e-5 * want.abs() + 2.0 ** -22 * floor).all())
