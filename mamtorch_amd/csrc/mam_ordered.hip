@@ -26,7 +26,7 @@
 //   dense kernels  exit at once unless the decision was "none".
 //
 // Measured against the dense tilings (forward call, hand-over arrays written).  Uniform weights or inputs, one-sided:
-// 207 -> 60 to 67 us at 256 x 4096 x 4096, 1.70 -> 0.49 ms and 1.48 -> 0.24 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.74 ms
+// 207 -> 60 to 67 us at 256 x 4096 x 4096, 1.70 -> 0.49 ms and 1.48 -> 0.24 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.72 ms
 // (values only) and 3.13 -> 0.36 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.36 ms
 // at 12608 x 768 -> 3072, 3.12 -> 0.92 ms at 16384 x 4096 -> 1024, 0.84 -> 0.43 ms at 4096 x 2048 x 2048.
 #include "mam_ordered.h"
@@ -821,19 +821,20 @@ __device__ __forceinline__ void scan_row(const float *src, int K, const float *b
 // listed row x 4 consecutive tile rows, and TB / 4 neighbouring lanes share a listed row, so that an entry costs
 // each lane one 16-byte LDS read for 4 products and the lanes of a row read TB * 4 contiguous bytes.  Waves take
 // blocks of 64 * 4 / TB listed rows in turn and need no barrier after the tile is loaded.  A wave looks at its
-// lists chunk by chunk until TOGETHER of its 256 outputs are not yet finished by their bound (53 entries at K = 4096, where all but
+// lists chunk by chunk until TOGETHER of its 256 outputs are not yet finished by their bound (41 entries at K = 4096, where all but
 // FEW take 90 and the mean output needs 28), then goes on with a lane for each of those -- one product per entry instead of four of
 // which most are decided -- and finishes the last FEW one by one with all its lanes.  (Us; TOGETHER, FEW = none, 2 / 32, 2 / 64, 2 / 64, 1 /
-// 48, 1 / 64, 0: 256 x 4096 x 4096 65.8 / 63.3 / 62.3 / 61.0 / 60.5 / 61.7, 12608 x 768 -> 3072 587 / 581 / 577 / 566 / 560 / 560, 16384 x 4096 ->
-// 4096 values only 752 / 756 / 758 / 751 / 745 / 779, 16384 x 4096 -> 1024 405 / 394 / 386 / 385 / 383 / 396.  Handing lanes out anew at every
-// quarter, 1 to 64 an output, costs more in exchanges than it saves: 64.0 / 625 / 898 / 422.)
+// 64, 0: 256 x 4096 x 4096 65.8 / 63.3 / 62.3 / 61.0 / 61.7, 12608 x 768 -> 3072 587 / 581 / 577 / 566 / 560, 16384 x 4096 ->
+// 4096 values only 752 / 756 / 758 / 751 / 779, 16384 x 4096 -> 1024 405 / 394 / 386 / 385 / 396; with the lanes in the order of the
+// rows, whose list entries are neighbours, 64, 1 and 48, 1: 60.1 and 60.2, 486 and 492, 724 and 729, 360 and 361.  Handing lanes out anew at every
+// quarter, 1 to 64 an output, costs more in exchanges than it saves: 64.0 / 625 / 898 / 422.  Lists two chunks ahead: 773 for 745.)
 // What bounds it (counters, values only at K = 4096): VALU instructions at 4 cycles take 0.63 of the busy cycles, the random
 // 16-byte LDS reads 0.67 (three fifths of it bank conflicts), list entries on their way from the caches to the registers 0.95
 // -- but with the lanes of a row loading a quarter or half of its entries each and passing them round the quad the calls take the
-// same: 562 / 735 / 384 us for 560 / 745 / 383.  16384 x 4096 -> 4096: 61 us before the search, 59 us of tile loads, 320 us until
-// TOGETHER, 260 us for those, 42 us for the last one.
+// same: 562 / 735 / 384 us for 560 / 745 / 383.  16384 x 4096 -> 4096 with 48: 61 us before the search, 59 us of tile loads, 320 us until
+// TOGETHER, 260 us for those (245 in the order of the rows), 42 us for the last one.
 constexpr int FEW = 1;
-constexpr int TOGETHER = 48;         // at most a wave's lanes
+constexpr int TOGETHER = 64;         // at most a wave's lanes
 // Outputs of a row that are scanned one by one, 8 to 17 us each beside the other waves' work; the whole row takes 30 to 60 us.
 constexpr int FEW_OF_ROW = 4;
 
@@ -1078,15 +1079,21 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
         // ---- the last TOGETHER outputs: a lane each instead of four on a lane of which most are finished ----
         const int unfinished = __popcll(open[0]) + __popcll(open[1]) + __popcll(open[2]) + __popcll(open[3]);
         if (unfinished > FEW && ch < chunks) {
+            // in the order of the lanes, that is of the rows: their list entries are neighbours in memory
             int rank[4], before = 0;
 #pragma unroll
+            for (int j = 0; j < 4; ++j)
+                before = __builtin_amdgcn_mbcnt_hi((uint32_t)(open[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)open[j], before));
+#pragma unroll
             for (int j = 0; j < 4; ++j) {
-                rank[j] = before + __builtin_amdgcn_mbcnt_hi((uint32_t)(open[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)open[j], 0));
-                if (open[j] >> own & 1) places[wave][rank[j]] = (uint8_t)(own * 4 + j);
-                before += __popcll(open[j]);
+                rank[j] = before;
+                if (open[j] >> own & 1) {
+                    places[wave][before] = (uint8_t)(own * 4 + j);
+                    ++before;
+                }
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-            const int task = own < unfinished ? places[wave][own] : 0, from = task & ~3, tj = task & 3, tl = task >> 2;
+            const int task = places[wave][own < unfinished ? own : unfinished - 1], from = task & ~3, tj = task & 3, tl = task >> 2;
             const int trow = blk * RW + L::row(tl) < a.rows ? blk * RW + L::row(tl) : a.rows - 1;
             uint4 first[CHUNK / 2], second[CHUNK / 2];
             float u1, u2;
