@@ -485,6 +485,121 @@ __device__ __forceinline__ void build_row(const Rows &rows, int row, int K, int 
     }
 }
 
+// The lists of four consecutive rows by a workgroup, a wave per row with R elements per lane: no barrier but the one before the
+// lists are written, 64 bytes of every pair of entries at a time.  Bound by instruction issue where build_row waits at its barriers
+// (12608 / 4096 / 2048 / 1024 rows of K = 768 or 1024: 36.6 / 15.2 / 13.2 / 7.4 us by build_row, 23.3 / 10.8 / 10.1 / 8.1 us like this): from 2048 rows on.
+// Up to K = 1024: a lane's elements of longer rows take registers that the other path's workgroups lack (K = 2048: 8192 rows 37.9 -> 33.8,
+// two-sided call of 4096 x 2048 x 2048 425 -> 436 us; K = 3072 71 -> 112).
+constexpr int WAVE_MAX_LENGTH = 256;
+constexpr int WAVE_MIN_ROWS = 2048;
+constexpr int WAVE_MAX_R = 4;            // of build_kernel: elements per thread of a row's workgroup
+struct WaveList {               // of one row, in LDS
+    uint32_t hist[BUCKETS];
+    uint2 items[WAVE_MAX_LENGTH];
+};
+template <int R>
+__device__ __forceinline__ void build_rows(const Rows &rows, int row0, int K, int len, uint4 *lists, float *bound, int pad, WaveList *all)
+{
+    static_assert(BUCKETS == 512, "eight buckets a lane");
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int row = row0 + wave;
+    WaveList &own = all[wave];
+    if (row < rows.rows) {
+        const int chunks = len / CHUNK;
+        const float *src = rows.at(row, 0);
+        float v[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t) v[t] = t * 64 + lane < K ? (src + t * 64)[(uint32_t)lane] : 0.0f;
+        uint4 *const zero = reinterpret_cast<uint4 *>(own.hist);
+        zero[lane] = zero[64 + lane] = make_uint4(0, 0, 0, 0);
+        for (int j = lane; j < len; j += 64) own.items[j] = make_uint2(0u, key(0, 0));
+        uint32_t top = 0;
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const uint32_t bits = __float_as_uint(v[t]) & 0x7fffffffu;
+            top = bits > top ? bits : top;
+        }
+        top = (uint32_t)wave_max((int)top);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // (buckets, clamped k and zeros as in build_row)
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const uint32_t b = (top - (__float_as_uint(v[t]) & 0x7fffffffu)) >> BUCKET_SHIFT;
+            if (b < (uint32_t)BUCKETS && lane < K - t * 64) atomicAdd(&own.hist[b], 1u);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint32_t count[8], sum = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            count[i] = own.hist[lane * 8 + i];
+            sum += count[i];
+        }
+        uint32_t incl = sum;
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) {
+            const uint32_t o = __shfl_up(incl, s);
+            if (lane >= s) incl += o;
+        }
+        uint32_t run = incl - sum;
+        int started = 0;                // buckets that start inside the list
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            own.hist[lane * 8 + i] = run;
+            started += run < (uint32_t)len;
+            run += count[i];
+        }
+        const uint32_t open = (uint32_t)wave_sum(started);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        uint32_t rest = 0;              // largest magnitude that is not listed
+        uint32_t top_again = top;       // (the buckets are computed anew: kept, they would take R more registers)
+        int lane_again = lane;
+        asm volatile("" : "+v"(top_again), "+v"(lane_again));
+#pragma unroll
+        for (int t = 0; t < R; ++t) {
+            const uint32_t bits = __float_as_uint(v[t]) & 0x7fffffffu;
+            const uint32_t b = (top_again - bits) >> BUCKET_SHIFT;
+            const int k = t * 64 + lane_again;
+            bool listed = false;
+            if (b < open && k < K) {
+                const uint32_t at = atomicAdd(&own.hist[b], 1u);
+                if (at < (uint32_t)len) {
+                    own.items[at] = make_uint2(__float_as_uint(v[t]), key((uint32_t)k, at + 1));
+                    listed = true;
+                }
+            }
+            if (!listed) rest = bits > rest ? bits : rest;
+        }
+        rest = (uint32_t)wave_max((int)rest);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        // bound[c], the special rows: as in build_row, a chunk a lane
+        static_assert(WAVE_MAX_LENGTH / CHUNK < 64, "a lane for each chunk and one for what follows");
+        uint32_t after = 0;
+        if (lane < chunks) {
+#pragma unroll
+            for (int e = 0; e < CHUNK; ++e) {
+                const uint32_t b = own.items[lane * CHUNK + e].x & 0x7fffffffu;
+                after = b > after ? b : after;
+            }
+        } else if (lane == chunks) {
+            after = rest;
+        }
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) {
+            const uint32_t o = __shfl_down(after, s);
+            if (lane + s < 64) after = o > after ? o : after;
+        }
+        const bool special = top >= INF_BITS || top == 0;
+        const float instead = top == 0 ? -1.0f : __builtin_nanf("");
+        if (lane <= chunks) bound[(int64_t)lane * pad + row] = special ? instead : __uint_as_float(after);
+    }
+    __syncthreads();
+    const int which = threadIdx.x & 3;
+    if (row0 + which >= rows.rows) return;
+    const uint4 *pairs = reinterpret_cast<const uint4 *>(all[which].items);
+    for (int j = threadIdx.x >> 2; j < len / 2; j += BUILD_NT / 4) lists[(int64_t)j * pad + row0 + which] = pairs[j];
+}
+
 // One work item per workgroup: the rows of the searched operand; with a leading share also the rows of the other one
 // and the 64 x 64 tiles of the transpose.
 template <int R>
@@ -494,7 +609,7 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     __shared__ uint32_t hist[BUCKETS];
     __shared__ uint32_t part[BUILD_NT / 64], part2[BUILD_NT / 64];
     __shared__ uint32_t chunk_top[BUILD_MAX_CHUNKS];
-    __shared__ float turn[64][65];
+    __shared__ __attribute__((aligned(16))) float turn[64][65];
     // (with turns the decision has been made before; the LDS of one more array would cost a workgroup per CU at K = 3072)
     Weighed (&weighed)[OPTIONS] = reinterpret_cast<Weighed (&)[OPTIONS]>(turn);
     static_assert(sizeof(weighed) <= sizeof(turn), "decision and transpose share LDS");
@@ -507,6 +622,7 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
         d.length = __builtin_amdgcn_readfirstlane(d.length);
         d.lead = 0;
         if (blockIdx.x == 0 && threadIdx.x == 0) *p.decision = d;       // for the kernels that follow
+        __syncthreads();        // every wave has read `weighed`, whose place build_rows takes
     }
     if (d.side == SIDE_NONE) return;
     const bool sx = d.side == SIDE_X;
@@ -515,6 +631,15 @@ __global__ __launch_bounds__(BUILD_NT) void build_kernel(const Params p)
     const int row_tiles = (a.rows + 63) / 64;
     const int turns = d.lead > 0 ? row_tiles * ((K + 63) / 64) : 0;
     const int total = a.rows + (d.lead > 0 ? b.rows : 0) + turns;
+    if (R <= WAVE_MAX_R && d.lead == 0 && d.length <= WAVE_MAX_LENGTH && a.rows >= WAVE_MIN_ROWS) {
+        constexpr int ROWS = BUILD_NT / 64;
+        static_assert(sizeof(WaveList) * ROWS <= sizeof(turn), "rows of a workgroup and the transpose share LDS");
+        const int groups = (a.rows + ROWS - 1) / ROWS;
+        if ((int)blockIdx.x < groups)
+            build_rows<R <= WAVE_MAX_R ? R * ROWS : 1>(a, xcd_remap(blockIdx.x, groups) * ROWS, K, d.length, sx ? p.lists_x : p.lists_w,
+                                               sx ? p.bound_x : p.bound_w, sx ? p.pad_x : p.pad_w, reinterpret_cast<WaveList *>(turn));
+        return;
+    }
     if ((int)blockIdx.x >= total) return;
     const int item = xcd_remap(blockIdx.x, total);
     if (item < total - turns) {

@@ -155,6 +155,26 @@ def test_a_few_bad_rows_among_good_ones():
     assert_index_equal(amin.cpu().numpy(), want[2], "argmin")
 
 
+@pytest.mark.parametrize("N, K", [(2047, 640), (2048, 700), (2049, 1023), (2051, 1024), (2050, 1025)])
+@pytest.mark.parametrize("listed", ["x", "w"])
+def test_lists_of_many_short_rows(N, K, listed):
+    """A wave per row from 2048 rows on, up to K = 1024; among the rows some of zeros, of one magnitude, with a NaN or an infinity, and
+    of fewer entries than a list holds, the last row too."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(N)
+    many = torch.randn(N, K, generator=g)
+    many[3], many[4], many[9, 17], many[10, K - 1], many[N - 1, 5:] = 0.0, 0.5, float("nan"), float("inf"), 0.0
+    few = torch.rand(40, K, generator=g) * 2 - 1
+    x, w = (many, few) if listed == "x" else (few, many)
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK)
+    (c, amax, amin), (side, lead, _) = _by_lists(x.to(DEV), w.to(DEV), capi.W_MK)
+    assert (side, lead) == (1 if listed == "x" else 2, 0)
+    assert_bits_equal(c.cpu().numpy(), want[0], "c")
+    assert_index_equal(amax.cpu().numpy(), want[1], "argmax")
+    assert_index_equal(amin.cpu().numpy(), want[2], "argmin")
+
+
 @pytest.mark.parametrize("N, K, M", [(640, 768, 640), (700, 1024, 701), (1000, 2432, 300), (300, 2432, 1000), (512, 4864, 513),
                                      (400, 4095, 402), (1200, 520, 333), (333, 520, 1201)])
 @pytest.mark.parametrize("kinds", [("normal", "normal"), ("relu", "normal")])
