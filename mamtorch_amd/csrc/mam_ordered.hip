@@ -178,6 +178,8 @@ __device__ __forceinline__ uint32_t prefix_buckets(uint32_t *hist, uint32_t *par
 }
 
 // ---- sampling ----------------------------------------------------------------------------------------------
+// R elements per thread of either row, read once: what counts here is how often a workgroup waits for memory.
+template <int R>
 __global__ __launch_bounds__(BUILD_NT) void sample_kernel(const Params p)
 {
     constexpr int WAVES = BUILD_NT / 64;
@@ -192,13 +194,20 @@ __global__ __launch_bounds__(BUILD_NT) void sample_kernel(const Params p)
     const int m = (int)((((uint64_t)(i * 2654435769u)) * (uint64_t)c.M) >> 32);
     const Rows xr = x_rows(c), wr = w_rows(c);
     float hi = -__builtin_inff(), lo = __builtin_inff(), ax = 0.0f, aw = 0.0f;
-#pragma unroll 4
-    for (int k = tid; k < K; k += BUILD_NT) {
-        const float a = *xr.at(n, k), b = *wr.at(m, k), q = a * b;
+    float xv[R], wv[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) {           // (past the end the last element again: it changes no extreme, and is not counted)
+        const int k = t * BUILD_NT + tid < K ? t * BUILD_NT + tid : K - 1;
+        xv[t] = *xr.at(n, k);
+        wv[t] = *wr.at(m, k);
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const float q = xv[t] * wv[t];
         hi = __builtin_fmaxf(hi, q);
         lo = __builtin_fminf(lo, q);
-        ax = __builtin_fmaxf(ax, __builtin_fabsf(a));
-        aw = __builtin_fmaxf(aw, __builtin_fabsf(b));
+        ax = __builtin_fmaxf(ax, __builtin_fabsf(xv[t]));
+        aw = __builtin_fmaxf(aw, __builtin_fabsf(wv[t]));
     }
 #pragma unroll
     for (int s = 32; s > 0; s >>= 1) {
@@ -222,11 +231,12 @@ __global__ __launch_bounds__(BUILD_NT) void sample_kernel(const Params p)
         // one-sided searches only: options 0 and LEADS
         __shared__ int counts[WAVES][2];
         int nx = 0, nw = 0;
-#pragma unroll 4
-        for (int k = tid; k < K; k += BUILD_NT) {
-            nx += !(__builtin_fabsf(*xr.at(n, k)) * aw < reach);
-            nw += !(__builtin_fabsf(*wr.at(m, k)) * ax < reach);
-        }
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+            if (t * BUILD_NT + tid < K) {
+                nx += !(__builtin_fabsf(xv[t]) * aw < reach);
+                nw += !(__builtin_fabsf(wv[t]) * ax < reach);
+            }
         nx = wave_sum(nx);
         nw = wave_sum(nw);
         if (lane == 0) { counts[wave][0] = nx; counts[wave][1] = nw; }
@@ -239,12 +249,13 @@ __global__ __launch_bounds__(BUILD_NT) void sample_kernel(const Params p)
         return;
     }
     const uint32_t top_x = __float_as_uint(ax), top_w = __float_as_uint(aw);
-#pragma unroll 4
-    for (int k = tid; k < K; k += BUILD_NT) {
-        const uint32_t bx = (top_x - (__float_as_uint(*xr.at(n, k)) & 0x7fffffffu)) >> BUCKET_SHIFT;
-        const uint32_t bw = (top_w - (__float_as_uint(*wr.at(m, k)) & 0x7fffffffu)) >> BUCKET_SHIFT;
-        if (bx < (uint32_t)BUCKETS) atomicAdd(&hist[0][bx], 1u);
-        if (bw < (uint32_t)BUCKETS) atomicAdd(&hist[1][bw], 1u);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+        const uint32_t bx = (top_x - (__float_as_uint(xv[t]) & 0x7fffffffu)) >> BUCKET_SHIFT;
+        const uint32_t bw = (top_w - (__float_as_uint(wv[t]) & 0x7fffffffu)) >> BUCKET_SHIFT;
+        const bool there = t * BUILD_NT + tid < K;
+        if (there && bx < (uint32_t)BUCKETS) atomicAdd(&hist[0][bx], 1u);
+        if (there && bw < (uint32_t)BUCKETS) atomicAdd(&hist[1][bw], 1u);
     }
     __syncthreads();
     prefix_buckets(hist[0], part, 0);
@@ -1545,7 +1556,9 @@ int launch(const Call &call, void *workspace, Guard &guard, hipStream_t st)
     const int64_t items = call.w_layout == MAM_W_MK ? build_items(N, K, M, p.turned_ld > 0) : N;
     p.decided = p.turned_ld > 0 || items > MAX_UNDECIDED;
     p.any_size = option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_LISTS;
-    hipLaunchKernelGGL(sample_kernel, dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
+    if (K <= 4 * BUILD_NT) hipLaunchKernelGGL((sample_kernel<4>), dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
+    else if (K <= 16 * BUILD_NT) hipLaunchKernelGGL((sample_kernel<16>), dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
+    else hipLaunchKernelGGL((sample_kernel<40>), dim3(SAMPLES), dim3(BUILD_NT), 0, st, p);
     int rc = check_launch("ordered::sample_kernel");
     if (rc != MAM_OK) return rc;
     if (p.decided) {
