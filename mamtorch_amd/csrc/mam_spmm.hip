@@ -51,6 +51,21 @@ __device__ __forceinline__ void axpy(float (&acc)[4], float v, const float4 &b)
     acc[3] = __builtin_fmaf(v, b.w, acc[3]);
 }
 
+// Which panel of columns a workgroup works on and which block of rows or entries: numbered panel by panel over the XCDs, or,
+// where that would be more than a launch holds in one dimension, a row of the grid each.
+struct Place { int panel, block; };
+__device__ __forceinline__ Place place_of(int blocks)
+{
+    if (gridDim.y > 1) return {(int)blockIdx.y, (int)blockIdx.x};
+    const int logical = xcd_remap(blockIdx.x, gridDim.x);
+    return {logical / blocks, logical % blocks};
+}
+static dim3 grid_of(int64_t panels, int64_t blocks)
+{
+    // less than 2^32 threads in a dimension
+    return panels * blocks < UINT32_MAX / NT ? dim3((unsigned)(panels * blocks)) : dim3((unsigned)blocks, (unsigned)panels);
+}
+
 // four consecutive words, 4-byte aligned
 typedef float words4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ void store4(float *dst, const float (&a)[4])
@@ -74,9 +89,8 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
-    const int panel = logical / row_blocks;
-    const int r = (logical - panel * row_blocks) * (NT / 64) + wave;
+    const Place at_block = place_of(row_blocks);
+    const int panel = at_block.panel, r = at_block.block * (NT / 64) + wave;
     if (r >= R) return;
     constexpr int LANES = 64 / PER;      // of one entry; the parts are added at the end
     const int c0 = panel * LANES * TI + lane % LANES * TI;
@@ -212,9 +226,9 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
-    const int panel = logical / chunk_blocks;
-    const int64_t e0 = ((int64_t)(logical - panel * chunk_blocks) * (NT / 64) + wave) * COO_CHUNK;
+    const Place at_block = place_of(chunk_blocks);
+    const int panel = at_block.panel;
+    const int64_t e0 = ((int64_t)at_block.block * (NT / 64) + wave) * COO_CHUNK;
     if (e0 >= nnz) return;
     const int n = (int)((nnz - e0) < COO_CHUNK ? (nnz - e0) : COO_CHUNK);
     const int c0 = panel * 64 * TI + lane * TI;
@@ -266,18 +280,19 @@ __global__ __launch_bounds__(NT) void row_offsets_kernel(const int64_t *__restri
                                                          int64_t *__restrict__ crow, int64_t R)
 {
     const int lane = threadIdx.x & 63;
-    const int64_t r = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6);
-    if (r > R) return;
-    int64_t lo = 0, count = nnz;          // the place is one of lo .. lo + count
-    while (count > 0) {
-        const int64_t step = (count + 63) >> 6, at = lo + (lane + 1) * step - 1;
-        const int below = __popcll(__ballot(at < lo + count && row[at < nnz ? at : nnz - 1] < r));
-        const int64_t end = lo + count;
-        lo += below * step;
-        // the next probe was not below r (or lay past the end): what is left lies before it
-        count = (end - lo) < step - 1 ? end - lo : step - 1;
+    const int64_t waves = (int64_t)gridDim.x * (NT / 64);
+    for (int64_t r = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6); r <= R; r += waves) {
+        int64_t lo = 0, count = nnz;          // the place is one of lo .. lo + count
+        while (count > 0) {
+            const int64_t step = (count + 63) >> 6, at = lo + (lane + 1) * step - 1;
+            const int below = __popcll(__ballot(at < lo + count && row[at < nnz ? at : nnz - 1] < r));
+            const int64_t end = lo + count;
+            lo += below * step;
+            // the next probe was not below r (or lay past the end): what is left lies before it
+            count = (end - lo) < step - 1 ? end - lo : step - 1;
+        }
+        if (lane == 0) crow[r] = lo;
     }
-    if (lane == 0) crow[r] = lo;
 }
 
 static int check_common(const float *b, int64_t ldb, float *c, int64_t R, int64_t K, int64_t C)
@@ -364,9 +379,9 @@ extern "C" int mam_csr_spmm(const int64_t *crow, const int64_t *col, const float
     const int per = !near ? 1 : C <= 64 ? 4 : C <= 128 ? 2 : 1;          // entries per load
     const int64_t panels = ceil_div(C, near || wide ? 256 / per : 64);
     const int64_t row_blocks = ceil_div(R, spmm::NT / 64);
-    if (panels * row_blocks > INT32_MAX / 4) return fail(MAM_ERR_UNSUPPORTED, "too many rows and columns for the SpMM grid");
+    if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(panels * row_blocks)), dim3(spmm::NT), 0, st, crow, col, val, b, ldb,
+        hipLaunchKernelGGL(kernel, spmm::grid_of(panels, row_blocks), dim3(spmm::NT), 0, st, crow, col, val, b, ldb,
                            (uint32_t)b_bytes, c, (int)R, (int)C, (int)row_blocks);
     };
     if (per == 4) launch(spmm::csr_spmm_kernel<4, true, 4>);
@@ -394,9 +409,9 @@ extern "C" int mam_coo_spmm(const int64_t *row, const int64_t *col, const float 
     const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
     const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
     const int64_t panels = ceil_div(C, near || wide ? 256 : 64);
-    if (panels * gx > INT32_MAX / 4) return fail(MAM_ERR_UNSUPPORTED, "too many entries and columns for the SpMM grid");
+    if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)(panels * gx)), dim3(spmm::NT), 0, st, row, col, val, nnz, b, ldb,
+        hipLaunchKernelGGL(kernel, spmm::grid_of(panels, gx), dim3(spmm::NT), 0, st, row, col, val, nnz, b, ldb,
                            (uint32_t)b_bytes, c, (int)C, (int)gx);
     };
     if (near) launch(spmm::coo_spmm_kernel<4, true>);
@@ -411,7 +426,8 @@ extern "C" int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *cro
     if (nnz < 0 || R < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
     if (R > INT32_MAX / 2) return fail(MAM_ERR_UNSUPPORTED, "a dimension exceeds 2^30");
     if (!crow || (nnz > 0 && !row)) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
-    hipLaunchKernelGGL(spmm::row_offsets_kernel, dim3((unsigned)ceil_div(R + 1, spmm::NT / 64)), dim3(spmm::NT), 0,
+    const int64_t blocks = ceil_div(R + 1, spmm::NT / 64);
+    hipLaunchKernelGGL(spmm::row_offsets_kernel, dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20)), dim3(spmm::NT), 0,
                        static_cast<hipStream_t>(stream), row, nnz, crow, R);
     return check_launch("row_offsets_kernel");
 }

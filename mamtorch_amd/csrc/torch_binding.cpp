@@ -595,8 +595,8 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     const int64_t nnz = val.numel();
     // A coalesced operand's rows ascend: with row offsets it is a CSR operand, whose kernel adds a row up in registers instead of
     // clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns: 364 -> 107 us).  A row is one wave's there, at most K / 8 rounds of
-    // loads, 0.4 us each: not for K so large that one crowded row would outlast the COO kernel.
-    const bool by_rows = a.is_coalesced() && K <= 32768;
+    // loads, 0.4 us each: not for K so large that one crowded row would outlast the COO kernel (nor for more rows than a launch holds waves).
+    const bool by_rows = a.is_coalesced() && K <= 32768 && R <= (int64_t(1) << 24);
     if (dense_route_pays(nnz, R, K, C, by_rows ? 8 : 16)) {
         auto dense = at::empty({R, K}, b.options());
         check_rc(mam_coo_to_dense(idx.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(), nnz,
