@@ -316,6 +316,14 @@ int mam_coo_spmm(const int64_t *row, const int64_t *col, const float *val, int64
  * operand of the same matrix.  Offsets lie in 0 .. nnz whatever the rows are.
  */
 int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, void *stream);
+/*
+ * mam_coo_spmm for an operand whose rows are expected to ascend: the device looks whether they do, adds up row by row as
+ * mam_csr_spmm does, and where they do not the call is mam_coo_spmm's.  `workspace`: mam_coo_spmm_by_rows_workspace(R) bytes,
+ * 16-byte aligned.
+ */
+size_t mam_coo_spmm_by_rows_workspace(int64_t R);
+int mam_coo_spmm_by_rows(const int64_t *row, const int64_t *col, const float *val, int64_t nnz, const float *b, int64_t ldb,
+                         float *c, int64_t R, int64_t K, int64_t C, void *workspace, size_t workspace_bytes, void *stream);
 
 /*
  * The sparse operand written out as a dense (R, K) fp32 matrix with row stride ld (cleared first; repeated

@@ -37,7 +37,8 @@ EXPORTS = (
     "mam_fc_backward", "mam_fc_backward_count", "mam_selection_count",
     "mam_fc_forward_ranges_workspace", "mam_fc_forward_ranges", "mam_fc_backward_ranges",
     "mam_csr_fc_forward_workspace", "mam_csr_fc_forward", "mam_csr_fc_backward", "mam_csr_validate",
-    "mam_csr_spmm", "mam_coo_spmm", "mam_coo_row_offsets", "mam_csr_to_dense", "mam_coo_to_dense",
+    "mam_csr_spmm", "mam_coo_spmm", "mam_coo_row_offsets", "mam_coo_spmm_by_rows_workspace",
+    "mam_coo_spmm_by_rows", "mam_csr_to_dense", "mam_coo_to_dense",
     "mam_fc_backward_bias_workspace", "mam_fc_backward_bias",
     "mam_blend", "mam_bias_grad_workspace", "mam_bias_grad", "mam_apply_keep", "mam_im2col", "mam_col2im",
     "mam_prune_row_offsets", "mam_prune_fill_csr", "mam_prune_apply",
@@ -101,6 +102,9 @@ def lib():
         l.mam_csr_validate.argtypes = [_ptr, _ptr, _i64, _i64, _i64, _ptr, _ptr]
         l.mam_csr_spmm.argtypes = [_ptr, _ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr]
         l.mam_coo_spmm.argtypes = [_ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr]
+        l.mam_coo_spmm_by_rows_workspace.argtypes = [_i64]
+        l.mam_coo_spmm_by_rows_workspace.restype = _size
+        l.mam_coo_spmm_by_rows.argtypes = [_ptr, _ptr, _ptr, _i64, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr, _size, _ptr]
         l.mam_coo_row_offsets.argtypes = [_ptr, _i64, _ptr, _i64, _ptr]
         l.mam_csr_to_dense.argtypes = [_ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _ptr]
         l.mam_coo_to_dense.argtypes = [_ptr, _ptr, _ptr, _i64, _ptr, _i64, _i64, _i64, _ptr]
@@ -319,6 +323,18 @@ def coo_row_offsets(row, R):
     with torch.cuda.device(row.device):
         _check(l.mam_coo_row_offsets(_p(row), row.numel(), _p(crow), R, _stream(row)))
     return crow
+
+
+def coo_spmm_by_rows(row, col, val, b, R):
+    """coo_spmm for rows that are expected to ascend."""
+    l = lib()
+    K, C = b.shape
+    c = torch.empty((R, C), dtype=torch.float32, device=b.device)
+    ws = torch.empty(max(l.mam_coo_spmm_by_rows_workspace(R), 1), dtype=torch.uint8, device=b.device)
+    with torch.cuda.device(b.device):
+        _check(l.mam_coo_spmm_by_rows(_p(row), _p(col), _p(val), val.numel(), _p(b), _ld(b), _p(c), R, K, C, _p(ws), ws.numel(),
+                                      _stream(b)))
+    return c
 
 
 def coo_spmm(row, col, val, b, R):

@@ -75,6 +75,17 @@ __device__ __forceinline__ void store4(float *dst, const float (&a)[4])
 }
 __device__ __forceinline__ void store4(float *, const float (&)[1]) {}
 
+// Whether any workgroup of row_offsets_kernel found that a COO operand may not be summed row by row.  One load per wave, beside
+// that of the row offsets.
+constexpr int VERDICTS = 256;         // a word of each checking workgroup
+__device__ __forceinline__ bool not_by_rows(const uint32_t *verdicts)
+{
+    const uint4 v = reinterpret_cast<const uint4 *>(verdicts)[threadIdx.x & 63];
+    static_assert(VERDICTS == 64 * 4, "four words a lane");
+    return __ballot((v.x | v.y | v.z | v.w) != 0) != 0;
+}
+
+// verdicts: of a COO operand's rows, nullptr: a CSR operand.  Where they forbid the sum by rows, c is cleared for coo_spmm_kernel.
 // PER: entries per load, each by 64 / PER lanes (NEAR only).
 // NEAR: b spans less than 4 GiB; a b row is then a buffer load with the row's byte offset in a scalar register, of any
 // alignment (a load of 4 words needs 4 bytes), and lanes past the last column read on into the next row or, past the end
@@ -84,7 +95,8 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
                                                       const int64_t *__restrict__ col,
                                                       const float *__restrict__ val,
                                                       const float *__restrict__ b, int64_t ldb, uint32_t b_bytes,
-                                                      float *__restrict__ c, int R, int C, int row_blocks)
+                                                      float *__restrict__ c, int R, int C, int row_blocks,
+                                                      const uint32_t *__restrict__ verdicts)
 {
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
@@ -100,7 +112,7 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     const_i64 *ccol = (const_i64 *)col;
     const_f32 *cval = (const_f32 *)val;
     const int64_t beg = ((const_i64 *)crow)[r], end = ((const_i64 *)crow)[r + 1];
-    const int nnz = (int)(end - beg);
+    const int nnz = verdicts && not_by_rows(verdicts) ? 0 : (int)(end - beg);
     const float *bl = b + cl;
     const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
     const uint32_t row_bytes = (uint32_t)ldb * 4u;
@@ -215,73 +227,90 @@ __device__ __forceinline__ void flush_row(float *__restrict__ c, int64_t row, in
     }
 }
 
-// Panels go to the XCDs as in csr_spmm_kernel, and b rows are read as there.
+// Panels go to the XCDs as in csr_spmm_kernel, and b rows are read as there.  With verdicts it runs only where they forbid the sum
+// by rows, and then in no more workgroups than the chip holds: one per block of entries and panel cost 4 us to find nothing to do.
+constexpr int FALLBACK_WORKGROUPS = 8 * kNumCU;
 template <int TI, bool NEAR>
 __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict__ row,
                                                       const int64_t *__restrict__ col,
                                                       const float *__restrict__ val, int64_t nnz,
                                                       const float *__restrict__ b, int64_t ldb, uint32_t b_bytes,
-                                                      float *__restrict__ c, int C, int chunk_blocks)
+                                                      float *__restrict__ c, int C, int chunk_blocks, int64_t total,
+                                                      const uint32_t *__restrict__ verdicts)
 {
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Place at_block = place_of(chunk_blocks);
-    const int panel = at_block.panel;
-    const int64_t e0 = ((int64_t)at_block.block * (NT / 64) + wave) * COO_CHUNK;
-    if (e0 >= nnz) return;
-    const int n = (int)((nnz - e0) < COO_CHUNK ? (nnz - e0) : COO_CHUNK);
-    const int c0 = panel * 64 * TI + lane * TI;
-    const bool live = c0 < C;
-    const int cl = live ? c0 : 0;
-    const float *bl = b + cl;
-    const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
-    const uint32_t row_bytes = (uint32_t)ldb * 4u;
-    auto b_row = [&](int64_t k) -> vec {
-        if constexpr (NEAR) return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(near, cl * 4, (uint32_t)k * row_bytes, 0));
-        else return *reinterpret_cast<const vec *>(bl + k * ldb);
-    };
+    if (verdicts && !not_by_rows(verdicts)) return;
+    for (int64_t at = xcd_remap(blockIdx.x, gridDim.x); at < total; at += gridDim.x) {
+        const int panel = (int)(at / chunk_blocks);
+        const int64_t e0 = ((at - (int64_t)panel * chunk_blocks) * (NT / 64) + wave) * COO_CHUNK;
+        if (e0 >= nnz) continue;
+        const int n = (int)((nnz - e0) < COO_CHUNK ? (nnz - e0) : COO_CHUNK);
+        const int c0 = panel * 64 * TI + lane * TI;
+        const bool live = c0 < C;
+        const int cl = live ? c0 : 0;
+        const float *bl = b + cl;
+        const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
+        const uint32_t row_bytes = (uint32_t)ldb * 4u;
+        auto b_row = [&](int64_t k) -> vec {
+            if constexpr (NEAR) return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(near, cl * 4, (uint32_t)k * row_bytes, 0));
+            else return *reinterpret_cast<const vec *>(bl + k * ldb);
+        };
 
-    const_i64 *crow = (const_i64 *)row;
-    const_i64 *ccol = (const_i64 *)col;
-    const_f32 *cval = (const_f32 *)val;
-    float acc[TI];
+        const_i64 *crow = (const_i64 *)row;
+        const_i64 *ccol = (const_i64 *)col;
+        const_f32 *cval = (const_f32 *)val;
+        float acc[TI];
 #pragma unroll
-    for (int t = 0; t < TI; ++t) acc[t] = 0.0f;
-    int64_t cur = crow[e0];
-    for (int i = 0; i < n; i += EG) {
-        // loads of up to EG entries first; entries past the end repeat the last one and are not added
-        vec xv[EG];
-        float wv[EG];
-        int64_t rv[EG];
+        for (int t = 0; t < TI; ++t) acc[t] = 0.0f;
+        int64_t cur = crow[e0];
+        for (int i = 0; i < n; i += EG) {
+            // loads of up to EG entries first; entries past the end repeat the last one and are not added
+            vec xv[EG];
+            float wv[EG];
+            int64_t rv[EG];
 #pragma unroll
-        for (int u = 0; u < EG; ++u) {
-            const bool ok = i + u < n;
-            const int64_t e = e0 + (ok ? i + u : n - 1);
-            xv[u] = b_row(ccol[e]);
-            wv[u] = cval[e];
-            rv[u] = crow[e];
-        }
-#pragma unroll
-        for (int u = 0; u < EG; ++u) {
-            if (rv[u] != cur) {  // wave-uniform
-                flush_row<TI>(c, cur, C, c0, live, acc);
-                cur = rv[u];
+            for (int u = 0; u < EG; ++u) {
+                const bool ok = i + u < n;
+                const int64_t e = e0 + (ok ? i + u : n - 1);
+                xv[u] = b_row(ccol[e]);
+                wv[u] = cval[e];
+                rv[u] = crow[e];
             }
-            if (i + u < n) axpy(acc, wv[u], xv[u]);
+#pragma unroll
+            for (int u = 0; u < EG; ++u) {
+                if (rv[u] != cur) {  // wave-uniform
+                    flush_row<TI>(c, cur, C, c0, live, acc);
+                    cur = rv[u];
+                }
+                if (i + u < n) axpy(acc, wv[u], xv[u]);
+            }
         }
+        flush_row<TI>(c, cur, C, c0, live, acc);
     }
-    flush_row<TI>(c, cur, C, c0, live, acc);
 }
 
 // crow[r] = entries whose row is below r, for rows in ascending order.  A wave per r narrows the place down to one entry
 // 64-fold a step (four steps for 2^24 entries); for rows in any other order it ends all the same, inside 0 .. nnz.
+// verdicts: the first VERDICTS workgroups look whether the rows ascend instead (a tensor may be flagged as coalesced without
+// being so).
 __global__ __launch_bounds__(NT) void row_offsets_kernel(const int64_t *__restrict__ row, int64_t nnz,
-                                                         int64_t *__restrict__ crow, int64_t R)
+                                                         int64_t *__restrict__ crow, int64_t R,
+                                                         uint32_t *__restrict__ verdicts)
 {
+    const int checking = verdicts ? VERDICTS : 0;
+    if ((int)blockIdx.x < checking) {
+        bool bad = false;
+#pragma unroll 4
+        for (int64_t e = (int64_t)blockIdx.x * NT + threadIdx.x; e < nnz - 1; e += (int64_t)VERDICTS * NT) bad |= row[e + 1] < row[e];
+        const int any = __syncthreads_or(bad);
+        if (threadIdx.x == 0) verdicts[blockIdx.x] = any ? 1u : 0u;
+        return;
+    }
     const int lane = threadIdx.x & 63;
-    const int64_t waves = (int64_t)gridDim.x * (NT / 64);
-    for (int64_t r = (int64_t)blockIdx.x * (NT / 64) + (threadIdx.x >> 6); r <= R; r += waves) {
+    const int64_t waves = (int64_t)(gridDim.x - checking) * (NT / 64);
+    for (int64_t r = (int64_t)((int)blockIdx.x - checking) * (NT / 64) + (threadIdx.x >> 6); r <= R; r += waves) {
         int64_t lo = 0, count = nnz;          // the place is one of lo .. lo + count
         while (count > 0) {
             const int64_t step = (count + 63) >> 6, at = lo + (lane + 1) * step - 1;
@@ -363,6 +392,56 @@ static bool wide(const float *b, int64_t ldb, const float *c, int64_t C)
     return C % 4 == 0 && ldb % 4 == 0 && (uintptr_t)b % 16 == 0 && (uintptr_t)c % 16 == 0;
 }
 
+// Launches of csr_spmm_kernel and coo_spmm_kernel (arguments checked, nothing empty).
+static int launch_csr(const int64_t *crow, const int64_t *col, const float *val, const float *b, int64_t ldb, float *c, int64_t R,
+                      int64_t K, int64_t C, const uint32_t *verdicts, hipStream_t st)
+{
+    const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
+    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
+    const int per = !near ? 1 : C <= 64 ? 4 : C <= 128 ? 2 : 1;          // entries per load
+    const int64_t panels = ceil_div(C, near || wide ? 256 / per : 64);
+    const int64_t row_blocks = ceil_div(R, NT / 64);
+    if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid_of(panels, row_blocks), dim3(NT), 0, st, crow, col, val, b, ldb, (uint32_t)b_bytes, c,
+                           (int)R, (int)C, (int)row_blocks, verdicts);
+    };
+    if (per == 4) launch(csr_spmm_kernel<4, true, 4>);
+    else if (per == 2) launch(csr_spmm_kernel<4, true, 2>);
+    else if (near) launch(csr_spmm_kernel<4, true, 1>);
+    else if (wide) launch(csr_spmm_kernel<4, false, 1>);
+    else launch(csr_spmm_kernel<1, false, 1>);
+    return check_launch("csr_spmm_kernel");
+}
+
+static int launch_coo(const int64_t *row, const int64_t *col, const float *val, int64_t nnz, const float *b, int64_t ldb, float *c,
+                      int64_t K, int64_t C, const uint32_t *verdicts, hipStream_t st)
+{
+    const int64_t gx = ceil_div(nnz, (int64_t)COO_CHUNK * (NT / 64));
+    if (gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "too many entries for the SpMM grid");
+    const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
+    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
+    const int64_t panels = ceil_div(C, near || wide ? 256 : 64);
+    if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
+    const int64_t total = panels * gx, most = verdicts ? FALLBACK_WORKGROUPS : UINT32_MAX / NT;      // (2^32 threads in a launch)
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)(total < most ? total : most)), dim3(NT), 0, st, row, col, val, nnz, b, ldb,
+                           (uint32_t)b_bytes, c, (int)C, (int)gx, total, verdicts);
+    };
+    if (near) launch(coo_spmm_kernel<4, true>);
+    else if (wide) launch(coo_spmm_kernel<4, false>);
+    else launch(coo_spmm_kernel<1, false>);
+    return check_launch("coo_spmm_kernel");
+}
+
+static int launch_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, uint32_t *verdicts, hipStream_t st)
+{
+    const int64_t blocks = ceil_div(R + 1, NT / 64);
+    hipLaunchKernelGGL(row_offsets_kernel, dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20) + (verdicts ? VERDICTS : 0)),
+                       dim3(NT), 0, st, row, nnz, crow, R, verdicts);
+    return check_launch("row_offsets_kernel");
+}
+
 }  // namespace spmm
 }  // namespace mam
 
@@ -373,23 +452,7 @@ extern "C" int mam_csr_spmm(const int64_t *crow, const int64_t *col, const float
     int rc = spmm::check_common(b, ldb, c, R, K, C);
     if (rc != MAM_OK || R == 0 || C == 0) return rc;
     if (!crow) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
-    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
-    const int per = !near ? 1 : C <= 64 ? 4 : C <= 128 ? 2 : 1;          // entries per load
-    const int64_t panels = ceil_div(C, near || wide ? 256 / per : 64);
-    const int64_t row_blocks = ceil_div(R, spmm::NT / 64);
-    if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, spmm::grid_of(panels, row_blocks), dim3(spmm::NT), 0, st, crow, col, val, b, ldb,
-                           (uint32_t)b_bytes, c, (int)R, (int)C, (int)row_blocks);
-    };
-    if (per == 4) launch(spmm::csr_spmm_kernel<4, true, 4>);
-    else if (per == 2) launch(spmm::csr_spmm_kernel<4, true, 2>);
-    else if (near) launch(spmm::csr_spmm_kernel<4, true, 1>);
-    else if (wide) launch(spmm::csr_spmm_kernel<4, false, 1>);
-    else launch(spmm::csr_spmm_kernel<1, false, 1>);
-    return check_launch("csr_spmm_kernel");
+    return spmm::launch_csr(crow, col, val, b, ldb, c, R, K, C, nullptr, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int mam_coo_spmm(const int64_t *row, const int64_t *col, const float *val, int64_t nnz,
@@ -404,20 +467,7 @@ extern "C" int mam_coo_spmm(const int64_t *row, const int64_t *col, const float 
     rc = fill_zero(c, R * C, st);
     if (rc != MAM_OK || nnz == 0) return rc;
     if (!row || !col || !val) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
-    const int64_t gx = ceil_div(nnz, (int64_t)spmm::COO_CHUNK * (spmm::NT / 64));
-    if (gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "too many entries for the SpMM grid");
-    const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
-    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
-    const int64_t panels = ceil_div(C, near || wide ? 256 : 64);
-    if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, spmm::grid_of(panels, gx), dim3(spmm::NT), 0, st, row, col, val, nnz, b, ldb,
-                           (uint32_t)b_bytes, c, (int)C, (int)gx);
-    };
-    if (near) launch(spmm::coo_spmm_kernel<4, true>);
-    else if (wide) launch(spmm::coo_spmm_kernel<4, false>);
-    else launch(spmm::coo_spmm_kernel<1, false>);
-    return check_launch("coo_spmm_kernel");
+    return spmm::launch_coo(row, col, val, nnz, b, ldb, c, K, C, nullptr, st);
 }
 
 extern "C" int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, void *stream)
@@ -426,10 +476,33 @@ extern "C" int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *cro
     if (nnz < 0 || R < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
     if (R > INT32_MAX / 2) return fail(MAM_ERR_UNSUPPORTED, "a dimension exceeds 2^30");
     if (!crow || (nnz > 0 && !row)) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
-    const int64_t blocks = ceil_div(R + 1, spmm::NT / 64);
-    hipLaunchKernelGGL(spmm::row_offsets_kernel, dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20)), dim3(spmm::NT), 0,
-                       static_cast<hipStream_t>(stream), row, nnz, crow, R);
-    return check_launch("row_offsets_kernel");
+    return spmm::launch_row_offsets(row, nnz, crow, R, nullptr, static_cast<hipStream_t>(stream));
+}
+
+extern "C" size_t mam_coo_spmm_by_rows_workspace(int64_t R)
+{
+    return R > 0 ? mam::spmm::VERDICTS * sizeof(uint32_t) + (size_t)(R + 1) * sizeof(int64_t) : 0;
+}
+
+extern "C" int mam_coo_spmm_by_rows(const int64_t *row, const int64_t *col, const float *val, int64_t nnz, const float *b, int64_t ldb,
+                                    float *c, int64_t R, int64_t K, int64_t C, void *workspace, size_t workspace_bytes, void *stream)
+{
+    using namespace mam;
+    if (nnz < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
+    int rc = spmm::check_common(b, ldb, c, R, K, C);
+    if (rc != MAM_OK || R == 0 || C == 0) return rc;
+    if (nnz > 0 && (!row || !col || !val)) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
+    const size_t need = mam_coo_spmm_by_rows_workspace(R);
+    if (!workspace || workspace_bytes < need || (uintptr_t)workspace % 16 != 0)
+        return fail(MAM_ERR_WORKSPACE, "the sum by rows needs %zu workspace bytes, 16-byte aligned, got %zu", need,
+                    workspace ? workspace_bytes : (size_t)0);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    uint32_t *verdicts = static_cast<uint32_t *>(workspace);
+    int64_t *crow = reinterpret_cast<int64_t *>(verdicts + spmm::VERDICTS);
+    rc = spmm::launch_row_offsets(row, nnz, crow, R, verdicts, st);
+    if (rc == MAM_OK) rc = spmm::launch_csr(crow, col, val, b, ldb, c, R, K, C, verdicts, st);
+    if (rc == MAM_OK && nnz > 0) rc = spmm::launch_coo(row, col, val, nnz, b, ldb, c, K, C, verdicts, st);
+    return rc;
 }
 
 extern "C" int mam_csr_to_dense(const int64_t *crow, const int64_t *col, const float *val, float *dense, int64_t ld,

@@ -593,8 +593,8 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     const at::Tensor idx = a._indices().to(at::kLong).contiguous();   // (2, nnz); need not be coalesced
     const at::Tensor val = a._values().contiguous();
     const int64_t nnz = val.numel();
-    // A coalesced operand's rows ascend: with row offsets it is a CSR operand, whose kernel adds a row up in registers instead of
-    // clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns: 364 -> 107 us).  A row is one wave's there, at most K / 8 rounds of
+    // A coalesced operand's rows ascend (the device looks whether they do: the flag can be set without it): with row offsets it is a
+    // CSR operand, whose kernel adds a row up in registers instead of clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns: 364 -> 107 us).  A row is one wave's there, at most K / 8 rounds of
     // loads, 0.4 us each: not for K so large that one crowded row would outlast the COO kernel (nor for more rows than a launch holds waves).
     const bool by_rows = a.is_coalesced() && K <= 32768 && R <= (int64_t(1) << 24);
     if (dense_route_pays(nnz, R, K, C, by_rows ? 8 : 16)) {
@@ -607,12 +607,12 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     auto c = at::empty({R, C}, b.options());
     if (R == 0 || C == 0) return c;
     if (by_rows) {
-        const at::Tensor crow = at::empty({R + 1}, idx.options());
-        check_rc(mam_coo_row_offsets(idx.data_ptr<int64_t>(), nnz, crow.data_ptr<int64_t>(), R, current_stream(b)),
-                 "mam_coo_row_offsets");
-        check_rc(mam_csr_spmm(crow.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(),
-                              b.data_ptr<float>(), row_stride(b, "b"), c.data_ptr<float>(), R, K, C, current_stream(b)),
-                 "mam_csr_spmm");
+        const size_t ws_bytes = mam_coo_spmm_by_rows_workspace(R);
+        const at::Tensor ws = workspace_for(ws_bytes, b);
+        check_rc(mam_coo_spmm_by_rows(idx.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(), nnz,
+                                      b.data_ptr<float>(), row_stride(b, "b"), c.data_ptr<float>(), R, K, C, ws.data_ptr(),
+                                      ws_bytes, current_stream(b)),
+                 "mam_coo_spmm_by_rows");
         return c;
     }
     check_rc(mam_coo_spmm(idx.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(), nnz,

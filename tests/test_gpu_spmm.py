@@ -86,6 +86,33 @@ def test_row_offsets(nnz, rows):
     assert torch.equal(got, torch.searchsorted(row, torch.arange(rows + 1)))
 
 
+@pytest.mark.parametrize("cols", [1, 40, 100, 260])                       # four, two, one entry per load; two panels
+@pytest.mark.parametrize("spoil", ["nothing", "first", "middle", "last", "reversed", "shuffled"])
+def test_operands_flagged_as_coalesced_whatever_their_order(cols, spoil):
+    """The flag is the caller's word (is_coalesced=True is not checked): rows out of order add up all the same."""
+    import mamtorch_amd as mt
+
+    rows, k, nnz = 90, 130, 70000 if spoil == "middle" else 900          # more entries than the check has threads, too
+    g = torch.Generator().manual_seed(cols)
+    row = torch.randint(0, rows, (nnz,), generator=g).sort()[0]
+    col = torch.randint(0, k, (nnz,), generator=g)
+    val = torch.randn(nnz, generator=g)
+    order = torch.arange(nnz)
+    if spoil in ("first", "middle", "last"):
+        at = {"first": 0, "middle": 65536 + 77, "last": nnz - 2}[spoil]
+        row[at], row[at + 1] = rows - 1, 0
+    elif spoil == "reversed":
+        order = order.flip(0)
+    elif spoil == "shuffled":
+        order = torch.randperm(nnz, generator=g)
+    row, col, val = row[order], col[order], val[order]
+    b = torch.randn(k, cols, generator=g)
+    want, floor = oracle.coo_spmm(row.numpy(), col.numpy(), val.numpy(), b.numpy(), rows)
+    a = torch.sparse_coo_tensor(torch.stack([row, col]).to(DEV), val.to(DEV), (rows, k), is_coalesced=True)
+    assert a.is_coalesced()
+    _check(mt.sparse.kernel.v1.cusparsemm(a, b.to(DEV)), want, floor, spoil)
+
+
 def test_coo_unsorted_with_duplicates_and_strided_b():
     from mamtorch_amd import capi
 
