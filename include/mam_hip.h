@@ -317,9 +317,9 @@ int mam_coo_spmm(const int64_t *row, const int64_t *col, const float *val, int64
  */
 int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, void *stream);
 /*
- * mam_coo_spmm for an operand whose rows are expected to ascend: the device looks whether they do, adds up row by row as
- * mam_csr_spmm does, and where they do not the call is mam_coo_spmm's.  `workspace`: mam_coo_spmm_by_rows_workspace(R) bytes,
- * 16-byte aligned.
+ * mam_coo_spmm for an operand whose rows are expected to ascend: the device looks whether they do, and none is crowded, and
+ * adds up row by row as mam_csr_spmm does; otherwise the call is mam_coo_spmm's.  `workspace`: mam_coo_spmm_by_rows_workspace(R)
+ * bytes, 16-byte aligned; its first 256 words are zeros after a call that added up by rows.
  */
 size_t mam_coo_spmm_by_rows_workspace(int64_t R);
 int mam_coo_spmm_by_rows(const int64_t *row, const int64_t *col, const float *val, int64_t nnz, const float *b, int64_t ldb,

@@ -326,15 +326,15 @@ def coo_row_offsets(row, R):
 
 
 def coo_spmm_by_rows(row, col, val, b, R):
-    """coo_spmm for rows that are expected to ascend."""
+    """coo_spmm for rows that are expected to ascend; c and whether it was added up row by row."""
     l = lib()
     K, C = b.shape
     c = torch.empty((R, C), dtype=torch.float32, device=b.device)
-    ws = torch.empty(max(l.mam_coo_spmm_by_rows_workspace(R), 1), dtype=torch.uint8, device=b.device)
+    ws = torch.empty(l.mam_coo_spmm_by_rows_workspace(R), dtype=torch.uint8, device=b.device)
     with torch.cuda.device(b.device):
         _check(l.mam_coo_spmm_by_rows(_p(row), _p(col), _p(val), val.numel(), _p(b), _ld(b), _p(c), R, K, C, _p(ws), ws.numel(),
                                       _stream(b)))
-    return c
+    return c, not bool(ws[:1024].any())
 
 
 def coo_spmm(row, col, val, b, R):

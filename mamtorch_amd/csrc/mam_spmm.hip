@@ -293,17 +293,21 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
 
 // crow[r] = entries whose row is below r, for rows in ascending order.  A wave per r narrows the place down to one entry
 // 64-fold a step (four steps for 2^24 entries); for rows in any other order it ends all the same, inside 0 .. nnz.
-// verdicts: the first VERDICTS workgroups look whether the rows ascend instead (a tensor may be flagged as coalesced without
-// being so).
+// verdicts: the first VERDICTS workgroups look instead whether the rows ascend (a tensor may be flagged as coalesced without
+// being so) and none holds more than `longest` entries.
 __global__ __launch_bounds__(NT) void row_offsets_kernel(const int64_t *__restrict__ row, int64_t nnz,
                                                          int64_t *__restrict__ crow, int64_t R,
-                                                         uint32_t *__restrict__ verdicts)
+                                                         uint32_t *__restrict__ verdicts, int64_t longest)
 {
     const int checking = verdicts ? VERDICTS : 0;
     if ((int)blockIdx.x < checking) {
         bool bad = false;
 #pragma unroll 4
-        for (int64_t e = (int64_t)blockIdx.x * NT + threadIdx.x; e < nnz - 1; e += (int64_t)VERDICTS * NT) bad |= row[e + 1] < row[e];
+        for (int64_t e = (int64_t)blockIdx.x * NT + threadIdx.x; e < nnz - 1; e += (int64_t)VERDICTS * NT) {
+            bad |= row[e + 1] < row[e];
+            const int64_t far = longest < nnz - e ? e + longest : nnz - 1;       // (loads without a condition: they are issued together)
+            bad |= (row[far] == row[e]) & (far - e == longest);
+        }
         const int any = __syncthreads_or(bad);
         if (threadIdx.x == 0) verdicts[blockIdx.x] = any ? 1u : 0u;
         return;
@@ -434,11 +438,22 @@ static int launch_coo(const int64_t *row, const int64_t *col, const float *val, 
     return check_launch("coo_spmm_kernel");
 }
 
-static int launch_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, uint32_t *verdicts, hipStream_t st)
+// Entries of a COO operand's row that its wave may take one after the other: 8 are loaded at once, 0.45 us (narrow c: 16 or 32,
+// 0.75 us), so that no row alone takes longer than the COO kernel, 12 us and at least 0.28 us per 2^20 entries times columns, takes for
+// everything.  (One row full, us by rows / by entries: 4096 x 4096 at 1 % x 4096 columns 296 / 382, by rows; 64 x 4096 at 1 % x 4096 235 / 25,
+// 4096 x 32768 with 8 entries in the others x 1024 1864 / 117, 300 x 1000 at 1 % x 260 34 / 14.)
+static int64_t longest_row(int64_t nnz, int64_t C)
+{
+    const int64_t entries = 256 + (int64_t)((double)nnz * (double)C / (1 << 17));
+    return C <= 128 ? 2 * entries : entries;
+}
+
+static int launch_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, uint32_t *verdicts, int64_t longest,
+                              hipStream_t st)
 {
     const int64_t blocks = ceil_div(R + 1, NT / 64);
     hipLaunchKernelGGL(row_offsets_kernel, dim3((unsigned)(blocks < (1 << 20) ? blocks : 1 << 20) + (verdicts ? VERDICTS : 0)),
-                       dim3(NT), 0, st, row, nnz, crow, R, verdicts);
+                       dim3(NT), 0, st, row, nnz, crow, R, verdicts, longest);
     return check_launch("row_offsets_kernel");
 }
 
@@ -476,7 +491,7 @@ extern "C" int mam_coo_row_offsets(const int64_t *row, int64_t nnz, int64_t *cro
     if (nnz < 0 || R < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
     if (R > INT32_MAX / 2) return fail(MAM_ERR_UNSUPPORTED, "a dimension exceeds 2^30");
     if (!crow || (nnz > 0 && !row)) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
-    return spmm::launch_row_offsets(row, nnz, crow, R, nullptr, static_cast<hipStream_t>(stream));
+    return spmm::launch_row_offsets(row, nnz, crow, R, nullptr, 0, static_cast<hipStream_t>(stream));
 }
 
 extern "C" size_t mam_coo_spmm_by_rows_workspace(int64_t R)
@@ -499,7 +514,7 @@ extern "C" int mam_coo_spmm_by_rows(const int64_t *row, const int64_t *col, cons
     hipStream_t st = static_cast<hipStream_t>(stream);
     uint32_t *verdicts = static_cast<uint32_t *>(workspace);
     int64_t *crow = reinterpret_cast<int64_t *>(verdicts + spmm::VERDICTS);
-    rc = spmm::launch_row_offsets(row, nnz, crow, R, verdicts, st);
+    rc = spmm::launch_row_offsets(row, nnz, crow, R, verdicts, spmm::longest_row(nnz, C), st);
     if (rc == MAM_OK) rc = spmm::launch_csr(crow, col, val, b, ldb, c, R, K, C, verdicts, st);
     if (rc == MAM_OK && nnz > 0) rc = spmm::launch_coo(row, col, val, nnz, b, ldb, c, K, C, verdicts, st);
     return rc;

@@ -594,8 +594,9 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     const at::Tensor val = a._values().contiguous();
     const int64_t nnz = val.numel();
     // A coalesced operand's rows ascend (the device looks whether they do: the flag can be set without it): with row offsets it is a
-    // CSR operand, whose kernel adds a row up in registers instead of clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns: 364 -> 107 us).  A row is one wave's there, at most K / 8 rounds of
-    // loads, 0.4 us each: not for K so large that one crowded row would outlast the COO kernel (nor for more rows than a launch holds waves).
+    // CSR operand, whose kernel adds a row up in registers instead of clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns:
+    // 364 -> 116 us).  A row is one wave's there, so the device looks for crowded ones too.  Up to the K that both were timed at
+    // (4096 x 32768 with 33 entries a row x 4096 columns: 477 -> 290 us), and no more rows than a launch holds waves.
     const bool by_rows = a.is_coalesced() && K <= 32768 && R <= (int64_t(1) << 24);
     if (dense_route_pays(nnz, R, K, C, by_rows ? 8 : 16)) {
         auto dense = at::empty({R, K}, b.options());

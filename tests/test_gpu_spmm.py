@@ -113,6 +113,31 @@ def test_operands_flagged_as_coalesced_whatever_their_order(cols, spoil):
     _check(mt.sparse.kernel.v1.cusparsemm(a, b.to(DEV)), want, floor, spoil)
 
 
+@pytest.mark.parametrize("rows,k,cols,each", [(64, 4096, 64, 41), (300, 1000, 260, 10), (5, 90, 3, 2), (40, 2000, 129, 0)])
+@pytest.mark.parametrize("at", [0, 1, -1])
+@pytest.mark.parametrize("more", [0, 1])
+def test_crowded_rows_are_not_one_wave_s(rows, k, cols, each, at, more):
+    """Rows of the most entries that a wave takes, and of one more: nnz * cols / 2^17 + 256, twice that up to 128 columns.  The
+    result either way, and which way it was."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator().manual_seed(rows)
+    lengths = [each] * rows
+    longest = lambda n: (256 + int(n * cols / 2 ** 17)) * (2 if cols <= 128 else 1)
+    while longest(sum(lengths)) != lengths[at % rows]:          # (it counts into nnz itself)
+        lengths[at % rows] = longest(sum(lengths))
+    lengths[at % rows] += more
+    row = torch.repeat_interleave(torch.arange(rows), torch.tensor(lengths))
+    nnz = row.numel()
+    assert (longest(nnz) < max(lengths)) == bool(more)
+    col, val = torch.randint(0, k, (nnz,), generator=g), torch.randn(nnz, generator=g)
+    b = torch.randn(k, cols, generator=g)
+    want, floor = oracle.coo_spmm(row.numpy(), col.numpy(), val.numpy(), b.numpy(), rows)
+    c, by_rows = capi.coo_spmm_by_rows(row.to(DEV), col.to(DEV), val.to(DEV), b.to(DEV), rows)
+    assert by_rows == (not more)
+    _check(c, want, floor, "crowded" if more else "not crowded")
+
+
 def test_coo_unsorted_with_duplicates_and_strided_b():
     from mamtorch_amd import capi
 
