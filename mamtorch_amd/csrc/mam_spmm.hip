@@ -23,7 +23,7 @@
 //        atomic adds when the row changes.  On row-sorted input (what Tensor.to_sparse() and
 //        coalesce() produce) that is about one flush per row and wave.
 // Products are fused multiply-adds in ascending entry order within a wave (narrow c: within each of the two or four
-// parts of a row); sums that span waves (COO only) are combined in no fixed order.
+// parts of a row), 64 of them at a time; sums that span waves (COO only) are combined in no fixed order.
 #include "mam_common.h"
 
 namespace mam {
@@ -102,7 +102,9 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Place at_block = place_of(row_blocks);
-    const int panel = at_block.panel, r = at_block.block * (NT / 64) + wave;
+    // (uniform, but the division leaves them in vector registers: 97 instead of 96 with several entries per load, and 65536 x 512
+    // with 10 entries a row x 50 columns takes 25 us for 21)
+    const int panel = __builtin_amdgcn_readfirstlane(at_block.panel), r = __builtin_amdgcn_readfirstlane(at_block.block) * (NT / 64) + wave;
     if (r >= R) return;
     constexpr int LANES = 64 / PER;      // of one entry; the parts are added at the end
     const int c0 = panel * LANES * TI + lane % LANES * TI;
@@ -162,8 +164,21 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
 #pragma unroll
         for (int u = 0; u < EG; ++u) axpy(acc, wv[u], xv[u]);
     };
+    // sums of 64 terms are added to a sum of their own, as coo_spmm_kernel adds its to c: a row's rounding errors grow with 64 + n /
+    // 64 instead of with n
+    float total[TI];
+#pragma unroll
+    for (int t = 0; t < TI; ++t) total[t] = 0.0f;
+    auto fold = [&] {
+#pragma unroll
+        for (int t = 0; t < TI; ++t) {
+            total[t] += acc[t];
+            acc[t] = 0.0f;
+        }
+    };
     if (ng > 0) issue(0, xa, wa);
     for (int g = 0; g < ng; g += 2) {
+        if (g % (COO_CHUNK / EG) == 0) fold();
         if (g + 1 < ng) issue(g + 1, xb, wb);
         __builtin_amdgcn_sched_barrier(0);
         consume(xa, wa);
@@ -198,6 +213,8 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
             axpy(acc, val[e], near_row((uint32_t)col[e] * row_bytes + cl * 4, 0));
         }
     }
+#pragma unroll
+    for (int t = 0; t < TI; ++t) acc[t] += total[t];
 #pragma unroll
     for (int s = LANES; s < 64; s <<= 1)
 #pragma unroll

@@ -75,6 +75,25 @@ def test_column_counts_around_the_panels(cols):
         _check(capi.coo_spmm(idx[0].contiguous(), idx[1].contiguous(), values, bd, rows), want, floor, "coo, offset %d" % offset)
 
 
+@pytest.mark.parametrize("n", [63, 64, 65, 127, 4000, 20000, 32768])
+@pytest.mark.parametrize("cols", [4, 100, 200])
+@pytest.mark.parametrize("layout", [torch.sparse_csr, torch.sparse_coo])
+def test_long_rows_are_added_up_in_short_sums(n, cols, layout):
+    """Equal terms round the same way each time: n of them in one running sum are off by up to n roundings (0.1 and 0.7, 4000 to
+    32768 terms: 4e-5 to 3e-4), sums of 64 that are then added by 64 + n / 64, and a few for the parts of a row."""
+    import mamtorch_amd as mt
+
+    rows, k = 20, n + 300
+    a = torch.zeros(rows, k)
+    a[7, 100:100 + n] = 1.0
+    a[12, :3] = 1.0
+    b = torch.full((k, cols), 0.1)
+    b[:, 1::2] = 0.7
+    got = mt.sparse.kernel.v1.cusparsemm(a.to(DEV).to_sparse(layout=layout), b.to(DEV)).cpu().double()
+    want = a.double() @ b.double()
+    assert bool(((got - want).abs() <= (64 + n / 64 + 4) * 2.0 ** -24 * want).all())
+
+
 @pytest.mark.parametrize("nnz,rows", [(0, 5), (1, 1), (63, 9), (64, 300), (65, 3), (4096, 70), (4097, 1), (300000, 4001)])
 def test_row_offsets(nnz, rows):
     from mamtorch_amd import capi
