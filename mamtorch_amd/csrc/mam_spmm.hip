@@ -95,7 +95,7 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
                                                       const int64_t *__restrict__ col,
                                                       const float *__restrict__ val,
                                                       const float *__restrict__ b, int64_t ldb, uint32_t b_bytes,
-                                                      float *__restrict__ c, int R, int C, int row_blocks,
+                                                      float *__restrict__ c, int R, int C, int row_blocks, int width,
                                                       const uint32_t *__restrict__ verdicts)
 {
     typedef typename Vec<TI>::type vec;
@@ -107,8 +107,10 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     const int panel = __builtin_amdgcn_readfirstlane(at_block.panel), r = __builtin_amdgcn_readfirstlane(at_block.block) * (NT / 64) + wave;
     if (r >= R) return;
     constexpr int LANES = 64 / PER;      // of one entry; the parts are added at the end
-    const int c0 = panel * LANES * TI + lane % LANES * TI;
-    const int cl = c0 < C ? c0 : 0;  // lanes past the last column read column 0 and store nothing
+    if (PER > 1) width = LANES * TI;     // (one panel)
+    const int c0 = panel * width + lane % LANES * TI;
+    const bool in = lane % LANES * TI < width && c0 < C;
+    const int cl = in ? c0 : panel * width;  // lanes past the panel's last column read its first and store nothing
     const int part = lane / LANES;
 
     const_i64 *ccol = (const_i64 *)col;
@@ -219,7 +221,7 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     for (int s = LANES; s < 64; s <<= 1)
 #pragma unroll
         for (int t = 0; t < TI; ++t) acc[t] += __shfl_xor(acc[t], s);
-    if (part != 0) return;
+    if (part != 0 || !in) return;
     float *dst = c + (int64_t)r * C + c0;
     if (TI == 4 && c0 + 3 < C) {
         store4(dst, acc);
@@ -421,11 +423,14 @@ static int launch_csr(const int64_t *crow, const int64_t *col, const float *val,
     const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
     const int per = !near ? 1 : C <= 64 ? 4 : C <= 128 ? 2 : 1;          // entries per load
     const int64_t panels = ceil_div(C, near || wide ? 256 / per : 64);
+    // panels of one width, whole lines: a narrow last one would leave the XCDs that work on it half idle (4096 x 4096 at 5 % x 260
+    // columns as 256 + 4: 64 us, 160 + 100: 54 us; 1 % x 300 columns 18 and 14 us)
+    const int width = (int)(ceil_div(ceil_div(C, panels), 32) * 32);
     const int64_t row_blocks = ceil_div(R, NT / 64);
     if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid_of(panels, row_blocks), dim3(NT), 0, st, crow, col, val, b, ldb, (uint32_t)b_bytes, c,
-                           (int)R, (int)C, (int)row_blocks, verdicts);
+                           (int)R, (int)C, (int)row_blocks, width, verdicts);
     };
     if (per == 4) launch(csr_spmm_kernel<4, true, 4>);
     else if (per == 2) launch(csr_spmm_kernel<4, true, 2>);
