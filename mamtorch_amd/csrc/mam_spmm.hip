@@ -460,15 +460,11 @@ static int launch_coo(const int64_t *row, const int64_t *col, const float *val, 
     return check_launch("coo_spmm_kernel");
 }
 
-// Entries of a COO operand's row that its wave may take one after the other: 8 are loaded at once, 0.45 us (narrow c: 16 or 32,
-// 0.75 us), so that no row alone takes longer than the COO kernel, 12 us and at least 0.28 us per 2^20 entries times columns, takes for
-// everything.  (One row full, us by rows / by entries: 4096 x 4096 at 1 % x 4096 columns 296 / 382, by rows; 64 x 4096 at 1 % x 4096 235 / 25,
+// Entries of a COO operand's row that its wave may take one after the other, 0.05 us each (8 in 0.45 us, narrow c: 16 in 0.85), so that
+// no row alone takes longer than the COO kernel, 12 us and at least 0.28 us per 2^20 entries times columns, takes for everything.
+// (One row full, us by rows / by entries: 4096 x 4096 at 1 % x 4096 columns 296 / 382, by rows; 64 x 4096 at 1 % x 4096 235 / 25,
 // 4096 x 32768 with 8 entries in the others x 1024 1864 / 117, 300 x 1000 at 1 % x 260 34 / 14.)
-static int64_t longest_row(int64_t nnz, int64_t C)
-{
-    const int64_t entries = 256 + (int64_t)((double)nnz * (double)C / (1 << 17));
-    return C <= 128 ? 2 * entries : entries;
-}
+static int64_t longest_row(int64_t nnz, int64_t C) { return 256 + (int64_t)((double)nnz * (double)C / (1 << 17)); }
 
 static int launch_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, uint32_t *verdicts, int64_t longest,
                               hipStream_t st)
