@@ -30,7 +30,10 @@ namespace mam {
 namespace spmm {
 
 constexpr int NT = 256;
-constexpr int EG = 8;          // entries whose loads are issued together
+// loads issued together: fewer where one holds four entries (65536 x 512 with 10 entries a row x 50 columns, 4 and 8: 16.9 and 20.9
+// us, 50 entries x 64 columns 42 and 54; one row of 32768 entries alone 1660 and 1560), not where it holds two (10 entries a row x
+// 100 columns 17.6 and 20.4, the row alone x 128 columns 2230 and 1730)
+constexpr int loads_of(int per) { return per > 2 ? 4 : 8; }
 constexpr int COO_CHUNK = 64;  // entries per wave and pass
 
 typedef const __attribute__((address_space(4))) int64_t const_i64;
@@ -102,10 +105,10 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const Place at_block = place_of(row_blocks);
-    // (uniform, but the division leaves them in vector registers: 97 instead of 96 with several entries per load, and 65536 x 512
-    // with 10 entries a row x 50 columns takes 25 us for 21)
+    // (uniform, but the division leaves them in vector registers: 97 of 96 with two entries per load)
     const int panel = __builtin_amdgcn_readfirstlane(at_block.panel), r = __builtin_amdgcn_readfirstlane(at_block.block) * (NT / 64) + wave;
     if (r >= R) return;
+    constexpr int EG = loads_of(PER);
     constexpr int LANES = 64 / PER;      // of one entry; the parts are added at the end
     if (PER > 1) width = LANES * TI;     // (one panel)
     const int c0 = panel * width + lane % LANES * TI;
@@ -258,6 +261,7 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
                                                       const uint32_t *__restrict__ verdicts)
 {
     typedef typename Vec<TI>::type vec;
+    constexpr int EG = loads_of(1);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (verdicts && !not_by_rows(verdicts)) return;
