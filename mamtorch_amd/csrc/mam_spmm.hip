@@ -54,8 +54,10 @@ __device__ __forceinline__ void axpy(float (&acc)[4], float v, const float4 &b)
     acc[3] = __builtin_fmaf(v, b.w, acc[3]);
 }
 
-// Which panel of columns a workgroup works on and which block of rows or entries: numbered panel by panel over the XCDs, or,
-// where that would be more than a launch holds in one dimension, a row of the grid each.
+// Which panel of columns a workgroup works on and which block of rows: numbered panel by panel over the XCDs, or a row of the grid
+// each, so that all XCDs walk one panel at a time: where the numbers would be more than a launch holds in one dimension, and where the
+// panels of eight XCDs are too much for the memory-side cache together (us by XCDs and in turn, 4096 columns: K = 4096 107 / 126, 16384 293 /
+// 310, 32768 346 / 346, 65536 354 / 346; 1024 columns, four panels: 65536 91.6 / 93.2).
 struct Place { int panel, block; };
 __device__ __forceinline__ Place place_of(int blocks)
 {
@@ -63,10 +65,11 @@ __device__ __forceinline__ Place place_of(int blocks)
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     return {logical / blocks, logical % blocks};
 }
-static dim3 grid_of(int64_t panels, int64_t blocks)
+constexpr int64_t MOST_PANEL_ROWS = 8 * 32768;           // of b, in the panels that are walked at once
+static dim3 grid_of(int64_t panels, int64_t blocks, int64_t K)
 {
     // less than 2^32 threads in a dimension
-    return panels * blocks < UINT32_MAX / NT ? dim3((unsigned)(panels * blocks)) : dim3((unsigned)blocks, (unsigned)panels);
+    return K * (panels < 8 ? panels : 8) <= MOST_PANEL_ROWS && panels * blocks < UINT32_MAX / NT ? dim3((unsigned)(panels * blocks)) : dim3((unsigned)blocks, (unsigned)panels);
 }
 
 // four consecutive words, 4-byte aligned
@@ -433,7 +436,7 @@ static int launch_csr(const int64_t *crow, const int64_t *col, const float *val,
     const int64_t row_blocks = ceil_div(R, NT / 64);
     if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid_of(panels, row_blocks), dim3(NT), 0, st, crow, col, val, b, ldb, (uint32_t)b_bytes, c,
+        hipLaunchKernelGGL(kernel, grid_of(panels, row_blocks, K), dim3(NT), 0, st, crow, col, val, b, ldb, (uint32_t)b_bytes, c,
                            (int)R, (int)C, (int)row_blocks, width, verdicts);
     };
     if (per == 4) launch(csr_spmm_kernel<4, true, 4>);

@@ -75,6 +75,21 @@ def test_column_counts_around_the_panels(cols):
         _check(capi.coo_spmm(idx[0].contiguous(), idx[1].contiguous(), values, bd, rows), want, floor, "coo, offset %d" % offset)
 
 
+@pytest.mark.parametrize("k,cols", [(32768, 2000), (32769, 2000), (70000, 600), (90000, 600), (300000, 64)])
+def test_panels_by_xcd_and_in_turn(k, cols):
+    """Workgroups are numbered panel by panel up to 2^18 rows of b in the (at most eight) panels, and have a grid row per panel
+    above: 8, 8, 3, 3 panels and one."""
+    from mamtorch_amd import capi
+
+    rows, each = 90, 70
+    g = torch.Generator(device=DEV).manual_seed(k)
+    crow, col = torch.arange(rows + 1, device=DEV) * each, torch.randint(0, k, (rows * each,), generator=g, device=DEV)
+    col[::7] = k - 1
+    val, b = torch.randn(rows * each, generator=g, device=DEV), torch.randn(k, cols, generator=g, device=DEV)
+    terms = (val.double()[:, None] * b[col].double()).view(rows, each, cols)
+    _check(capi.csr_spmm(crow, col, val, b, rows), terms.sum(1).cpu().numpy(), terms.abs().sum(1).cpu().numpy(), "csr")
+
+
 @pytest.mark.parametrize("n", [63, 64, 65, 127, 4000, 20000, 32768])
 @pytest.mark.parametrize("cols", [4, 100, 200])
 @pytest.mark.parametrize("layout", [torch.sparse_csr, torch.sparse_coo])
