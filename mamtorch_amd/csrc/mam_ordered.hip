@@ -989,7 +989,8 @@ struct Lanes {
     static __device__ __forceinline__ int base(int quad, int K) { return TWO ? quad * K * 4 : quad * 4; }
 };
 
-template <int TB, bool ARGS, bool TWO>
+// PAST: stores that are lines by this layout go past the L2 (launch_forward says when they are lines in memory).
+template <int TB, bool ARGS, bool TWO, bool PAST>
 __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 {
     typedef Extremes<ARGS> E;
@@ -1355,7 +1356,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                     if (blk * RW + sr >= a.rows) {
                     } else if (whole && ((uintptr_t)dst & 15) == 0) {
                         const floats4 all = {t[0], t[1], t[2], t[3]};
-                        if constexpr (TB == 32) __builtin_nontemporal_store(all, reinterpret_cast<floats4 *>(to + lane_off));
+                        if constexpr (PAST && TB == 32) __builtin_nontemporal_store(all, reinterpret_cast<floats4 *>(to + lane_off));
                         else *reinterpret_cast<floats4 *>(to + lane_off) = all;
                     } else {
 #pragma unroll
@@ -1366,7 +1367,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
 #pragma unroll
                     for (int j = 0; j < 4; ++j)
                         if (b0 + q * 4 + j < b.rows) {
-                            if constexpr (RW >= 32) __builtin_nontemporal_store(v[j], to + lane_off + j * (uint32_t)c.M);
+                            if constexpr (PAST && RW >= 32) __builtin_nontemporal_store(v[j], to + lane_off + j * (uint32_t)c.M);
                             else to[lane_off + j * (uint32_t)c.M] = v[j];
                         }
                 }
@@ -1470,21 +1471,30 @@ static int launch_forward(const Params &p, hipStream_t st)
     const int tx = (int)ceil_div(M, TB), tw = (int)ceil_div(N, TB);
     const int64_t bx = (int64_t)tx * splits_of(TB, N, tx, p.cus), bw = (int64_t)tw * splits_of(TB, M, tw, p.cus);
     const unsigned blocks = (unsigned)(bx > bw || p.call.w_layout != MAM_W_MK ? bx : bw);
-    if (p.call.argmax)
-        hipLaunchKernelGGL((forward_kernel<TB, true, TWO>), dim3(blocks), dim3(NT), lds, st, p);
-    else
-        hipLaunchKernelGGL((forward_kernel<TB, false, TWO>), dim3(blocks), dim3(NT), lds, st, p);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(NT), lds, st, p); };
+    // The 32 words that neighbouring lanes store are one line in memory only where rows of c start lines.  Elsewhere they are parts of
+    // two, which the five or seven planes of a one-sided search had better leave to the L2 (past it / to it, us: 12608 x 768 -> 3004 862 /
+    // 718, -> 3040 559 / 619; 16384 x 4096 -> 1001 444 / 374, -> 1024 353 / 364); the values alone go past it either way (-> 1001 253 /
+    // 261, 12608 x 768 -> 3004 401 / 402), and two-sided searches do (12608 x 768 -> 3001 2058 / 2148, 16384 x 2048 -> 1000 645 / 670).
+    const Call &c = p.call;
+    const bool lines = c.M % 32 == 0 && (((uintptr_t)c.c | (uintptr_t)c.argmax | (uintptr_t)c.argmin | (uintptr_t)c.wsel | (uintptr_t)c.xsel) & 127) == 0;
+    constexpr bool always = TWO, never = TB == 16;      // (16 rows: no lines by the layout)
+    if (!c.argmax) launch(forward_kernel<TB, false, TWO, true>);
+    else if (always || (lines && !never)) launch(forward_kernel<TB, true, TWO, !never>);
+    else launch(forward_kernel<TB, true, TWO, always>);
     return check_launch("ordered::forward_kernel");
 }
 
 static int setup_device(int)
 {
     const void *kernels[] = {
-        (const void *)forward_kernel<4, true, false>,   (const void *)forward_kernel<8, true, false>,
-        (const void *)forward_kernel<16, true, false>,  (const void *)forward_kernel<32, true, false>,
-        (const void *)forward_kernel<4, false, false>,  (const void *)forward_kernel<8, false, false>,
-        (const void *)forward_kernel<16, false, false>, (const void *)forward_kernel<32, false, false>,
-        (const void *)forward_kernel<8, true, true>,    (const void *)forward_kernel<8, false, true>};
+        (const void *)forward_kernel<4, true, false, true>,   (const void *)forward_kernel<4, true, false, false>,
+        (const void *)forward_kernel<8, true, false, true>,   (const void *)forward_kernel<8, true, false, false>,
+        (const void *)forward_kernel<32, true, false, true>,  (const void *)forward_kernel<32, true, false, false>,
+        (const void *)forward_kernel<16, true, false, false>, (const void *)forward_kernel<8, true, true, true>,
+        (const void *)forward_kernel<4, false, false, true>,  (const void *)forward_kernel<8, false, false, true>,
+        (const void *)forward_kernel<16, false, false, true>, (const void *)forward_kernel<32, false, false, true>,
+        (const void *)forward_kernel<8, false, true, true>};
     for (const void *k : kernels)
         if (hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 158 * 1024) != hipSuccess) {
             (void)hipGetLastError();

@@ -118,6 +118,13 @@ def test_equal_products_met_by_different_lanes(N, K, M, kinds):
     _check(N, K, M, *kinds, seed=N)
 
 
+@pytest.mark.parametrize("K", [800, 3000, 5000])                      # 32, 8 and 4 tile rows
+@pytest.mark.parametrize("M", [32, 64, 96, 100, 101])
+@pytest.mark.parametrize("kinds", [("normal", "uniform"), ("uniform", "normal")])
+def test_outputs_that_are_lines_and_parts_of_lines(K, M, kinds):
+    _check(70, K, M, *kinds, seed=M)
+
+
 @pytest.mark.parametrize("kind", ["ties", "positive", "zero rows", "nan and inf", "sparse", "denormal", "overflow"])
 @pytest.mark.parametrize("other", ["uniform", "normal", "same"])
 def test_data_the_lists_do_not_finish(kind, other):
