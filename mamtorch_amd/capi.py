@@ -213,6 +213,23 @@ def fc_backward(x, w, grad, argmax, argmin, layout=W_KM, want_x=True, want_w=Tru
     return xg, wg
 
 
+def fc_backward_bias(x, w, grad, argmax, argmin, layout=W_KM, w_sel=None, x_sel=None, range_len=0, workspace_bytes=None):
+    """fc_backward (range_len 0) or fc_backward_ranges and the column sums of grad as one call -> (x_grad, w_grad, bias_grad)."""
+    l = lib()
+    N, K, M = _dims(x, w, layout)
+    xg = torch.empty((N, K), dtype=torch.float32, device=x.device)
+    wg = torch.empty(tuple(w.shape), dtype=torch.float32, device=x.device)
+    bg = torch.empty(M, dtype=torch.float32, device=x.device)
+    if workspace_bytes is None:
+        workspace_bytes = l.mam_fc_backward_bias_workspace(N, K, M)
+    ws = torch.empty(max(workspace_bytes, 1), dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        _check(l.mam_fc_backward_bias(_p(x), _ld(x), _p(w), _ld(w), layout, _p(grad), _p(argmax), _p(argmin), _p(w_sel),
+                                      _p(x_sel), _p(xg), _p(wg), _p(bg), N, K, M, range_len, _p(ws) if workspace_bytes else None,
+                                      workspace_bytes, _stream(x)))
+    return xg, wg, bg
+
+
 def fc_backward_count(x, w, grad, argmax, argmin, max_count, min_count, mode=COUNT_HITS, layout=W_KM, want_x=True,
                       want_w=True, w_sel=None, x_sel=None):
     """fc_backward and selection_count (in place on the (M, K) int32 counters) as one call."""

@@ -1120,8 +1120,8 @@ extern "C" int mam_fc_backward(const float *x, int64_t ldx, const float *w, int6
 
 extern "C" size_t mam_fc_backward_bias_workspace(int64_t N, int64_t K, int64_t M)
 {
-    if (N <= 0 || K <= 0 || M <= 0) return 0;
-    const size_t shares = N >= 2048 ? (size_t)mam::bwd::most_shares(N, K) * (size_t)M * sizeof(float) : 0;
+    if (N <= 0 || K < 0 || M <= 0) return 0;
+    const size_t shares = K > 0 && N >= 2048 ? (size_t)mam::bwd::most_shares(N, K) * (size_t)M * sizeof(float) : 0;
     const size_t slabs = mam_bias_grad_workspace(N, M);
     return shares > slabs ? shares : slabs;
 }
@@ -1134,9 +1134,9 @@ extern "C" int mam_fc_backward_bias(const float *x, int64_t ldx, const float *w,
 {
     using namespace mam;
     if (range_len < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative range_len");
-    if (N > 0 && K > 0 && M > 0 && workspace_bytes < mam_fc_backward_bias_workspace(N, K, M))
-        return fail(MAM_ERR_WORKSPACE, "the bias gradient needs %zu workspace bytes, got %zu",
-                    mam_fc_backward_bias_workspace(N, K, M), workspace_bytes);
+    const size_t need = mam_fc_backward_bias_workspace(N, K, M);
+    if (need > 0 && (!workspace || workspace_bytes < need))
+        return fail(MAM_ERR_WORKSPACE, "the bias gradient needs %zu workspace bytes, got %zu", need, workspace ? workspace_bytes : (size_t)0);
     if (M > 0 && !bias_grad) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     const int64_t planes = range_len > 0 && K > 0 ? (K + range_len - 1) / range_len : 1;
     if (planes > 65535) return fail(MAM_ERR_UNSUPPORTED, "more than 65535 ranges");

@@ -459,3 +459,29 @@ def test_backward_count_equals_the_two_calls(shape, mode):
     else:
         want_m, want_n = oracle.selection_count(amax.cpu().numpy(), amin.cpu().numpy(), before, before, mode=mode)
     assert np.array_equal(mc2.cpu().numpy(), want_m) and np.array_equal(nc2.cpu().numpy(), want_n)
+
+
+@pytest.mark.parametrize("N", [1, 512, 513, 2048, 5000])
+@pytest.mark.parametrize("K", [0, 7])
+@pytest.mark.parametrize("M", [3, 8])
+def test_bias_entry_with_the_workspace_it_asks_for_and_less(N, K, M):
+    """mam_fc_backward_bias: what the query says is enough, without inputs too; one byte less is refused before any launch."""
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    gen = torch.Generator().manual_seed(N)
+    x, w, grad = torch.randn(N, K, generator=gen), torch.randn(M, K, generator=gen), torch.randn(N, M, generator=gen)
+    picks = torch.randint(0, max(K, 1), (2, N, M), generator=gen, dtype=torch.int32).to(dev)
+    args = (x.to(dev), w.to(dev), grad.to(dev), picks[0], picks[1], capi.W_MK)
+    xg, wg, bg = capi.fc_backward_bias(*args)
+    want, floor = grad.double().sum(0), grad.abs().double().sum(0)
+    assert bool(((bg.cpu().double() - want).abs() <= RTOL * want.abs() + FLOOR * floor).all())
+    if K > 0:
+        xo, wo = oracle.backward(x.numpy(), w.numpy(), grad.numpy(), picks[0].cpu().numpy(), picks[1].cpu().numpy(), oracle.W_MK)
+        np.testing.assert_allclose(xg.cpu().numpy(), xo, rtol=RTOL, atol=1e-5)
+        np.testing.assert_allclose(wg.cpu().numpy(), wo, rtol=RTOL, atol=FLOOR * N * 16)
+    need = capi.lib().mam_fc_backward_bias_workspace(N, K, M)
+    assert (need > 0) == (N > 512)
+    if need > 0:
+        with pytest.raises(RuntimeError, match="workspace bytes"):
+            capi.fc_backward_bias(*args, workspace_bytes=need - 1)
