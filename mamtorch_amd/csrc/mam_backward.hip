@@ -424,8 +424,10 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
 // scatters are counted in a second LDS plane behind the histogram and added to max_count / min_count when the
 // slab is streamed out -- the index arrays are read once for both, and one launch serves both.
 // bias_out ([share][M], workgroups of the first k chunk): the sum of grad over the share's rows, from the items that are read
-// anyway; a thread's items lie in one quad of neurons, so it adds in registers and the threads of a quad are added in a
-// fixed order.
+// anyway; a thread's items lie in one quad of neurons, so it adds in registers, and the threads of a quad are added in a
+// fixed order.  BIAS_TERMS of a thread's items make a sum of their own, so that rounding errors do not grow with the batch (one
+// running sum per thread: 2-norm error 1.07e-6 for 400000 rows where mam_bias_grad's 256 running sums give 6.5e-7).
+constexpr int BIAS_TERMS = 64;
 template <int LAYOUT, int NT, bool COUNT = false>
 __device__ __forceinline__ void bwd_w_vec_body(
     float *hist, int bx, int nbx, int by, int bz, int nbz,
@@ -493,7 +495,11 @@ __device__ __forceinline__ void bwd_w_vec_body(
             *reinterpret_cast<float4 *>(&hist[i]) = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
         if (have) scatter_quad<LAYOUT, COUNT>(hist, g, i1, i2, x1, x2, r_first, k0, kn, kc, log2r, cnt);
-        float4 bias_sum = have && pf == 0 ? g : make_float4(0.f, 0.f, 0.f, 0.f);
+        float4 bias_now = have && pf == 0 ? g : make_float4(0.f, 0.f, 0.f, 0.f), bias_sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        auto fold = [&] {
+            bias_sum = make_float4(bias_sum.x + bias_now.x, bias_sum.y + bias_now.y, bias_sum.z + bias_now.z, bias_sum.w + bias_now.w);
+            bias_now = make_float4(0.f, 0.f, 0.f, 0.f);
+        };
         for (int64_t it = tid + NT; it < items; it += NT) {
             const int pl = npl > 1 ? (int)(it / per_plane) : 0;
             const int64_t rem = npl > 1 ? it - pl * per_plane : it;
@@ -515,13 +521,15 @@ __device__ __forceinline__ void bwd_w_vec_body(
             }
             scatter_quad<LAYOUT, COUNT>(hist, gg, j1, j2, y1, y2, r0, k0, kn, kc, log2r, cnt);
             if (sum_bias && pl == 0) {
-                bias_sum.x += gg.x;
-                bias_sum.y += gg.y;
-                bias_sum.z += gg.z;
-                bias_sum.w += gg.w;
+                bias_now.x += gg.x;
+                bias_now.y += gg.y;
+                bias_now.z += gg.z;
+                bias_now.w += gg.w;
+                if (it / NT % BIAS_TERMS == BIAS_TERMS - 1) fold();
             }
         }
         if (sum_bias) {
+            fold();
             for (int s = qpr; s < 64; s <<= 1) {
                 bias_sum.x += __shfl_xor(bias_sum.x, s);
                 bias_sum.y += __shfl_xor(bias_sum.y, s);
@@ -741,7 +749,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
     extern __shared__ float hist[];
     __shared__ float bias_part[NT_W / 64][MAX_NEURONS];
     const bool sum_bias = bias_out != nullptr && blockIdx.y == 0;       // as in bwd_w_vec_body, a neuron per thread
-    float bias_sum = 0.0f;
+    float bias_now = 0.0f, bias_sum = 0.0f;
     const int tid = threadIdx.x;
     const int R = 1 << log2r;
     const int mt = xcd_remap(blockIdx.x, gridDim.x);
@@ -766,7 +774,10 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
             if (r >= rn) continue;
             const int64_t o = (int64_t)n * M + m0 + r;
             const float g = grad[o];
-            if (sum_bias && pl == 0) bias_sum += g;
+            if (sum_bias && pl == 0) {
+                bias_now += g;
+                if (pi / NT_W % BIAS_TERMS == BIAS_TERMS - 1) { bias_sum += bias_now; bias_now = 0.0f; }
+            }
             const int a1 = amax_pl[o] - k0, a2 = amin_pl[o] - k0;
             const float *xr = x + (int64_t)n * ldx + k0;
             if ((unsigned)a1 < (unsigned)kn)
@@ -778,6 +789,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
         }
     }
     if (sum_bias) {
+        bias_sum += bias_now;
         for (int s = R; s < 64; s <<= 1) bias_sum += __shfl_xor(bias_sum, s);
         if ((tid & 63) < R) bias_part[tid >> 6][tid & 63] = bias_sum;
     }

@@ -485,3 +485,23 @@ def test_bias_entry_with_the_workspace_it_asks_for_and_less(N, K, M):
     if need > 0:
         with pytest.raises(RuntimeError, match="workspace bytes"):
             capi.fc_backward_bias(*args, workspace_bytes=need - 1)
+
+
+@pytest.mark.parametrize("N,M", [(65536, 3), (65536, 8), (400000, 3), (400000, 8), (400000, 33), (400000, 36)])
+@pytest.mark.parametrize("layout", [0, 1])
+def test_bias_gradient_of_large_batches_in_short_sums(N, M, layout):
+    """Equal terms round the same way each time.  16 to 512 threads add up a neuron, each in sums of 64 terms, and are added by lane,
+    by wave and by share: at most 64 + N / 16 / 64 roundings and 24 for what follows.  (Running sums of 16 threads, 65536 rows: 3.9e-5,
+    of 128, 400000 rows: 3.2e-5.)"""
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    K = 8
+    threads = 128 if layout == capi.W_MK else 16
+    x, w = torch.ones(N, K, device=dev), torch.ones((M, K) if layout == capi.W_MK else (K, M), device=dev)
+    picks = torch.randint(0, K, (2, N, M), device=dev, dtype=torch.int32)
+    grad = torch.full((N, M), 0.1, device=dev)
+    grad[:, 1::2] = 0.7
+    _, _, bg = capi.fc_backward_bias(x, w, grad, picks[0], picks[1], layout)
+    want = grad.double().sum(0)
+    assert bool(((bg.double() - want).abs() <= (64 + N / threads / 64 + 24) * 2.0 ** -24 * want).all())
