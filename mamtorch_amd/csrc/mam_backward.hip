@@ -428,7 +428,7 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
 // fixed order.  BIAS_TERMS of a thread's items make a sum of their own, so that rounding errors do not grow with the batch (one
 // running sum per thread: 2-norm error 1.07e-6 for 400000 rows where mam_bias_grad's 256 running sums give 6.5e-7).
 constexpr int BIAS_TERMS = 64;
-template <int LAYOUT, int NT, bool COUNT = false>
+template <int LAYOUT, int NT, bool COUNT, bool BIAS>
 __device__ __forceinline__ void bwd_w_vec_body(
     float *hist, int bx, int nbx, int by, int bz, int nbz,
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
@@ -438,8 +438,9 @@ __device__ __forceinline__ void bwd_w_vec_body(
     int32_t *__restrict__ max_count = nullptr, int32_t *__restrict__ min_count = nullptr,
     float *__restrict__ bias_out = nullptr)
 {
-    __shared__ float bias_part[COUNT ? 1 : NT / 64][MAX_NEURONS];
-    const bool sum_bias = !COUNT && bias_out != nullptr && by == 0;
+    // (a form of its own without the bias gradient: its registers and LDS cost 2 % of 16384 x 2480 -> 1024, 242 and 248 us)
+    __shared__ __attribute__((aligned(16))) float bias_part[BIAS ? NT / 64 : 1][MAX_NEURONS];
+    const bool sum_bias = BIAS && by == 0;
     uint32_t *cnt = reinterpret_cast<uint32_t *>(hist) + ((size_t)kc << log2r);
     const int tid = threadIdx.x;
     const int R = 1 << log2r;
@@ -542,7 +543,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
         if (sum_bias && tid < rn) {
             float sum = bias_part[0][tid];
 #pragma unroll
-            for (int v = 1; v < (COUNT ? 1 : NT / 64); ++v) sum += bias_part[v][tid];
+            for (int v = 1; v < (BIAS ? NT / 64 : 1); ++v) sum += bias_part[v][tid];
             bias_out[(int64_t)bz * M + m0 + tid] = sum;
         }
         if (t + 1 < tiles_per_wg && mt + 1 < mtiles) load_first(m0 + R);
@@ -555,7 +556,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
     }
 }
 
-template <int LAYOUT>
+template <int LAYOUT, bool BIAS>
 __global__ __launch_bounds__(NT_W) void mam_bwd_w_vec_kernel(
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
@@ -564,7 +565,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_vec_kernel(
     float *__restrict__ bias_out)
 {
     extern __shared__ float hist[];
-    bwd_w_vec_body<LAYOUT, NT_W>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
+    bwd_w_vec_body<LAYOUT, NT_W, false, BIAS>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
                                  argmin, x_sel, nm, w_grad, N, K, M, log2r, kc, vec_out, mtiles, tiles_per_wg,
                                  rows_per_split, planes, range_len, nullptr, nullptr, bias_out);
 }
@@ -578,7 +579,7 @@ __global__ __launch_bounds__(NT_C) void mam_bwd_w_count_kernel(
     int32_t *__restrict__ min_count, int N, int K, int M, int log2r, int kc, int mtiles, int tiles_per_wg)
 {
     extern __shared__ float hist[];
-    bwd_w_vec_body<MAM_W_MK, NT_C, true>(hist, blockIdx.x, gridDim.x, blockIdx.y, 0, 1, x, ldx, grad, argmax, argmin,
+    bwd_w_vec_body<MAM_W_MK, NT_C, true, false>(hist, blockIdx.x, gridDim.x, blockIdx.y, 0, 1, x, ldx, grad, argmax, argmin,
                                          x_sel, nm, w_grad, N, K, M, log2r, kc, 1, mtiles, tiles_per_wg, N, 1, K,
                                          max_count, min_count);
 }
@@ -723,7 +724,7 @@ struct BothParams {
     int N, K, M, planes, range_len, span, kc_x;
     int log2r, kc_w, vec_out, mtiles, tiles_per_wg, x_wgs;
 };
-template <int LAYOUT>
+template <int LAYOUT, bool BIAS>
 __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
 {
     extern __shared__ unsigned long long both_lds[];
@@ -731,7 +732,7 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
         bwd_x_body<LAYOUT>(both_lds, blockIdx.x, p.w, p.ldw, p.grad, p.argmax, p.argmin, p.w_sel, p.nm, p.x_grad, p.K,
                            p.M, p.kc_x, p.planes, p.span);
     } else {
-        bwd_w_vec_body<LAYOUT, NT_X>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
+        bwd_w_vec_body<LAYOUT, NT_X, false, BIAS>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
                                      0, 1, p.x, p.ldx, p.grad, p.argmax, p.argmin, p.x_sel, p.nm, p.w_grad, p.N, p.K,
                                      p.M, p.log2r, p.kc_w, p.vec_out, p.mtiles, p.tiles_per_wg, p.N, p.planes,
                                      p.range_len, nullptr, nullptr, p.bias_grad);
@@ -739,7 +740,7 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
 }
 
 // Generic path: any M, any alignment; one (batch row, neuron) pair per thread and trip.
-template <int LAYOUT>
+template <int LAYOUT, bool BIAS>
 __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
@@ -747,8 +748,8 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
     int kc, int vec_out, int planes, int range_len, float *__restrict__ bias_out)
 {
     extern __shared__ float hist[];
-    __shared__ float bias_part[NT_W / 64][MAX_NEURONS];
-    const bool sum_bias = bias_out != nullptr && blockIdx.y == 0;       // as in bwd_w_vec_body, a neuron per thread
+    __shared__ float bias_part[BIAS ? NT_W / 64 : 1][MAX_NEURONS];
+    const bool sum_bias = BIAS && blockIdx.y == 0;       // as in bwd_w_vec_body, a neuron per thread
     float bias_now = 0.0f, bias_sum = 0.0f;
     const int tid = threadIdx.x;
     const int R = 1 << log2r;
@@ -797,7 +798,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
     if (sum_bias && tid < rn) {
         float sum = bias_part[0][tid];
 #pragma unroll
-        for (int v = 1; v < NT_W / 64; ++v) sum += bias_part[v][tid];
+        for (int v = 1; v < (BIAS ? NT_W / 64 : 1); ++v) sum += bias_part[v][tid];
         bias_out[m0 + tid] = sum;
     }
     store_slab<LAYOUT, NT_W>(hist, w_grad, tid, m0, k0, rn, kn, kc, log2r, K, M, vec_out, false);
@@ -818,9 +819,12 @@ static int setup_device(int dev)
     const void *kernels[] = {
         (const void *)mam_bwd_x_rows_kernel<MAM_W_MK>, (const void *)mam_bwd_x_rows_kernel<MAM_W_KM>,
         (const void *)mam_bwd_x_kernel<MAM_W_MK>,      (const void *)mam_bwd_x_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_w_kernel<MAM_W_MK>,      (const void *)mam_bwd_w_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK>,  (const void *)mam_bwd_w_vec_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_both_kernel<MAM_W_MK>,   (const void *)mam_bwd_w_count_kernel,
+        (const void *)mam_bwd_w_kernel<MAM_W_MK, false>,      (const void *)mam_bwd_w_kernel<MAM_W_KM, false>,
+        (const void *)mam_bwd_w_kernel<MAM_W_MK, true>,       (const void *)mam_bwd_w_kernel<MAM_W_KM, true>,
+        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false>,  (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, false>,
+        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true>,   (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, true>,
+        (const void *)mam_bwd_both_kernel<MAM_W_MK, false>,   (const void *)mam_bwd_both_kernel<MAM_W_MK, true>,
+        (const void *)mam_bwd_w_count_kernel,
     };
     bool all = true;
     for (const void *k : kernels)
@@ -918,7 +922,9 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
             int tpw = (int)(mtiles * ktiles / (2 * cus));
             if (tpw < 1) tpw = 1;
             if (tpw > 8) tpw = 8;
-            // shares of the batch per slab: two rounds of as many workgroups as fit the chip (LDS, threads)
+            // shares of the batch per slab: two rounds of as many workgroups as fit the chip by the slab's LDS and their threads
+            // (registers leave room for two per CU, so the bias gradient's 1 KiB beside the slab changes nothing: 16384 x 620 / 640 /
+            // 656 -> 1024, three or four by LDS, 176 / 176 / 180 us)
             int64_t shares = 1;
             if (large_batch) {
                 int64_t per_cu = (160 * 1024) / ((int64_t)R * kc * 4);
@@ -937,7 +943,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
                 if (rc != MAM_OK) return rc;
             }
             float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
-            hipLaunchKernelGGL((mam_bwd_w_vec_kernel<LAYOUT>),
+            hipLaunchKernelGGL((bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true> : mam_bwd_w_vec_kernel<LAYOUT, false>),
                                dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT_W),
                                (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
                                w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
@@ -950,7 +956,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
                 }
             }
         } else {
-            hipLaunchKernelGGL((mam_bwd_w_kernel<LAYOUT>), dim3((unsigned)mtiles, (unsigned)ktiles),
+            hipLaunchKernelGGL((bias ? mam_bwd_w_kernel<LAYOUT, true> : mam_bwd_w_kernel<LAYOUT, false>), dim3((unsigned)mtiles, (unsigned)ktiles),
                                dim3(NT_W), (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax,
                                argmin, x_sel, N * M, w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, planes,
                                range_len, bias ? bias->out : nullptr);
@@ -1004,7 +1010,7 @@ static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw,
     p.log2r = log2r; p.kc_w = (int)kc_w; p.vec_out = (K % 4 == 0) && ((uintptr_t)w_grad % 16 == 0);
     p.mtiles = (int)mtiles; p.tiles_per_wg = tpw; p.x_wgs = (int)N;
     const size_t lds = (size_t)(K * 8 > R * kc_w * 4 ? K * 8 : R * kc_w * 4);
-    hipLaunchKernelGGL((mam_bwd_both_kernel<MAM_W_MK>), dim3((unsigned)(N + w_wgs)), dim3(NT_X), lds, st, p);
+    hipLaunchKernelGGL((bias ? mam_bwd_both_kernel<MAM_W_MK, true> : mam_bwd_both_kernel<MAM_W_MK, false>), dim3((unsigned)(N + w_wgs)), dim3(NT_X), lds, st, p);
     return check_launch("mam_bwd_both_kernel");
 }
 
