@@ -374,11 +374,24 @@ def test_bias_gradient_through_the_module():
 
 
 @pytest.mark.parametrize("N,K,M", [(1, 40, 4), (64, 784, 256), (65, 784, 260), (50, 33, 7), (250, 1001, 517), (300, 5000, 68),
-                                   (2048, 768, 96), (2600, 3072, 40), (5000, 96, 132), (2100, 64, 33), (3000, 9000, 12)])
+                                   (2048, 768, 96), (2600, 3072, 40), (5000, 96, 132), (2100, 64, 33), (3000, 9000, 12),
+                                   (8, 100, 8192), (64, 4096, 8192), (8192, 96, 1024)])
 @pytest.mark.parametrize("splits", [1, 3])
-def test_bias_gradient_from_the_launch_that_forms_the_weight_gradient(N, K, M, splits):
+@pytest.mark.parametrize("exact", [False, True])
+def test_bias_gradient_from_the_launch_that_forms_the_weight_gradient(N, K, M, splits, exact):
     """Every route of the weight gradient (one launch for both gradients, quads, single neurons, several k chunks, shares of a
-    large batch): the column sums within the rounding of an fp32 sum, the same bits on every call."""
+    large batch, several slabs per workgroup in either launch, shares beside the x gradient on a stream of its own), and exact sums, which
+    leave the bias to its own kernel: the column sums within the rounding of an fp32 sum, the same bits on every call."""
+    from mamtorch_amd import capi
+
+    capi.set_option(capi.OPT_BACKWARD_EXACT, int(exact))
+    try:
+        _bias_gradient(N, K, M, splits)
+    finally:
+        capi.set_option(capi.OPT_BACKWARD_EXACT, 0)
+
+
+def _bias_gradient(N, K, M, splits):
     layer = mt.nn.FullyConnected(K, M, bias=True, splits=splits).to(DEV).train()
     gen = torch.Generator().manual_seed(N + M)
     x = torch.randn(N, K, generator=gen).to(DEV).requires_grad_(True)

@@ -271,14 +271,14 @@ def test_operator_at_high_density(layout, n, l, m, rate):
     assert bool(((res.double() - want).abs() <= 1e-5 * want.abs() + 2.0 ** -22 * floor).all())
 
 
-@pytest.mark.parametrize("layout", [torch.sparse_csr, torch.sparse_coo])
+@pytest.mark.parametrize("operand,one_in", [("csr", 8), ("coo", 8), ("coo in any order", 16), ("wide coo", 16)])
 @pytest.mark.parametrize("above", [False, True])
-def test_operator_either_side_of_the_density_threshold(layout, above):
-    """The operator changes route at one stored entry in eight (CSR; one in sixteen for COO): sparse kernel below,
-    dense copy + library GEMM from there on, and with it the order of summation: one entry below and exactly at
-    the threshold, both against the fp64 defining sum within rtol 1e-5 plus the rounding floor of an fp32 sum."""
-    R, K, C = 96, 256, 128
-    nnz = R * K // (8 if layout == torch.sparse_csr else 16) + (0 if above else -1)
+def test_operator_either_side_of_the_density_threshold(operand, one_in, above):
+    """The operator changes route at one stored entry in eight (CSR, and coalesced COO up to K = 32768; other COO operands at
+    one in sixteen): sparse kernel below, dense copy + library GEMM from there on, and with it the order of summation: one entry
+    below and exactly at the threshold, both against the fp64 defining sum within rtol 1e-5 plus the rounding floor of an fp32 sum."""
+    R, K, C = (2, 32784, 64) if operand == "wide coo" else (96, 256, 128)
+    nnz = R * K // one_in + (0 if above else -1)
     g = torch.Generator().manual_seed(17 + int(above))
     where = torch.randperm(R * K, generator=g)[:nnz]
     a = torch.zeros(R * K)
@@ -286,10 +286,68 @@ def test_operator_either_side_of_the_density_threshold(layout, above):
     a = a.view(R, K).to(DEV)
     assert int((a != 0).sum()) == nnz
     b = torch.randn(K, C, generator=g).to(DEV)
-    res = torch.ops.mamtorch_kernel_sparsev1.cusparsemm(a.to_sparse(layout=layout), b)
+    if operand == "coo in any order":
+        coo = a.to_sparse()
+        order = torch.randperm(nnz, generator=g).to(DEV)
+        sparse = torch.sparse_coo_tensor(coo.indices()[:, order], coo.values()[order], a.shape)
+    else:
+        sparse = a.to_sparse(layout=torch.sparse_csr if operand == "csr" else torch.sparse_coo)
+    assert operand == "csr" or sparse.is_coalesced() == (operand != "coo in any order")
+    res = torch.ops.mamtorch_kernel_sparsev1.cusparsemm(sparse, b)
     want = a.double() @ b.double()
     floor = a.abs().double() @ b.abs().double()
     assert bool(((res.double() - want).abs() <= 1e-5 * want.abs() + 2.0 ** -22 * floor).all())
+
+
+@pytest.mark.parametrize("rows,k,cols,nnz", [(50, 60, 64, 150), (50, 60, 70, 186), (50, 60, 70, 188), (300, 32768, 130, 9000),
+                                             (300, 32769, 130, 9000)])
+@pytest.mark.parametrize("order", ["coalesced", "shuffled", "repeated"])
+def test_coo_operands_of_the_operator(rows, k, cols, nnz, order):
+    """Coalesced, in any order, and with coordinates that occur up to three times, below and above one entry in sixteen, and on
+    either side of the K up to which coalesced operands are summed by rows."""
+    import mamtorch_amd as mt
+
+    g = torch.Generator().manual_seed(nnz + cols)
+    where = torch.randperm(rows * k, generator=g)[:nnz].sort()[0]
+    val = torch.randn(nnz, generator=g)
+    if order != "coalesced":
+        shuffle = torch.randperm(nnz, generator=g)
+        where, val = where[shuffle], val[shuffle]
+    if order == "repeated":
+        where = torch.cat([where[: nnz // 3], where[: nnz // 3], where[: nnz - 2 * (nnz // 3)]])
+    row, col, b = where // k, where % k, torch.randn(k, cols, generator=g)
+    want, floor = oracle.coo_spmm(row.numpy(), col.numpy(), val.numpy(), b.numpy(), rows)
+    a = torch.sparse_coo_tensor(torch.stack([row, col]), val, (rows, k))
+    a = a.coalesce() if order == "coalesced" else a
+    _check(mt.sparse.kernel.v1.cusparsemm(a.to(DEV), b.to(DEV)), want, floor, order)
+
+
+@pytest.mark.parametrize("cols,ldb", [(8, 2 ** 27 + 4), (300, 2 ** 27 + 4), (7, 2 ** 27 + 4), (129, 2 ** 27 + 4), (64, 2 ** 27 + 3)])
+def test_b_of_more_than_4_gib(cols, ldb):
+    """b rows whose byte offsets do not fit 32 bits: four columns a lane where everything is aligned, else one; 9 rows of b in
+    4.8 GB, all three entry points."""
+    from mamtorch_amd import capi
+
+    rows, k = 37, 9
+    g = torch.Generator().manual_seed(cols)
+    a = _random_sparse(rows, k, 0.4, seed=cols)
+    b = torch.randn(k, cols, generator=g)
+    wide = torch.empty((k - 1) * ldb + cols, device=DEV)
+    bd = wide.as_strided((k, cols), (ldb, 1))
+    bd.copy_(b)
+    csr, coo = a.to_sparse_csr(), a.to_sparse_coo().coalesce()
+    crow, col, val = (t.to(DEV) for t in (csr.crow_indices(), csr.col_indices(), csr.values()))
+    want, floor = oracle.csr_spmm(csr.crow_indices().numpy(), csr.col_indices().numpy(), csr.values().numpy(), b.numpy())
+    row = coo.indices()[0].contiguous().to(DEV)
+    _check(capi.csr_spmm(crow, col, val, bd, rows), want, floor, "csr")
+    _check(capi.coo_spmm(row, col, val, bd, rows), want, floor, "coo")
+    c, by_rows = capi.coo_spmm_by_rows(row, col, val, bd, rows)
+    assert by_rows
+    _check(c, want, floor, "by rows")
+    back = torch.arange(val.numel() - 1, -1, -1, device=DEV)
+    c, by_rows = capi.coo_spmm_by_rows(row[back], col[back], val[back], bd, rows)
+    assert not by_rows
+    _check(c, want, floor, "rows that fall")
 
 
 def test_to_dense_skips_coordinates_outside_the_matrix():
