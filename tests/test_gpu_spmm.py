@@ -75,6 +75,31 @@ def test_column_counts_around_the_panels(cols):
         _check(capi.coo_spmm(idx[0].contiguous(), idx[1].contiguous(), values, bd, rows), want, floor, "coo, offset %d" % offset)
 
 
+@pytest.mark.parametrize("cols", [129, 130, 131, 257, 385, 386, 5121, 5122, 5123])
+def test_last_columns_are_read_inside_b(cols):
+    """Four columns a lane where their number is no multiple of four, a last panel of one to three columns among them: lanes at the
+    end take the last four columns, each written by one lane, and no load leaves its row, which for the last row is the end of b."""
+    from mamtorch_amd import capi
+
+    rows, k = 21, 40
+    g = torch.Generator().manual_seed(cols)
+    a = _random_sparse(rows, k, 0.3, seed=cols)
+    a[:, k - 1] = 1.0
+    store = torch.full((k * cols + 4,), float("nan"))
+    store[: k * cols] = torch.randn(k * cols, generator=g)
+    b = store[: k * cols].view(k, cols)
+    bd = store.to(DEV)[: k * cols].view(k, cols)
+    csr, coo = a.to_sparse_csr(), a.to_sparse_coo().coalesce()
+    crow, col, val = (t.to(DEV) for t in (csr.crow_indices(), csr.col_indices(), csr.values()))
+    row = coo.indices()[0].contiguous().to(DEV)
+    want, floor = oracle.csr_spmm(csr.crow_indices().numpy(), csr.col_indices().numpy(), csr.values().numpy(), b.numpy())
+    _check(capi.csr_spmm(crow, col, val, bd, rows), want, floor, "csr")
+    _check(capi.coo_spmm(row, col, val, bd, rows), want, floor, "coo")
+    c, by_rows = capi.coo_spmm_by_rows(row, col, val, bd, rows)
+    assert by_rows
+    _check(c, want, floor, "by rows")
+
+
 @pytest.mark.parametrize("k,cols", [(32768, 2000), (32769, 2000), (70000, 600), (90000, 600), (300000, 64)])
 def test_panels_by_xcd_and_in_turn(k, cols):
     """Workgroups are numbered panel by panel up to 2^18 rows of b in the (at most eight) panels, and have a grid row per panel
