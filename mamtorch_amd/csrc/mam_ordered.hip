@@ -28,7 +28,7 @@
 // Measured against the dense tilings (forward call, hand-over arrays written).  Uniform weights or inputs, one-sided:
 // 207 -> 60 to 67 us at 256 x 4096 x 4096, 1.70 -> 0.49 ms and 1.48 -> 0.24 ms for 12608 x 768 -> 3072 -> 768, 10.2 -> 0.72 ms
 // (values only) and 3.13 -> 0.36 ms at 16384 x 4096 -> 4096 / 1024.  Normal weights and inputs, two-sided: 1.70 -> 1.36 ms
-// at 12608 x 768 -> 3072, 3.12 -> 0.92 ms at 16384 x 4096 -> 1024, 0.84 -> 0.43 ms at 4096 x 2048 x 2048.
+// at 12608 x 768 -> 3072, 3.12 -> 0.92 ms at 16384 x 4096 -> 1024, 0.84 -> 0.40 ms at 4096 x 2048 x 2048.
 #include "mam_ordered.h"
 
 #include <math.h>
@@ -42,14 +42,15 @@ constexpr int BUILD_NT = 256;         // threads of the build, per listed row
 constexpr int BUILD_MAX_K = 40 * BUILD_NT;
 constexpr int NT = 1024;              // threads of the forward
 constexpr int MAX_TILE_BYTES = 152 * 1024;
-// N * K * M from which two-sided searches are considered.  They cost two launches and a longer sampling, 9 us, where they are not
-// taken (256 x 4096 -> 4096, uniform weights, 2^32 products: 67 us without, 76 us with them; normal weights 224 and 147 us, dense
-// 207 us): up to 2^33 products 2 to 13 % of the call.
+// N * K * M from which two-sided searches are considered.  They cost two launches and a longer sampling, 7 to 13 us, where they are not
+// taken (256 x 4096 -> 4096, uniform weights, 2^32 products: 60 us without, 67 us with them; 64 x 4096 -> 16384, normal weights, by the
+// dense tilings: 242 and 255 us): up to 2^33 products 3 to 11 % of the call.  Where they are taken they win earlier (256 x 4096 -> 4096,
+// normal weights: 225 us without, 126 us with them; 1024 x 2048 x 2048: 235 and 122).
 constexpr int64_t MIN_TWO_SIDED = 1ll << 33;
 constexpr int LEAD_CAP = 96;          // leading entries kept per tile row (LDS)
 // N * K * M from which a call takes the lists.  Uniform on one side, they win from 2^30 products on (lists / dense, with indices:
-// 128 x 2048 -> 4096 50 / 65 us, 128 x 4096 -> 4096 68 / 109), but only the device finds out what the data is, and a call that it
-// hands to the dense tilings has paid for sampling and idle launches: 13 to 20 us, 6 to 9 % of the 165 to 210 us that 2^32
+// 128 x 2048 -> 4096 46 / 68 us, 128 x 4096 -> 4096 62 / 116), but only the device finds out what the data is, and a call that it
+// hands to the dense tilings has paid for sampling and idle launches: 8 to 11 us, 4 to 5 % of the 214 to 240 us that 2^32
 // products take there, twice that share at 2^31.
 constexpr int64_t MIN_PRODUCTS = 1ll << 32;
 constexpr uint32_t INF_BITS = 0x7f800000u;
@@ -64,9 +65,10 @@ constexpr int OPTIONS = 2 * LEADS;
 // Microseconds of the dense kernels and of the lists of a call, from its sizes alone; launches that come either way are
 // left out.  What a search costs per product is not all: its workgroups load their tiles (14.5 us for 128 KiB), a round of 16 blocks
 // of rows costs 4 to 6 us beside its products, a round of fewer waves hardly less, and the lists themselves 2 to 10 ns a row.
-// Calls of few rows on either side lose there what the search saves (normal x normal, lists / dense: 64 x 4096 -> 16384 416 / 241 us,
-// 65536 x 1024 -> 64 896 / 317, 40 x 8000 -> 16384 2014 / 444; 256 x 4096 -> 4096 148 / 217).  Constants fitted to 180 timed
-// calls (K 256 .. 8000, N and M 40 .. 65536), most of which they give within 20 %.
+// Calls of few rows on either side lose there what the search saves (normal x normal, lists / dense: 64 x 4096 -> 16384 357 / 234 us,
+// 65536 x 1024 -> 64 822 / 339, 40 x 8000 -> 16384 1499 / 464; 256 x 4096 -> 4096 126 / 214).  Constants fitted to 180 timed
+// calls (K 256 .. 8000, N and M 40 .. 65536), most of which they gave within 20 %; the search has become 10 to 25 % faster since, so
+// that calls near the border stay with the dense kernels a little longer than they need to.
 struct Times {
     struct Side { float fixed, per_entry, rounds, round; };      // of a search of this operand's rows
     float dense, product, led;
@@ -1512,7 +1514,7 @@ static Times::Side side_times(int64_t listed, int64_t tiled, int64_t K, bool arg
     const float alone = two_sided ? 0.45f : 0.3f;                // of a full round's time, by a single wave
     const float rounds = (float)(per_split / waves) + (last ? alone + (1.0f - alone) * (float)last / (float)waves : 0.0f);
     const float lds = (float)K * (float)tb * 4.0f + (two_sided ? (float)(LEAD_CAP * TWO_SIDED_ROWS * 8) : 0.0f);
-    const float load = 4.4e-4f * (float)K * (float)tb * (lds <= 80.0f * 1024.0f ? 0.5f : 1.0f);     // two workgroups share a CU where their tiles fit
+    const float load = 4.4e-4f * (float)K * (float)tb * (lds <= 80.0f * 1024.0f ? 0.5f : 1.0f);     // (the fit's: a CU holds one workgroup, by registers, whatever its tile)
     float workgroups = (float)tiles * (float)splits / (float)cus;
     workgroups = workgroups < 4.0f ? ceilf(workgroups) : workgroups + 0.3f;
     const float row = 1e-3f + (K > 16 * BUILD_NT ? 1.4e-6f : 0.95e-6f) * (float)K;
