@@ -18,6 +18,7 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/library.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "../../include/mam_hip.h"
@@ -583,6 +584,17 @@ at::Tensor cusparsemm_csr(const at::Tensor &a, const at::Tensor &b)
     return c;
 }
 
+// Whether the sum by rows pays for a coalesced COO operand (nanoseconds).  It takes a wave per row, however empty (0.13), 0.08 more where the row
+// has entries; the COO kernel clears c (0.0007 a value), adds a run of entries to it (0.007 a value) and takes 0.038 longer per entry and
+// 10 us longer in all.  By rows / by entries, us: 2^20 rows of 0.05 / 0.5 / 2 / 8 entries x 1 column 147 / 18, 189 / 42, 230 / 125, 299 / 409, x 16
+// 149 / 36, 194 / 111, 232 / 213, 303 / 426, x 64 151 / 88, 196 / 396, 235 / 817, 305 / 1026; 2^23 rows of 0.05 x 1 1121 / 48; 4096 rows of 0.05 to 60
+// x 1 to 4096 columns 9 to 142 / 12 to 421, 65536 rows of 2 x 1 17.5 / 16.3, x 4 17.8 / 22.4.
+bool rows_pay(int64_t nnz, int64_t R, int64_t C)
+{
+    const double rows = (double)R, filled = (double)std::min(nnz, R);
+    return 0.13 * rows < 10000.0 + 0.0007 * rows * (double)C + filled * (0.007 * (double)C - 0.08) + 0.038 * (double)nnz;
+}
+
 at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
 {
     TORCH_CHECK(a.layout() == at::kSparse, "a must be a torch.sparse_coo tensor");
@@ -595,9 +607,9 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     const int64_t nnz = val.numel();
     // A coalesced operand's rows ascend (the device looks whether they do: the flag can be set without it): with row offsets it is a
     // CSR operand, whose kernel adds a row up in registers instead of clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns:
-    // 364 -> 116 us).  A row is one wave's there, so the device looks for crowded ones too.  Up to the K that both were timed at
+    // 364 -> 116 us), where that pays.  A row is one wave's there, so the device looks for crowded ones too.  Up to the K that both were timed at
     // (4096 x 32768 with 33 entries a row x 4096 columns: 477 -> 290 us), and no more rows than a launch holds waves.
-    const bool by_rows = a.is_coalesced() && K <= 32768 && R <= (int64_t(1) << 24);
+    const bool by_rows = a.is_coalesced() && K <= 32768 && R <= (int64_t(1) << 24) && rows_pay(nnz, R, C);
     if (dense_route_pays(nnz, R, K, C, by_rows ? 8 : 16)) {
         auto dense = at::empty({R, K}, b.options());
         check_rc(mam_coo_to_dense(idx.data_ptr<int64_t>(), idx.data_ptr<int64_t>() + nnz, val.data_ptr<float>(), nnz,

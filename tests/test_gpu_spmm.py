@@ -134,7 +134,8 @@ def test_long_rows_are_added_up_in_short_sums(n, cols, layout):
     assert bool(((got - want).abs() <= (64 + n / 64 + 4) * 2.0 ** -24 * want).all())
 
 
-@pytest.mark.parametrize("nnz,rows", [(0, 5), (1, 1), (63, 9), (64, 300), (65, 3), (4096, 70), (4097, 1), (300000, 4001)])
+@pytest.mark.parametrize("nnz,rows", [(0, 5), (1, 1), (63, 9), (64, 300), (65, 3), (4096, 70), (4097, 1), (300000, 4001), (0, 256), (70, 255),
+                                      (70, 256), (1000, 300000), (2000000, 100003)])
 def test_row_offsets(nnz, rows):
     from mamtorch_amd import capi
 
@@ -195,6 +196,25 @@ def test_crowded_rows_are_not_one_wave_s(rows, k, cols, each, at, more):
     c, by_rows = capi.coo_spmm_by_rows(row.to(DEV), col.to(DEV), val.to(DEV), b.to(DEV), rows)
     assert by_rows == (not more)
     _check(c, want, floor, "crowded" if more else "not crowded")
+
+
+@pytest.mark.parametrize("cols", [1, 4, 16, 64, 260])
+@pytest.mark.parametrize("nnz", [0, 700, 130000, 1300000])
+@pytest.mark.parametrize("rows", [65536, 262147])
+def test_operands_of_many_rows(rows, nnz, cols):
+    """Coalesced COO operands of many rows, most of them empty or not: by rows or by entries, as the operator chooses (both
+    within these), and the CSR operator."""
+    import mamtorch_amd as mt
+
+    k = 60
+    g = torch.Generator().manual_seed(nnz + cols)
+    row, col = torch.randint(0, rows, (nnz,), generator=g), torch.randint(0, k, (nnz,), generator=g)
+    a = torch.sparse_coo_tensor(torch.stack([row, col]), torch.randn(nnz, generator=g), (rows, k)).coalesce()
+    b = torch.randn(k, cols, generator=g)
+    idx, val = a.indices(), a.values()
+    want, floor = oracle.coo_spmm(idx[0].numpy(), idx[1].numpy(), val.numpy(), b.numpy(), rows)
+    _check(mt.sparse.kernel.v1.cusparsemm(a.to(DEV), b.to(DEV)), want, floor, "coo")
+    _check(mt.sparse.kernel.v1.cusparsemm(a.to(DEV).to_sparse_csr(), b.to(DEV)), want, floor, "csr")
 
 
 def test_coo_unsorted_with_duplicates_and_strided_b():
