@@ -59,18 +59,20 @@ __device__ __forceinline__ void axpy(float (&acc)[4], float v, const float4 &b)
 // panels of eight XCDs are too much for the memory-side cache together (us by XCDs and in turn, 4096 columns: K = 4096 107 / 126, 16384 293 /
 // 310, 32768 346 / 346, 65536 354 / 346; 1024 columns, four panels: 65536 91.6 / 93.2).
 struct Place { int panel, block; };
-__device__ __forceinline__ Place place_of(int blocks)
+// (`panels` by XCD, 0: a row of the grid each.  An argument and no division for one panel: the grid's size would be one more wait, and
+// 2^20 rows x 1 column with 0.05 entries each take 171 us with both, 134 without the division, 130 without either; 103 where empty rows are done with at once.)
+__device__ __forceinline__ Place place_of(int blocks, int panels)
 {
-    if (gridDim.y > 1) return {(int)blockIdx.y, (int)blockIdx.x};
-    const int logical = xcd_remap(blockIdx.x, gridDim.x);
-    if ((int)gridDim.x == blocks) return {0, logical};       // (without the division: 2^20 rows of no entries 171 -> 125 us)
+    if (panels == 0) return {(int)blockIdx.y, (int)blockIdx.x};
+    const int logical = xcd_remap(blockIdx.x, panels * blocks);
+    if (panels == 1) return {0, logical};
     return {logical / blocks, logical % blocks};
 }
 constexpr int64_t MOST_PANEL_ROWS = 8 * 32768;           // of b, in the panels that are walked at once
-static dim3 grid_of(int64_t panels, int64_t blocks, int64_t K)
+static bool by_xcd(int64_t panels, int64_t blocks, int64_t K)
 {
     // less than 2^32 threads in a dimension
-    return K * (panels < 8 ? panels : 8) <= MOST_PANEL_ROWS && panels * blocks < UINT32_MAX / NT ? dim3((unsigned)(panels * blocks)) : dim3((unsigned)blocks, (unsigned)panels);
+    return K * (panels < 8 ? panels : 8) <= MOST_PANEL_ROWS && panels * blocks < UINT32_MAX / NT;
 }
 
 // four consecutive words, 4-byte aligned; past the L2 whether or not rows of c start lines (past it / to it, us: 4096 x 4096 with 8
@@ -105,13 +107,13 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
                                                       const int64_t *__restrict__ col,
                                                       const float *__restrict__ val,
                                                       const float *__restrict__ b, int64_t ldb, uint32_t b_bytes,
-                                                      float *__restrict__ c, int R, int C, int row_blocks, int width,
+                                                      float *__restrict__ c, int R, int C, int row_blocks, int panels, int width,
                                                       const uint32_t *__restrict__ verdicts)
 {
     typedef typename Vec<TI>::type vec;
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const Place at_block = place_of(row_blocks);
+    const Place at_block = place_of(row_blocks, panels);
     // (uniform, but the division leaves them in vector registers: 97 of 96 with two entries per load)
     const int panel = __builtin_amdgcn_readfirstlane(at_block.panel), r = __builtin_amdgcn_readfirstlane(at_block.block) * (NT / 64) + wave;
     if (r >= R) return;
@@ -128,6 +130,23 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     const_f32 *cval = (const_f32 *)val;
     const int64_t beg = ((const_i64 *)crow)[r], end = ((const_i64 *)crow)[r + 1];
     const int nnz = verdicts && not_by_rows(verdicts) ? 0 : (int)(end - beg);
+    float acc[TI];
+#pragma unroll
+    for (int t = 0; t < TI; ++t) acc[t] = 0.0f;
+    auto put = [&] {
+        if (part != 0 || !in) return;
+        const int first = PER == 1 ? cl : c0;
+        float *dst = c + (int64_t)r * C + first;
+        if (TI == 4 && c0 + 3 < C) {
+            store4(dst, acc);
+        } else {            // (those below c0 are other lanes')
+#pragma unroll
+            for (int t = 0; t < TI; ++t)
+                if (first + t >= c0 && first + t < C) dst[t] = acc[t];
+        }
+    };
+    if (PER > 1 && nnz == 0) return put();
+
     const float *bl = b + cl;
     const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
     const uint32_t row_bytes = (uint32_t)ldb * 4u;
@@ -158,10 +177,6 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
         }
         return v;
     };
-
-    float acc[TI];
-#pragma unroll
-    for (int t = 0; t < TI; ++t) acc[t] = 0.0f;
 
     const int ng = nnz / (EG * PER);
     vec xa[EG], xb[EG];
@@ -228,22 +243,11 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     }
 #pragma unroll
     for (int t = 0; t < TI; ++t) acc[t] += total[t];
-    if (PER > 1 && nnz > 0) {
 #pragma unroll
-        for (int s = LANES; s < 64; s <<= 1)
+    for (int s = LANES; s < 64; s <<= 1)
 #pragma unroll
-            for (int t = 0; t < TI; ++t) acc[t] += __shfl_xor(acc[t], s);
-    }
-    if (part != 0 || !in) return;
-    const int first = PER == 1 ? cl : c0;
-    float *dst = c + (int64_t)r * C + first;
-    if (TI == 4 && c0 + 3 < C) {
-        store4(dst, acc);
-    } else {            // (those below c0 are other lanes')
-#pragma unroll
-        for (int t = 0; t < TI; ++t)
-            if (first + t >= c0 && first + t < C) dst[t] = acc[t];
-    }
+        for (int t = 0; t < TI; ++t) acc[t] += __shfl_xor(acc[t], s);
+    put();
 }
 
 template <int TI>
@@ -441,9 +445,11 @@ static int launch_csr(const int64_t *crow, const int64_t *col, const float *val,
     const int width = (int)(ceil_div(ceil_div(C, panels), 32) * 32);
     const int64_t row_blocks = ceil_div(R, NT / 64);
     if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
+    const bool linear = by_xcd(panels, row_blocks, K);
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid_of(panels, row_blocks, K), dim3(NT), 0, st, crow, col, val, b, ldb, (uint32_t)b_bytes, c,
-                           (int)R, (int)C, (int)row_blocks, width, verdicts);
+        const dim3 grid = linear ? dim3((unsigned)(panels * row_blocks)) : dim3((unsigned)row_blocks, (unsigned)panels);
+        hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, st, crow, col, val, b, ldb, (uint32_t)b_bytes, c, (int)R, (int)C, (int)row_blocks,
+                           linear ? (int)panels : 0, width, verdicts);
     };
     if (per == 4) launch(csr_spmm_kernel<4, true, 4>);
     else if (per == 2) launch(csr_spmm_kernel<4, true, 2>);

@@ -586,9 +586,9 @@ at::Tensor cusparsemm_csr(const at::Tensor &a, const at::Tensor &b)
 
 // Whether the sum by rows pays for a coalesced COO operand (nanoseconds).  It takes a wave per row, however empty (0.13), 0.08 more where the row
 // has entries; the COO kernel clears c (0.0007 a value), adds a run of entries to it (0.007 a value) and takes 0.038 longer per entry and
-// 10 us longer in all.  By rows / by entries, us: 2^20 rows of 0.05 / 0.5 / 2 / 8 entries x 1 column 147 / 18, 189 / 42, 230 / 125, 299 / 409, x 16
-// 149 / 36, 194 / 111, 232 / 213, 303 / 426, x 64 151 / 88, 196 / 396, 235 / 817, 305 / 1026; 2^23 rows of 0.05 x 1 1121 / 48; 4096 rows of 0.05 to 60
-// x 1 to 4096 columns 9 to 142 / 12 to 421, 65536 rows of 2 x 1 17.5 / 16.3, x 4 17.8 / 22.4.
+// 10 us longer in all.  By rows / by entries, us: 2^20 rows of 0.05 / 0.5 / 2 / 8 entries x 1 column 126 / 18, 156 / 43, 208 / 125, 267 / 408, x 16
+// 119 / 36, 165 / 111, 214 / 213, 273 / 424, x 64 119 / 88, 167 / 398, 217 / 818, 278 / 1029; 2^23 rows of 0.05 x 1 952 / 47; 200000 rows of 1 x 1 35 / 24,
+// of 2 x 16 40 / 54; 65536 rows of 2 x 1 17.6 / 16.7, x 4 17.5 / 21.8; 4096 rows of 0.05 to 60 x 1 to 4096 columns 9 to 142 / 12 to 421.
 bool rows_pay(int64_t nnz, int64_t R, int64_t C)
 {
     const double rows = (double)R, filled = (double)std::min(nnz, R);
