@@ -21,7 +21,9 @@
 //   COO: entries may come in any order and may repeat, so c is cleared first; a wave takes 64
 //        consecutive entries, keeps a run of equal row indices in registers and flushes it with
 //        atomic adds when the row changes.  On row-sorted input (what Tensor.to_sparse() and
-//        coalesce() produce) that is about one flush per row and wave.
+//        coalesce() produce) that is about one flush per row and wave.  A lane's columns are 64 apart: adds of 64
+//        neighbouring words (four neighbouring columns a lane, as in the CSR kernel, us: 236641 entries in any order x 2252
+//        columns 7180, like this 1970; 24684 x 6871 2840 and 800; 222063 ascending x 704 613 and 178).
 // Products are fused multiply-adds in ascending entry order within a wave (narrow c: within each of the two or four
 // parts of a row), 64 of them at a time; sums that span waves (COO only) are combined in no fixed order.
 #include "mam_common.h"
@@ -250,22 +252,21 @@ __global__ __launch_bounds__(NT) void csr_spmm_kernel(const int64_t *__restrict_
     put();
 }
 
+// A lane's TI columns are 64 apart, so that the adds of a wave, and its loads of b, are of 64 neighbouring words.
 template <int TI>
-__device__ __forceinline__ void flush_row(float *__restrict__ c, int64_t row, int C, int c0, bool live,
-                                          float (&acc)[TI])
+__device__ __forceinline__ void flush_row(float *__restrict__ c, int64_t row, int C, int c0, float (&acc)[TI])
 {
-    if (live) {
-        float *dst = c + row * C + c0;
+    float *dst = c + row * C + c0;
 #pragma unroll
-        for (int t = 0; t < TI; ++t) {
-            if (c0 + t < C) unsafeAtomicAdd(dst + t, acc[t]);
-            acc[t] = 0.0f;
-        }
+    for (int t = 0; t < TI; ++t) {
+        if (c0 + 64 * t < C) unsafeAtomicAdd(dst + 64 * t, acc[t]);
+        acc[t] = 0.0f;
     }
 }
 
-// Panels go to the XCDs as in csr_spmm_kernel, and b rows are read as there with PER > 1.  With verdicts it runs only where they forbid the sum
+// Panels go to the XCDs as in csr_spmm_kernel.  With verdicts it runs only where they forbid the sum
 // by rows, and then in no more workgroups than the chip holds: one per block of entries and panel cost 4 us to find nothing to do.
+// NEAR: b spans less than 4 GiB; no lane reads past its row either way (those past the last column read that).
 constexpr int FALLBACK_WORKGROUPS = 8 * kNumCU;
 template <int TI, bool NEAR>
 __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict__ row,
@@ -275,26 +276,29 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
                                                       float *__restrict__ c, int C, int chunk_blocks, int64_t total,
                                                       const uint32_t *__restrict__ verdicts)
 {
-    typedef typename Vec<TI>::type vec;
     constexpr int EG = loads_of(1);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (verdicts && !not_by_rows(verdicts)) return;
-    for (int64_t at = xcd_remap(blockIdx.x, gridDim.x); at < total; at += gridDim.x) {
+    // fewer workgroups than blocks (a multiple of the XCDs): an XCD's share in turn, so that it works on panels of its own then too (4096 x
+    // 4096 at 1 % with a full row x 4096 columns: 335 -> 240 us)
+    const bool turns = total > gridDim.x;
+    const int xcd = blockIdx.x % kNumXCD;
+    const int64_t end = turns ? total * (xcd + 1) / kNumXCD : total, step = turns ? gridDim.x / kNumXCD : total;
+    for (int64_t at = turns ? total * xcd / kNumXCD + blockIdx.x / kNumXCD : xcd_remap(blockIdx.x, gridDim.x); at < end; at += step) {
         const int panel = (int)(at / chunk_blocks);
         const int64_t e0 = ((at - (int64_t)panel * chunk_blocks) * (NT / 64) + wave) * COO_CHUNK;
         if (e0 >= nnz) continue;
         const int n = (int)((nnz - e0) < COO_CHUNK ? (nnz - e0) : COO_CHUNK);
-        const int c0 = panel * 64 * TI + lane * TI;
-        const bool live = c0 < C;
-        const int cl = live ? c0 : 0;
-        const float *bl = b + cl;
+        const int c0 = panel * 64 * TI + lane;
+        uint32_t word[TI];
+#pragma unroll
+        for (int t = 0; t < TI; ++t) word[t] = c0 + 64 * t < C ? c0 + 64 * t : C - 1;
         const __amdgpu_buffer_rsrc_t near = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(b), 0, (int)b_bytes, 0x00020000);
         const uint32_t row_bytes = (uint32_t)ldb * 4u;
-        auto b_row = [&](int64_t k) -> vec {
-            // (the whole offset in the vector register: the range check need not count a scalar one, and zeros stand past the end of b)
-            if constexpr (NEAR) return __builtin_bit_cast(vec, __builtin_amdgcn_raw_buffer_load_b128(near, (uint32_t)k * row_bytes + cl * 4, 0, 0));
-            else return *reinterpret_cast<const vec *>(bl + k * ldb);
+        auto b_word = [&](int64_t k, int t) -> float {
+            if constexpr (NEAR) return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(near, word[t] * 4, (uint32_t)k * row_bytes, 0));
+            else return (b + k * ldb)[word[t]];
         };
 
         const_i64 *crow = (const_i64 *)row;
@@ -306,27 +310,31 @@ __global__ __launch_bounds__(NT) void coo_spmm_kernel(const int64_t *__restrict_
         int64_t cur = crow[e0];
         for (int i = 0; i < n; i += EG) {
             // loads of up to EG entries first; entries past the end repeat the last one and are not added
-            vec xv[EG];
+            float xv[EG][TI];
             float wv[EG];
             int64_t rv[EG];
 #pragma unroll
             for (int u = 0; u < EG; ++u) {
                 const bool ok = i + u < n;
-                const int64_t e = e0 + (ok ? i + u : n - 1);
-                xv[u] = b_row(ccol[e]);
+                const int64_t e = e0 + (ok ? i + u : n - 1), k = ccol[e];
+#pragma unroll
+                for (int t = 0; t < TI; ++t) xv[u][t] = b_word(k, t);
                 wv[u] = cval[e];
                 rv[u] = crow[e];
             }
 #pragma unroll
             for (int u = 0; u < EG; ++u) {
                 if (rv[u] != cur) {  // wave-uniform
-                    flush_row<TI>(c, cur, C, c0, live, acc);
+                    flush_row<TI>(c, cur, C, c0, acc);
                     cur = rv[u];
                 }
-                if (i + u < n) axpy(acc, wv[u], xv[u]);
+                if (i + u < n) {
+#pragma unroll
+                    for (int t = 0; t < TI; ++t) acc[t] = __builtin_fmaf(wv[u], xv[u][t], acc[t]);
+                }
             }
         }
-        flush_row<TI>(c, cur, C, c0, live, acc);
+        flush_row<TI>(c, cur, C, c0, acc);
     }
 }
 
@@ -465,25 +473,29 @@ static int launch_coo(const int64_t *row, const int64_t *col, const float *val, 
     const int64_t gx = ceil_div(nnz, (int64_t)COO_CHUNK * (NT / 64));
     if (gx > INT32_MAX) return fail(MAM_ERR_UNSUPPORTED, "too many entries for the SpMM grid");
     const int64_t b_bytes = K > 0 ? ((K - 1) * ldb + C) * 4 : 0;
-    const bool near = b_bytes < ((int64_t)1 << 32), wide = spmm::wide(b, ldb, c, C);
-    const int64_t panels = ceil_div(C, near || wide ? 256 : 64);
+    const bool near = b_bytes < ((int64_t)1 << 32);
+    // columns per lane: fewer where waves are few, each of which adds up to 64 rows one after the other (4 / 2 / 1, us: 194 entries in any order x 4041
+    // columns, 64 waves of four, 26 / 20 / 17; 10207 ascending x 723, 480 waves, 15 / 13 / 14; 103372 ascending x 197, 1616 waves, 15 / 18 / 27)
+    const int64_t fours = gx * ceil_div(C, 256);
+    const int per_lane = C <= 64 || fours < kNumCU ? 1 : C <= 128 || fours < 4 * kNumCU ? 2 : 4;
+    const int64_t panels = ceil_div(C, 64 * per_lane);
     if (panels > 65535) return fail(MAM_ERR_UNSUPPORTED, "too many columns for the SpMM grid");
-    const int64_t total = panels * gx, most = verdicts ? FALLBACK_WORKGROUPS : UINT32_MAX / NT;      // (2^32 threads in a launch)
+    const int64_t total = panels * gx, most = verdicts ? FALLBACK_WORKGROUPS : UINT32_MAX / NT / kNumXCD * kNumXCD;      // (2^32 threads in a launch)
     auto launch = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, dim3((unsigned)(total < most ? total : most)), dim3(NT), 0, st, row, col, val, nnz, b, ldb,
                            (uint32_t)b_bytes, c, (int)C, (int)gx, total, verdicts);
     };
-    if (near) launch(coo_spmm_kernel<4, true>);
-    else if (wide) launch(coo_spmm_kernel<4, false>);
-    else launch(coo_spmm_kernel<1, false>);
+    if (per_lane == 1) near ? launch(coo_spmm_kernel<1, true>) : launch(coo_spmm_kernel<1, false>);
+    else if (per_lane == 2) near ? launch(coo_spmm_kernel<2, true>) : launch(coo_spmm_kernel<2, false>);
+    else near ? launch(coo_spmm_kernel<4, true>) : launch(coo_spmm_kernel<4, false>);
     return check_launch("coo_spmm_kernel");
 }
 
 // Entries of a COO operand's row that its wave may take one after the other, 0.05 us each (8 in 0.45 us, narrow c: 16 in 0.85), so that
-// no row alone takes longer than the COO kernel, 12 us and at least 0.28 us per 2^20 entries times columns, takes for everything.
-// (One row full, us by rows / by entries: 4096 x 4096 at 1 % x 4096 columns 296 / 382, by rows; 64 x 4096 at 1 % x 4096 235 / 25,
-// 4096 x 32768 with 8 entries in the others x 1024 1864 / 117, 300 x 1000 at 1 % x 260 34 / 14.)
-static int64_t longest_row(int64_t nnz, int64_t C) { return 256 + (int64_t)((double)nnz * (double)C / (1 << 17)); }
+// no row alone takes longer than the COO kernel, 12 us and at least 0.2 us per 2^20 entries times columns, takes for everything.
+// (One row full, us by rows / by entries after the look: 4096 x 4096 at 10 % x 1024 columns 393 / 366 and 40, by rows; at 1 % x 4096 301 / 240,
+// 64 x 4096 at 1 % x 4096 245 / 23, 4096 x 32768 with 8 entries in the others x 1024 1990 / 59, 300 x 1000 at 1 % x 260 38 / 16.)
+static int64_t longest_row(int64_t nnz, int64_t C) { return 256 + (int64_t)((double)nnz * (double)C / (1 << 18)); }
 
 static int launch_row_offsets(const int64_t *row, int64_t nnz, int64_t *crow, int64_t R, uint32_t *verdicts, int64_t longest,
                               hipStream_t st)

@@ -552,8 +552,8 @@ void check_spmm_operands(const at::Tensor &a, const at::Tensor &b)
 // product is the platform's library GEMM.  4096 x 4096 x 4096: 3.06 -> ~1.05 ms at 30 % density; the two
 // routes cross at ~10 %.
 // `one_in`: the density from which the route is taken, one stored entry in `one_in`: 8 for the CSR kernel; 16 for the
-// COO kernel (any order, duplicates, atomics), which takes about twice as long per entry (4096^3 at
-// 10 % density: 1.89 against 0.87 ms, the GEMM 0.99 ms).
+// COO kernel (any order, duplicates, atomics), which takes at least one and a half times as long per entry (4096^3 at
+// 10 % density: 1.46 ms with ascending rows, 20.8 in random order, against 0.87, the GEMM 0.99 ms).
 bool dense_route_pays(int64_t nnz, int64_t R, int64_t K, int64_t C, int64_t one_in)
 {
     return R > 0 && K > 0 && C >= 64 && nnz >= (R * K + one_in - 1) / one_in && R * K <= (int64_t(1) << 29);
@@ -584,15 +584,15 @@ at::Tensor cusparsemm_csr(const at::Tensor &a, const at::Tensor &b)
     return c;
 }
 
-// Whether the sum by rows pays for a coalesced COO operand (nanoseconds).  It takes a wave per row, however empty (0.13), 0.08 more where the row
-// has entries; the COO kernel clears c (0.0007 a value), adds a run of entries to it (0.007 a value) and takes 0.038 longer per entry and
-// 10 us longer in all.  By rows / by entries, us: 2^20 rows of 0.05 / 0.5 / 2 / 8 entries x 1 column 126 / 18, 156 / 43, 208 / 125, 267 / 408, x 16
-// 119 / 36, 165 / 111, 214 / 213, 273 / 424, x 64 119 / 88, 167 / 398, 217 / 818, 278 / 1029; 2^23 rows of 0.05 x 1 952 / 47; 200000 rows of 1 x 1 35 / 24,
-// of 2 x 16 40 / 54; 65536 rows of 2 x 1 17.6 / 16.7, x 4 17.5 / 21.8; 4096 rows of 0.05 to 60 x 1 to 4096 columns 9 to 142 / 12 to 421.
+// Whether the sum by rows pays for a coalesced COO operand (nanoseconds).  It takes a wave per row, however empty (0.115), 0.075 more where the row
+// has entries; the COO kernel clears c (0.0007 a value), adds a run of entries to it (0.002 a value) and takes 0.033 longer per entry and
+// 5 us longer in all.  By rows / by entries, us: 2^20 rows of 0.05 / 0.5 / 2 / 8 entries x 1 column 125 / 17, 156 / 41, 209 / 111, 268 / 388, x 16
+// 120 / 27, 164 / 49, 212 / 118, 273 / 393, x 64 119 / 57, 167 / 129, 214 / 226, 275 / 465, x 256 174 / 246, 208 / 565, 261 / 994, 410 / 1197; 2^23 rows of
+// 0.05 x 1 957 / 41; 65536 rows of 2 / 4 x 1 17.8 / 16.0, 19.5 / 20.1; 4096 rows of 1 x 64 14.3 / 14.2, x 4096 25 / 46, of 41 x 4096 118 / 169.
 bool rows_pay(int64_t nnz, int64_t R, int64_t C)
 {
     const double rows = (double)R, filled = (double)std::min(nnz, R);
-    return 0.13 * rows < 10000.0 + 0.0007 * rows * (double)C + filled * (0.007 * (double)C - 0.08) + 0.038 * (double)nnz;
+    return 0.115 * rows < 5000.0 + 0.0007 * rows * (double)C + filled * (0.002 * (double)C - 0.075) + 0.033 * (double)nnz;
 }
 
 at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
@@ -607,8 +607,8 @@ at::Tensor cusparsemm_coo(const at::Tensor &a, const at::Tensor &b)
     const int64_t nnz = val.numel();
     // A coalesced operand's rows ascend (the device looks whether they do: the flag can be set without it): with row offsets it is a
     // CSR operand, whose kernel adds a row up in registers instead of clearing c and adding to it (4096 x 4096 at 1 % x 4096 columns:
-    // 364 -> 116 us), where that pays.  A row is one wave's there, so the device looks for crowded ones too.  Up to the K that both were timed at
-    // (4096 x 32768 with 33 entries a row x 4096 columns: 477 -> 290 us), and no more rows than a launch holds waves.
+    // 170 -> 114 us), where that pays.  A row is one wave's there, so the device looks for crowded ones too.  Up to the K that both were timed at
+    // (4096 x 32768 with 33 entries a row x 4096 columns: 308 -> 291 us), and no more rows than a launch holds waves.
     const bool by_rows = a.is_coalesced() && K <= 32768 && R <= (int64_t(1) << 24) && rows_pay(nnz, R, C);
     if (dense_route_pays(nnz, R, K, C, by_rows ? 8 : 16)) {
         auto dense = at::empty({R, K}, b.options());

@@ -177,13 +177,13 @@ def test_operands_flagged_as_coalesced_whatever_their_order(cols, spoil):
 @pytest.mark.parametrize("at", [0, 1, -1])
 @pytest.mark.parametrize("more", [0, 1])
 def test_crowded_rows_are_not_one_wave_s(rows, k, cols, each, at, more):
-    """Rows of the most entries that a wave takes, and of one more: nnz * cols / 2^17 + 256.  The result either way,
+    """Rows of the most entries that a wave takes, and of one more: nnz * cols / 2^18 + 256.  The result either way,
     and which way it was."""
     from mamtorch_amd import capi
 
     g = torch.Generator().manual_seed(rows)
     lengths = [each] * rows
-    longest = lambda n: 256 + int(n * cols / 2 ** 17)
+    longest = lambda n: 256 + int(n * cols / 2 ** 18)
     while longest(sum(lengths)) != lengths[at % rows]:          # (it counts into nnz itself)
         lengths[at % rows] = longest(sum(lengths))
     lengths[at % rows] += more
