@@ -552,11 +552,12 @@ def run_spmm_sweep(torch, capi, lib, dev, args):
                 asp = ad.to_sparse(layout=layout)
                 ms = timed(lambda: op(asp, b), steps)
                 lib_ms = timed(lambda: torch.sparse.mm(asp, b), max(steps // 4, 3))
-                dense_route = size >= 64 and nnz * (16 if name == "coo" else 8) >= size * size
+                # (to_sparse's COO operands are coalesced: summed by rows, by the CSR kernel after row_offsets_kernel)
+                dense_route = size >= 64 and nnz * 8 >= size * size
                 cells.append({"size": size, "sparse_rate": rate, "layout": name, "nnz": nnz,
                               "cusparsemm_ms": round(ms, 5), "torch_matmul_dense_ms": round(dense_ms, 5),
                               "torch_sparse_mm_ms": round(lib_ms, 5),
-                              "route": "densify + at::mm" if dense_route else "%s_spmm_kernel" % name})
+                              "route": "densify + at::mm" if dense_route else "csr_spmm_kernel"})
                 total_ops += nnz * size
                 total_ms += ms
     biggest = [c for c in cells if c["size"] == 4096 and c["sparse_rate"] == 0.9 and c["layout"] == "csr"][0]

@@ -1474,15 +1474,16 @@ static int launch_forward(const Params &p, hipStream_t st)
     const int64_t bx = (int64_t)tx * splits_of(TB, N, tx, p.cus), bw = (int64_t)tw * splits_of(TB, M, tw, p.cus);
     const unsigned blocks = (unsigned)(bx > bw || p.call.w_layout != MAM_W_MK ? bx : bw);
     auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(blocks), dim3(NT), lds, st, p); };
-    // The 32 words that neighbouring lanes store are one line in memory only where rows of c start lines.  Elsewhere they are parts of
-    // two, which the five or seven planes of a one-sided search had better leave to the L2 (past it / to it, us: 12608 x 768 -> 3004 862 /
-    // 718, -> 3040 559 / 619; 16384 x 4096 -> 1001 444 / 374, -> 1024 353 / 364); the values alone go past it either way (-> 1001 253 /
-    // 261, 12608 x 768 -> 3004 401 / 402), and two-sided searches do (12608 x 768 -> 3001 2058 / 2148, 16384 x 2048 -> 1000 645 / 670).
+    // The 32 words that neighbouring lanes store are whole half lines in memory, 64 bytes, only where rows of c start such halves.  Elsewhere
+    // the five or seven planes of a one-sided search had better leave them to the L2 (past it / to it, us: 12608 x 768 -> 3004 862 / 718, -> 3032 727 /
+    // 715, -> 3024 561 / 696, -> 3040 559 / 619; 16384 x 4096 -> 1001 444 / 374, -> 1000 390 / 374, -> 1008 368 / 382, -> 1024 353 / 364); the values
+    // alone go past it either way (-> 1001 253 / 261, 12608 x 768 -> 3004 401 / 402), and two-sided searches do (12608 x 768 -> 3001 2058 / 2148, 16384 x
+    // 2048 -> 1000 645 / 670).
     const Call &c = p.call;
-    const bool lines = c.M % 32 == 0 && (((uintptr_t)c.c | (uintptr_t)c.argmax | (uintptr_t)c.argmin | (uintptr_t)c.wsel | (uintptr_t)c.xsel) & 127) == 0;
+    const bool halves = c.M % 16 == 0 && (((uintptr_t)c.c | (uintptr_t)c.argmax | (uintptr_t)c.argmin | (uintptr_t)c.wsel | (uintptr_t)c.xsel) & 63) == 0;
     constexpr bool always = TWO, never = TB == 16;      // (16 rows: no lines by the layout)
     if (!c.argmax) launch(forward_kernel<TB, false, TWO, true>);
-    else if (always || (lines && !never)) launch(forward_kernel<TB, true, TWO, !never>);
+    else if (always || (halves && !never)) launch(forward_kernel<TB, true, TWO, !never>);
     else launch(forward_kernel<TB, true, TWO, always>);
     return check_launch("ordered::forward_kernel");
 }

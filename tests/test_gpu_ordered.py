@@ -119,7 +119,7 @@ def test_equal_products_met_by_different_lanes(N, K, M, kinds):
 
 
 @pytest.mark.parametrize("K", [800, 3000, 5000])                      # 32, 8 and 4 tile rows
-@pytest.mark.parametrize("M", [32, 64, 96, 100, 101])
+@pytest.mark.parametrize("M", [32, 48, 64, 96, 100, 101, 112])
 @pytest.mark.parametrize("kinds", [("normal", "uniform"), ("uniform", "normal")])
 def test_outputs_that_are_lines_and_parts_of_lines(K, M, kinds):
     _check(70, K, M, *kinds, seed=M)

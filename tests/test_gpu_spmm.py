@@ -395,6 +395,33 @@ def test_b_of_more_than_4_gib(cols, ldb):
     _check(c, want, floor, "rows that fall")
 
 
+@pytest.mark.parametrize("ldb", [0, 2 ** 27 + 5])
+@pytest.mark.parametrize("cols,blocks", [(1, 300), (100, 255), (100, 256), (300, 127), (300, 128), (300, 511), (300, 512), (513, 342),
+                                         (600, 1300)])
+@pytest.mark.parametrize("ascending", [False, True])
+def test_entries_by_columns_per_lane(cols, blocks, ldb, ascending):
+    """One column a lane below 256 workgroups of four columns a lane (256 entries and columns each), two below 1024, four from
+    there on; b of more and of less than 4 GiB; more workgroups than the fallback launches, in turns."""
+    from mamtorch_amd import capi
+
+    rows, k, nnz = 500, 9, 256 * (blocks - 1) + 1
+    g = torch.Generator().manual_seed(cols + blocks)
+    row = torch.randint(0, rows, (nnz,), generator=g)
+    row = row.sort()[0] if ascending else row
+    col, val, b = torch.randint(0, k, (nnz,), generator=g), torch.randn(nnz, generator=g), torch.randn(k, cols, generator=g)
+    want, floor = oracle.coo_spmm(row.numpy(), col.numpy(), val.numpy(), b.numpy(), rows)
+    if ldb:
+        bd = torch.empty((k - 1) * ldb + cols, device=DEV).as_strided((k, cols), (ldb, 1))
+        bd.copy_(b)
+    else:
+        bd = b.to(DEV)
+    row, col, val = row.to(DEV), col.to(DEV), val.to(DEV)
+    _check(capi.coo_spmm(row, col, val, bd, rows), want, floor, "coo")
+    c, by_rows = capi.coo_spmm_by_rows(row, col, val, bd, rows)
+    assert ascending or not by_rows
+    _check(c, want, floor, "by rows" if by_rows else "after the look")
+
+
 def test_to_dense_skips_coordinates_outside_the_matrix():
     """mam_csr_to_dense / mam_coo_to_dense write at the coordinates they are given: an entry outside the
     matrix (a malformed tensor) is dropped instead of written out of range."""
