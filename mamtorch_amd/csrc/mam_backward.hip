@@ -223,12 +223,13 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
     do {                                                                                            \
         if (row_ok && (m) < M) {                                                                    \
             const int64_t o_ = (int64_t)n * M + (m);                                                \
-            g = *reinterpret_cast<const float4 *>(grad + o_);                                       \
-            i1 = *reinterpret_cast<const int4 *>(argmax + (pl) * nm + o_);                          \
-            i2 = *reinterpret_cast<const int4 *>(argmin + (pl) * nm + o_);                          \
+            const int left_ = M - (m);                                                              \
+            g = row_quad(grad + o_, left_);                                                         \
+            i1 = row_quad(argmax + (pl) * nm + o_, left_);                                          \
+            i2 = row_quad(argmin + (pl) * nm + o_, left_);                                          \
             if (w_sel) {                                                                            \
-                s1 = *reinterpret_cast<const float4 *>(w_sel + (pl) * 2 * nm + o_);                 \
-                s2 = *reinterpret_cast<const float4 *>(w_sel + (pl) * 2 * nm + nm + o_);            \
+                s1 = row_quad(w_sel + (pl) * 2 * nm + o_, left_);                                   \
+                s2 = row_quad(w_sel + (pl) * 2 * nm + nm + o_, left_);                              \
             }                                                                                       \
         } else {                                                                                    \
             i1 = make_int4(-1, -1, -1, -1);                                                         \
@@ -474,12 +475,13 @@ __device__ __forceinline__ void bwd_w_vec_body(
         have = tid < items && m0 + r_first < M;
         if (have) {
             const int64_t o = (int64_t)n_first * M + m0 + r_first;
-            g = *reinterpret_cast<const float4 *>(grad + o);
-            i1 = *reinterpret_cast<const int4 *>(argmax + po_first + o);
-            i2 = *reinterpret_cast<const int4 *>(argmin + po_first + o);
+            const int left = M - m0 - r_first;
+            g = row_quad(grad + o, left);
+            i1 = row_quad(argmax + po_first + o, left);
+            i2 = row_quad(argmin + po_first + o, left);
             if (x_sel) {
-                s1 = *reinterpret_cast<const float4 *>(x_sel + 2 * po_first + o);
-                s2 = *reinterpret_cast<const float4 *>(x_sel + 2 * po_first + nm + o);
+                s1 = row_quad(x_sel + 2 * po_first + o, left);
+                s2 = row_quad(x_sel + 2 * po_first + nm + o, left);
             }
         }
     };
@@ -508,13 +510,14 @@ __device__ __forceinline__ void bwd_w_vec_body(
             if (m0 + r0 >= M) continue;
             const int64_t o = (int64_t)n * M + m0 + r0;
             const int64_t po = (int64_t)(pl_lo + pl) * nm;
-            const float4 gg = *reinterpret_cast<const float4 *>(grad + o);
-            const int4 j1 = *reinterpret_cast<const int4 *>(argmax + po + o);
-            const int4 j2 = *reinterpret_cast<const int4 *>(argmin + po + o);
+            const int left = M - m0 - r0;
+            const float4 gg = row_quad(grad + o, left);
+            const int4 j1 = row_quad(argmax + po + o, left);
+            const int4 j2 = row_quad(argmin + po + o, left);
             float y1[4], y2[4];
             if (x_sel) {
-                const float4 t1 = *reinterpret_cast<const float4 *>(x_sel + 2 * po + o);
-                const float4 t2 = *reinterpret_cast<const float4 *>(x_sel + 2 * po + nm + o);
+                const float4 t1 = row_quad(x_sel + 2 * po + o, left);
+                const float4 t2 = row_quad(x_sel + 2 * po + nm + o, left);
                 y1[0] = t1.x; y1[1] = t1.y; y1[2] = t1.z; y1[3] = t1.w;
                 y2[0] = t2.x; y2[1] = t2.y; y2[2] = t2.z; y2[3] = t2.w;
             } else {
@@ -739,71 +742,6 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
     }
 }
 
-// Generic path: any M, any alignment; one (batch row, neuron) pair per thread and trip.
-template <int LAYOUT, bool BIAS>
-__global__ __launch_bounds__(NT_W) void mam_bwd_w_kernel(
-    const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
-    const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
-    const float *__restrict__ x_sel, int64_t nm, float *__restrict__ w_grad, int N, int K, int M, int log2r,
-    int kc, int vec_out, int planes, int range_len, float *__restrict__ bias_out)
-{
-    extern __shared__ float hist[];
-    __shared__ float bias_part[BIAS ? NT_W / 64 : 1][MAX_NEURONS];
-    const bool sum_bias = BIAS && blockIdx.y == 0;       // as in bwd_w_vec_body, a neuron per thread
-    float bias_now = 0.0f, bias_sum = 0.0f;
-    const int tid = threadIdx.x;
-    const int R = 1 << log2r;
-    const int mt = xcd_remap(blockIdx.x, gridDim.x);
-    const int m0 = mt * R;
-    const int k0 = blockIdx.y * kc;
-    const int rn = (M - m0) < R ? (M - m0) : R;
-    const int kn = (K - k0) < kc ? (K - k0) : kc;
-
-    for (int i = tid * 4; i < R * kc; i += NT_W * 4)
-        *reinterpret_cast<float4 *>(&hist[i]) = make_float4(0.f, 0.f, 0.f, 0.f);
-    __syncthreads();
-    const int64_t pairs = (int64_t)N << log2r;
-    // one (argmax, argmin) pair of absolute k per K range; only the planes whose ranges meet this k chunk
-    const int pl_lo = planes > 1 ? k0 / range_len : 0;
-    int pl_hi = planes > 1 ? (k0 + kn - 1) / range_len : 0;
-    pl_hi = pl_hi < planes - 1 ? pl_hi : planes - 1;
-    for (int pl = pl_lo; pl <= pl_hi; ++pl) {
-        const int32_t *amax_pl = argmax + pl * nm, *amin_pl = argmin + pl * nm;
-        const float *x_sel_pl = x_sel ? x_sel + pl * 2 * nm : nullptr;
-        for (int64_t pi = tid; pi < pairs; pi += NT_W) {
-            const int n = (int)(pi >> log2r), r = (int)(pi & (R - 1));
-            if (r >= rn) continue;
-            const int64_t o = (int64_t)n * M + m0 + r;
-            const float g = grad[o];
-            if (sum_bias && pl == 0) {
-                bias_now += g;
-                if (pi / NT_W % BIAS_TERMS == BIAS_TERMS - 1) { bias_sum += bias_now; bias_now = 0.0f; }
-            }
-            const int a1 = amax_pl[o] - k0, a2 = amin_pl[o] - k0;
-            const float *xr = x + (int64_t)n * ldx + k0;
-            if ((unsigned)a1 < (unsigned)kn)
-                lds_add_sparse(&hist[LAYOUT == MAM_W_MK ? r * kc + a1 : (a1 << log2r) + r],
-                               (x_sel_pl ? x_sel_pl[o] : xr[a1]) * g);
-            if ((unsigned)a2 < (unsigned)kn)
-                lds_add_sparse(&hist[LAYOUT == MAM_W_MK ? r * kc + a2 : (a2 << log2r) + r],
-                               (x_sel_pl ? x_sel_pl[nm + o] : xr[a2]) * g);
-        }
-    }
-    if (sum_bias) {
-        bias_sum += bias_now;
-        for (int s = R; s < 64; s <<= 1) bias_sum += __shfl_xor(bias_sum, s);
-        if ((tid & 63) < R) bias_part[tid >> 6][tid & 63] = bias_sum;
-    }
-    __syncthreads();
-    if (sum_bias && tid < rn) {
-        float sum = bias_part[0][tid];
-#pragma unroll
-        for (int v = 1; v < (BIAS ? NT_W / 64 : 1); ++v) sum += bias_part[v][tid];
-        bias_out[m0 + tid] = sum;
-    }
-    store_slab<LAYOUT, NT_W>(hist, w_grad, tid, m0, k0, rn, kn, kc, log2r, K, M, vec_out, false);
-}
-
 // LDS a workgroup may use for a histogram, in floats, per device.  gfx950 has 160 KiB per CU; above
 // 64 KiB the kernel attribute has to be raised first, once per device, which the device's set-up does
 // for every kernel of this file.
@@ -819,8 +757,6 @@ static int setup_device(int dev)
     const void *kernels[] = {
         (const void *)mam_bwd_x_rows_kernel<MAM_W_MK>, (const void *)mam_bwd_x_rows_kernel<MAM_W_KM>,
         (const void *)mam_bwd_x_kernel<MAM_W_MK>,      (const void *)mam_bwd_x_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_w_kernel<MAM_W_MK, false>,      (const void *)mam_bwd_w_kernel<MAM_W_KM, false>,
-        (const void *)mam_bwd_w_kernel<MAM_W_MK, true>,       (const void *)mam_bwd_w_kernel<MAM_W_KM, true>,
         (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false>,  (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, false>,
         (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true>,   (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, true>,
         (const void *)mam_bwd_both_kernel<MAM_W_MK, false>,   (const void *)mam_bwd_both_kernel<MAM_W_MK, true>,
@@ -860,9 +796,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
     const int cus = num_cus();
     // 64-bit fixed-point cells: room for 2 * M * planes terms of 24 + span - 1 bits each, and one bit to spare
     const int span = window_span(2 * M * planes);
-    const bool x_rows = N >= 2048 && K * 16 <= ((int64_t)lds_cap * 4 - 8192 < 64 * 1024 ? (int64_t)lds_cap * 4 - 8192 : 64 * 1024) && (M % 4 == 0) && ((uintptr_t)grad % 16 == 0) &&
-                        ((uintptr_t)argmax % 16 == 0) && ((uintptr_t)argmin % 16 == 0) &&
-                        ((uintptr_t)w_sel % 16 == 0);
+    const bool x_rows = N >= 2048 && K * 16 <= ((int64_t)lds_cap * 4 - 8192 < 64 * 1024 ? (int64_t)lds_cap * 4 - 8192 : 64 * 1024);
     if (x_grad && x_rows) {
         // as many rows per workgroup (2 to 16) as fit 64 KiB of LDS in 8-byte cells
         // (the queue and the window's scratch are static LDS on top of the cells: 8 KiB kept free for them)
@@ -887,14 +821,14 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
     if (w_grad) {
         // (M,K): 4 whole-K rows in 64 KiB, so two workgroups share a CU.  (K,M): 32 columns x
         // 1024 k in 128 KiB.
-        const int vec_in = (M % 4 == 0) && ((uintptr_t)grad % 16 == 0) && ((uintptr_t)argmax % 16 == 0) &&
-                           ((uintptr_t)argmin % 16 == 0) && ((uintptr_t)x_sel % 16 == 0) && (N * M % 4 == 0);
+        const bool aligned = (M % 4 == 0) && ((uintptr_t)grad % 16 == 0) && ((uintptr_t)argmax % 16 == 0) &&
+                             ((uintptr_t)argmin % 16 == 0) && ((uintptr_t)x_sel % 16 == 0) && (N * M % 4 == 0);
         int log2r = LAYOUT == MAM_W_MK ? 2 : 5;
         // Large batches: a thread reads 16 bytes of a batch row per array, so a slab of 4 neurons uses
         // a quarter of every 64-byte sector it touches.  When K is small enough, 16 neurons (whole
         // sectors) share a slab, and the batch is split over several workgroups per slab to keep the
         // chip filled; they add their shares to the cleared w_grad.
-        if (LAYOUT == MAM_W_MK && vec_in && planes == 1 && K % 4 == 0 && (uintptr_t)w_grad % 16 == 0 &&
+        if (LAYOUT == MAM_W_MK && aligned && planes == 1 && K % 4 == 0 && (uintptr_t)w_grad % 16 == 0 &&
             option(MAM_OPT_BACKWARD_EXACT) == MAM_BACKWARD_EXACT_ON) {
             // 4 neurons x kc columns of 8-byte cells in 64 KiB
             int kce = 2048;
@@ -907,7 +841,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
                 return check_launch("mam_bwd_w_exact_kernel");
             }
         }
-        const bool large_batch = LAYOUT == MAM_W_MK && vec_in && N >= 2048;
+        const bool large_batch = LAYOUT == MAM_W_MK && N >= 2048;
         if (large_batch)
             while (log2r < 4 && ((int64_t)2 << log2r) * ((K + 3) / 4 * 4) * 4 <= 64 * 1024) ++log2r;
         const int R = 1 << log2r;
@@ -917,58 +851,49 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
         const int64_t mtiles = ceil_div(M, R), ktiles = ceil_div(K, kc);
         if (ktiles > 65535) return fail(MAM_ERR_UNSUPPORTED, "K too large for the w_grad grid");
         const int vec_out = (K % 4 == 0) && ((uintptr_t)w_grad % 16 == 0);
-        if (vec_in) {
-            // slabs per workgroup: enough workgroups for two per CU, the rest goes into pipelining
-            int tpw = (int)(mtiles * ktiles / (2 * cus));
-            if (tpw < 1) tpw = 1;
-            if (tpw > 8) tpw = 8;
-            // shares of the batch per slab: two rounds of as many workgroups as fit the chip by the slab's LDS and their threads
-            // (registers leave room for two per CU, so the bias gradient's 1 KiB beside the slab changes nothing: 16384 x 620 / 640 /
-            // 656 -> 1024, three or four by LDS, 176 / 176 / 180 us)
-            int64_t shares = 1;
-            if (large_batch) {
-                int64_t per_cu = (160 * 1024) / ((int64_t)R * kc * 4);
-                if (per_cu > 2048 / NT_W) per_cu = 2048 / NT_W;
-                if (per_cu < 1) per_cu = 1;
-                shares = (2 * per_cu * cus + mtiles * ktiles / 2) / (mtiles * ktiles);
-                // a share adds a whole slab to w_grad with atomics: worth it only against >= K rows of work
-                if (shares > most_shares(N, K)) shares = most_shares(N, K);
-                if (shares > 65535) shares = 65535;
-                if (shares < 1) shares = 1;
-            }
-            const int64_t rows_per_share = ceil_div(N, shares);
-            shares = ceil_div(N, rows_per_share);
-            if (shares > 1) {
-                rc = fill_zero(w_grad, M * K, st);
-                if (rc != MAM_OK) return rc;
-            }
-            float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
-            hipLaunchKernelGGL((bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true> : mam_bwd_w_vec_kernel<LAYOUT, false>),
-                               dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT_W),
-                               (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
-                               w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
-                               (int)rows_per_share, planes, range_len, bias_out);
-            if (bias_out) {
-                bias->done = true;
-                if (shares > 1) {
-                    rc = check_launch("mam_bwd_w_kernel");
-                    return rc != MAM_OK ? rc : sum_slabs(bias_out, bias->out, M, shares, st);
-                }
-            }
-        } else {
-            hipLaunchKernelGGL((bias ? mam_bwd_w_kernel<LAYOUT, true> : mam_bwd_w_kernel<LAYOUT, false>), dim3((unsigned)mtiles, (unsigned)ktiles),
-                               dim3(NT_W), (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax,
-                               argmin, x_sel, N * M, w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, planes,
-                               range_len, bias ? bias->out : nullptr);
-            if (bias) bias->done = true;
+        // slabs per workgroup: enough workgroups for two per CU, the rest goes into pipelining
+        int tpw = (int)(mtiles * ktiles / (2 * cus));
+        if (tpw < 1) tpw = 1;
+        if (tpw > 8) tpw = 8;
+        // shares of the batch per slab: two rounds of as many workgroups as fit the chip by the slab's LDS and their threads
+        // (registers leave room for two per CU, so the bias gradient's 1 KiB beside the slab changes nothing: 16384 x 620 / 640 /
+        // 656 -> 1024, three or four by LDS, 176 / 176 / 180 us)
+        int64_t shares = 1;
+        if (large_batch) {
+            int64_t per_cu = (160 * 1024) / ((int64_t)R * kc * 4);
+            if (per_cu > 2048 / NT_W) per_cu = 2048 / NT_W;
+            if (per_cu < 1) per_cu = 1;
+            shares = (2 * per_cu * cus + mtiles * ktiles / 2) / (mtiles * ktiles);
+            // a share adds a whole slab to w_grad with atomics: worth it only against >= K rows of work
+            if (shares > most_shares(N, K)) shares = most_shares(N, K);
+            if (shares > 65535) shares = 65535;
+            if (shares < 1) shares = 1;
         }
-        rc = check_launch("mam_bwd_w_kernel");
+        const int64_t rows_per_share = ceil_div(N, shares);
+        shares = ceil_div(N, rows_per_share);
+        if (shares > 1) {
+            rc = fill_zero(w_grad, M * K, st);
+            if (rc != MAM_OK) return rc;
+        }
+        float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
+        hipLaunchKernelGGL((bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true> : mam_bwd_w_vec_kernel<LAYOUT, false>),
+                           dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT_W),
+                           (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
+                           w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
+                           (int)rows_per_share, planes, range_len, bias_out);
+        if (bias_out) {
+            bias->done = true;
+            if (shares > 1) {
+                rc = check_launch("mam_bwd_w_vec_kernel");
+                return rc != MAM_OK ? rc : sum_slabs(bias_out, bias->out, M, shares, st);
+            }
+        }
+        rc = check_launch("mam_bwd_w_vec_kernel");
     }
     return rc;
 }
 
-// Both gradients in one launch (mam_bwd_both_kernel) where the shape allows it: (M,K) weights, the 16-byte
-// paths of both kernels, a batch small enough that the x_grad workgroups (one per batch row) are all resident
+// Both gradients in one launch (mam_bwd_both_kernel) where the shape allows it: (M,K) weights, a batch small enough that the x_grad workgroups (one per batch row) are all resident
 // at once, K in one chunk of either kernel -- and, unless the option forces it, at most 2^16 outputs.
 // Returns MAM_OK after launching, 1 when the shape is not served.
 static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *grad,
@@ -980,9 +905,6 @@ static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw,
     const int dev = ensure_device(st);
     if (dev < 0) return dev;
     const int cus = num_cus();
-    const bool vec_in = (M % 4 == 0) && (N * M % 4 == 0) && ((uintptr_t)grad % 16 == 0) &&
-                        ((uintptr_t)argmax % 16 == 0) && ((uintptr_t)argmin % 16 == 0) &&
-                        ((uintptr_t)x_sel % 16 == 0);
     constexpr int64_t kLds = 64 * 1024;               // dynamic LDS of the launch: two workgroups per CU
     const int log2r = 2, R = 4;
     const int64_t kc_w = (K + 3) / 4 * 4;
@@ -990,7 +912,7 @@ static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw,
     // 256 x 4096 x 4096 one launch took 35.6 us against 29.2 us for two, with one slab or two per w_grad
     // workgroup: the x_grad workgroups hold one of the two slots of every CU for as long as they run.
     const bool small = (auto_mode ? N * M <= (1 << 16) : true);
-    if (!small || !vec_in || N >= 2048 || N > 2 * cus || K * 8 > kLds || R * kc_w * 4 > kLds ||
+    if (!small || N >= 2048 || N > 2 * cus || K * 8 > kLds || R * kc_w * 4 > kLds ||
         g_lds_floats[dev] * 4 < (int)kLds + 8192)
         return 1;
     const int64_t mtiles = ceil_div(M, R);

@@ -94,6 +94,38 @@ __device__ __forceinline__ float load_w(const float *__restrict__ w, int64_t ldw
     return LAYOUT == MAM_W_MK ? w[m * ldw + k] : w[k * ldw + m];
 }
 
+// Four consecutive words of a row of which `left` are left: one load where there are four, of 4-byte aligned addresses (what a load
+// of four words needs), so that neither the number of neurons nor an operand's alignment takes a call off the kernels that read in
+// fours; past the end of the row `none`.
+typedef float floats4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef int ints4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 row_quad(const float *p, int left)
+{
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (left >= 4) {
+        const floats4 t = *reinterpret_cast<const floats4 *>(p);
+        v = make_float4(t.x, t.y, t.z, t.w);
+    } else {
+        if (left > 0) v.x = p[0];
+        if (left > 1) v.y = p[1];
+        if (left > 2) v.z = p[2];
+    }
+    return v;
+}
+__device__ __forceinline__ int4 row_quad(const int32_t *p, int left)
+{
+    int4 v = make_int4(-1, -1, -1, -1);
+    if (left >= 4) {
+        const ints4 t = *reinterpret_cast<const ints4 *>(p);
+        v = make_int4(t.x, t.y, t.z, t.w);
+    } else {
+        if (left > 0) v.x = p[0];
+        if (left > 1) v.y = p[1];
+        if (left > 2) v.z = p[2];
+    }
+    return v;
+}
+
 // out[m] = sum over s of partial[s][m], in slab order (mam_module.hip).
 int sum_slabs(const float *partial, float *out, int64_t M, int64_t slabs, hipStream_t stream);
 

@@ -40,7 +40,6 @@
 namespace mam {
 namespace csr {
 
-constexpr int NT = 256;
 constexpr int NT_B = 512;  // backward workgroup
 constexpr int EG = 8;      // entries whose loads are issued together
 constexpr int NT_F = 1024;      // forward workgroup
@@ -492,79 +491,10 @@ __device__ __forceinline__ void lds_add_sparse(float *addr, float v)
 #define MAM_CSR_RB 16
 #endif
 constexpr int RB = MAM_CSR_RB;   // CSR rows per val_grad workgroup
-constexpr int VAL_CAP = 16384;   // histogram floats per pass (64 KiB)
 
 // val_grad of the entries of RB consecutive CSR rows, from the entry positions recorded by the
-// forward (pos_sel, (2, N, M), -1 where an implicit zero was selected).
-__global__ __launch_bounds__(NT) void csr_bwd_val_kernel(
-    const float *__restrict__ x, int64_t ldx, const int64_t *__restrict__ crow,
-    const float *__restrict__ grad, const int32_t *__restrict__ argmax,
-    const int32_t *__restrict__ argmin, const int32_t *__restrict__ pos_sel,
-    const float *__restrict__ x_sel, int64_t nm, float *__restrict__ val_grad, int N, int M, int vec_in)
-{
-    __shared__ float hist[VAL_CAP];
-    const int tid = threadIdx.x;
-    const int m0 = blockIdx.x * RB;
-    const int rows = (M - m0) < RB ? (M - m0) : RB;
-    const int64_t e_beg = crow[m0], e_end = crow[m0 + rows];
-    for (int64_t c0 = e_beg; c0 < e_end; c0 += VAL_CAP) {
-        const int len = (int)((e_end - c0) < VAL_CAP ? (e_end - c0) : VAL_CAP);
-        for (int i = tid; i < len; i += NT) hist[i] = 0.0f;
-        __syncthreads();
-        for (int n = tid; n < N; n += NT) {
-            const int64_t o = (int64_t)n * M + m0;
-            const float *xr = x + (int64_t)n * ldx;
-            float g[RB];
-            int p1[RB], p2[RB], a1[RB], a2[RB];
-            if (vec_in && rows == RB) {
-#pragma unroll
-                for (int q = 0; q < RB / 4; ++q) {
-                    const float4 gv = *reinterpret_cast<const float4 *>(grad + o + 4 * q);
-                    const int4 u1 = *reinterpret_cast<const int4 *>(pos_sel + o + 4 * q);
-                    const int4 u2 = *reinterpret_cast<const int4 *>(pos_sel + nm + o + 4 * q);
-                    const int4 k1 = *reinterpret_cast<const int4 *>(argmax + o + 4 * q);
-                    const int4 k2 = *reinterpret_cast<const int4 *>(argmin + o + 4 * q);
-                    g[4 * q + 0] = gv.x; g[4 * q + 1] = gv.y; g[4 * q + 2] = gv.z; g[4 * q + 3] = gv.w;
-                    p1[4 * q + 0] = u1.x; p1[4 * q + 1] = u1.y; p1[4 * q + 2] = u1.z; p1[4 * q + 3] = u1.w;
-                    p2[4 * q + 0] = u2.x; p2[4 * q + 1] = u2.y; p2[4 * q + 2] = u2.z; p2[4 * q + 3] = u2.w;
-                    a1[4 * q + 0] = k1.x; a1[4 * q + 1] = k1.y; a1[4 * q + 2] = k1.z; a1[4 * q + 3] = k1.w;
-                    a2[4 * q + 0] = k2.x; a2[4 * q + 1] = k2.y; a2[4 * q + 2] = k2.z; a2[4 * q + 3] = k2.w;
-                }
-            } else {
-#pragma unroll
-                for (int r = 0; r < RB; ++r) {
-                    const bool ok = r < rows;
-                    g[r] = ok ? grad[o + r] : 0.0f;
-                    p1[r] = ok ? pos_sel[o + r] : -1;
-                    p2[r] = ok ? pos_sel[nm + o + r] : -1;
-                    a1[r] = ok ? argmax[o + r] : 0;
-                    a2[r] = ok ? argmin[o + r] : 0;
-                }
-            }
-            float x1[RB], x2[RB];
-#pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                const int64_t q1 = (int64_t)p1[r] - c0, q2 = (int64_t)p2[r] - c0;
-                p1[r] = (p1[r] >= 0 && q1 >= 0 && q1 < len) ? (int)q1 : -1;
-                p2[r] = (p2[r] >= 0 && q2 >= 0 && q2 < len) ? (int)q2 : -1;
-                // (the forward can hand the selected inputs over; else gather them)
-                x1[r] = p1[r] >= 0 ? (x_sel ? x_sel[o + r] : xr[a1[r]]) : 0.0f;
-                x2[r] = p2[r] >= 0 ? (x_sel ? x_sel[nm + o + r] : xr[a2[r]]) : 0.0f;
-            }
-#pragma unroll
-            for (int r = 0; r < RB; ++r) {
-                if (p1[r] >= 0) lds_add_sparse(&hist[p1[r]], x1[r] * g[r]);
-                if (p2[r] >= 0) lds_add_sparse(&hist[p2[r]], x2[r] * g[r]);
-            }
-        }
-        __syncthreads();
-        for (int i = tid; i < len; i += NT) val_grad[c0 + i] = hist[i];
-        __syncthreads();
-    }
-}
-
-// The same for 16-byte aligned inputs with M a multiple of 4 (what the operators produce): 1024 threads,
-// a thread's item is one batch row x 4 consecutive CSR rows -- five 16-byte loads (the selected inputs as
+// forward (pos_sel, (2, N, M), -1 where an implicit zero was selected): 1024 threads,
+// a thread's item is one batch row x 4 consecutive CSR rows -- five loads of four words (the selected inputs as
 // handed over by the forward; without them up to eight single-word gathers from x, which then take two
 // thirds of the kernel's time)
 // -- so that the four threads of a batch row cover whole 64-byte sectors and sixteen waves hide each
@@ -576,7 +506,7 @@ __global__ __launch_bounds__(NT) void csr_bwd_val_kernel(
 constexpr int NT_V = 1024;
 constexpr int VAL_CELLS = 7168;    // entries per pass (56 KiB of 8-byte cells: with the queue under 64 KiB)
 
-__global__ __launch_bounds__(NT_V) void csr_bwd_val_vec_kernel(
+__global__ __launch_bounds__(NT_V) void csr_bwd_val_kernel(
     const float *__restrict__ x, int64_t ldx, const int64_t *__restrict__ crow,
     const float *__restrict__ grad, const int32_t *__restrict__ argmax,
     const int32_t *__restrict__ argmin, const int32_t *__restrict__ pos_sel,
@@ -592,7 +522,7 @@ __global__ __launch_bounds__(NT_V) void csr_bwd_val_vec_kernel(
     const int rows = (M - m0) < RB ? (M - m0) : RB;
     const int64_t e_beg = crow[m0], e_end = crow[m0 + rows];
     constexpr int QPR = RB / 4;                      // items per batch row
-    const int items = N * QPR;
+    const int64_t items = (int64_t)N * QPR;
 
     // one item: batch row n, CSR rows m0 + r0 .. r0 + 3; positions relative to the pass, -1 = nothing to add
     float4 g, s1, s2;
@@ -601,22 +531,23 @@ __global__ __launch_bounds__(NT_V) void csr_bwd_val_vec_kernel(
     int p1[4], p2[4];
 #define MAM_VAL_LOAD(it, c0, len)                                                                    \
     do {                                                                                             \
-        const int n_ = (it) / QPR, r0_ = ((it) % QPR) * 4;                                           \
+        const int n_ = (int)((it) / QPR), r0_ = (int)((it) % QPR) * 4;                                           \
         const bool ok_ = (it) < items && r0_ < rows;                                                 \
         u1 = u2 = make_int4(-1, -1, -1, -1);                                                         \
         k1 = k2 = make_int4(0, 0, 0, 0);                                                             \
         g = s1 = s2 = make_float4(0.f, 0.f, 0.f, 0.f);                                               \
         if (ok_) {                                                                                   \
             const int64_t o_ = (int64_t)n_ * M + m0 + r0_;                                           \
-            g = *reinterpret_cast<const float4 *>(grad + o_);                                        \
-            u1 = *reinterpret_cast<const int4 *>(pos_sel + o_);                                      \
-            u2 = *reinterpret_cast<const int4 *>(pos_sel + nm + o_);                                 \
+            const int left_ = rows - r0_;                                                            \
+            g = row_quad(grad + o_, left_);                                                          \
+            u1 = row_quad(pos_sel + o_, left_);                                                      \
+            u2 = row_quad(pos_sel + nm + o_, left_);                                                 \
             if (x_sel) {                                                                             \
-                s1 = *reinterpret_cast<const float4 *>(x_sel + o_);                                  \
-                s2 = *reinterpret_cast<const float4 *>(x_sel + nm + o_);                             \
+                s1 = row_quad(x_sel + o_, left_);                                                    \
+                s2 = row_quad(x_sel + nm + o_, left_);                                               \
             } else {                                                                                 \
-                k1 = *reinterpret_cast<const int4 *>(argmax + o_);                                   \
-                k2 = *reinterpret_cast<const int4 *>(argmin + o_);                                   \
+                k1 = row_quad(argmax + o_, left_);                                                   \
+                k2 = row_quad(argmin + o_, left_);                                                   \
             }                                                                                        \
         }                                                                                            \
         const float sa_[4] = {s1.x, s1.y, s1.z, s1.w}, sb_[4] = {s2.x, s2.y, s2.z, s2.w};            \
@@ -664,7 +595,7 @@ __global__ __launch_bounds__(NT_V) void csr_bwd_val_vec_kernel(
             if (fx) for (int i = tid; i < len; i += NT_V) cells[i] = 0ull;
             else for (int i = tid; i < len; i += NT_V) hist[i] = 0.0f;
             __syncthreads();
-            for (int it = tid; it < items; it += NT_V) {
+            for (int64_t it = tid; it < items; it += NT_V) {
                 if (!loaded) MAM_VAL_LOAD(it, c0, len);
                 loaded = false;
                 const float gv[4] = {g.x, g.y, g.z, g.w};
@@ -870,17 +801,9 @@ extern "C" int mam_csr_fc_backward(const float *x, int64_t ldx, const int64_t *c
             fork.join_later();
         }
         if (val_grad) {
-            const int vec_in = (M % 4 == 0) && ((uintptr_t)grad % 16 == 0) && ((uintptr_t)argmax % 16 == 0) &&
-                               ((uintptr_t)argmin % 16 == 0) && ((uintptr_t)pos_sel % 16 == 0) &&
-                               ((uintptr_t)x_sel % 16 == 0) && ((N * M) % 4 == 0);
-            if (vec_in)
-                hipLaunchKernelGGL(csr::csr_bwd_val_vec_kernel, dim3((unsigned)ceil_div(M, csr::RB)), dim3(csr::NT_V),
-                                   0, st, x, ldx, crow, grad, argmax, argmin, pos_sel, x_sel, N * M, val_grad, (int)N,
-                                   (int)M, fixedpoint::window_span(2 * N));
-            else
-                hipLaunchKernelGGL(csr::csr_bwd_val_kernel, dim3((unsigned)ceil_div(M, csr::RB)), dim3(csr::NT), 0,
-                                   st, x, ldx, crow, grad, argmax, argmin, pos_sel, x_sel, N * M, val_grad, (int)N,
-                                   (int)M, 0);
+            hipLaunchKernelGGL(csr::csr_bwd_val_kernel, dim3((unsigned)ceil_div(M, csr::RB)), dim3(csr::NT_V),
+                               0, st, x, ldx, crow, grad, argmax, argmin, pos_sel, x_sel, N * M, val_grad, (int)N,
+                               (int)M, fixedpoint::window_span(2 * N));
             rc = check_launch("csr_bwd_val_kernel");
         }
         const int rc_join = fork.join();

@@ -505,3 +505,30 @@ def test_bias_gradient_of_large_batches_in_short_sums(N, M, layout):
     _, _, bg = capi.fc_backward_bias(x, w, grad, picks[0], picks[1], layout)
     want = grad.double().sum(0)
     assert bool(((bg.double() - want).abs() <= (64 + N / threads / 64 + 24) * 2.0 ** -24 * want).all())
+
+
+@pytest.mark.parametrize("shape", [(2051, 24, 1), (2048, 130, 3), (2500, 288, 5), (3001, 1300, 42), (2100, 70, 83), (300, 96, 7), (1, 40, 2)])
+def test_rows_of_any_length_at_any_word(shape):
+    """Quads of neurons that end a row (of one, two or three), and arrays that start at any word: the kernels of large batches and of small
+    ones, bias gradient among them (64 terms a sum: as tight as the other sums)."""
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    N, K, M = shape
+    x, w, grad = random_case(N, K, M, seed=sum(shape))
+    g = torch.Generator().manual_seed(N)
+    amax = torch.randint(0, K, (N, M), generator=g, dtype=torch.int32)
+    amin = torch.randint(0, min(K, 3), (N, M), generator=g, dtype=torch.int32)
+    _check(x, w, grad, amax.numpy(), amin.numpy(), "any length %s" % (shape,))
+
+    def at_word(t, off):
+        flat = torch.empty(t.numel() + off, dtype=t.dtype, device=dev)[off:]
+        return flat.copy_(t.reshape(-1)).view(t.shape)
+
+    xo, wo = oracle.backward(x.numpy(), w.numpy(), grad.numpy(), amax.numpy(), amin.numpy(), oracle.W_MK)
+    xs, ws = oracle.backward(x.abs().numpy(), w.abs().numpy(), grad.abs().numpy(), amax.numpy(), amin.numpy(), oracle.W_MK)
+    xg, wg, bg = capi.fc_backward_bias(x.to(dev), w.to(dev), at_word(grad, 1), at_word(amax, 2), at_word(amin, 3), capi.W_MK)
+    assert (np.abs(xg.cpu().numpy() - xo) <= RTOL * np.abs(xo) + FLOOR * xs + 1e-30).all()
+    assert (np.abs(wg.cpu().numpy() - wo) <= RTOL * np.abs(wo) + FLOOR * ws + 1e-30).all()
+    gd = grad.double()
+    assert ((bg.cpu().double() - gd.sum(0)).abs() <= RTOL * gd.sum(0).abs() + FLOOR * gd.abs().sum(0) + 1e-30).all()
