@@ -216,6 +216,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
     const int m_step = (NT_W / 64) * lpr * 4;     // neurons of a row the workgroup covers per trip
     const int trips = (M + m_step - 1) / m_step;     // the same for every thread: lanes past M hold no item
 
+    const bool quads = M % 4 == 0;
     float4 g = make_float4(0.f, 0.f, 0.f, 0.f), s1 = g, s2 = g;
     int4 i1 = make_int4(-1, -1, -1, -1), i2 = i1;
 // (a macro, not a lambda: captured by reference the five vectors end up in scratch memory)
@@ -223,7 +224,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
     do {                                                                                            \
         if (row_ok && (m) < M) {                                                                    \
             const int64_t o_ = (int64_t)n * M + (m);                                                \
-            const int left_ = M - (m);                                                              \
+            const int left_ = quads ? 4 : M - (m);                                                           \
             g = row_quad(grad + o_, left_);                                                         \
             i1 = row_quad(argmax + (pl) * nm + o_, left_);                                          \
             i2 = row_quad(argmin + (pl) * nm + o_, left_);                                          \
@@ -331,40 +332,90 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
 #undef MAM_LOAD_ITEM
 }
 
-// Scatter of one (batch row, 4 consecutive neurons) item into the slab histogram.  COUNT ((M,K) layout): the
-// picks are also counted in `cnt`, a second LDS plane of the slab's shape whose words hold two 16-bit fields
-// (low: argmax picks, high: argmin picks).
-template <int LAYOUT, bool COUNT = false>
-__device__ __forceinline__ void scatter_quad(float *hist, const float4 &g, const int4 &i1, const int4 &i2,
-                                             const float (&x1)[4], const float (&x2)[4], int r0, int k0,
-                                             int kn, int kc, int log2r, uint32_t *cnt = nullptr)
+// One batch row and Q consecutive neurons (2 or 4): the gradient, the two picks and the inputs picked.
+template <int Q>
+struct Item {
+    float g[Q], x1[Q], x2[Q];
+    int32_t a1[Q], a2[Q];
+};
+
+// (one branch for all loads of an item, which are then in flight together)
+template <int Q>
+__device__ __forceinline__ void load_item(Item<Q> &it, const float *grad, const int32_t *argmax, const int32_t *argmin,
+                                          const float *x_sel, int64_t nm, int left)
 {
-    const float gv[4] = {g.x, g.y, g.z, g.w};
-    const int a1[4] = {i1.x - k0, i1.y - k0, i1.z - k0, i1.w - k0};
-    const int a2[4] = {i2.x - k0, i2.y - k0, i2.z - k0, i2.w - k0};
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const int r = r0 + u;
-        if ((unsigned)a1[u] < (unsigned)kn) {
-            lds_add_sparse(&hist[LAYOUT == MAM_W_MK ? r * kc + a1[u] : (a1[u] << log2r) + r], x1[u] * gv[u]);
-            if (COUNT) atomicAdd(&cnt[r * kc + a1[u]], 1u);
+    if (left >= Q) {
+        row_words<Q>(grad, Q, 0.0f, it.g);
+        row_words<Q>(argmax, Q, -1, it.a1);
+        row_words<Q>(argmin, Q, -1, it.a2);
+        if (x_sel) {
+            row_words<Q>(x_sel, Q, 0.0f, it.x1);
+            row_words<Q>(x_sel + nm, Q, 0.0f, it.x2);
         }
-        if ((unsigned)a2[u] < (unsigned)kn) {
-            lds_add_sparse(&hist[LAYOUT == MAM_W_MK ? r * kc + a2[u] : (a2[u] << log2r) + r], x2[u] * gv[u]);
-            if (COUNT) atomicAdd(&cnt[r * kc + a2[u]], 0x10000u);
+    } else {
+        row_words<Q>(grad, left, 0.0f, it.g);
+        row_words<Q>(argmax, left, -1, it.a1);
+        row_words<Q>(argmin, left, -1, it.a2);
+        if (x_sel) {
+            row_words<Q>(x_sel, left, 0.0f, it.x1);
+            row_words<Q>(x_sel + nm, left, 0.0f, it.x2);
         }
     }
 }
 
-__device__ __forceinline__ void gather_quad(const float *xr, const int4 &i1, const int4 &i2, int k0, int kn,
-                                            float (&x1)[4], float (&x2)[4])
+// the inputs picked, without the hand-over: from row xr of x
+template <int Q>
+__device__ __forceinline__ void gather_item(Item<Q> &it, const float *xr, int k0, int kn)
 {
-    const int a1[4] = {i1.x - k0, i1.y - k0, i1.z - k0, i1.w - k0};
-    const int a2[4] = {i2.x - k0, i2.y - k0, i2.z - k0, i2.w - k0};
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        x1[u] = (unsigned)a1[u] < (unsigned)kn ? xr[a1[u]] : 0.0f;
-        x2[u] = (unsigned)a2[u] < (unsigned)kn ? xr[a2[u]] : 0.0f;
+    for (int u = 0; u < Q; ++u) {
+        it.x1[u] = (unsigned)(it.a1[u] - k0) < (unsigned)kn ? xr[it.a1[u]] : 0.0f;
+        it.x2[u] = (unsigned)(it.a2[u] - k0) < (unsigned)kn ? xr[it.a2[u]] : 0.0f;
+    }
+}
+
+// v[u] = v[(u + n) % Q]
+template <class T>
+__device__ __forceinline__ void turn(T (&v)[2], int n)
+{
+    const T a = n & 1 ? v[1] : v[0], b = n & 1 ? v[0] : v[1];
+    v[0] = a;
+    v[1] = b;
+}
+template <class T>
+__device__ __forceinline__ void turn(T (&v)[4], int n)
+{
+    const T a = n & 1 ? v[1] : v[0], b = n & 1 ? v[2] : v[1], c = n & 1 ? v[3] : v[2], d = n & 1 ? v[0] : v[3];
+    v[0] = n & 2 ? c : a;
+    v[1] = n & 2 ? d : b;
+    v[2] = n & 2 ? a : c;
+    v[3] = n & 2 ? b : d;
+}
+
+// Scatter of an item of batch row n, neurons r0 .. of the slab, into the slab histogram.  Batch rows begin at different neurons: the lanes of
+// one instruction that hold one neuron each pick among its few largest weights, and the fewer of them, the fewer contend for a cell.
+// COUNT ((M,K) layout): the
+// picks are also counted in `cnt`, a second LDS plane of the slab's shape whose words hold two 16-bit fields
+// (low: argmax picks, high: argmin picks).
+template <int LAYOUT, bool COUNT, int Q>
+__device__ __forceinline__ void scatter_item(float *hist, Item<Q> it, int n, int r0, int k0, int kn, int kc, int log2r, uint32_t *cnt)
+{
+    turn(it.g, n);
+    turn(it.x1, n);
+    turn(it.x2, n);
+    turn(it.a1, n);
+    turn(it.a2, n);
+#pragma unroll
+    for (int u = 0; u < Q; ++u) {
+        const int r = r0 + ((u + n) & (Q - 1)), a1 = it.a1[u] - k0, a2 = it.a2[u] - k0;
+        if ((unsigned)a1 < (unsigned)kn) {
+            lds_add_sparse(&hist[LAYOUT == MAM_W_MK ? r * kc + a1 : (a1 << log2r) + r], it.x1[u] * it.g[u]);
+            if (COUNT) atomicAdd(&cnt[r * kc + a1], 1u);
+        }
+        if ((unsigned)a2 < (unsigned)kn) {
+            lds_add_sparse(&hist[LAYOUT == MAM_W_MK ? r * kc + a2 : (a2 << log2r) + r], it.x2[u] * it.g[u]);
+            if (COUNT) atomicAdd(&cnt[r * kc + a2], 0x10000u);
+        }
     }
 }
 
@@ -376,18 +427,14 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
 {
     const int R = 1 << log2r;
     if (accumulate) {
-        // the batch is split over several workgroups per slab: w_grad was cleared beforehand and
-        // every workgroup adds its share (cells it never touched are skipped)
-        for (int e = tid; e < (LAYOUT == MAM_W_MK ? rn * kn : (kn << log2r)); e += NT) {
-            int r, kk;
-            float v;
-            if (LAYOUT == MAM_W_MK) { r = e / kn; kk = e - r * kn; v = hist[r * kc + kk]; }
-            else { kk = e >> log2r; r = e & (R - 1); v = hist[e]; }
-            if (v != 0.0f && r < rn) {
-                float *cell = LAYOUT == MAM_W_MK ? w_grad + (int64_t)(m0 + r) * K + k0 + kk
-                                                 : w_grad + (int64_t)(k0 + kk) * M + m0 + r;
-                __hip_atomic_fetch_add(cell, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
+        // the batch is split over several workgroups per slab ((M,K) layout): w_grad was cleared beforehand and
+        // every workgroup adds its share (cells it never touched are skipped), the lanes of a wave to 64 neighbouring
+        // words (to every fourth of 256: 12608 x 768 -> 3072 290 us instead of 212)
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, pieces = (kn + 63) >> 6;
+        for (int i = wave; i < rn * pieces; i += NT / 64) {
+            const int r = i / pieces, kk = (i - r * pieces) * 64 + lane;
+            const float v = kk < kn ? hist[r * kc + kk] : 0.0f;
+            if (v != 0.0f) __hip_atomic_fetch_add(w_grad + (int64_t)(m0 + r) * K + k0 + kk, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         return;
     }
@@ -413,9 +460,8 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
     }
 }
 
-// Fast path (M a multiple of 4, 16-byte aligned grad / argmax / argmin).  A thread's unit of work
-// is one batch row x 4 consecutive neurons: three 16-byte loads, eight x gathers from one row,
-// eight LDS adds.  A workgroup walks `tiles_per_wg` consecutive slabs and software-pipelines them:
+// A thread's unit of work is one batch row x Q consecutive neurons (4 or 2): five loads of Q words, or three and 2 Q x gathers from one
+// row without the hand-over, and 2 Q LDS adds.  A workgroup walks `tiles_per_wg` consecutive slabs and software-pipelines them:
 // the index loads of the next slab are issued before the current slab is streamed out, and the x
 // gathers are in flight while the histogram is cleared, so the scatter phase's latency chain
 // (index load -> gather -> LDS add) overlaps the store phase instead of alternating with it.
@@ -429,7 +475,7 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
 // fixed order.  BIAS_TERMS of a thread's items make a sum of their own, so that rounding errors do not grow with the batch (one
 // running sum per thread: 2-norm error 1.07e-6 for 400000 rows where mam_bias_grad's 256 running sums give 6.5e-7).
 constexpr int BIAS_TERMS = 64;
-template <int LAYOUT, int NT, bool COUNT, bool BIAS>
+template <int LAYOUT, int NT, bool COUNT, bool BIAS, int Q>
 __device__ __forceinline__ void bwd_w_vec_body(
     float *hist, int bx, int nbx, int by, int bz, int nbz,
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
@@ -445,7 +491,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
     uint32_t *cnt = reinterpret_cast<uint32_t *>(hist) + ((size_t)kc << log2r);
     const int tid = threadIdx.x;
     const int R = 1 << log2r;
-    const int qpr = R >> 2;
+    const int qpr = R / Q;
     // bz: which share of the batch rows (one share = the whole batch unless the host split it)
     const int n_begin = bz * rows_per_split;
     const int n_rows = (N - n_begin) < rows_per_split ? (N - n_begin) : rows_per_split;
@@ -465,24 +511,15 @@ __device__ __forceinline__ void bwd_w_vec_body(
     // this thread's first item of a slab: plane pl_lo + pf, row n_first, neurons m0 + r_first .. +3
     const int pf = npl > 1 ? (int)(tid / per_plane) : 0;
     const int rem_first = npl > 1 ? (int)(tid - pf * per_plane) : tid;
-    const int n_first = n_begin + rem_first / qpr, r_first = (rem_first % qpr) * 4;
+    const int n_first = n_begin + rem_first / qpr, r_first = (rem_first % qpr) * Q;
     const int64_t po_first = (int64_t)(pl_lo + pf) * nm;
-    float4 g = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 s1 = g, s2 = g;      // selected inputs handed over by the forward, if any
-    int4 i1 = make_int4(-1, -1, -1, -1), i2 = make_int4(-1, -1, -1, -1);
+    Item<Q> it1;
     bool have = false;
     auto load_first = [&](int m0) {
         have = tid < items && m0 + r_first < M;
         if (have) {
             const int64_t o = (int64_t)n_first * M + m0 + r_first;
-            const int left = M - m0 - r_first;
-            g = row_quad(grad + o, left);
-            i1 = row_quad(argmax + po_first + o, left);
-            i2 = row_quad(argmin + po_first + o, left);
-            if (x_sel) {
-                s1 = row_quad(x_sel + 2 * po_first + o, left);
-                s2 = row_quad(x_sel + 2 * po_first + nm + o, left);
-            }
+            load_item(it1, grad + o, argmax + po_first + o, argmin + po_first + o, x_sel ? x_sel + 2 * po_first + o : nullptr, nm, M - m0 - r_first);
         }
     };
     if (first < mtiles) load_first(first * R);
@@ -492,55 +529,49 @@ __device__ __forceinline__ void bwd_w_vec_body(
         if (mt >= mtiles) break;
         const int m0 = mt * R;
         const int rn = (M - m0) < R ? (M - m0) : R;
-        float x1[4] = {s1.x, s1.y, s1.z, s1.w}, x2[4] = {s2.x, s2.y, s2.z, s2.w};
-        if (have && !x_sel) gather_quad(x + (int64_t)n_first * ldx + k0, i1, i2, k0, kn, x1, x2);
+        if (have && !x_sel) gather_item(it1, x + (int64_t)n_first * ldx, k0, kn);
         for (int i = tid * 4; i < (COUNT ? 2 : 1) * R * kc; i += NT * 4)
             *reinterpret_cast<float4 *>(&hist[i]) = make_float4(0.f, 0.f, 0.f, 0.f);
         __syncthreads();
-        if (have) scatter_quad<LAYOUT, COUNT>(hist, g, i1, i2, x1, x2, r_first, k0, kn, kc, log2r, cnt);
-        float4 bias_now = have && pf == 0 ? g : make_float4(0.f, 0.f, 0.f, 0.f), bias_sum = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (have) scatter_item<LAYOUT, COUNT>(hist, it1, n_first, r_first, k0, kn, kc, log2r, cnt);
+        float bias_now[Q], bias_sum[Q];
+#pragma unroll
+        for (int u = 0; u < Q; ++u) {
+            bias_now[u] = have && pf == 0 ? it1.g[u] : 0.0f;
+            bias_sum[u] = 0.0f;
+        }
         auto fold = [&] {
-            bias_sum = make_float4(bias_sum.x + bias_now.x, bias_sum.y + bias_now.y, bias_sum.z + bias_now.z, bias_sum.w + bias_now.w);
-            bias_now = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int u = 0; u < Q; ++u) {
+                bias_sum[u] += bias_now[u];
+                bias_now[u] = 0.0f;
+            }
         };
-        for (int64_t it = tid + NT; it < items; it += NT) {
-            const int pl = npl > 1 ? (int)(it / per_plane) : 0;
-            const int64_t rem = npl > 1 ? it - pl * per_plane : it;
-            const int n = n_begin + (int)(rem / qpr), r0 = (int)(rem % qpr) * 4;
+        for (int64_t i = tid + NT; i < items; i += NT) {
+            const int pl = npl > 1 ? (int)(i / per_plane) : 0;
+            const int64_t rem = npl > 1 ? i - pl * per_plane : i;
+            const int n = n_begin + (int)(rem / qpr), r0 = (int)(rem % qpr) * Q;
             if (m0 + r0 >= M) continue;
             const int64_t o = (int64_t)n * M + m0 + r0;
             const int64_t po = (int64_t)(pl_lo + pl) * nm;
-            const int left = M - m0 - r0;
-            const float4 gg = row_quad(grad + o, left);
-            const int4 j1 = row_quad(argmax + po + o, left);
-            const int4 j2 = row_quad(argmin + po + o, left);
-            float y1[4], y2[4];
-            if (x_sel) {
-                const float4 t1 = row_quad(x_sel + 2 * po + o, left);
-                const float4 t2 = row_quad(x_sel + 2 * po + nm + o, left);
-                y1[0] = t1.x; y1[1] = t1.y; y1[2] = t1.z; y1[3] = t1.w;
-                y2[0] = t2.x; y2[1] = t2.y; y2[2] = t2.z; y2[3] = t2.w;
-            } else {
-                gather_quad(x + (int64_t)n * ldx + k0, j1, j2, k0, kn, y1, y2);
-            }
-            scatter_quad<LAYOUT, COUNT>(hist, gg, j1, j2, y1, y2, r0, k0, kn, kc, log2r, cnt);
+            Item<Q> it;
+            load_item(it, grad + o, argmax + po + o, argmin + po + o, x_sel ? x_sel + 2 * po + o : nullptr, nm, M - m0 - r0);
+            if (!x_sel) gather_item(it, x + (int64_t)n * ldx, k0, kn);
+            scatter_item<LAYOUT, COUNT>(hist, it, n, r0, k0, kn, kc, log2r, cnt);
             if (sum_bias && pl == 0) {
-                bias_now.x += gg.x;
-                bias_now.y += gg.y;
-                bias_now.z += gg.z;
-                bias_now.w += gg.w;
-                if (it / NT % BIAS_TERMS == BIAS_TERMS - 1) fold();
+#pragma unroll
+                for (int u = 0; u < Q; ++u) bias_now[u] += it.g[u];
+                if (i / NT % BIAS_TERMS == BIAS_TERMS - 1) fold();
             }
         }
         if (sum_bias) {
             fold();
-            for (int s = qpr; s < 64; s <<= 1) {
-                bias_sum.x += __shfl_xor(bias_sum.x, s);
-                bias_sum.y += __shfl_xor(bias_sum.y, s);
-                bias_sum.z += __shfl_xor(bias_sum.z, s);
-                bias_sum.w += __shfl_xor(bias_sum.w, s);
-            }
-            if ((tid & 63) < qpr) *reinterpret_cast<float4 *>(&bias_part[tid >> 6][(tid & 63) * 4]) = bias_sum;
+            for (int s = qpr; s < 64; s <<= 1)
+#pragma unroll
+                for (int u = 0; u < Q; ++u) bias_sum[u] += __shfl_xor(bias_sum[u], s);
+            if ((tid & 63) < qpr)
+#pragma unroll
+                for (int u = 0; u < Q; ++u) bias_part[tid >> 6][(tid & 63) * Q + u] = bias_sum[u];
         }
         __syncthreads();
         if (sum_bias && tid < rn) {
@@ -559,8 +590,8 @@ __device__ __forceinline__ void bwd_w_vec_body(
     }
 }
 
-template <int LAYOUT, bool BIAS>
-__global__ __launch_bounds__(NT_W) void mam_bwd_w_vec_kernel(
+template <int LAYOUT, bool BIAS, int NT, int Q>
+__global__ __launch_bounds__(NT) void mam_bwd_w_vec_kernel(
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
     const float *__restrict__ x_sel, int64_t nm, float *__restrict__ w_grad, int N, int K, int M, int log2r,
@@ -568,7 +599,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_w_vec_kernel(
     float *__restrict__ bias_out)
 {
     extern __shared__ float hist[];
-    bwd_w_vec_body<LAYOUT, NT_W, false, BIAS>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
+    bwd_w_vec_body<LAYOUT, NT, false, BIAS, Q>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
                                  argmin, x_sel, nm, w_grad, N, K, M, log2r, kc, vec_out, mtiles, tiles_per_wg,
                                  rows_per_split, planes, range_len, nullptr, nullptr, bias_out);
 }
@@ -582,7 +613,7 @@ __global__ __launch_bounds__(NT_C) void mam_bwd_w_count_kernel(
     int32_t *__restrict__ min_count, int N, int K, int M, int log2r, int kc, int mtiles, int tiles_per_wg)
 {
     extern __shared__ float hist[];
-    bwd_w_vec_body<MAM_W_MK, NT_C, true, false>(hist, blockIdx.x, gridDim.x, blockIdx.y, 0, 1, x, ldx, grad, argmax, argmin,
+    bwd_w_vec_body<MAM_W_MK, NT_C, true, false, 4>(hist, blockIdx.x, gridDim.x, blockIdx.y, 0, 1, x, ldx, grad, argmax, argmin,
                                          x_sel, nm, w_grad, N, K, M, log2r, kc, 1, mtiles, tiles_per_wg, N, 1, K,
                                          max_count, min_count);
 }
@@ -735,7 +766,7 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
         bwd_x_body<LAYOUT>(both_lds, blockIdx.x, p.w, p.ldw, p.grad, p.argmax, p.argmin, p.w_sel, p.nm, p.x_grad, p.K,
                            p.M, p.kc_x, p.planes, p.span);
     } else {
-        bwd_w_vec_body<LAYOUT, NT_X, false, BIAS>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
+        bwd_w_vec_body<LAYOUT, NT_X, false, BIAS, 4>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
                                      0, 1, p.x, p.ldx, p.grad, p.argmax, p.argmin, p.x_sel, p.nm, p.w_grad, p.N, p.K,
                                      p.M, p.log2r, p.kc_w, p.vec_out, p.mtiles, p.tiles_per_wg, p.N, p.planes,
                                      p.range_len, nullptr, nullptr, p.bias_grad);
@@ -757,8 +788,8 @@ static int setup_device(int dev)
     const void *kernels[] = {
         (const void *)mam_bwd_x_rows_kernel<MAM_W_MK>, (const void *)mam_bwd_x_rows_kernel<MAM_W_KM>,
         (const void *)mam_bwd_x_kernel<MAM_W_MK>,      (const void *)mam_bwd_x_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false>,  (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, false>,
-        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true>,   (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, true>,
+        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false, NT_W, 4>, (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false, NT_W, 2>,  (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, false, NT_X, 4>,
+        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 4>, (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 2>,   (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, true, NT_X, 4>,
         (const void *)mam_bwd_both_kernel<MAM_W_MK, false>,   (const void *)mam_bwd_both_kernel<MAM_W_MK, true>,
         (const void *)mam_bwd_w_count_kernel,
     };
@@ -779,8 +810,37 @@ struct BiasGrad {
     int64_t partials;        // rows of M that `partial` holds
     bool done;
 };
-// shares of the batch that a w_grad launch may use and the partial sums of a bias gradient they need
-static int64_t most_shares(int64_t N, int64_t K) { return N / (K > 512 ? K : 512) < 1 ? 1 : N / (K > 512 ? K : 512); }
+// Shares of the batch that a w_grad launch uses for `slabs` slabs.  A share adds its slab to w_grad with atomics, and the clearing of w_grad is
+// one more launch (the bias gradient's sum over the shares another), which below 1536 rows cost the host what they save.
+//   Few slabs: as many shares (a power of two, at least four of 64 rows and a quarter of K) as leave a CU a workgroup.  us without / with, kernels
+//   alone: 5408 x 288 -> 40 17.8 (10 shares) / 9.5, 4704 x 234 -> 36 18.0 / 9.7, 8192 x 4096 -> 64 36 / 20.8, 3152 x 1536 -> 384 24 / 20.6, 496 x 691
+//   in four ranges -> 105 21.6 / 9.7; but 1900 x 2048 -> 200 13.2 / 14.2, 1000 x 1024 -> 256 10.9 / 11.5.
+//   Many rows: two rounds of as many workgroups as fit the chip, as long as a share has K rows, and 768 (12608 x 768 -> 3072 with 1 / 3 / 8 / 16
+//   shares 257 / 220 / 211 / 230; 3152 x 384 -> 1536 with 4 / 6 35 / 46).
+constexpr int64_t FEW_ROWS = 1536, SHARE_ROWS = 64, MANY_ROWS = 768;
+static int64_t shares_of_many_rows(int64_t N, int64_t K) { return N < 2048 ? 1 : N / (K > MANY_ROWS ? K : MANY_ROWS); }
+static int64_t shares_of(int64_t N, int64_t K, int planes, int64_t slabs, int64_t per_cu, int64_t cus)
+{
+    if (N * planes < FEW_ROWS) return 1;
+    int64_t most = N * planes / (K / 4 > SHARE_ROWS ? K / 4 : SHARE_ROWS), few = 1;
+    if (most > N / SHARE_ROWS) most = N / SHARE_ROWS;
+    if (most > cus / slabs) most = cus / slabs;
+    while (2 * few <= most) few *= 2;
+    if (few < 4) few = 1;
+    int64_t many = (2 * per_cu * cus + slabs / 2) / slabs;
+    if (many > shares_of_many_rows(N, K)) many = shares_of_many_rows(N, K);
+    const int64_t shares = few > many ? few : many;
+    return shares < 1 ? 1 : shares > 65535 ? 65535 : shares;
+}
+// what they are at most from 513 rows on, for the partial sums of a bias gradient (below, its own launch sums in one piece): a slab is of 16
+// neurons at most
+static int64_t most_shares(int64_t N, int64_t K, int64_t M)
+{
+    int64_t few = (int64_t)kNumCU * 16 / M;
+    if (few > N / SHARE_ROWS) few = N / SHARE_ROWS;
+    const int64_t many = shares_of_many_rows(N, K);
+    return few > many ? few : many;
+}
 
 template <int LAYOUT>
 static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *grad,
@@ -855,29 +915,29 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
         int tpw = (int)(mtiles * ktiles / (2 * cus));
         if (tpw < 1) tpw = 1;
         if (tpw > 8) tpw = 8;
-        // shares of the batch per slab: two rounds of as many workgroups as fit the chip by the slab's LDS and their threads
-        // (registers leave room for two per CU, so the bias gradient's 1 KiB beside the slab changes nothing: 16384 x 620 / 640 /
-        // 656 -> 1024, three or four by LDS, 176 / 176 / 180 us)
-        int64_t shares = 1;
-        if (large_batch) {
-            int64_t per_cu = (160 * 1024) / ((int64_t)R * kc * 4);
-            if (per_cu > 2048 / NT_W) per_cu = 2048 / NT_W;
-            if (per_cu < 1) per_cu = 1;
-            shares = (2 * per_cu * cus + mtiles * ktiles / 2) / (mtiles * ktiles);
-            // a share adds a whole slab to w_grad with atomics: worth it only against >= K rows of work
-            if (shares > most_shares(N, K)) shares = most_shares(N, K);
-            if (shares > 65535) shares = 65535;
-            if (shares < 1) shares = 1;
-        }
+        // workgroups of a CU by the slab's LDS and their threads (registers leave room for two, so the bias gradient's 1 KiB beside the slab
+        // changes nothing: 16384 x 620 / 640 / 656 -> 1024, three or four by LDS, 176 / 176 / 180 us)
+        constexpr int NT = LAYOUT == MAM_W_MK ? NT_W : NT_X;
+        int64_t per_cu = (160 * 1024) / ((int64_t)R * kc * 4);
+        if (per_cu > 2048 / NT_W) per_cu = 2048 / NT_W;
+        if (per_cu < 1) per_cu = 1;
+        int64_t shares = LAYOUT == MAM_W_MK ? shares_of(N, K, planes, mtiles * ktiles, per_cu, cus) : 1;
         const int64_t rows_per_share = ceil_div(N, shares);
         shares = ceil_div(N, rows_per_share);
         if (shares > 1) {
             rc = fill_zero(w_grad, M * K, st);
             if (rc != MAM_OK) return rc;
         }
+        // Items of two neurons where the items of a slab are few, so that more lanes share them and more waves fit (65 registers instead of 91): us with
+        // four / two, kernel alone: 496 x 691 in four ranges -> 105 9.6 / 9.0, 910 x 192 -> 768 10.4 / 9.5, 472 x 1050 in four ranges -> 2145 71 / 62,
+        // 1238 x 662 -> 3590 38.4 / 35.0; not for long slabs, which their stores bound (256 x 4096 -> 4096 16.4 / 18.2).  From 2048 rows on where
+        // quads straddle lines and no shares are there (2178 x 1494 -> 1982 39 / 28, -> 1983 47 / 37, -> 1984 25.5 / 27).
+        constexpr int Q = LAYOUT == MAM_W_MK ? 2 : 4;
+        const bool pairs = Q == 2 && (N < 2048 ? K <= 2048 || M % 4 != 0 : shares == 1 && M % 4 != 0);
         float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
-        hipLaunchKernelGGL((bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true> : mam_bwd_w_vec_kernel<LAYOUT, false>),
-                           dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT_W),
+        hipLaunchKernelGGL((pairs ? bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true, NT, Q> : mam_bwd_w_vec_kernel<LAYOUT, false, NT, Q>
+                                  : bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true, NT, 4> : mam_bwd_w_vec_kernel<LAYOUT, false, NT, 4>),
+                           dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT),
                            (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
                            w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
                            (int)rows_per_share, planes, range_len, bias_out);
@@ -911,7 +971,8 @@ static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw,
     // Worth it only where the launches themselves are what a call costs (config 1: 10 -> 7 us).  At
     // 256 x 4096 x 4096 one launch took 35.6 us against 29.2 us for two, with one slab or two per w_grad
     // workgroup: the x_grad workgroups hold one of the two slots of every CU for as long as they run.
-    const bool small = (auto_mode ? N * M <= (1 << 16) : true);
+    // Not where w_grad takes the batch in shares (496 x 691 in four ranges -> 105: 9 of two launches' 22 us, here 22).
+    const bool small = (auto_mode ? N * M <= (1 << 16) && N * planes < FEW_ROWS : true);
     if (!small || N >= 2048 || N > 2 * cus || K * 8 > kLds || R * kc_w * 4 > kLds ||
         g_lds_floats[dev] * 4 < (int)kLds + 8192)
         return 1;
@@ -1061,7 +1122,7 @@ extern "C" int mam_fc_backward(const float *x, int64_t ldx, const float *w, int6
 extern "C" size_t mam_fc_backward_bias_workspace(int64_t N, int64_t K, int64_t M)
 {
     if (N <= 0 || K < 0 || M <= 0) return 0;
-    const size_t shares = K > 0 && N >= 2048 ? (size_t)mam::bwd::most_shares(N, K) * (size_t)M * sizeof(float) : 0;
+    const size_t shares = K > 0 && N > 512 ? (size_t)mam::bwd::most_shares(N, K, M) * (size_t)M * sizeof(float) : 0;
     const size_t slabs = mam_bias_grad_workspace(N, M);
     return shares > slabs ? shares : slabs;
 }

@@ -94,9 +94,23 @@ __device__ __forceinline__ float load_w(const float *__restrict__ w, int64_t ldw
     return LAYOUT == MAM_W_MK ? w[m * ldw + k] : w[k * ldw + m];
 }
 
-// Four consecutive words of a row of which `left` are left: one load where there are four, of 4-byte aligned addresses (what a load
-// of four words needs), so that neither the number of neurons nor an operand's alignment takes a call off the kernels that read in
-// fours; past the end of the row `none`.
+// Q consecutive words of a row of which `left` are left: one load where there are Q, of 4-byte aligned addresses (what a load
+// of several words needs), so that neither the number of neurons nor an operand's alignment takes a call off the kernels that read
+// several words a lane; past the end of the row `none`.
+template <int Q, class T>
+__device__ __forceinline__ void row_words(const T *p, int left, T none, T (&v)[Q])
+{
+    typedef T words __attribute__((ext_vector_type(Q), aligned(4)));
+    if (left >= Q) {
+        const words t = *reinterpret_cast<const words *>(p);
+#pragma unroll
+        for (int u = 0; u < Q; ++u) v[u] = t[u];
+    } else {
+#pragma unroll
+        for (int u = 0; u < Q; ++u) v[u] = u < left ? p[u] : none;
+    }
+}
+// (by name and not by index: through arrays mam_bwd_x_rows_kernel takes 73 us for 12608 x 3072 -> 768, like this 65)
 typedef float floats4 __attribute__((ext_vector_type(4), aligned(4)));
 typedef int ints4 __attribute__((ext_vector_type(4), aligned(4)));
 __device__ __forceinline__ float4 row_quad(const float *p, int left)

@@ -507,10 +507,11 @@ def test_bias_gradient_of_large_batches_in_short_sums(N, M, layout):
     assert bool(((bg.double() - want).abs() <= (64 + N / threads / 64 + 24) * 2.0 ** -24 * want).all())
 
 
-@pytest.mark.parametrize("shape", [(2051, 24, 1), (2048, 130, 3), (2500, 288, 5), (3001, 1300, 42), (2100, 70, 83), (300, 96, 7), (1, 40, 2)])
+@pytest.mark.parametrize("shape", [(2051, 24, 1), (2048, 130, 3), (2500, 288, 5), (3001, 1300, 42), (2100, 70, 83), (300, 96, 7), (1, 40, 2),
+                                   (1600, 60, 37), (2178, 50, 203), (4096, 33, 1022)])
 def test_rows_of_any_length_at_any_word(shape):
-    """Quads of neurons that end a row (of one, two or three), and arrays that start at any word: the kernels of large batches and of small
-    ones, bias gradient among them (64 terms a sum: as tight as the other sums)."""
+    """Quads and pairs of neurons that end a row, and arrays that start at any word: the kernels of large batches and of small
+    ones, with the batch in one share and in several, bias gradient among them (64 terms a sum: as tight as the other sums)."""
     from mamtorch_amd import capi
 
     dev = torch.device("cuda:0")
