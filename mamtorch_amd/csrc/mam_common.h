@@ -45,8 +45,10 @@ int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t co
 
 // dst (rows, ld_dst) = src (rows, cols) with row stride ld, the last element of a row repeated up to ld_dst; two matrices
 // in one launch (rows == 0: none).  ld_dst is a multiple of 4, dst 16-byte aligned, at most 65535 rows together.
+// range_len > 0: rows are consecutive ranges of range_len (the last one shorter), of which each is lengthened to ld_dst / their number
+// (a multiple of 4).
 struct LengthenRows { const float *src; int64_t ld; float *dst; int rows; };
-int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, hipStream_t stream,
+int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, int64_t range_len, hipStream_t stream,
                   const ordered::Guard *guard = nullptr);
 
 // Two independent kernels of one call side by side: the first runs on a second stream of the library

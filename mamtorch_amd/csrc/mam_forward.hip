@@ -74,6 +74,7 @@ struct Params {
     int group_n;       // row tiles swept under one W panel (tile order of the launch)
     ordered::Guard guard;   // the kernels exit at once where the lists serve the call (mam_ordered.hip)
     int gt;            // products per recorded group: G, or 2 G on the wave-uniform-rows tiling at large K
+    int range_len;     // ranges of the caller's that were lengthened to k_per_split: their length (indices count in it)
 };
 
 // An extreme that still holds its initial value (-inf for the max, +inf for the min) was never strictly
@@ -210,9 +211,8 @@ __device__ __forceinline__ int quad_min(int v)
 //   lane, so a caller whose 64 outputs share bases hands in something cheaper.
 //   GT: the k loop's tracking span, 16 or 32 products per recorded group; a lane takes GT/4 of them (one or two
 //   16-byte loads per operand), and the loads of 8 * 16 / GT rounds are in flight together.
-template <int GT, class NM, class OP>
-__device__ __forceinline__ void resolve_wave(const Params &p, const float *vals, const int *grps, float *res,
-                                             int lane, NM nm_of, OP operands)
+template <int GT, class OP>
+__device__ __forceinline__ void resolve_tasks(const float *vals, const int *grps, float *res, int lane, OP operands)
 {
     static_assert(GT == 16 || GT == 32, "tracking span");
     constexpr int PPL = GT / LPT;             // products per lane
@@ -275,6 +275,15 @@ __device__ __forceinline__ void resolve_wave(const Params &p, const float *vals,
             }
         }
     }
+}
+
+template <int GT, class NM, class OP>
+__device__ __forceinline__ void resolve_wave(const Params &p, const float *vals, const int *grps, float *res,
+                                             int lane, NM nm_of, OP operands)
+{
+    resolve_tasks<GT>(vals, grps, res, lane, operands);
+    const float *res_v = res, *res_w = res + 256, *res_x = res + 384;
+    const int *res_i = reinterpret_cast<const int *>(res + 128);
     // lane s finishes output s
     int n, m;
     bool valid;
@@ -781,10 +790,56 @@ __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
 // as their K ranges and leave (max, min, group) partials per range; this kernel resolves every range's
 // extremes exactly (first index, sign of a zero) and adds them up.  argmax / argmin, when asked for, are
 // [range][N*M] planes of ABSOLUTE k.
-template <int LAYOUT, bool ARGS>
+// COOP: with indices on operands that the cooperative resolve takes, range after range, patches as in mam_fwd_merge_kernel (a
+// resolve per lane walks two lines an output and range on its own).
+template <int LAYOUT, bool ARGS, bool COOP>
 __global__ __launch_bounds__(256) void mam_fwd_range_sum_kernel(const Params p)
 {
     const int64_t nm = (int64_t)p.N * p.M;
+    if constexpr (COOP) {
+        constexpr int PC = 64, PR = 4;
+        __shared__ float vals_s[4][2][64];
+        __shared__ int grps_s[4][2][64];
+        __shared__ float res_s[4][RES_WORDS];
+        const int patches_n = (p.N + PR - 1) / PR;
+        const int logical = xcd_remap(blockIdx.x, gridDim.x);
+        const int pm = logical / patches_n, pn = logical - pm * patches_n;
+        const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        const int n = pn * PR + wave, mbase = pm * PC, m = mbase + lane;     // (mbase < M)
+        const bool live = n < p.N && m < p.M;
+        const int64_t o = live ? (int64_t)n * p.M + m : 0;
+        const char *xrow = reinterpret_cast<const char *>(p.x + (int64_t)(n < p.N ? n : p.N - 1) * p.ldx);
+        const char *wrows = reinterpret_cast<const char *>(p.w + (int64_t)mbase * p.ldw);
+        const uint32_t ldw4 = (uint32_t)p.ldw * 4u, last = last_row_offset(p.M, mbase, PC, ldw4), mine = (uint32_t)(lane >> 3) * ldw4;
+        const float *res_v = &res_s[wave][0];
+        const int *res_i = reinterpret_cast<const int *>(res_v + 128);
+        float total = 0.0f;
+        for (int s = 0; s < p.splits; ++s) {
+            const float *base = p.part + (int64_t)s * 3 * nm;
+            const int kb = s * p.k_per_split, g0 = kb / G, pk = __float_as_int(base[2 * nm + o]);
+            vals_s[wave][0][lane] = base[o];
+            vals_s[wave][1][lane] = base[nm + o];
+            grps_s[wave][0][lane] = g0 + (pk & 0xffff);
+            grps_s[wave][1][lane] = g0 + ((pk >> 16) & 0xffff);
+            __syncthreads();
+            resolve_tasks<G>(&vals_s[wave][0][0], &grps_s[wave][0][0], &res_s[wave][0], lane,
+                             [&](int r, int, int, int k, const float *&xp, const float *&wp) {
+                                 const uint32_t row = mine + (uint32_t)(8 * (r & (PC / 8 - 1))) * ldw4, k4 = (uint32_t)k * 4u;
+                                 xp = reinterpret_cast<const float *>(xrow + k4);
+                                 wp = reinterpret_cast<const float *>(wrows + (clamped_row_offset(row, last) + k4));
+                             });
+            __syncthreads();
+            const float v = res_v[lane] + res_v[64 + lane];
+            total = s == 0 ? v : total + v;
+            if (live) {
+                const int shift = p.range_len > 0 ? s * p.range_len - kb : 0;
+                p.argmax[(int64_t)s * nm + o] = res_i[lane] + shift;
+                p.argmin[(int64_t)s * nm + o] = res_i[64 + lane] + shift;
+            }
+        }
+        if (live) p.c[o] = p.bias ? total + p.bias[m] : total;
+        return;
+    }
     const int patches_n = (p.N + 15) / 16;
     const int logical = xcd_remap(blockIdx.x, gridDim.x);
     const int pm = logical / patches_n, pn = logical - pm * patches_n;
@@ -804,8 +859,9 @@ __global__ __launch_bounds__(256) void mam_fwd_range_sum_kernel(const Params p)
             float w_unused, x_unused;
             resolve<LAYOUT>(p, n, m, kb + (pk & 0xffff) * G, ke - 1, hi, false, hi, ih, w_unused, x_unused);
             resolve<LAYOUT>(p, n, m, kb + ((pk >> 16) & 0xffff) * G, ke - 1, lo, true, lo, il, w_unused, x_unused);
-            p.argmax[(int64_t)s * nm + o] = ih;
-            p.argmin[(int64_t)s * nm + o] = il;
+            const int shift = p.range_len > 0 ? s * p.range_len - kb : 0;
+            p.argmax[(int64_t)s * nm + o] = ih + shift;
+            p.argmin[(int64_t)s * nm + o] = il + shift;
         } else {
             if (hi == 0.0f) hi = first_zero_product<LAYOUT>(p.x + (int64_t)n * p.ldx, p.w, p.ldw, m, kb, ke);
             if (lo == 0.0f) lo = first_zero_product<LAYOUT>(p.x + (int64_t)n * p.ldx, p.w, p.ldw, m, kb, ke);
@@ -1335,6 +1391,7 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     }
     p.splits = (int)ceil_div(K, p.k_per_split);
     p.part = nullptr;
+    p.range_len = 0;
     p.guard = ordered::Guard{nullptr};
     plan.need = p.splits > 1 ? (size_t)p.splits * (args ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float) : 0;
     // the fused merge keeps one ticket per tile behind the partials
@@ -1367,10 +1424,11 @@ struct Staging {
     size_t x_bytes, w_bytes;
     size_t bytes() const { return x_bytes + w_bytes; }
 };
-static Staging staging_of(bool x_fits, bool w_fits, int64_t N, int64_t K, int64_t M)
+static Staging staging_of(bool x_fits, bool w_fits, int64_t N, int64_t K, int64_t M, int64_t range_len = 0)
 {
     Staging s;
-    s.K = K % G == 0 ? K : ceil_div(K, sx::KT) * sx::KT;
+    if (range_len > 0 && range_len < K) s.K = ceil_div(K, range_len) * ceil_div(range_len, sx::KT) * sx::KT;
+    else s.K = K % G == 0 ? K : ceil_div(K, sx::KT) * sx::KT;
     s.x = !x_fits || s.K != K;
     s.w = !w_fits || s.K != K;
     auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
@@ -1408,6 +1466,16 @@ static bool lengthened_rows_pay(int64_t N, int64_t K, int64_t M, bool turn, bool
     return K > 32 && !turn && N >= 64 && outputs >= 16384 && outputs <= (1 << 18);
 }
 
+// The same for the caller's ranges, each lengthened to whole 64-k tiles ((N, K, M) in four ranges, us on the general tiling / lengthened, with
+// indices: 496 x 691 x 105 67 / 31, 160 x 3200 x 512 152 / 76, 9536 x 2809 x 1432 6784 / 3003, 16 x 260 x 64 40 / 20; in ranges of 32, 2000 x
+// 500 x 2000 1272 / 1161 but 100 x 128 x 100 18.5 / 19.5).  Values only, where padding short ranges to 64 instead of 32 costs less than the better
+// loop gains: 4000 x 531 x 3712 681 / 641, 500 x 200 x 500 23 / 18, 1441 x 2280 x 94 120 / 48; not 8098 x 278 x 71 43 / 47.
+static bool lengthened_ranges_pay(int64_t N, int64_t M, int64_t range_len, bool args)
+{
+    if (N + M > 65535 || range_len < 32 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
+    return args ? range_len > 32 || N * M > 16384 : range_len >= 96 || N * M <= (1 << 18);
+}
+
 // The plan of a call on staged operands, for a call that the wave-uniform-rows tiling does not take as it is; false:
 // there is none, or it does not pay.
 static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, const float *x, int64_t ldx, const float *w,
@@ -1415,14 +1483,15 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
                         float *x_sel, int64_t N, int64_t K, int64_t M, int64_t range_len)
 {
     if (plan.use_sx) return false;
-    const bool turn = w_layout == MAM_W_KM;
-    st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M);
+    const bool turn = w_layout == MAM_W_KM, ranges = range_len > 0 && range_len < K;
+    st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M, range_len);
     const bool lengthen = st.x || (st.w && !turn);
     if (turn && !transposed_operand_pays(N, K, M)) return false;
-    if (lengthen && (!lengthened_rows_pay(N, K, M, turn, args) || range_len > 0)) return false;
+    if (ranges ? turn || st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args) : lengthen && !lengthened_rows_pay(N, K, M, turn, args)) return false;
     float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
     const int rc = make_plan(staged, args, st.x ? aligned : x, st.x ? st.K : ldx, st.w ? aligned : w, st.w ? st.K : ldw, MAM_W_MK, bias,
-                             c, argmax, argmin, w_sel, x_sel, N, st.K, M, range_len);
+                             c, argmax, argmin, w_sel, x_sel, N, st.K, M, ranges ? st.K / ceil_div(K, range_len) : range_len);
+    if (ranges) staged.p.range_len = (int)range_len;
     return rc == MAM_OK && staged.use_sx;
 }
 
@@ -1525,7 +1594,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
         float *const ws = reinterpret_cast<float *>(scratch_base), *const xs = reinterpret_cast<float *>(scratch_base + stage.w_bytes);
         const bool turn = operand_layout == MAM_W_KM;
         const LengthenRows rx = {x, ldx, xs, stage.x ? (int)N : 0}, rw = {w, ldw, ws, stage.w && !turn ? (int)M : 0};
-        rc = lengthen_rows(rx, rw, operand_K, K, st, &p.guard);
+        rc = lengthen_rows(rx, rw, operand_K, K, range_len, st, &p.guard);
         if (rc == MAM_OK && turn) rc = transpose(w, ldw, ws, operand_K, M, K, st, &p.guard);
         if (rc != MAM_OK) return rc;
         if (stage.x) p.x = xs;
@@ -1546,11 +1615,14 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     if (rc != MAM_OK) return rc;
     if (p.splits > 1 && range_len > 0) {
         // the caller's ranges are neurons of their own: resolve each and add them up
-        const unsigned mb = (unsigned)(ceil_div(N, 16) * ceil_div(M, 16));
-        if (w_layout == MAM_W_MK)
-            hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_MK, ARGS>), dim3(mb), dim3(256), 0, st, p);
+        const bool coop = ARGS && p.coop && p.k_per_split % G == 0;
+        const unsigned mb = coop ? (unsigned)(ceil_div(N, 4) * ceil_div(M, 64)) : (unsigned)(ceil_div(N, 16) * ceil_div(M, 16));
+        if (coop)
+            hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_MK, ARGS, ARGS>), dim3(mb), dim3(256), 0, st, p);
+        else if (w_layout == MAM_W_MK)
+            hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_MK, ARGS, false>), dim3(mb), dim3(256), 0, st, p);
         else
-            hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_KM, ARGS>), dim3(mb), dim3(256), 0, st, p);
+            hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_KM, ARGS, false>), dim3(mb), dim3(256), 0, st, p);
         rc = check_launch("mam_fwd_range_sum_kernel");
     } else if (p.splits > 1 && !fuse) {
         // 16 x 16 patches; 4 x 64 with the cooperative resolve
@@ -1598,7 +1670,10 @@ extern "C" size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t 
 {
     if (N <= 0 || K <= 0 || M <= 0 || range_len <= 0 || range_len >= K) return 0;
     const size_t ranges = (size_t)((K + range_len - 1) / range_len);
-    return ranges * (with_indices ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float);
+    size_t bytes = ranges * (with_indices ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float);
+    // room for lengthened ranges (see launch); without it the call still works
+    if (mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0)) bytes += mam::fwd::staging_of(false, false, N, K, M, range_len).bytes();
+    return bytes;
 }
 
 extern "C" int mam_fc_forward_ranges(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,

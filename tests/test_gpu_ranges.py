@@ -166,3 +166,30 @@ def test_module_splits_run_as_one_operator_and_train():
     wt = torch.randn(7, 40, generator=g).to(DEV).requires_grad_(True)
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_ranges, (a, wt, None, 16, True),
                           test_utils=("test_schema", "test_faketensor", "test_autograd_registration"))
+
+
+@pytest.mark.parametrize("N,K,M,range_len", [(40, 129, 70, 64), (33, 193, 130, 48), (5, 1000, 65, 333), (70, 97, 300, 96), (130, 264, 64, 66)])
+def test_lengthened_ranges_equal_the_general_tiling(N, K, M, range_len):
+    """Ranges copied to whole tiles (a last one of a single input, lengths around a tile's) against the tiling that takes them as they are, with
+    NaN, infinities, signed zeros, ranges without a product and ties in the operands: every output bit for bit."""
+    from mamtorch_amd import capi
+
+    x, w, _ = random_case(N, K, M, seed=K)
+    x[0], x[1, : min(K, 2 * range_len)], x[2, -1], x[3, ::3] = 0.0, float("nan"), float("inf"), -0.0
+    w[0], w[1, -1], w[2, :range_len], w[3, 1::2] = -0.0, float("nan"), 0.0, 0.5
+    x[4, : range_len], w[4] = 0.25, 1.0
+    xd, wd = x.to(DEV), w.to(DEV)
+    outs = []
+    for tiling in (capi.FORWARD_TILING_WIDE, capi.FORWARD_TILING_AUTO):
+        capi.set_option(capi.OPT_FORWARD_TILING, tiling)
+        try:
+            c, amax, amin = capi.fc_forward_ranges(xd, wd, range_len, capi.W_MK)
+            cv, _, _ = capi.fc_forward_ranges(xd, wd, range_len, capi.W_MK, with_indices=False)
+            torch.cuda.synchronize()
+        finally:
+            capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+        outs.append([t.cpu().numpy() for t in (c, cv, amax, amin)])
+    for a, b, what in zip(outs[0][:2], outs[1][:2], ("c", "values")):
+        assert_bits_equal(b, a, what)
+    for a, b, what in zip(outs[0][2:], outs[1][2:], ("argmax", "argmin")):
+        assert_index_equal(b, a, what)
