@@ -426,6 +426,9 @@ int mam_select_accumulate(void *workspace, const float *w, int64_t ldw, int mode
                           const void *aux2, int64_t ld_aux, int64_t M, int64_t K, int pass, void *stream);
 int mam_select_advance(void *workspace, int pass, void *stream);
 int mam_select_result(void *workspace, int mode, float *out, void *stream);
+/* The calls above for one matrix as one. */
+int mam_select_ranks(const float *w, int64_t ldw, int mode, const void *aux, const void *aux2, int64_t ld_aux, int64_t M, int64_t K,
+                     const int64_t *ranks, int nranks, float *out, void *workspace, size_t workspace_bytes, void *stream);
 
 #ifdef __cplusplus
 }

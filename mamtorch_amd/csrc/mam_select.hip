@@ -294,3 +294,15 @@ extern "C" int mam_select_result(void *workspace, int mode, float *out, void *st
                        static_cast<const selectk::State *>(workspace), out, mode == MAM_PRUNE_COUNT ? 1 : 0);
     return check_launch("select result_kernel");
 }
+
+extern "C" int mam_select_ranks(const float *w, int64_t ldw, int mode, const void *aux, const void *aux2, int64_t ld_aux, int64_t M,
+                                int64_t K, const int64_t *ranks, int nranks, float *out, void *workspace, size_t workspace_bytes,
+                                void *stream)
+{
+    int rc = mam_select_begin(workspace, workspace_bytes, ranks, nranks, stream);
+    for (int pass = 0; pass < mam::selectk::PASSES && rc == MAM_OK; ++pass) {
+        rc = mam_select_accumulate(workspace, w, ldw, mode, aux, aux2, ld_aux, M, K, pass, stream);
+        if (rc == MAM_OK) rc = mam_select_advance(workspace, pass, stream);
+    }
+    return rc == MAM_OK ? mam_select_result(workspace, mode, out, stream) : rc;
+}
