@@ -39,7 +39,7 @@ EXPORTS = (
     "mam_csr_fc_forward_workspace", "mam_csr_fc_forward", "mam_csr_fc_backward", "mam_csr_validate",
     "mam_csr_spmm", "mam_coo_spmm", "mam_coo_row_offsets", "mam_coo_spmm_by_rows_workspace",
     "mam_coo_spmm_by_rows", "mam_csr_to_dense", "mam_coo_to_dense",
-    "mam_fc_backward_bias_workspace", "mam_fc_backward_bias",
+    "mam_fc_backward_bias_workspace", "mam_fc_backward_bias", "mam_fc_forward_picks", "mam_fc_backward_picks",
     "mam_blend", "mam_bias_grad_workspace", "mam_bias_grad", "mam_apply_keep", "mam_im2col", "mam_col2im",
     "mam_prune_row_offsets", "mam_prune_fill_csr", "mam_prune_apply",
     "mam_select_workspace", "mam_select_begin", "mam_select_accumulate", "mam_select_advance", "mam_select_result",
@@ -228,6 +228,36 @@ def fc_backward_bias(x, w, grad, argmax, argmin, layout=W_KM, w_sel=None, x_sel=
         _check(l.mam_fc_backward_bias(_p(x), _ld(x), _p(w), _ld(w), layout, _p(grad), _p(argmax), _p(argmin), _p(w_sel),
                                       _p(x_sel), _p(xg), _p(wg), _p(bg), N, K, M, range_len, _p(ws) if workspace_bytes else None,
                                       workspace_bytes, _stream(x)))
+    return xg, wg, bg
+
+
+def fc_forward_picks(x, w, layout=W_KM, bias=None, w_sel=None, x_sel=None, workspace_bytes=None):
+    """-> (c, picks): fc_forward with both indices of an output in one word, argmax in its low half."""
+    l = lib()
+    N, K, M = _dims(x, w, layout)
+    c = torch.empty((N, M), dtype=torch.float32, device=x.device)
+    picks = torch.empty((N, M), dtype=torch.int32, device=x.device)
+    if workspace_bytes is None:
+        workspace_bytes = l.mam_fc_forward_workspace_for(N, K, M, layout, 1)
+    ws = torch.empty(max(workspace_bytes, 1), dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        _check(l.mam_fc_forward_picks(_p(x), _i64(_ld(x)), _p(w), _i64(_ld(w)), layout, _p(bias), _p(c), _p(picks), _p(w_sel), _p(x_sel),
+                                      _i64(N), _i64(K), _i64(M), _p(ws), _size(workspace_bytes), _stream(x)))
+    return c, picks
+
+
+def fc_backward_picks(x, w, grad, picks, layout=W_KM, w_sel=None, x_sel=None, with_bias=False):
+    """fc_backward (and the column sums of grad) from the picks of fc_forward_picks -> (x_grad, w_grad, bias_grad or None)."""
+    l = lib()
+    N, K, M = _dims(x, w, layout)
+    xg = torch.empty((N, K), dtype=torch.float32, device=x.device)
+    wg = torch.empty(tuple(w.shape), dtype=torch.float32, device=x.device)
+    bg = torch.empty(M, dtype=torch.float32, device=x.device) if with_bias else None
+    nbytes = l.mam_fc_backward_bias_workspace(N, K, M) if with_bias else 0
+    ws = torch.empty(max(nbytes, 1), dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        _check(l.mam_fc_backward_picks(_p(x), _i64(_ld(x)), _p(w), _i64(_ld(w)), layout, _p(grad), _p(picks), _p(w_sel), _p(x_sel), _p(xg),
+                                       _p(wg), _p(bg), _i64(N), _i64(K), _i64(M), _p(ws) if nbytes else None, _size(nbytes), _stream(x)))
     return xg, wg, bg
 
 

@@ -80,15 +80,18 @@ __device__ __forceinline__ void bwd_x_body(
     int a1[4], a2[4];
     auto load_trip = [&](int pl, int mb, int k0, int kn) {
         const int32_t *amax_row = argmax + pl * nm + (int64_t)n * M;
-        const int32_t *amin_row = argmin + pl * nm + (int64_t)n * M;
+        const int32_t *amin_row = argmin ? argmin + pl * nm + (int64_t)n * M : nullptr;
         const float *w_sel_pl = w_sel ? w_sel + pl * 2 * nm : nullptr;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int m = mb + u * NT_X;
             const bool ok = m < M;
             g[u] = ok ? g_row[m] : 0.0f;
-            a1[u] = ok ? amax_row[m] - k0 : -1;
-            a2[u] = ok ? amin_row[m] - k0 : -1;
+            a1[u] = ok ? amax_row[m] : -1;
+            if (amin_row) a2[u] = ok ? amin_row[m] : -1;
+            else unpack_picks(a1[u], a2[u]);
+            a1[u] -= k0;
+            a2[u] -= k0;
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -227,7 +230,14 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
             const int left_ = quads ? 4 : M - (m);                                                           \
             g = row_quad(grad + o_, left_);                                                         \
             i1 = row_quad(argmax + (pl) * nm + o_, left_);                                          \
-            i2 = row_quad(argmin + (pl) * nm + o_, left_);                                          \
+            if (argmin) {                                                                           \
+                i2 = row_quad(argmin + (pl) * nm + o_, left_);                                      \
+            } else {                                                                                \
+                unpack_picks(i1.x, i2.x);                                                           \
+                unpack_picks(i1.y, i2.y);                                                           \
+                unpack_picks(i1.z, i2.z);                                                           \
+                unpack_picks(i1.w, i2.w);                                                           \
+            }                                                                                       \
             if (w_sel) {                                                                            \
                 s1 = row_quad(w_sel + (pl) * 2 * nm + o_, left_);                                   \
                 s2 = row_quad(w_sel + (pl) * 2 * nm + nm + o_, left_);                              \
@@ -347,7 +357,7 @@ __device__ __forceinline__ void load_item(Item<Q> &it, const float *grad, const 
     if (left >= Q) {
         row_words<Q>(grad, Q, 0.0f, it.g);
         row_words<Q>(argmax, Q, -1, it.a1);
-        row_words<Q>(argmin, Q, -1, it.a2);
+        if (argmin) row_words<Q>(argmin, Q, -1, it.a2);
         if (x_sel) {
             row_words<Q>(x_sel, Q, 0.0f, it.x1);
             row_words<Q>(x_sel + nm, Q, 0.0f, it.x2);
@@ -355,12 +365,15 @@ __device__ __forceinline__ void load_item(Item<Q> &it, const float *grad, const 
     } else {
         row_words<Q>(grad, left, 0.0f, it.g);
         row_words<Q>(argmax, left, -1, it.a1);
-        row_words<Q>(argmin, left, -1, it.a2);
+        if (argmin) row_words<Q>(argmin, left, -1, it.a2);
         if (x_sel) {
             row_words<Q>(x_sel, left, 0.0f, it.x1);
             row_words<Q>(x_sel + nm, left, 0.0f, it.x2);
         }
     }
+    if (!argmin)
+#pragma unroll
+        for (int u = 0; u < Q; ++u) unpack_picks(it.a1[u], it.a2[u]);
 }
 
 // the inputs picked, without the hand-over: from row xr of x
@@ -519,7 +532,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
         have = tid < items && m0 + r_first < M;
         if (have) {
             const int64_t o = (int64_t)n_first * M + m0 + r_first;
-            load_item(it1, grad + o, argmax + po_first + o, argmin + po_first + o, x_sel ? x_sel + 2 * po_first + o : nullptr, nm, M - m0 - r_first);
+            load_item(it1, grad + o, argmax + po_first + o, argmin ? argmin + po_first + o : nullptr, x_sel ? x_sel + 2 * po_first + o : nullptr, nm, M - m0 - r_first);
         }
     };
     if (first < mtiles) load_first(first * R);
@@ -555,7 +568,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
             const int64_t o = (int64_t)n * M + m0 + r0;
             const int64_t po = (int64_t)(pl_lo + pl) * nm;
             Item<Q> it;
-            load_item(it, grad + o, argmax + po + o, argmin + po + o, x_sel ? x_sel + 2 * po + o : nullptr, nm, M - m0 - r0);
+            load_item(it, grad + o, argmax + po + o, argmin ? argmin + po + o : nullptr, x_sel ? x_sel + 2 * po + o : nullptr, nm, M - m0 - r0);
             if (!x_sel) gather_item(it, x + (int64_t)n * ldx, k0, kn);
             scatter_item<LAYOUT, COUNT>(hist, it, n, r0, k0, kn, kc, log2r, cnt);
             if (sum_bias && pl == 0) {
@@ -650,8 +663,15 @@ __global__ __launch_bounds__(NT_E) void mam_bwd_w_exact_kernel(
     auto load_item = [&](int n) {
         const int64_t o = (int64_t)n * M + m0;
         const float4 g = *reinterpret_cast<const float4 *>(grad + o);
-        const int4 i1 = *reinterpret_cast<const int4 *>(argmax + o);
-        const int4 i2 = *reinterpret_cast<const int4 *>(argmin + o);
+        int4 i1 = *reinterpret_cast<const int4 *>(argmax + o), i2;
+        if (argmin) {
+            i2 = *reinterpret_cast<const int4 *>(argmin + o);
+        } else {
+            unpack_picks(i1.x, i2.x);
+            unpack_picks(i1.y, i2.y);
+            unpack_picks(i1.z, i2.z);
+            unpack_picks(i1.w, i2.w);
+        }
         const float gv[4] = {g.x, g.y, g.z, g.w};
         const int a1[4] = {i1.x - k0, i1.y - k0, i1.z - k0, i1.w - k0};
         const int a2[4] = {i2.x - k0, i2.y - k0, i2.z - k0, i2.w - k0};
@@ -1056,7 +1076,7 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
                          const float *grad, const int32_t *argmax, const int32_t *argmin,
                          const float *w_sel, const float *x_sel, float *x_grad, float *w_grad,
                          int64_t N, int64_t K, int64_t M, int planes, int range_len, void *stream,
-                         mam::bwd::BiasGrad *bias = nullptr)
+                         mam::bwd::BiasGrad *bias = nullptr, bool packed = false)
 {
     using namespace mam;
     if (N < 0 || K < 0 || M < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
@@ -1072,7 +1092,7 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
         if (rc == MAM_OK && w_grad && M > 0) rc = fill_zero(w_grad, M * K, st);
         return rc;
     }
-    if (!x || !w || !grad || !argmax || !argmin) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
+    if (!x || !w || !grad || !argmax || (!argmin && !packed)) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     if (ldx < K || ldw < (w_layout == MAM_W_MK ? K : M))
         return fail(MAM_ERR_INVALID_ARGUMENT, "leading dimension smaller than the row length");
     auto launch = [&](float *xg, float *wg, hipStream_t on) {
@@ -1146,6 +1166,26 @@ extern "C" int mam_fc_backward_bias(const float *x, int64_t ldx, const float *w,
     const int rc = backward_impl(x, ldx, w, ldw, w_layout, grad, argmax, argmin, w_sel, x_sel, x_grad, w_grad, N, K, M,
                                  (int)planes, (int)(range_len > 0 && range_len < K ? range_len : K), stream, &bias);
     if (rc != MAM_OK || bias.done) return rc;
+    return mam_bias_grad(grad, M, bias_grad, N, M, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mam_fc_backward_picks(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, const float *grad,
+                                     const int32_t *picks, const float *w_sel, const float *x_sel, float *x_grad, float *w_grad,
+                                     float *bias_grad, int64_t N, int64_t K, int64_t M, void *workspace, size_t workspace_bytes,
+                                     void *stream)
+{
+    using namespace mam;
+    if (K > MOST_PACKED_K) return fail(MAM_ERR_UNSUPPORTED, "K = %lld: two indices do not fit a word", (long long)K);
+    bwd::BiasGrad bias = {bias_grad, static_cast<float *>(workspace), 0, false};
+    if (bias_grad) {
+        const size_t need = mam_fc_backward_bias_workspace(N, K, M);
+        if (need > 0 && (!workspace || workspace_bytes < need))
+            return fail(MAM_ERR_WORKSPACE, "the bias gradient needs %zu workspace bytes, got %zu", need, workspace ? workspace_bytes : (size_t)0);
+        if (workspace && N > 0 && M > 0) bias.partials = (int64_t)(workspace_bytes / ((size_t)M * sizeof(float)));
+    }
+    const int rc = backward_impl(x, ldx, w, ldw, w_layout, grad, picks, nullptr, w_sel, x_sel, x_grad, w_grad, N, K, M, 1, (int)K, stream,
+                                 bias_grad ? &bias : nullptr, true);
+    if (rc != MAM_OK || !bias_grad || bias.done) return rc;
     return mam_bias_grad(grad, M, bias_grad, N, M, workspace, workspace_bytes, stream);
 }
 

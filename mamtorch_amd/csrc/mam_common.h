@@ -96,6 +96,16 @@ __device__ __forceinline__ float load_w(const float *__restrict__ w, int64_t ldw
     return LAYOUT == MAM_W_MK ? w[m * ldw + k] : w[k * ldw + m];
 }
 
+// Both picks of an output in one word (argmin == nullptr, K at most 65535): what a backward reads of the indices, at half the
+// planes.  The word of an output that is not there, -1, is a pick that no K has.
+constexpr int64_t MOST_PACKED_K = 65535;
+__device__ __forceinline__ int32_t pack_picks(int hi, int lo) { return (int32_t)((uint32_t)hi | (uint32_t)lo << 16); }
+__device__ __forceinline__ void unpack_picks(int32_t &a1, int32_t &a2)
+{
+    a2 = (int32_t)((uint32_t)a1 >> 16);
+    a1 &= 0xffff;
+}
+
 // Q consecutive words of a row of which `left` are left: one load where there are Q, of 4-byte aligned addresses (what a load
 // of several words needs), so that neither the number of neurons nor an operand's alignment takes a call off the kernels that read
 // several words a lane; past the end of the row `none`.

@@ -61,7 +61,7 @@ struct Params {
     const float *bias;
     float *c;
     int32_t *argmax;
-    int32_t *argmin;
+    int32_t *argmin;  // nullptr: argmax holds both, packed (pack_picks)
     float *wsel;      // optional [2][N*M]: the selected weights w[argmax], w[argmin] (for the backward)
     float *xsel;      // optional [2][N*M]: the selected inputs x[argmax], x[argmin] (for the backward)
     float *part;      // split-K partials: [split][3 or 2][N*M]: max, min, (group ids packed 16:16)
@@ -166,8 +166,12 @@ __device__ __forceinline__ void finish(const Params &p, int n, int m, float vmax
     const int64_t o = (int64_t)n * p.M + m;
     p.c[o] = s;
     if (ARGS) {
-        p.argmax[o] = ih;
-        p.argmin[o] = il;
+        if (p.argmin) {
+            p.argmax[o] = ih;
+            p.argmin[o] = il;
+        } else {
+            p.argmax[o] = pack_picks(ih, il);
+        }
         if (p.wsel) {
             p.wsel[o] = wh;
             p.wsel[(int64_t)p.N * p.M + o] = wl;
@@ -293,8 +297,12 @@ __device__ __forceinline__ void resolve_wave(const Params &p, const float *vals,
     if (valid) {
         const int64_t o = (int64_t)n * p.M + m;
         p.c[o] = sum;
-        p.argmax[o] = res_i[lane];
-        p.argmin[o] = res_i[64 + lane];
+        if (p.argmin) {
+            p.argmax[o] = res_i[lane];
+            p.argmin[o] = res_i[64 + lane];
+        } else {
+            p.argmax[o] = pack_picks(res_i[lane], res_i[64 + lane]);
+        }
         if (p.wsel) {
             p.wsel[o] = res_w[lane];
             p.wsel[(int64_t)p.N * p.M + o] = res_w[64 + lane];
@@ -1517,13 +1525,13 @@ template <bool ARGS>
 static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                   const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel, float *x_sel,
                   int64_t N, int64_t K, int64_t M, void *workspace, size_t workspace_size, void *stream,
-                  bool static_scratch = false, int64_t range_len = 0)
+                  bool static_scratch = false, int64_t range_len = 0, bool packed = false)
 {
     Plan plan;
     int rc = make_plan(plan, ARGS, x, ldx, w, ldw, w_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M,
                        range_len);
     if (rc != MAM_OK || N == 0 || M == 0) return rc;
-    if (!x || !w || !c || (ARGS && (!argmax || !argmin)))
+    if (!x || !w || !c || (ARGS && (!argmax || (!argmin && !packed))))
         return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
     const size_t avail = static_scratch ? static_scratch_bytes() : (workspace ? workspace_size : (size_t)0);
     // Large calls go by magnitude-ordered lists where the workspace has room for them (the kernels below then run only if
@@ -1787,6 +1795,15 @@ extern "C" int mam_fc_forward(const float *x, int64_t ldx, const float *w, int64
 {
     return mam::fwd::launch<true>(x, ldx, w, ldw, w_layout, bias, c, argmax, argmin, w_sel, x_sel, N, K, M,
                                   workspace, workspace_bytes, stream);
+}
+
+extern "C" int mam_fc_forward_picks(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, const float *bias, float *c,
+                                    int32_t *picks, float *w_sel, float *x_sel, int64_t N, int64_t K, int64_t M, void *workspace,
+                                    size_t workspace_bytes, void *stream)
+{
+    if (K > mam::MOST_PACKED_K) return mam::fail(MAM_ERR_UNSUPPORTED, "K = %lld: two indices do not fit a word", (long long)K);
+    return mam::fwd::launch<true>(x, ldx, w, ldw, w_layout, bias, c, picks, nullptr, w_sel, x_sel, N, K, M, workspace, workspace_bytes, stream,
+                                  false, 0, true);
 }
 
 extern "C" int mam_fc_forward_values(const float *x, int64_t ldx, const float *w, int64_t ldw,

@@ -23,7 +23,7 @@ struct Call {
     const float *x; int64_t ldx;
     const float *w; int64_t ldw; int w_layout;
     const float *bias;
-    float *c; int32_t *argmax, *argmin;      // argmax == nullptr: values only
+    float *c; int32_t *argmax, *argmin;      // argmax == nullptr: values only; argmin == nullptr: both packed in argmax
     float *wsel, *xsel;
     int64_t N, K, M;
 };

@@ -1375,6 +1375,12 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                 }
             };
             if constexpr (ARGS) {
+                if (!c.argmin) {
+                    float both[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) both[j] = __int_as_float(pack_picks(index_in(key_of(e.mx[j])), index_in(key_of(e.mn[j]))));
+                    put(reinterpret_cast<float *>(c.argmax), both);
+                }
 #pragma unroll
                 for (int side2 = 0; side2 < 2; ++side2) {
                     uint32_t kk[4];
@@ -1384,7 +1390,7 @@ __global__ __launch_bounds__(NT) void forward_kernel(const Params p)
                         kk[j] = key_of(side2 ? e.mn[j] : e.mx[j]);
                         f[j] = __int_as_float(index_in(kk[j]));
                     }
-                    put(reinterpret_cast<float *>(side2 ? c.argmin : c.argmax), f);
+                    if (c.argmin) put(reinterpret_cast<float *>(side2 ? c.argmin : c.argmax), f);
                     if (c.wsel || c.xsel) {
                         // the selected operands, of the tile and of the listed row: from the list, which this
                         // XCD's L2 still holds, rather than from anywhere in the row (16384 x 4096 -> 1024: 593 ->

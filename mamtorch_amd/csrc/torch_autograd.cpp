@@ -370,6 +370,51 @@ Tensor col2im(const Tensor &cols, int64_t B, int64_t C, int64_t H, int64_t W, in
     return col2im_op().call(cols, B, C, H, W, k1, k2, s1, s2);
 }
 
+// ---- fullyconnected_wt_picks(a, weight, bias) -> [C, picks, sel] ----
+Tensors picks_below(const Tensor &a, const Tensor &weight, const MaybeTensor &bias)
+{
+    static const auto op = find<Tensors(const Tensor &, const Tensor &, const MaybeTensor &)>(
+        "mamtorch_kernel_v4::fullyconnected_wt_picks");
+    at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(a, weight, bias);
+}
+
+struct Picks : public Function<Picks> {
+    static variable_list forward(AutogradContext *ctx, const Tensor &a, const Tensor &weight, const MaybeTensor &bias)
+    {
+        Tensors out = picks_below(a, weight, bias);
+        const bool operands = a.requires_grad() || weight.requires_grad();
+        ctx->saved_data["operands"] = operands;
+        ctx->saved_data["bias"] = bias.has_value() && bias->defined() && bias->requires_grad();
+        if (operands) ctx->save_for_backward({a, weight, out[1], out[2]});
+        ctx->mark_non_differentiable({out[1], out[2]});
+        ctx->set_materialize_grads(false);
+        return out;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list grads)
+    {
+        static const auto op = find<Tensors(const Tensor &, const Tensor &, const Tensor &, const Tensor &, const Tensor &, bool)>(
+            "mamtorch_kernel_v4::fullyconnected_wt_picks_backward");
+        variable_list out(3);
+        const Tensor &g = grads[0];
+        if (!g.defined()) return out;
+        const bool bias = ctx->saved_data["bias"].toBool();
+        if (ctx->saved_data["operands"].toBool()) {
+            const variable_list s = ctx->get_saved_variables();
+            const Tensors all = op.call(s[0], s[1], g.contiguous(), s[2], s[3], bias);
+            for (size_t i = 0; i < all.size(); ++i) out[i] = all[i];
+        } else if (bias) {
+            out[2] = bias_grad(g);
+        }
+        return out;
+    }
+};
+
+Tensors fullyconnected_wt_picks(const Tensor &a, const Tensor &weight, const MaybeTensor &bias)
+{
+    return recording(a, weight, bias) ? Picks::apply(a, weight, bias) : picks_below(a, weight, bias);
+}
+
 Tensors exact_v1(Tensor a, Tensor b) { return exact<V1>(a, b); }
 Tensors exact_v4(Tensor a, Tensor b) { return exact<V4>(a, b); }
 Tensor fast_v4(Tensor a, Tensor b) { return fullyconnected_fast(a, b); }
@@ -383,6 +428,7 @@ TORCH_LIBRARY_IMPL(mamtorch_kernel_v4, Autograd, m)
     m.impl("fullyconnected", &exact_v4);
     m.impl("fullyconnected_fast", &fast_v4);
     m.impl("fullyconnected_wt", &fullyconnected_wt);
+    m.impl("fullyconnected_wt_picks", &fullyconnected_wt_picks);
     m.impl("fullyconnected_fast_wt", &fullyconnected_fast_wt);
     m.impl("fullyconnected_ranges", &fullyconnected_ranges);
     m.impl("blend", &blend);

@@ -228,6 +228,54 @@ std::vector<at::Tensor> fullyconnected_wt(const at::Tensor &a, const at::Tensor 
     return forward_impl(a, weight, MAM_W_MK, bias, true, hand_over);
 }
 
+// For a backward that is all that reads the indices: [C, picks, sel], both indices of an output in one word.
+std::vector<at::Tensor> fullyconnected_wt_picks(const at::Tensor &a, const at::Tensor &weight,
+                                                const c10::optional<at::Tensor> &bias)
+{
+    const FwdShape s = check_forward(a, weight, MAM_W_MK, bias);
+    const c10::DeviceGuard guard(a.device());
+    auto c = at::empty({s.N, s.M}, a.options());
+    auto picks = at::empty({s.N, s.M}, a.options().dtype(at::kInt));
+    auto sel = at::empty({4, s.N, s.M}, a.options());
+    if (s.N == 0 || s.M == 0) return {c, picks, sel};
+    auto ws = forward_workspace(s, MAM_W_MK, true, a);
+    float *w_sel = sel.data_ptr<float>();
+    check_rc(mam_fc_forward_picks(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
+                                  row_stride(weight, "the weight operand"), MAM_W_MK, bias_ptr(bias), c.data_ptr<float>(),
+                                  picks.data_ptr<int32_t>(), w_sel, w_sel + 2 * s.N * s.M, s.N, s.K, s.M,
+                                  ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, current_stream(a)),
+             "mam_fc_forward_picks");
+    return {c, picks, sel};
+}
+
+std::vector<at::Tensor> fullyconnected_wt_picks_backward(const at::Tensor &a, const at::Tensor &weight, const at::Tensor &grad,
+                                                         const at::Tensor &picks, const at::Tensor &sel, bool with_bias)
+{
+    const FwdShape s = check_forward(a, weight, MAM_W_MK, c10::nullopt);
+    check_f32_2d(grad, "grad");
+    TORCH_CHECK(grad.size(0) == s.N && grad.size(1) == s.M, "grad must be (batch, out_features)");
+    check_same_device(a, grad, "grad");
+    check_index(picks, grad, "picks");
+    TORCH_CHECK(sel.is_cuda() && sel.scalar_type() == at::kFloat && sel.is_contiguous() && sel.dim() == 3 && sel.size(0) == 4 &&
+                    sel.size(1) == s.N && sel.size(2) == s.M,
+                "sel must be a contiguous float32 GPU tensor of shape (4, batch, out_features)");
+    check_same_device(a, sel, "sel");
+    const c10::DeviceGuard guard(a.device());
+    const at::Tensor g = grad.contiguous();
+    std::vector<at::Tensor> out = {at::empty({s.N, s.K}, a.options()), at::empty(weight.sizes(), weight.options())};
+    if (with_bias) out.push_back(at::empty({s.M}, a.options()));
+    const size_t ws_bytes = with_bias ? mam_fc_backward_bias_workspace(s.N, s.K, s.M) : 0;
+    auto ws = workspace_for(ws_bytes, a);
+    const float *w_sel = sel.data_ptr<float>();
+    check_rc(mam_fc_backward_picks(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
+                                   row_stride(weight, "the weight operand"), MAM_W_MK, g.data_ptr<float>(), picks.data_ptr<int32_t>(),
+                                   w_sel, w_sel + 2 * s.N * s.M, out[0].data_ptr<float>(), out[1].data_ptr<float>(),
+                                   with_bias ? out[2].data_ptr<float>() : nullptr, s.N, s.K, s.M,
+                                   ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
+             "mam_fc_backward_picks");
+    return out;
+}
+
 at::Tensor fullyconnected_fast_wt(const at::Tensor &a, const at::Tensor &weight,
                                   const c10::optional<at::Tensor> &bias)
 {
@@ -649,6 +697,8 @@ TORCH_LIBRARY(mamtorch_kernel_v4, m)
     m.def("fullyconnected_fast(Tensor a, Tensor b) -> Tensor");
     m.def("fullyconnected_backward(Tensor a, Tensor b, Tensor grad, Tensor argmax, Tensor argmin) -> Tensor[]");
     m.def("fullyconnected_wt(Tensor a, Tensor weight, Tensor? bias, bool hand_over) -> Tensor[]");
+    m.def("fullyconnected_wt_picks(Tensor a, Tensor weight, Tensor? bias) -> Tensor[]");
+    m.def("fullyconnected_wt_picks_backward(Tensor a, Tensor weight, Tensor grad, Tensor picks, Tensor sel, bool with_bias) -> Tensor[]");
     m.def("fullyconnected_fast_wt(Tensor a, Tensor weight, Tensor? bias) -> Tensor");
     m.def("fullyconnected_wt_backward(Tensor a, Tensor weight, Tensor grad, Tensor argmax, Tensor argmin, Tensor? sel) -> Tensor[]");
     m.def("fullyconnected_wt_backward_bias(Tensor a, Tensor weight, Tensor grad, Tensor argmax, Tensor argmin, Tensor? sel) -> Tensor[]");
@@ -685,6 +735,8 @@ TORCH_LIBRARY_IMPL(mamtorch_kernel_v4, CUDA, m)
     m.impl("fullyconnected_fast", &fullyconnected_fast);
     m.impl("fullyconnected_backward", &fullyconnected_backward);
     m.impl("fullyconnected_wt", &fullyconnected_wt);
+    m.impl("fullyconnected_wt_picks", &fullyconnected_wt_picks);
+    m.impl("fullyconnected_wt_picks_backward", &fullyconnected_wt_picks_backward);
     m.impl("fullyconnected_fast_wt", &fullyconnected_fast_wt);
     m.impl("fullyconnected_wt_backward", &fullyconnected_wt_backward);
     m.impl("fullyconnected_wt_backward_bias", &fullyconnected_wt_backward_bias);

@@ -161,7 +161,7 @@ class FullyConnected(Module):
     def _mam_noargs(self, x: Tensor, w: Tensor, bias) -> Tensor:
         if self.beta < 1:
             if self.training:
-                return K.v4.fullyconnected_wt(x, w, bias)[0]
+                return K.v4.fullyconnected_wt_output(x, w, bias)
             return K.v4.fullyconnected_fast_wt(x, w, bias)
         return torch.zeros((x.shape[0], w.shape[0]), device=w.device, dtype=w.dtype)
 

@@ -533,3 +533,51 @@ def test_rows_of_any_length_at_any_word(shape):
     assert (np.abs(wg.cpu().numpy() - wo) <= RTOL * np.abs(wo) + FLOOR * ws + 1e-30).all()
     gd = grad.double()
     assert ((bg.cpu().double() - gd.sum(0)).abs() <= RTOL * gd.sum(0).abs() + FLOOR * gd.abs().sum(0) + 1e-30).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1), (33, 100, 70), (64, 784, 256), (130, 1001, 65), (2051, 130, 3), (2100, 70, 83), (300, 65535, 5),
+                                   (300, 4096, 4096), (12, 3000, 130)])
+@pytest.mark.parametrize("layout", ["MK", "KM"])
+@pytest.mark.parametrize("tiling", ["AUTO", "WIDE", "DENSE", "LISTS"])
+def test_both_picks_in_one_word(shape, layout, tiling):
+    """Picks and gradients of the packed form against the two index arrays: the same selections, outputs, exact gradients bit for bit; the weight
+    gradient (its adds in any order) within the floor of such sums."""
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    N, K, M = shape
+    x, w, grad = random_case(N, K, M, seed=N + K)
+    lay = capi.W_MK if layout == "MK" else capi.W_KM
+    xd, gd = x.to(dev), grad.to(dev)
+    wd = (w if layout == "MK" else w.T).contiguous().to(dev)
+    bias = torch.randn(M, device=dev)
+    capi.set_option(capi.OPT_FORWARD_TILING, getattr(capi, "FORWARD_TILING_" + tiling))
+    try:
+        sel = [torch.empty((2, N, M), device=dev) for _ in range(4)]
+        c, amax, amin = capi.fc_forward(xd, wd, lay, bias, None, sel[0], sel[1])
+        c2, picks = capi.fc_forward_picks(xd, wd, lay, bias, sel[2], sel[3])
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    assert torch.equal(c.view(torch.int32), c2.view(torch.int32))
+    assert torch.equal(picks & 0xFFFF, amax) and torch.equal((picks >> 16) & 0xFFFF, amin)
+    for a, b in zip(sel[:2], sel[2:]):
+        assert torch.equal(a.view(torch.int32), b.view(torch.int32))
+    for handed in ((sel[0], sel[1]), (None, None)):
+        xg, wg, bg = capi.fc_backward_bias(xd, wd, gd, amax, amin, lay, *handed)
+        xg2, wg2, bg2 = capi.fc_backward_picks(xd, wd, gd, picks, lay, *handed, with_bias=True)
+        _, wabs = capi.fc_backward(xd.abs(), wd.abs(), gd.abs(), amax, amin, lay)
+        assert torch.equal(xg, xg2) and torch.equal(bg, bg2)
+        assert ((wg - wg2).abs() <= RTOL * wg.abs() + FLOOR * wabs + 1e-30).all()
+        _, _, none = capi.fc_backward_picks(xd, wd, gd, picks, lay, *handed)
+        assert none is None
+
+
+def test_indices_that_do_not_fit_a_word_are_refused():
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    x, w, g = torch.randn(2, 65536, device=dev), torch.randn(3, 65536, device=dev), torch.randn(2, 3, device=dev)
+    with pytest.raises(RuntimeError):
+        capi.fc_forward_picks(x, w, capi.W_MK)
+    with pytest.raises(RuntimeError):
+        capi.fc_backward_picks(x, w, g, torch.zeros(2, 3, dtype=torch.int32, device=dev), capi.W_MK)

@@ -63,6 +63,10 @@ def test_opcheck():
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected, (a, b), test_utils=tests)
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_fast, (a, b), test_utils=tests)
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_wt, (a, wt, bias, True), test_utils=tests)
+    torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_wt_picks, (a, wt, bias), test_utils=tests)
+    _, picks, sel = torch.ops.mamtorch_kernel_v4.fullyconnected_wt_picks(a.detach(), wt.detach(), bias.detach())
+    torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_wt_picks_backward,
+                          (a.detach(), wt.detach(), grad.to(DEV), picks, sel, True), test_utils=("test_schema", "test_faketensor"))
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_fast_wt, (a, wt, None), test_utils=tests)
     _, amax, amin = torch.ops.mamtorch_kernel_v4.fullyconnected(a.detach(), b.detach())
     torch.library.opcheck(torch.ops.mamtorch_kernel_v4.fullyconnected_backward,
