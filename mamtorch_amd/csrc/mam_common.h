@@ -48,8 +48,11 @@ int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t co
 // range_len > 0: rows are consecutive ranges of range_len (the last one shorter), of which each is lengthened to ld_dst / their number
 // (a multiple of 4).
 struct LengthenRows { const float *src; int64_t ld; float *dst; int rows; };
-int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, int64_t range_len, hipStream_t stream,
-                  const ordered::Guard *guard = nullptr);
+// Other ends, of ranges of at least 64: tiles of 64, the last one of which holds the range's last 64; the range, then (64 before
+// its copy's end) its last 64 once more.
+enum RowsEnd { ROWS_REPEAT_LAST, ROWS_END_WHOLE_TILES, ROWS_AND_LAST_64 };
+int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, int64_t range_len, RowsEnd end,
+                  hipStream_t stream, const ordered::Guard *guard = nullptr);
 
 // Two independent kernels of one call side by side: the first runs on a second stream of the library
 // (default priority, one per device) between a fork and a join event on the caller's stream.

@@ -102,10 +102,10 @@ int transpose(const float *src, int64_t ld, float *dst, int64_t rows, int64_t co
     return check_launch("transpose_kernel");
 }
 
-// Two matrices copied with their rows lengthened: row r of dst is row r of src, then its last element up to ld_dst.
+// Two matrices copied with their rows lengthened (see RowsEnd).
 // Bound by memory; a workgroup takes 1024 consecutive floats of a row.
 __global__ __launch_bounds__(256) void lengthen_rows_kernel(const LengthenRows a, const LengthenRows b, int cols, int ld_dst, int range_len,
-                                                            int longer, const ordered::Guard guard)
+                                                            int longer, RowsEnd end, const ordered::Guard guard)
 {
     if (ordered::guarded_off(guard)) return;
     const bool first = (int)blockIdx.y < a.rows;
@@ -113,9 +113,12 @@ __global__ __launch_bounds__(256) void lengthen_rows_kernel(const LengthenRows a
     const int64_t row = first ? blockIdx.y : blockIdx.y - a.rows;
     const int c = (blockIdx.x * 256 + threadIdx.x) * 4;
     if (c >= ld_dst) return;
-    const int range = c / longer, first_k = range * range_len, k = first_k + (c - range * longer);
+    const int range = c / longer, first_k = range * range_len, in_range = c - range * longer;
     const float *src = m.src + row * m.ld;
     const int last = (cols - first_k < range_len ? cols : first_k + range_len) - 1;
+    // from where on the last 64 stand
+    const int tail = end == ROWS_END_WHOLE_TILES ? (last - first_k) / 64 * 64 : end == ROWS_AND_LAST_64 ? longer - 64 : longer;
+    const int k = in_range < tail ? first_k + in_range : last - 63 + in_range - tail;
     float4 v;
     v.x = src[k < last ? k : last];
     v.y = src[k + 1 < last ? k + 1 : last];
@@ -124,14 +127,14 @@ __global__ __launch_bounds__(256) void lengthen_rows_kernel(const LengthenRows a
     *reinterpret_cast<float4 *>(m.dst + row * ld_dst + c) = v;
 }
 
-int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, int64_t range_len, hipStream_t stream,
-                  const ordered::Guard *guard)
+int lengthen_rows(const LengthenRows &a, const LengthenRows &b, int64_t cols, int64_t ld_dst, int64_t range_len, RowsEnd end,
+                  hipStream_t stream, const ordered::Guard *guard)
 {
     if (a.rows + b.rows == 0) return MAM_OK;
     if (range_len <= 0 || range_len > cols) range_len = cols;
     const int64_t longer = ld_dst / ceil_div(cols, range_len);
     hipLaunchKernelGGL(lengthen_rows_kernel, dim3((unsigned)ceil_div(ld_dst, 1024), (unsigned)(a.rows + b.rows)), dim3(256), 0,
-                       stream, a, b, (int)cols, (int)ld_dst, (int)range_len, (int)longer, guard ? *guard : ordered::Guard{nullptr});
+                       stream, a, b, (int)cols, (int)ld_dst, (int)range_len, (int)longer, end, guard ? *guard : ordered::Guard{nullptr});
     return check_launch("lengthen_rows_kernel");
 }
 

@@ -52,6 +52,7 @@ constexpr int TJ = 8;         // columns per thread
 constexpr int NT = 256;       // threads per workgroup
 constexpr int GROUP_N = 8;    // row tiles swept together so that W panels are reused from L2
 constexpr int MAX_SPLITS = 16;
+namespace sx { constexpr int KT = 64; }   // k extent of one W tile of the wave-uniform-rows tiling (further down)
 
 struct Params {
     const float *x;
@@ -75,6 +76,10 @@ struct Params {
     ordered::Guard guard;   // the kernels exit at once where the lists serve the call (mam_ordered.hip)
     int gt;            // products per recorded group: G, or 2 G on the wave-uniform-rows tiling at large K
     int range_len;     // ranges of the caller's that were lengthened to k_per_split: their length (indices count in it)
+    int ragged;        // wave-uniform rows, x as it is: the last k tile of a range ends where the range ends (see walked)
+    int own_ranges;    // the K ranges are the caller's
+    int w_step;        // columns of w from one of them to the next (k_per_split, more in a copy)
+    int w_tail;        // values only, w copied: column at which the last 64 of the (first) range stand once more, aligned; else -1
 };
 
 // An extreme that still holds its initial value (-inf for the max, +inf for the min) was never strictly
@@ -84,6 +89,16 @@ struct Params {
 __device__ __forceinline__ bool never_improved(float target, bool is_min)
 {
     return target == (is_min ? __builtin_inff() : -__builtin_inff());
+}
+
+// A ragged range of K (at least 64 long) is walked in tiles of 64 of which the last one begins 64 before the range's end, inside the
+// tile before it: what it repeats never wins a strict comparison, so neither operand has to be padded, and x, which a call has N
+// rows of, is not copied.  Where the k-th product of the walk stands in a range of `length`:
+// (43120 x 1300 -> 42 with indices: 120 us of copies beside 310 us of kernel; 10233 x 3316 -> 78 51 beside 246.)
+__device__ __forceinline__ int walked(int k, int length)
+{
+    const int last = length - sx::KT + (k & (sx::KT - 1));
+    return k < last ? k : last;
 }
 
 // First k in group g (ascending) whose product equals `target`; value recomputed from it.
@@ -192,7 +207,7 @@ __device__ __forceinline__ void finish(const Params &p, int n, int m, float vmax
 // consecutive slots are consecutive neurons.  128 tasks (64 outputs x {max, min}), 64/(G/4) per
 // round.
 //   vals : LDS, [2][64]  running max, running min of the wave's outputs
-//   grps : LDS, [2][64]  absolute group id of the max, of the min
+//   grps : LDS, [2][64]  first k of the group of the max, of the min, as the k loop walked it
 //   res  : LDS, [8][64]  scratch of this wave: value, index, weight, input of the max and of the min
 //   nm_of(slot, n, m, valid): output coordinates of slot 0..63 (clamped into range when !valid)
 constexpr int LPT = G / 4;             // lanes per task
@@ -213,10 +228,11 @@ __device__ __forceinline__ int quad_min(int v)
 //   operands(r, slot, sub, kb, xp, wp): where the GT/4 x and GT/4 w operands k = kb .. kb+GT/4-1 of the task in
 //   round r live.  The addresses are most of the instructions of a round when they are formed in 64 bits per
 //   lane, so a caller whose 64 outputs share bases hands in something cheaper.
+//   at(k): where product k of the walk stands in x.
 //   GT: the k loop's tracking span, 16 or 32 products per recorded group; a lane takes GT/4 of them (one or two
 //   16-byte loads per operand), and the loads of 8 * 16 / GT rounds are in flight together.
-template <int GT, class OP>
-__device__ __forceinline__ void resolve_tasks(const float *vals, const int *grps, float *res, int lane, OP operands)
+template <int GT, class OP, class AT>
+__device__ __forceinline__ void resolve_tasks(const float *vals, const int *grps, float *res, int lane, OP operands, AT at)
 {
     static_assert(GT == 16 || GT == 32, "tracking span");
     constexpr int PPL = GT / LPT;             // products per lane
@@ -240,10 +256,11 @@ __device__ __forceinline__ void resolve_tasks(const float *vals, const int *grps
             target[b] = vals[ext * 64 + slot];
             grp[b] = grps[ext * 64 + slot];
             const float *xp, *wp;
-            operands(r, slot, sub, grp[b] * GT + sub * PPL, xp, wp);
+            operands(r, slot, sub, grp[b] + sub * PPL, xp, wp);
 #pragma unroll
             for (int v = 0; v < NV; ++v) {
-                xa[b][v] = reinterpret_cast<const float4 *>(xp)[v];
+                const floats4 xq = reinterpret_cast<const floats4 *>(xp)[v];       // (ragged rows: 4-byte aligned)
+                xa[b][v] = make_float4(xq.x, xq.y, xq.z, xq.w);
                 wa[b][v] = reinterpret_cast<const float4 *>(wp)[v];
             }
         }
@@ -273,7 +290,7 @@ __device__ __forceinline__ void resolve_tasks(const float *vals, const int *grps
             if ((key == best && key != 255) || fallback) {
                 // the value is recomputed from the selected operands (the sign of a zero follows them)
                 res_v[ext * 64 + slot] = fallback ? target[b] : xsel * wsel;
-                res_i[ext * 64 + slot] = grp[b] * GT + (fallback ? 0 : key);
+                res_i[ext * 64 + slot] = at(grp[b] + (fallback ? 0 : key));
                 res_w[ext * 64 + slot] = wsel;
                 res_x[ext * 64 + slot] = xsel;
             }
@@ -281,11 +298,11 @@ __device__ __forceinline__ void resolve_tasks(const float *vals, const int *grps
     }
 }
 
-template <int GT, class NM, class OP>
+template <int GT, bool RAGGED = false, class NM, class OP>
 __device__ __forceinline__ void resolve_wave(const Params &p, const float *vals, const int *grps, float *res,
                                              int lane, NM nm_of, OP operands)
 {
-    resolve_tasks<GT>(vals, grps, res, lane, operands);
+    resolve_tasks<GT>(vals, grps, res, lane, operands, [&](int k) { return RAGGED ? walked(k, p.K) : k; });
     const float *res_v = res, *res_w = res + 256, *res_x = res + 384;
     const int *res_i = reinterpret_cast<const int *>(res + 128);
     // lane s finishes output s
@@ -637,8 +654,8 @@ __global__ __launch_bounds__(NT, 2) void mam_fwd_kernel(const Params p)
             for (int j = 0; j < TJ; ++j) {
                 vals[(j * 2 + 0) * 64 + lane] = vmax[i][j];
                 vals[(j * 2 + 1) * 64 + lane] = vmin[i][j];
-                grps[(j * 2 + 0) * 64 + lane] = g0 + gmax[i][j];
-                grps[(j * 2 + 1) * 64 + lane] = g0 + gmin[i][j];
+                grps[(j * 2 + 0) * 64 + lane] = (g0 + gmax[i][j]) * G;
+                grps[(j * 2 + 1) * 64 + lane] = (g0 + gmin[i][j]) * G;
             }
             __builtin_amdgcn_wave_barrier();
 #pragma unroll 1
@@ -701,7 +718,7 @@ __global__ __launch_bounds__(NT, 2) void mam_fwd_kernel(const Params p)
 
 // Combines split-K partials in ascending k order (strict comparisons keep the earliest
 // group on ties), then resolves indices / zero signs exactly as the single-pass epilogue.
-template <int LAYOUT, bool ARGS, bool COOP, int GT = G>
+template <int LAYOUT, bool ARGS, bool COOP, int GT = G, bool RAGGED = false>
 __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
 {
     // (the arguments of the prologue in one fetch with the guard's, not in a second one behind its branch)
@@ -755,8 +772,8 @@ __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
         const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         vals_s[wave][0][lane] = vmax;
         vals_s[wave][1][lane] = vmin;
-        grps_s[wave][0][lane] = gmax;
-        grps_s[wave][1][lane] = gmin;
+        grps_s[wave][0][lane] = gmax * GT;
+        grps_s[wave][1][lane] = gmin * GT;
         __syncthreads();
         const int nbase = pn * PR + (PR / 4) * wave, mbase = pm * PC;
         // slot = 8 r + lane / 8 in round r: batch row nbase + slot / PC (the same for the whole wave) and
@@ -767,7 +784,7 @@ __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
         const uint32_t ldw4 = (uint32_t)p.ldw * 4u;
         const uint32_t last = last_row_offset(p.M, mb, PC, ldw4);
         const uint32_t mine = (uint32_t)(lane >> 3) * ldw4;
-        resolve_wave<GT>(p, &vals_s[wave][0][0], &grps_s[wave][0][0], &res_s[wave][0], lane,
+        resolve_wave<GT, RAGGED>(p, &vals_s[wave][0][0], &grps_s[wave][0][0], &res_s[wave][0], lane,
                      [&](int slot, int &n, int &m, bool &valid) {
                          n = nbase + (slot >> LOG2PC);
                          m = mbase + (slot & (PC - 1));
@@ -781,7 +798,7 @@ __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
                          const char *xrow = reinterpret_cast<const char *>(p.x + (int64_t)n * p.ldx);
                          const uint32_t row = mine + (uint32_t)(8 * (r & (PC / 8 - 1))) * ldw4;
                          const uint32_t k4 = (uint32_t)kb * 4u;
-                         xp = reinterpret_cast<const float *>(xrow + k4);
+                         xp = reinterpret_cast<const float *>(xrow + (RAGGED ? (uint32_t)walked(kb, p.K) * 4u : k4));
                          wp = reinterpret_cast<const float *>(wrows + (clamped_row_offset(row, last) + k4));
                      });
     } else if (live) {
@@ -800,7 +817,7 @@ __global__ __launch_bounds__(256) void mam_fwd_merge_kernel(const Params p)
 // [range][N*M] planes of ABSOLUTE k.
 // COOP: with indices on operands that the cooperative resolve takes, range after range, patches as in mam_fwd_merge_kernel (a
 // resolve per lane walks two lines an output and range on its own).
-template <int LAYOUT, bool ARGS, bool COOP>
+template <int LAYOUT, bool ARGS, bool COOP, bool RAGGED = false>
 __global__ __launch_bounds__(256) void mam_fwd_range_sum_kernel(const Params p)
 {
     const int64_t nm = (int64_t)p.N * p.M;
@@ -824,25 +841,28 @@ __global__ __launch_bounds__(256) void mam_fwd_range_sum_kernel(const Params p)
         float total = 0.0f;
         for (int s = 0; s < p.splits; ++s) {
             const float *base = p.part + (int64_t)s * 3 * nm;
-            const int kb = s * p.k_per_split, g0 = kb / G, pk = __float_as_int(base[2 * nm + o]);
+            const int kb = s * p.k_per_split, pk = __float_as_int(base[2 * nm + o]);
+            const int length = p.K - kb < p.k_per_split ? p.K - kb : p.k_per_split;
+            const char *const xrange = xrow + (int64_t)kb * (int64_t)sizeof(float), *const wrange = wrows + (int64_t)s * p.w_step * (int64_t)sizeof(float);
             vals_s[wave][0][lane] = base[o];
             vals_s[wave][1][lane] = base[nm + o];
-            grps_s[wave][0][lane] = g0 + (pk & 0xffff);
-            grps_s[wave][1][lane] = g0 + ((pk >> 16) & 0xffff);
+            grps_s[wave][0][lane] = (pk & 0xffff) * G;
+            grps_s[wave][1][lane] = ((pk >> 16) & 0xffff) * G;
             __syncthreads();
             resolve_tasks<G>(&vals_s[wave][0][0], &grps_s[wave][0][0], &res_s[wave][0], lane,
                              [&](int r, int, int, int k, const float *&xp, const float *&wp) {
                                  const uint32_t row = mine + (uint32_t)(8 * (r & (PC / 8 - 1))) * ldw4, k4 = (uint32_t)k * 4u;
-                                 xp = reinterpret_cast<const float *>(xrow + k4);
-                                 wp = reinterpret_cast<const float *>(wrows + (clamped_row_offset(row, last) + k4));
-                             });
+                                 xp = reinterpret_cast<const float *>(xrange + (RAGGED ? (uint32_t)walked(k, length) * 4u : k4));
+                                 wp = reinterpret_cast<const float *>(wrange + (clamped_row_offset(row, last) + k4));
+                             },
+                             [&](int k) { return RAGGED ? walked(k, length) : k; });
             __syncthreads();
             const float v = res_v[lane] + res_v[64 + lane];
             total = s == 0 ? v : total + v;
             if (live) {
-                const int shift = p.range_len > 0 ? s * p.range_len - kb : 0;
-                p.argmax[(int64_t)s * nm + o] = res_i[lane] + shift;
-                p.argmin[(int64_t)s * nm + o] = res_i[64 + lane] + shift;
+                const int first = p.range_len > 0 ? s * p.range_len : kb;
+                p.argmax[(int64_t)s * nm + o] = res_i[lane] + first;
+                p.argmin[(int64_t)s * nm + o] = res_i[64 + lane] + first;
             }
         }
         if (live) p.c[o] = p.bias ? total + p.bias[m] : total;
@@ -871,8 +891,9 @@ __global__ __launch_bounds__(256) void mam_fwd_range_sum_kernel(const Params p)
             p.argmax[(int64_t)s * nm + o] = ih + shift;
             p.argmin[(int64_t)s * nm + o] = il + shift;
         } else {
-            if (hi == 0.0f) hi = first_zero_product<LAYOUT>(p.x + (int64_t)n * p.ldx, p.w, p.ldw, m, kb, ke);
-            if (lo == 0.0f) lo = first_zero_product<LAYOUT>(p.x + (int64_t)n * p.ldx, p.w, p.ldw, m, kb, ke);
+            const float *const wr = p.w + (int64_t)s * (p.w_step - p.k_per_split);
+            if (hi == 0.0f) hi = first_zero_product<LAYOUT>(p.x + (int64_t)n * p.ldx, wr, p.ldw, m, kb, ke);
+            if (lo == 0.0f) lo = first_zero_product<LAYOUT>(p.x + (int64_t)n * p.ldx, wr, p.ldw, m, kb, ke);
         }
         const float v = hi + lo;
         total = s == 0 ? v : total + v;
@@ -904,7 +925,6 @@ namespace sx {
 constexpr int BN = 32;    // batch rows per workgroup
 constexpr int NT = 512;   // threads per workgroup
 constexpr int TI = 4;     // batch rows per wave
-constexpr int KT = 64;    // k extent of one W tile
 constexpr int CHUNKS = KT / 4;    // 16-byte chunks per neuron and tile
 constexpr int RPB = 64 / KT < 1 ? 1 : 64 / KT;   // neurons per 256 bytes of LDS (all 64 banks)
 // TJ = neurons per lane.  2 (128 neurons per workgroup) is what the launch uses unless half of the last tile would be
@@ -929,8 +949,12 @@ constexpr int BM_MAX = Cfg<2>::BM;
 
 typedef const __attribute__((address_space(4))) float const_f32;
 
-// TAIL: K (or the last K range) is a multiple of G = 16 but not of 64; the last tile is partial.  A separate
-// instantiation, so that the whole-tile kernel stays exactly what it was.
+// REST: of a range of K that is not whole 64-k tiles.  Separate instantiations, so that the whole-tile kernel stays exactly
+// what it was (with the choice made per call 2000 x 768 -> 2048 takes 189 us instead of 187).
+//   REST_GROUPS: K (or the last K range) is a multiple of G = 16 but not of 64; the last tile is partial
+//   REST_ANY:    the last tile of a range ends where the range ends (see walked); x may begin and end anywhere.  With indices w is a
+//                copy that holds every range as it is walked: the resolve reads a line of it per output and extreme where
+//                groups are aligned, two where they are not (1000 x 4092 -> 1000, 32 and 49 us of merge)
 // GT: products per recorded group.  G = 16 costs a compare and a select per extreme and 16 products; with
 // GT = 32 the pair is issued after every second group (the running extremes of the first are kept as the
 // baseline), which takes 64 of a tile's 1160 instructions off the k loop and doubles what the resolve scans
@@ -939,13 +963,15 @@ typedef const __attribute__((address_space(4))) float const_f32;
 // tile (an integer in the workspace, zero at launch); the workgroup that draws the last ticket of a tile finds
 // all the tile's partials complete, combines them in ascending k with strict compares and resolves in its
 // own epilogue, as the unsplit kernel does.
-template <int TJ, bool ARGS, bool SPLIT, bool TAIL, int GT = G, bool FUSE = false>
+enum Rest { REST_NONE, REST_GROUPS, REST_ANY };
+template <int TJ, bool ARGS, bool SPLIT, Rest REST, int GT = G, bool FUSE = false>
 __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
 {
     // (the arguments of the prologue in one fetch with the guard's, not in a second one behind its branch)
     asm volatile("" ::"s"(p.x), "s"(p.w), "s"(p.ldx), "s"(p.ldw), "s"(p.tiles_n), "s"(p.k_per_split), "s"(p.group_n));
     if (ordered::guarded_off(p.guard)) return;
     using C = sx::Cfg<TJ>;
+    constexpr bool TAIL = REST == REST_GROUPS, RAGGED = REST == REST_ANY;
     __shared__ __attribute__((aligned(16))) float tile_a[C::TILE_FLOATS];
     __shared__ __attribute__((aligned(16))) float tile_b[C::TILE_FLOATS];
 
@@ -967,7 +993,9 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
     const int row0 = tn * sx::BN + sx::TI * wave, col0 = tm * C::BM;
     const int kb = split * p.k_per_split;
     const int ke = (kb + p.k_per_split) < p.K ? (kb + p.k_per_split) : p.K;
-    const int ntiles = (ke - kb) / sx::KT;    // whole tiles; a rest of whole 16-k groups follows as a partial tile
+    // whole tiles; a rest of whole 16-k groups follows as a partial tile.  Ragged ranges: tiles of which the last one begins at k = last
+    const int ntiles = (ke - kb + (RAGGED ? sx::KT - 1 : 0)) / sx::KT;
+    const int last = RAGGED ? ke - sx::KT - kb : INT32_MAX;
 
     static_assert(GT == G || (GT == 2 * G && !TAIL), "tracking span");
     float vmax[sx::TI][TJ], vmin[sx::TI][TJ];
@@ -1032,12 +1060,13 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
         for (int gg = 0; gg < sx::KT / G; ++gg) {
             if (TAIL && gg >= ng) break;
             const int grel = (t * sx::KT + gg * G) / GT;       // the span this group belongs to
+            const int kt = RAGGED && t * sx::KT > last ? last : t * sx::KT;
             const bool opens = (gg * G) % GT == 0, closes = ((gg + 1) * G) % GT == 0;
             float xv[sx::TI][G];
 #pragma unroll
             for (int i = 0; i < sx::TI; ++i)
 #pragma unroll
-                for (int q = 0; q < G; ++q) xv[i][q] = xr[i][t * sx::KT + gg * G + q];
+                for (int q = 0; q < G; ++q) xv[i][q] = xr[i][kt + gg * G + q];
 #pragma unroll
             for (int j = 0; j < TJ; ++j) {
                 float wv[G];
@@ -1068,8 +1097,11 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
             }
         }
     };
+    const char *wk_last = nullptr;      // the columns of a ragged range's last tile
     auto dma_any = [&](const char *wk, float *tile, int t) {
-        if (!TAIL || t < ntiles) {
+        if (!TAIL) {
+            dma(RAGGED && !ARGS && t * sx::KT > last ? wk_last : wk, tile);
+        } else if (t < ntiles) {
             dma(wk, tile);
         } else {
 #pragma unroll
@@ -1086,7 +1118,9 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
         }
     };
 
-    const char *wk = reinterpret_cast<const char *>(p.w + (int64_t)col0 * p.ldw + kb);
+    const char *const wrow = reinterpret_cast<const char *>(p.w + (int64_t)col0 * p.ldw);
+    const char *wk = wrow + (RAGGED && p.own_ranges ? (int64_t)split * p.w_step : kb) * (int64_t)sizeof(float);
+    if (RAGGED && !ARGS) wk_last = wrow + (p.w_tail < 0 ? ke - sx::KT : (p.own_ranges ? (int64_t)split * p.w_step : 0) + p.w_tail) * (int64_t)sizeof(float);
     if (nt_all > 0) {
         dma_any(wk, tile_a, 0);
         __syncthreads();
@@ -1190,8 +1224,8 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
             for (int j = 0; j < TJ; ++j) {
                 vals[(j * 2 + 0) * 64 + lane] = vmax[i][j];
                 vals[(j * 2 + 1) * 64 + lane] = vmin[i][j];
-                grps[(j * 2 + 0) * 64 + lane] = g0 + gmax[i][j];
-                grps[(j * 2 + 1) * 64 + lane] = g0 + gmin[i][j];
+                grps[(j * 2 + 0) * 64 + lane] = (g0 + gmax[i][j]) * GT;
+                grps[(j * 2 + 1) * 64 + lane] = (g0 + gmin[i][j]) * GT;
             }
             __builtin_amdgcn_wave_barrier();
             const int nrow = row0 + i;
@@ -1206,7 +1240,7 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
                 const char *wrows = reinterpret_cast<const char *>(p.w + (int64_t)mb * p.ldw);
                 const uint32_t last = last_row_offset(p.M, mb, 64, ldw4);   // neurons past M repeat the last one
                 const uint32_t mine = (uint32_t)(lane >> 3) * ldw4;         // slot = 8 r + lane / 8
-                resolve_wave<GT>(p, vals + j * 128, grps + j * 128, res, lane,
+                resolve_wave<GT, RAGGED>(p, vals + j * 128, grps + j * 128, res, lane,
                              [&](int slot, int &n, int &m, bool &valid) {
                                  n = nrow;
                                  m = mbase + slot;
@@ -1217,7 +1251,7 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
                              [&](int r, int, int, int kb, const float *&xp, const float *&wp) {
                                  const uint32_t row = mine + (uint32_t)(8 * r) * ldw4;
                                  const uint32_t k4 = (uint32_t)kb * 4u;
-                                 xp = reinterpret_cast<const float *>(xrow + k4);
+                                 xp = reinterpret_cast<const float *>(xrow + (RAGGED ? (uint32_t)walked(kb, p.K) * 4u : k4));
                                  wp = reinterpret_cast<const float *>(wrows + (clamped_row_offset(row, last) + k4));
                              });
             }
@@ -1351,9 +1385,12 @@ static bool narrow_tiles_pay(int64_t N, int64_t K, int64_t M, int64_t range_len)
     return length(sx::Cfg<1>::BM, 1.07f) < length(sx::BM_MAX, 2.0f);
 }
 
+// Rows of x as they are, whose length is no multiple of 64 or which are not 16-byte aligned (w_step, w_tail of Params).
+struct Ragged { int64_t w_step, w_tail; };
+
 static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                      const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel, float *x_sel,
-                     int64_t N, int64_t K, int64_t M, int64_t range_len = 0)
+                     int64_t N, int64_t K, int64_t M, int64_t range_len = 0, const Ragged *ragged = nullptr)
 {
     if (N < 0 || K < 0 || M < 0) return fail(MAM_ERR_INVALID_ARGUMENT, "negative size");
     if (w_layout != MAM_W_KM && w_layout != MAM_W_MK)
@@ -1376,11 +1413,14 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     // comparisons and tests).
     // (range_len > 0: the caller fixes the K ranges -- the module's `splits` -- instead of the launch
     // heuristics; the wave-uniform-rows tiling then also needs whole 64-k tiles per range)
-    const bool use_sx = (w_layout == MAM_W_MK) && p.vec_x && p.vec_w && (K % G == 0) &&
-                        (range_len % sx::KT == 0) && (ldw * sx::BM_MAX < (1ll << 30)) &&
+    const bool use_sx = (w_layout == MAM_W_MK) && p.vec_w && (ragged || (p.vec_x && K % G == 0 && range_len % sx::KT == 0)) && (ldw * sx::BM_MAX < (1ll << 30)) &&
                         option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
     plan.use_sx = use_sx;
-    plan.narrow = use_sx && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_FUSED_MERGE && narrow_tiles_pay(N, K, M, range_len);
+    // what the tiles walk
+    const int64_t own = range_len < K ? range_len : K, whole_range = ragged ? ceil_div(own, sx::KT) * sx::KT : range_len;
+    const int64_t whole_K = !ragged || (own == 0 && K % G == 0) ? K :
+                            own > 0 ? ceil_div(K, own) * whole_range : ceil_div(K, sx::KT) * sx::KT;
+    plan.narrow = use_sx && option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_FUSED_MERGE && narrow_tiles_pay(N, whole_K, M, whole_range);
     const int bn = use_sx ? sx::BN : BN, bm = use_sx ? (plan.narrow ? sx::Cfg<1>::BM : sx::BM_MAX) : BM;
     p.tiles_n = (int)ceil_div(N, bn);
     p.tiles_m = (int)ceil_div(M, bm);
@@ -1393,13 +1433,17 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     if (range_len > 0) {
         p.k_per_split = (int)(range_len < K ? range_len : K);
     } else {
-        p.splits = choose_splits(N, K, M, bn, bm);
+        p.splits = choose_splits(N, whole_K, M, bn, bm);
         const int kt = use_sx ? sx::KT : KT;
-        p.k_per_split = (int)(ceil_div(ceil_div(K, p.splits), kt) * kt);
+        p.k_per_split = (int)(ceil_div(ceil_div(whole_K, p.splits), kt) * kt);
     }
     p.splits = (int)ceil_div(K, p.k_per_split);
     p.part = nullptr;
     p.range_len = 0;
+    p.ragged = ragged != nullptr;
+    p.own_ranges = range_len > 0;
+    p.w_step = ragged && p.own_ranges ? (int)ragged->w_step : p.k_per_split;
+    p.w_tail = ragged ? (int)ragged->w_tail : -1;
     p.guard = ordered::Guard{nullptr};
     plan.need = p.splits > 1 ? (size_t)p.splits * (args ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float) : 0;
     // the fused merge keeps one ticket per tile behind the partials
@@ -1412,9 +1456,9 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     p.fast = p.vec_x && p.vec_w && (ldx * fwd::BN < (1ll << 30)) && (ldw * w_rows < (1ll << 30)) &&
              (p.k_per_split % 4 == 0);
     // (64 rows of w within 4 GiB: the merge kernel addresses a patch's operands by 32-bit offsets)
-    p.coop = (w_layout == MAM_W_MK) && p.vec_x && p.vec_w && (K % G == 0) && (ldw < (1ll << 24));
+    p.coop = (w_layout == MAM_W_MK) && p.vec_w && (ragged || (p.vec_x && K % G == 0)) && (ldw < (1ll << 24));
     // two groups per recorded span where the resolve is cheap next to the k loop (see mam_fwd_sx_kernel)
-    p.gt = (args && use_sx && range_len == 0 && K >= 2048 && K % sx::KT == 0 && p.k_per_split % sx::KT == 0 &&
+    p.gt = (args && use_sx && range_len == 0 && whole_K >= 2048 && (ragged || K % sx::KT == 0) && p.k_per_split % sx::KT == 0 &&
             option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_GROUPS16) ? 2 * G : G;
     // group ids are kept as 16-bit offsets from the first group of a workgroup's k range
     if ((int64_t)p.k_per_split / G > 65536)
@@ -1425,10 +1469,11 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
 // Operands that the wave-uniform-rows tiling does not take as they are -- a (K, M) weight, rows that are not 16-byte
 // aligned, K not a multiple of 16 -- are copied into the workspace once per call in the form that it does take.  Rows of
 // a ragged K are lengthened to whole 64-k tiles by their own last element: a repeated product never wins a strict
-// comparison, so every result stays what it was.
+// comparison, so every result stays what it was.  Most calls need no copy of x (see walked and ragged_staging).
 struct Staging {
     bool x, w;             // copied
-    int64_t K;             // row length of the copies (and of the call)
+    int64_t K;             // row length of the call (and of lengthened copies)
+    int64_t w_ld;          // row stride of the copy of w
     size_t x_bytes, w_bytes;
     size_t bytes() const { return x_bytes + w_bytes; }
 };
@@ -1439,10 +1484,33 @@ static Staging staging_of(bool x_fits, bool w_fits, int64_t N, int64_t K, int64_
     else s.K = K % G == 0 ? K : ceil_div(K, sx::KT) * sx::KT;
     s.x = !x_fits || s.K != K;
     s.w = !w_fits || s.K != K;
+    s.w_ld = s.K;
     auto padded = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
     s.x_bytes = s.x ? padded((size_t)N * (size_t)s.K * sizeof(float)) : 0;
     s.w_bytes = s.w ? padded((size_t)M * (size_t)s.K * sizeof(float)) : 0;
     return s;
+}
+
+// Rows of x as they are (see walked): ranges of at least 64, (M, K) weights.  With indices those weights are copied as they are
+// walked; values only where a range's tiles do not begin at 16-byte addresses, every range up to a multiple of 4, then its last 64
+// once more.  K below 128 stays with the lengthened copies: two tiles of which one is mostly repeated cost as much, and
+// the operands are small.  With indices so do calls of many neurons, whose resolve touches two lines of x where a copy's groups
+// have one, half as often in spans of 32 ((N, K, M), x copied / as it is, us: 10233 x 3316 -> 78 in training 429 / 409, 4000 x 4095 -> 250
+// 247 / 238, but 1000 x 4095 -> 500 122 / 125, 500 x 4095 -> 2000 223 / 232; in spans of 16, 43120 x 1300 -> 42 in training 718 / 598,
+// 8000 x 1001 -> 500 253 / 250, 9536 x 2809 -> 1432 in four ranges, training 5951 / 5858, but 3000 x 150 -> 1500 104 / 106; values only,
+// 16000 x 300 -> 200 72 / 59, 30 x 260 -> 4000 21 / 13, 1 x 4092 -> 16000 194 / 104, 4000 x 531 -> 3712 183 / 181).
+static bool ragged_staging(Staging &s, Ragged &tail, bool args, bool w_aligned, int64_t N, int64_t K, int64_t M, int64_t range_len)
+{
+    const int64_t ranges = ceil_div(K, range_len);
+    if (K < 2 * sx::KT || K - (ranges - 1) * range_len < sx::KT) return false;
+    if (args && M > (ranges > 1 ? 1536 : K > 2048 - sx::KT ? 320 : 1024) && N + M <= 65535) return false;
+    const bool copy = args || !w_aligned || K % 4 != 0 || (ranges > 1 && range_len % 4 != 0);
+    const int64_t step = args ? ceil_div(range_len, sx::KT) * sx::KT : ceil_div(range_len, 4) * 4 + sx::KT;
+    if (copy && (M > 65535 || ranges * step > (1 << 23))) return false;
+    tail.w_step = copy ? step : range_len;
+    tail.w_tail = copy && !args ? step - sx::KT : -1;
+    s = Staging{false, copy, K, ranges * step, 0, copy ? ((size_t)M * (size_t)(ranges * step) * sizeof(float) + 255) / 256 * 256 : 0};
+    return true;
 }
 
 // Whether to transpose a (K, M) operand once and run the (M, K) tilings on the copy: two more passes
@@ -1465,7 +1533,7 @@ static bool transposed_operand_pays(int64_t N, int64_t K, int64_t M)
 // 25 / 16; 4000 x 130 x 1000 42 / 45, 30000 x 31 x 60 14 / 32).
 static bool lengthened_rows_pay(int64_t N, int64_t K, int64_t M, bool turn, bool args)
 {
-    if (N + M > 65535 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
+    if (option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
     if (K >= 256) return true;
     const int64_t outputs = N * M;
     if (args) return K >= 64 || (outputs >= 16384 ? K > 4 || N >= 64 : outputs >= 1000 && K > (turn ? 32 : 16));
@@ -1480,7 +1548,7 @@ static bool lengthened_rows_pay(int64_t N, int64_t K, int64_t M, bool turn, bool
 // loop gains: 4000 x 531 x 3712 681 / 641, 500 x 200 x 500 23 / 18, 1441 x 2280 x 94 120 / 48; not 8098 x 278 x 71 43 / 47.
 static bool lengthened_ranges_pay(int64_t N, int64_t M, int64_t range_len, bool args)
 {
-    if (N + M > 65535 || range_len < 32 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
+    if (range_len < 32 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
     return args ? range_len > 32 || N * M > 16384 : range_len >= 96 || N * M <= (1 << 18);
 }
 
@@ -1492,9 +1560,17 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
 {
     if (plan.use_sx) return false;
     const bool turn = w_layout == MAM_W_KM, ranges = range_len > 0 && range_len < K;
+    Ragged tail;
+    if (!turn && ragged_staging(st, tail, args, plan.p.vec_w, N, K, M, ranges ? range_len : K) &&
+        (ranges ? lengthened_ranges_pay(N, M, range_len, args) : lengthened_rows_pay(N, K, M, turn, args))) {
+        float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
+        const int rc = make_plan(staged, args, x, ldx, st.w ? aligned : w, st.w ? st.w_ld : ldw, MAM_W_MK, bias, c, argmax, argmin, w_sel, x_sel,
+                                 N, K, M, range_len, &tail);
+        if (rc == MAM_OK && staged.use_sx && staged.p.coop) return true;
+    }
     st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M, range_len);
+    if (N + M > 65535 || (turn && !transposed_operand_pays(N, K, M))) return false;
     const bool lengthen = st.x || (st.w && !turn);
-    if (turn && !transposed_operand_pays(N, K, M)) return false;
     if (ranges ? turn || st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args) : lengthen && !lengthened_rows_pay(N, K, M, turn, args)) return false;
     float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
     const int rc = make_plan(staged, args, st.x ? aligned : x, st.x ? st.K : ldx, st.w ? aligned : w, st.w ? st.K : ldw, MAM_W_MK, bias,
@@ -1503,22 +1579,18 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
     return rc == MAM_OK && staged.use_sx;
 }
 
-// The wave-uniform-rows tiling with 64 * TJ neurons per workgroup; tail: a partial last k tile.
-template <int TJ, bool ARGS>
+// The wave-uniform-rows tiling with 64 * TJ neurons per workgroup.
+template <int TJ, bool ARGS, bool SPLIT>
 static void launch_sx(const Params &p, bool tail, unsigned blocks, hipStream_t st)
 {
     constexpr int GT = ARGS ? 2 * G : G;
     const dim3 grid(blocks), block(sx::NT);
     const bool spans = ARGS && p.gt == 2 * G;
-    if (p.splits > 1) {
-        if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, true, true>), grid, block, 0, st, p);
-        else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, true, false, GT>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, true, false>), grid, block, 0, st, p);
-    } else {
-        if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, false, true>), grid, block, 0, st, p);
-        else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, false, false, GT>), grid, block, 0, st, p);
-        else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, false, false>), grid, block, 0, st, p);
-    }
+    if (p.ragged && spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_ANY, GT>), grid, block, 0, st, p);
+    else if (p.ragged) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_ANY>), grid, block, 0, st, p);
+    else if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_GROUPS>), grid, block, 0, st, p);
+    else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_NONE, GT>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_NONE>), grid, block, 0, st, p);
 }
 
 template <bool ARGS>
@@ -1542,7 +1614,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     const int64_t operand_K = K;
     const bool on_16 = static_scratch || (uintptr_t)workspace % 16 == 0;
     Plan tplan;
-    Staging stage = {false, false, K, 0, 0}, st_plan;
+    Staging stage = {false, false, K, K, 0, 0}, st_plan;
     const bool can_stage = on_16 && staged_plan(tplan, st_plan, plan, ARGS, x, ldx, w, ldw, w_layout, bias, c, argmax, argmin, w_sel,
                                                 x_sel, N, K, M, range_len);
     const size_t staged_need = can_stage ? st_plan.bytes() + tplan.need : 0;
@@ -1586,7 +1658,7 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     hipStream_t st = static_cast<hipStream_t>(stream);
     // the merge inside the forward launch (option MAM_FORWARD_TILING_FUSED_MERGE): whole 64-k tiles, spans of 32
     const bool tail_k = K % sx::KT != 0;
-    const bool fuse = ARGS && use_sx && p.splits > 1 && !tail_k && p.gt == 2 * G && p.coop && range_len == 0 &&
+    const bool fuse = ARGS && use_sx && p.splits > 1 && !tail_k && !p.ragged && p.gt == 2 * G && p.coop && range_len == 0 &&
                       option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_FUSED_MERGE;
     if (fuse) {
         p.tickets = reinterpret_cast<int *>(scratch_base + wt_bytes + plan.tickets_at);
@@ -1602,19 +1674,19 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
         float *const ws = reinterpret_cast<float *>(scratch_base), *const xs = reinterpret_cast<float *>(scratch_base + stage.w_bytes);
         const bool turn = operand_layout == MAM_W_KM;
         const LengthenRows rx = {x, ldx, xs, stage.x ? (int)N : 0}, rw = {w, ldw, ws, stage.w && !turn ? (int)M : 0};
-        rc = lengthen_rows(rx, rw, operand_K, K, range_len, st, &p.guard);
+        rc = lengthen_rows(rx, rw, operand_K, stage.w && p.ragged ? stage.w_ld : K, range_len,
+                           !p.ragged ? ROWS_REPEAT_LAST : ARGS ? ROWS_END_WHOLE_TILES : ROWS_AND_LAST_64, st, &p.guard);
         if (rc == MAM_OK && turn) rc = transpose(w, ldw, ws, operand_K, M, K, st, &p.guard);
         if (rc != MAM_OK) return rc;
         if (stage.x) p.x = xs;
         if (stage.w) p.w = ws;
     }
-    const bool tail = K % sx::KT != 0;
     if (fuse)
-        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, false, ARGS ? 2 * G : G, ARGS>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && plan.narrow)
-        launch_sx<1, ARGS>(p, tail, (unsigned)nblk, st);
+        hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, REST_NONE, ARGS ? 2 * G : G, ARGS>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
+    else if (use_sx && p.splits > 1)
+        (plan.narrow ? launch_sx<1, ARGS, true> : launch_sx<2, ARGS, true>)(p, tail_k, (unsigned)nblk, st);
     else if (use_sx)
-        launch_sx<2, ARGS>(p, tail, (unsigned)nblk, st);
+        (plan.narrow ? launch_sx<1, ARGS, false> : launch_sx<2, ARGS, false>)(p, tail_k, (unsigned)nblk, st);
     else if (w_layout == MAM_W_MK)
         hipLaunchKernelGGL((mam_fwd_kernel<MAM_W_MK, ARGS>), dim3((unsigned)nblk), dim3(NT), 0, st, p);
     else
@@ -1623,9 +1695,11 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     if (rc != MAM_OK) return rc;
     if (p.splits > 1 && range_len > 0) {
         // the caller's ranges are neurons of their own: resolve each and add them up
-        const bool coop = ARGS && p.coop && p.k_per_split % G == 0;
+        const bool coop = ARGS && p.coop && (p.ragged || p.k_per_split % G == 0);
         const unsigned mb = coop ? (unsigned)(ceil_div(N, 4) * ceil_div(M, 64)) : (unsigned)(ceil_div(N, 16) * ceil_div(M, 16));
-        if (coop)
+        if (coop && p.ragged)
+            hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_MK, ARGS, ARGS, ARGS>), dim3(mb), dim3(256), 0, st, p);
+        else if (coop)
             hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_MK, ARGS, ARGS>), dim3(mb), dim3(256), 0, st, p);
         else if (w_layout == MAM_W_MK)
             hipLaunchKernelGGL((mam_fwd_range_sum_kernel<MAM_W_MK, ARGS, false>), dim3(mb), dim3(256), 0, st, p);
@@ -1636,7 +1710,11 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
         // 16 x 16 patches; 4 x 64 with the cooperative resolve
         const unsigned mb = (ARGS && p.coop) ? (unsigned)(ceil_div(N, 4) * ceil_div(M, 64))
                                              : (unsigned)(ceil_div(N, 16) * ceil_div(M, 16));
-        if (ARGS && p.coop && p.gt == 2 * G)
+        if (ARGS && p.ragged && p.gt == 2 * G)
+            hipLaunchKernelGGL((mam_fwd_merge_kernel<MAM_W_MK, ARGS, ARGS, ARGS ? 2 * G : G, ARGS>), dim3(mb), dim3(256), 0, st, p);
+        else if (ARGS && p.ragged)
+            hipLaunchKernelGGL((mam_fwd_merge_kernel<MAM_W_MK, ARGS, ARGS, G, ARGS>), dim3(mb), dim3(256), 0, st, p);
+        else if (ARGS && p.coop && p.gt == 2 * G)
             hipLaunchKernelGGL((mam_fwd_merge_kernel<MAM_W_MK, ARGS, ARGS, ARGS ? 2 * G : G>), dim3(mb), dim3(256), 0, st, p);
         else if (ARGS && p.coop)
             hipLaunchKernelGGL((mam_fwd_merge_kernel<MAM_W_MK, ARGS, ARGS>), dim3(mb), dim3(256), 0, st, p);
@@ -1668,7 +1746,12 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     size_t bytes = mam::fwd::workspace_bytes(N, K, M, with_indices != 0);
     // room for staged operands (see launch); without it the call still works
     const bool turn = w_layout == MAM_W_KM, ragged = K % mam::fwd::G != 0;
-    if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0)))
+    mam::fwd::Staging st;
+    mam::fwd::Ragged tail;
+    const bool pays = ragged && mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0);
+    if (pays && !turn && mam::fwd::ragged_staging(st, tail, with_indices != 0, K % 4 == 0, N, K, M, K))
+        bytes += st.bytes() + (st.w ? mam::fwd::staging_of(false, true, N, K, M).x_bytes : 0);
+    else if (N + M <= 65535 && (turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || pays))
         bytes += mam::fwd::staging_of(true, !turn, N, K, M).bytes();
     if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M, w_layout);
     return bytes;
@@ -1680,7 +1763,12 @@ extern "C" size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t 
     const size_t ranges = (size_t)((K + range_len - 1) / range_len);
     size_t bytes = ranges * (with_indices ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float);
     // room for lengthened ranges (see launch); without it the call still works
-    if (mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0)) bytes += mam::fwd::staging_of(false, false, N, K, M, range_len).bytes();
+    if (mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0)) {
+        mam::fwd::Staging st;
+        mam::fwd::Ragged tail;
+        if (mam::fwd::ragged_staging(st, tail, with_indices != 0, K % 4 == 0, N, K, M, range_len)) bytes += st.bytes();
+        else if (N + M <= 65535) bytes += mam::fwd::staging_of(false, false, N, K, M, range_len).bytes();
+    }
     return bytes;
 }
 
@@ -1709,7 +1797,7 @@ static void describe_plan(const mam::fwd::Plan &plan, int w_layout, int64_t K, b
     const char *what = with_indices ? "args" : "values";
     if (plan.use_sx)
         snprintf(text, text_bytes, "mam_fwd_sx_kernel<%s%s%s%s> %d x %d tiles of 32 x %d", what, p.splits > 1 ? ", split" : "",
-                 K % fwd::sx::KT != 0 ? ", partial last k tile" : "", p.gt > fwd::G ? ", indices per 32 k" : "", p.tiles_n,
+                 K % fwd::sx::KT == 0 ? "" : p.ragged ? ", last k tile at the end of K" : ", partial last k tile", p.gt > fwd::G ? ", indices per 32 k" : "", p.tiles_n,
                  p.tiles_m, plan.narrow ? 64 : 128);
     else
         snprintf(text, text_bytes, "mam_fwd_kernel<%s, %s> %d x %d tiles of 64 x 128", w_layout == MAM_W_MK ? "(M,K)" : "(K,M)",
@@ -1754,7 +1842,7 @@ extern "C" int mam_fc_forward_describe(const float *x, int64_t ldx, const float 
     if (staged) {
         const bool turn = w_layout == MAM_W_KM;
         int used = snprintf(text, text_bytes, "with %zu workspace bytes: %s%s", st.bytes() + tplan.need,
-                            st.x || !turn ? "lengthen_rows_kernel + " : "", turn ? "transpose_kernel + " : "");
+                            st.x || (st.w && !turn) ? "lengthen_rows_kernel + " : "", turn ? "transpose_kernel + " : "");
         if (used < 0 || (size_t)used >= text_bytes) return MAM_OK;
         describe_plan(tplan, MAM_W_MK, st.K, with_indices != 0, text + used, text_bytes - used);
         used = (int)strlen(text);

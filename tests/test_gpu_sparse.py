@@ -89,6 +89,32 @@ def test_batch_tiles_and_ragged_shapes(N, M, K):
     _forward_backward(x, dense, crow, col, val, "N%d M%d K%d" % (N, M, K))
 
 
+# batch rows per lane 1, 2 and 4 (by how many workgroups there are), each with rows that stay in LDS and rows that do not
+@pytest.mark.parametrize("N,M,K", [(33, 70, 300), (70, 4100, 290), (130, 8195, 640)])
+def test_rows_of_mixed_lengths(N, M, K):
+    """Neighbouring rows, which share a wave, of any two lengths: none, parts of a quad, of a block of 16 and of what
+    LDS holds, whole rows.  Small whole numbers, so that most extremes are ties, and zeros of both signs."""
+    g = torch.Generator().manual_seed(M)
+    lengths = torch.tensor([0, 1, 2, 3, 4, 5, 7, 8, 9, 15, 16, 17, 31, 33] * 8 + [255, 256, 257, 272, 289, 575, 576, 577, K - 1, K])
+    lengths = lengths.clamp(max=K)[torch.randint(len(lengths), (M,), generator=g)]
+    lengths[M - 1] = K
+    crow = torch.zeros(M + 1, dtype=torch.int64)
+    crow[1:] = lengths.cumsum(0)
+    # every third row is a prefix of the columns, so that its lowest missing column lies behind its last entry
+    col = torch.cat([torch.arange(int(l)) if m % 3 == 0 else torch.randperm(K, generator=g)[:l].sort()[0]
+                     for m, l in enumerate(lengths.tolist())])
+    val = torch.randint(-3, 4, (len(col),), generator=g).float()
+    val[::7] = -0.0
+    dense = torch.zeros(M, K)
+    dense[torch.repeat_interleave(torch.arange(M), lengths), col] = val
+    x = torch.randint(-3, 4, (N, K), generator=g).float()
+    x[1] = x[1].abs()
+    x[2] = -0.0
+    x[3] = torch.randn(K, generator=g)
+    x[4, K - 1] = float("nan")
+    _forward_backward(x, dense, crow, col, val, "mixed rows N%d M%d K%d" % (N, M, K))
+
+
 def test_implicit_zero_rules():
     g = torch.Generator().manual_seed(3)
     M, K, N = 64, 96, 20

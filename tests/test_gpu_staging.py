@@ -65,3 +65,71 @@ def test_tiles_of_64_neurons(N, K, M):
         assert_index_equal(got.cpu().numpy(), index, tag + " index")
         assert_bits_equal(x_sel[plane].cpu().numpy(), x.numpy()[rows, index], tag + " x_sel")
         assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
+
+
+def _planted(N, K, M, seed):
+    """Ties across the whole row and at its end, zeros of both signs, rows without a product."""
+    g = torch.Generator().manual_seed(seed)
+    x, w = torch.randn(N, K, generator=g), torch.randn(M, K, generator=g)
+    x[0] = -x[0].abs()                               # one sign throughout, the extreme at the last element
+    w[0] = w[0].abs()
+    x[0, -1], w[0, -1] = -1e-3, 1e-3
+    x[1], x[2] = torch.randint(-2, 3, (K,), generator=g).float(), 0.25
+    w[1:3] = torch.randint(-2, 3, (2, K), generator=g).float()
+    x[3, : K - 20], x[4, K - 70:] = -0.0, float("nan")
+    w[3], w[4, K - 64:] = 0.5, 7.0
+    return x, w
+
+
+# operand rows: aligned, 16 bytes apart but begun off them, of odd stride
+@pytest.mark.parametrize("pad,shift", [(0, 0), (4, 1), (3, 2)])
+@pytest.mark.parametrize("N,K,M", [(33, 128, 64), (37, 129, 130), (33, 191, 70), (64, 192, 129), (200, 260, 300), (31, 1300, 42), (40, 2050, 192),
+                                   (5, 4092, 65)])
+def test_last_tile_at_the_end_of_the_row(N, K, M, pad, shift):
+    """Rows of any length and alignment without a copy of x: all of K in one range and in several, tails of one to 63 columns."""
+    from mamtorch_amd import capi
+
+    x, w = _planted(N, K, M, N + K)
+    bias = torch.randn(M, generator=torch.Generator().manual_seed(1))
+
+    def padded(t):      # infinities all round: a column too many would win
+        buf = torch.full((t.size(0) * (K + pad) + 8,), float("inf"), device=DEV)
+        view = buf[shift: shift + t.size(0) * (K + pad)].view(t.size(0), K + pad)[:, :K]
+        view.copy_(t)
+        return view
+
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, bias.numpy())
+    for xd, wd in ((padded(x), w.to(DEV)), (padded(x), padded(w)), (x.to(DEV), padded(w))):
+        w_sel, x_sel = torch.zeros(2, N, M, device=DEV), torch.zeros(2, N, M, device=DEV)
+        c, amax, amin = capi.fc_forward(xd, wd, capi.W_MK, bias.to(DEV), w_sel=w_sel, x_sel=x_sel)
+        values = capi.fc_forward_values(xd, wd, capi.W_MK, bias.to(DEV))
+        tag = "N %d K %d M %d" % (N, K, M)
+        assert_bits_equal(c.cpu().numpy(), want[0], tag + " c")
+        assert_bits_equal(values.cpu().numpy(), want[0], tag + " values-only c")
+        rows, cols = np.arange(N)[:, None], np.arange(M)[None, :]
+        for plane, (got, index) in enumerate(zip((amax, amin), want[1:3])):
+            assert_index_equal(got.cpu().numpy(), index, tag + " index")
+            assert_bits_equal(x_sel[plane].cpu().numpy(), x.numpy()[rows, index], tag + " x_sel")
+            assert_bits_equal(w_sel[plane].cpu().numpy(), w.numpy()[cols, index], tag + " w_sel")
+
+
+@pytest.mark.parametrize("pad", [0, 3])
+@pytest.mark.parametrize("N,K,M,range_len", [(33, 128, 70, 64), (33, 130, 70, 65), (40, 264, 129, 100), (5, 448, 65, 128), (70, 1000, 300, 250),
+                                             (64, 1001, 64, 333), (130, 999, 64, 201)])
+def test_last_tile_at_the_end_of_each_range(N, K, M, range_len, pad):
+    from mamtorch_amd import capi
+
+    x, w = _planted(N, K, M, N + K)
+    xd = torch.full((N, K + pad), float("inf"), device=DEV)[:, :K].copy_(x)
+    wd = torch.full((M, K + pad), float("inf"), device=DEV)[:, :K].copy_(w)
+    c, amax, amin = capi.fc_forward_ranges(xd, wd, range_len, capi.W_MK)
+    values, _, _ = capi.fc_forward_ranges(xd, wd, range_len, capi.W_MK, with_indices=False)
+    total = None
+    for s, k in enumerate(range(0, K, range_len)):
+        part = oracle.forward(x[:, k:k + range_len].contiguous().numpy(), w[:, k:k + range_len].contiguous().numpy(), oracle.W_MK)
+        total = part[0] if total is None else total + part[0]
+        tag = "N %d K %d M %d range %d" % (N, K, M, s)
+        assert_index_equal(amax[s].cpu().numpy(), part[1] + k, tag + " argmax")
+        assert_index_equal(amin[s].cpu().numpy(), part[2] + k, tag + " argmin")
+    assert_bits_equal(c.cpu().numpy(), total, tag + " c")
+    assert_bits_equal(values.cpu().numpy(), total, tag + " values")
