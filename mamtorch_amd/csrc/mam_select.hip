@@ -8,7 +8,8 @@
 // bit patterns of the scores: a non-negative fp32 orders like its bit pattern (NaN above infinity, where
 // torch.sort puts it too), so three histogram passes over the 31 key bits (11 + 9 + 11 bits, 2048-bin
 // histograms in LDS, flushed to a global histogram with integer atomics) narrow the bins down to the one
-// key that holds the rank; a one-workgroup step after each pass walks the histogram and fixes the digit.
+// key that holds the rank.  Between two passes a prefix sum over the histogram fixes the digit: for one matrix every workgroup
+// of the next pass takes it by itself, for several tensors a launch of one workgroup does, after the last of them.
 // One or two ranks are followed at once (torch.quantile interpolates between two neighbours), and the
 // passes take any number of tensors, so the global rule needs no concatenated copy.  Every pass streams
 // the scores once: 3 x 4 bytes per element (plus the second operand of a product or count score).
@@ -33,10 +34,12 @@ struct State {
     uint32_t nranks, pad;
     int64_t rank[MAX_RANKS];        // rank still to go within the elements that share the prefix
 };
-// workspace: State, then hist[PASSES][MAX_RANKS][BINS] of 64-bit counts (the tensors of one selection may hold
+// workspace: a State for each pass to start from, then hist[PASSES][MAX_RANKS][BINS] of 64-bit counts (the tensors of one selection may hold
 // more than 2^32 elements together; a workgroup's own LDS bins are 32 bits)
 typedef unsigned long long count_t;
 constexpr size_t kHistWords = (size_t)PASSES * MAX_RANKS * BINS;
+constexpr size_t kStateStride = 2;     // 64 bytes from one to the next
+static_assert(sizeof(State) == 32 && (PASSES * kStateStride + 1) * sizeof(State) <= 256, "the states precede the histograms");
 constexpr size_t kWorkspaceBytes = 256 + kHistWords * sizeof(count_t);
 
 // Keys are 31 bits wide (absolute values: the sign bit is clear): digits of 11, 9 and 11 bits.  The second pass is the
@@ -67,11 +70,78 @@ __global__ __launch_bounds__(NT) void begin_kernel(State *st, count_t *hist, int
     }
 }
 
-// One histogram pass over one matrix.  vec: 16-byte loads (K a multiple of 4, aligned rows).
-template <int MODE>
+// What `st` becomes once pass `pass` has seen every score: the digit of each rank, found by a prefix sum of the workgroup over
+// the histogram (8.3 -> 3.8 us against one thread that walks the bins).  next: LDS; st may be the state that is written afterwards.
+template <int THREADS>
+__device__ __forceinline__ void advance(const State *__restrict__ st, const count_t *__restrict__ hist, int pass, State *next)
+{
+    __shared__ int64_t wave_total[MAX_RANKS][THREADS / 64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int nr = (int)st->nranks;
+    const uint32_t prefix[MAX_RANKS] = {st->prefix[0], st->prefix[1]};
+    const int64_t wanted[MAX_RANKS] = {st->rank[0], st->rank[1]};
+    const bool one = nr < 2 || prefix[0] == prefix[1];
+    const int nbins = 1 << pass_bits(pass);
+    constexpr int per = BINS / THREADS;
+    int64_t own[MAX_RANKS][per];
+#pragma unroll
+    for (int s = 0; s < MAX_RANKS; ++s)
+#pragma unroll
+        for (int b = 0; b < per; ++b) {
+            const count_t *h = hist + ((size_t)pass * MAX_RANKS + (one ? 0 : s)) * BINS;
+            own[s][b] = s < nr && tid * per + b < nbins ? (int64_t)h[tid * per + b] : 0;
+        }
+    int64_t sum[MAX_RANKS], upto[MAX_RANKS];       // elements up to and with this thread's bins
+#pragma unroll
+    for (int s = 0; s < MAX_RANKS; ++s) {
+        sum[s] = 0;
+#pragma unroll
+        for (int b = 0; b < per; ++b) sum[s] += own[s][b];
+        upto[s] = sum[s];
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int64_t o = __shfl_up(upto[s], off);
+            if (lane >= off) upto[s] += o;
+        }
+        if (lane == 63) wave_total[s][wave] = upto[s];
+    }
+    __syncthreads();
+    if (tid == 0) {
+        next->nranks = (uint32_t)nr;
+        next->pad = 0u;
+        if (nr < MAX_RANKS) {
+            next->prefix[1] = prefix[1];
+            next->rank[1] = wanted[1];
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < MAX_RANKS; ++s) {
+        if (s >= nr) break;
+        for (int w = 0; w < wave; ++w) upto[s] += wave_total[s][w];
+        const int64_t r = wanted[s], before = upto[s] - sum[s];
+        if ((before <= r && r < upto[s]) || (tid == THREADS - 1 && r >= upto[s])) {
+            int64_t below = before;
+            int digit = tid * per;
+#pragma unroll
+            for (int b = 0; b < per; ++b)
+                if (digit == tid * per + b && digit < nbins - 1 && below + own[s][b] <= r) {
+                    below += own[s][b];
+                    ++digit;
+                }
+            next->prefix[s] = (prefix[s] << pass_bits(pass)) | (uint32_t)digit;
+            next->rank[s] = r - below;
+        }
+    }
+    __syncthreads();
+}
+
+// One histogram pass over one matrix.  CHAINED: the only matrix, st is the state before the last pass, whose histogram is complete; the
+// state that follows from it is left behind st for the next pass (4096 x 4096: the steps by themselves 13 us and the gaps between four
+// launches, 7 us and one launch here).  vec: 16-byte loads (K a multiple of 4, aligned rows).
+template <int MODE, bool CHAINED>
 __global__ __launch_bounds__(NT_H) void hist_kernel(const float *__restrict__ w, int64_t ldw, const void *aux,
                                                   const void *aux2, int64_t ld_aux, int64_t M, int64_t K, int vec,
-                                                  const State *__restrict__ st, count_t *__restrict__ hist, int pass)
+                                                  State *st, count_t *hist, int pass)
 {
     // Scores crowd into few bins (the first pass looks at the exponent and three mantissa bits), and an LDS atomic
     // costs per lane that shares an address: neighbouring lanes count into copies of the histogram, which start on
@@ -80,6 +150,12 @@ __global__ __launch_bounds__(NT_H) void hist_kernel(const float *__restrict__ w,
     // like this (12 us: the load of 67 MB).  What is left above the load is the histogram's global atomics.
     __shared__ uint32_t bins[MAX_RANKS][COPIES][COPY_STRIDE];
     const int tid = threadIdx.x;
+    if (CHAINED) {
+        __shared__ State next;
+        advance<NT_H>(st, hist, pass - 1, &next);
+        if (blockIdx.x == 0 && tid == 0) st[kStateStride] = next;
+        st = &next;
+    }
     const int nr = (int)st->nranks;
     const int shift = pass_shift(pass), nb = pass_bits(pass);
     const uint32_t mask = (1u << nb) - 1u;
@@ -160,55 +236,24 @@ __global__ __launch_bounds__(NT_H) void hist_kernel(const float *__restrict__ w,
     }
 }
 
-// After every tensor has been through pass `pass`: find the digit of each rank in the histogram(s).  One prefix sum over
-// the workgroup (8.3 -> 3.8 us against one thread that walks the bins).
+// After every tensor has been through pass `pass`.
 __global__ __launch_bounds__(NT) void advance_kernel(State *st, const count_t *__restrict__ hist, int pass)
 {
-    __shared__ int64_t wave_total[NT / 64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int nr = (int)st->nranks;
-    const uint32_t prefix[MAX_RANKS] = {st->prefix[0], st->prefix[1]};
-    const int64_t wanted[MAX_RANKS] = {st->rank[0], st->rank[1]};
-    const bool one = nr < 2 || prefix[0] == prefix[1];
-    const int nbins = 1 << pass_bits(pass);
-    constexpr int per = BINS / NT;     // 8 bins per thread
-    for (int s = 0; s < nr; ++s) {
-        const count_t *h = hist + ((size_t)pass * MAX_RANKS + (one ? 0 : s)) * BINS;
-        int64_t own[per], sum = 0;
-#pragma unroll
-        for (int b = 0; b < per; ++b) {
-            own[b] = (tid * per + b) < nbins ? (int64_t)h[tid * per + b] : 0;
-            sum += own[b];
-        }
-        int64_t upto = sum;            // elements up to and with this thread's bins
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int64_t o = __shfl_up(upto, off);
-            if (lane >= off) upto += o;
-        }
-        __syncthreads();               // also: the state and the last rank's totals have been read
-        if (lane == 63) wave_total[wave] = upto;
-        __syncthreads();
-        for (int w = 0; w < wave; ++w) upto += wave_total[w];
-        const int64_t r = wanted[s], before = upto - sum;
-        if ((before <= r && r < upto) || (tid == NT - 1 && r >= upto)) {
-            int64_t below = before;
-            int digit = tid * per;
-#pragma unroll
-            for (int b = 0; b < per; ++b)
-                if (digit == tid * per + b && digit < nbins - 1 && below + own[b] <= r) {
-                    below += own[b];
-                    ++digit;
-                }
-            st->prefix[s] = (prefix[s] << pass_bits(pass)) | (uint32_t)digit;
-            st->rank[s] = r - below;
-        }
-    }
+    __shared__ State next;
+    advance<NT>(st, hist, pass, &next);
+    if (threadIdx.x == 0) *st = next;
 }
 
-__global__ void result_kernel(const State *st, float *out, int as_count)
+// The last digits are in the histogram yet (CHAINED) or in the state.
+template <bool CHAINED>
+__global__ __launch_bounds__(NT) void result_kernel(const State *st, const count_t *hist, float *out, int as_count)
 {
     const int s = threadIdx.x;
+    if (CHAINED) {
+        __shared__ State next;
+        advance<NT>(st, hist, PASSES - 1, &next);
+        st = &next;
+    }
     if (s < (int)st->nranks) out[s] = as_count ? (float)(int)st->prefix[s] : __uint_as_float(st->prefix[s]);
 }
 
@@ -234,8 +279,8 @@ extern "C" int mam_select_begin(void *workspace, size_t workspace_bytes, const i
     return check_launch("select begin_kernel");
 }
 
-extern "C" int mam_select_accumulate(void *workspace, const float *w, int64_t ldw, int mode, const void *aux,
-                                     const void *aux2, int64_t ld_aux, int64_t M, int64_t K, int pass, void *stream)
+static int accumulate(void *workspace, const float *w, int64_t ldw, int mode, const void *aux, const void *aux2, int64_t ld_aux,
+                      int64_t M, int64_t K, int pass, bool chained, void *stream)
 {
     using namespace mam;
     if (!workspace) return fail(MAM_ERR_WORKSPACE, "no workspace");
@@ -264,16 +309,26 @@ extern "C" int mam_select_accumulate(void *workspace, const float *w, int64_t ld
     if (blocks > cap) blocks = cap;
     if (blocks < 1) blocks = 1;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const selectk::State *state = static_cast<const selectk::State *>(workspace);
+    // in a chain, pass p > 0 starts from the state that pass p - 1 started from
+    selectk::State *state = static_cast<selectk::State *>(workspace) + (chained ? (pass - 1) * selectk::kStateStride : 0);
     selectk::count_t *hist = selectk::hist_of(workspace);
-#define MAM_SELECT_LAUNCH(MODE)                                                                                      \
-    hipLaunchKernelGGL(selectk::hist_kernel<MODE>, dim3((unsigned)blocks), dim3(selectk::NT_H), 0, st, w, ldw, aux, aux2, \
-                       ld_aux, M, K, vec ? 1 : 0, state, hist, pass)
-    if (mode == MAM_PRUNE_MAGNITUDE) MAM_SELECT_LAUNCH(MAM_PRUNE_MAGNITUDE);
-    else if (mode == MAM_PRUNE_WEIGHT_TIMES) MAM_SELECT_LAUNCH(MAM_PRUNE_WEIGHT_TIMES);
-    else MAM_SELECT_LAUNCH(MAM_PRUNE_COUNT);
+#define MAM_SELECT_LAUNCH(MODE, CHAINED)                                                                             \
+    hipLaunchKernelGGL((selectk::hist_kernel<MODE, CHAINED>), dim3((unsigned)blocks), dim3(selectk::NT_H), 0, st, w, ldw, aux, \
+                       aux2, ld_aux, M, K, vec ? 1 : 0, state, hist, pass)
+    if (mode == MAM_PRUNE_MAGNITUDE && chained) MAM_SELECT_LAUNCH(MAM_PRUNE_MAGNITUDE, true);
+    else if (mode == MAM_PRUNE_MAGNITUDE) MAM_SELECT_LAUNCH(MAM_PRUNE_MAGNITUDE, false);
+    else if (mode == MAM_PRUNE_WEIGHT_TIMES && chained) MAM_SELECT_LAUNCH(MAM_PRUNE_WEIGHT_TIMES, true);
+    else if (mode == MAM_PRUNE_WEIGHT_TIMES) MAM_SELECT_LAUNCH(MAM_PRUNE_WEIGHT_TIMES, false);
+    else if (chained) MAM_SELECT_LAUNCH(MAM_PRUNE_COUNT, true);
+    else MAM_SELECT_LAUNCH(MAM_PRUNE_COUNT, false);
 #undef MAM_SELECT_LAUNCH
     return check_launch("select hist_kernel");
+}
+
+extern "C" int mam_select_accumulate(void *workspace, const float *w, int64_t ldw, int mode, const void *aux,
+                                     const void *aux2, int64_t ld_aux, int64_t M, int64_t K, int pass, void *stream)
+{
+    return accumulate(workspace, w, ldw, mode, aux, aux2, ld_aux, M, K, pass, false, stream);
 }
 
 extern "C" int mam_select_advance(void *workspace, int pass, void *stream)
@@ -290,8 +345,8 @@ extern "C" int mam_select_result(void *workspace, int mode, float *out, void *st
 {
     using namespace mam;
     if (!workspace || !out) return fail(MAM_ERR_INVALID_ARGUMENT, "null pointer");
-    hipLaunchKernelGGL(selectk::result_kernel, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const selectk::State *>(workspace), out, mode == MAM_PRUNE_COUNT ? 1 : 0);
+    hipLaunchKernelGGL(selectk::result_kernel<false>, dim3(1), dim3(64), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const selectk::State *>(workspace), selectk::hist_of(workspace), out, mode == MAM_PRUNE_COUNT ? 1 : 0);
     return check_launch("select result_kernel");
 }
 
@@ -299,10 +354,21 @@ extern "C" int mam_select_ranks(const float *w, int64_t ldw, int mode, const voi
                                 int64_t K, const int64_t *ranks, int nranks, float *out, void *workspace, size_t workspace_bytes,
                                 void *stream)
 {
+    using namespace mam;
     int rc = mam_select_begin(workspace, workspace_bytes, ranks, nranks, stream);
-    for (int pass = 0; pass < mam::selectk::PASSES && rc == MAM_OK; ++pass) {
-        rc = mam_select_accumulate(workspace, w, ldw, mode, aux, aux2, ld_aux, M, K, pass, stream);
-        if (rc == MAM_OK) rc = mam_select_advance(workspace, pass, stream);
+    if (rc == MAM_OK && (!out || M == 0 || K == 0)) {
+        // no score to find a digit in: the checks, and what the steps by themselves give
+        for (int pass = 0; pass < selectk::PASSES && rc == MAM_OK; ++pass) {
+            rc = mam_select_accumulate(workspace, w, ldw, mode, aux, aux2, ld_aux, M, K, pass, stream);
+            if (rc == MAM_OK) rc = mam_select_advance(workspace, pass, stream);
+        }
+        return rc == MAM_OK ? mam_select_result(workspace, mode, out, stream) : rc;
     }
-    return rc == MAM_OK ? mam_select_result(workspace, mode, out, stream) : rc;
+    for (int pass = 0; pass < selectk::PASSES && rc == MAM_OK; ++pass)
+        rc = accumulate(workspace, w, ldw, mode, aux, aux2, ld_aux, M, K, pass, pass > 0, stream);
+    if (rc != MAM_OK) return rc;
+    hipLaunchKernelGGL(selectk::result_kernel<true>, dim3(1), dim3(selectk::NT), 0, static_cast<hipStream_t>(stream),
+                       static_cast<const selectk::State *>(workspace) + (selectk::PASSES - 1) * selectk::kStateStride,
+                       selectk::hist_of(workspace), out, mode == MAM_PRUNE_COUNT ? 1 : 0);
+    return check_launch("select result_kernel");
 }
