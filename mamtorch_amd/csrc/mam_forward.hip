@@ -77,6 +77,7 @@ struct Params {
     int gt;            // products per recorded group: G, or 2 G on the wave-uniform-rows tiling at large K
     int range_len;     // ranges of the caller's that were lengthened to k_per_split: their length (indices count in it)
     int ragged;        // wave-uniform rows, x as it is: the last k tile of a range ends where the range ends (see walked)
+    int touch_x;       // x is fetched into the L2 ahead of its use
     int own_ranges;    // the K ranges are the caller's
     int w_step;        // columns of w from one of them to the next (k_per_split, more in a copy)
     int w_tail;        // values only, w copied: column at which the last 64 of the (first) range stand once more, aligned; else -1
@@ -964,7 +965,8 @@ typedef const __attribute__((address_space(4))) float const_f32;
 // all the tile's partials complete, combines them in ascending k with strict compares and resolves in its
 // own epilogue, as the unsplit kernel does.
 enum Rest { REST_NONE, REST_GROUPS, REST_ANY };
-template <int TJ, bool ARGS, bool SPLIT, Rest REST, int GT = G, bool FUSE = false>
+// TOUCH: a wave fetches its x into the L2 a tile ahead (see touch_x; the choice made per call costs the calls that don't 1 to 3 %).
+template <int TJ, bool ARGS, bool SPLIT, Rest REST, int GT = G, bool FUSE = false, bool TOUCH = false>
 __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
 {
     // (the arguments of the prologue in one fetch with the guard's, not in a second one behind its branch)
@@ -1121,19 +1123,31 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
     const char *const wrow = reinterpret_cast<const char *>(p.w + (int64_t)col0 * p.ldw);
     const char *wk = wrow + (RAGGED && p.own_ranges ? (int64_t)split * p.w_step : kb) * (int64_t)sizeof(float);
     if (RAGGED && !ARGS) wk_last = wrow + (p.w_tail < 0 ? ke - sx::KT : (p.own_ranges ? (int64_t)split * p.w_step : 0) + p.w_tail) * (int64_t)sizeof(float);
+    // The wave's x of a tile: 64 lanes reach every line of four rows of 256 bytes
+    const float *const xlane = p.x + (int64_t)(row0 + (lane >> 4) < p.N ? row0 + (lane >> 4) : p.N - 1) * p.ldx + kb;
+    auto touch = [&](int t) {
+        const int k = t * sx::KT + (lane & 15) * 4, end = ke - kb - 1;
+        return TOUCH ? xlane[k < end ? k : end] : 0.0f;
+    };
     if (nt_all > 0) {
+        float seen = touch(0);
         dma_any(wk, tile_a, 0);
         __syncthreads();
+        if (TOUCH) asm volatile("" ::"v"(seen));
         for (int t = 0; t < nt_all; t += 2) {
             wk += sx::KT * sizeof(float);
+            seen = touch(t + 1);
             if (t + 1 < nt_all) dma_any(wk, tile_b, t + 1);
             compute(tile_a, t);
             __syncthreads();
+            if (TOUCH) asm volatile("" ::"v"(seen));
             if (t + 1 >= nt_all) break;
             wk += sx::KT * sizeof(float);
+            seen = touch(t + 2);
             if (t + 2 < nt_all) dma_any(wk, tile_a, t + 2);
             compute(tile_b, t + 1);
             __syncthreads();
+            if (TOUCH) asm volatile("" ::"v"(seen));
         }
     }
 
@@ -1388,6 +1402,14 @@ static bool narrow_tiles_pay(int64_t N, int64_t K, int64_t M, int64_t range_len)
 // Rows of x as they are, whose length is no multiple of 64 or which are not 16-byte aligned (w_step, w_tail of Params).
 struct Ragged { int64_t w_step, w_tail; };
 
+// Whether the waves fetch their x into the L2 a tile ahead.  The scalar loads, 64 bytes per row and 16 k, wait for memory otherwise:
+// nothing else has read an x of more than an XCD's L2 holds (4 MiB) lately where there are few neurons.  From 16 MiB and up
+// to 1024 neurons; an x that stays in the L2s, or that many neurons' tiles share, only loses the loads' issue.
+// ((N, K, M), us without / with: 16000 x 4096 -> 64 314 / 221, 1100 x 4000 -> 300 135 / 117, -> 900 256 / 238, 4000 x 1100 -> 64 34.5 / 31.5,
+// 43120 x 1300 -> 42 in training 597 / 522, 10233 x 3316 -> 78 409 / 365, 16000 x 512 -> 256 143 / 140; but 2000 x 768 -> 2048, values
+// only, 124.7 / 126.3, 256 x 4096 -> 2048 108 / 110, 9536 x 2809 -> 1432 in training 5739 / 5795.)
+constexpr int64_t TOUCHED_WORDS = (int64_t)4 << 20, TOUCHED_NEURONS = 1024;
+
 static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                      const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel, float *x_sel,
                      int64_t N, int64_t K, int64_t M, int64_t range_len = 0, const Ragged *ragged = nullptr)
@@ -1442,6 +1464,7 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     p.range_len = 0;
     p.ragged = ragged != nullptr;
     p.own_ranges = range_len > 0;
+    p.touch_x = use_sx && N * K >= TOUCHED_WORDS && M <= TOUCHED_NEURONS;
     p.w_step = ragged && p.own_ranges ? (int)ragged->w_step : p.k_per_split;
     p.w_tail = ragged ? (int)ragged->w_tail : -1;
     p.guard = ordered::Guard{nullptr};
@@ -1580,17 +1603,24 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
 }
 
 // The wave-uniform-rows tiling with 64 * TJ neurons per workgroup.
-template <int TJ, bool ARGS, bool SPLIT>
+template <int TJ, bool ARGS, bool SPLIT, bool TOUCH>
 static void launch_sx(const Params &p, bool tail, unsigned blocks, hipStream_t st)
 {
     constexpr int GT = ARGS ? 2 * G : G;
     const dim3 grid(blocks), block(sx::NT);
     const bool spans = ARGS && p.gt == 2 * G;
-    if (p.ragged && spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_ANY, GT>), grid, block, 0, st, p);
-    else if (p.ragged) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_ANY>), grid, block, 0, st, p);
-    else if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_GROUPS>), grid, block, 0, st, p);
-    else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_NONE, GT>), grid, block, 0, st, p);
-    else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_NONE>), grid, block, 0, st, p);
+    if (p.ragged && spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_ANY, GT, false, TOUCH>), grid, block, 0, st, p);
+    else if (p.ragged) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_ANY, G, false, TOUCH>), grid, block, 0, st, p);
+    else if (tail) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_GROUPS, G, false, TOUCH>), grid, block, 0, st, p);
+    else if (spans) hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_NONE, GT, false, TOUCH>), grid, block, 0, st, p);
+    else hipLaunchKernelGGL((mam_fwd_sx_kernel<TJ, ARGS, SPLIT, REST_NONE, G, false, TOUCH>), grid, block, 0, st, p);
+}
+
+template <int TJ, bool ARGS>
+static void launch_sx(const Params &p, bool tail, unsigned blocks, hipStream_t st)
+{
+    if (p.splits > 1) (p.touch_x ? launch_sx<TJ, ARGS, true, true> : launch_sx<TJ, ARGS, true, false>)(p, tail, blocks, st);
+    else (p.touch_x ? launch_sx<TJ, ARGS, false, true> : launch_sx<TJ, ARGS, false, false>)(p, tail, blocks, st);
 }
 
 template <bool ARGS>
@@ -1683,10 +1713,10 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     }
     if (fuse)
         hipLaunchKernelGGL((mam_fwd_sx_kernel<2, ARGS, true, REST_NONE, ARGS ? 2 * G : G, ARGS>), dim3((unsigned)nblk), dim3(sx::NT), 0, st, p);
-    else if (use_sx && p.splits > 1)
-        (plan.narrow ? launch_sx<1, ARGS, true> : launch_sx<2, ARGS, true>)(p, tail_k, (unsigned)nblk, st);
+    else if (use_sx && plan.narrow)
+        launch_sx<1, ARGS>(p, tail_k, (unsigned)nblk, st);
     else if (use_sx)
-        (plan.narrow ? launch_sx<1, ARGS, false> : launch_sx<2, ARGS, false>)(p, tail_k, (unsigned)nblk, st);
+        launch_sx<2, ARGS>(p, tail_k, (unsigned)nblk, st);
     else if (w_layout == MAM_W_MK)
         hipLaunchKernelGGL((mam_fwd_kernel<MAM_W_MK, ARGS>), dim3((unsigned)nblk), dim3(NT), 0, st, p);
     else

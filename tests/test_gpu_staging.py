@@ -133,3 +133,20 @@ def test_last_tile_at_the_end_of_each_range(N, K, M, range_len, pad):
         assert_index_equal(amin[s].cpu().numpy(), part[2] + k, tag + " argmin")
     assert_bits_equal(c.cpu().numpy(), total, tag + " c")
     assert_bits_equal(values.cpu().numpy(), total, tag + " values")
+
+
+# x of 16 MiB and more, few neurons: a part of the last row tile, whole tiles, a partial last one, one that ends with the row
+@pytest.mark.parametrize("N,K,M", [(16390, 256, 33), (8193, 528, 70), (4101, 1027, 200), (2053, 2048, 65), (1033, 4093, 129)])
+def test_rows_fetched_ahead(N, K, M):
+    from mamtorch_amd import capi
+
+    x, w = _planted(N, K, M, N + K)
+    xd, wd = x.to(DEV), w.to(DEV)
+    c, amax, amin = capi.fc_forward(xd, wd, capi.W_MK)
+    values = capi.fc_forward_values(xd, wd, capi.W_MK)
+    want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, None)
+    tag = "N %d K %d M %d" % (N, K, M)
+    assert_bits_equal(c.cpu().numpy(), want[0], tag + " c")
+    assert_bits_equal(values.cpu().numpy(), want[0], tag + " values-only c")
+    assert_index_equal(amax.cpu().numpy(), want[1], tag + " argmax")
+    assert_index_equal(amin.cpu().numpy(), want[2], tag + " argmin")
