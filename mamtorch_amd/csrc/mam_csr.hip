@@ -24,7 +24,7 @@
 // hits, at about half of the path's 64 bytes per clock and CU) with the arithmetic hidden under it.
 // The lowest column missing from the row is found once per row; the
 // implicit-zero candidate x[n, missing] * 0 is compared last under the dense rule (greater wins,
-// equal -> lower index wins).  The 16 waves of a workgroup own 16 consecutive neurons and hand
+// equal -> lower index wins).  TI follows the number of workgroups (below, at the launch).  The 16 waves of a workgroup own 16 consecutive neurons and hand
 // their results over through LDS so that every batch row stores 64 contiguous bytes per array.
 //
 // Backward: when the forward handed over the selected values and their entry positions, x_grad is the
@@ -70,8 +70,10 @@ __global__ __launch_bounds__(256) void transpose_kernel(const float *__restrict_
 
 template <int TI> struct XVec;
 template <> struct XVec<1> { typedef float type; };
+template <> struct XVec<2> { typedef float2 type; };
 template <> struct XVec<4> { typedef float4 type; };
 __device__ __forceinline__ float lane_elem(const float &v, int) { return v; }
+__device__ __forceinline__ float lane_elem(const float2 &v, int t) { return t == 0 ? v.x : v.y; }
 __device__ __forceinline__ float lane_elem(const float4 &v, int t)
 {
     return t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;
@@ -665,7 +667,7 @@ __global__ __launch_bounds__(256) void csr_validate_kernel(const int64_t *__rest
     if (bad) atomicOr(status, bad);
 }
 
-// Once per device: the forward kernels park 7 planes of results per workgroup in dynamic LDS (more than
+// Once per device: the forward kernels park 9 planes of results per workgroup in dynamic LDS (more than
 // the 64 KiB a launch gets by default), and the fallback backward keeps up to 128 KiB of histogram.
 static int g_bwd_lds_floats[kMaxDevices];
 
@@ -673,9 +675,12 @@ static int setup_device(int dev)
 {
     bool ok = true;
     const void *small[] = {(const void *)csr_fwd_kernel<1, false>, (const void *)csr_fwd_kernel<1, true>};
+    const void *middle[] = {(const void *)csr_fwd_kernel<2, false>, (const void *)csr_fwd_kernel<2, true>};
     const void *large[] = {(const void *)csr_fwd_kernel<4, false>, (const void *)csr_fwd_kernel<4, true>};
     for (const void *k : small)
         ok = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 9 * ROWS * 64 * 4) == hipSuccess && ok;
+    for (const void *k : middle)
+        ok = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 9 * ROWS * 128 * 4) == hipSuccess && ok;
     for (const void *k : large)
         ok = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 9 * ROWS * 256 * 4) == hipSuccess && ok;
     if (!ok) {
@@ -757,18 +762,29 @@ extern "C" int mam_csr_fc_forward(const float *x, int64_t ldx, const int64_t *cr
                         ((uintptr_t)pos_sel % 16 == 0) && ((uintptr_t)x_sel % 16 == 0);
     // the lane-held entry data needs every xT row's byte offset in 32 bits
     const bool lm = (int64_t)K * ldt * 4 < ((int64_t)1 << 32);
-    const dim3 grid1((unsigned)ceil_div(M, csr::ROWS), 1u);
-    const int64_t gy = ceil_div(N, 256);
+    // Batch rows per lane, 4, 2 or 1: a workgroup spends about twice on its CSR rows what it spends on each of them, so the
+    // fewest rounds of workgroups (one per CU) times 2 + rows, the larger one of equals.  Kernel alone, us, with 4 / as chosen: 500 rows,
+    // 4000 -> 512, 10 % 89 / 40 (1), 1 % 20.8 / 10.9 (1); 150 rows, 2000 -> 1000, 1.5 % 16.4 / 9.6 (1); 112 rows, 3584 -> 3456, 10 % 75 / 59 (2), 1 %
+    // 18.1 / 15.1 (2); 150 rows, 2000 -> 2000, 5 % 28.9 / 23.7 (2).
+    int ti = 4;
+    int64_t least = INT64_MAX;
+    for (int rows = 4; rows >= 1; rows /= 2) {
+        const int64_t cost = ceil_div(ceil_div(M, csr::ROWS) * ceil_div(N, 64 * rows), num_cus()) * (2 + rows);
+        if (cost < least) { least = cost; ti = rows; }
+    }
+    const int64_t gy = ceil_div(N, 64 * ti);
     if (gy > 65535) return fail(MAM_ERR_UNSUPPORTED, "N too large for the CSR forward grid");
-    const dim3 grid4((unsigned)ceil_div(M, csr::ROWS), (unsigned)gy);
-    const size_t lds1 = (size_t)9 * csr::ROWS * 64 * sizeof(float), lds4 = (size_t)9 * csr::ROWS * 256 * sizeof(float);
-#define MAM_CSR_LAUNCH(TI, LM, GRID, LDS)                                                                           \
-    hipLaunchKernelGGL((csr::csr_fwd_kernel<TI, LM>), GRID, dim3(csr::NT_F), LDS, st, xT, (int)ldt, crow, col, val, \
+    const dim3 grid((unsigned)ceil_div(M, csr::ROWS), (unsigned)gy);
+    const size_t lds = (size_t)9 * csr::ROWS * 64 * ti * sizeof(float);
+#define MAM_CSR_LAUNCH(TI, LM)                                                                                      \
+    hipLaunchKernelGGL((csr::csr_fwd_kernel<TI, LM>), grid, dim3(csr::NT_F), lds, st, xT, (int)ldt, crow, col, val, \
                        bias, c, argmax, argmin, w_sel, pos_sel, x_sel, (int)N, (int)K, (int)M, vec_out)
-    if (N <= 64 && lm) MAM_CSR_LAUNCH(1, true, grid1, lds1);
-    else if (N <= 64) MAM_CSR_LAUNCH(1, false, grid1, lds1);
-    else if (lm) MAM_CSR_LAUNCH(4, true, grid4, lds4);
-    else MAM_CSR_LAUNCH(4, false, grid4, lds4);
+    if (ti == 1 && lm) MAM_CSR_LAUNCH(1, true);
+    else if (ti == 1) MAM_CSR_LAUNCH(1, false);
+    else if (ti == 2 && lm) MAM_CSR_LAUNCH(2, true);
+    else if (ti == 2) MAM_CSR_LAUNCH(2, false);
+    else if (lm) MAM_CSR_LAUNCH(4, true);
+    else MAM_CSR_LAUNCH(4, false);
 #undef MAM_CSR_LAUNCH
     return check_launch("csr_fwd_kernel");
 }
