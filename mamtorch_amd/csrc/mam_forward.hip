@@ -26,8 +26,8 @@
 // a wave's W reads cover all banks and its X reads broadcast.  Ragged edges are handled by
 // replicating the last row / column / k on load: a replicated k duplicates an earlier product
 // and can never win a strict comparison.  The second one (mam_fwd_sx_kernel, further down)
-// serves the module's case -- (out, in) weight, aligned rows, K a multiple of 16 -- with
-// wave-uniform batch rows whose x operands come through the scalar cache; calls with other operands are
+// serves the module's case -- (out, in) weight, aligned rows of a multiple of 16 or x of any length from
+// 128 on -- with wave-uniform batch rows whose x operands come through the scalar cache; other operands are
 // copied into that form once where the workspace has room (Staging).
 //
 // Small N*M (the 256 x 4096 headline shape has only 256 tiles for 256 CUs x 2) is split
