@@ -1499,6 +1499,9 @@ struct Staging {
     int64_t w_ld;          // row stride of the copy of w
     size_t x_bytes, w_bytes;
     size_t bytes() const { return x_bytes + w_bytes; }
+    // whether one launch of lengthen_rows holds the rows it copies; a transposed w is copied by columns (70000 x 512 -> 64 as (512, 64):
+    // no row is lengthened)
+    bool rows_fit(int64_t N, int64_t M, bool turn) const { return (x ? N : 0) + (w && !turn ? M : 0) <= 65535; }
 };
 static Staging staging_of(bool x_fits, bool w_fits, int64_t N, int64_t K, int64_t M, int64_t range_len = 0)
 {
@@ -1592,7 +1595,7 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
         if (rc == MAM_OK && staged.use_sx && staged.p.coop) return true;
     }
     st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M, range_len);
-    if (N + M > 65535 || (turn && !transposed_operand_pays(N, K, M))) return false;
+    if (!st.rows_fit(N, M, turn) || (turn && !transposed_operand_pays(N, K, M))) return false;
     const bool lengthen = st.x || (st.w && !turn);
     if (ranges ? turn || st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args) : lengthen && !lengthened_rows_pay(N, K, M, turn, args)) return false;
     float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
@@ -1781,8 +1784,10 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     const bool pays = ragged && mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0);
     if (pays && !turn && mam::fwd::ragged_staging(st, tail, with_indices != 0, K % 4 == 0, N, K, M, K))
         bytes += st.bytes() + (st.w ? mam::fwd::staging_of(false, true, N, K, M).x_bytes : 0);
-    else if (N + M <= 65535 && (turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || pays))
-        bytes += mam::fwd::staging_of(true, !turn, N, K, M).bytes();
+    else if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || pays)) {
+        st = mam::fwd::staging_of(true, !turn, N, K, M);
+        if (st.rows_fit(N, M, turn)) bytes += st.bytes();
+    }
     if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M, w_layout);
     return bytes;
 }

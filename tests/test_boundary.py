@@ -108,6 +108,19 @@ def test_ragged_rows_are_lengthened_where_the_copy_pays(N, K, M, with_indices, m
     assert (copies >= 4 * (N + M) * K) if copied else copies == 0
 
 
+@pytest.mark.parametrize("N, K, M, with_indices", [(70000, 512, 64, 1), (70000, 512, 64, 0), (65535, 1024, 16, 1), (64, 512, 65536, 1),
+                                                   (64, 1001, 65536, 1)])
+def test_a_transposed_weight_of_any_number_of_rows(N, K, M, with_indices):
+    # no row of x (but of a ragged K) and none of w is lengthened: the grid of that copy does not limit the call
+    l = capi.lib()
+    text = ctypes.create_string_buffer(640)
+    one = ctypes.c_void_p(256)
+    ldx = (K + 3) // 4 * 4
+    assert l.mam_fc_forward_describe(one, ldx, one, M, capi.W_KM, N, K, M, with_indices, text, 640) == 0
+    assert b"transpose_kernel + mam_fwd_sx_kernel" in text.value, text.value
+    assert l.mam_fc_forward_workspace_for(N, K, M, capi.W_KM, with_indices) >= int(text.value.split(b"with ")[1].split()[0]) > 0
+
+
 def test_workspace_queries_are_pure_host_calls():
     l = capi.lib()
     assert l.mam_fc_forward_workspace(12608, 768, 3072) == 0          # enough tiles: no split-K

@@ -150,3 +150,22 @@ def test_rows_fetched_ahead(N, K, M):
     assert_bits_equal(values.cpu().numpy(), want[0], tag + " values-only c")
     assert_index_equal(amax.cpu().numpy(), want[1], tag + " argmax")
     assert_index_equal(amin.cpu().numpy(), want[2], tag + " argmin")
+
+
+@pytest.mark.parametrize("N,K,M", [(65600, 80, 33), (65535, 64, 65), (40, 130, 65600)])
+def test_a_transposed_weight_of_any_number_of_rows(N, K, M):
+    """More rows together than one launch of lengthen_rows holds, against the tiling that takes a (K, M) weight as it is."""
+    from mamtorch_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(N)
+    x, w = torch.randint(-9, 10, (N, K), generator=g, device=DEV).float(), torch.randn(K, M, generator=g, device=DEV)
+    assert "transpose_kernel + mam_fwd_sx_kernel" in capi.fc_forward_describe(x, w, capi.W_KM)
+    outs = []
+    for tiling in (capi.FORWARD_TILING_AUTO, capi.FORWARD_TILING_WIDE):
+        capi.set_option(capi.OPT_FORWARD_TILING, tiling)
+        try:
+            outs.append(capi.fc_forward(x, w, capi.W_KM) + (capi.fc_forward_values(x, w, capi.W_KM),))
+        finally:
+            capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    for got, want in zip(*outs):
+        assert torch.equal(got, want)
