@@ -1783,7 +1783,7 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     mam::fwd::Ragged tail;
     const bool pays = ragged && mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0);
     if (pays && !turn && mam::fwd::ragged_staging(st, tail, with_indices != 0, K % 4 == 0, N, K, M, K))
-        bytes += st.bytes() + (st.w ? mam::fwd::staging_of(false, true, N, K, M).x_bytes : 0);
+        bytes += st.bytes();
     else if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || pays)) {
         st = mam::fwd::staging_of(true, !turn, N, K, M);
         if (st.rows_fit(N, M, turn)) bytes += st.bytes();

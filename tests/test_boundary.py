@@ -105,7 +105,32 @@ def test_ragged_rows_are_lengthened_where_the_copy_pays(N, K, M, with_indices, m
     # the workspace query asks for the copies of the operands exactly where they are made
     need = (l.mam_fc_forward_workspace if with_indices else l.mam_fc_forward_values_workspace)(N, K, M)
     copies = l.mam_fc_forward_workspace_for(N, K, M, layout, with_indices) - need
-    assert (copies >= 4 * (N + M) * K) if copied else copies == 0
+    assert copies == (_bytes_of_copies(text.value) if copied else 0)
+
+
+def _bytes_of_copies(text):
+    # what mam_fc_forward_describe names for a call on copies, less its partials
+    staged = text.split(b"; with less: ")[0]
+    partials = re.search(rb"\((\d+) bytes of partials\)", staged)
+    return int(re.match(rb"with (\d+) workspace bytes: ", staged).group(1)) - (int(partials.group(1)) if partials else 0)
+
+
+@pytest.mark.parametrize("N, K, M", [(43120, 1300, 42), (10233, 3316, 78), (250, 1001, 517), (8000, 4095, 256), (70000, 300, 64)])
+def test_a_call_that_takes_x_as_it_is_asks_for_no_copy_of_it(N, K, M):
+    l = capi.lib()
+    text = ctypes.create_string_buffer(640)
+    one = ctypes.c_void_p(256)
+    assert l.mam_fc_forward_describe(one, K, one, K, capi.W_MK, N, K, M, 1, text, 640) == 0
+    lists_first, _, dense = text.value.rpartition(b"otherwise ")
+    assert b"last k tile at the end of K" in dense, text.value
+    with_lists = l.mam_fc_forward_workspace_for(N, K, M, capi.W_MK, 1)
+    capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_DENSE)
+    try:
+        asked = l.mam_fc_forward_workspace_for(N, K, M, capi.W_MK, 1)
+    finally:
+        capi.set_option(capi.OPT_FORWARD_TILING, capi.FORWARD_TILING_AUTO)
+    assert asked - l.mam_fc_forward_workspace(N, K, M) == _bytes_of_copies(dense) < 4 * M * (K + 64) + 256
+    assert (asked < with_lists) == (lists_first != b"")
 
 
 @pytest.mark.parametrize("N, K, M, with_indices", [(70000, 512, 64, 1), (70000, 512, 64, 0), (65535, 1024, 16, 1), (64, 512, 65536, 1),
