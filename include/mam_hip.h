@@ -122,9 +122,14 @@ int mam_set_option(int option, int value);
  * calls (2^32 products and more; 1.2 to 12 times as fast where the data suits
  * them, 2 to 10 % slower where the device finds that it does not).  A call whose workspace only has
  * mam_fc_forward_workspace() bytes still works, without them.
+ * mam_fc_forward_workspace_at() is mam_fc_forward_workspace_for() for given operands, whose alignment decides which of them are copied: what
+ * a call with these operands makes use of, in a workspace at a 16-byte address (1 x 4092 -> 16000, values only: nothing for a weight at one, a
+ * copy of 266 MB for a weight off it).  The pointers are looked at but never dereferenced.
  */
 size_t mam_fc_forward_workspace(int64_t N, int64_t K, int64_t M);
 size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, int w_layout, int with_indices);
+size_t mam_fc_forward_workspace_at(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K, int64_t M,
+                                   int with_indices);
 int mam_fc_forward(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                    const float *bias, float *c, int32_t *argmax, int32_t *argmin, float *w_sel,
                    float *x_sel, int64_t N, int64_t K, int64_t M,

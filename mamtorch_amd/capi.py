@@ -32,7 +32,7 @@ COUNT_FLAGS = 2
 EXPORTS = (
     "mam_version", "mam_error_string", "mam_last_error", "mam_init", "mam_set_option", "mam_device_info",
     "mam_fc_forward_static_limit", "mam_fc_forward_static", "mam_fc_forward_describe",
-    "mam_fc_forward_workspace", "mam_fc_forward_workspace_for", "mam_fc_forward",
+    "mam_fc_forward_workspace", "mam_fc_forward_workspace_for", "mam_fc_forward_workspace_at", "mam_fc_forward",
     "mam_fc_forward_values_workspace", "mam_fc_forward_values",
     "mam_fc_backward", "mam_fc_backward_count", "mam_selection_count",
     "mam_fc_forward_ranges_workspace", "mam_fc_forward_ranges", "mam_fc_backward_ranges",
@@ -67,6 +67,8 @@ def lib():
             fn.argtypes = [_i64, _i64, _i64]
         l.mam_fc_forward_workspace_for.restype = _size
         l.mam_fc_forward_workspace_for.argtypes = [_i64, _i64, _i64, _int, _int]
+        l.mam_fc_forward_workspace_at.restype = _size
+        l.mam_fc_forward_workspace_at.argtypes = [_ptr, _i64, _ptr, _i64, _int, _i64, _i64, _i64, _int]
         l.mam_fc_forward.argtypes = [_ptr, _i64, _ptr, _i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64,
                                      _i64, _i64, _ptr, _size, _ptr]
         l.mam_fc_forward_static_limit.restype = _size
@@ -155,7 +157,7 @@ def fc_forward(x, w, layout=W_KM, bias=None, workspace=None, w_sel=None, x_sel=N
     c = torch.empty((N, M), dtype=torch.float32, device=x.device)
     amax = torch.empty((N, M), dtype=torch.int32, device=x.device)
     amin = torch.empty((N, M), dtype=torch.int32, device=x.device)
-    need = l.mam_fc_forward_workspace_for(N, K, M, layout, 1)
+    need = l.mam_fc_forward_workspace_at(_p(x), _ld(x), _p(w), _ld(w), layout, N, K, M, 1)
     if workspace is None and need:
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     with torch.cuda.device(x.device):
@@ -192,7 +194,7 @@ def fc_forward_values(x, w, layout=W_KM, bias=None, workspace=None):
     l = lib()
     N, K, M = _dims(x, w, layout)
     c = torch.empty((N, M), dtype=torch.float32, device=x.device)
-    need = l.mam_fc_forward_workspace_for(N, K, M, layout, 0)
+    need = l.mam_fc_forward_workspace_at(_p(x), _ld(x), _p(w), _ld(w), layout, N, K, M, 0)
     if workspace is None and need:
         workspace = torch.empty(need, dtype=torch.uint8, device=x.device)
     with torch.cuda.device(x.device):
@@ -238,7 +240,7 @@ def fc_forward_picks(x, w, layout=W_KM, bias=None, w_sel=None, x_sel=None, works
     c = torch.empty((N, M), dtype=torch.float32, device=x.device)
     picks = torch.empty((N, M), dtype=torch.int32, device=x.device)
     if workspace_bytes is None:
-        workspace_bytes = l.mam_fc_forward_workspace_for(N, K, M, layout, 1)
+        workspace_bytes = l.mam_fc_forward_workspace_at(_p(x), _ld(x), _p(w), _ld(w), layout, N, K, M, 1)
     ws = torch.empty(max(workspace_bytes, 1), dtype=torch.uint8, device=x.device)
     with torch.cuda.device(x.device):
         _check(l.mam_fc_forward_picks(_p(x), _i64(_ld(x)), _p(w), _i64(_ld(w)), layout, _p(bias), _p(c), _p(picks), _p(w_sel), _p(x_sel),

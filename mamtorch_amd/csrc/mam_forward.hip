@@ -1760,6 +1760,19 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
     return rc;
 }
 
+// What a call makes use of (see launch): its lists, the copies of operands that are not in the form the tiling takes, the partials.
+static size_t usable_workspace(bool args, const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K,
+                               int64_t M)
+{
+    Plan plan, staged;
+    Staging st;
+    if (make_plan(plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N, K, M) != MAM_OK) return 0;
+    const bool copies = K % G != 0 || w_layout == MAM_W_KM;
+    const size_t dense = copies && staged_plan(staged, st, plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr,
+                                               nullptr, N, K, M, 0) ? st.bytes() + staged.need : plan.need;
+    return dense + (ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22)) ? ordered::workspace_bytes(N, K, M, w_layout) : 0);
+}
+
 // Every word of the partials that the merge reads is written by the same call's first kernel: nothing in
 // the array has to be cleared between calls.
 static int launch_static(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, const float *bias,
@@ -1782,7 +1795,8 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     mam::fwd::Staging st;
     mam::fwd::Ragged tail;
     const bool pays = ragged && mam::fwd::lengthened_rows_pay(N, K, M, turn, with_indices != 0);
-    if (pays && !turn && mam::fwd::ragged_staging(st, tail, with_indices != 0, K % 4 == 0, N, K, M, K))
+    // (rows of w of any alignment, which decides whether a call for values copies it)
+    if (pays && !turn && mam::fwd::ragged_staging(st, tail, with_indices != 0, false, N, K, M, K))
         bytes += st.bytes();
     else if ((turn || ragged) && (!turn || mam::fwd::transposed_operand_pays(N, K, M)) && (!ragged || pays)) {
         st = mam::fwd::staging_of(true, !turn, N, K, M);
@@ -1790,6 +1804,12 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
     }
     if (mam::ordered::applies(N, K, M)) bytes = (bytes + 255) / 256 * 256 + mam::ordered::workspace_bytes(N, K, M, w_layout);
     return bytes;
+}
+
+extern "C" size_t mam_fc_forward_workspace_at(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K,
+                                              int64_t M, int with_indices)
+{
+    return N <= 0 || K <= 0 || M <= 0 ? 0 : mam::fwd::usable_workspace(with_indices != 0, x, ldx, w, ldw, w_layout, N, K, M);
 }
 
 extern "C" size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t M, int64_t range_len, int with_indices)

@@ -74,17 +74,18 @@ struct FwdShape { int64_t N, K, M; };
 
 // The workspace of a forward call with room for all that makes it faster (lists and copies of the operands: 0.5 GB at 16384 x
 // 4096 -> 4096), or, where the device has not that much left, what the call cannot do without.
-at::Tensor forward_workspace(const FwdShape &s, int layout, bool with_indices, const at::Tensor &like)
+at::Tensor forward_workspace(const FwdShape &s, const at::Tensor &a, const at::Tensor &w, int layout, bool with_indices)
 {
-    const size_t most = mam_fc_forward_workspace_for(s.N, s.K, s.M, layout, with_indices ? 1 : 0);
+    const size_t most = mam_fc_forward_workspace_at(a.data_ptr<float>(), row_stride(a, "a"), w.data_ptr<float>(),
+                                                    row_stride(w, "the weight operand"), layout, s.N, s.K, s.M, with_indices ? 1 : 0);
     size_t least = 0;
     try {
-        return workspace_for(most, like);
+        return workspace_for(most, a);
     } catch (const c10::OutOfMemoryError &) {
         least = with_indices ? mam_fc_forward_workspace(s.N, s.K, s.M) : mam_fc_forward_values_workspace(s.N, s.K, s.M);
         if (least >= most) throw;
     }
-    return workspace_for(least, like);
+    return workspace_for(least, a);
 }
 
 FwdShape check_forward(const at::Tensor &a, const at::Tensor &w, int layout,
@@ -130,7 +131,7 @@ std::vector<at::Tensor> forward_impl(const at::Tensor &a, const at::Tensor &w, i
         if (with_sel) return {c, argmax, argmin, sel};
         return {c, argmax, argmin};
     }
-    auto ws = forward_workspace(s, layout, true, a);
+    auto ws = forward_workspace(s, a, w, layout, true);
     check_rc(mam_fc_forward(a.data_ptr<float>(), row_stride(a, "a"), w.data_ptr<float>(),
                             row_stride(w, "the weight operand"), layout, bias_ptr(bias),
                             c.data_ptr<float>(), argmax.data_ptr<int32_t>(), argmin.data_ptr<int32_t>(),
@@ -148,7 +149,7 @@ at::Tensor forward_values_impl(const at::Tensor &a, const at::Tensor &w, int lay
     const c10::DeviceGuard guard(a.device());
     auto c = at::empty({s.N, s.M}, a.options());
     if (s.N == 0 || s.M == 0) return c;
-    auto ws = forward_workspace(s, layout, false, a);
+    auto ws = forward_workspace(s, a, w, layout, false);
     check_rc(mam_fc_forward_values(a.data_ptr<float>(), row_stride(a, "a"), w.data_ptr<float>(),
                                    row_stride(w, "the weight operand"), layout, bias_ptr(bias),
                                    c.data_ptr<float>(), s.N, s.K, s.M,
@@ -238,7 +239,7 @@ std::vector<at::Tensor> fullyconnected_wt_picks(const at::Tensor &a, const at::T
     auto picks = at::empty({s.N, s.M}, a.options().dtype(at::kInt));
     auto sel = at::empty({4, s.N, s.M}, a.options());
     if (s.N == 0 || s.M == 0) return {c, picks, sel};
-    auto ws = forward_workspace(s, MAM_W_MK, true, a);
+    auto ws = forward_workspace(s, a, weight, MAM_W_MK, true);
     float *w_sel = sel.data_ptr<float>();
     check_rc(mam_fc_forward_picks(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
                                   row_stride(weight, "the weight operand"), MAM_W_MK, bias_ptr(bias), c.data_ptr<float>(),

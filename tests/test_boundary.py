@@ -146,6 +146,36 @@ def test_a_transposed_weight_of_any_number_of_rows(N, K, M, with_indices):
     assert l.mam_fc_forward_workspace_for(N, K, M, capi.W_KM, with_indices) >= int(text.value.split(b"with ")[1].split()[0]) > 0
 
 
+# what an operand's rows are: at 16-byte addresses, begun off them, of a stride off them
+ROWS = {"aligned": (256, 0), "shifted": (260, 0), "strided": (256, 1)}
+
+
+@pytest.mark.parametrize("rows_x", sorted(ROWS))
+@pytest.mark.parametrize("rows_w", sorted(ROWS))
+@pytest.mark.parametrize("with_indices", [0, 1])
+@pytest.mark.parametrize("N, K, M, mk", [(2000, 300, 2000, 1), (1, 4092, 16000, 1), (200, 260, 300, 1), (250, 1001, 517, 1), (31, 1300, 42, 1),
+                                         (64, 768, 256, 1), (16384, 4092, 1024, 1), (128, 2048, 4096, 0), (33, 63, 64, 0), (4, 63, 10, 1)])
+def test_the_workspace_of_a_call_holds_what_the_call_makes_use_of(N, K, M, mk, with_indices, rows_x, rows_w):
+    l = capi.lib()
+    text = ctypes.create_string_buffer(900)
+    layout = capi.W_MK if mk else capi.W_KM
+    (px, dx), (pw, dw) = ROWS[rows_x], ROWS[rows_w]
+    whole = (K + 3) // 4 * 4
+    row = (M + 3) // 4 * 4 if not mk else whole
+    call = (ctypes.c_void_p(px), whole + dx, ctypes.c_void_p(pw), row + dw, layout, N, K, M, with_indices)
+    assert l.mam_fc_forward_describe(*call, text, 900) == 0
+    lists_first, _, dense = text.value.rpartition(b"otherwise ")
+    named = re.match(rb"with (\d+) workspace bytes: ", dense)
+    asked, any_rows = l.mam_fc_forward_workspace_at(*call), l.mam_fc_forward_workspace_for(N, K, M, layout, with_indices)
+    assert asked <= any_rows
+    if lists_first:
+        assert asked > int(named.group(1)) if named else asked > 0
+    elif K % 16 != 0 or not mk:
+        # copies, where the call makes them, and partials, and nothing else
+        partials = re.search(rb"\((\d+) bytes of partials\)", dense)
+        assert asked == (int(named.group(1)) if named else int(partials.group(1)) if partials else 0)
+
+
 def test_workspace_queries_are_pure_host_calls():
     l = capi.lib()
     assert l.mam_fc_forward_workspace(12608, 768, 3072) == 0          # enough tiles: no split-K
