@@ -124,7 +124,8 @@ int mam_set_option(int option, int value);
  * mam_fc_forward_workspace() bytes still works, without them.
  * mam_fc_forward_workspace_at() is mam_fc_forward_workspace_for() for given operands, whose alignment decides which of them are copied: what
  * a call with these operands makes use of, in a workspace at a 16-byte address (1 x 4092 -> 16000, values only: nothing for a weight at one, a
- * copy of 266 MB for a weight off it).  The pointers are looked at but never dereferenced.
+ * copy of 266 MB for a weight off it; K a multiple of 16, for which mam_fc_forward_workspace_for() has no room for copies: those of rows off
+ * 16-byte addresses).  The pointers are looked at but never dereferenced.
  */
 size_t mam_fc_forward_workspace(int64_t N, int64_t K, int64_t M);
 size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, int w_layout, int with_indices);

@@ -1767,9 +1767,8 @@ static size_t usable_workspace(bool args, const float *x, int64_t ldx, const flo
     Plan plan, staged;
     Staging st;
     if (make_plan(plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N, K, M) != MAM_OK) return 0;
-    const bool copies = K % G != 0 || w_layout == MAM_W_KM;
-    const size_t dense = copies && staged_plan(staged, st, plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr,
-                                               nullptr, N, K, M, 0) ? st.bytes() + staged.need : plan.need;
+    const size_t dense = staged_plan(staged, st, plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N,
+                                     K, M, 0) ? st.bytes() + staged.need : plan.need;
     return dense + (ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22)) ? ordered::workspace_bytes(N, K, M, w_layout) : 0);
 }
 
