@@ -253,11 +253,17 @@ int mam_fc_backward_count(const float *x, int64_t ldx, const float *w, int64_t l
  * `C_flat += ...` statements.  argmax / argmin (both or neither; NULL = values only, the eval path):
  * [ranges][N][M] int32, plane r holding the lowest ABSOLUTE k of range r attaining its extreme (the
  * reference's per-slice operators return k relative to the slice).  `workspace`:
- * mam_fc_forward_ranges_workspace() bytes (0 when range_len >= K, which is mam_fc_forward).
+ * mam_fc_forward_ranges_workspace() bytes (0 when range_len >= K, which is mam_fc_forward): partials for every range and, for ranges that
+ * are not whole 64-k tiles, the copies of (M, K) operands that make the call 1.1 to 2.5 times as fast.  Partials are enough
+ * (ranges * N * M * (with_indices ? 12 : 8) bytes), and all that a (K, M) weight in such ranges makes use of.
+ * mam_fc_forward_ranges_workspace_at(): what a call with these operands makes use of, in a workspace at a 16-byte address; the pointers
+ * are looked at but never dereferenced.
  *   mam_fc_backward_ranges: the gradient of that c: every range routes grad[n,m] to its own two
  * selected positions.  x_grad (N,K), w_grad (shape and layout of w), either may be NULL.
  */
 size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t M, int64_t range_len, int with_indices);
+size_t mam_fc_forward_ranges_workspace_at(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K,
+                                          int64_t M, int64_t range_len, int with_indices);
 int mam_fc_forward_ranges(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                           const float *bias, float *c, int32_t *argmax, int32_t *argmin, int64_t N, int64_t K,
                           int64_t M, int64_t range_len, void *workspace, size_t workspace_bytes, void *stream);

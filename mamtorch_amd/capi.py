@@ -35,7 +35,7 @@ EXPORTS = (
     "mam_fc_forward_workspace", "mam_fc_forward_workspace_for", "mam_fc_forward_workspace_at", "mam_fc_forward",
     "mam_fc_forward_values_workspace", "mam_fc_forward_values",
     "mam_fc_backward", "mam_fc_backward_count", "mam_selection_count",
-    "mam_fc_forward_ranges_workspace", "mam_fc_forward_ranges", "mam_fc_backward_ranges",
+    "mam_fc_forward_ranges_workspace", "mam_fc_forward_ranges_workspace_at", "mam_fc_forward_ranges", "mam_fc_backward_ranges",
     "mam_csr_fc_forward_workspace", "mam_csr_fc_forward", "mam_csr_fc_backward", "mam_csr_validate",
     "mam_csr_spmm", "mam_coo_spmm", "mam_coo_row_offsets", "mam_coo_spmm_by_rows_workspace",
     "mam_coo_spmm_by_rows", "mam_csr_to_dense", "mam_coo_to_dense",
@@ -87,6 +87,8 @@ def lib():
                                       _i64, _i64, _i64, _ptr]
         l.mam_fc_forward_ranges_workspace.restype = _size
         l.mam_fc_forward_ranges_workspace.argtypes = [_i64, _i64, _i64, _i64, _int]
+        l.mam_fc_forward_ranges_workspace_at.restype = _size
+        l.mam_fc_forward_ranges_workspace_at.argtypes = [_ptr, _i64, _ptr, _i64, _int, _i64, _i64, _i64, _i64, _int]
         l.mam_fc_forward_ranges.argtypes = [_ptr, _i64, _ptr, _i64, _int, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64,
                                             _i64, _ptr, _size, _ptr]
         l.mam_fc_backward_count.argtypes = [_ptr, _i64, _ptr, _i64, _int, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
@@ -286,7 +288,7 @@ def fc_forward_ranges(x, w, range_len, layout=W_KM, bias=None, with_indices=True
     c = torch.empty((N, M), dtype=torch.float32, device=x.device)
     amax = torch.empty((ranges, N, M), dtype=torch.int32, device=x.device) if with_indices else None
     amin = torch.empty((ranges, N, M), dtype=torch.int32, device=x.device) if with_indices else None
-    need = l.mam_fc_forward_ranges_workspace(N, K, M, range_len, int(with_indices))
+    need = l.mam_fc_forward_ranges_workspace_at(_p(x), _ld(x), _p(w), _ld(w), layout, N, K, M, range_len, int(with_indices))
     ws = torch.empty(max(need, 1), dtype=torch.uint8, device=x.device)
     with torch.cuda.device(x.device):
         _check(l.mam_fc_forward_ranges(_p(x), _ld(x), _p(w), _ld(w), layout, _p(bias), _p(c), _p(amax), _p(amin),

@@ -1762,14 +1762,15 @@ static int launch(const float *x, int64_t ldx, const float *w, int64_t ldw, int 
 
 // What a call makes use of (see launch): its lists, the copies of operands that are not in the form the tiling takes, the partials.
 static size_t usable_workspace(bool args, const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K,
-                               int64_t M)
+                               int64_t M, int64_t range_len)
 {
     Plan plan, staged;
     Staging st;
-    if (make_plan(plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N, K, M) != MAM_OK) return 0;
+    if (make_plan(plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N, K, M, range_len) != MAM_OK) return 0;
     const size_t dense = staged_plan(staged, st, plan, args, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N,
-                                     K, M, 0) ? st.bytes() + staged.need : plan.need;
-    return dense + (ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22)) ? ordered::workspace_bytes(N, K, M, w_layout) : 0);
+                                     K, M, range_len) ? st.bytes() + staged.need : plan.need;
+    const bool lists = range_len == 0 && ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22));
+    return dense + (lists ? ordered::workspace_bytes(N, K, M, w_layout) : 0);
 }
 
 // Every word of the partials that the merge reads is written by the same call's first kernel: nothing in
@@ -1808,7 +1809,7 @@ extern "C" size_t mam_fc_forward_workspace_for(int64_t N, int64_t K, int64_t M, 
 extern "C" size_t mam_fc_forward_workspace_at(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K,
                                               int64_t M, int with_indices)
 {
-    return N <= 0 || K <= 0 || M <= 0 ? 0 : mam::fwd::usable_workspace(with_indices != 0, x, ldx, w, ldw, w_layout, N, K, M);
+    return N <= 0 || K <= 0 || M <= 0 ? 0 : mam::fwd::usable_workspace(with_indices != 0, x, ldx, w, ldw, w_layout, N, K, M, 0);
 }
 
 extern "C" size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t M, int64_t range_len, int with_indices)
@@ -1816,14 +1817,22 @@ extern "C" size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t 
     if (N <= 0 || K <= 0 || M <= 0 || range_len <= 0 || range_len >= K) return 0;
     const size_t ranges = (size_t)((K + range_len - 1) / range_len);
     size_t bytes = ranges * (with_indices ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float);
-    // room for lengthened ranges (see launch); without it the call still works
-    if (mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0)) {
+    // room for lengthened ranges (see launch), where they are not whole tiles as they are; without it the call still works
+    const bool whole = range_len % mam::fwd::sx::KT == 0 && K % mam::fwd::G == 0;
+    if (!whole && mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0)) {
         mam::fwd::Staging st;
         mam::fwd::Ragged tail;
-        if (mam::fwd::ragged_staging(st, tail, with_indices != 0, K % 4 == 0, N, K, M, range_len)) bytes += st.bytes();
+        if (mam::fwd::ragged_staging(st, tail, with_indices != 0, false, N, K, M, range_len)) bytes += st.bytes();
         else if (N + M <= 65535) bytes += mam::fwd::staging_of(false, false, N, K, M, range_len).bytes();
     }
     return bytes;
+}
+
+extern "C" size_t mam_fc_forward_ranges_workspace_at(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N,
+                                                     int64_t K, int64_t M, int64_t range_len, int with_indices)
+{
+    if (N <= 0 || K <= 0 || M <= 0 || range_len <= 0) return 0;
+    return mam::fwd::usable_workspace(with_indices != 0, x, ldx, w, ldw, w_layout, N, K, M, range_len);
 }
 
 extern "C" int mam_fc_forward_ranges(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,

@@ -312,7 +312,9 @@ std::vector<at::Tensor> fullyconnected_ranges(const at::Tensor &a, const at::Ten
     auto argmax = at::empty({with_indices ? ranges : 0, s.N, s.M}, a.options().dtype(at::kInt));
     auto argmin = at::empty({with_indices ? ranges : 0, s.N, s.M}, a.options().dtype(at::kInt));
     if (s.N == 0 || s.M == 0) return {c, argmax, argmin};
-    const size_t ws_bytes = mam_fc_forward_ranges_workspace(s.N, s.K, s.M, range_len, with_indices ? 1 : 0);
+    const size_t ws_bytes = mam_fc_forward_ranges_workspace_at(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
+                                                               row_stride(weight, "weight"), MAM_W_MK, s.N, s.K, s.M, range_len,
+                                                               with_indices ? 1 : 0);
     auto ws = workspace_for(ws_bytes, a);
     check_rc(mam_fc_forward_ranges(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
                                    row_stride(weight, "weight"), MAM_W_MK, bias_ptr(bias), c.data_ptr<float>(),

@@ -176,6 +176,40 @@ def test_the_workspace_of_a_call_holds_what_the_call_makes_use_of(N, K, M, mk, w
         assert asked == (int(named.group(1)) if named else int(partials.group(1)) if partials else 0)
 
 
+@pytest.mark.parametrize("N, K, M, range_len", [(16384, 4096, 4096, 1024), (256, 4096, 4096, 1024), (300, 208, 90, 128), (40, 128, 64, 64)])
+@pytest.mark.parametrize("with_indices", [0, 1])
+def test_whole_ranges_ask_for_their_partials_alone(N, K, M, range_len, with_indices):
+    # ranges of whole tiles run on the operands as they are, as they do by any (K, M) weight
+    l = capi.lib()
+    one, ranges = ctypes.c_void_p(256), -(-K // range_len)
+    partials = ranges * N * M * (12 if with_indices else 8)
+    assert l.mam_fc_forward_ranges_workspace(N, K, M, range_len, with_indices) == partials
+    assert l.mam_fc_forward_ranges_workspace_at(one, K, one, K, capi.W_MK, N, K, M, range_len, with_indices) == partials
+    odd = range_len - 3
+    assert l.mam_fc_forward_ranges_workspace_at(one, K, one, (M + 3) // 4 * 4, capi.W_KM, N, K, M, odd, with_indices) == -(-K // odd) * partials // ranges
+
+
+@pytest.mark.parametrize("rows_x", sorted(ROWS))
+@pytest.mark.parametrize("rows_w", sorted(ROWS))
+@pytest.mark.parametrize("with_indices", [0, 1])
+@pytest.mark.parametrize("N, K, M, range_len", [(33, 130, 70, 65), (496, 691, 105, 173), (4000, 531, 3712, 133), (160, 3200, 512, 800), (64, 1000, 64, 250),
+                                                (40, 8, 5, 2), (9536, 2809, 1432, 703)])
+def test_the_workspace_of_ranges_holds_their_copies(N, K, M, range_len, with_indices, rows_x, rows_w):
+    l = capi.lib()
+    (px, dx), (pw, dw) = ROWS[rows_x], ROWS[rows_w]
+    whole = (K + 3) // 4 * 4
+    asked = l.mam_fc_forward_ranges_workspace_at(ctypes.c_void_p(px), whole + dx, ctypes.c_void_p(pw), whole + dw, capi.W_MK, N, K, M, range_len,
+                                                 with_indices)
+    partials = -(-K // range_len) * N * M * (12 if with_indices else 8)
+    # never more than the query by sizes, and no copy of x of as many neurons as these
+    assert partials <= asked <= l.mam_fc_forward_ranges_workspace(N, K, M, range_len, with_indices)
+    if range_len < 32:
+        assert asked == partials
+    elif with_indices:
+        copy = 4 * M * -(-K // range_len) * -(-range_len // 64) * 64
+        assert asked == partials + -(-copy // 256) * 256 if M <= 1536 else asked > partials + copy
+
+
 def test_workspace_queries_are_pure_host_calls():
     l = capi.lib()
     assert l.mam_fc_forward_workspace(12608, 768, 3072) == 0          # enough tiles: no split-K
