@@ -256,8 +256,8 @@ int mam_fc_backward_count(const float *x, int64_t ldx, const float *w, int64_t l
  * mam_fc_forward_ranges_workspace() bytes (0 when range_len >= K, which is mam_fc_forward): partials for every range and, for ranges that
  * are not whole 64-k tiles, the copies of (M, K) operands that make the call 1.1 to 2.5 times as fast.  Partials are enough
  * (ranges * N * M * (with_indices ? 12 : 8) bytes), and all that a (K, M) weight in such ranges makes use of.
- * mam_fc_forward_ranges_workspace_at(): what a call with these operands makes use of, in a workspace at a 16-byte address; the pointers
- * are looked at but never dereferenced.
+ * mam_fc_forward_ranges_workspace_at(): what a call with these operands makes use of (of a (K, M) weight in ranges of whole tiles, its
+ * transposed copy), in a workspace at a 16-byte address; the pointers are looked at but never dereferenced.
  *   mam_fc_backward_ranges: the gradient of that c: every range routes grad[n,m] to its own two
  * selected positions.  x_grad (N,K), w_grad (shape and layout of w), either may be NULL.
  */

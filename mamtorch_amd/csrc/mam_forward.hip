@@ -1594,13 +1594,15 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
                                  N, K, M, range_len, &tail);
         if (rc == MAM_OK && staged.use_sx && staged.p.coop) return true;
     }
-    st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M, range_len);
+    // (a transposed weight keeps its ranges as they are: they have to be whole tiles, and x is not copied)
+    st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M, turn ? 0 : range_len);
     if (!st.rows_fit(N, M, turn) || (turn && !transposed_operand_pays(N, K, M))) return false;
     const bool lengthen = st.x || (st.w && !turn);
-    if (ranges ? turn || st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args) : lengthen && !lengthened_rows_pay(N, K, M, turn, args)) return false;
+    if (ranges ? (turn ? st.x || range_len % sx::KT != 0 : st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args))
+               : lengthen && !lengthened_rows_pay(N, K, M, turn, args)) return false;
     float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
     const int rc = make_plan(staged, args, st.x ? aligned : x, st.x ? st.K : ldx, st.w ? aligned : w, st.w ? st.K : ldw, MAM_W_MK, bias,
-                             c, argmax, argmin, w_sel, x_sel, N, st.K, M, ranges ? st.K / ceil_div(K, range_len) : range_len);
+                             c, argmax, argmin, w_sel, x_sel, N, st.K, M, ranges && !turn ? st.K / ceil_div(K, range_len) : range_len);
     if (ranges) staged.p.range_len = (int)range_len;
     return rc == MAM_OK && staged.use_sx;
 }

@@ -189,6 +189,17 @@ def test_whole_ranges_ask_for_their_partials_alone(N, K, M, range_len, with_indi
     assert l.mam_fc_forward_ranges_workspace_at(one, K, one, (M + 3) // 4 * 4, capi.W_KM, N, K, M, odd, with_indices) == -(-K // odd) * partials // ranges
 
 
+@pytest.mark.parametrize("N, K, M, range_len, turned", [(256, 4096, 4096, 1024, True), (16, 208, 90, 128, True), (15, 4096, 64, 1024, False),
+                                                        (64, 208, 90, 104, False), (64, 200, 90, 128, False)])
+@pytest.mark.parametrize("with_indices", [0, 1])
+def test_whole_ranges_of_a_km_weight_run_on_its_transposed_copy(N, K, M, range_len, turned, with_indices):
+    l = capi.lib()
+    x, w = ctypes.c_void_p(256), ctypes.c_void_p(260)
+    partials = -(-K // range_len) * N * M * (12 if with_indices else 8)
+    copy = -(-4 * M * K // 256) * 256 if turned else 0
+    assert l.mam_fc_forward_ranges_workspace_at(x, K, w, M, capi.W_KM, N, K, M, range_len, with_indices) == partials + copy
+
+
 @pytest.mark.parametrize("rows_x", sorted(ROWS))
 @pytest.mark.parametrize("rows_w", sorted(ROWS))
 @pytest.mark.parametrize("with_indices", [0, 1])
