@@ -70,22 +70,31 @@ at::Tensor workspace_for(size_t bytes, const at::Tensor &like)
     return at::empty({static_cast<int64_t>(bytes)}, like.options().dtype(at::kByte));
 }
 
+// `most` bytes, or, where the device has not that much left, the `least()` that the call cannot do without
+template <class Least>
+at::Tensor workspace_for(size_t most, const at::Tensor &like, const Least &least)
+{
+    size_t bytes = 0;
+    try {
+        return workspace_for(most, like);
+    } catch (const c10::OutOfMemoryError &) {
+        bytes = least();
+        if (bytes >= most) throw;
+    }
+    return workspace_for(bytes, like);
+}
+
 struct FwdShape { int64_t N, K, M; };
 
 // The workspace of a forward call with room for all that makes it faster (lists and copies of the operands: 0.5 GB at 16384 x
-// 4096 -> 4096), or, where the device has not that much left, what the call cannot do without.
+// 4096 -> 4096), or what the call cannot do without.
 at::Tensor forward_workspace(const FwdShape &s, const at::Tensor &a, const at::Tensor &w, int layout, bool with_indices)
 {
     const size_t most = mam_fc_forward_workspace_at(a.data_ptr<float>(), row_stride(a, "a"), w.data_ptr<float>(),
                                                     row_stride(w, "the weight operand"), layout, s.N, s.K, s.M, with_indices ? 1 : 0);
-    size_t least = 0;
-    try {
-        return workspace_for(most, a);
-    } catch (const c10::OutOfMemoryError &) {
-        least = with_indices ? mam_fc_forward_workspace(s.N, s.K, s.M) : mam_fc_forward_values_workspace(s.N, s.K, s.M);
-        if (least >= most) throw;
-    }
-    return workspace_for(least, a);
+    return workspace_for(most, a, [&] {
+        return with_indices ? mam_fc_forward_workspace(s.N, s.K, s.M) : mam_fc_forward_values_workspace(s.N, s.K, s.M);
+    });
 }
 
 FwdShape check_forward(const at::Tensor &a, const at::Tensor &w, int layout,
@@ -315,12 +324,15 @@ std::vector<at::Tensor> fullyconnected_ranges(const at::Tensor &a, const at::Ten
     const size_t ws_bytes = mam_fc_forward_ranges_workspace_at(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
                                                                row_stride(weight, "weight"), MAM_W_MK, s.N, s.K, s.M, range_len,
                                                                with_indices ? 1 : 0);
-    auto ws = workspace_for(ws_bytes, a);
+    // (the partials alone: copies of the operands are left out)
+    auto ws = workspace_for(ws_bytes, a, [&] {
+        return ranges > 1 ? (size_t)ranges * (with_indices ? 3 : 2) * (size_t)s.N * (size_t)s.M * sizeof(float) : (size_t)0;
+    });
     check_rc(mam_fc_forward_ranges(a.data_ptr<float>(), row_stride(a, "a"), weight.data_ptr<float>(),
                                    row_stride(weight, "weight"), MAM_W_MK, bias_ptr(bias), c.data_ptr<float>(),
                                    with_indices ? argmax.data_ptr<int32_t>() : nullptr,
                                    with_indices ? argmin.data_ptr<int32_t>() : nullptr, s.N, s.K, s.M, range_len,
-                                   ws.defined() ? ws.data_ptr() : nullptr, ws_bytes, current_stream(a)),
+                                   ws.defined() ? ws.data_ptr() : nullptr, ws.defined() ? ws.numel() : 0, current_stream(a)),
              "mam_fc_forward_ranges");
     return {c, argmax, argmin};
 }

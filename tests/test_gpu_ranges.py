@@ -193,3 +193,27 @@ def test_lengthened_ranges_equal_the_general_tiling(N, K, M, range_len):
         assert_bits_equal(b, a, what)
     for a, b, what in zip(outs[0][2:], outs[1][2:], ("argmax", "argmin")):
         assert_index_equal(b, a, what)
+
+
+@pytest.mark.parametrize("indices", [True, False])
+def test_ranges_without_room_for_their_copies_still_run(indices):
+    """A device with too little memory left for the copies of the operands: the operator asks for the partials alone."""
+    N, K, M, range_len = 64, 8188, 8188, 4094
+    g = torch.Generator(device=DEV).manual_seed(10)
+    x, w = torch.randn(N, K, generator=g, device=DEV), torch.randn(M, K + 1, generator=g, device=DEV)[:, :K]
+    forward = lambda: torch.ops.mamtorch_kernel_v4.fullyconnected_ranges(x, w, None, range_len, indices)
+    want = forward()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    from mamtorch_amd import capi
+    least = 2 * (3 if indices else 2) * N * M * 4 + 5 * N * M * 4
+    assert capi.lib().mam_fc_forward_ranges_workspace(N, K, M, range_len, int(indices)) > least + (96 << 20)
+    total = torch.cuda.get_device_properties(DEV).total_memory
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved(DEV) + least + (80 << 20)) / total, DEV)
+    try:
+        got = forward()
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0, DEV)
+    for one, other in zip(got, want):
+        assert torch.equal(one, other)
