@@ -58,8 +58,11 @@ __device__ __forceinline__ void lds_add_sparse(float *addr, float v)
     if (!done) lds_add(addr, v);
 }
 
+// PICKS, here and below: argmax holds both picks, packed, and argmin is not looked at.  Two instantiations: decided per load, calls with two
+// planes took 3 to 9 % longer (12608 x 768 -> 3072 w_grad 201 -> 210 us, 1536 x 1024 -> 256 11.4 -> 12.2, x_grad 19.7 -> 20.3).
+
 // The work of one workgroup of mam_bwd_x_kernel: batch row n, its kc cells in `cells`.
-template <int LAYOUT>
+template <int LAYOUT, bool PICKS>
 __device__ __forceinline__ void bwd_x_body(
     unsigned long long *cells, int n, const float *__restrict__ w, int64_t ldw, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
@@ -80,7 +83,7 @@ __device__ __forceinline__ void bwd_x_body(
     int a1[4], a2[4];
     auto load_trip = [&](int pl, int mb, int k0, int kn) {
         const int32_t *amax_row = argmax + pl * nm + (int64_t)n * M;
-        const int32_t *amin_row = argmin ? argmin + pl * nm + (int64_t)n * M : nullptr;
+        const int32_t *amin_row = PICKS ? nullptr : argmin + pl * nm + (int64_t)n * M;
         const float *w_sel_pl = w_sel ? w_sel + pl * 2 * nm : nullptr;
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -88,8 +91,8 @@ __device__ __forceinline__ void bwd_x_body(
             const bool ok = m < M;
             g[u] = ok ? g_row[m] : 0.0f;
             a1[u] = ok ? amax_row[m] : -1;
-            if (amin_row) a2[u] = ok ? amin_row[m] : -1;
-            else unpack_picks(a1[u], a2[u]);
+            if (PICKS) unpack_picks(a1[u], a2[u]);
+            else a2[u] = ok ? amin_row[m] : -1;
             a1[u] -= k0;
             a2[u] -= k0;
         }
@@ -181,7 +184,7 @@ __device__ __forceinline__ void bwd_x_body(
     }
 }
 
-template <int LAYOUT>
+template <int LAYOUT, bool PICKS>
 __global__ __launch_bounds__(NT_X) void mam_bwd_x_kernel(
     const float *__restrict__ w, int64_t ldw, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
@@ -189,7 +192,7 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_x_kernel(
     int span)
 {
     extern __shared__ unsigned long long cells[];
-    bwd_x_body<LAYOUT>(cells, blockIdx.x, w, ldw, grad, argmax, argmin, w_sel, nm, x_grad, K, M, kc, planes, span);
+    bwd_x_body<LAYOUT, PICKS>(cells, blockIdx.x, w, ldw, grad, argmax, argmin, w_sel, nm, x_grad, K, M, kc, planes, span);
 }
 
 // x_grad for large batches: a workgroup owns R = 2 .. 16 batch rows with their whole K cells in LDS,
@@ -199,7 +202,7 @@ __global__ __launch_bounds__(NT_X) void mam_bwd_x_kernel(
 // same row can, and the loads of a wave are whole 64-byte (R = 16) to 512-byte (R = 2) pieces of R rows.
 // Cells are 64-bit fixed point as above; the fp32 fallback settles a term by one compare-and-swap round
 // where it can.
-template <int LAYOUT>
+template <int LAYOUT, bool PICKS>
 __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
     const float *__restrict__ w, int64_t ldw, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
@@ -227,10 +230,10 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
     do {                                                                                            \
         if (row_ok && (m) < M) {                                                                    \
             const int64_t o_ = (int64_t)n * M + (m);                                                \
-            const int left_ = quads ? 4 : M - (m);                                                           \
+            const int left_ = quads ? 4 : M - (m);                                                  \
             g = row_quad(grad + o_, left_);                                                         \
             i1 = row_quad(argmax + (pl) * nm + o_, left_);                                          \
-            if (argmin) {                                                                           \
+            if (!PICKS) {                                                                           \
                 i2 = row_quad(argmin + (pl) * nm + o_, left_);                                      \
             } else {                                                                                \
                 unpack_picks(i1.x, i2.x);                                                           \
@@ -350,14 +353,14 @@ struct Item {
 };
 
 // (one branch for all loads of an item, which are then in flight together)
-template <int Q>
+template <bool PICKS, int Q>
 __device__ __forceinline__ void load_item(Item<Q> &it, const float *grad, const int32_t *argmax, const int32_t *argmin,
                                           const float *x_sel, int64_t nm, int left)
 {
     if (left >= Q) {
         row_words<Q>(grad, Q, 0.0f, it.g);
         row_words<Q>(argmax, Q, -1, it.a1);
-        if (argmin) row_words<Q>(argmin, Q, -1, it.a2);
+        if (!PICKS) row_words<Q>(argmin, Q, -1, it.a2);
         if (x_sel) {
             row_words<Q>(x_sel, Q, 0.0f, it.x1);
             row_words<Q>(x_sel + nm, Q, 0.0f, it.x2);
@@ -365,13 +368,13 @@ __device__ __forceinline__ void load_item(Item<Q> &it, const float *grad, const 
     } else {
         row_words<Q>(grad, left, 0.0f, it.g);
         row_words<Q>(argmax, left, -1, it.a1);
-        if (argmin) row_words<Q>(argmin, left, -1, it.a2);
+        if (!PICKS) row_words<Q>(argmin, left, -1, it.a2);
         if (x_sel) {
             row_words<Q>(x_sel, left, 0.0f, it.x1);
             row_words<Q>(x_sel + nm, left, 0.0f, it.x2);
         }
     }
-    if (!argmin)
+    if (PICKS)
 #pragma unroll
         for (int u = 0; u < Q; ++u) unpack_picks(it.a1[u], it.a2[u]);
 }
@@ -488,7 +491,7 @@ __device__ __forceinline__ void store_slab(const float *hist, float *__restrict_
 // fixed order.  BIAS_TERMS of a thread's items make a sum of their own, so that rounding errors do not grow with the batch (one
 // running sum per thread: 2-norm error 1.07e-6 for 400000 rows where mam_bias_grad's 256 running sums give 6.5e-7).
 constexpr int BIAS_TERMS = 64;
-template <int LAYOUT, int NT, bool COUNT, bool BIAS, int Q>
+template <int LAYOUT, int NT, bool COUNT, bool BIAS, int Q, bool PICKS>
 __device__ __forceinline__ void bwd_w_vec_body(
     float *hist, int bx, int nbx, int by, int bz, int nbz,
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
@@ -532,7 +535,8 @@ __device__ __forceinline__ void bwd_w_vec_body(
         have = tid < items && m0 + r_first < M;
         if (have) {
             const int64_t o = (int64_t)n_first * M + m0 + r_first;
-            load_item(it1, grad + o, argmax + po_first + o, argmin ? argmin + po_first + o : nullptr, x_sel ? x_sel + 2 * po_first + o : nullptr, nm, M - m0 - r_first);
+            load_item<PICKS>(it1, grad + o, argmax + po_first + o, PICKS ? nullptr : argmin + po_first + o,
+                             x_sel ? x_sel + 2 * po_first + o : nullptr, nm, M - m0 - r_first);
         }
     };
     if (first < mtiles) load_first(first * R);
@@ -568,7 +572,8 @@ __device__ __forceinline__ void bwd_w_vec_body(
             const int64_t o = (int64_t)n * M + m0 + r0;
             const int64_t po = (int64_t)(pl_lo + pl) * nm;
             Item<Q> it;
-            load_item(it, grad + o, argmax + po + o, argmin ? argmin + po + o : nullptr, x_sel ? x_sel + 2 * po + o : nullptr, nm, M - m0 - r0);
+            load_item<PICKS>(it, grad + o, argmax + po + o, PICKS ? nullptr : argmin + po + o, x_sel ? x_sel + 2 * po + o : nullptr, nm,
+                             M - m0 - r0);
             if (!x_sel) gather_item(it, x + (int64_t)n * ldx, k0, kn);
             scatter_item<LAYOUT, COUNT>(hist, it, n, r0, k0, kn, kc, log2r, cnt);
             if (sum_bias && pl == 0) {
@@ -603,7 +608,7 @@ __device__ __forceinline__ void bwd_w_vec_body(
     }
 }
 
-template <int LAYOUT, bool BIAS, int NT, int Q>
+template <int LAYOUT, bool BIAS, int NT, int Q, bool PICKS>
 __global__ __launch_bounds__(NT) void mam_bwd_w_vec_kernel(
     const float *__restrict__ x, int64_t ldx, const float *__restrict__ grad,
     const int32_t *__restrict__ argmax, const int32_t *__restrict__ argmin,
@@ -612,7 +617,7 @@ __global__ __launch_bounds__(NT) void mam_bwd_w_vec_kernel(
     float *__restrict__ bias_out)
 {
     extern __shared__ float hist[];
-    bwd_w_vec_body<LAYOUT, NT, false, BIAS, Q>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
+    bwd_w_vec_body<LAYOUT, NT, false, BIAS, Q, PICKS>(hist, blockIdx.x, gridDim.x, blockIdx.y, blockIdx.z, gridDim.z, x, ldx, grad, argmax,
                                  argmin, x_sel, nm, w_grad, N, K, M, log2r, kc, vec_out, mtiles, tiles_per_wg,
                                  rows_per_split, planes, range_len, nullptr, nullptr, bias_out);
 }
@@ -626,7 +631,7 @@ __global__ __launch_bounds__(NT_C) void mam_bwd_w_count_kernel(
     int32_t *__restrict__ min_count, int N, int K, int M, int log2r, int kc, int mtiles, int tiles_per_wg)
 {
     extern __shared__ float hist[];
-    bwd_w_vec_body<MAM_W_MK, NT_C, true, false, 4>(hist, blockIdx.x, gridDim.x, blockIdx.y, 0, 1, x, ldx, grad, argmax, argmin,
+    bwd_w_vec_body<MAM_W_MK, NT_C, true, false, 4, false>(hist, blockIdx.x, gridDim.x, blockIdx.y, 0, 1, x, ldx, grad, argmax, argmin,
                                          x_sel, nm, w_grad, N, K, M, log2r, kc, 1, mtiles, tiles_per_wg, N, 1, K,
                                          max_count, min_count);
 }
@@ -778,15 +783,15 @@ struct BothParams {
     int N, K, M, planes, range_len, span, kc_x;
     int log2r, kc_w, vec_out, mtiles, tiles_per_wg, x_wgs;
 };
-template <int LAYOUT, bool BIAS>
+template <int LAYOUT, bool BIAS, bool PICKS>
 __global__ __launch_bounds__(NT_X) void mam_bwd_both_kernel(const BothParams p)
 {
     extern __shared__ unsigned long long both_lds[];
     if ((int)blockIdx.x < p.x_wgs) {
-        bwd_x_body<LAYOUT>(both_lds, blockIdx.x, p.w, p.ldw, p.grad, p.argmax, p.argmin, p.w_sel, p.nm, p.x_grad, p.K,
+        bwd_x_body<LAYOUT, PICKS>(both_lds, blockIdx.x, p.w, p.ldw, p.grad, p.argmax, p.argmin, p.w_sel, p.nm, p.x_grad, p.K,
                            p.M, p.kc_x, p.planes, p.span);
     } else {
-        bwd_w_vec_body<LAYOUT, NT_X, false, BIAS, 4>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
+        bwd_w_vec_body<LAYOUT, NT_X, false, BIAS, 4, PICKS>(reinterpret_cast<float *>(both_lds), blockIdx.x - p.x_wgs, gridDim.x - p.x_wgs, 0,
                                      0, 1, p.x, p.ldx, p.grad, p.argmax, p.argmin, p.x_sel, p.nm, p.w_grad, p.N, p.K,
                                      p.M, p.log2r, p.kc_w, p.vec_out, p.mtiles, p.tiles_per_wg, p.N, p.planes,
                                      p.range_len, nullptr, nullptr, p.bias_grad);
@@ -805,12 +810,20 @@ constexpr int64_t kRowsLdsBytes = MAM_BWD_ROWS_LDS;
 static int setup_device(int dev)
 {
     constexpr int kWant = 128 * 1024;
+#define MAM_BOTH_FORMS(...) (const void *)__VA_ARGS__, false>, (const void *)__VA_ARGS__, true>
     const void *kernels[] = {
-        (const void *)mam_bwd_x_rows_kernel<MAM_W_MK>, (const void *)mam_bwd_x_rows_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_x_kernel<MAM_W_MK>,      (const void *)mam_bwd_x_kernel<MAM_W_KM>,
-        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false, NT_W, 4>, (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, false, NT_W, 2>,  (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, false, NT_X, 4>,
-        (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 4>, (const void *)mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 2>,   (const void *)mam_bwd_w_vec_kernel<MAM_W_KM, true, NT_X, 4>,
-        (const void *)mam_bwd_both_kernel<MAM_W_MK, false>,   (const void *)mam_bwd_both_kernel<MAM_W_MK, true>,
+        MAM_BOTH_FORMS(mam_bwd_x_rows_kernel<MAM_W_MK),
+        MAM_BOTH_FORMS(mam_bwd_x_rows_kernel<MAM_W_KM),
+        MAM_BOTH_FORMS(mam_bwd_x_kernel<MAM_W_MK),
+        MAM_BOTH_FORMS(mam_bwd_x_kernel<MAM_W_KM),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_MK, false, NT_W, 4),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 4),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_MK, false, NT_W, 2),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 2),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, false, NT_X, 4),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, true, NT_X, 4),
+        MAM_BOTH_FORMS(mam_bwd_both_kernel<MAM_W_MK, false),
+        MAM_BOTH_FORMS(mam_bwd_both_kernel<MAM_W_MK, true),
         (const void *)mam_bwd_w_count_kernel,
     };
     bool all = true;
@@ -862,6 +875,13 @@ static int64_t most_shares(int64_t N, int64_t K, int64_t M)
     return few > many ? few : many;
 }
 
+template <int LAYOUT, int NT, int Q>
+static auto w_kernel(bool bias, bool picks)
+{
+    if (picks) return bias ? mam_bwd_w_vec_kernel<LAYOUT, true, NT, Q, true> : mam_bwd_w_vec_kernel<LAYOUT, false, NT, Q, true>;
+    return bias ? mam_bwd_w_vec_kernel<LAYOUT, true, NT, Q, false> : mam_bwd_w_vec_kernel<LAYOUT, false, NT, Q, false>;
+}
+
 template <int LAYOUT>
 static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *grad,
                          const int32_t *argmax, const int32_t *argmin, const float *w_sel, const float *x_sel,
@@ -884,7 +904,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
         int log2r = 1;
         while (log2r < 4 && ((int64_t)2 << log2r) * K * 8 <= rows_budget) ++log2r;
         const int R = 1 << log2r;
-        hipLaunchKernelGGL((mam_bwd_x_rows_kernel<LAYOUT>), dim3((unsigned)ceil_div(N, R)), dim3(NT_W),
+        hipLaunchKernelGGL((argmin ? mam_bwd_x_rows_kernel<LAYOUT, false> : mam_bwd_x_rows_kernel<LAYOUT, true>), dim3((unsigned)ceil_div(N, R)), dim3(NT_W),
                            (size_t)R * K * 8, st, w, ldw, grad, argmax, argmin, w_sel, N * M, x_grad,
                            (int)N, (int)K, (int)M, log2r, planes, span);
         rc = check_launch("mam_bwd_x_rows_kernel");
@@ -892,7 +912,7 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
     } else if (x_grad) {
         const int cells_cap = (lds_cap - 2048) / 2;     // 8-byte cells, 8 KiB kept free for the static LDS
         const int kc = (int)(K < cells_cap ? K : cells_cap);
-        hipLaunchKernelGGL((mam_bwd_x_kernel<LAYOUT>), dim3((unsigned)N), dim3(NT_X),
+        hipLaunchKernelGGL((argmin ? mam_bwd_x_kernel<LAYOUT, false> : mam_bwd_x_kernel<LAYOUT, true>), dim3((unsigned)N), dim3(NT_X),
                            (size_t)kc * 8, st, w, ldw, grad, argmax, argmin, w_sel, N * M,
                            x_grad, (int)K, (int)M, kc, planes, span);
         rc = check_launch("mam_bwd_x_kernel");
@@ -955,9 +975,8 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
         constexpr int Q = LAYOUT == MAM_W_MK ? 2 : 4;
         const bool pairs = Q == 2 && (N < 2048 ? K <= 2048 || M % 4 != 0 : shares == 1 && M % 4 != 0);
         float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
-        hipLaunchKernelGGL((pairs ? bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true, NT, Q> : mam_bwd_w_vec_kernel<LAYOUT, false, NT, Q>
-                                  : bias_out ? mam_bwd_w_vec_kernel<LAYOUT, true, NT, 4> : mam_bwd_w_vec_kernel<LAYOUT, false, NT, 4>),
-                           dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT),
+        const auto kernel = pairs ? w_kernel<LAYOUT, NT, Q>(bias_out, !argmin) : w_kernel<LAYOUT, NT, 4>(bias_out, !argmin);
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT),
                            (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
                            w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
                            (int)rows_per_share, planes, range_len, bias_out);
@@ -1013,7 +1032,9 @@ static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw,
     p.log2r = log2r; p.kc_w = (int)kc_w; p.vec_out = (K % 4 == 0) && ((uintptr_t)w_grad % 16 == 0);
     p.mtiles = (int)mtiles; p.tiles_per_wg = tpw; p.x_wgs = (int)N;
     const size_t lds = (size_t)(K * 8 > R * kc_w * 4 ? K * 8 : R * kc_w * 4);
-    hipLaunchKernelGGL((bias ? mam_bwd_both_kernel<MAM_W_MK, true> : mam_bwd_both_kernel<MAM_W_MK, false>), dim3((unsigned)(N + w_wgs)), dim3(NT_X), lds, st, p);
+    const auto two_planes = bias ? mam_bwd_both_kernel<MAM_W_MK, true, false> : mam_bwd_both_kernel<MAM_W_MK, false, false>;
+    const auto picks = bias ? mam_bwd_both_kernel<MAM_W_MK, true, true> : mam_bwd_both_kernel<MAM_W_MK, false, true>;
+    hipLaunchKernelGGL((argmin ? two_planes : picks), dim3((unsigned)(N + w_wgs)), dim3(NT_X), lds, st, p);
     return check_launch("mam_bwd_both_kernel");
 }
 
@@ -1063,7 +1084,7 @@ int x_grad_from_selected(const float *grad, const int32_t *argmax, const int32_t
     if (dev < 0) return dev;
     const int cells_cap = (g_lds_floats[dev] - 2048) / 2;
     const int kc = (int)(K < cells_cap ? K : cells_cap);
-    hipLaunchKernelGGL((mam_bwd_x_kernel<MAM_W_MK>), dim3((unsigned)N), dim3(NT_X), (size_t)kc * 8,
+    hipLaunchKernelGGL((mam_bwd_x_kernel<MAM_W_MK, false>), dim3((unsigned)N), dim3(NT_X), (size_t)kc * 8,
                        st, (const float *)nullptr, (int64_t)0, grad, argmax, argmin, w_sel, N * M, x_grad, (int)K,
                        (int)M, kc, 1, window_span(2 * M));
     return check_launch("mam_bwd_x_kernel");
