@@ -822,6 +822,10 @@ static int setup_device(int dev)
         MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_MK, true, NT_W, 2),
         MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, false, NT_X, 4),
         MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, true, NT_X, 4),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, false, NT_X, 2),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, true, NT_X, 2),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, false, NT_W, 4),
+        MAM_BOTH_FORMS(mam_bwd_w_vec_kernel<MAM_W_KM, true, NT_W, 4),
         MAM_BOTH_FORMS(mam_bwd_both_kernel<MAM_W_MK, false),
         MAM_BOTH_FORMS(mam_bwd_both_kernel<MAM_W_MK, true),
         (const void *)mam_bwd_w_count_kernel,
@@ -873,6 +877,32 @@ static int64_t most_shares(int64_t N, int64_t K, int64_t M)
     if (few > N / SHARE_ROWS) few = N / SHARE_ROWS;
     const int64_t many = shares_of_many_rows(N, K);
     return few > many ? few : many;
+}
+
+// Neurons of an item of w_grad and threads of a workgroup.
+enum WForm { QUADS, PAIRS, QUADS_1024 };
+
+// (M,K), 512 threads: pairs where the items of a slab are few, so that more lanes share them and more waves fit (65 registers instead of 91): us with
+// quads / pairs, kernel alone: 496 x 691 in four ranges -> 105 9.6 / 9.0, 910 x 192 -> 768 10.4 / 9.5, 472 x 1050 in four ranges -> 2145 71 / 62,
+// 1238 x 662 -> 3590 38.4 / 35.0; not for long slabs, which their stores bound (256 x 4096 -> 4096 16.4 / 18.2).  From 2048 rows on where
+// quads straddle lines and no shares are there (2178 x 1494 -> 1982 39 / 28, -> 1983 47 / 37, -> 1984 25.5 / 27).
+static WForm w_form_mk(int64_t N, int64_t K, int64_t M, int64_t shares)
+{
+    return (N < 2048 ? K <= 2048 || M % 4 != 0 : shares == 1 && M % 4 != 0) ? PAIRS : QUADS;
+}
+
+// (K,M), a workgroup per CU (its 128 KiB slab): us with quads of 512 threads / quads of 1024 / pairs of 1024, kernel alone: 256 x 1024 -> 1024 17.6 /
+// 15.6 / 13.4, 512 x 768 -> 3072 30.5 / 31.0 / 26.8, 2048 x 1024 -> 256 130 / 140 / 114, 12608 x 384 -> 1536 464 / 551 / 395, 19136 x 368 -> 256 831 /
+// 910 / 507.  Quads of 1024 where pairs of them find no work (64 x 784 -> 256 9.0 / 7.4 / 7.9, 64 x 64 -> 64 5.9 / 5.8 / 6.6; 128 x 300 -> 1000 9.2 / 9.9 /
+// 8.7) and where a slab holds less than a third of the picks that it reads (1024 x 4096 -> 1024 45 / 32 / 34, 4000 x 4096 -> 1024 140 / 96 / 106; 2500 x
+// 2500 -> 2500 101 / 101 / 84, 1024 x 3072 -> 1024 46 / 37 / 35).  Quads of 512 where a slab is a few KiB that all lanes add to (3708 x 64 -> 44 123 / 173 /
+// 164, 1000 x 96 -> 1000 38 / 49 / 45, 462 x 105 -> 107 19.4 / 23 / 21.5; 1000 x 200 -> 500 35.8 / 39.6 / 36.0) and where gradient and picks are more than
+// the memory-side cache holds (12608 x 768 -> 3072 644 / 792 / 806, 6300 x 1024 -> 4096 354 / 411 / 406; 12608 x 384 -> 1536 as above).
+static WForm w_form_km(int64_t N, int64_t K, int64_t M, int planes)
+{
+    constexpr int64_t kMemorySideCache = (int64_t)256 << 20;
+    if (N < 128 || K > 3072) return QUADS_1024;
+    return K < 128 || N * M * (4 + 8 * planes) > kMemorySideCache ? QUADS : PAIRS;
 }
 
 template <int LAYOUT, int NT, int Q>
@@ -957,7 +987,6 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
         if (tpw > 8) tpw = 8;
         // workgroups of a CU by the slab's LDS and their threads (registers leave room for two, so the bias gradient's 1 KiB beside the slab
         // changes nothing: 16384 x 620 / 640 / 656 -> 1024, three or four by LDS, 176 / 176 / 180 us)
-        constexpr int NT = LAYOUT == MAM_W_MK ? NT_W : NT_X;
         int64_t per_cu = (160 * 1024) / ((int64_t)R * kc * 4);
         if (per_cu > 2048 / NT_W) per_cu = 2048 / NT_W;
         if (per_cu < 1) per_cu = 1;
@@ -968,15 +997,13 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
             rc = fill_zero(w_grad, M * K, st);
             if (rc != MAM_OK) return rc;
         }
-        // Items of two neurons where the items of a slab are few, so that more lanes share them and more waves fit (65 registers instead of 91): us with
-        // four / two, kernel alone: 496 x 691 in four ranges -> 105 9.6 / 9.0, 910 x 192 -> 768 10.4 / 9.5, 472 x 1050 in four ranges -> 2145 71 / 62,
-        // 1238 x 662 -> 3590 38.4 / 35.0; not for long slabs, which their stores bound (256 x 4096 -> 4096 16.4 / 18.2).  From 2048 rows on where
-        // quads straddle lines and no shares are there (2178 x 1494 -> 1982 39 / 28, -> 1983 47 / 37, -> 1984 25.5 / 27).
-        constexpr int Q = LAYOUT == MAM_W_MK ? 2 : 4;
-        const bool pairs = Q == 2 && (N < 2048 ? K <= 2048 || M % 4 != 0 : shares == 1 && M % 4 != 0);
         float *bias_out = !bias ? nullptr : shares == 1 ? bias->out : bias->partials >= shares ? bias->partial : nullptr;
-        const auto kernel = pairs ? w_kernel<LAYOUT, NT, Q>(bias_out, !argmin) : w_kernel<LAYOUT, NT, 4>(bias_out, !argmin);
-        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3(NT),
+        const WForm form = LAYOUT == MAM_W_MK ? w_form_mk(N, K, M, shares) : w_form_km(N, K, M, planes);
+        const auto kernel = form == PAIRS ? w_kernel<LAYOUT, LAYOUT == MAM_W_MK ? NT_W : NT_X, 2>(bias_out, !argmin) :
+                            form == QUADS ? w_kernel<LAYOUT, NT_W, 4>(bias_out, !argmin) :
+                                            w_kernel<LAYOUT, LAYOUT == MAM_W_MK ? NT_W : NT_X, 4>(bias_out, !argmin);
+        const int threads = LAYOUT == MAM_W_MK || form == QUADS ? NT_W : NT_X;
+        hipLaunchKernelGGL(kernel, dim3((unsigned)ceil_div(mtiles, tpw), (unsigned)ktiles, (unsigned)shares), dim3((unsigned)threads),
                            (size_t)R * kc * sizeof(float), st, x, ldx, grad, argmax, argmin, x_sel, N * M,
                            w_grad, (int)N, (int)K, (int)M, log2r, kc, vec_out, (int)mtiles, tpw,
                            (int)rows_per_share, planes, range_len, bias_out);

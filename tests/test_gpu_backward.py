@@ -581,3 +581,42 @@ def test_indices_that_do_not_fit_a_word_are_refused():
         capi.fc_forward_picks(x, w, capi.W_MK)
     with pytest.raises(RuntimeError):
         capi.fc_backward_picks(x, w, g, torch.zeros(2, 3, dtype=torch.int32, device=dev), capi.W_MK)
+
+
+@pytest.mark.parametrize("shape", [(127, 300, 70), (128, 127, 65), (128, 128, 65), (130, 129, 31), (128, 3072, 34), (128, 3073, 34), (1030, 128, 33),
+                                   (2051, 96, 7), (300, 1025, 97)])
+def test_every_form_of_a_km_weight_gradient(shape):
+    """Quads and pairs of neurons, workgroups of 512 and of 1024 threads: either side of each line between them, slabs of K and of M that end
+    early, arrays at any word, bias gradient among them."""
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    N, K, M = shape
+    x, w, grad = random_case(N, K, M, seed=sum(shape))
+    g = torch.Generator().manual_seed(N)
+    amax = torch.randint(0, K, (N, M), generator=g, dtype=torch.int32)
+    amin = torch.randint(0, min(K, 3), (N, M), generator=g, dtype=torch.int32)
+    _, wo = _check(x, w, grad, amax.numpy(), amin.numpy(), "(K, M) form %s" % (shape,), layouts=(0,))
+    _, ws = oracle.backward(x.abs().numpy(), w.abs().numpy(), grad.abs().numpy(), amax.numpy(), amin.numpy(), oracle.W_MK)
+    at_word = lambda t, off: torch.empty(t.numel() + off, dtype=t.dtype, device=dev)[off:].copy_(t.reshape(-1)).view(t.shape)
+    wd = w.T.contiguous().to(dev)
+    _, wg, bg = capi.fc_backward_bias(x.to(dev), wd, at_word(grad, 1), at_word(amax, 2), at_word(amin, 3), capi.W_KM)
+    assert (np.abs(wg.cpu().numpy().T - wo) <= RTOL * np.abs(wo) + FLOOR * ws + 1e-30).all()
+    gd = grad.double()
+    assert ((bg.cpu().double() - gd.sum(0)).abs() <= RTOL * gd.sum(0).abs() + FLOOR * gd.abs().sum(0) + 1e-30).all()
+
+
+def test_a_km_weight_gradient_of_more_than_the_memory_side_cache():
+    """Gradient and picks of 268 MB, whole numbers: sums in any order are exact."""
+    from mamtorch_amd import capi
+
+    dev = torch.device("cuda:0")
+    N, K, M = 22001, 130, 1017
+    g = torch.Generator(device=dev).manual_seed(5)
+    x, grad = (torch.randint(-9, 10, shape, generator=g, device=dev).float() for shape in ((N, K), (N, M)))
+    picks = [torch.randint(0, K, (N, M), generator=g, device=dev, dtype=torch.int32) for _ in range(2)]
+    _, wg = capi.fc_backward(x, torch.zeros(K, M, device=dev), grad, *picks, capi.W_KM, want_x=False)
+    want = torch.zeros(K, M, device=dev)
+    for p in picks:
+        want.scatter_add_(0, p.long(), torch.gather(x, 1, p.long()) * grad)
+    assert torch.equal(wg, want)
