@@ -1166,7 +1166,12 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
         // 8192 x 2048 -> 1024 113 / 121, 16384 x 4096 -> 1024 272 / 282; but 4096 x 1024 -> 1024 62 / 56, and with
         // 768 neurons (the rows kernel's workgroups are short and mostly waiting, and hold the LDS the w_grad
         // workgroups need) 12608 x 3072 -> 768 180 / 165, 25216 rows 335 / 316, 8192 rows 116 / 113.
-        ForkedStream fork(st, N * M, N * M >= (1 << 23) && M >= 1024);
+        // Not at all without the inputs handed over, from 2^21 outputs and 512 inputs on, (M,K): w_grad's workgroups then gather x, all of them along
+        // the batch at one pace, a row fetched once for all; beside x_grad they fall out of step and fetch it again (in a captured graph, us side by
+        // side / one after the other: 9792 x 1728 -> 803 371 / 278, 2500 x 1000 -> 1001 102 / 85, 12608 x 3072 -> 768 683 / 490, in four ranges 4000 x
+        // 1400 -> 704 432 / 240, 9000 x 600 -> 300 235 / 146, 4000 x 1024 -> 1500 470 / 477; but 2100 x 400 -> 2000 in four ranges 179 / 221).
+        const bool in_step = w_layout == MAM_W_MK && !x_sel && N * M >= (1 << 21) && K >= 512;
+        ForkedStream fork(st, N * M, !in_step && N * M >= (1 << 23) && M >= 1024, !in_step);
         if (fork.forked()) {
             const int rc_x = launch(x_grad, nullptr, fork.side());
             fork.join_later();
