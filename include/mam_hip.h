@@ -156,6 +156,9 @@ int mam_fc_forward_picks(const float *x, int64_t ldx, const float *w, int64_t ld
  */
 int mam_fc_forward_describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
                             int64_t N, int64_t K, int64_t M, int with_indices, char *text, size_t text_bytes);
+/* The same for mam_fc_forward_ranges (with_indices: with argmax and argmin). */
+int mam_fc_forward_ranges_describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K, int64_t M,
+                                   int64_t range_len, int with_indices, char *text, size_t text_bytes);
 
 /*
  * mam_fc_forward for callers that can neither allocate nor bring a workspace (code under HIP graph

@@ -31,7 +31,7 @@ COUNT_FLAGS = 2
 
 EXPORTS = (
     "mam_version", "mam_error_string", "mam_last_error", "mam_init", "mam_set_option", "mam_device_info",
-    "mam_fc_forward_static_limit", "mam_fc_forward_static", "mam_fc_forward_describe",
+    "mam_fc_forward_static_limit", "mam_fc_forward_static", "mam_fc_forward_describe", "mam_fc_forward_ranges_describe",
     "mam_fc_forward_workspace", "mam_fc_forward_workspace_for", "mam_fc_forward_workspace_at", "mam_fc_forward",
     "mam_fc_forward_values_workspace", "mam_fc_forward_values",
     "mam_fc_backward", "mam_fc_backward_count", "mam_selection_count",
@@ -78,6 +78,7 @@ def lib():
         l.mam_set_option.argtypes = [_int, _int]
         l.mam_fc_forward_describe.argtypes = [_ptr, _i64, _ptr, _i64, _int, _i64, _i64, _i64, _int, ctypes.c_char_p,
                                               _size]
+        l.mam_fc_forward_ranges_describe.argtypes = [_ptr, _i64, _ptr, _i64, _int, _i64, _i64, _i64, _i64, _int, ctypes.c_char_p, _size]
         l.mam_fc_forward_values.argtypes = [_ptr, _i64, _ptr, _i64, _int, _ptr, _ptr, _i64, _i64, _i64,
                                             _ptr, _size, _ptr]
         l.mam_fc_backward_bias_workspace.argtypes = [_i64, _i64, _i64]
@@ -189,6 +190,15 @@ def fc_forward_describe(x, w, layout=W_KM, with_indices=True):
     N, K, M = _dims(x, w, layout)
     buf = ctypes.create_string_buffer(640)
     _check(l.mam_fc_forward_describe(_p(x), _ld(x), _p(w), _ld(w), layout, N, K, M, 1 if with_indices else 0, buf, 640))
+    return buf.value.decode()
+
+
+def fc_forward_ranges_describe(x, w, range_len, layout=W_KM, with_indices=True):
+    """The same for mam_fc_forward_ranges."""
+    l = lib()
+    N, K, M = _dims(x, w, layout)
+    buf = ctypes.create_string_buffer(640)
+    _check(l.mam_fc_forward_ranges_describe(_p(x), _ld(x), _p(w), _ld(w), layout, N, K, M, range_len, 1 if with_indices else 0, buf, 640))
     return buf.value.decode()
 
 

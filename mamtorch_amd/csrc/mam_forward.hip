@@ -1860,41 +1860,43 @@ static void describe_plan(const mam::fwd::Plan &plan, int w_layout, int64_t K, b
     const fwd::Params &p = plan.p;
     const char *what = with_indices ? "args" : "values";
     if (plan.use_sx)
-        snprintf(text, text_bytes, "mam_fwd_sx_kernel<%s%s%s%s> %d x %d tiles of 32 x %d", what, p.splits > 1 ? ", split" : "",
-                 K % fwd::sx::KT == 0 ? "" : p.ragged ? ", last k tile at the end of K" : ", partial last k tile", p.gt > fwd::G ? ", indices per 32 k" : "", p.tiles_n,
-                 p.tiles_m, plan.narrow ? 64 : 128);
+        snprintf(text, text_bytes, "mam_fwd_sx_kernel<%s%s%s%s%s> %d x %d tiles of 32 x %d", what, p.splits > 1 ? ", split" : "",
+                 p.ragged ? ", last k tile at the end of K" : K % fwd::sx::KT == 0 ? "" : ", partial last k tile",
+                 p.gt > fwd::G ? ", indices per 32 k" : "", p.touch_x ? ", x fetched ahead" : "", p.tiles_n, p.tiles_m,
+                 plan.narrow ? 64 : 128);
     else
         snprintf(text, text_bytes, "mam_fwd_kernel<%s, %s> %d x %d tiles of 64 x 128", w_layout == MAM_W_MK ? "(M,K)" : "(K,M)",
                  what, p.tiles_n, p.tiles_m);
     if (p.splits > 1) {
         const size_t used = strlen(text);
-        snprintf(text + used, text_bytes - used, " x %d ranges of %d k + mam_fwd_merge_kernel<%s> (%zu bytes of partials)",
-                 p.splits, p.k_per_split, (with_indices && p.coop) ? "cooperative resolve" : "per-thread resolve",
+        const bool coop = with_indices && p.coop && (!p.own_ranges || p.ragged || p.k_per_split % fwd::G == 0);
+        snprintf(text + used, text_bytes - used, " x %d ranges of %d k + %s<%s> (%zu bytes of partials)", p.splits, p.k_per_split,
+                 p.own_ranges ? "mam_fwd_range_sum_kernel" : "mam_fwd_merge_kernel", coop ? "cooperative resolve" : "per-thread resolve",
                  plan.need);
     }
 }
 
-extern "C" int mam_fc_forward_describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
-                                       int64_t N, int64_t K, int64_t M, int with_indices, char *text, size_t text_bytes)
+static int describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K, int64_t M, int64_t range_len,
+                    int with_indices, char *text, size_t text_bytes)
 {
     using namespace mam;
     fwd::Plan plan;
     const int rc = fwd::make_plan(plan, with_indices != 0, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr,
-                                  nullptr, nullptr, nullptr, N, K, M);
+                                  nullptr, nullptr, nullptr, N, K, M, range_len);
     if (rc != MAM_OK) return rc;
     if (!text || text_bytes == 0) return fail(MAM_ERR_INVALID_ARGUMENT, "no text buffer");
     if (N == 0 || M == 0) {
         snprintf(text, text_bytes, "nothing to launch");
         return MAM_OK;
     }
-    // Operands are staged in the workspace when that has room (what mam_fc_forward_workspace_for() asks for) and the
+    // Operands are staged in the workspace when that has room (what mam_fc_forward_workspace_at() asks for) and the
     // wave-uniform-rows tiling then runs on the copies, and large calls go by lists: every route is named, the one a call
     // takes depends on the workspace it brings and, with lists, on the data.
     fwd::Plan tplan;
     fwd::Staging st;
     const bool staged = fwd::staged_plan(tplan, st, plan, with_indices != 0, x, ldx, w, ldw, w_layout, nullptr, nullptr, nullptr, nullptr,
-                                         nullptr, nullptr, N, K, M, 0);
-    if (ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22))) {
+                                         nullptr, nullptr, N, K, M, range_len);
+    if (range_len == 0 && ordered::applies(N, K, M) && (w_layout == MAM_W_MK || ldw < (1 << 22))) {
         const size_t dense = staged && st.bytes() + tplan.need < plan.need ? st.bytes() + tplan.need : plan.need;
         const int used = snprintf(text, text_bytes, "with %zu workspace bytes: magnitude-ordered lists (ordered::sample_kernel, build_kernel, "
                                   "forward_kernel) where the device finds that the data suits them; otherwise ",
@@ -1917,6 +1919,19 @@ extern "C" int mam_fc_forward_describe(const float *x, int64_t ldx, const float 
     }
     describe_plan(plan, w_layout, K, with_indices != 0, text, text_bytes);
     return MAM_OK;
+}
+
+extern "C" int mam_fc_forward_describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout,
+                                       int64_t N, int64_t K, int64_t M, int with_indices, char *text, size_t text_bytes)
+{
+    return describe(x, ldx, w, ldw, w_layout, N, K, M, 0, with_indices, text, text_bytes);
+}
+
+extern "C" int mam_fc_forward_ranges_describe(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, int64_t N, int64_t K,
+                                              int64_t M, int64_t range_len, int with_indices, char *text, size_t text_bytes)
+{
+    if (range_len <= 0) return mam::fail(MAM_ERR_INVALID_ARGUMENT, "range_len must be positive");
+    return describe(x, ldx, w, ldw, w_layout, N, K, M, range_len, with_indices, text, text_bytes);
 }
 
 extern "C" size_t mam_fc_forward_static_limit(void) { return mam::fwd::kStaticScratchBytes; }

@@ -179,6 +179,10 @@ def test_lengthened_ranges_equal_the_general_tiling(N, K, M, range_len):
     w[0], w[1, -1], w[2, :range_len], w[3, 1::2] = -0.0, float("nan"), 0.0, 0.5
     x[4, : range_len], w[4] = 0.25, 1.0
     xd, wd = x.to(DEV), w.to(DEV)
+    text = capi.fc_forward_ranges_describe(xd, wd, range_len, capi.W_MK)
+    assert "lengthen_rows_kernel" in text, text
+    room = capi.lib().mam_fc_forward_ranges_workspace_at(capi._p(xd), K, capi._p(wd), K, capi.W_MK, N, K, M, range_len, 1)
+    assert room >= int(text.split()[1])
     outs = []
     for tiling in (capi.FORWARD_TILING_WIDE, capi.FORWARD_TILING_AUTO):
         capi.set_option(capi.OPT_FORWARD_TILING, tiling)

@@ -81,6 +81,25 @@ def _planted(N, K, M, seed):
     return x, w
 
 
+def _runs_as(x, w, with_indices, route, range_len=None):
+    """The route that the call is described by, which the workspace that it brings has room for."""
+    from mamtorch_amd import capi
+
+    l = capi.lib()
+    (N, K), M = x.shape, w.shape[0]
+    call = (capi._p(x), capi._ld(x), capi._p(w), capi._ld(w), capi.W_MK, N, K, M)
+    if range_len is None:
+        text = capi.fc_forward_describe(x, w, capi.W_MK, with_indices)
+        room = l.mam_fc_forward_workspace_at(*call, int(with_indices))
+    else:
+        text = capi.fc_forward_ranges_describe(x, w, range_len, capi.W_MK, with_indices)
+        room = l.mam_fc_forward_ranges_workspace_at(*call, range_len, int(with_indices))
+    first = text.split("; with less: ")[0]
+    assert route in first, text
+    if first.startswith("with "):
+        assert room >= int(first.split()[1]), text
+
+
 # operand rows: aligned, 16 bytes apart but begun off them, of odd stride
 @pytest.mark.parametrize("pad,shift", [(0, 0), (4, 1), (3, 2)])
 @pytest.mark.parametrize("N,K,M", [(33, 128, 64), (37, 129, 130), (33, 191, 70), (64, 192, 129), (200, 260, 300), (31, 1300, 42), (40, 2050, 192),
@@ -101,6 +120,8 @@ def test_last_tile_at_the_end_of_the_row(N, K, M, pad, shift):
     want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, bias.numpy())
     for xd, wd in ((padded(x), w.to(DEV)), (padded(x), padded(w)), (x.to(DEV), padded(w))):
         w_sel, x_sel = torch.zeros(2, N, M, device=DEV), torch.zeros(2, N, M, device=DEV)
+        _runs_as(xd, wd, True, "last k tile at the end of K" if K % 16 or pad or shift else "mam_fwd_sx_kernel")
+        _runs_as(xd, wd, False, "last k tile at the end of K" if K % 16 or pad or shift else "mam_fwd_sx_kernel")
         c, amax, amin = capi.fc_forward(xd, wd, capi.W_MK, bias.to(DEV), w_sel=w_sel, x_sel=x_sel)
         values = capi.fc_forward_values(xd, wd, capi.W_MK, bias.to(DEV))
         tag = "N %d K %d M %d" % (N, K, M)
@@ -122,6 +143,11 @@ def test_last_tile_at_the_end_of_each_range(N, K, M, range_len, pad):
     x, w = _planted(N, K, M, N + K)
     xd = torch.full((N, K + pad), float("inf"), device=DEV)[:, :K].copy_(x)
     wd = torch.full((M, K + pad), float("inf"), device=DEV)[:, :K].copy_(w)
+    route = "mam_fwd_sx_kernel" if (K % 16 == 0 and range_len % 64 == 0 and pad == 0) else "last k tile at the end of K"
+    if K - K // range_len * range_len in range(1, 64):
+        route = "lengthen_rows_kernel"      # a last range too short for a tile of its own
+    for with_indices in (True, False):
+        _runs_as(xd, wd, with_indices, route, range_len)
     c, amax, amin = capi.fc_forward_ranges(xd, wd, range_len, capi.W_MK)
     values, _, _ = capi.fc_forward_ranges(xd, wd, range_len, capi.W_MK, with_indices=False)
     total = None
@@ -142,6 +168,8 @@ def test_rows_fetched_ahead(N, K, M):
 
     x, w = _planted(N, K, M, N + K)
     xd, wd = x.to(DEV), w.to(DEV)
+    for with_indices in (True, False):
+        _runs_as(xd, wd, with_indices, "x fetched ahead")
     c, amax, amin = capi.fc_forward(xd, wd, capi.W_MK)
     values = capi.fc_forward_values(xd, wd, capi.W_MK)
     want = oracle.forward(x.numpy(), w.numpy(), oracle.W_MK, None)
