@@ -1570,11 +1570,14 @@ static bool lengthened_rows_pay(int64_t N, int64_t K, int64_t M, bool turn, bool
 // The same for the caller's ranges, each lengthened to whole 64-k tiles ((N, K, M) in four ranges, us on the general tiling / lengthened, with
 // indices: 496 x 691 x 105 67 / 31, 160 x 3200 x 512 152 / 76, 9536 x 2809 x 1432 6784 / 3003, 16 x 260 x 64 40 / 20; in ranges of 32, 2000 x
 // 500 x 2000 1272 / 1161 but 100 x 128 x 100 18.5 / 19.5).  Values only, where padding short ranges to 64 instead of 32 costs less than the better
-// loop gains: 4000 x 531 x 3712 681 / 641, 500 x 200 x 500 23 / 18, 1441 x 2280 x 94 120 / 48; not 8098 x 278 x 71 43 / 47.
-static bool lengthened_ranges_pay(int64_t N, int64_t M, int64_t range_len, bool args)
+// loop gains: 4000 x 531 x 3712 681 / 641, 500 x 200 x 500 23 / 18, 1441 x 2280 x 94 120 / 48; not 8098 x 278 x 71 43 / 47, and of many outputs
+// not three or five whole 32-k tiles of the general tiling, of rows that it reads 16 bytes at a time (`fast`): lengthened by a third or a fifth (6300 x
+// 4 ranges x 1536, of 96 287 / 324, of 160 384 / 411, but of 97 389 / 329, of 161 522 / 417 and of 224 487 / 498; 4000 x 4 x 96 x 200 41 / 44).
+static bool lengthened_ranges_pay(int64_t N, int64_t M, int64_t range_len, bool args, bool fast)
 {
     if (range_len < 32 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
-    return args ? range_len > 32 || N * M > 16384 : range_len >= 96 || N * M <= (1 << 18);
+    if (args) return range_len > 32 || N * M > 16384;
+    return N * M <= (1 << 18) || (range_len >= 3 * KT && !(fast && (range_len == 3 * KT || range_len == 5 * KT)));
 }
 
 // The plan of a call on staged operands, for a call that the wave-uniform-rows tiling does not take as it is; false:
@@ -1587,7 +1590,7 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
     const bool turn = w_layout == MAM_W_KM, ranges = range_len > 0 && range_len < K;
     Ragged tail;
     if (!turn && ragged_staging(st, tail, args, plan.p.vec_w, N, K, M, ranges ? range_len : K) &&
-        (ranges ? lengthened_ranges_pay(N, M, range_len, args) : lengthened_rows_pay(N, K, M, turn, args))) {
+        (ranges ? lengthened_ranges_pay(N, M, range_len, args, plan.p.fast) : lengthened_rows_pay(N, K, M, turn, args))) {
         float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
         const int rc = make_plan(staged, args, x, ldx, st.w ? aligned : w, st.w ? st.w_ld : ldw, MAM_W_MK, bias, c, argmax, argmin, w_sel, x_sel,
                                  N, K, M, range_len, &tail);
@@ -1597,7 +1600,7 @@ static bool staged_plan(Plan &staged, Staging &st, const Plan &plan, bool args, 
     st = staging_of(K % G == 0 && plan.p.vec_x, !turn && plan.p.vec_w, N, K, M, turn ? 0 : range_len);
     if (!st.rows_fit(N, M, turn) || (turn && !transposed_operand_pays(N, K, M))) return false;
     const bool lengthen = st.x || (st.w && !turn);
-    if (ranges ? (turn ? st.x || range_len % sx::KT != 0 : st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args))
+    if (ranges ? (turn ? st.x || range_len % sx::KT != 0 : st.K > INT32_MAX / 2 || !lengthened_ranges_pay(N, M, range_len, args, plan.p.fast))
                : lengthen && !lengthened_rows_pay(N, K, M, turn, args)) return false;
     float *const aligned = reinterpret_cast<float *>((uintptr_t)256);   // stands in for the workspace
     const int rc = make_plan(staged, args, st.x ? aligned : x, st.x ? st.K : ldx, st.w ? aligned : w, st.w ? st.K : ldw, MAM_W_MK, bias,
@@ -1820,7 +1823,7 @@ extern "C" size_t mam_fc_forward_ranges_workspace(int64_t N, int64_t K, int64_t 
     size_t bytes = ranges * (with_indices ? 3 : 2) * (size_t)N * (size_t)M * sizeof(float);
     // room for lengthened ranges (see launch), where they are not whole tiles as they are; without it the call still works
     const bool whole = range_len % mam::fwd::sx::KT == 0 && K % mam::fwd::G == 0;
-    if (!whole && mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0)) {
+    if (!whole && mam::fwd::lengthened_ranges_pay(N, M, range_len, with_indices != 0, false)) {
         mam::fwd::Staging st;
         mam::fwd::Ragged tail;
         if (mam::fwd::ragged_staging(st, tail, with_indices != 0, false, N, K, M, range_len)) bytes += st.bytes();

@@ -200,6 +200,20 @@ def test_whole_ranges_of_a_km_weight_run_on_its_transposed_copy(N, K, M, range_l
     assert l.mam_fc_forward_ranges_workspace_at(x, K, w, M, capi.W_KM, N, K, M, range_len, with_indices) == partials + copy
 
 
+@pytest.mark.parametrize("range_len, lengthened", [(96, False), (160, False), (92, False), (97, True), (100, True), (161, True), (224, True)])
+def test_values_of_whole_32_k_tiles_stay_on_them(range_len, lengthened):
+    # (a weight at 16-byte addresses is copied for values only where its ranges begin off them)
+    l = capi.lib()
+    N, K, M = 6300, 4 * range_len, 1536
+    x, w, off = ctypes.c_void_p(256), ctypes.c_void_p(256), ctypes.c_void_p(260)
+    text = ctypes.create_string_buffer(640)
+    assert l.mam_fc_forward_ranges_describe(x, K, w, K, capi.W_MK, N, K, M, range_len, 0, text, 640) == 0
+    assert (b"mam_fwd_sx_kernel" in text.value) == lengthened, text.value
+    partials = 4 * N * M * 8
+    assert (l.mam_fc_forward_ranges_workspace_at(x, K, w, K, capi.W_MK, N, K, M, range_len, 0) > partials) == (range_len % 4 != 0)
+    assert (l.mam_fc_forward_ranges_workspace_at(x, K, off, K, capi.W_MK, N, K, M, range_len, 0) > partials) == (range_len >= 96)
+
+
 @pytest.mark.parametrize("rows_x", sorted(ROWS))
 @pytest.mark.parametrize("rows_w", sorted(ROWS))
 @pytest.mark.parametrize("with_indices", [0, 1])
