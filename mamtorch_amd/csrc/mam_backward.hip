@@ -90,11 +90,15 @@ __device__ __forceinline__ void bwd_x_body(
             const int m = mb + u * NT_X;
             const bool ok = m < M;
             g[u] = ok ? g_row[m] : 0.0f;
-            a1[u] = ok ? amax_row[m] : -1;
-            if (PICKS) unpack_picks(a1[u], a2[u]);
-            else a2[u] = ok ? amin_row[m] : -1;
-            a1[u] -= k0;
-            a2[u] -= k0;
+            if (PICKS) {
+                a1[u] = ok ? amax_row[m] : -1;
+                unpack_picks(a1[u], a2[u]);
+                a1[u] -= k0;
+                a2[u] -= k0;
+            } else {
+                a1[u] = ok ? amax_row[m] - k0 : -1;
+                a2[u] = ok ? amin_row[m] - k0 : -1;
+            }
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -226,24 +230,29 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
     float4 g = make_float4(0.f, 0.f, 0.f, 0.f), s1 = g, s2 = g;
     int4 i1 = make_int4(-1, -1, -1, -1), i2 = i1;
 // (a macro, not a lambda: captured by reference the five vectors end up in scratch memory)
+// (one branch for all loads of an item, which are then in flight together)
+#define MAM_LOAD_QUADS(pl, o, left)                                                                 \
+    do {                                                                                            \
+        g = row_quad(grad + (o), left);                                                             \
+        i1 = row_quad(argmax + (pl) * nm + (o), left);                                              \
+        if (!PICKS) i2 = row_quad(argmin + (pl) * nm + (o), left);                                  \
+        if (w_sel) {                                                                                \
+            s1 = row_quad(w_sel + (pl) * 2 * nm + (o), left);                                       \
+            s2 = row_quad(w_sel + (pl) * 2 * nm + nm + (o), left);                                  \
+        }                                                                                           \
+    } while (0)
 #define MAM_LOAD_ITEM(pl, m)                                                                        \
     do {                                                                                            \
         if (row_ok && (m) < M) {                                                                    \
             const int64_t o_ = (int64_t)n * M + (m);                                                \
-            const int left_ = quads ? 4 : M - (m);                                                  \
-            g = row_quad(grad + o_, left_);                                                         \
-            i1 = row_quad(argmax + (pl) * nm + o_, left_);                                          \
-            if (!PICKS) {                                                                           \
-                i2 = row_quad(argmin + (pl) * nm + o_, left_);                                      \
-            } else {                                                                                \
+            const int left_ = M - (m);                                                              \
+            if (quads || left_ >= 4) MAM_LOAD_QUADS(pl, o_, 4);                                     \
+            else MAM_LOAD_QUADS(pl, o_, left_);                                                     \
+            if (PICKS) {                                                                            \
                 unpack_picks(i1.x, i2.x);                                                           \
                 unpack_picks(i1.y, i2.y);                                                           \
                 unpack_picks(i1.z, i2.z);                                                           \
                 unpack_picks(i1.w, i2.w);                                                           \
-            }                                                                                       \
-            if (w_sel) {                                                                            \
-                s1 = row_quad(w_sel + (pl) * 2 * nm + o_, left_);                                   \
-                s2 = row_quad(w_sel + (pl) * 2 * nm + nm + o_, left_);                              \
             }                                                                                       \
         } else {                                                                                    \
             i1 = make_int4(-1, -1, -1, -1);                                                         \
@@ -343,6 +352,7 @@ __global__ __launch_bounds__(NT_W) void mam_bwd_x_rows_kernel(
         break;
     }
 #undef MAM_LOAD_ITEM
+#undef MAM_LOAD_QUADS
 }
 
 // One batch row and Q consecutive neurons (2 or 4): the gradient, the two picks and the inputs picked.
