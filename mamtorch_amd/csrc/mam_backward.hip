@@ -906,13 +906,14 @@ static WForm w_form_mk(int64_t N, int64_t K, int64_t M, int64_t shares)
 // 910 / 507.  Quads of 1024 where pairs of them find no work (64 x 784 -> 256 9.0 / 7.4 / 7.9, 64 x 64 -> 64 5.9 / 5.8 / 6.6; 128 x 300 -> 1000 9.2 / 9.9 /
 // 8.7) and where a slab holds less than a third of the picks that it reads (1024 x 4096 -> 1024 45 / 32 / 34, 4000 x 4096 -> 1024 140 / 96 / 106; 2500 x
 // 2500 -> 2500 101 / 101 / 84, 1024 x 3072 -> 1024 46 / 37 / 35).  Quads of 512 where a slab is a few KiB that all lanes add to (3708 x 64 -> 44 123 / 173 /
-// 164, 1000 x 96 -> 1000 38 / 49 / 45, 462 x 105 -> 107 19.4 / 23 / 21.5; 1000 x 200 -> 500 35.8 / 39.6 / 36.0) and where gradient and picks are more than
-// the memory-side cache holds (12608 x 768 -> 3072 644 / 792 / 806, 6300 x 1024 -> 4096 354 / 411 / 406; 12608 x 384 -> 1536 as above).
+// 164, 1000 x 96 -> 1000 38 / 49 / 45, 462 x 105 -> 107 19.4 / 23 / 21.5; 1000 x 200 -> 500 35.8 / 39.6 / 36.0) and, where gradient and picks are more than
+// the memory-side cache holds, where one is too long for two on a CU (12608 x 768 -> 3072 644 / 792 / 806, 12608 x 512 -> 2048 566 / 712 / 647; 22000 x
+// 320 -> 1024 870 / 1098 / 737, 12608 x 96 -> 3072 560 / 488 / 404; below that size 12608 x 384 -> 1536 as above).
 static WForm w_form_km(int64_t N, int64_t K, int64_t M, int planes)
 {
     constexpr int64_t kMemorySideCache = (int64_t)256 << 20;
     if (N < 128 || K > 3072) return QUADS_1024;
-    return K < 128 || N * M * (4 + 8 * planes) > kMemorySideCache ? QUADS : PAIRS;
+    return (N * M * (4 + 8 * planes) > kMemorySideCache ? K > 384 : K < 128) ? QUADS : PAIRS;
 }
 
 template <int LAYOUT, int NT, int Q>
@@ -1180,7 +1181,9 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
         // the batch at one pace, a row fetched once for all; beside x_grad they fall out of step and fetch it again (in a captured graph, us side by
         // side / one after the other: 9792 x 1728 -> 803 371 / 278, 2500 x 1000 -> 1001 102 / 85, 12608 x 3072 -> 768 683 / 490, in four ranges 4000 x
         // 1400 -> 704 432 / 240, 9000 x 600 -> 300 235 / 146, 4000 x 1024 -> 1500 470 / 477; but 2100 x 400 -> 2000 in four ranges 179 / 221).
-        const bool in_step = w_layout == MAM_W_MK && !x_sel && N * M >= (1 << 21) && K >= 512;
+        // (K,M) likewise where both kernels take two workgroups a CU (2200 x 384 -> 1536 123 / 105, 4000 x 384 -> 1536 193 / 154, 4000 x 211 -> 2560 180 /
+        // 162; 2200 x 768 -> 768 133 / 131, 9000 x 384 -> 1536 328 / 362, 1000 x 384 -> 1536 46 / 55).
+        const bool in_step = w_layout == MAM_W_MK ? !x_sel && N * M >= (1 << 21) && K >= 512 : N >= 2048 && N < 8192 && K <= 512;
         ForkedStream fork(st, N * M, !in_step && N * M >= (1 << 23) && M >= 1024, !in_step);
         if (fork.forked()) {
             const int rc_x = launch(x_grad, nullptr, fork.side());
