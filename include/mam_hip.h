@@ -73,8 +73,8 @@ extern "C" {
 #define MAM_BACKWARD_FORK_ON 1
 #define MAM_BACKWARD_ONE_LAUNCH_OFF 0
 #define MAM_BACKWARD_ONE_LAUNCH_AUTO 1 /* small calls only (<= 2^16 outputs), where the launches are the cost */
-#define MAM_BACKWARD_ONE_LAUNCH_ON 2   /* wherever the shape allows it: (M,K) weights, 16-byte aligned operands,
-                                          batch below 2 x CUs, K <= 4096 */
+#define MAM_BACKWARD_ONE_LAUNCH_ON 2   /* wherever the shape allows it: (M,K) weights, batch below 2 x CUs,
+                                          K <= 4096 */
 #define MAM_BACKWARD_EXACT_OFF 0 /* w_grad in fp32 cells: each sum within the rounding floor of its order    */
 #define MAM_BACKWARD_EXACT_ON 1  /* w_grad = the exact sum of its fp32 terms rounded once (the w_grad kernel
                                     takes 45 instead of 17 us at 256 x 4096 x 4096, 1.7 to 1.8 times as long at
@@ -140,7 +140,8 @@ int mam_fc_forward(const float *x, int64_t ldx, const float *w, int64_t ldw, int
 /*
  * mam_fc_forward for callers that hand the indices to a backward and to nobody else: picks (N, M) int32 contiguous = argmax in the low
  * half of a word, argmin in the high half (K at most 65535).  A plane less to write here and to read in either kernel of the
- * backward (training step of 12608 rows through 768 -> 3072 -> 768: 1579 -> 1493 us).  Same outputs, workspace and errors otherwise.  No counterpart in the reference.
+ * backward (training step of 12608 rows through 768 -> 3072 -> 768: 1579 -> 1493 us).  Same outputs, workspace and errors otherwise.  No
+ * counterpart in the reference.
  */
 int mam_fc_forward_picks(const float *x, int64_t ldx, const float *w, int64_t ldw, int w_layout, const float *bias, float *c,
                          int32_t *picks, float *w_sel, float *x_sel, int64_t N, int64_t K, int64_t M, void *workspace,

@@ -6,7 +6,7 @@
 // the work is bandwidth: write every output byte exactly once and read the (grad, argmax, argmin)
 // triples as few times as possible.  Each workgroup OWNS a slab of an output, accumulates the
 // scattered terms for that slab in LDS, and then streams the slab to HBM with coalesced stores --
-// no zero-fill pass and no global atomics:
+// no zero-fill pass and no global atomics but where the batch is shared (below):
 //
 //   x_grad : one workgroup per batch row n; cells over k (chunked when they exceed LDS).  From 2048
 //            batch rows on: 2 to 16 rows per workgroup, the lanes of a wave spread over them.  The cells
@@ -14,8 +14,9 @@
 //   w_grad : one workgroup per R consecutive output neurons x KC consecutive k, fp32 cells.  For the (M,K)
 //            layout R = 4 so a slab is 4 whole rows of the weight gradient (64 KiB: two
 //            workgroups per CU); for the (K,M) layout R = 32 so that every stored row segment is
-//            128 bytes.  From 2048 batch rows on, (M,K): up to 16 neurons per slab and the batch shared
-//            by several workgroups per slab, which add their shares to the cleared w_grad.
+//            128 bytes.  (M,K): from 2048 batch rows on up to 16 neurons per slab, and from 1536 terms a
+//            neuron (rows times the caller's ranges) on the batch is shared by several workgroups per slab,
+//            which add their shares to the cleared w_grad, where that fills the chip better (shares_of).
 //
 // Each term is one fp32 product (operand of the reference's atomicAdd).  x_grad is the exact sum of its
 // terms rounded once -- as long as at most QCAP (512) terms of a workgroup's slab fall outside its
@@ -863,7 +864,9 @@ struct BiasGrad {
 //   alone: 5408 x 288 -> 40 17.8 (10 shares) / 9.5, 4704 x 234 -> 36 18.0 / 9.7, 8192 x 4096 -> 64 36 / 20.8, 3152 x 1536 -> 384 24 / 20.6, 496 x 691
 //   in four ranges -> 105 21.6 / 9.7; but 1900 x 2048 -> 200 13.2 / 14.2, 1000 x 1024 -> 256 10.9 / 11.5.
 //   Many rows: two rounds of as many workgroups as fit the chip, as long as a share has K rows, and 768 (12608 x 768 -> 3072 with 1 / 3 / 8 / 16
-//   shares 257 / 220 / 211 / 230; 3152 x 384 -> 1536 with 4 / 6 35 / 46).
+//   shares 257 / 220 / 211 / 230; 3152 x 384 -> 1536 with 4 / 6 35 / 46).  Over 98 shapes of 2048 to 20000 rows, 100 to 1024 inputs, 192 to 3072
+//   neurons 512 rows take 1.2 % longer and 1024 0.3 %; single ones gain or lose a third by their rounds of workgroups (512 / 768 / 1024: 5000 x 192
+//   -> 768 30 / 40 / 33, 8000 x 384 -> 768 51 / 39 / 48).
 constexpr int64_t FEW_ROWS = 1536, SHARE_ROWS = 64, MANY_ROWS = 768;
 static int64_t shares_of_many_rows(int64_t N, int64_t K) { return N < 2048 ? 1 : N / (K > MANY_ROWS ? K : MANY_ROWS); }
 static int64_t shares_of(int64_t N, int64_t K, int planes, int64_t slabs, int64_t per_cu, int64_t cus)
@@ -892,23 +895,24 @@ static int64_t most_shares(int64_t N, int64_t K, int64_t M)
 // Neurons of an item of w_grad and threads of a workgroup.
 enum WForm { QUADS, PAIRS, QUADS_1024 };
 
-// (M,K), 512 threads: pairs where the items of a slab are few, so that more lanes share them and more waves fit (65 registers instead of 91): us with
-// quads / pairs, kernel alone: 496 x 691 in four ranges -> 105 9.6 / 9.0, 910 x 192 -> 768 10.4 / 9.5, 472 x 1050 in four ranges -> 2145 71 / 62,
-// 1238 x 662 -> 3590 38.4 / 35.0; not for long slabs, which their stores bound (256 x 4096 -> 4096 16.4 / 18.2).  From 2048 rows on where
+// (M,K), 512 threads: pairs where the items of a slab are few, so that more lanes share them and more waves fit (65 registers instead of 91): us
+// with quads / pairs, kernel alone: 496 x 691 in four ranges -> 105 9.6 / 9.0, 910 x 192 -> 768 10.4 / 9.5, 472 x 1050 in four ranges -> 2145 71
+// / 62, 1238 x 662 -> 3590 38.4 / 35.0; not for long slabs, which their stores bound (256 x 4096 -> 4096 16.4 / 18.2).  From 2048 rows on where
 // quads straddle lines and no shares are there (2178 x 1494 -> 1982 39 / 28, -> 1983 47 / 37, -> 1984 25.5 / 27).
 static WForm w_form_mk(int64_t N, int64_t K, int64_t M, int64_t shares)
 {
     return (N < 2048 ? K <= 2048 || M % 4 != 0 : shares == 1 && M % 4 != 0) ? PAIRS : QUADS;
 }
 
-// (K,M), a workgroup per CU (its 128 KiB slab): us with quads of 512 threads / quads of 1024 / pairs of 1024, kernel alone: 256 x 1024 -> 1024 17.6 /
-// 15.6 / 13.4, 512 x 768 -> 3072 30.5 / 31.0 / 26.8, 2048 x 1024 -> 256 130 / 140 / 114, 12608 x 384 -> 1536 464 / 551 / 395, 19136 x 368 -> 256 831 /
-// 910 / 507.  Quads of 1024 where pairs of them find no work (64 x 784 -> 256 9.0 / 7.4 / 7.9, 64 x 64 -> 64 5.9 / 5.8 / 6.6; 128 x 300 -> 1000 9.2 / 9.9 /
-// 8.7) and where a slab holds less than a third of the picks that it reads (1024 x 4096 -> 1024 45 / 32 / 34, 4000 x 4096 -> 1024 140 / 96 / 106; 2500 x
-// 2500 -> 2500 101 / 101 / 84, 1024 x 3072 -> 1024 46 / 37 / 35).  Quads of 512 where a slab is a few KiB that all lanes add to (3708 x 64 -> 44 123 / 173 /
-// 164, 1000 x 96 -> 1000 38 / 49 / 45, 462 x 105 -> 107 19.4 / 23 / 21.5; 1000 x 200 -> 500 35.8 / 39.6 / 36.0) and, where gradient and picks are more than
-// the memory-side cache holds, where one is too long for two on a CU (12608 x 768 -> 3072 644 / 792 / 806, 12608 x 512 -> 2048 566 / 712 / 647; 22000 x
-// 320 -> 1024 870 / 1098 / 737, 12608 x 96 -> 3072 560 / 488 / 404; below that size 12608 x 384 -> 1536 as above).
+// (K,M), a workgroup per CU (its 128 KiB slab): us with quads of 512 threads / quads of 1024 / pairs of 1024, kernel alone: 256 x 1024 -> 1024
+// 17.6 / 15.6 / 13.4, 512 x 768 -> 3072 30.5 / 31.0 / 26.8, 2048 x 1024 -> 256 130 / 140 / 114, 12608 x 384 -> 1536 464 / 551 / 395, 19136 x 368
+// -> 256 831 / 910 / 507.  Quads of 1024 where pairs of them find no work (64 x 784 -> 256 9.0 / 7.4 / 7.9, 64 x 64 -> 64 5.9 / 5.8 / 6.6; 128 x
+// 300 -> 1000 9.2 / 9.9 / 8.7) and where a slab holds less than a third of the picks that it reads (1024 x 4096 -> 1024 45 / 32 / 34, 4000 x
+// 4096 -> 1024 140 / 96 / 106; 2500 x 2500 -> 2500 101 / 101 / 84, 1024 x 3072 -> 1024 46 / 37 / 35).  Quads of 512 where a slab is a few KiB
+// that all lanes add to (3708 x 64 -> 44 123 / 173 / 164, 1000 x 96 -> 1000 38 / 49 / 45, 462 x 105 -> 107 19.4 / 23 / 21.5; 1000 x 200 -> 500
+// 35.8 / 39.6 / 36.0) and, where gradient and picks are more than the memory-side cache holds, where one is too long for two on a CU (12608 x
+// 768 -> 3072 644 / 792 / 806, 12608 x 512 -> 2048 566 / 712 / 647; 22000 x 320 -> 1024 870 / 1098 / 737, 12608 x 96 -> 3072 560 / 488 / 404;
+// below that size 12608 x 384 -> 1536 as above).
 static WForm w_form_km(int64_t N, int64_t K, int64_t M, int planes)
 {
     constexpr int64_t kMemorySideCache = (int64_t)256 << 20;
@@ -945,8 +949,8 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
         int log2r = 1;
         while (log2r < 4 && ((int64_t)2 << log2r) * K * 8 <= rows_budget) ++log2r;
         const int R = 1 << log2r;
-        hipLaunchKernelGGL((argmin ? mam_bwd_x_rows_kernel<LAYOUT, false> : mam_bwd_x_rows_kernel<LAYOUT, true>), dim3((unsigned)ceil_div(N, R)), dim3(NT_W),
-                           (size_t)R * K * 8, st, w, ldw, grad, argmax, argmin, w_sel, N * M, x_grad,
+        hipLaunchKernelGGL((argmin ? mam_bwd_x_rows_kernel<LAYOUT, false> : mam_bwd_x_rows_kernel<LAYOUT, true>),
+                           dim3((unsigned)ceil_div(N, R)), dim3(NT_W), (size_t)R * K * 8, st, w, ldw, grad, argmax, argmin, w_sel, N * M, x_grad,
                            (int)N, (int)K, (int)M, log2r, planes, span);
         rc = check_launch("mam_bwd_x_rows_kernel");
         if (rc != MAM_OK) return rc;
@@ -1030,8 +1034,9 @@ static int launch_layout(const float *x, int64_t ldx, const float *w, int64_t ld
     return rc;
 }
 
-// Both gradients in one launch (mam_bwd_both_kernel) where the shape allows it: (M,K) weights, a batch small enough that the x_grad workgroups (one per batch row) are all resident
-// at once, K in one chunk of either kernel -- and, unless the option forces it, at most 2^16 outputs.
+// Both gradients in one launch (mam_bwd_both_kernel) where the shape allows it: (M,K) weights, a batch small enough that the x_grad
+// workgroups (one per batch row) are all resident at once, K in one chunk of either kernel -- and, unless the option forces it, at most 2^16
+// outputs and a w_grad that takes the batch in one piece.
 // Returns MAM_OK after launching, 1 when the shape is not served.
 static int launch_both(const float *x, int64_t ldx, const float *w, int64_t ldw, const float *grad,
                        const int32_t *argmax, const int32_t *argmin, const float *w_sel, const float *x_sel,
@@ -1177,12 +1182,13 @@ static int backward_impl(const float *x, int64_t ldx, const float *w, int64_t ld
         // 8192 x 2048 -> 1024 113 / 121, 16384 x 4096 -> 1024 272 / 282; but 4096 x 1024 -> 1024 62 / 56, and with
         // 768 neurons (the rows kernel's workgroups are short and mostly waiting, and hold the LDS the w_grad
         // workgroups need) 12608 x 3072 -> 768 180 / 165, 25216 rows 335 / 316, 8192 rows 116 / 113.
-        // Not at all without the inputs handed over, from 2^21 outputs and 512 inputs on, (M,K): w_grad's workgroups then gather x, all of them along
-        // the batch at one pace, a row fetched once for all; beside x_grad they fall out of step and fetch it again (in a captured graph, us side by
-        // side / one after the other: 9792 x 1728 -> 803 371 / 278, 2500 x 1000 -> 1001 102 / 85, 12608 x 3072 -> 768 683 / 490, in four ranges 4000 x
-        // 1400 -> 704 432 / 240, 9000 x 600 -> 300 235 / 146, 4000 x 1024 -> 1500 470 / 477; but 2100 x 400 -> 2000 in four ranges 179 / 221).
-        // (K,M) likewise where both kernels take two workgroups a CU (2200 x 384 -> 1536 123 / 105, 4000 x 384 -> 1536 193 / 154, 4000 x 211 -> 2560 180 /
-        // 162; 2200 x 768 -> 768 133 / 131, 9000 x 384 -> 1536 328 / 362, 1000 x 384 -> 1536 46 / 55).
+        // Not at all without the inputs handed over, from 2^21 outputs and 512 inputs on, (M,K): w_grad's workgroups then gather x, all of
+        // them along the batch at one pace, a row fetched once for all; beside x_grad they fall out of step and fetch it again (in a
+        // captured graph, us side by side / one after the other: 9792 x 1728 -> 803 371 / 278, 2500 x 1000 -> 1001 102 / 85, 12608 x 3072
+        // -> 768 683 / 490, in four ranges 4000 x 1400 -> 704 432 / 240, 9000 x 600 -> 300 235 / 146, 4000 x 1024 -> 1500 470 / 477; but
+        // 2100 x 400 -> 2000 in four ranges 179 / 221). (K,M) likewise where both kernels take two workgroups a CU (2200 x 384 -> 1536 123
+        // / 105, 4000 x 384 -> 1536 193 / 154, 4000 x 211 -> 2560 180 / 162; 2200 x 768 -> 768 133 / 131, 9000 x 384 -> 1536 328 / 362,
+        // 1000 x 384 -> 1536 46 / 55).
         const bool in_step = w_layout == MAM_W_MK ? !x_sel && N * M >= (1 << 21) && K >= 512 : N >= 2048 && N < 8192 && K <= 512;
         ForkedStream fork(st, N * M, !in_step && N * M >= (1 << 23) && M >= 1024, !in_step);
         if (fork.forked()) {

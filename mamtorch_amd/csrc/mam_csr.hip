@@ -24,7 +24,8 @@
 // hits, at about half of the path's 64 bytes per clock and CU) with the arithmetic hidden under it.
 // The lowest column missing from the row is found once per row; the
 // implicit-zero candidate x[n, missing] * 0 is compared last under the dense rule (greater wins,
-// equal -> lower index wins).  TI follows the number of workgroups (below, at the launch).  The 16 waves of a workgroup own 16 consecutive neurons and hand
+// equal -> lower index wins).  TI follows the number of workgroups (below, at the launch).  The 16 waves of a workgroup own 16
+// consecutive neurons and hand
 // their results over through LDS so that every batch row stores 64 contiguous bytes per array.
 //
 // Backward: when the forward handed over the selected values and their entry positions, x_grad is the
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(NT_F) void csr_fwd_kernel(
 {
     typedef typename XVec<TI>::type xvec;
     constexpr int TILE_N = 64 * TI;
-    // results of the workgroup's 16 neurons, [array][neuron][batch row]: 7 x 16 KiB for TI = 4
+    // results of the workgroup's 16 neurons, [array][neuron][batch row]: 9 x 16 KiB for TI = 4
     extern __shared__ float out_lds[];
     float (*out_c)[TILE_N] = reinterpret_cast<float (*)[TILE_N]>(out_lds);
     int (*out_hi)[TILE_N] = reinterpret_cast<int (*)[TILE_N]>(out_lds + 1 * ROWS * TILE_N);
@@ -533,7 +534,7 @@ __global__ __launch_bounds__(NT_V) void csr_bwd_val_kernel(
     int p1[4], p2[4];
 #define MAM_VAL_LOAD(it, c0, len)                                                                    \
     do {                                                                                             \
-        const int n_ = (int)((it) / QPR), r0_ = (int)((it) % QPR) * 4;                                           \
+        const int n_ = (int)((it) / QPR), r0_ = (int)((it) % QPR) * 4;                               \
         const bool ok_ = (it) < items && r0_ < rows;                                                 \
         u1 = u2 = make_int4(-1, -1, -1, -1);                                                         \
         k1 = k2 = make_int4(0, 0, 0, 0);                                                             \

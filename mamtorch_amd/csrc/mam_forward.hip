@@ -843,7 +843,8 @@ __global__ __launch_bounds__(256) void mam_fwd_range_sum_kernel(const Params p)
             const float *base = p.part + (int64_t)s * 3 * nm;
             const int kb = s * p.k_per_split, pk = __float_as_int(base[2 * nm + o]);
             const int length = p.K - kb < p.k_per_split ? p.K - kb : p.k_per_split;
-            const char *const xrange = xrow + (int64_t)kb * (int64_t)sizeof(float), *const wrange = wrows + (int64_t)s * p.w_step * (int64_t)sizeof(float);
+            const char *const xrange = xrow + (int64_t)kb * (int64_t)sizeof(float);
+            const char *const wrange = wrows + (int64_t)s * p.w_step * (int64_t)sizeof(float);
             vals_s[wave][0][lane] = base[o];
             vals_s[wave][1][lane] = base[nm + o];
             grps_s[wave][0][lane] = (pk & 0xffff) * G;
@@ -1121,7 +1122,8 @@ __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
 
     const char *const wrow = reinterpret_cast<const char *>(p.w + (int64_t)col0 * p.ldw);
     const char *wk = wrow + (RAGGED && p.own_ranges ? (int64_t)split * p.w_step : kb) * (int64_t)sizeof(float);
-    if (RAGGED && !ARGS) wk_last = wrow + (p.w_tail < 0 ? ke - sx::KT : (p.own_ranges ? (int64_t)split * p.w_step : 0) + p.w_tail) * (int64_t)sizeof(float);
+    if (RAGGED && !ARGS)
+        wk_last = wrow + (p.w_tail < 0 ? ke - sx::KT : (p.own_ranges ? (int64_t)split * p.w_step : 0) + p.w_tail) * (int64_t)sizeof(float);
     // The wave's x of a tile: 64 lanes reach every line of four rows of 256 bytes
     const float *const xlane = p.x + (int64_t)(row0 + (lane >> 4) < p.N ? row0 + (lane >> 4) : p.N - 1) * p.ldx + kb;
     auto touch = [&](int t) {
@@ -1429,12 +1431,14 @@ static int make_plan(Plan &plan, bool args, const float *x, int64_t ldx, const f
     p.N = (int)N; p.K = (int)K; p.M = (int)M;
     p.vec_x = (ldx % 4 == 0) && ((uintptr_t)x % 16 == 0);
     p.vec_w = (ldw % 4 == 0) && ((uintptr_t)w % 16 == 0);
-    // The wave-uniform-rows tiling takes (M,K) weights with aligned rows and K a multiple of 16; option
+    // The wave-uniform-rows tiling takes aligned (M,K) weights, with aligned rows of x and K a multiple of 16, or with rows of x as
+    // they are and a last tile that ends where the row ends (`ragged`, see walked and ragged_staging); option
     // MAM_OPT_FORWARD_TILING = MAM_FORWARD_TILING_WIDE keeps every shape on the first tiling (for
     // comparisons and tests).
     // (range_len > 0: the caller fixes the K ranges -- the module's `splits` -- instead of the launch
-    // heuristics; the wave-uniform-rows tiling then also needs whole 64-k tiles per range)
-    const bool use_sx = (w_layout == MAM_W_MK) && p.vec_w && (ragged || (p.vec_x && K % G == 0 && range_len % sx::KT == 0)) && (ldw * sx::BM_MAX < (1ll << 30)) &&
+    // heuristics; they are whole 64-k tiles, or each of them ends with a tile of its own)
+    const bool use_sx = (w_layout == MAM_W_MK) && p.vec_w && (ragged || (p.vec_x && K % G == 0 && range_len % sx::KT == 0)) &&
+                        (ldw * sx::BM_MAX < (1ll << 30)) &&
                         option(MAM_OPT_FORWARD_TILING) != MAM_FORWARD_TILING_WIDE;
     plan.use_sx = use_sx;
     // what the tiles walk
@@ -1516,14 +1520,16 @@ static Staging staging_of(bool x_fits, bool w_fits, int64_t N, int64_t K, int64_
     return s;
 }
 
-// Rows of x as they are (see walked): ranges of at least 64, (M, K) weights.  With indices those weights are copied as they are
-// walked; values only where a range's tiles do not begin at 16-byte addresses, every range up to a multiple of 4, then its last 64
-// once more.  K below 128 stays with the lengthened copies: two tiles of which one is mostly repeated cost as much, and
-// the operands are small.  With indices so do calls of many neurons, whose resolve touches two lines of x where a copy's groups
-// have one, half as often in spans of 32 ((N, K, M), x copied / as it is, us: 10233 x 3316 -> 78 in training 429 / 409, 4000 x 4095 -> 250
-// 247 / 238, but 1000 x 4095 -> 500 122 / 125, 500 x 4095 -> 2000 223 / 232; in spans of 16, 43120 x 1300 -> 42 in training 718 / 598,
-// 8000 x 1001 -> 500 253 / 250, 9536 x 2809 -> 1432 in four ranges, training 5951 / 5858, but 3000 x 150 -> 1500 104 / 106; values only,
-// 16000 x 300 -> 200 72 / 59, 30 x 260 -> 4000 21 / 13, 1 x 4092 -> 16000 194 / 104, 4000 x 531 -> 3712 183 / 181).
+// Rows of x as they are (see walked): ranges of at least 64, (M, K) weights.  With indices those weights are copied as they are walked; values
+// only where a range's tiles do not begin at 16-byte addresses, every range up to a multiple of 4, then its last 64 once more.  K below 128
+// stays with the lengthened copies: two tiles of which one is mostly repeated cost as much, and the operands are small.  With indices so do
+// calls of many neurons, whose resolve touches two lines of x where a copy's groups have one, half as often in spans of 32 ((N, K, M), x copied
+// / as it is, us: 10233 x 3316 -> 78 in training 429 / 409, 4000 x 4095 -> 250 247 / 238, but 1000 x 4095 -> 500 122 / 125, 500 x 4095 -> 2000
+// 223 / 232; in spans of 16, 43120 x 1300 -> 42 in training 718 / 598, 8000 x 1001 -> 500 253 / 250, 9536 x 2809 -> 1432 in four ranges,
+// training 5951 / 5858, but 3000 x 150 -> 1500 104 / 106; over 250 to 12000 rows of 300 to 4095 inputs the copy takes 7 to 20 % longer at 100
+// neurons, 2 to 15 % at 320, and of 1000 rows and more either way is within 4 % from 500 on in spans of 32, from 1024 on in spans of 16, from
+// 1500 on in ranges; values only, 16000 x 300 -> 200 72 / 59, 30 x 260 -> 4000 21 / 13, 1 x 4092 -> 16000 194 / 104, 4000 x 531 -> 3712 183 /
+// 181).
 static bool ragged_staging(Staging &s, Ragged &tail, bool args, bool w_aligned, int64_t N, int64_t K, int64_t M, int64_t range_len)
 {
     const int64_t ranges = ceil_div(K, range_len);
@@ -1569,10 +1575,11 @@ static bool lengthened_rows_pay(int64_t N, int64_t K, int64_t M, bool turn, bool
 
 // The same for the caller's ranges, each lengthened to whole 64-k tiles ((N, K, M) in four ranges, us on the general tiling / lengthened, with
 // indices: 496 x 691 x 105 67 / 31, 160 x 3200 x 512 152 / 76, 9536 x 2809 x 1432 6784 / 3003, 16 x 260 x 64 40 / 20; in ranges of 32, 2000 x
-// 500 x 2000 1272 / 1161 but 100 x 128 x 100 18.5 / 19.5).  Values only, where padding short ranges to 64 instead of 32 costs less than the better
-// loop gains: 4000 x 531 x 3712 681 / 641, 500 x 200 x 500 23 / 18, 1441 x 2280 x 94 120 / 48; not 8098 x 278 x 71 43 / 47, and of many outputs
-// not three or five whole 32-k tiles of the general tiling, of rows that it reads 16 bytes at a time (`fast`): lengthened by a third or a fifth (6300 x
-// 4 ranges x 1536, of 96 287 / 324, of 160 384 / 411, but of 97 389 / 329, of 161 522 / 417 and of 224 487 / 498; 4000 x 4 x 96 x 200 41 / 44).
+// 500 x 2000 1272 / 1161 but 100 x 128 x 100 18.5 / 19.5).  Values only, where padding short ranges to 64 instead of 32 costs less than the
+// better loop gains: 4000 x 531 x 3712 681 / 641, 500 x 200 x 500 23 / 18, 1441 x 2280 x 94 120 / 48; not 8098 x 278 x 71 43 / 47, and of many
+// outputs not three or five whole 32-k tiles of the general tiling, of rows that it reads 16 bytes at a time (`fast`): lengthened by a third or
+// a fifth (6300 x 4 ranges x 1536, of 96 287 / 324, of 160 384 / 411, but of 97 389 / 329, of 161 522 / 417 and of 224 487 / 498; 4000 x 4 x 96
+// x 200 41 / 44).
 static bool lengthened_ranges_pay(int64_t N, int64_t M, int64_t range_len, bool args, bool fast)
 {
     if (range_len < 32 || option(MAM_OPT_FORWARD_TILING) == MAM_FORWARD_TILING_WIDE) return false;
