@@ -63,7 +63,6 @@ struct Params {
     float *c;
     int32_t *argmax;
     int32_t *argmin;  // packed: argmax
-    int32_t packed;   // all bits set: argmax holds both, packed (pack_picks); else 0
     float *wsel;      // optional [2][N*M]: the selected weights w[argmax], w[argmin] (for the backward)
     float *xsel;      // optional [2][N*M]: the selected inputs x[argmax], x[argmin] (for the backward)
     float *part;      // split-K partials: [split][3 or 2][N*M]: max, min, (group ids packed 16:16)
@@ -82,6 +81,8 @@ struct Params {
     int own_ranges;    // the K ranges are the caller's
     int w_step;        // columns of w from one of them to the next (k_per_split, more in a copy)
     int w_tail;        // values only, w copied: column at which the last 64 of the (first) range stand once more, aligned; else -1
+    int packed;        // all bits set: argmax holds both picks, packed (pack_picks); else 0.  (Last: before the pointers it moves what the kernels
+                       // fetch first, and a call of 74 us in four launches takes 0.8 us longer.)
 };
 
 // An extreme that still holds its initial value (-inf for the max, +inf for the min) was never strictly
