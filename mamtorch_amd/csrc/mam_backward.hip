@@ -904,20 +904,22 @@ static WForm w_form_mk(int64_t N, int64_t K, int64_t M, int64_t shares)
     return (N < 2048 ? K <= 2048 || M % 4 != 0 : shares == 1 && M % 4 != 0) ? PAIRS : QUADS;
 }
 
-// (K,M), a workgroup per CU (its 128 KiB slab): us with quads of 512 threads / quads of 1024 / pairs of 1024, kernel alone: 256 x 1024 -> 1024
-// 17.6 / 15.6 / 13.4, 512 x 768 -> 3072 30.5 / 31.0 / 26.8, 2048 x 1024 -> 256 130 / 140 / 114, 12608 x 384 -> 1536 464 / 551 / 395, 19136 x 368
-// -> 256 831 / 910 / 507.  Quads of 1024 where pairs of them find no work (64 x 784 -> 256 9.0 / 7.4 / 7.9, 64 x 64 -> 64 5.9 / 5.8 / 6.6; 128 x
-// 300 -> 1000 9.2 / 9.9 / 8.7) and where a slab holds less than a third of the picks that it reads (1024 x 4096 -> 1024 45 / 32 / 34, 4000 x
-// 4096 -> 1024 140 / 96 / 106; 2500 x 2500 -> 2500 101 / 101 / 84, 1024 x 3072 -> 1024 46 / 37 / 35).  Quads of 512 where a slab is a few KiB
-// that all lanes add to (3708 x 64 -> 44 123 / 173 / 164, 1000 x 96 -> 1000 38 / 49 / 45, 462 x 105 -> 107 19.4 / 23 / 21.5; 1000 x 200 -> 500
-// 35.8 / 39.6 / 36.0) and, where gradient and picks are more than the memory-side cache holds, where one is too long for two on a CU (12608 x
-// 768 -> 3072 644 / 792 / 806, 12608 x 512 -> 2048 566 / 712 / 647; 22000 x 320 -> 1024 870 / 1098 / 737, 12608 x 96 -> 3072 560 / 488 / 404;
-// below that size 12608 x 384 -> 1536 as above).
+// (K,M), a workgroup per CU (its 128 KiB slab).  Over 5100 calls (64 to 4096 inputs, 32 to 4096 neurons, 128 to 16384 rows, normal, rectified
+// and uniform inputs); us with quads of 512 threads / quads of 1024 / pairs of 1024, kernel alone.  Pairs: 256 x 1024 -> 1024 17.6 / 15.6 /
+// 13.4, 512 x 768 -> 3072 30.5 / 31.0 / 26.8, 2048 x 1024 -> 256 130 / 140 / 114, 12608 x 384 -> 1536 464 / 551 / 395, 940 x 1345 -> 354 46 / 47
+// / 32; on average 9 % less than quads of 1024 below 1024 rows and 25 % above.  Quads of 1024 where pairs of them find no work (64 x 784
+// -> 256 9.0 / 7.4 / 7.9, 64 x 64 -> 64 5.9 / 5.8 / 6.6; 128 x 300 -> 1000 9.2 / 9.9 / 8.7) and where a slab holds less than half of the picks
+// that it reads: from 2048 to 3072 inputs pairs take between 8 % less and 17 % more (600 x 2400 -> 1000 21.7 / 21.2, but 858 x 2176 -> 2802 40.0
+// / 46.8, 576 x 2944 -> 256 15.3 / 17.8), beyond that more (1024 x 4096 -> 1024 32 / 34, 4000 x 4096 -> 1024 96 / 106).  Quads of 512 only where
+// gradient and picks are more than the memory-side cache holds and a slab is too long for two on a CU (12608 x 768 -> 3072 644 / 792 / 806,
+// 12608 x 512 -> 2048 566 / 712 / 647; 22000 x 320 -> 1024 870 / 1098 / 737, 12608 x 96 -> 3072 560 / 488 / 404).  Below 128 inputs they take 20 %
+// less than pairs for uniform inputs (3708 x 64 -> 44 156 / 172) and 5 to 40 % more for normal and rectified ones (1000 x 100 -> 1000 39 / 28).
 static WForm w_form_km(int64_t N, int64_t K, int64_t M, int planes)
 {
     constexpr int64_t kMemorySideCache = (int64_t)256 << 20;
     if (N < 128 || K > 3072) return QUADS_1024;
-    return (N * M * (4 + 8 * planes) > kMemorySideCache ? K > 384 : K < 128) ? QUADS : PAIRS;
+    if (N * M * (4 + 8 * planes) > kMemorySideCache) return K > 384 ? QUADS : PAIRS;
+    return K > 2048 ? QUADS_1024 : PAIRS;
 }
 
 template <int LAYOUT, int NT, int Q>

@@ -583,7 +583,7 @@ def test_indices_that_do_not_fit_a_word_are_refused():
         capi.fc_backward_picks(x, w, g, torch.zeros(2, 3, dtype=torch.int32, device=dev), capi.W_MK)
 
 
-@pytest.mark.parametrize("shape", [(127, 300, 70), (128, 127, 65), (128, 128, 65), (130, 129, 31), (128, 3072, 34), (128, 3073, 34), (1030, 128, 33),
+@pytest.mark.parametrize("shape", [(127, 300, 70), (128, 127, 65), (128, 128, 65), (130, 129, 31), (128, 2048, 34), (128, 2049, 34), (128, 3073, 34), (1030, 128, 33),
                                    (2051, 96, 7), (300, 1025, 97)])
 def test_every_form_of_a_km_weight_gradient(shape):
     """Quads and pairs of neurons, workgroups of 512 and of 1024 threads: either side of each line between them, slabs of K and of M that end
