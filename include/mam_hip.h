@@ -67,8 +67,9 @@ extern "C" {
                                       does not suit them, and K too large for the LDS)                   */
 #define MAM_FORWARD_TILING_DENSE 5 /* as AUTO, but never by lists                                         */
 #define MAM_BACKWARD_FORK_AUTO (-1) /* where it pays: from 2^23 outputs on with at least 1024 neurons (dense),
-                                       2^22 outputs (CSR); under stream capture from 2^16 outputs; (M,K) weights
-                                       without x_sel not from 2^21 outputs and 512 inputs on                     */
+                                       2^22 outputs (CSR); under stream capture from 2^16 outputs; not for (M,K)
+                                       weights without x_sel from 2^21 outputs and 512 inputs on, nor for (K,M)
+                                       weights, 2048 to 8191 rows and up to 512 inputs                           */
 #define MAM_BACKWARD_FORK_OFF 0
 #define MAM_BACKWARD_FORK_ON 1
 #define MAM_BACKWARD_ONE_LAUNCH_OFF 0

@@ -24,9 +24,9 @@
 // hits, at about half of the path's 64 bytes per clock and CU) with the arithmetic hidden under it.
 // The lowest column missing from the row is found once per row; the
 // implicit-zero candidate x[n, missing] * 0 is compared last under the dense rule (greater wins,
-// equal -> lower index wins).  TI follows the number of workgroups (below, at the launch).  The 16 waves of a workgroup own 16
-// consecutive neurons and hand
-// their results over through LDS so that every batch row stores 64 contiguous bytes per array.
+// equal -> lower index wins).  TI follows the number of workgroups (below, at the launch).  The 16 waves of
+// a workgroup own 16 consecutive neurons and hand their results over through LDS so that every batch row stores 64
+// contiguous bytes per array.
 //
 // Backward: when the forward handed over the selected values and their entry positions, x_grad is the
 // dense x_grad kernel fed with those values (an implicit zero contributes 0), and val_grad is

@@ -966,7 +966,8 @@ typedef const __attribute__((address_space(4))) float const_f32;
 // all the tile's partials complete, combines them in ascending k with strict compares and resolves in its
 // own epilogue, as the unsplit kernel does.
 enum Rest { REST_NONE, REST_GROUPS, REST_ANY };
-// TOUCH: a wave fetches its x into the L2 a tile ahead (see touch_x; the choice made per call costs the calls that don't 1 to 3 %).
+// TOUCH: a wave fetches its x into the L2 a tile ahead (see touch_x; over 28 calls of all forms the choice made per call costs those that don't
+// 0 to 4 %, 1.4 on average).
 template <int TJ, bool ARGS, bool SPLIT, Rest REST, int GT = G, bool FUSE = false, bool TOUCH = false>
 __global__ __launch_bounds__(sx::NT, 4) void mam_fwd_sx_kernel(const Params p)
 {
